@@ -266,6 +266,15 @@ int tv_selective_state_update(void* state, const void* x, const void* dt,
                               int batch, int nheads, int headdim, int ngroups,
                               int dstate, int dtype, int dt_softplus,
                               void* stream);
+/* The same on rows of a wider buffer: x (batch, nheads * headdim), dt (batch, nheads), Bm / Cm (batch, ngroups * dstate) by row
+ * strides in elements (the slices of the mixer's projection, read in place); y dense. */
+int tv_selective_state_update_rows(void* state, const void* x, const void* dt,
+                                   const void* A, const void* Bm, const void* Cm,
+                                   const void* D, const void* dt_bias, void* y,
+                                   int batch, int nheads, int headdim, int ngroups,
+                                   int dstate, int64_t x_stride, int64_t dt_stride,
+                                   int64_t b_stride, int64_t c_stride, int dtype,
+                                   int dt_softplus, void* stream);
 
 /* ------------------------------------------------------------------------
  * ViT linears with fused epilogues: C = epilogue(A . W^T), A (M,K), W (N,K) =
@@ -577,6 +586,24 @@ int tv_gemv_add_fwd(const void* x, const void* W, const void* bias, const float*
                     int M, int N, int K, int64_t x_stride, int64_t ldw, void* stream);
 int tv_gemv_glu_fwd(const void* z, const void* u, const int64_t* u_ids, int64_t u_rows, const void* W, void* y, int M, int N,
                     int K, int64_t z_stride, int64_t u_stride, int64_t ldw, int64_t y_stride, void* stream);
+
+/* ------------------------------------------------------------------------
+ * Products of a few rows (csrc/gemm_skinny.hip; M = 2..TV_GEMM_ROWS_MAX bf16 rows, K % 64 == 0, rows 16-byte aligned), on the
+ * matrix cores: y = x W^T + bias (bias bf16 or NULL), fp32 sums, one rounding.
+ * tv_gemm_rows_fwd: y bf16, or fp32 without epilogue; epilogue TV_GEMM_ROWS_RELU2: y = relu(bf16(.))^2; conv_state not NULL: the
+ *   outputs [conv_row0, conv_row0 + conv_channels) pass through tv_causal_conv1d_update (width 4, SiLU) on conv_state
+ *   (M, conv_channels, 4), as in tv_gemv_bf16_fwd.
+ * tv_gemm_rows_add_fwd, tv_gemm_rows_pair_fwd: tv_gemv_add_fwd and tv_gemv_pair_fwd for these rows.                        */
+#define TV_GEMM_ROWS_MAX 32
+#define TV_GEMM_ROWS_RELU2 1
+int tv_gemm_rows_fwd(const void* x, const void* W, const void* bias, void* y, int y_dtype, int M, int N, int K, int64_t x_stride,
+                     int64_t ldw, int64_t y_stride, int epilogue, void* conv_state, const void* conv_weight,
+                     const void* conv_bias, int conv_row0, int conv_channels, void* stream);
+int tv_gemm_rows_add_fwd(const void* x, const void* W, const void* bias, const float* residual, float* residual_out, void* h_out,
+                         int M, int N, int K, int64_t x_stride, int64_t ldw, void* stream);
+int tv_gemm_rows_pair_fwd(const void* x, const void* x2, const void* W, const void* bias, void* y, void* act, int M, int n1,
+                          int ff, int K, int64_t x_stride, int64_t x2_stride, int64_t ldw, int64_t y_stride,
+                          int64_t act_stride, void* stream);
 
 /* ------------------------------------------------------------------------
  * Linear attention with one constant decay per head, ragged batches:

@@ -42,6 +42,7 @@ SIGNATURES = {
     "tv_ssd_scan_last_impl": (_i, []),
     "tv_ssd_head_set_asm": (None, [_i]),
     "tv_selective_state_update": (_i, [_p] * 9 + [_i] * 7 + [_p]),
+    "tv_selective_state_update_rows": (_i, [_p] * 9 + [_i] * 5 + [_l] * 4 + [_i, _i, _p]),
     "tv_gemm_bf16_fwd": (_i, [_p, _p, _p, _p, _l, _i, _i, _l, _l, _l, _i, _i, _p]),
     "tv_gemm_set_persist": (None, [_i, _i]),
     "tv_gemm_set_drip": (None, [_i]),
@@ -80,6 +81,9 @@ SIGNATURES = {
     "tv_gemv_pair_fwd": (_i, [_p] * 6 + [_i] * 4 + [_l] * 5 + [_p]),
     "tv_gemv_add_fwd": (_i, [_p] * 6 + [_i] * 3 + [_l] * 2 + [_p]),
     "tv_gemv_glu_fwd": (_i, [_p] * 3 + [_l] + [_p] * 2 + [_i] * 3 + [_l] * 4 + [_p]),
+    "tv_gemm_rows_fwd": (_i, [_p] * 4 + [_i] * 4 + [_l] * 3 + [_i] + [_p] * 3 + [_i, _i, _p]),
+    "tv_gemm_rows_add_fwd": (_i, [_p] * 6 + [_i] * 3 + [_l] * 2 + [_p]),
+    "tv_gemm_rows_pair_fwd": (_i, [_p] * 6 + [_i] * 4 + [_l] * 5 + [_p]),
     "tv_lightning_workspace_bytes": (_z, [_i] * 6),
     "tv_lightning_fwd": (_i, [_p] * 8 + [_i, _i, _p, _z] + [_i] * 3 + [_l] * 4 + [_i, _i, _p]),
     "tv_attn_generic_fwd": (_i, [_p] * 8 + [_i, _l] + [_i] * 4 + [_l] * 10 + [_f] + [_i] * 3 + [_p, _l, _l, _i, _p]),
@@ -100,7 +104,7 @@ class TimeViperHipError(RuntimeError):
     pass
 
 
-ABI_VERSION = 14      # tv_abi_version() of the library these SIGNATURES describe (csrc/capi.cpp)
+ABI_VERSION = 15      # tv_abi_version() of the library these SIGNATURES describe (csrc/capi.cpp)
 
 
 def lib_path() -> Path:

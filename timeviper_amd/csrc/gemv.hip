@@ -22,7 +22,7 @@
 // (the last three belong to models on a 32-bit residual stream and agree with tv_rmsnorm_ex_fwd and tv_gated_mul_fwd)
 // with the rounding points of the stand-alone kernels (norms.hip), so the fused step and the unfused one agree to the
 // accumulation order of the dot products.  fp32 accumulation (v_dot2c_f32_bf16), one rounding of y.
-#include "ssd_common.hpp"
+#include "gemm_skinny.hpp"
 
 namespace {
 
@@ -956,7 +956,11 @@ extern "C" int tv_gemv_post_fwd(const void* x, const void* W, void* y, int y_dty
   if (y_dtype == TV_F32) a.y32 = (float*)y; else a.y = (bf16_t*)y;
   a.M = M; a.N = N; a.K = K; a.group = K; a.xs = x_stride; a.ldw = ldw; a.ys = y_stride; a.eps = eps;
   hipStream_t st = (hipStream_t)stream;
-  if (prologue == PRO_NONE) return launch_gemv<PRO_NONE>(a, st);
+  if (prologue == PRO_NONE) {
+    if (tv_skinny_takes(x, W, M, K, x_stride, ldw, 0))
+      return tv_gemm_rows_fwd(x, W, nullptr, y, y_dtype, M, N, K, x_stride, ldw, y_stride, 0, nullptr, nullptr, nullptr, 0, 0, stream);
+    return launch_gemv<PRO_NONE>(a, st);
+  }
   TV_CHECK_ARG(norm_weight && (norm_weight_dtype == TV_F32 || norm_weight_dtype == TV_BF16), "gemv_post: norm weight (fp32 or bf16) needed");
   a.norm_w = norm_weight; a.norm_w_f32 = norm_weight_dtype == TV_F32; a.woff = weight_offset; a.mult = mult;
   if (prologue == PRO_POSTNORM) {
@@ -977,6 +981,9 @@ extern "C" int tv_gemv_add_fwd(const void* x, const void* W, const void* bias, c
   if (K % 8 || ldw % 8 || x_stride % 8 || ((uintptr_t)x & 15) || ((uintptr_t)W & 15))
     TV_UNSUPPORTED("gemv_add: K and the row strides must be multiples of 8 elements, operands 16-byte aligned");
   if ((size_t)M * K * 2 > 128 * 1024) TV_UNSUPPORTED("gemv_add: M x K = %d x %d does not fit the 128 KiB of LDS x is held in", M, K);
+  // several rows: the matrix cores (2 048 x 7 680, four rows: 12.3 -> 7.4 us)
+  if (tv_skinny_takes(x, W, M, K, x_stride, ldw, 0))
+    return tv_skinny_add(x, W, bias, residual, residual_out, h_out, M, N, K, x_stride, ldw, (hipStream_t)stream);
   GemvArgs a{};
   a.x = (const bf16_t*)x; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias;
   a.M = M; a.N = N; a.K = K; a.group = K; a.xs = x_stride; a.ldw = ldw; a.ys = N;
@@ -1019,6 +1026,8 @@ extern "C" int tv_gemv_pair_fwd(const void* x, const void* x2, const void* W, co
   if (K % 8 || ldw % 8 || x_stride % 8 || x2_stride % 8 || ((uintptr_t)x & 15) || ((uintptr_t)x2 & 15) || ((uintptr_t)W & 15))
     TV_UNSUPPORTED("gemv_pair: K and the row strides must be multiples of 8 elements, operands 16-byte aligned");
   if ((size_t)M * K * 2 > 128 * 1024) TV_UNSUPPORTED("gemv_pair: M x K = %d x %d does not fit the 128 KiB of LDS", M, K);
+  if (tv_skinny_takes(x, W, M, K, x_stride, ldw, ff) && (!ff || tv_skinny_takes(x2, W, M, K, x2_stride, ldw, ff)))
+    return tv_skinny_pair(x, x2, W, bias, y, act, M, n1, ff, K, x_stride, x2_stride, ldw, y_stride, act_stride, (hipStream_t)stream);
   PairArgs a{(const bf16_t*)x, (const bf16_t*)x2, (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)y, (bf16_t*)act, M, n1, ff, K, 0,
              x_stride, x2_stride, ldw, y_stride, act_stride};
   // two work-groups per CU, shared out by rows; no more than there are groups for the waves

@@ -147,19 +147,20 @@ __global__ void state_update_kernel(float* __restrict__ state, const T* __restri
                                     const T* __restrict__ dt, const float* __restrict__ A,
                                     const T* __restrict__ Bm, const T* __restrict__ Cm,
                                     const float* __restrict__ D, const float* __restrict__ dt_bias,
-                                    T* __restrict__ y, int H, int P, int G, int N, int softplus) {
+                                    T* __restrict__ y, int H, int P, int G, int N, int64_t xs, int64_t ds, int64_t bs,
+                                    int64_t cs, int softplus) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   const int h = blockIdx.y, b = blockIdx.z;
   if (p >= P) return;
   const int g = h / (H / G);
-  float d = to_f32(dt[(int64_t)b * H + h]) + (dt_bias ? dt_bias[h] : 0.f);
+  float d = to_f32(dt[b * ds + h]) + (dt_bias ? dt_bias[h] : 0.f);
   if (softplus) d = softplus_f(d);
   const float dec = expf(d * A[h]);
-  const float xr = to_f32(x[((int64_t)b * H + h) * P + p]);
+  const float xr = to_f32(x[b * xs + h * P + p]);
   const float xv = d * xr;
   float* s = state + (((int64_t)b * H + h) * P + p) * N;
-  const T* Br = Bm + ((int64_t)b * G + g) * N;
-  const T* Cr = Cm + ((int64_t)b * G + g) * N;
+  const T* Br = Bm + b * bs + g * N;
+  const T* Cr = Cm + b * cs + g * N;
   float acc = 0.f;
   for (int n = 0; n < N; ++n) {
     const float v = fmaf(dec, s[n], xv * to_f32(Br[n]));
@@ -196,7 +197,8 @@ __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restri
                                                                         const T* __restrict__ Bm, const T* __restrict__ Cm,
                                                                         const float* __restrict__ D,
                                                                         const float* __restrict__ dt_bias, T* __restrict__ y,
-                                                                        int H, int P, int G, int softplus, int rows_total) {
+                                                                        int H, int P, int G, int64_t xs, int64_t ds, int64_t bs,
+                                                                        int64_t cs, int softplus, int rows_total) {
   constexpr int N = 4 * LPR, RPW = 64 / LPR, IT = 1, WAVES = 4;      // IT: state rows per lane group in flight
   typedef typename std::conditional<std::is_same<T, float>::value, f32x4, typename std::conditional<std::is_same<T, bf16_t>::value, bf16x4, f16x4>::type>::type vec4_t;
   const int lane = threadIdx.x & 63;
@@ -216,13 +218,13 @@ __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restri
     const int h = bh - b * H;
     const int g = (int)((unsigned)h / (unsigned)hpg);
     sv[it] = __builtin_nontemporal_load((const f32x4*)(state + (int64_t)rc * N) + ln);
-    dtv[it] = to_f32(dt[bh]);
-    xr[it] = to_f32(x[rc]);
+    dtv[it] = to_f32(dt[b * ds + h]);
+    xr[it] = to_f32(x[b * xs + (rc - b * H * P)]);
     av[it] = A[h];
     bv[it] = dt_bias ? dt_bias[h] : 0.f;
     dv[it] = D ? D[h] : 0.f;
-    Bv[it] = *(const vec4_t*)(Bm + (int64_t)(b * G + g) * N + 4 * ln);
-    Cv[it] = *(const vec4_t*)(Cm + (int64_t)(b * G + g) * N + 4 * ln);
+    Bv[it] = *(const vec4_t*)(Bm + b * bs + g * N + 4 * ln);
+    Cv[it] = *(const vec4_t*)(Cm + b * cs + g * N + 4 * ln);
   }
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -277,6 +279,15 @@ extern "C" int tv_selective_state_update(void* state, const void* x, const void*
                                          const void* D, const void* dt_bias, void* y, int batch,
                                          int nheads, int headdim, int ngroups, int dstate,
                                          int dtype, int dt_softplus, void* stream) {
+  return tv_selective_state_update_rows(state, x, dt, A, Bm, Cm, D, dt_bias, y, batch, nheads, headdim, ngroups, dstate,
+                                        (int64_t)nheads * headdim, nheads, (int64_t)ngroups * dstate, (int64_t)ngroups * dstate, dtype,
+                                        dt_softplus, stream);
+}
+
+extern "C" int tv_selective_state_update_rows(void* state, const void* x, const void* dt, const void* A, const void* Bm, const void* Cm,
+                                              const void* D, const void* dt_bias, void* y, int batch, int nheads, int headdim, int ngroups,
+                                              int dstate, int64_t x_stride, int64_t dt_stride, int64_t b_stride, int64_t c_stride, int dtype,
+                                              int dt_softplus, void* stream) {
   TV_CHECK_ARG(state && x && dt && A && Bm && Cm && y, "selective_state_update: null pointer");
   TV_CHECK_ARG(batch > 0 && nheads > 0 && headdim > 0 && ngroups > 0 && dstate > 0 &&
                    nheads % ngroups == 0,
@@ -285,14 +296,14 @@ extern "C" int tv_selective_state_update(void* state, const void* x, const void*
   // d_state 16 / 32 / 64 / 128 / 256 with 16-byte aligned rows: lanes share a row (coalesced); anything else: a thread per row
   const int lpr = dstate / 4;
   if (dstate % 4 == 0 && (lpr == 4 || lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64) && (((uintptr_t)state) & 15) == 0 &&
-      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && (int64_t)batch * nheads * headdim < (1ll << 31)) {
+      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && b_stride % 4 == 0 && c_stride % 4 == 0 && (int64_t)batch * nheads * headdim < (1ll << 31)) {
     const int64_t rows = (int64_t)batch * nheads * headdim;
     const int64_t rows_per_block = 4 * (64 / lpr);              // 4 waves x rows per wave-instruction
     const dim3 rgrid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
 #define TV_SUR(T, LPR)                                                                                        \
     state_update_chain_kernel<T, LPR><<<rgrid, 256, 0, s>>>((float*)state, (const T*)x, (const T*)dt,         \
         (const float*)A, (const T*)Bm, (const T*)Cm, (const float*)D, (const float*)dt_bias, (T*)y, nheads,   \
-        headdim, ngroups, dt_softplus, (int)rows)
+        headdim, ngroups, x_stride, dt_stride, b_stride, c_stride, dt_softplus, (int)rows)
 #define TV_SUR_T(T)                                                                                           \
     switch (lpr) { case 4: TV_SUR(T, 4); break; case 8: TV_SUR(T, 8); break; case 16: TV_SUR(T, 16); break;     \
                    case 32: TV_SUR(T, 32); break; default: TV_SUR(T, 64); break; }
@@ -310,7 +321,7 @@ extern "C" int tv_selective_state_update(void* state, const void* x, const void*
 #define TV_SU(T)                                                                              \
   state_update_kernel<T><<<grid, 64, 0, s>>>((float*)state, (const T*)x, (const T*)dt,        \
       (const float*)A, (const T*)Bm, (const T*)Cm, (const float*)D, (const float*)dt_bias,    \
-      (T*)y, nheads, headdim, ngroups, dstate, dt_softplus)
+      (T*)y, nheads, headdim, ngroups, dstate, x_stride, dt_stride, b_stride, c_stride, dt_softplus)
   switch (dtype) {
     case TV_F32: TV_SU(float); break;
     case TV_BF16: TV_SU(bf16_t); break;

@@ -440,12 +440,17 @@ def selective_state_update(state, x, dt, A, B, C, D=None, z=None, dt_bias=None,
     head = lambda t, nd: None if t is None else \
         (t if t.dim() == nd else t[(..., *([0] * (t.dim() - nd)))]).to(torch.float32).contiguous()
     A1, D1, b1 = head(A, 1), head(D, 1), head(dt_bias, 1)
-    dt1 = (dt if dt.dim() == 2 else dt[..., 0]).to(x.dtype).contiguous()
-    xc, Bc, Cc = x.contiguous(), B.to(x.dtype).contiguous(), C.to(x.dtype).contiguous()
-    y = torch.empty_like(xc)
-    check(_capi.lib().tv_selective_state_update(
+    # slices of the mixer's projection are read in place (one row per sequence, dense behind the batch dimension)
+    rows = lambda t: t if all(t.stride(d) == t[0].numel() // math.prod(t.shape[1:d + 1]) for d in range(1, t.dim())) and t.data_ptr() % 16 == 0 \
+        and t.stride(0) % 8 == 0 else t.contiguous()
+    dt1 = (dt if dt.dim() == 2 else dt[..., 0]).to(x.dtype)
+    dt1 = dt1 if dt1.stride(1) == 1 else dt1.contiguous()
+    xc, Bc, Cc = rows(x), rows(B.to(x.dtype)), rows(C.to(x.dtype))
+    y = torch.empty((Bsz, H, P), dtype=x.dtype, device=x.device)
+    check(_capi.lib().tv_selective_state_update_rows(
         _p(state), _p(xc), _p(dt1), _p(A1), _p(Bc), _p(Cc), _p(D1), _p(b1), _p(y), Bsz, H, P, G,
-        N, _dt(x), int(bool(dt_softplus)), _stream()), "tv_selective_state_update")
+        N, xc.stride(0), dt1.stride(0), Bc.stride(0), Cc.stride(0), _dt(x), int(bool(dt_softplus)), _stream()),
+        "tv_selective_state_update_rows")
     return y
 
 
@@ -618,11 +623,86 @@ def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=Non
         if (cst.dtype != x.dtype or cw.dtype != x.dtype or not cst.is_contiguous() or not cw.is_contiguous()
                 or cst.shape != (M, nch, 4) or cw.shape != (nch, 4) or (cb is not None and (cb.dtype != x.dtype or not cb.is_contiguous()))):
             raise TimeViperHipError("gemv_fused: conv needs a contiguous (rows, C, 4) state and (C, 4) weight of x's dtype")
+    if rows_take(x2, weight) and M * K * 2 <= 128 * 1024:
+        # several rows: the operator in front as its own launch and the product on the matrix cores (22 656 x 4 480, four rows: 42.8 us with
+        # the prologue in the matrix-vector kernel, 30.5 + 5); same rounding points
+        f = _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd=K)
+        _rows_product(f, weight, bias, y, 0, cst, cw, cb, row0, nch)
+        return y
     check(_capi.lib().tv_gemv_bf16_fwd(
         _p(x2), _p(weight), _p(bias), _p(y), M, N, K, x2.stride(0), weight.stride(0), N, int(prologue),
         _p(d2), 0 if d2 is None else d2.stride(0), _p(s2), 0 if s2 is None else s2.stride(0),
         _p(norm_weight), nw_dt, float(eps), _p(g2), 0 if g2 is None else g2.stride(0), int(group_size),
         _p(cst), _p(cw), _p(cb), int(row0), int(nch), _stream()), "tv_gemv_bf16_fwd")
+    return y
+
+
+ROWS_MAX = 32
+
+
+def rows_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Shapes tv_gemm_rows_fwd is written for: 2..32 rows of bf16 against a bf16 (N, K) weight, K a multiple of 64."""
+    Kd = x.shape[-1]
+    n = x.numel() // max(Kd, 1)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2 and 2 <= n <= ROWS_MAX
+            and Kd % 64 == 0 and Kd > 0 and weight.stride(1) == 1 and weight.stride(0) % 8 == 0 and weight.stride(0) < (1 << 24)
+            and weight.data_ptr() % 16 == 0)
+
+
+def _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd):
+    """f(x) of gemv_fused for several rows, by the stand-alone kernels"""
+    if prologue == GEMV_NONE:
+        ok = x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.stride(0) < (1 << 24) and x2.data_ptr() % 16 == 0
+        return x2 if ok else x2.contiguous()
+    if prologue not in (GEMV_RMSNORM, GEMV_RELU2, GEMV_GATED):
+        raise TimeViperHipError(f"gemv_fused: prologue {prologue}")
+    M = x2.shape[0]
+    f = torch.empty((M, Kd), dtype=x2.dtype, device=x2.device)
+    lib = _capi.lib()
+    if prologue == GEMV_RELU2:
+        xc = x2 if x2.is_contiguous() else x2.contiguous()
+        check(lib.tv_relu2_fwd(_p(xc), _p(f), xc.numel(), _dt(xc), _stream()), "tv_relu2_fwd")
+        return f
+    if norm_weight is None or nw_dt not in (TV_F32, TV_BF16):
+        raise TimeViperHipError("gemv_fused: norm weight (fp32 or bf16) needed")
+    if prologue == GEMV_RMSNORM:
+        check(lib.tv_rmsnorm_fwd(_p(x2), _p(d2), _p(norm_weight), _p(s2), _p(f), M, Kd, x2.stride(0),
+                                 0 if d2 is None else d2.stride(0), 0 if s2 is None else s2.stride(0), Kd, float(eps), _dt(x2), nw_dt, _stream()),
+              "tv_rmsnorm_fwd")
+    else:
+        check(lib.tv_rmsnorm_gated_fwd(_p(x2), _p(g2), _p(norm_weight), _p(f), M, Kd, int(group_size), x2.stride(0),
+                                       0 if g2 is None else g2.stride(0), Kd, float(eps), _dt(x2), nw_dt, _stream()), "tv_rmsnorm_gated_fwd")
+    return f
+
+
+def _rows_product(f, weight, bias, y, epilogue=0, cst=None, cw=None, cb=None, row0=0, nch=0):
+    N = weight.shape[0]
+    y2 = y.view(-1, N)
+    check(_capi.lib().tv_gemm_rows_fwd(_p(f), _p(weight), _p(bias), _p(y2), _dt(y2), f.shape[0], N, f.shape[1], f.stride(0), weight.stride(0),
+                                       y2.stride(0), int(epilogue), _p(cst), _p(cw), _p(cb), int(row0), int(nch), _stream()), "tv_gemm_rows_fwd")
+
+
+def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None):
+    """x @ weight.T (+ bias) for 2..32 bf16 rows on the matrix cores (a decoded token for each of several sequences).  `relu2`: the squared
+    ReLU of the bf16 product; `conv=(conv_state, weight, bias, row0)`: the outputs [row0, row0 + C) go through
+    `causal_conv1d_update` (width 4, SiLU) on conv_state (rows, C, 4), as in `gemv_fused`.  out_dtype: bf16, or fp32 without either."""
+    _gpu(x, weight, bias)
+    if not rows_take(x, weight) or weight.shape[1] != x.shape[-1]:
+        raise TimeViperHipError(f"rows_linear: 2..{ROWS_MAX} bf16 rows of a multiple of 64 elements, got {tuple(x.shape)} against {tuple(weight.shape)}")
+    if bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous() or bias.numel() != weight.shape[0]):
+        raise TimeViperHipError("rows_linear: bias must be contiguous, of x's dtype")
+    x2 = _rows_prologue(_rows2d(x), GEMV_NONE, *(None,) * 7, Kd=x.shape[-1])
+    cst = cw = cb = None
+    row0 = nch = 0
+    if conv is not None:
+        cst, cw, cb, row0 = conv
+        _gpu(cst, cw, cb)
+        nch = cst.shape[1]
+        if (cst.dtype != x.dtype or cw.dtype != x.dtype or not cst.is_contiguous() or not cw.is_contiguous() or cst.shape != (x2.shape[0], nch, 4)
+                or cw.shape != (nch, 4) or (cb is not None and (cb.dtype != x.dtype or not cb.is_contiguous()))):
+            raise TimeViperHipError("rows_linear: conv needs a contiguous (rows, C, 4) state and (C, 4) weight of x's dtype")
+    y = torch.empty(x.shape[:-1] + (weight.shape[0],), dtype=out_dtype or x.dtype, device=x.device)
+    _rows_product(x2, weight, bias, y, 1 if relu2 else 0, cst, cw, cb, row0, nch)
     return y
 
 
@@ -1354,7 +1434,7 @@ def _bf16_bias(t, n, what):
             raise TimeViperHipError(f"{what}: bf16")
 
 
-def gemv_pair(x, x2, weight, n1, bias=None, act_out=None):
+def gemv_pair(x, x2, weight, n1, bias=None, act_out=None, many=False):
     """Both input products of a parallel layer for 1..4 bf16 rows, one launch: y = x @ weight[:n1].T (returned) and, when weight has more
     rows (gate | up), act_out = gelu_tanh(x2 @ gate.T + b) * (x2 @ up.T + b), bias = their biases."""
     _gpu(x, x2, weight, bias, act_out)
@@ -1367,13 +1447,19 @@ def gemv_pair(x, x2, weight, n1, bias=None, act_out=None):
     if ff:
         _bf16_bias(bias, 2 * ff, "gemv_pair bias")
     y = torch.empty((M, n1), dtype=x.dtype, device=x.device)
-    check(_capi.lib().tv_gemv_pair_fwd(_p(x), _p(x2) if ff else None, _p(weight), _p(bias), _p(y), _p(act_out) if ff else None, M, int(n1), ff, D,
-                                       x.stride(0), x2.stride(0) if ff else 0, weight.stride(0), n1, act_out.stride(0) if ff else 0, _stream()),
-          "tv_gemv_pair_fwd")
+    lib = _capi.lib()
+    fn, what = (lib.tv_gemv_pair_fwd, "tv_gemv_pair_fwd") if not many else (lib.tv_gemm_rows_pair_fwd, "tv_gemm_rows_pair_fwd")
+    check(fn(_p(x), _p(x2) if ff else None, _p(weight), _p(bias), _p(y), _p(act_out) if ff else None, M, int(n1), ff, D,
+             x.stride(0), x2.stride(0) if ff else 0, weight.stride(0), n1, act_out.stride(0) if ff else 0, _stream()), what)
     return y
 
 
-def gemv_add(x, weight, residual, bias=None):
+def rows_pair(x, x2, weight, n1, bias=None, act_out=None):
+    """gemv_pair for 2..32 rows (`rows_take`)"""
+    return gemv_pair(x, x2, weight, n1, bias, act_out, many=True)
+
+
+def gemv_add(x, weight, residual, bias=None, many=False):
     """(residual + x @ weight.T + bias in fp32, its bf16 rounding) for 1..4 bf16 rows; residual (M, N) fp32"""
     _gpu(x, weight, bias, residual)
     _gemv_rows("gemv_add", weight, x)
@@ -1382,9 +1468,15 @@ def gemv_add(x, weight, residual, bias=None):
     if residual.dtype != torch.float32 or residual.shape != (M, N) or not residual.is_contiguous():
         raise TimeViperHipError("gemv_add: a dense fp32 residual (M, N)")
     xo, h = torch.empty_like(residual), torch.empty((M, N), dtype=x.dtype, device=x.device)
-    check(_capi.lib().tv_gemv_add_fwd(_p(x), _p(weight), _p(bias), _p(residual), _p(xo), _p(h), M, N, x.shape[1], x.stride(0), weight.stride(0),
-                                      _stream()), "tv_gemv_add_fwd")
+    lib = _capi.lib()
+    fn, what = (lib.tv_gemv_add_fwd, "tv_gemv_add_fwd") if not many else (lib.tv_gemm_rows_add_fwd, "tv_gemm_rows_add_fwd")
+    check(fn(_p(x), _p(weight), _p(bias), _p(residual), _p(xo), _p(h), M, N, x.shape[1], x.stride(0), weight.stride(0), _stream()), what)
     return xo, h
+
+
+def rows_add(x, weight, residual, bias=None):
+    """gemv_add for 2..32 rows (`rows_take`)"""
+    return gemv_add(x, weight, residual, bias, many=True)
 
 
 def gemv_glu(z, u, weight, ids=None):

@@ -298,10 +298,23 @@ def _fused_decode(x: torch.Tensor) -> bool:
             and not torch.is_grad_enabled() and os.environ.get("TV_DECODE_FUSED", "1") != "0")
 
 
+def _rows_decode(x: torch.Tensor) -> bool:
+    """5..32 sequences: the products run on the matrix cores (tv_gemm_rows_fwd), whatever does not fit their epilogues beside them."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] == 1 and 4 < x.shape[0] <= K.ROWS_MAX
+            and not torch.is_grad_enabled() and os.environ.get("TV_DECODE_FUSED", "1") != "0")
+
+
 def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     if _fused_decode(x) and K.gemv_takes(x, mod.weight):
         return K.gemv_fused(x, mod.weight, mod.bias)
+    if _rows_decode(x) and K.rows_take(x, mod.weight):
+        return K.rows_linear(x, mod.weight, mod.bias)
     return mod(x)
+
+
+def _norm_add(norm, hidden, delta):
+    """(norm of hidden + delta, the sum)"""
+    return norm(hidden, residual=delta, return_sum=True) if delta is not None else (norm(hidden), hidden)
 
 
 # ------------------------------------------------------------------ layers
@@ -438,28 +451,38 @@ class NemotronHMamba2Mixer(nn.Module):
 
     def decode_fused(self, hidden, delta, norm, cache_params):
         """One decode token with the block's RMSNorm (+ residual add) inside in_proj and the gated norm inside out_proj:
-        in_proj (+ conv update in its epilogue) -> state update -> out_proj, 3 launches.  Returns (residual stream, mixer output)."""
+        in_proj (+ conv update in its epilogue) -> state update -> out_proj, 3 launches.  Returns (residual stream, mixer output).
+        More than four sequences: the norms as launches of their own."""
         B = hidden.shape[0]
-        new_hidden = torch.empty_like(hidden) if delta is not None else hidden
+        rows = B > 4
+        if rows:
+            normed, new_hidden = _norm_add(norm, hidden, delta)
+        else:
+            new_hidden = torch.empty_like(hidden) if delta is not None else hidden
         gts = self.n_groups * self.ssm_state_size
         d_in = self.intermediate_size
         conv_state = cache_params.conv_states[self.layer_idx]
         w = self.conv1d.weight.squeeze(1)
         # the conv update rides in the product's epilogue where the kernel offers it (width 4, SiLU, K < 8192)
-        conv_in = (self.conv_kernel_size == 4 and self.activation in ("silu", "swish") and hidden.shape[-1] < 8192
+        conv_in = (self.conv_kernel_size == 4 and self.activation in ("silu", "swish") and (rows or hidden.shape[-1] < 8192)
                    and conv_state.dtype == hidden.dtype and conv_state.is_contiguous() and w.is_contiguous())
-        proj = K.gemv_fused(hidden, self.in_proj.weight, self.in_proj.bias, K.GEMV_RMSNORM, delta=delta,
-                            sum_out=new_hidden if delta is not None else None, norm_weight=norm.weight,
-                            eps=norm.variance_epsilon,
-                            conv=(conv_state, w, self.conv1d.bias, d_in) if conv_in else None)
+        conv = (conv_state, w, self.conv1d.bias, d_in) if conv_in else None
+        if rows:
+            proj = K.rows_linear(normed, self.in_proj.weight, self.in_proj.bias, conv=conv)
+        else:
+            proj = K.gemv_fused(hidden, self.in_proj.weight, self.in_proj.bias, K.GEMV_RMSNORM, delta=delta,
+                                sum_out=new_hidden if delta is not None else None, norm_weight=norm.weight,
+                                eps=norm.variance_epsilon, conv=conv)
         gate, xBC, dt = proj.split([d_in, self.conv_dim, self.num_heads], dim=-1)
         negA, D32, dtb32 = self._consts()
         xBC = xBC[:, 0] if conv_in else K.causal_conv1d_update(xBC[:, 0], conv_state, w, self.conv1d.bias, self.activation)
         x, Bm, Cm = torch.split(xBC, [d_in, gts, gts], dim=-1)
         y = K.selective_state_update(
-            cache_params.ssm_states[self.layer_idx], x.reshape(B, self.num_heads, self.head_dim), dt[:, 0], negA,
-            Bm.reshape(B, self.n_groups, -1), Cm.reshape(B, self.n_groups, -1), D32, z=None, dt_bias=dtb32,
+            cache_params.ssm_states[self.layer_idx], x.unflatten(1, (self.num_heads, self.head_dim)), dt[:, 0], negA,
+            Bm.unflatten(1, (self.n_groups, -1)), Cm.unflatten(1, (self.n_groups, -1)), D32, z=None, dt_bias=dtb32,
             dt_softplus=True)
+        if rows:
+            return new_hidden, K.rows_linear(self.norm(y.view(B, 1, d_in), gate), self.out_proj.weight, self.out_proj.bias)
         out = K.gemv_fused(y.reshape(B, 1, d_in), self.out_proj.weight, self.out_proj.bias, K.GEMV_GATED,
                            norm_weight=self.norm.weight, eps=self.norm.variance_epsilon, gate=gate,
                            group_size=self.norm.group_size)
@@ -486,7 +509,12 @@ class NemotronHMLP(nn.Module):
         return self.down_proj(K.relu2(self.up_proj(x), inplace=True))
 
     def decode_fused(self, hidden, delta, norm):
-        """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches."""
+        """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches (more than four sequences: 3,
+        relu^2 behind up_proj)."""
+        if hidden.shape[0] > 4:
+            normed, new_hidden = _norm_add(norm, hidden, delta)
+            u = K.rows_linear(normed, self.up_proj.weight, self.up_proj.bias, relu2=True)
+            return new_hidden, K.rows_linear(u, self.down_proj.weight, self.down_proj.bias)
         new_hidden = torch.empty_like(hidden) if delta is not None else hidden
         u = K.gemv_fused(hidden, self.up_proj.weight, self.up_proj.bias, K.GEMV_RMSNORM, delta=delta,
                          sum_out=new_hidden if delta is not None else None, norm_weight=norm.weight,
@@ -550,11 +578,15 @@ class NemotronHAttention(nn.Module):
         """One decode token: the block's RMSNorm (+ residual add) in the prologue of ONE q / k / v product, cache append,
         split-KV attention, o_proj — 4 launches + the cache writes, against 7."""
         B = hidden.shape[0]
-        new_hidden = torch.empty_like(hidden) if delta is not None else hidden
         nq, nkv = self.num_heads * self.head_dim, self.num_key_value_heads * self.head_dim
-        qkv = K.gemv_fused(hidden, self._qkv_weight(), None, K.GEMV_RMSNORM, delta=delta,
-                           sum_out=new_hidden if delta is not None else None, norm_weight=norm.weight,
-                           eps=norm.variance_epsilon)
+        if B > 4:
+            normed, new_hidden = _norm_add(norm, hidden, delta)
+            qkv = K.rows_linear(normed, self._qkv_weight())
+        else:
+            new_hidden = torch.empty_like(hidden) if delta is not None else hidden
+            qkv = K.gemv_fused(hidden, self._qkv_weight(), None, K.GEMV_RMSNORM, delta=delta,
+                               sum_out=new_hidden if delta is not None else None, norm_weight=norm.weight,
+                               eps=norm.variance_epsilon)
         q, k, v = qkv.split([nq, nkv, nkv], dim=-1)
         q = q.view(B, 1, self.num_heads, self.head_dim)
         k = k.view(B, 1, self.num_key_value_heads, self.head_dim)
@@ -758,7 +790,9 @@ class NemotronHModel(PdropMixin, nn.Module):
         train_pdrop_args = kwargs.get("train_pdrop_args")
         self.last_pdrop_trace = []
         delta = None  # pending mixer output, added inside the next fused norm
-        fused_step = (_fused_decode(hidden) and past_key_values is not None and cache_position is not None
+        c = self.config
+        fused_step = ((_fused_decode(hidden) or (_rows_decode(hidden) and all(n % 64 == 0 for n in (
+                          c.hidden_size, c.intermediate_size, c.mamba_num_heads * c.mamba_head_dim)))) and past_key_values is not None and cache_position is not None
                       and int(cache_position[0]) > 0 and not output_hidden_states and not self.check_nan
                       and hidden.shape[-1] % 8 == 0 and hidden.shape[-1] <= 8192
                       and self._all_matrices_bf16())

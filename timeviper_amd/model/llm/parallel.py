@@ -52,6 +52,8 @@ class TokenSide(nn.Module):
         return F.linear(K.gated_mul(F.linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
 
     def decode(self, h, ids, rows):
+        if h.shape[0] > 4:
+            return K.rows_linear(K.gated_mul(K.rows_linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
         return K.gemv_glu(K.gemv_post(h, self.gate), rows, self.proj, ids=ids)
 
 
@@ -87,6 +89,8 @@ class ParallelLayer(nn.Module):
         return x, (self.side(h, ids, side_rows), self.side.norm)
 
     def decode_takes(self, rows, dtype):
+        if 4 < rows <= K.ROWS_MAX:               # the products on the matrix cores: a multiple of 64 columns each
+            return dtype == torch.bfloat16 and self.k1 % 8 == 0 and all(n % 64 == 0 for n in (self.shift.numel(), self.out.shape[1], self.side.dim))
         return all(K.gemv_rows_take(rows, n, dtype) for n in (self.shift.numel(), self.out.shape[1], self.side.dim)) and self.k1 % 8 == 0
 
     def decode(self, x, pending, ids, side_rows, state, kv_rows, plan):
@@ -95,7 +99,8 @@ class ParallelLayer(nn.Module):
         y, w = pending or (None, None)
         x, h, hs = K.norm_shift(x, self.gain, self.eps, y, w, self.shift, state, plan, need_h=self.mlp is not None)
         u = torch.empty((x.shape[0], self.out.shape[1]), dtype=hs.dtype, device=hs.device)
-        p = K.gemv_pair(hs, h, self.inp, self.n1, self.inp_bias, act_out=u[:, self.k1:])
+        pair, add = (K.rows_pair, K.rows_add) if x.shape[0] > 4 else (K.gemv_pair, K.gemv_add)
+        p = pair(hs, h, self.inp, self.n1, self.inp_bias, act_out=u[:, self.k1:])
         self.mixer.attend(p, kv_rows, plan, out=u[:, :self.k1])
-        x, h = K.gemv_add(u, self.out, x, self.out_bias)
+        x, h = add(u, self.out, x, self.out_bias)
         return x, (self.side.decode(h, ids, side_rows), self.side.norm)
