@@ -655,6 +655,16 @@ int tv_flash_attn_window_fwd(const void* q, const void* k, const void* v, void* 
                              int64_t q_stride_l, int64_t q_stride_h, int64_t k_stride_l, int64_t k_stride_h,
                              int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_l, int64_t o_stride_h,
                              int64_t gate_stride_l, int64_t gate_stride_h, float softmax_scale, int dtype, void* stream);
+/* The same for the sequences of a packed step, one launch per 32 of them: sequence s owns rows [rows[s], rows[s] + lens_q[s]) of
+ * q, o and gate and sees the first lens_k[s] rows of entry slots[s] of k and v (k / v_stride_b apart).  rows, lens_q, lens_k and
+ * slots are HOST arrays, read before the call returns. */
+int tv_flash_attn_window_packed_fwd(const void* q, const void* k, const void* v, void* o, const void* gate, int window,
+                                    int keep_first, int v_dim, int nseq, const int* rows, const int* lens_q, const int* lens_k,
+                                    const int* slots, int nheads_q, int nheads_kv, int headdim, int64_t q_stride_l,
+                                    int64_t q_stride_h, int64_t k_stride_b, int64_t k_stride_l, int64_t k_stride_h,
+                                    int64_t v_stride_b, int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_l,
+                                    int64_t o_stride_h, int64_t gate_stride_l, int64_t gate_stride_h, float softmax_scale,
+                                    int dtype, void* stream);
 
 /* The same attention for one token per sequence (bf16; dims multiples of 8, at most 256): query row b (nheads_q x dim)
  * against the first keys[b] rows of block slot[b] of cache (slots, capacity, nheads_kv (dim + v_dim)), a row = all keys,

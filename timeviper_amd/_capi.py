@@ -49,6 +49,7 @@ SIGNATURES = {
     "tv_flash_attn_fwd": (_i, [_p] * 5 + [_i] * 6 + [_l] * 12 + [_f, _i, _i, _p]),
     "tv_flash_attn_sink_fwd": (_i, [_p] * 5 + [_i] * 7 + [_l] * 12 + [_f, _i, _p]),
     "tv_flash_attn_window_fwd": (_i, [_p] * 5 + [_i] * 8 + [_l] * 10 + [_f, _i, _p]),
+    "tv_flash_attn_window_packed_fwd": (_i, [_p] * 5 + [_i] * 4 + [_p] * 4 + [_i] * 3 + [_l] * 12 + [_f, _i, _p]),
     "tv_attn_window_decode_workspace_bytes": (_z, [_i] * 7),
     "tv_attn_window_decode_fwd": (_i, [_p] * 7 + [_i] * 8 + [_l] * 4 + [_f, _p, _z, _p]),
     "tv_flash_attn_set_variant": (None, [_i]),

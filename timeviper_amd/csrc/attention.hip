@@ -18,6 +18,7 @@
 // (flash_attention_class.py:59-66).
 #include "ssd_common.hpp"
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -88,6 +89,26 @@ struct AttnArgs {
   int notrim;        // streaming kernel (dev, TV_FA_TRIM=0): the last key tile runs all its sub-tiles
 };
 
+// Sequences of a packed step (WIN): rows [row, row + len_q) of q, o and gate against the first len_k rows of batch entry `slot`
+constexpr int FA_SEQS = 32;
+struct AttnSeqs {
+  int row[FA_SEQS], len_q[FA_SEQS], len_k[FA_SEQS], slot[FA_SEQS];
+};
+struct NoSeqs {};
+
+// Work-group `id` of a grid of query blocks x (batch, head) pairs, the pairs fastest: block `t` of `pair`.  A causal block's cost
+// grows with its position, so the blocks of all heads are dealt out by falling cost (a grid that finishes one head after
+// the other ends with the last heads' heaviest blocks running alone: 40 heads x 5 003 tokens 402 us, dealt out 309; 10 007 tokens: 1 475, 1 215).
+// An XCD (id % 8) gets a contiguous range of the pairs in every round, about the same one: heads that share K / V share an L2.
+__device__ __forceinline__ void block_of(int id, int pairs, int& t, int& pair) {
+  t = id / pairs;
+  const int p = id - t * pairs, q = pairs >> 3, rem = pairs & 7;
+  const int x0 = (id - p) & 7, x = id & 7;             // XCD of the round's first work-group, and of this one
+  // an XCD gets q pairs of a round, the `rem` XCDs from x0 on (modulo 8) one more: those in front of XCD x
+  const int more = x0 + rem <= 8 ? min(max(x - x0, 0), rem) : min(x, x0 + rem - 8) + max(x - x0, 0);
+  pair = x * q + more + (p >> 3);
+}
+
 // KS = ceil(D/16) k-steps of QK^T, DT = ceil(D/32) d-tiles of PV, NW waves per workgroup.
 // K/V tiles of 32*KT keys go global -> LDS by LDS-DMA (global_load_lds_dwordx4, 16 bytes per
 // lane, no VGPR round trip: staging through registers cost a third of the kernel) into a
@@ -97,9 +118,10 @@ struct AttnArgs {
 // row%16) and the transposing reads of V (ds_read_b64_tr_b16, chunk ^ 4(row%4)) are bank
 // conflict free.  Chunks past head_dim are never copied (the K ones QK^T reads are zeroed once).
 // WIN: causal with a sliding window and kept first keys.  The work-group visits the tiles that hold kept keys, then jumps to the
-// first tile of its first row's window: ring, copies and waits count the visited tiles.
+// first tile of its first row's window: ring, copies and waits count the visited tiles.  All sequences of a packed step share the
+// launch (a launch per prompt leaves most of the chip idle: six prompts, 6 011 tokens, 16 heads on 4 x 128, window 1 024: 265 us, in one launch 95).
 template <typename T, int KS, int DT, int NW, int KT, bool WIN = false>
-__global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
+__global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename std::conditional<WIN, AttnSeqs, NoSeqs>::type sq) {
   constexpr int FA_KB = 32 * KT;     // keys per tile
   constexpr int NPK = FA_KB / 4;     // 1 KiB DMA pieces (4 key rows) of K per tile; as many of V
   typedef typename Frag<T>::v8 v8;
@@ -118,12 +140,26 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 31, hh = lane >> 5;
-  // causal: launch the heaviest (last) query blocks first
-  // 3-D grid (causal: heaviest query blocks first), or — many short sequences (ViT frames) — a 1-D
-  // grid whose ids walk the query blocks of ONE (batch, head) on one XCD (id % 8): the blocks that
+  // 1-D grid.  Few sequences: `block_of` (causal: the heaviest query blocks of all heads first).  Many short sequences (ViT
+  // frames): ids walk the query blocks of ONE (batch, head) on one XCD (id % 8): the blocks that
   // share K / V then share an L2 instead of pulling the same keys into three of them
-  int qblk, h, b;
-  if (a.nqb > 0) {
+  int qblk, h, b, Lq = a.Lq, Lk = a.Lk;
+  int64_t row0 = 0;                             // WIN: the sequence's first row of q, o and gate
+  if constexpr (WIN) {
+    int t;
+    block_of(blockIdx.x, a.Hq, t, h);
+    int s = 0, nblk;
+    for (;; ++s) {                              // (t is below the sum of the sequences' blocks: launcher)
+      nblk = (sq.len_q[s] + QB - 1) / QB;
+      if (t < nblk) break;
+      t -= nblk;
+    }
+    qblk = nblk - 1 - t;
+    Lq = sq.len_q[s];
+    Lk = sq.len_k[s];
+    row0 = sq.row[s];
+    b = sq.slot[s];
+  } else if (a.nqb > 0) {
     const int slot = blockIdx.x >> 3;
     // an XCD owns a contiguous range of (batch, head) pairs: neighbouring heads of a frame interleave
     // in memory (head_dim 72 = 144-byte rows inside 128-byte lines), so their shared lines hit one L2
@@ -133,17 +169,20 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
     b = pair / a.Hq;
     if (b >= a.nb) return;                    // (batch, head) pairs are padded to a multiple of 8
   } else {
-    qblk = a.causal ? (gridDim.x - 1 - blockIdx.x) : blockIdx.x;
-    h = blockIdx.y;
-    b = blockIdx.z;
+    const int pairs = a.nb * a.Hq;
+    int pair;
+    block_of(blockIdx.x, pairs, qblk, pair);
+    if (a.causal) qblk = (int)gridDim.x / pairs - 1 - qblk;
+    h = pair % a.Hq;
+    b = pair / a.Hq;
   }
   const int hk = h / (a.Hq / a.Hkv);
   const int q0 = qblk * QB + wave * FA_QW;      // first query row of this wave
   const int qrow = q0 + r;                      // this lane's query row
   const int D = a.D;
-  const int shift = a.Lk - a.Lq;                // bottom-right causal alignment
+  const int shift = Lk - Lq;                // bottom-right causal alignment
 
-  const T* qp = (const T*)a.q + (int64_t)b * a.qsb + (int64_t)h * a.qsh;
+  const T* qp = (const T*)a.q + (WIN ? row0 * a.qsl : (int64_t)b * a.qsb) + (int64_t)h * a.qsh;
   const T* kp = (const T*)a.k + (int64_t)b * a.ksb + (int64_t)hk * a.ksh;
   const T* vp = (const T*)a.v + (int64_t)b * a.vsb + (int64_t)hk * a.vsh;
 
@@ -166,7 +205,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int d0 = ks * 16 + hh * 8;
-    qraw[ks] = gload16_async((qrow < a.Lq && d0 < D) ? qp + (int64_t)qrow * a.qsl + d0 : qp);
+    qraw[ks] = gload16_async((qrow < Lq && d0 < D) ? qp + (int64_t)qrow * a.qsl + d0 : qp);
   }
 
   f32x16 oacc[DT];
@@ -177,8 +216,8 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
   float m_run = -INFINITY, l_run = 0.f;
 
   // key range this workgroup needs
-  const int wg_q_last = min(qblk * QB + QB, a.Lq) - 1;
-  int k_end = a.causal ? min(a.Lk, wg_q_last + shift + 1) : a.Lk;
+  const int wg_q_last = min(qblk * QB + QB, Lq) - 1;
+  int k_end = a.causal ? min(Lk, wg_q_last + shift + 1) : Lk;
   if (k_end < 0) k_end = 0;
   int ntiles = (k_end + FA_KB - 1) / FA_KB;
   int tkeep = 0, tskip = 0;                     // WIN: visited tile i is tile i, or i + tskip from tkeep on
@@ -211,7 +250,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
     const bool isK = pc < NPK;           // wave-uniform
     const void* tb = ssdk::uniform_ptr(isK ? (const void*)(kp + (int64_t)kbase * a.ksl)
                                            : (const void*)(vp + (int64_t)kbase * a.vsl));
-    const int left = a.Lk - kbase;          // rows of this tile that exist
+    const int left = Lk - kbase;          // rows of this tile that exist
     unsigned off = p_off[i];
     if (left < FA_KB) {                  // last tile: rows past the end repeat the last key (masked later)
       const int rr = min(p_row[i], left - 1);
@@ -249,7 +288,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
   for (int ks = 0; ks < KS; ++ks) {      // the Q loads are older than every copy: landed
     settle(qraw[ks]);
     const v8 z = {};
-    qf[ks] = (qrow < a.Lq && ks * 16 + hh * 8 < D) ? __builtin_bit_cast(v8, qraw[ks]) : z;
+    qf[ks] = (qrow < Lq && ks * 16 + hh * 8 < D) ? __builtin_bit_cast(v8, qraw[ks]) : z;
   }
 
   for (int kt = 0; kt < ntiles; ++kt) {
@@ -297,7 +336,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
       // ---- mask, running max on the raw scores (the scale is positive, so it commutes with
       // max), then p = 2^(s*scale - m) as one FMA + v_exp per score; packed fp32 math ----
       typedef float f32x2 __attribute__((ext_vector_type(2)));
-      bool need_mask = (kbase + FA_KB > a.Lk) || (a.causal && kbase + FA_KB - 1 > q0 + shift);
+      bool need_mask = (kbase + FA_KB > Lk) || (a.causal && kbase + FA_KB - 1 > q0 + shift);
       if constexpr (WIN) need_mask = need_mask || (kbase <= wave_q_last + shift - a.window && kbase + FA_KB > a.keep);
       if (need_mask) {
 #pragma unroll
@@ -305,7 +344,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const int key = kbase + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh;
-            bool ok = key < a.Lk && (!a.causal || key <= qrow + shift);
+            bool ok = key < Lk && (!a.causal || key <= qrow + shift);
             if constexpr (WIN) ok = ok && (key > qrow + shift - a.window || key < a.keep);
             sacc[t][i] = ok ? sacc[t][i] : -INFINITY;
           }
@@ -392,8 +431,8 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
   float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   if (a.sink) l_tot += __builtin_amdgcn_exp2f(a.sink[h] * 1.4426950408889634f - m_run);      // (not scaled; inf: the keys weigh nothing)
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (qrow < a.Lq) {
-    T* op = (T*)a.o + (int64_t)b * a.osb + (int64_t)qrow * a.osl + (int64_t)h * a.osh;
+  if (qrow < Lq) {
+    T* op = (T*)a.o + (WIN ? 0 : (int64_t)b * a.osb) + (row0 + qrow) * a.osl + (int64_t)h * a.osh;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -403,7 +442,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
           v4 pk;
           if constexpr (WIN) {
             if (a.gate) {
-              const v4 gt = *(const v4*)((const T*)a.gate + (int64_t)qrow * a.gsl + (int64_t)h * a.gsh + d0);
+              const v4 gt = *(const v4*)((const T*)a.gate + (row0 + qrow) * a.gsl + (int64_t)h * a.gsh + d0);
 #pragma unroll
               for (int j = 0; j < 4; ++j) oacc[dt][4 * g + j] *= sigmoid_f((float)gt[j]);
             }
@@ -413,9 +452,9 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a) {
           *(v4*)(op + d0) = pk;
         }
       }
-    if (a.lse && hh == 0) {
+    if (!WIN && a.lse && hh == 0) {
       const float lse = l_tot > 0.f ? (m_run * 0.6931471805599453f + logf(l_tot)) : -INFINITY;
-      a.lse[((int64_t)b * a.Hq + h) * a.Lq + qrow] = lse;
+      a.lse[((int64_t)b * a.Hq + h) * Lq + qrow] = lse;
     }
   }
 }
@@ -871,7 +910,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
         static const int stream_ = [] { const char* v = getenv("TV_FA_STREAM"); return v ? atoi(v) : 1; }();
         const int64_t slots = (int64_t)ax.ppx * nqb;          // query blocks per XCD
         if constexpr (KS > 6) {                                // head_dim 128: the second Q set does not fit the registers
-          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax);
+          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax, NoSeqs{});
         } else if (stream_ && a.Lk > 32 * KT && slots > tv_cu_count() / 8) {
           // one resident work-group per CU streams its share of the query blocks
           static const int ones_ = [] { const char* v = getenv("TV_FA_ONES"); return v ? atoi(v) : 1; }();
@@ -895,19 +934,17 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
             if (e == hipSuccess) flash_fwd_stream_kernel<T, KS, DT, KT, false><<<grid_s, 512, lds, st>>>(ax);
           }
         } else {
-          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax);
+          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax, NoSeqs{});
         }
       } else {
-        dim3 grid(nqb, a.Hq, B);
-        flash_fwd_kernel<T, KS, DT, 8, KT><<<grid, 512, lds, st>>>(a);
+        flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)((int64_t)nqb * a.Hq * B)), 512, lds, st>>>(a, NoSeqs{});
       }
     }
   } else {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e == hipSuccess) {
-      dim3 grid((a.Lq + 127) / 128, a.Hq, B);
-      flash_fwd_kernel<T, KS, DT, 4, KT><<<grid, 256, lds, st>>>(a);
+      flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3((unsigned)((int64_t)((a.Lq + 127) / 128) * a.Hq * B)), 256, lds, st>>>(a, NoSeqs{});
     }
   }
   if (e != hipSuccess) {
@@ -917,33 +954,39 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-// windowed form: bf16, one query block of 256 (or, for short portions, 128) rows a work-group; 64-key tiles at head dim 128
-// (the bounds of the window do not fit beside 96 keys' fragments)
+// windowed form: bf16, one query block of 256 (or, if no sequence has more than 128 rows, 128) rows a work-group; 64-key tiles at head dim
+// 128 (the bounds of the window do not fit beside 96 keys' fragments)
 template <int KS, int DT>
-int launch_fa_win(const AttnArgs& a, int B, hipStream_t st) {
+int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) {
   constexpr int KT = KS > 6 ? 2 : FA_KT, lds = 2 * 3 * 32 * KT * 256;
-  const bool big = a.Lq > 128;
+  int most = 0;
+  for (int s = 0; s < nseq; ++s) most = sq.len_q[s] > most ? sq.len_q[s] : most;
+  const bool big = most > 128;
+  const int qb = big ? 256 : 128;
+  int64_t blocks = 0;
+  for (int s = 0; s < nseq; ++s) blocks += (sq.len_q[s] + qb - 1) / qb;
   const void* f = big ? (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true> : (const void*)flash_fwd_kernel<bf16_t, KS, DT, 4, KT, true>;
   const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) {
     tv_set_error("flash_attn: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     return TV_ERR_LAUNCH;
   }
-  if (big) flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<dim3((a.Lq + 255) / 256, a.Hq, B), 512, lds, st>>>(a);
-  else flash_fwd_kernel<bf16_t, KS, DT, 4, KT, true><<<dim3((a.Lq + 127) / 128, a.Hq, B), 256, lds, st>>>(a);
+  const dim3 grid((unsigned)(blocks * a.Hq));
+  if (big) flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<grid, 512, lds, st>>>(a, sq);
+  else flash_fwd_kernel<bf16_t, KS, DT, 4, KT, true><<<grid, 256, lds, st>>>(a, sq);
   TV_LAUNCH_CHECK();
+}
+
+int launch_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) {
+  const int D = a.D > a.Dv ? a.D : a.Dv;
+  if (D <= 64) return launch_fa_win<4, 2>(a, sq, nseq, st);
+  if (D <= 96) return launch_fa_win<6, 3>(a, sq, nseq, st);
+  return launch_fa_win<8, 4>(a, sq, nseq, st);                 // (<= 128: caller)
 }
 
 template <typename T>
 int launch_fa(const AttnArgs& a, int B, hipStream_t st) {
   const int D = a.D > a.Dv ? a.D : a.Dv;
-  if constexpr (std::is_same<T, bf16_t>::value) {
-    if (a.window > 0) {
-      if (D <= 64) return launch_fa_win<4, 2>(a, B, st);
-      if (D <= 96) return launch_fa_win<6, 3>(a, B, st);
-      if (D <= 128) return launch_fa_win<8, 4>(a, B, st);
-    }
-  }
   if (D <= 64) return launch_fa_d<T, 4, 2>(a, B, st);
   if (D <= 80) return launch_fa_d<T, 5, 3>(a, B, st);
   if (D <= 96) return launch_fa_d<T, 6, 3>(a, B, st);
@@ -961,13 +1004,7 @@ extern "C" int tv_fa_debug_stamps(unsigned long long* out) {
 
 extern "C" void tv_flash_attn_set_variant(int variant) { g_fa_variant.store(variant, std::memory_order_relaxed); }
 
-struct FlashWindow {
-  int window = 0, keep = 0;      // window 0: every key up to the query's own position
-  const void* gate = nullptr;
-  int64_t gsl = 0, gsh = 0;
-};
-
-static int flash_fwd(const FlashWindow& win, const void* q, const void* k, const void* v, void* o, void* lse, const float* sink, int v_dim,
+static int flash_fwd(const void* q, const void* k, const void* v, void* o, void* lse, const float* sink, int v_dim,
                                  int batch, int seqlen_q, int seqlen_k, int nheads_q,
                                  int nheads_kv, int headdim, int64_t q_stride_b,
                                  int64_t q_stride_l, int64_t q_stride_h, int64_t k_stride_b,
@@ -1007,7 +1044,7 @@ static int flash_fwd(const FlashWindow& win, const void* q, const void* k, const
   a.nb = batch;
   a.Dv = v_dim;
   a.sink = sink;
-  a.window = win.window; a.keep = win.keep; a.gate = win.gate; a.gsl = win.gsl; a.gsh = win.gsh;
+  a.window = a.keep = 0; a.gate = nullptr; a.gsl = a.gsh = 0;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == TV_BF16) return launch_fa<bf16_t>(a, batch, st);
   return launch_fa<f16_t>(a, batch, st);
@@ -1021,7 +1058,7 @@ extern "C" int tv_flash_attn_fwd(const void* q, const void* k, const void* v, vo
                                  int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_b,
                                  int64_t o_stride_l, int64_t o_stride_h, float softmax_scale,
                                  int causal, int dtype, void* stream) {
-  return flash_fwd(FlashWindow{}, q, k, v, o, lse, nullptr, headdim, batch, seqlen_q, seqlen_k, nheads_q, nheads_kv, headdim, q_stride_b, q_stride_l,
+  return flash_fwd(q, k, v, o, lse, nullptr, headdim, batch, seqlen_q, seqlen_k, nheads_q, nheads_kv, headdim, q_stride_b, q_stride_l,
                    q_stride_h, k_stride_b, k_stride_l, k_stride_h, v_stride_b, v_stride_l, v_stride_h, o_stride_b, o_stride_l, o_stride_h,
                    softmax_scale, causal, dtype, stream);
 }
@@ -1035,7 +1072,7 @@ extern "C" int tv_flash_attn_sink_fwd(const void* q, const void* k, const void* 
                                  int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_b,
                                  int64_t o_stride_l, int64_t o_stride_h, float softmax_scale,
                                  int dtype, void* stream) {
-  return flash_fwd(FlashWindow{}, q, k, v, o, nullptr, sink, v_dim, batch, seqlen_q, seqlen_k, nheads_q, nheads_kv, headdim, q_stride_b, q_stride_l,
+  return flash_fwd(q, k, v, o, nullptr, sink, v_dim, batch, seqlen_q, seqlen_k, nheads_q, nheads_kv, headdim, q_stride_b, q_stride_l,
                    q_stride_h, k_stride_b, k_stride_l, k_stride_h, v_stride_b, v_stride_l, v_stride_h, o_stride_b, o_stride_l, o_stride_h,
                    softmax_scale, 1, dtype, stream);
 }
@@ -1047,13 +1084,64 @@ extern "C" int tv_flash_attn_window_fwd(const void* q, const void* k, const void
                                         int64_t q_stride_l, int64_t q_stride_h, int64_t k_stride_l, int64_t k_stride_h,
                                         int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_l, int64_t o_stride_h,
                                         int64_t gate_stride_l, int64_t gate_stride_h, float softmax_scale, int dtype, void* stream) {
-  TV_CHECK_ARG(window > 0 && keep_first >= 0 && seqlen_k >= seqlen_q, "flash_attn_window: bad window or lengths");
+  const int zero = 0;
+  return tv_flash_attn_window_packed_fwd(q, k, v, o, gate, window, keep_first, v_dim, 1, &zero, &seqlen_q, &seqlen_k, &zero, nheads_q, nheads_kv, headdim,
+                                         q_stride_l, q_stride_h, 0, k_stride_l, k_stride_h, 0, v_stride_l, v_stride_h, o_stride_l, o_stride_h,
+                                         gate_stride_l, gate_stride_h, softmax_scale, dtype, stream);
+}
+
+// The same for the sequences of a packed step: sequence s owns rows [rows[s], rows[s] + lens_q[s]) of q, o and gate and sees the first
+// lens_k[s] rows of batch entry slots[s] of k and v (host arrays, read before the call returns).
+extern "C" int tv_flash_attn_window_packed_fwd(const void* q, const void* k, const void* v, void* o, const void* gate, int window, int keep_first,
+                                               int v_dim, int nseq, const int* rows, const int* lens_q, const int* lens_k, const int* slots,
+                                               int nheads_q, int nheads_kv, int headdim, int64_t q_stride_l, int64_t q_stride_h,
+                                               int64_t k_stride_b, int64_t k_stride_l, int64_t k_stride_h, int64_t v_stride_b,
+                                               int64_t v_stride_l, int64_t v_stride_h, int64_t o_stride_l, int64_t o_stride_h,
+                                               int64_t gate_stride_l, int64_t gate_stride_h, float softmax_scale, int dtype, void* stream) {
+  TV_CHECK_ARG(nseq >= 0 && (nseq == 0 || (rows && lens_q && lens_k && slots)), "flash_attn_window: sequences");
+  int64_t total = 0;
+  for (int s = 0; s < nseq; ++s) {
+    TV_CHECK_ARG(rows[s] >= 0 && lens_q[s] >= 0 && slots[s] >= 0 && lens_k[s] >= lens_q[s], "flash_attn_window: bad window or lengths");
+    total += lens_q[s];
+  }
+  TV_CHECK_ARG(window > 0 && keep_first >= 0, "flash_attn_window: bad window or lengths");
+  TV_CHECK_ARG(total == 0 || (q && o && k && v), "flash_attn: null pointer");
+  TV_CHECK_ARG(nheads_q > 0 && nheads_kv > 0 && nheads_q % nheads_kv == 0 && headdim > 0 && v_dim > 0 && softmax_scale > 0.f,
+               "flash_attn: bad sizes (or non-positive softmax scale)");
   if (dtype != TV_BF16) TV_UNSUPPORTED("flash_attn_window: dtype must be bf16");
+  if (headdim % 8 || v_dim % 8) TV_UNSUPPORTED("flash_attn: headdim %d / %d not a multiple of 8", headdim, v_dim);
   if (headdim > 128 || v_dim > 128) TV_UNSUPPORTED("flash_attn_window: headdim %d / %d > 128", headdim, v_dim);
   if (gate && (gate_stride_l % 4 || gate_stride_h % 4 || ((uintptr_t)gate & 7)))
     TV_UNSUPPORTED("flash_attn_window: gate rows must be 8-byte aligned");
-  FlashWindow w;
-  w.window = window; w.keep = keep_first; w.gate = gate; w.gsl = gate_stride_l; w.gsh = gate_stride_h;
-  return flash_fwd(w, q, k, v, o, nullptr, nullptr, v_dim, 1, seqlen_q, seqlen_k, nheads_q, nheads_kv, headdim, 0, q_stride_l, q_stride_h,
-                   0, k_stride_l, k_stride_h, 0, v_stride_l, v_stride_h, 0, o_stride_l, o_stride_h, softmax_scale, 1, dtype, stream);
+  const int64_t strides[] = {q_stride_l, q_stride_h, k_stride_b, k_stride_l, k_stride_h, v_stride_b, v_stride_l, v_stride_h};
+  for (int64_t s : strides)
+    if (s % 8) TV_UNSUPPORTED("flash_attn: q/k/v strides must be multiples of 8 elements");
+  if (o_stride_l % 4 || o_stride_h % 4 || ((uintptr_t)o & 7)) TV_UNSUPPORTED("flash_attn: o strides must be multiples of 4 elements");
+  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15)) TV_UNSUPPORTED("flash_attn: q/k/v must be 16-byte aligned");
+  if (128 * k_stride_l * 2 >= (1ll << 31) || 128 * v_stride_l * 2 >= (1ll << 31)) TV_UNSUPPORTED("flash_attn: k/v row stride too large");
+  if (total == 0) return TV_OK;
+  AttnArgs a{};
+  a.q = q; a.k = k; a.v = v; a.o = o;
+  a.Hq = nheads_q; a.Hkv = nheads_kv; a.D = headdim; a.Dv = v_dim;
+  a.qsl = q_stride_l; a.qsh = q_stride_h; a.ksb = k_stride_b; a.ksl = k_stride_l; a.ksh = k_stride_h;
+  a.vsb = v_stride_b; a.vsl = v_stride_l; a.vsh = v_stride_h; a.osl = o_stride_l; a.osh = o_stride_h;
+  a.scale_log2 = softmax_scale * 1.4426950408889634f;
+  a.causal = 1;
+  a.window = window; a.keep = keep_first; a.gate = gate; a.gsl = gate_stride_l; a.gsh = gate_stride_h;
+  // FA_SEQS sequences a launch, the longest of them first
+  for (int i = 0; i < nseq;) {
+    AttnSeqs sq{};
+    int n = 0;
+    for (; i < nseq && n < FA_SEQS; ++i) {
+      if (lens_q[i] == 0) continue;
+      int j = n++;
+      for (; j > 0 && sq.len_k[j - 1] < lens_k[i]; --j) {
+        sq.row[j] = sq.row[j - 1]; sq.len_q[j] = sq.len_q[j - 1]; sq.len_k[j] = sq.len_k[j - 1]; sq.slot[j] = sq.slot[j - 1];
+      }
+      sq.row[j] = rows[i]; sq.len_q[j] = lens_q[i]; sq.len_k[j] = lens_k[i]; sq.slot[j] = slots[i];
+    }
+    const int rc = n ? launch_win(a, sq, n, (hipStream_t)stream) : TV_OK;
+    if (rc != TV_OK) return rc;
+  }
+  return TV_OK;
 }

@@ -17,6 +17,7 @@ eager fallback: tensors must live on the GPU and the HIP library must be built.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 from typing import Optional
@@ -1229,15 +1230,14 @@ def attention_window(q, cache, plan, kv_heads, scale, window=NO_WINDOW, keep_fir
     _gpu(q, cache, gate, o)
     if H % kv_heads or any(t is not None and (t.shape != (T, H, dv) or t.dtype != q.dtype) for t in (gate, o)):
         raise TimeViperHipError("attention_window: gate and out (T, H, dv) of q's dtype")
-    lib, at = _capi.lib(), 0
-    for s, n, a in zip(plan.slots, plan.counts, plan.starts):
-        sl = slice(at, at + n)
-        gb = None if gate is None else gate[sl]
-        check(lib.tv_flash_attn_window_fwd(
-            _p(q[sl]), _p(k[s]), _p(v[s]), _p(o[sl]), _p(gb), int(window), int(keep_first), dv, n, a + n, H, kv_heads, dk, q.stride(0), q.stride(1),
-            k.stride(1), k.stride(2), v.stride(1), v.stride(2), o.stride(0), o.stride(1), 0 if gate is None else gate.stride(0),
-            0 if gate is None else gate.stride(1), float(scale), _dt(q), _stream()), "tv_flash_attn_window_fwd")
-        at += n
+    n = len(plan.counts)
+    ints = lambda v: (ctypes.c_int * n)(*v)
+    rows = [sum(plan.counts[:i]) for i in range(n)]
+    check(_capi.lib().tv_flash_attn_window_packed_fwd(
+        _p(q), _p(k), _p(v), _p(o), _p(gate), int(window), int(keep_first), dv, n, ints(rows), ints(plan.counts),
+        ints([a + c for a, c in zip(plan.starts, plan.counts)]), ints(plan.slots), H, kv_heads, dk, q.stride(0), q.stride(1), k.stride(0), k.stride(1),
+        k.stride(2), v.stride(0), v.stride(1), v.stride(2), o.stride(0), o.stride(1), 0 if gate is None else gate.stride(0),
+        0 if gate is None else gate.stride(1), float(scale), _dt(q), _stream()), "tv_flash_attn_window_packed_fwd")
     return o
 
 
