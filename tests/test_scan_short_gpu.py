@@ -1,0 +1,70 @@
+"""The scan of short sequences (csrc/ssd_cols.hip: column slices, no segments) against the token recurrence in 64 bits, over its modes."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from timeviper_amd import kernels
+    return kernels
+
+
+def recurrence(x, dt, A, B, C, D, S, heads_of):
+    """one sequence, token by token: x (L, H, P), dt (L, H) discretised, B / C (L, G, N), S (H, P, N); all fp64"""
+    y = torch.empty_like(x)
+    for t in range(x.shape[0]):
+        b, c = B[t, heads_of], C[t, heads_of]
+        S = torch.exp(dt[t] * A)[:, None, None] * S + (dt[t, :, None] * x[t])[:, :, None] * b[:, None]
+        y[t] = (S * c[:, None]).sum(-1) + D[:, None] * x[t]
+    return y, S
+
+
+# chunk edges, one token, the last chunk nearly empty / nearly full; head dims of one to five slices; a group's slices spread over
+# several heads; dt_std moves heads through floating, re-based, reset and standard steps
+@pytest.mark.parametrize("L", [1, 63, 64, 65, 129, 200, 390])
+@pytest.mark.parametrize("B,H,P,G,group_map", [(1, 8, 80, 2, "block"), (2, 8, 80, 2, "tile"), (1, 4, 32, 1, "block"), (1, 8, 64, 4, "block")])
+@pytest.mark.parametrize("decay", ["slow", "mixed", "fast"])
+def test_short_scan(K, L, B, H, P, G, group_map, decay):
+    N = 128
+    g = torch.Generator(device=DEV).manual_seed(L * 7 + H)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    proj = (1.3 * r(B, L, H * P + 16)).bfloat16()              # x and dt as slices of a wider row
+    x, dt = proj[..., :H * P].unflatten(-1, (H, P)), proj[..., H * P + 2:H * P + 2 + H]
+    bc = (0.3 * r(B, 2 * G, L, N)).bfloat16()
+    Bm, Cm = bc[:, :G].transpose(1, 2), bc[:, G:].transpose(1, 2)
+    A = -{"slow": torch.linspace(0.01, 1, H, device=DEV), "mixed": torch.linspace(0.01, 16, H, device=DEV),
+          "fast": torch.linspace(8, 60, H, device=DEV)}[decay]
+    bias, D = torch.linspace(-6, -1, H, device=DEV), r(H)
+    init = r(B, H, P, N)
+    y, fin, dec = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
+                                              group_map=group_map, return_total_decay=True)
+    assert K.ssd_scan_last_impl() == 6
+    h = torch.arange(H, device=DEV)
+    of = h % G if group_map == "tile" else h // (H // G)
+    for b in range(B):
+        d = F.softplus(dt[b].double() + bias.double())
+        yr, Sr = recurrence(x[b].double(), d, A.double(), Bm[b].double(), Cm[b].double(), D.double(), init[b].double(), of)
+        # bf16 operands (x~, C.B^T, the state's copy) and output: 2^-8 of the largest terms of a head
+        for got, want in ((y[b], yr), (fin[b][None].transpose(0, 1), Sr[:, None])):
+            ax = 0 if got is y[b] else 1
+            scale = want.abs().amax(dim=(0, 2) if want.dim() == 3 else (1, 2, 3), keepdim=True) + 1e-6
+            assert torch.isfinite(got).all() and ((got.double() - want).abs() / scale).max() < 2e-2, ax
+        assert torch.allclose(dec[b].double(), (d * A.double()).sum(0), rtol=1e-4, atol=1e-4)
+
+
+def test_segments_and_slices_agree(K):
+    """either side of the rule's line: 24 chunks in one pass, 25 in segments"""
+    H, P, G, N = 16, 80, 2, 128
+    g = torch.Generator(device=DEV).manual_seed(3)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    L = 25 * 64
+    x, dt, Bm, Cm = r(1, L, H, P).bfloat16(), r(1, L, H).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16()
+    A, bias, D = -torch.linspace(0.02, 16, H, device=DEV), torch.full((H,), -4.0, device=DEV), r(H)
+    f = lambda n: K.mamba_chunk_scan_combined(x[:, :n], dt[:, :n], A, Bm[:, :n], Cm[:, :n], D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
+    (long, _), (short, _) = f(L), f(L - 64)
+    rel = (long[:, :L - 64].float() - short.float()).norm() / short.float().norm()
+    assert rel < 5e-3, rel

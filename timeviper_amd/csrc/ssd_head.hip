@@ -41,6 +41,12 @@
 int tv_ssd_cb_prepass_launch(const void* Bm, const void* Cm, void* cb, int batch, int seqlen, int ngroups,
                              int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
                              hipStream_t st);
+// ssd_cols.hip: a 16-column slice of a head per wave, one pass without segments
+int tv_ssd_cols_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* cb, const void* D,
+                       const void* dt_bias, const void* init_state, void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads,
+                       int headdim, int ngroups, int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg,
+                       int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map,
+                       hipStream_t st);
 // ssd_correct.hip
 size_t tv_ssd_correct_all_workspace_bytes(int batch, int nheads, int nchunks, int nseg, int headdim);
 unsigned* tv_ssd_correct_all_counters(void* workspace, int batch, int nheads, int nchunks, int nseg, int headdim);
@@ -1216,26 +1222,49 @@ static_assert(sizeof(HeadSmemA) <= 160 * 1024, "LDS budget");
 // heads of one group per work-group: 4, 2 or 1
 int pick_nw(int hpg) { return hpg % 4 == 0 ? 4 : hpg % 2 == 0 ? 2 : 1; }
 
-// 1 024 waves fill the chip (one per SIMD); a segment is at least 16 chunks long
+// 1 024 waves fill the chip (one per SIMD); a segment is at least 7 chunks long (128 heads x 80: 2 048 tokens in 2 | 4 | 8 segments 128 | 99 | 99
+// us, 3 000 in 2 | 6 | 8 162 | 113 | 116, 5 000 in 4 | 8 171 | 150)
 int pick_segments(int batch, int nheads, int nchunks) {
   if (const char* e = getenv("TV_SSD_NSEG")) return atoi(e) > 0 ? atoi(e) : 1;     // dev tool
   const int waves = batch * nheads;
   int nseg = waves >= 768 ? 1 : 1024 / waves;
   if (nseg > 16) nseg = 16;
-  while (nseg > 1 && nchunks / nseg < 16) --nseg;
+  while (nseg > 1 && nchunks / nseg < 7) --nseg;
   return nseg < 1 ? 1 : nseg;
+}
+
+int cu_count() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
+      cus = 256;                               // MI355X
+    return cus;
+  }();
+  return n;
+}
+
+// Short sequences: column slices (ssd_cols.hip) while their work-groups (4 slices) all run at once and the march over them is no longer than
+// segments would make it.  128 heads x 80, 8 groups, whole operator, one segment | best number of segments | slices: 203 tokens 35 | 51 |
+// 17 us, 512: 56 | 59 | 29, 1 501: 146 | 89 | 83 - 93, 2 048: 180 | 98 | 107, 3 000: 244 | 113 | 128.
+bool use_cols(int batch, int nheads, int headdim, int ngroups, int nchunks) {
+  const int slices = nheads / ngroups * (headdim / 16);        // of a group
+  return nchunks <= 24 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= cu_count();
 }
 
 struct HeadLayout {
   size_t cb, seg_state, seg_decay, ctot, corr, dtt, total;
   int nseg, seg_chunks;
+  bool cols;
 };
 HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngroups) {
   HeadLayout l;
   const size_t nchunks = (size_t)(seqlen + HQ - 1) / HQ;
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-  l.nseg = pick_segments(batch, nheads, (int)nchunks);
+  l.cols = use_cols(batch, nheads, headdim, ngroups, (int)nchunks);
+  l.nseg = l.cols ? 1 : pick_segments(batch, nheads, (int)nchunks);
   l.seg_chunks = (int)((nchunks + l.nseg - 1) / l.nseg);
+  l.nseg = (int)((nchunks + l.seg_chunks - 1) / l.seg_chunks);         // no segment is empty (the march reads its first chunk)
   l.cb = 0;
   l.seg_state = up((size_t)batch * ngroups * nchunks * CBE * sizeof(bf16_t));
   const size_t st = (size_t)batch * nheads * headdim * HN * sizeof(float);
@@ -1319,6 +1348,14 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
   a.seg_state = lay.nseg > 1 ? (float*)(wsb + lay.seg_state) : nullptr;
   a.seg_decay = lay.nseg > 1 ? (float*)(wsb + lay.seg_decay) : nullptr;
   a.chunk_tot = lay.nseg > 1 ? (float*)(wsb + lay.ctot) : nullptr;
+  if (lay.cols && dsl < (1 << 24)) {           // (64 rows of dt at 32-bit offsets)
+    if (!cb_pre) {
+      const int rc = tv_ssd_cb_prepass_launch(Bm, Cm, workspace, batch, seqlen, ngroups, bsb, bsl, bsg, csb, csl, csg, st);
+      if (rc != TV_OK) return rc;
+    }
+    return tv_ssd_cols_launch(x, dt, A, Bm, Cm, a.cb, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups,
+                              xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, st);
+  }
   // dt head-major into the workspace (one small launch: 2 x 42 MB at 164 k tokens); both the march and the correction read it
   {
     const int64_t lp = (int64_t)a.nchunks * HQ;
