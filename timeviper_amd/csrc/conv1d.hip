@@ -1,152 +1,141 @@
-// S2: causal depthwise conv1d (+bias +SiLU), channels-last, HBM-bound.
-// Each lane owns 16 bytes of channels and slides a K-row register window down
-// TL consecutive tokens, so every x row is read once per tile (+K-1 halo rows
-// that hit L2) with fully coalesced 16-byte accesses.
+// S2: causal depthwise conv1d (+bias +SiLU), channels-last.
+// Each lane owns 16 bytes of channels of a strip of 8 consecutive tokens: all its rows in flight at once, fully coalesced, then a K-row
+// register window slides down them.  The K-1 rows in front of a strip are read again, from a cache.
+// Long sequences are bound by HBM (5.3 TB/s of x once in and once out), short ones by the one round trip to memory and the weights' loads in
+// front of it.  8 tokens, because a longer strip's rows come in several round trips; 12 288 channels, bf16, all with C.B^T, us for strips
+// of 8 | 16 | 32 | 64: 203 tokens 6.3 | 7.2 | 11.2 | 19.3, 1 501: 17 | 16 | 17 | 23, 49 999: 467 | 472 | 486 | 505 (of 4: 508).  With 64, weights
+// loaded two bytes at a time and B / C in a launch of their own it was 33, 35 and 534 us.
 // Reference semantics: modeling_nano.py:619-624 / :705 (zero left pad).
 #include "ssd_common.hpp"
 
 namespace {
 
-constexpr int CONV_TL = 64;       // tokens per tile
 constexpr int CONV_THREADS = 256;
+constexpr int CONV_TL = 8;       // tokens a strip
 
+// A lane's V channels: V K weights = K 16-byte vectors, where w and bias are aligned (wide); else one by one
 template <typename T, int K>
-__global__ __launch_bounds__(CONV_THREADS) void conv1d_fwd_kernel(
-    const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias,
-    const T* __restrict__ halo, T* __restrict__ y, int L, int C, int64_t xsb,
-    int64_t xsl, int64_t ysb, int64_t ysl, int silu) {
-  constexpr int V = Vec16<T>::N;
-  typedef typename Vec16<T>::type vec_t;
-  const int cv = blockIdx.x * CONV_THREADS + threadIdx.x;
-  const int c0 = cv * V;
-  if (c0 >= C) return;
-  const int b = blockIdx.z;
-  const int t0 = blockIdx.y * CONV_TL;
-  const int t1 = min(t0 + CONV_TL, L);
-
+struct ConvTaps {
+  enum { V = Vec16<T>::N };
   float wk[K][V], bs[V];
+  __device__ __forceinline__ void load(const T* __restrict__ w, const T* __restrict__ bias, int c0, int wide) {
+    typedef typename Vec16<T>::type vec_t;
+    if (wide) {
+      vec_t wv[K], bv = {};
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
+      for (int j = 0; j < K; ++j) wv[j] = *(const vec_t*)(w + (int64_t)c0 * K + j * V);
+      if (bias) bv = *(const vec_t*)(bias + c0);
 #pragma unroll
-    for (int j = 0; j < K; ++j) wk[j][i] = to_f32(w[(int64_t)(c0 + i) * K + j]);
-    bs[i] = bias ? to_f32(bias[c0 + i]) : 0.f;
-  }
-
-  const T* xb = x + (int64_t)b * xsb + c0;
-  T* yb = y + (int64_t)b * ysb + c0;
-  const T* hb = halo ? halo + (int64_t)b * (K - 1) * C + c0 : nullptr;
-
-  // window[j] holds row t-(K-1)+j
-  float win[K][V];
+      for (int i = 0; i < V; ++i) {
 #pragma unroll
-  for (int j = 0; j < K - 1; ++j) {
-    const int t = t0 - (K - 1) + j;
-    vec_t v;
-    bool have = true;
-    if (t >= 0) v = *(const vec_t*)(xb + (int64_t)t * xsl);
-    else if (hb) v = *(const vec_t*)(hb + (int64_t)(t + K - 1) * C);
-    else have = false;
+        for (int j = 0; j < K; ++j) wk[j][i] = to_f32(wv[(i * K + j) / V][(i * K + j) % V]);
+        bs[i] = to_f32(bv[i]);
+      }
+    } else {
 #pragma unroll
-    for (int i = 0; i < V; ++i) win[j][i] = have ? to_f32(v[i]) : 0.f;
-  }
-
-  for (int t = t0; t < t1; ++t) {
-    vec_t v = *(const vec_t*)(xb + (int64_t)t * xsl);
-    vec_t o;
+      for (int i = 0; i < V; ++i) {
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      win[K - 1][i] = to_f32(v[i]);
-      float acc = bs[i];
-#pragma unroll
-      for (int j = 0; j < K; ++j) acc = fmaf(wk[j][i], win[j][i], acc);
-      if (silu) acc = silu_f(acc);
-      o[i] = from_f32<T>(acc);
-#pragma unroll
-      for (int j = 0; j < K - 1; ++j) win[j][i] = win[j + 1][i];
+        for (int j = 0; j < K; ++j) wk[j][i] = to_f32(w[(int64_t)(c0 + i) * K + j]);
+        bs[i] = bias ? to_f32(bias[c0 + i]) : 0.f;
+      }
     }
-    *(vec_t*)(yb + (int64_t)t * ysl) = o;
   }
+};
+
+struct ConvArgs {
+  const void *x, *w, *bias, *halo;
+  void *yx, *yb, *yc, *cb;       // the plain form writes yx alone
+  int L, C, d_inner, G, N, silu, wide;
+  int nxb, per_xcd;              // blocks a strip of tokens; strips an XCD
+  int nchunks, nbc;              // blocks of the B / C part (0: its channels are in the strips)
+  int64_t xsb, xsl, ysb, ysl;
+};
+
+// A block's strip and channels: each XCD has a run of strips, so that the rows in front of a strip are in its L2 (4 096 tokens x 12 288
+// channels: 40.5 -> 35.5 us; no difference where a run is larger than the L2)
+template <typename T>
+__device__ __forceinline__ bool conv_place(const ConvArgs& a, int block, int c_end, int& c0, int& t0) {
+  const int xcd = block & 7, j = block >> 3;
+  c0 = (j % a.nxb * CONV_THREADS + (int)threadIdx.x) * Vec16<T>::N;
+  t0 = (xcd * a.per_xcd + j / a.nxb) * CONV_TL;
+  return c0 < c_end && t0 < a.L;
 }
 
-// Mamba-2 xBC variant: the three channel segments go to three destinations; B and C are
-// written group-major (B,G,L,N) so that one group's consecutive tokens are contiguous.
-struct XbcOut {
-  void *yx, *yb, *yc;
-  int d_inner, G, N;
-};
-template <typename T, int K>
-__global__ __launch_bounds__(CONV_THREADS) void conv1d_xbc_kernel(
-    const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias,
-    const T* __restrict__ halo, XbcOut o, int L, int C, int c_end, int64_t xsb, int64_t xsl, int silu) {
+// One lane's strip of CONV_TL rows from t0 on, of a sequence of L: all its rows and the K-1 in front of it are in flight before the
+// arithmetic; rows past the end repeat the last one and are not stored.  FAST: SiLU with the reciprocal instruction (the mixer's convolution).
+template <typename T, int K, bool FAST>
+__device__ __forceinline__ void conv_strip(const ConvArgs& a, int c0, int t0, int b, T* __restrict__ yb, int64_t ysl) {
   constexpr int V = Vec16<T>::N;
   typedef typename Vec16<T>::type vec_t;
-  const int cv = blockIdx.x * CONV_THREADS + threadIdx.x;
-  const int c0 = cv * V;
-  if (c0 >= c_end) return;       // c_end = C, or d_inner when the B / C channels run in conv1d_bc_cb_kernel
-  const int b = blockIdx.z;
-  const int t0 = blockIdx.y * CONV_TL;
-  const int t1 = min(t0 + CONV_TL, L);
-  // destination of this lane's 16 bytes: row pointer at t=0 and row stride
-  T* yb;
-  int64_t ysl;
-  const int gn = o.G * o.N;
-  if (c0 < o.d_inner) {
-    yb = (T*)o.yx + (int64_t)b * L * o.d_inner + c0;
-    ysl = o.d_inner;
-  } else {
-    const bool isB = c0 < o.d_inner + gn;
-    const int cc = c0 - o.d_inner - (isB ? 0 : gn);
-    const int g = cc / o.N, n = cc - g * o.N;
-    yb = (T*)(isB ? o.yb : o.yc) + ((int64_t)b * o.G + g) * L * o.N + n;
-    ysl = o.N;
-  }
-  float wk[K][V], bs[V];
-#pragma unroll
-  for (int i = 0; i < V; ++i) {
-#pragma unroll
-    for (int j = 0; j < K; ++j) wk[j][i] = to_f32(w[(int64_t)(c0 + i) * K + j]);
-    bs[i] = bias ? to_f32(bias[c0 + i]) : 0.f;
-  }
-  const T* xb = x + (int64_t)b * xsb + c0;
-  const T* hb = halo ? halo + (int64_t)b * (K - 1) * C + c0 : nullptr;
-  float win[K][V];
+  const T* xb = (const T*)a.x + (int64_t)b * a.xsb + c0;
+  const T* hb = a.halo ? (const T*)a.halo + (int64_t)b * (K - 1) * a.C + c0 : nullptr;
+  vec_t v[K - 1 + CONV_TL];
 #pragma unroll
   for (int j = 0; j < K - 1; ++j) {
     const int t = t0 - (K - 1) + j;
-    vec_t v;
-    bool have = true;
-    if (t >= 0) v = *(const vec_t*)(xb + (int64_t)t * xsl);
-    else if (hb) v = *(const vec_t*)(hb + (int64_t)(t + K - 1) * C);
-    else have = false;
-#pragma unroll
-    for (int i = 0; i < V; ++i) win[j][i] = have ? to_f32(v[i]) : 0.f;
+    v[j] = vec_t{};
+    if (t >= 0) v[j] = *(const vec_t*)(xb + (int64_t)t * a.xsl);
+    else if (hb) v[j] = *(const vec_t*)(hb + (int64_t)(t + K - 1) * a.C);
   }
-  auto step = [&](int t, const vec_t& v) {
+#pragma unroll
+  for (int u = 0; u < CONV_TL; ++u) v[K - 1 + u] = *(const vec_t*)(xb + (int64_t)min(t0 + u, a.L - 1) * a.xsl);
+  ConvTaps<T, K> tp;
+  tp.load((const T*)a.w, (const T*)a.bias, c0, a.wide);
+  float win[K][V];               // win[j] holds row t-(K-1)+j
+#pragma unroll
+  for (int j = 0; j < K - 1; ++j)
+#pragma unroll
+    for (int i = 0; i < V; ++i) win[j][i] = to_f32(v[j][i]);
+#pragma unroll
+  for (int u = 0; u < CONV_TL; ++u) {
     vec_t ov;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      win[K - 1][i] = to_f32(v[i]);
-      float acc = bs[i];
+      win[K - 1][i] = to_f32(v[K - 1 + u][i]);
+      float acc = tp.bs[i];
 #pragma unroll
-      for (int j = 0; j < K; ++j) acc = fmaf(wk[j][i], win[j][i], acc);
-      if (silu) acc *= __builtin_amdgcn_rcpf(1.f + __expf(-acc));   // x * sigmoid(x)
+      for (int j = 0; j < K; ++j) acc = fmaf(tp.wk[j][i], win[j][i], acc);
+      if (a.silu) acc = FAST ? acc * __builtin_amdgcn_rcpf(1.f + __expf(-acc)) : silu_f(acc);
       ov[i] = from_f32<T>(acc);
 #pragma unroll
       for (int j = 0; j < K - 1; ++j) win[j][i] = win[j + 1][i];
     }
-    *(vec_t*)(yb + (int64_t)t * ysl) = ov;
-  };
-  // four rows of loads in flight ahead of the arithmetic
-  constexpr int U = 4;
-  int t = t0;
-  for (; t + U <= t1; t += U) {
-    vec_t v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = *(const vec_t*)(xb + (int64_t)(t + u) * xsl);
-#pragma unroll
-    for (int u = 0; u < U; ++u) step(t + u, v[u]);
+    if (t0 + u < a.L) *(vec_t*)(yb + (int64_t)(t0 + u) * ysl) = ov;
   }
-  for (; t < t1; ++t) step(t, *(const vec_t*)(xb + (int64_t)t * xsl));
+}
+
+template <typename T, int K>
+__global__ __launch_bounds__(CONV_THREADS) void conv1d_fwd_kernel(ConvArgs a) {
+  int c0, t0;
+  if (!conv_place<T>(a, blockIdx.x, a.C, c0, t0)) return;
+  conv_strip<T, K, false>(a, c0, t0, blockIdx.y, (T*)a.yx + (int64_t)blockIdx.y * a.ysb + c0, a.ysl);
+}
+
+// Mamba-2 xBC variant: the three channel segments go to three destinations; B and C are
+// written group-major (B,G,L,N) so that one group's consecutive tokens are contiguous.
+template <typename T, int K>
+__device__ __forceinline__ void conv_xbc_block(const ConvArgs& a, int block, int b, int c_end) {
+  int c0, t0;
+  if (!conv_place<T>(a, block, c_end, c0, t0)) return;
+  // destination of this lane's 16 bytes: row pointer at t=0 and row stride
+  T* yb;
+  int64_t ysl;
+  const int gn = a.G * a.N;
+  if (c0 < a.d_inner) {
+    yb = (T*)a.yx + (int64_t)b * a.L * a.d_inner + c0;
+    ysl = a.d_inner;
+  } else {
+    const bool isB = c0 < a.d_inner + gn;
+    const int cc = c0 - a.d_inner - (isB ? 0 : gn);
+    const int g = cc / a.N, n = cc - g * a.N;
+    yb = (T*)(isB ? a.yb : a.yc) + ((int64_t)b * a.G + g) * a.L * a.N + n;
+    ysl = a.N;
+  }
+  conv_strip<T, K, true>(a, c0, t0, b, yb, ysl);
+}
+template <typename T, int K>
+__global__ __launch_bounds__(CONV_THREADS) void conv1d_xbc_kernel(ConvArgs a) {
+  conv_xbc_block<T, K>(a, blockIdx.x, blockIdx.y, a.C);
 }
 
 
@@ -157,42 +146,32 @@ __global__ __launch_bounds__(CONV_THREADS) void conv1d_xbc_kernel(
 // (ssd_slice.hip: 6 fragments of 512 bf16 per (chunk, group); fragment (ti, sp), lane (lc, kq) holds
 // CB[16 ti + lc][32 sp + 8 kq + 0..7]).  Round 2 recomputed it in a pre-pass of the scan that read B and C back from
 // memory (0.8 GB and ~100 us per layer at 164 k tokens).
-// grid (nchunks, G, batch), 256 threads: thread = (strip of 8 tokens, 16 bytes of the group's 256 B / C channels).
+// 256 threads: thread = (strip of 8 tokens, 16 bytes of the group's 256 B / C channels).
 constexpr int CBQ = 64, CBN = 128, CB_FRAGS = 6;
 template <int K>
-__global__ __launch_bounds__(256) void conv1d_bc_cb_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
-    const bf16_t* __restrict__ halo, bf16_t* __restrict__ yb, bf16_t* __restrict__ yc, bf16_t* __restrict__ cb,
-    int L, int C, int d_inner, int G, int nchunks, int64_t xsb, int64_t xsl, int silu) {
-  using namespace ssdk;
-  __shared__ __attribute__((aligned(16))) bf16_t tile[2][CBQ * CBN];     // [B | C][token][n], 16-byte chunk ^ (token & 15)
-  const int c = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x;
+__device__ __forceinline__ void conv_bc_cb_block(const ConvArgs& a, bf16_t (*tile)[CBQ * CBN], int c, int g, int b) {
+  using namespace ssdk;                                    // tile: [B | C][token][n], 16-byte chunk ^ (token & 15)
+  const int tid = threadIdx.x, L = a.L, C = a.C, silu = a.silu;
+  const int64_t xsl = a.xsl;
   const int strip = tid >> 5, l32 = tid & 31;
   const int isC = l32 >> 4, nch = l32 & 15;                // 16-byte chunk of the group's 128 states
-  const int c0 = d_inner + (isC ? G * CBN : 0) + g * CBN + nch * 8;
+  const int c0 = a.d_inner + (isC ? a.G * CBN : 0) + g * CBN + nch * 8;
   const int t0 = c * CBQ + strip * 8;
-  float wk[K][8], bs[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-#pragma unroll
-    for (int j = 0; j < K; ++j) wk[j][i] = to_f32(w[(int64_t)(c0 + i) * K + j]);
-    bs[i] = bias ? to_f32(bias[c0 + i]) : 0.f;
-  }
-  const bf16_t* xb = x + (int64_t)b * xsb + c0;
-  const bf16_t* hb = halo ? halo + (int64_t)b * (K - 1) * C + c0 : nullptr;
-  bf16_t* yg = (isC ? yc : yb) + ((int64_t)b * G + g) * L * CBN + nch * 8;
+  const bf16_t* xb = (const bf16_t*)a.x + (int64_t)b * a.xsb + c0;
+  const bf16_t* hb = a.halo ? (const bf16_t*)a.halo + (int64_t)b * (K - 1) * C + c0 : nullptr;
+  bf16_t* yg = (bf16_t*)(isC ? a.yc : a.yb) + ((int64_t)b * a.G + g) * L * CBN + nch * 8;
   bf16_t* tl = tile[isC];
   // all rows of the strip (and its K-1 predecessors) in flight, then the arithmetic
   bf16x8 v[K - 1 + 8];
 #pragma unroll
   for (int j = 0; j < K - 1 + 8; ++j) {
     const int t = t0 - (K - 1) + j;
-    bf16x8 z = {};
+    v[j] = bf16x8{};
     if (t >= 0 && t < L) v[j] = *(const bf16x8*)(xb + (int64_t)t * xsl);
     else if (t < 0 && hb) v[j] = *(const bf16x8*)(hb + (int64_t)(t + K - 1) * C);
-    else v[j] = z;
   }
+  ConvTaps<bf16_t, K> tp;
+  tp.load((const bf16_t*)a.w, (const bf16_t*)a.bias, c0, a.wide);
   float win[K][8];
 #pragma unroll
   for (int j = 0; j < K - 1; ++j)
@@ -205,9 +184,9 @@ __global__ __launch_bounds__(256) void conv1d_bc_cb_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       win[K - 1][i] = to_f32(v[K - 1 + u][i]);
-      float acc = bs[i];
+      float acc = tp.bs[i];
 #pragma unroll
-      for (int j = 0; j < K; ++j) acc = fmaf(wk[j][i], win[j][i], acc);
+      for (int j = 0; j < K; ++j) acc = fmaf(tp.wk[j][i], win[j][i], acc);
       if (silu) acc *= __builtin_amdgcn_rcpf(1.f + __expf(-acc));   // x * sigmoid(x)
       ov[i] = (bf16_t)acc;
 #pragma unroll
@@ -219,7 +198,6 @@ __global__ __launch_bounds__(256) void conv1d_bc_cb_kernel(
     *(bf16x8*)(tl + row * CBN + ((nch ^ (row & 15)) << 3)) = ov;
   }
   __syncthreads();
-  if (!cb) return;
   const int lane = tid & 63, wave = tid >> 6;
   if (wave == 3) return;
   const int lc = lane & 15, kq = lane >> 4;
@@ -264,8 +242,16 @@ __global__ __launch_bounds__(256) void conv1d_bc_cb_kernel(
       o[r] = s_in + r <= t_in ? (bf16_t)d0[r] : (bf16_t)0.f;
       o[4 + r] = s_in + 4 + r <= t_in ? (bf16_t)d1[r] : (bf16_t)0.f;
     }
-    *(bf16x8*)(cb + ((((int64_t)b * G + g) * nchunks + c) * CB_FRAGS + f) * 512 + lane * 8) = o;
+    *(bf16x8*)((bf16_t*)a.cb + ((((int64_t)b * a.G + g) * a.nchunks + c) * CB_FRAGS + f) * 512 + lane * 8) = o;
   }
+}
+// Both parts in one launch: first the blocks of B / C, whose chain is the longer one, then the strips of x
+template <int K>
+__global__ __launch_bounds__(CONV_THREADS) void conv1d_xbc_cb_kernel(ConvArgs a) {
+  __shared__ __attribute__((aligned(16))) bf16_t tile[2][CBQ * CBN];
+  const int i = blockIdx.x;
+  if (i < a.nbc) conv_bc_cb_block<K>(a, tile, i % a.nchunks, i / a.nchunks, blockIdx.y);
+  else conv_xbc_block<bf16_t, K>(a, i - a.nbc, blockIdx.y, a.d_inner);
 }
 
 template <typename T, int K>
@@ -290,45 +276,33 @@ __global__ void conv1d_update_kernel(const T* __restrict__ x, T* __restrict__ st
   y[(int64_t)b * C + c] = from_f32<T>(acc);
 }
 
-template <typename T>
-int launch_conv(const void* x, const void* w, const void* bias, const void* halo, void* y,
-                int B, int L, int C, int K, int64_t xsb, int64_t xsl, int64_t ysb, int64_t ysl,
-                int silu, hipStream_t s) {
+enum { CONV_PLAIN, CONV_XBC, CONV_XBC_CB };
+template <typename T, int K>
+int launch_conv_k(int form, ConvArgs a, int B, hipStream_t s) {
   constexpr int V = Vec16<T>::N;
-  dim3 grid((C / V + CONV_THREADS - 1) / CONV_THREADS, (L + CONV_TL - 1) / CONV_TL, B);
-#define TV_CONV_CASE(KK)                                                                   \
-  case KK:                                                                                 \
-    conv1d_fwd_kernel<T, KK><<<grid, CONV_THREADS, 0, s>>>((const T*)x, (const T*)w,       \
-        (const T*)bias, (const T*)halo, (T*)y, L, C, xsb, xsl, ysb, ysl, silu);            \
-    break;
-  switch (K) {
-    TV_CONV_CASE(2)
-    TV_CONV_CASE(3)
-    TV_CONV_CASE(4)
-  }
-#undef TV_CONV_CASE
+  const int c_end = form == CONV_XBC_CB ? a.d_inner : a.C;
+  a.nxb = (c_end / V + CONV_THREADS - 1) / CONV_THREADS;
+  a.wide = !((uintptr_t)a.w & 15) && !((uintptr_t)a.bias & 15);
+  a.per_xcd = ((a.L + CONV_TL - 1) / CONV_TL + 7) / 8;
+  a.nchunks = (a.L + CBQ - 1) / CBQ;
+  a.nbc = form == CONV_XBC_CB ? a.nchunks * a.G : 0;
+  const dim3 grid(a.nbc + 8 * a.nxb * a.per_xcd, B);
+  if (form == CONV_PLAIN) conv1d_fwd_kernel<T, K><<<grid, CONV_THREADS, 0, s>>>(a);
+  else if (form == CONV_XBC) conv1d_xbc_kernel<T, K><<<grid, CONV_THREADS, 0, s>>>(a);
+  else if constexpr (std::is_same<T, bf16_t>::value) conv1d_xbc_cb_kernel<K><<<grid, CONV_THREADS, 0, s>>>(a);
   TV_LAUNCH_CHECK();
 }
-
 template <typename T>
-int launch_conv_xbc(const void* x, const void* w, const void* bias, const void* halo, XbcOut o,
-                    int B, int L, int C, int K, int64_t xsb, int64_t xsl, int silu, hipStream_t s,
-                    int c_end = -1) {
-  constexpr int V = Vec16<T>::N;
-  if (c_end < 0) c_end = C;
-  dim3 grid((c_end / V + CONV_THREADS - 1) / CONV_THREADS, (L + CONV_TL - 1) / CONV_TL, B);
-#define TV_CONVX_CASE(KK)                                                                  \
-  case KK:                                                                                 \
-    conv1d_xbc_kernel<T, KK><<<grid, CONV_THREADS, 0, s>>>((const T*)x, (const T*)w,       \
-        (const T*)bias, (const T*)halo, o, L, C, c_end, xsb, xsl, silu);                   \
-    break;
-  switch (K) {
-    TV_CONVX_CASE(2)
-    TV_CONVX_CASE(3)
-    TV_CONVX_CASE(4)
+int launch_conv(int form, const ConvArgs& a, int B, int K, hipStream_t s) {
+  return K == 2 ? launch_conv_k<T, 2>(form, a, B, s) : K == 3 ? launch_conv_k<T, 3>(form, a, B, s) : launch_conv_k<T, 4>(form, a, B, s);
+}
+int launch_conv_dtype(int form, int dtype, const ConvArgs& a, int B, int K, hipStream_t s, const char* who) {
+  switch (dtype) {
+    case TV_F32: return launch_conv<float>(form, a, B, K, s);
+    case TV_BF16: return launch_conv<bf16_t>(form, a, B, K, s);
+    case TV_F16: return launch_conv<f16_t>(form, a, B, K, s);
   }
-#undef TV_CONVX_CASE
-  TV_LAUNCH_CHECK();
+  TV_UNSUPPORTED("%s: dtype %d", who, dtype);
 }
 
 template <typename T>
@@ -365,18 +339,11 @@ extern "C" int tv_causal_conv1d_fwd(const void* x, const void* weight, const voi
   if (channels % vec || x_stride_l % vec || y_stride_l % vec || x_stride_b % vec ||
       y_stride_b % vec || ((uintptr_t)x & 15) || ((uintptr_t)y & 15))
     TV_UNSUPPORTED("conv1d: channels/strides/pointers must be 16-byte aligned");
-  switch (dtype) {
-    case TV_F32:
-      return launch_conv<float>(x, weight, bias, halo, y, batch, seqlen, channels, kernel,
-                                x_stride_b, x_stride_l, y_stride_b, y_stride_l, silu, s);
-    case TV_BF16:
-      return launch_conv<bf16_t>(x, weight, bias, halo, y, batch, seqlen, channels, kernel,
-                                 x_stride_b, x_stride_l, y_stride_b, y_stride_l, silu, s);
-    case TV_F16:
-      return launch_conv<f16_t>(x, weight, bias, halo, y, batch, seqlen, channels, kernel,
-                                x_stride_b, x_stride_l, y_stride_b, y_stride_l, silu, s);
-  }
-  TV_UNSUPPORTED("conv1d: dtype %d", dtype);
+  ConvArgs a{};
+  a.x = x; a.w = weight; a.bias = bias; a.halo = halo; a.yx = y;
+  a.L = seqlen; a.C = channels; a.silu = silu;
+  a.xsb = x_stride_b; a.xsl = x_stride_l; a.ysb = y_stride_b; a.ysl = y_stride_l;
+  return launch_conv_dtype(CONV_PLAIN, dtype, a, batch, kernel, s, "conv1d");
 }
 
 static int conv1d_xbc_impl(const void* x, const void* weight, const void* bias,
@@ -394,45 +361,18 @@ static int conv1d_xbc_impl(const void* x, const void* weight, const void* bias,
   if (d_inner % vec || dstate % vec || x_stride_l % vec || x_stride_b % vec ||
       ((uintptr_t)x & 15) || ((uintptr_t)y_x & 15) || ((uintptr_t)y_b & 15) || ((uintptr_t)y_c & 15))
     TV_UNSUPPORTED("%s: segments/strides/pointers must be 16-byte aligned", who);
-  XbcOut o;
-  o.yx = y_x; o.yb = y_b; o.yc = y_c; o.d_inner = d_inner; o.G = ngroups; o.N = dstate;
+  ConvArgs a{};
+  a.x = x; a.w = weight; a.bias = bias; a.halo = halo; a.yx = y_x; a.yb = y_b; a.yc = y_c; a.cb = cb;
+  a.L = seqlen; a.C = C; a.d_inner = d_inner; a.G = ngroups; a.N = dstate; a.silu = silu;
+  a.xsb = x_stride_b; a.xsl = x_stride_l;
   hipStream_t s = (hipStream_t)stream;
   if (cb) {
-    // the scan's C.B^T fragments ride along: x channels in the streaming kernel, the B / C channels of every
-    // (chunk, group) in conv1d_bc_cb_kernel, which multiplies the two tiles while they are in LDS
+    // the scan's C.B^T fragments ride along: the B / C channels of every (chunk, group) are multiplied while they are in LDS
     if (dtype != TV_BF16 || dstate != CBN || ((uintptr_t)cb & 15))
       TV_UNSUPPORTED("%s: the C.B^T output needs bf16 and d_state %d (got dtype %d, N %d)", who, CBN, dtype, dstate);
-    const int rc = launch_conv_xbc<bf16_t>(x, weight, bias, halo, o, batch, seqlen, C, kernel, x_stride_b,
-                                           x_stride_l, silu, s, d_inner);
-    if (rc != TV_OK) return rc;
-    const int nchunks = (seqlen + CBQ - 1) / CBQ;
-    const dim3 grid(nchunks, ngroups, batch);
-#define TV_CONVCB_CASE(KK)                                                                                  \
-  case KK:                                                                                                  \
-    conv1d_bc_cb_kernel<KK><<<grid, 256, 0, s>>>((const bf16_t*)x, (const bf16_t*)weight,                   \
-        (const bf16_t*)bias, (const bf16_t*)halo, (bf16_t*)y_b, (bf16_t*)y_c, (bf16_t*)cb, seqlen, C,       \
-        d_inner, ngroups, nchunks, x_stride_b, x_stride_l, silu);                                           \
-    break;
-    switch (kernel) {
-      TV_CONVCB_CASE(2)
-      TV_CONVCB_CASE(3)
-      TV_CONVCB_CASE(4)
-    }
-#undef TV_CONVCB_CASE
-    TV_LAUNCH_CHECK();
+    return launch_conv<bf16_t>(CONV_XBC_CB, a, batch, kernel, s);
   }
-  switch (dtype) {
-    case TV_F32:
-      return launch_conv_xbc<float>(x, weight, bias, halo, o, batch, seqlen, C, kernel, x_stride_b,
-                                    x_stride_l, silu, s);
-    case TV_BF16:
-      return launch_conv_xbc<bf16_t>(x, weight, bias, halo, o, batch, seqlen, C, kernel, x_stride_b,
-                                     x_stride_l, silu, s);
-    case TV_F16:
-      return launch_conv_xbc<f16_t>(x, weight, bias, halo, o, batch, seqlen, C, kernel, x_stride_b,
-                                    x_stride_l, silu, s);
-  }
-  TV_UNSUPPORTED("%s: dtype %d", who, dtype);
+  return launch_conv_dtype(CONV_XBC, dtype, a, batch, kernel, s, who);
 }
 
 extern "C" int tv_causal_conv1d_xbc_fwd(const void* x, const void* weight, const void* bias,
