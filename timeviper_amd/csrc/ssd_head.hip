@@ -1248,6 +1248,7 @@ int cu_count() {
 // segments would make it.  128 heads x 80, 8 groups, whole operator, one segment | best number of segments | slices: 203 tokens 35 | 51 |
 // 17 us, 512: 56 | 59 | 29, 1 501: 146 | 89 | 83 - 93, 2 048: 180 | 98 | 107, 3 000: 244 | 113 | 128.
 bool use_cols(int batch, int nheads, int headdim, int ngroups, int nchunks) {
+  if (ngroups < 1 || nchunks < 1) return false;
   const int slices = nheads / ngroups * (headdim / 16);        // of a group
   return nchunks <= 24 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= cu_count();
 }
@@ -1264,7 +1265,7 @@ HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngrou
   l.cols = use_cols(batch, nheads, headdim, ngroups, (int)nchunks);
   l.nseg = l.cols ? 1 : pick_segments(batch, nheads, (int)nchunks);
   l.seg_chunks = (int)((nchunks + l.nseg - 1) / l.nseg);
-  l.nseg = (int)((nchunks + l.seg_chunks - 1) / l.seg_chunks);         // no segment is empty (the march reads its first chunk)
+  if (l.seg_chunks > 0) l.nseg = (int)((nchunks + l.seg_chunks - 1) / l.seg_chunks);      // no segment is empty (the march reads its first chunk)
   l.cb = 0;
   l.seg_state = up((size_t)batch * ngroups * nchunks * CBE * sizeof(bf16_t));
   const size_t st = (size_t)batch * nheads * headdim * HN * sizeof(float);
