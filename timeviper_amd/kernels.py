@@ -624,7 +624,7 @@ def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=Non
         if (cst.dtype != x.dtype or cw.dtype != x.dtype or not cst.is_contiguous() or not cw.is_contiguous()
                 or cst.shape != (M, nch, 4) or cw.shape != (nch, 4) or (cb is not None and (cb.dtype != x.dtype or not cb.is_contiguous()))):
             raise TimeViperHipError("gemv_fused: conv needs a contiguous (rows, C, 4) state and (C, 4) weight of x's dtype")
-    if rows_take(x2, weight) and M * K * 2 <= 128 * 1024:
+    if M <= 4 and rows_take(x2, weight) and M * K * 2 <= 128 * 1024:
         # several rows: the operator in front as its own launch and the product on the matrix cores (22 656 x 4 480, four rows: 42.8 us with
         # the prologue in the matrix-vector kernel, 30.5 + 5); same rounding points
         f = _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd=K)
