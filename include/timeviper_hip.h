@@ -605,6 +605,14 @@ int tv_gemm_rows_pair_fwd(const void* x, const void* x2, const void* W, const vo
                           int ff, int K, int64_t x_stride, int64_t x2_stride, int64_t ldw, int64_t y_stride,
                           int64_t act_stride, void* stream);
 
+/* Products of a short prompt's rows (csrc/gemm_mid.hip): y = x W^T + bias for 1..TV_GEMM_MID_MAX bf16 rows, K % 64 == 0, N % 4 == 0,
+ * bias bf16 or NULL, fp32 sums, one rounding; epilogue 0 or TV_GEMM_ROWS_RELU2.  workspace: partial sums where K is split
+ * (tv_gemm_mid_workspace_bytes, 0 where it is not), 16-byte aligned, not shared by launches that may run at once. */
+#define TV_GEMM_MID_MAX 256
+size_t tv_gemm_mid_workspace_bytes(int M, int N, int K);
+int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
+                    int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Linear attention with one constant decay per head, ragged batches:
  *   S_t = decay[h] S_(t-1) + k_t v_t^T,  o_t = S_t^T q_t

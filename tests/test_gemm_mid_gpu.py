@@ -1,0 +1,65 @@
+"""Products of a short prompt's rows (csrc/gemm_mid.hip) against float64, at the edges of its tiles and splits, and the layers that take them."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+# rows: edges of the 32-row tiles and of the three layouts of waves; N: below a tile, ragged, with and without a split of K;
+# K: fewer stages than the rings have, odd counts of them
+@pytest.mark.parametrize("M", [2, 31, 33, 64, 65, 97, 128, 129, 203, 256])
+@pytest.mark.parametrize("N,K", [(4, 64), (100, 192), (1000, 1152), (4480, 4544), (8196, 320), (24580, 128)])
+@pytest.mark.parametrize("relu2,bias", [(False, False), (True, True)])
+def test_products(M, N, K, relu2, bias):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M * 31 + N + K)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x = r(M, K + 24).to(BF)[:, 8:8 + K]                        # a slice: rows of another stride
+    w = (r(N, K + 8) * K ** -0.5).to(BF)[:, :K]
+    b = r(N).to(BF) if bias else None
+    got = ops.mid_linear(x, w, b, relu2).double()
+    s = x.double() @ w.double().T + (0 if b is None else b.double())
+    # fp32 sums of K products (relative 2^-24 each, of the sum of magnitudes), one rounding to bf16 (8 significant bits: 2^-8; squared: twice that and one more)
+    acc = (x.double().abs() @ w.double().abs().T + (0 if b is None else b.double().abs())) * K * 2.0 ** -24
+    e = acc * (1 + 2.0 ** -8) + s.abs() * 2.0 ** -8
+    if relu2:
+        want = F.relu(s) ** 2
+        bound = 2 * F.relu(s) * e + e * e + (want + e) * 2.0 ** -8 + 1e-30
+    else:
+        want, bound = s, e + 1e-30
+    assert ((got - want).abs() <= bound).all()
+    assert torch.equal(got, ops.mid_linear(x, w, b, relu2).double())      # the splits add in one order
+
+
+@pytest.mark.parametrize("tokens", [2, 17, 48, 200, 256, 257])
+def test_layers_take_them(tokens, monkeypatch):
+    """The hybrid stack's projections: the short-prompt products within a rounding of torch.nn.Linear; hooks and gradients keep the module."""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    torch.manual_seed(tokens)
+    lin = torch.nn.Linear(4096, 2048, bias=True, device=DEV, dtype=BF).requires_grad_(False)
+    x = torch.randn(1, tokens, 4096, device=DEV, dtype=BF)
+    calls = []
+    for name in ("mid_linear", "rows_linear"):
+        real = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, _r=real, _n=name, **k: (calls.append(_n), _r(*a, **k))[1])
+    want = F.linear(x.double(), lin.weight.double(), lin.bias.double())
+    for relu2 in (False, True):
+        calls.clear()
+        with torch.no_grad():
+            got = nano._prompt_linear(lin, x, relu2)
+        assert calls == (["rows_linear"] if tokens <= 32 else ["mid_linear"] if tokens <= 256 else [])
+        ref = F.relu(want) ** 2 if relu2 else want
+        # 2^-8 a rounding of bf16: one, or a squared one (twice) and another; 5 % for the fp32 sums
+        assert (got.double() - ref).abs().max() <= 1.05 * (3 if relu2 else 1) * 2.0 ** -8 * ref.abs().max()
+    calls.clear()
+    nano._prompt_linear(lin, x)                                # gradients enabled
+    seen = []
+    handle = lin.register_forward_hook(lambda *a: seen.append(1))
+    with torch.no_grad():
+        nano._prompt_linear(lin, x)
+    handle.remove()
+    assert not calls and seen

@@ -1,0 +1,372 @@
+// Products of a short prompt's rows with a weight matrix, y[m][n] = sum_k x[m][k] W[n][k], m <= 256: each weight byte is read once, for all
+// rows, so that W from HBM is the floor (N K 2 bytes); at 256 rows the products are as long (1.3 PFLOP/s).
+//
+//   * A work-group owns 64, 96 or 128 rows of W and all rows of x; narrow outputs split K over work-groups as well, partial sums in fp32 to
+//     a workspace and a second launch that adds them in order (the library runs 4 480 outputs on 35 - 70 of 256 compute units).
+//   * Both operands arrive by LDS-DMA, a stage of 64 columns at a time.  Waves 0 - 3 copy x, waves 4 - 7 copy W: vmcnt counts in order, so a
+//     wave that copied both would wait for W's latency with x.
+//   * One barrier a stage, in the middle of its products: the fragments of a 16-column step are read while the step before is multiplied
+//     (v_mfma_f32_32x32x16_bf16, W on the A side: a lane's registers are consecutive outputs of one row of x).
+//   * The waves along K meet over the rings, in an order that stores whole rows of y.
+// What bounds it: a compute unit takes in W and x together at about 45 bytes a ns — alone, x comes from L2 at 80, but loads return in order
+// and those of x queue behind W's — so the time grows with the rows: x is read again by every work-group.
+// fp32 accumulation, one rounding of y.
+// Measured (weights not in any cache; library -> here): 4 480 x 15 680, 33 | 128 | 203 | 256 rows 65 | 89 | 131 | 148 -> 31 | 44 | 52 | 52 us; 4 480 x 10 240
+// 52 | 57 | 83 | 92 -> 24 | 35 | 41 | 42; 15 680 x 4 480 with 33 | 64 rows 40 | 42 -> 28 | 32.
+#include "gemm_skinny.hpp"
+
+namespace {
+using namespace ssdk;
+
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
+constexpr int GM_KC = 64;                          // columns of a stage
+constexpr int GM_WAVES = 8;
+
+struct GmArgs {
+  const bf16_t *x, *W, *bias;
+  bf16_t* y;
+  float* part;                                     // split K: [split][M][N rounded up to tiles]
+  int M, N, K, tiles, splits, per_xcd, relu2;
+  int64_t xs, ldw, ys;
+};
+
+// four consecutive outputs n.. of row m: bias, one rounding, squared ReLU of what was rounded
+__device__ __forceinline__ void put(const GmArgs& a, int m, int n, f32x4 s) {
+  if (a.bias) {
+    const bf16x4 b = *(const bf16x4*)(a.bias + n);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] += (float)b[j];
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    o[j] = (bf16_t)s[j];
+    if (a.relu2) {
+      const float r = fmaxf((float)o[j], 0.f);
+      o[j] = (bf16_t)(r * r);
+    }
+  }
+  *(bf16x4*)(a.y + (int64_t)m * a.ys + n) = o;
+}
+
+template <int J, bool NT>
+__device__ __forceinline__ void glds_many(const void* src, const unsigned (&v)[J], unsigned dst) {
+  if constexpr (J <= 4) glds_rows<J, NT>(src, v, dst);
+  else {
+    unsigned lo[4], hi[J - 4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lo[i] = v[i];
+#pragma unroll
+    for (int i = 4; i < J; ++i) hi[i - 4] = v[i];
+    glds_rows<4, NT>(src, lo, dst);
+    glds_many<J - 4, NT>(src, hi, dst + 4096);
+  }
+}
+
+// NI: 32-row tiles of W a work-group; waves: WM along the rows of x, MI tiles of 32 each, x WK along a stage's four 16-column steps;
+// NSX, NSW: ring stages of x and of W
+template <int NI, int MI, int WM, int WK, int NSX, int NSW>
+__global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
+  static_assert(WM * WK == GM_WAVES && (WK == 2 || WK == 4), "waves");
+  constexpr int XT = MI * WM, KS = 4 / WK;
+  constexpr int XST = XT * 4096, WST = NI * 4096;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wk = wave / WM;
+  const int r = lane & 31, hh = lane >> 5;
+  // units (split, tile of N), tiles fastest: an XCD (id % 8) has a run of them, so that its work-groups share x's columns
+  const int unit = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+  if (unit >= a.tiles * a.splits) return;
+  const int split = unit / a.tiles, tile = unit - split * a.tiles;
+  const int n0 = tile * (32 * NI);
+  const int nst = a.K / GM_KC;
+  const int s0 = (int)((int64_t)nst * split / a.splits), ns = (int)((int64_t)nst * (split + 1) / a.splits) - s0;
+
+  // ---- copies: piece p (1 KiB), lane l -> LDS row 8 p + l / 8, 16-byte chunk l % 8, which holds source chunk (l % 8) ^ ((row >> 1) & 7)
+  const bool xside = wave < 4;
+  const unsigned ringx = lds_addr_of(gm_smem), ringw = ringx + (unsigned)(NSX * XST);
+  unsigned vw[NI], vx[XT];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = 8 * ((wave & 3) * NI + i) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+    vw[i] = (unsigned)(((int64_t)min(row, a.N - 1 - n0) * a.ldw + ch * 8) * 2);
+  }
+#pragma unroll
+  for (int i = 0; i < XT; ++i) {
+    const int row = 8 * ((wave & 3) * XT + i) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+    vx[i] = (unsigned)(((int64_t)min(row, a.M - 1) * a.xs + ch * 8) * 2);
+  }
+  const bf16_t* Wb = a.W + (int64_t)n0 * a.ldw + (int64_t)s0 * GM_KC;
+  const bf16_t* xb = a.x + (int64_t)s0 * GM_KC;
+  f32x16_t acc[MI][NI];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[mi][ni][j] = 0.f;
+  const bool busy = wm * MI * 32 < a.M;            // (rows past M: no products)
+  unsigned fr[KS];                                 // fragment reads: row r of a 32-row tile, 16-byte chunk 2 ks + hh
+#pragma unroll
+  for (int k = 0; k < KS; ++k) fr[k] = (unsigned)(r * 128 + (((2 * (wk * KS + k) + hh) ^ ((r >> 1) & 7)) << 4));
+  bf16x8 fx[2][MI], fw[2][NI];                     // two sets: the fragments of a step are read while the step before is multiplied
+  auto read = [&](bf16x8 (&x)[MI], bf16x8 (&w)[NI], int k, int rx, int rw) __attribute__((always_inline)) {
+    const unsigned px = ringx + (unsigned)(rx * XST) + fr[k] + (unsigned)(wm * MI * 4096), pw = ringw + (unsigned)(rw * WST) + fr[k];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) x[mi] = *(lds_bf16x8*)(size_t)(px + (unsigned)(mi * 4096));
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) w[ni] = *(lds_bf16x8*)(size_t)(pw + (unsigned)(ni * 4096));
+  };
+  auto multiply = [&](const bf16x8 (&x)[MI], const bf16x8 (&w)[NI]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ni], x[mi], acc[mi][ni], 0, 0, 0);
+  };
+  // The loop of a wave that copies x (SIDE 0) or W (SIDE 1): J copies a stage into NS slots.  At a step's meeting stage i + 1 is in LDS for
+  // all waves and every wave has read stage i, whose slot is filled again behind it.
+  auto run = [&](auto side) __attribute__((always_inline)) {
+    constexpr bool XS = decltype(side)::value == 0;
+    constexpr int NS = XS ? NSX : NSW, J = XS ? XT : NI, ST = XS ? XST : WST;
+    const unsigned base = __builtin_amdgcn_readfirstlane((XS ? ringx : ringw) + 1024u * J * (wave & 3));
+    auto issue = [&](int i, int slot) __attribute__((always_inline)) {
+      const unsigned dst = __builtin_amdgcn_readfirstlane(base + (unsigned)(slot * ST));
+      if constexpr (XS) glds_many<XT, false>(uniform_ptr(xb + (int64_t)i * GM_KC), vx, dst);
+      else glds_many<NI, true>(uniform_ptr(Wb + (int64_t)i * GM_KC), vw, dst);
+    };
+    auto meet_counted = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(J * (NS - 2)) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    auto meet_all = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    auto next = [](int v, int n) __attribute__((always_inline)) { return v == n - 1 ? 0 : v + 1; };
+    for (int j = 0; j < NS - 1 && j < ns; ++j) issue(j, j);
+    if (ns >= NS - 1) meet_counted();
+    else meet_all();
+    if (ns > NS - 1) issue(NS - 1, NS - 1);
+    int i = 0, rx = 0, rw = 0, sl = 0;             // stage being multiplied; slots of the stage being read; slot of stage i in this wave's ring
+    if (!busy) {
+      for (; i + NS < ns; ++i) {
+        meet_counted();
+        issue(i + NS, sl);
+        sl = next(sl, NS);
+      }
+      for (; i + 1 < ns; ++i) meet_all();
+      return;
+    }
+    read(fx[0], fw[0], 0, 0, 0);
+    if constexpr (KS == 2) {
+      for (; i + NS < ns; ++i) {
+        read(fx[1], fw[1], 1, rx, rw);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fx[0], fw[0]);
+        meet_counted();
+        issue(i + NS, sl);
+        sl = next(sl, NS); rx = next(rx, NSX); rw = next(rw, NSW);
+        read(fx[0], fw[0], 0, rx, rw);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fx[1], fw[1]);
+      }
+      for (; i + 1 < ns; ++i) {
+        read(fx[1], fw[1], 1, rx, rw);
+        multiply(fx[0], fw[0]);
+        meet_all();
+        rx = next(rx, NSX); rw = next(rw, NSW);
+        read(fx[0], fw[0], 0, rx, rw);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fx[1], fw[1]);
+      }
+      read(fx[1], fw[1], 1, rx, rw);
+      multiply(fx[0], fw[0]);
+      multiply(fx[1], fw[1]);
+    } else {
+      for (; i + 1 + NS < ns; i += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          meet_counted();
+          issue(i + u + NS, sl);
+          sl = next(sl, NS); rx = next(rx, NSX); rw = next(rw, NSW);
+          read(fx[1 - u], fw[1 - u], 0, rx, rw);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(fx[u], fw[u]);
+        }
+      }
+      for (; i + 1 < ns; ++i) {
+        if (i + NS < ns) {
+          meet_counted();
+          issue(i + NS, sl);
+          sl = next(sl, NS);
+        } else {
+          meet_all();
+        }
+        rx = next(rx, NSX); rw = next(rw, NSW);
+        read(fx[1], fw[1], 0, rx, rw);
+        multiply(fx[0], fw[0]);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) fx[0][mi] = fx[1][mi];
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) fw[0][ni] = fw[1][ni];
+      }
+      multiply(fx[0], fw[0]);
+    }
+  };
+  if (xside) run(std::integral_constant<int, 0>{});
+  else run(std::integral_constant<int, 1>{});
+  // ---- the waves along K meet over the rings, MI rounds: [wave][n-tile][register quad][hh][r rotated] f32x4, summed in the order of rows of y
+  f32x4* meet = (f32x4*)gm_smem;
+  constexpr int NC = 8 * NI;                       // chunks of four outputs a row
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    __syncthreads();
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        meet[((wave * NI + ni) * 8 + 2 * g + hh) * 32 + ((r + 2 * g + hh + 8 * ni) & 31)] =
+            f32x4{acc[mi][ni][4 * g], acc[mi][ni][4 * g + 1], acc[mi][ni][4 * g + 2], acc[mi][ni][4 * g + 3]};
+    __syncthreads();
+#pragma unroll
+    for (int e0 = 0; e0 < WM * 32 * NC; e0 += GM_WAVES * 64) {
+      const int e = e0 + tid, c = e % NC, row = e / NC, w = row >> 5, rr = row & 31;
+      const int m = 32 * (w * MI + mi) + rr, n = n0 + 4 * c;
+      f32x4 s = meet[(w * NC + c) * 32 + ((rr + c) & 31)];
+#pragma unroll
+      for (int k = 1; k < WK; ++k) s += meet[((k * WM + w) * NC + c) * 32 + ((rr + c) & 31)];
+      if (m >= a.M) continue;
+      if (a.part) *(f32x4*)(a.part + ((int64_t)split * a.M + m) * (a.tiles * 32 * NI) + n) = s;
+      else if (n < a.N) put(a, m, n, s);
+    }
+  }
+}
+
+// sum over the splits, in their order
+__global__ __launch_bounds__(256) void gemm_mid_sum_kernel(GmArgs a, int np) {
+  const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y;
+  if (n >= a.N) return;
+  const float* p = a.part + (int64_t)m * np + n;
+  const int64_t step = (int64_t)a.M * np;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < a.splits; c += 4) {
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(p + (int64_t)min(c + u, a.splits - 1) * step);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c + u < a.splits) s += v[u];
+  }
+  put(a, m, n, s);
+}
+
+template <int NI, int MI, int WM, int WK, int NSX, int NSW>
+int launch_one(const GmArgs& a, hipStream_t st) {
+  constexpr int RING = (NSX * MI * WM + NSW * NI) * 4096, MEET = GM_WAVES * NI * 4096;
+  constexpr int LDS = RING > MEET ? RING : MEET;
+  static_assert(LDS <= 160 * 1024, "ring");
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)gemm_mid_kernel<NI, MI, WM, WK, NSX, NSW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (attr != hipSuccess) {
+    tv_set_error("gemm_mid: cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr));
+    return TV_ERR_LAUNCH;
+  }
+  gemm_mid_kernel<NI, MI, WM, WK, NSX, NSW><<<dim3((unsigned)(8 * a.per_xcd)), GM_WAVES * 64, LDS, st>>>(a);
+  if (a.part) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      tv_set_error("gemm_mid: %s", hipGetErrorString(e));
+      return TV_ERR_LAUNCH;
+    }
+    gemm_mid_sum_kernel<<<dim3((unsigned)((a.N + 1023) / 1024), (unsigned)a.M), 256, 0, st>>>(a, a.tiles * 32 * NI);
+  }
+  TV_LAUNCH_CHECK();
+}
+
+int cu_count() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
+      cus = 256;                               // MI355X
+    return cus;
+  }();
+  return n;
+}
+
+struct GmPlan {
+  int ni, splits, xt;
+};
+// The tile width and split of K with the smallest estimate: per stage the larger of W from HBM (6.3 TB/s over all compute units) and W and x through
+// the compute unit's memory pipe (45 bytes a ns, measured: x hits the L2, but its loads queue behind those of W), per work-group 3 us of
+// fill and epilogue, per split 4 M N bytes written and read at 5 TB/s and a second launch.
+GmPlan plan(int M, int N, int K) {
+  GmPlan best{4, 1, M <= 64 ? 2 : M <= 128 ? 4 : 8};
+  const int cus = cu_count(), nst = K / GM_KC;
+  double least = 1e30;
+  for (int ni = 4; ni >= 2; --ni)
+    for (int s = 1; s <= 16 && s * 8 <= nst; ++s) {
+      const int64_t units = (int64_t)((N + 32 * ni - 1) / (32 * ni)) * s, rounds = (units + cus - 1) / cus;
+      const double hbm = ni * 4096. * cus / 6300., pipe = (ni + best.xt) * 4096. / 45.;
+      const double t = rounds * (((nst + s - 1) / s) * (hbm > pipe ? hbm : pipe) + 3000.) + (s > 1 ? 3000. + 2. * s * N * M * 4 / 5000. : 0.);
+      if (t < least) {
+        least = t;
+        best.ni = ni;
+        best.splits = s;
+      }
+    }
+  return best;
+}
+
+template <int NI>
+int launch_ni(const GmArgs& a, int xt, hipStream_t st) {
+  if (xt == 2) return launch_one<NI, 1, 2, 4, 4, 32 / NI>(a, st);
+  if (xt == 4) return launch_one<NI, 2, 2, 4, 3, 28 / NI>(a, st);
+  return launch_one<NI, 2, 4, 2, 3, 16 / NI>(a, st);
+}
+
+bool takes(const void* x, const void* W, int M, int N, int K, int64_t xs, int64_t ldw) {
+  // (copies are 16 bytes a lane at 32-bit offsets from a work-group's first row; a stage is 64 columns; four outputs a store)
+  return M >= 1 && M <= TV_GEMM_MID_MAX && N >= 4 && N % 4 == 0 && K >= GM_KC && K % GM_KC == 0 && xs % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)x & 15) == 0 &&
+         ((uintptr_t)W & 15) == 0 && xs >= 0 && ldw >= 0 && (int64_t)TV_GEMM_MID_MAX * xs * 2 < (1ll << 31) && 128 * ldw * 2 < (1ll << 31);
+}
+
+}  // namespace
+
+extern "C" size_t tv_gemm_mid_workspace_bytes(int M, int N, int K) {
+  if (M < 1 || M > TV_GEMM_MID_MAX || N < 1 || K < GM_KC) return 0;
+  const GmPlan p = plan(M, N, K);
+  return p.splits > 1 ? (size_t)p.splits * M * ((N + 32 * p.ni - 1) / (32 * p.ni)) * (128 * p.ni) : 0;
+}
+
+extern "C" int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
+                               int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(x && W && y, "gemm_mid: null pointer");
+  TV_CHECK_ARG(M >= 1 && M <= TV_GEMM_MID_MAX && N >= 1 && K >= 1, "gemm_mid: M %d must be 1..%d, N %d and K %d positive", M, TV_GEMM_MID_MAX, N, K);
+  TV_CHECK_ARG(epilogue == 0 || epilogue == TV_GEMM_ROWS_RELU2, "gemm_mid: epilogue %d", epilogue);
+  if (!takes(x, W, M, N, K, x_stride, ldw) || y_stride % 4 || ((uintptr_t)y & 7) || ((uintptr_t)bias & 7))
+    TV_UNSUPPORTED("gemm_mid: K must be a multiple of %d, N and the row stride of y of 4, those of x and W of 8, x and W 16-byte, y and bias 8-byte aligned",
+                   GM_KC);
+  const GmPlan p = plan(M, N, K);
+  const size_t need = tv_gemm_mid_workspace_bytes(M, N, K);
+  TV_CHECK_ARG(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0), "gemm_mid: workspace of %zu bytes needed", need);
+  GmArgs a{};
+  a.x = (const bf16_t*)x; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.y = (bf16_t*)y;
+  a.M = M; a.N = N; a.K = K; a.xs = x_stride; a.ldw = ldw; a.ys = y_stride; a.relu2 = epilogue == TV_GEMM_ROWS_RELU2;
+  a.tiles = (N + 32 * p.ni - 1) / (32 * p.ni);
+  a.splits = p.splits;
+  a.per_xcd = (a.tiles * a.splits + 7) / 8;
+  a.part = p.splits > 1 ? (float*)workspace : nullptr;
+  hipStream_t st = (hipStream_t)stream;
+  switch (p.ni) {
+    case 2: return launch_ni<2>(a, p.xt, st);
+    case 3: return launch_ni<3>(a, p.xt, st);
+    default: return launch_ni<4>(a, p.xt, st);
+  }
+}

@@ -707,6 +707,43 @@ def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None):
     return y
 
 
+MID_MAX = 256
+
+
+def mid_takes(x, weight, relu2=False) -> bool:
+    """Products of up to 256 rows that tv_gemm_mid_fwd runs faster than the library: a long contraction into fewer outputs (4 480 x 15 680, 203
+    rows: 131 us in the library, 52 here), any of at most 64 rows (15 680 x 4 480, 64 rows: 42, 32), and the squared ReLU of up to 256 (its own pass
+    saved; without it 128 rows 42 and 44, 203: 50 and 51).  Shorter contractions and a thousand outputs are the library's (6 144 x 2 048, 128 rows: 12
+    and 20 us; 1 024 x 4 480, 256: 14.5 and 16)."""
+    N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
+    n = x.numel() // max(x.shape[-1], 1)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and 2 <= n <= MID_MAX and Kd >= 4096
+            and Kd % 64 == 0 and N % 4 == 0 and (n <= 64 or relu2 or 2048 <= N < Kd) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
+            and weight.stride(0) < (1 << 22) and weight.data_ptr() % 16 == 0)
+
+
+def mid_linear(x, weight, bias=None, relu2=False):
+    """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) for up to 256 bf16 rows (a short prompt)."""
+    _gpu(x, weight, bias)
+    N, Kd = weight.shape
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[-1] != Kd:
+        raise TimeViperHipError(f"mid_linear: bf16 rows of {Kd} elements, got {tuple(x.shape)} {x.dtype} against {weight.dtype}")
+    if bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous() or bias.numel() != N):
+        raise TimeViperHipError("mid_linear: bias must be contiguous, of x's dtype")
+    x2 = _rows2d(x)
+    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) >= (1 << 22) or x2.data_ptr() % 16:
+        x2 = x2.contiguous()
+    if bias is not None and bias.data_ptr() % 8:
+        bias = bias.clone()
+    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    lib, M = _capi.lib(), x2.shape[0]
+    need = int(lib.tv_gemm_mid_workspace_bytes(M, N, Kd))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib.tv_gemm_mid_fwd(_p(x2), _p(weight), _p(bias), _p(y), M, N, Kd, x2.stride(0), weight.stride(0), N, 1 if relu2 else 0, _p(ws), need, _stream()),
+          "tv_gemm_mid_fwd")
+    return y
+
+
 def _decode_attn_takes(q, k, v) -> bool:
     """Shapes tv_attn_decode_fwd is written for (the rest stays on tv_flash_attn_fwd with one query row)."""
     return (q.dtype == torch.bfloat16 and q.shape[-1] == 128 and k.shape[1] >= 256

@@ -309,7 +309,21 @@ def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
         return K.gemv_fused(x, mod.weight, mod.bias)
     if _rows_decode(x) and K.rows_take(x, mod.weight):
         return K.rows_linear(x, mod.weight, mod.bias)
-    return mod(x)
+    return _prompt_linear(mod, x)
+
+
+def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torch.Tensor:
+    """mod(x), or its squared ReLU.  A short prompt's rows (2..256) run on tv_gemm_rows_fwd / tv_gemm_mid_fwd where those are faster than the
+    library; what a caller may have put around the module (hooks, a subclass, autocast) sees it called as ever."""
+    if (x.is_cuda and x.dim() == 3 and x.shape[0] * x.shape[1] <= K.MID_MAX and x.shape[1] > 1 and not torch.is_grad_enabled()
+            and type(mod) is nn.Linear and not mod._forward_hooks and not mod._forward_pre_hooks and not torch.is_autocast_enabled()
+            and (mod.bias is None or (mod.bias.dtype == x.dtype and mod.bias.is_contiguous()))):
+        if K.rows_take(x, mod.weight):
+            return K.rows_linear(x, mod.weight, mod.bias, relu2=relu2)
+        if K.mid_takes(x, mod.weight, relu2):
+            return K.mid_linear(x, mod.weight, mod.bias, relu2)
+    y = mod(x)
+    return K.relu2(y, inplace=True) if relu2 else y
 
 
 def _norm_add(norm, hidden, delta):
@@ -399,7 +413,7 @@ class NemotronHMamba2Mixer(nn.Module):
         batch_size, seq_len, _ = hidden_states.shape
         if attention_mask is not None and attention_mask.shape[1] > 1 and attention_mask.shape[0] > 1:
             hidden_states = (hidden_states * attention_mask[:, :, None]).to(hidden_states.dtype)
-        projected_states = self.in_proj(hidden_states)
+        projected_states = _prompt_linear(self.in_proj, hidden_states)
         gts = self.n_groups * self.ssm_state_size
         d_in = self.intermediate_size
         decode = (cache_params is not None and cache_position is not None
@@ -443,7 +457,7 @@ class NemotronHMamba2Mixer(nn.Module):
         if cache_params is not None:
             cache_params.update_ssm_state(self.layer_idx, ssm_state)
         scan_output = self.norm(scan_output.view(batch_size, seq_len, -1), gate)
-        out = self.out_proj(scan_output)
+        out = _prompt_linear(self.out_proj, scan_output)
         if return_shard_state:
             return out, ssm_state, res[2]
         return out
@@ -506,7 +520,7 @@ class NemotronHMLP(nn.Module):
 
     def forward(self, x):
         # `act_fn` stays for the module tree; the activation runs as one in-place HIP pass
-        return self.down_proj(K.relu2(self.up_proj(x), inplace=True))
+        return _prompt_linear(self.down_proj, _prompt_linear(self.up_proj, x, relu2=True))
 
     def decode_fused(self, hidden, delta, norm):
         """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches (more than four sequences: 3,
