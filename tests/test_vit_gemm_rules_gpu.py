@@ -1,0 +1,58 @@
+"""The hand-written ViT products below a few tiles per compute unit, where the dispatch now takes the persistent kernels, against float64;
+and the blocks' choice between them and the library."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+# fewer tiles than work-groups (and than XCDs), one ragged row or column of tiles, one and two rounds of either tile shape
+@pytest.mark.parametrize("M,N,K", [(256, 256, 256), (257, 264, 1152), (729, 1152, 1152), (2916, 3456, 1152), (7290, 1152, 1152), (10935, 1152, 1152),
+                                   (13122, 1152, 1152), (700, 1152, 4352)])
+@pytest.mark.parametrize("epilogue", ["bias", "gelu", "accumulate"])
+def test_few_tiles(M, N, K, epilogue):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, w, b = r(M, K).to(BF), (r(N, K) * K ** -0.5).to(BF), r(N).to(BF)
+    s = x.double() @ w.double().T
+    mag = x.double().abs() @ w.double().abs().T * (K * 2.0 ** -24)             # fp32 sums of K products
+    if epilogue == "accumulate":
+        c = r(M, N).to(BF)
+        want = s + c.double()
+        got = ops.linear_fused(x, w, None, epilogue=ops.GEMM_ACCUM, out=c.clone())
+        bound = mag + want.abs() * 2.0 ** -8                                   # one rounding to bf16
+    else:
+        z = s + b.double()
+        got = ops.linear_fused(x, w, b, epilogue=ops.GEMM_BIAS_GELU if epilogue == "gelu" else ops.GEMM_BIAS)
+        if epilogue == "gelu":                                                 # of the rounded sum (slope below 1.13), rounded again
+            want, bound = F.gelu(z), 1.13 * (mag + z.abs() * 2.0 ** -8) + F.gelu(z).abs() * 2.0 ** -8 + 2.0 ** -20
+        else:
+            want, bound = z, mag + z.abs() * 2.0 ** -8
+    assert ((got.double() - want).abs() <= bound * 1.01 + 1e-30).all()
+
+
+@pytest.mark.parametrize("frames,own", [(1, ()), (4, ("gelu",)), (10, ("qkv", "gelu", "accumulate")), (18, ("qkv", "gelu"))])
+def test_blocks_choose(frames, own, monkeypatch):
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.vit.siglip import Block
+    torch.manual_seed(frames)
+    blk = Block(1152, 16, 4304).to(DEV, BF).eval().requires_grad_(False)
+    x = torch.randn(frames, 729, 1152, device=DEV).to(BF)
+    names = {ops.GEMM_BIAS: "qkv", ops.GEMM_BIAS_GELU: "gelu", ops.GEMM_ACCUM: "accumulate"}
+    calls, real = [], ops.linear_fused
+    monkeypatch.setattr(ops, "linear_fused", lambda *a, **k: (calls.append(names[k["epilogue"]]), real(*a, **k))[1])
+    with torch.no_grad():
+        y, pend = blk.forward_stream(x.clone(), None)
+        got = y.float() + pend
+        blk.float()
+        z = x.float()
+        n, t, c = z.shape
+        q, k, v = blk.attn.qkv(blk.norm1(z)).view(n, t, 3, 16, c // 16).permute(2, 0, 3, 1, 4)
+        z = z + blk.attn.proj(((q @ k.transpose(-1, -2)) * blk.attn.scale).softmax(-1).matmul(v).transpose(1, 2).reshape(n, t, c))
+        ref = z + blk.mlp.fc2(F.gelu(blk.mlp.fc1(blk.norm2(z))))
+    assert sorted(set(calls)) == sorted(own)
+    assert ((got - ref).norm() / ref.norm()) < 1e-2

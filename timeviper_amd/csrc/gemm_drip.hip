@@ -581,7 +581,14 @@ bool drip_takes(const GemmArgs& a, int epilogue, int grid) {
   if (epilogue != EPI_ACCUM && (a.bias == nullptr || !a.bias_f32)) return false;
   if (256 * a.ldc * 2 >= (1ll << 31)) return false;
   const int64_t tiles = (int64_t)a.tiles_m * ((a.N + DBN - 1) / DBN);
-  if (g_drip_mode < 0 && tiles < 4ll * grid) return false;
+  if (g_drip_mode < 0 && tiles < 4ll * grid) {
+    // A few rounds of tiles: accumulating, by the rounds that each tile shape takes; a round of these is 0.77 of one of gemm.hip's 256 x 256
+    // (N 1 152, K 1 152: 27 and 35 us; K 4 352: 80 and 100).  7 290 rows, one round each: 28 | 33 us; 10 935 rows, two and one: 52 | 36;
+    // 26 244, three each: 83 | 95; 33 534, four and three: 109 | 107.
+    if (epilogue != EPI_ACCUM) return false;
+    const int64_t rounds = (tiles + grid - 1) / grid, theirs = ((int64_t)a.tiles_m * a.tiles_n + grid - 1) / grid;
+    return 10 * rounds <= 13 * theirs;
+  }
   return true;
 }
 

@@ -63,6 +63,14 @@ class PatchEmbed(nn.Module):
 GEMM_ALIGN = 256     # hipBLASLt's bf16 macro-tile on gfx950
 
 
+CUS = 256            # compute units of an MI355X: work-groups of one round
+
+
+def _tiles(rows: int, n: int, width: int = 256) -> int:
+    """256-row output tiles of a (rows, n) product"""
+    return -(-rows // 256) * -(-n // width)
+
+
 def _aligned(n: int) -> int:
     return -(-n // GEMM_ALIGN) * GEMM_ALIGN
 
@@ -135,16 +143,15 @@ class Attention(nn.Module):
         return o.reshape(B, N, C)
 
     def _own_qkv(self, x) -> bool:
-        """qkv projection + bias on the hand-written persistent GEMM instead of hipBLASLt — opt-in (TV_VIT_OWN_QKV=1).
-        Stand-alone on 2 048 SigLIP frames it wins (9.5 ms against 10.2 ms for the library on the weights as stored and
-        9.7 ms on the copies zero-padded to 3 584 columns, same box); inside the 10 240-frame forward the library on the
-        padded copies is 0.5 % of the step ahead (1 225.6 against 1 219.9 frames/s, same box, round 5), so that stays
-        the default.  bf16 on the GPU, inference, K a multiple of 128, N of 8, enough rows for every compute unit to
-        walk a few tiles."""
-        w = self.qkv.weight
-        return (os.environ.get("TV_VIT_OWN_QKV", "0") == "1" and x.is_cuda and x.dtype == torch.bfloat16
-                and w.dtype == torch.bfloat16 and self.qkv.bias is not None and not torch.is_grad_enabled()
-                and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and x.numel() // x.shape[-1] >= 65536)
+        """qkv projection + bias on the hand-written persistent GEMM instead of hipBLASLt: where its 256 x 256 tiles are two to eight
+        rounds of the compute units (library on the padded copy | persistent, us, SigLIP so400m: 9 frames 68 | 58, 16: 107 | 96, 24: 142 | 128, 33: 213 |
+        181, 41: 208 | 214, 48: 254 | 246; one round: 5 frames 31 | 33; more than eight: 64 frames 326 | 333, and 0.5 % of a 10 240-frame
+        forward), or everywhere with TV_VIT_OWN_QKV=1.  bf16 on the GPU, inference, K a multiple of 128, N of 8."""
+        w, rows = self.qkv.weight, x.numel() // x.shape[-1]
+        rounds = -(-_tiles(rows, w.shape[0]) // CUS)
+        own = rows >= 65536 if os.environ.get("TV_VIT_OWN_QKV", "0") == "1" else 2 <= rounds <= 8
+        return (own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
+                and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0)
 
     def forward(self, x):
         return self.proj(self.heads(x))
@@ -180,27 +187,38 @@ class Mlp(nn.Module):
     def _fused_fc1(self, x, w1) -> bool:
         """fc1 + bias + exact GELU in ONE kernel (csrc/gemm_persist.hip from 4 tiles per compute unit on, csrc/gemm.hip
         below: the activation is applied to the accumulators, same rounding points as GEMM-then-GELU): 14.0 ms
-        (persistent) / 14.8 ms (per tile) against 16.7 ms for hipBLASLt + tv_gelu_fwd per 2 048 SigLIP frames.  bf16 on the GPU, inference, K a multiple of 128, enough rows to fill the chip; TV_VIT_FUSED_FC1=0
-        switches it off."""
+        (persistent) / 14.8 ms (per tile) against 16.7 ms for hipBLASLt + tv_gelu_fwd per 2 048 SigLIP frames.  bf16 on the GPU, inference, K
+        a multiple of 128, tiles for three quarters of the compute units (4 frames, 204 tiles: library + GELU 42 us, fused 41; 3 frames, 153:
+        34 and 39); TV_VIT_FUSED_FC1=0 switches it off."""
         return (self.exact_gelu and x.is_cuda and x.dtype == torch.bfloat16 and w1.dtype == torch.bfloat16
                 and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0
-                and x.numel() // x.shape[-1] >= 4096 and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
+                and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
 
     def forward(self, x):
         h, w2 = self.hidden(x)
         return F.linear(h, w2, self.fc2.bias)
 
 
+def _own_accumulate(rows: int, n: int) -> bool:
+    """Whether the hand-written accumulating GEMM is the faster one: its tiles (256 x 192 or 256 x 256, csrc/gemm_drip.hip) fill their rounds of
+    the compute units to 63 % or more, up to 131 072 rows.  us, library | own, SigLIP so400m, proj (K 1 152): 9 frames 26 | 27 (61 %), 10: 34 | 28
+    (68 %), 16: 50 | 37, 18: 46 | 53 (61 %), 26: 93 | 58, 33: 96 | 79, 48: 156 | 111, 128: 335 | 273; fc2 (K 4 352): 10: 79 | 75, 16: 112 | 101, 18: 127 |
+    153, 26: 228 | 169, 33: 220 | 212, 45: 301 | 320, 48: 404 | 323, 128: 847 | 836, 256: 1 599 | 1 663."""
+    if rows > 131072:
+        return False
+    fill = max(t / (-(-t // CUS) * CUS) for t in (_tiles(rows, n), _tiles(rows, n, 192)))
+    return fill >= 0.63
+
+
 def _accumulate(x2: torch.Tensor, h2: torch.Tensor, w: torch.Tensor, role: str) -> None:
-    """x2 += h2 @ w.T (one rounding of the sum to bf16), the residual stream's output projections.  Default: hipBLASLt
-    (`torch.addmm`, beta = 1).  The hand-written GEMM with the accumulating epilogue (csrc/gemm_drip.hip: 256 x 192 tiles —
-    1 152 columns are 6 of them, 4.5 of the library's 256-wide ones) takes the roles named in TV_VIT_OWN_ACCUM (comma
-    separated: proj, fc2) when the shape allows: bf16, K a multiple of 128 and >= 1 152, enough rows for every compute
-    unit to walk a few tiles."""
-    own = _OWN_ACCUM
-    if (role in own and x2.is_cuda and x2.dtype == torch.bfloat16 and h2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[1] >= 1152 and w.shape[0] % 8 == 0
-            and x2.shape[0] >= 65536 and h2.stride(1) == 1 and w.stride(1) == 1):
+    """x2 += h2 @ w.T (one rounding of the sum to bf16), the residual stream's output projections: the hand-written GEMM with the
+    accumulating epilogue where it is the faster one (`_own_accumulate`; more than 65 536 rows also for the roles named in
+    TV_VIT_OWN_ACCUM, comma separated: proj, fc2) and the shape allows (bf16, K a multiple of 128 and >= 1 152), else hipBLASLt
+    (`torch.addmm`, beta = 1)."""
+    rows, n = x2.shape
+    if ((_own_accumulate(rows, n) or (role in _OWN_ACCUM and rows >= 65536)) and x2.is_cuda and x2.dtype == torch.bfloat16
+            and h2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0
+            and w.shape[1] >= 1152 and n % 8 == 0 and h2.stride(1) == 1 and w.stride(1) == 1):
         K.linear_fused(h2, w, None, epilogue=K.GEMM_ACCUM, out=x2)
     else:
         torch.addmm(x2, h2, w.t(), out=x2)
