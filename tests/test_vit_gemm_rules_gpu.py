@@ -12,7 +12,7 @@ BF = torch.bfloat16
 # fewer tiles than work-groups (and than XCDs), one ragged row or column of tiles, one and two rounds of either tile shape
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (257, 264, 1152), (729, 1152, 1152), (2916, 3456, 1152), (7290, 1152, 1152), (10935, 1152, 1152),
                                    (13122, 1152, 1152), (700, 1152, 4352)])
-@pytest.mark.parametrize("epilogue", ["bias", "gelu", "accumulate"])
+@pytest.mark.parametrize("epilogue", ["bias", "gelu", "relu2", "accumulate"])
 def test_few_tiles(M, N, K, epilogue):
     from timeviper_amd import kernels as ops
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
@@ -27,9 +27,13 @@ def test_few_tiles(M, N, K, epilogue):
         bound = mag + want.abs() * 2.0 ** -8                                   # one rounding to bf16
     else:
         z = s + b.double()
-        got = ops.linear_fused(x, w, b, epilogue=ops.GEMM_BIAS_GELU if epilogue == "gelu" else ops.GEMM_BIAS)
+        got = ops.linear_fused(x, w, b, epilogue={"bias": ops.GEMM_BIAS, "gelu": ops.GEMM_BIAS_GELU, "relu2": ops.GEMM_BIAS_RELU2}[epilogue])
         if epilogue == "gelu":                                                 # of the rounded sum (slope below 1.13), rounded again
             want, bound = F.gelu(z), 1.13 * (mag + z.abs() * 2.0 ** -8) + F.gelu(z).abs() * 2.0 ** -8 + 2.0 ** -20
+        elif epilogue == "relu2":                                              # of the rounded sum, rounded again
+            e = mag + z.abs() * 2.0 ** -8
+            want = F.relu(z) ** 2
+            bound = 2 * F.relu(z) * e + e * e + (want + e) * 2.0 ** -8
         else:
             want, bound = z, mag + z.abs() * 2.0 ** -8
     assert ((got.double() - want).abs() <= bound * 1.01 + 1e-30).all()
@@ -56,3 +60,27 @@ def test_blocks_choose(frames, own, monkeypatch):
         ref = z + blk.mlp.fc2(F.gelu(blk.mlp.fc1(blk.norm2(z))))
     assert sorted(set(calls)) == sorted(own)
     assert ((got - ref).norm() / ref.norm()) < 1e-2
+
+
+@pytest.mark.parametrize("rows,N,K,relu2,own", [(1500, 22656, 4480, False, True), (300, 22656, 4480, False, False), (6011, 4480, 10240, False, True),
+                                                (8000, 4480, 10240, False, False), (2048, 15680, 4480, True, True), (2048, 15680, 4480, False, False)])
+def test_long_prompts(rows, N, K, relu2, own, monkeypatch):
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    torch.manual_seed(rows)
+    with torch.device("meta"):
+        lin = torch.nn.Linear(K, N, bias=False, dtype=BF)
+    lin = lin.to_empty(device=DEV).requires_grad_(False)
+    lin.weight.normal_(0, K ** -0.5)
+    x = torch.randn(1, rows, K, device=DEV).to(BF)
+    calls, real = [], ops.linear_fused
+    monkeypatch.setattr(ops, "linear_fused", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        got = nano._prompt_linear(lin, x, relu2)
+        sel = slice(rows - 300, rows)                          # (the last, ragged tile among them)
+        ref = x[0, sel].double() @ lin.weight.double().T
+    if relu2:
+        ref = F.relu(ref) ** 2
+    assert bool(calls) == own
+    # 2^-8 a rounding of bf16: one, or a squared one (twice) and another; 5 % for the fp32 sums
+    assert (got[0, sel].double() - ref).abs().max() <= 1.05 * (3 if relu2 else 1) * 2.0 ** -8 * ref.abs().max()

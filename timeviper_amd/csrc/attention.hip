@@ -172,9 +172,9 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     const int pairs = a.nb * a.Hq;
     int pair;
     block_of(blockIdx.x, pairs, qblk, pair);
-    if (a.causal) qblk = (int)gridDim.x / pairs - 1 - qblk;
-    h = pair % a.Hq;
-    b = pair / a.Hq;
+    if (a.causal) qblk = (a.Lq + QB - 1) / QB - 1 - qblk;
+    b = a.nb == 1 ? 0 : pair / a.Hq;           // (a division is 30 instructions of a short call)
+    h = pair - b * a.Hq;
   }
   const int hk = h / (a.Hq / a.Hkv);
   const int q0 = qblk * QB + wave * FA_QW;      // first query row of this wave

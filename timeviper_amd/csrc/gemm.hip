@@ -397,7 +397,7 @@ extern "C" int tv_gemm_bf16_fwd(const void* A, const void* W, const void* bias, 
   TV_CHECK_ARG(M >= 0 && N > 0 && K > 0, "gemm: bad sizes (M %lld N %d K %d)", (long long)M, N, K);
   if (M == 0) return TV_OK;
   TV_CHECK_ARG(A && W && C, "gemm: null pointer");
-  TV_CHECK_ARG(epilogue >= 0 && epilogue <= 2, "gemm: epilogue %d", epilogue);
+  TV_CHECK_ARG(epilogue >= 0 && epilogue <= 3, "gemm: epilogue %d", epilogue);
   TV_CHECK_ARG(bias == nullptr || bias_dtype == TV_F32 || bias_dtype == TV_BF16, "gemm: bias dtype %d", bias_dtype);
   if (K % (2 * BK) || N % 4 || lda % 8 || ldw % 8 || ldc % 4 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) || ((uintptr_t)C & 7) ||
       ((uintptr_t)bias & 15))
@@ -421,6 +421,10 @@ extern "C" int tv_gemm_bf16_fwd(const void* A, const void* W, const void* bias, 
   hipStream_t st = (hipStream_t)stream;
   // whole tiles: persistent work-groups — 256 x 192 tiles that leave during the next tile's K loop (gemm_drip.hip),
   // else 256 x 256 tiles with the epilogue by quadrants inside the main loop (gemm_persist.hip)
+  if (epilogue == 3) {
+    if (!persist_takes(a, EPI_BIAS_RELU2)) TV_UNSUPPORTED("gemm: the squared ReLU takes M and N of at least 256, N %% 8 == 0 (M %lld N %d)", (long long)M, N);
+    return launch_persist(a, EPI_BIAS_RELU2, st);
+  }
   if (drip_takes(a, epilogue, persist_grid())) return launch_drip(a, epilogue, persist_grid(), st);
   if (persist_takes(a, epilogue)) return launch_persist(a, epilogue, st);
   switch (epilogue) {

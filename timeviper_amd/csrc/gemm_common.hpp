@@ -9,7 +9,7 @@
 namespace tvgemm {
 using namespace ssdk;
 
-enum { EPI_BIAS = 0, EPI_BIAS_GELU = 1, EPI_ACCUM = 2, EPI_RELU2 = 3 };
+enum { EPI_BIAS = 0, EPI_BIAS_GELU = 1, EPI_ACCUM = 2, EPI_RELU2 = 3, EPI_BIAS_RELU2 = 4 };      // EPI_RELU2: of the fp32 sum (moe); EPI_BIAS_RELU2: of the rounded one
 
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int HALF_BYTES = 128 * BK * 2;          // one half-tile: 128 rows x 128 bytes

@@ -1,6 +1,6 @@
 // Persistent bf16 GEMM for the ViT linears (timm block via base_vision.py:146-170,274-278, InternVideo2
 // Attention / Mlp vit_scale_clean.py:188-320):  C[M][N] = epilogue( A[M][K] . W[N][K]^T ) for the bias epilogues of gemm.hip
-// (EPI_BIAS: the qkv projection; EPI_BIAS_GELU: fc1 + exact GELU).
+// (EPI_BIAS: the qkv projection; EPI_BIAS_GELU: fc1 + exact GELU; EPI_BIAS_RELU2: the hybrid stack's up projection + squared ReLU).
 //
 // Why a second kernel.  The linears of a SigLIP block have K = 1 152: 18 K-tiles of 64.  With one work-group per output
 // tile every tile pays, outside its K loop, the pipeline fill, the conversion of 256 x 256 accumulators (with the
@@ -205,6 +205,13 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
         if (EPI == EPI_BIAS_GELU) {
 #pragma unroll
           for (int r = 0; r < 8; ++r) v[r] = gelu_erf_f((float)(bf16_t)v[r]);       // the GEMM's own bf16 rounding first
+        }
+        if (EPI == EPI_BIAS_RELU2) {
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {
+            const float p = fmaxf((float)(bf16_t)v[r], 0.f);
+            v[r] = p * p;
+          }
         }
         u32x4e o;
 #pragma unroll
@@ -429,6 +436,7 @@ int launch_persist(const GemmArgs& a, int epilogue, hipStream_t st) {
   const int grid = grid_size();
   switch (epilogue) {
     case EPI_BIAS: return launch<EPI_BIAS>(pa, grid, st);
+    case EPI_BIAS_RELU2: return launch<EPI_BIAS_RELU2>(pa, grid, st);
     default: return launch<EPI_BIAS_GELU>(pa, grid, st);
   }
 }

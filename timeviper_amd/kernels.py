@@ -257,13 +257,13 @@ def rmsnorm_fn(x, weight, bias=None, z=None, eps=1e-6, group_size=None,
 
 
 # ------------------------------------------------------------------- linears with fused epilogues
-GEMM_BIAS, GEMM_BIAS_GELU, GEMM_ACCUM = 0, 1, 2
+GEMM_BIAS, GEMM_BIAS_GELU, GEMM_ACCUM, GEMM_BIAS_RELU2 = 0, 1, 2, 3
 
 
 def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
     """F.linear(x, weight, bias) on the hand-written bf16 GEMM (csrc/gemm.hip) with the epilogue fused:
-    GEMM_BIAS (plain), GEMM_BIAS_GELU (exact GELU of the bf16-rounded result: the timm Mlp's fc1 + act) or
-    GEMM_ACCUM (out += x @ weight.T, `out` required, bias ignored).  x (..., K) bf16 with dense rows,
+    GEMM_BIAS (plain), GEMM_BIAS_GELU (exact GELU of the bf16-rounded result: the timm Mlp's fc1 + act), GEMM_BIAS_RELU2 (its squared
+    ReLU; at least 256 rows and columns) or GEMM_ACCUM (out += x @ weight.T, `out` required, bias ignored).  x (..., K) bf16 with dense rows,
     weight (N, K) bf16; K % 128 == 0, N % 4 == 0."""
     _gpu(x, weight, bias, out)
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
@@ -718,6 +718,26 @@ def mid_takes(x, weight, relu2=False) -> bool:
     return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and 2 <= n <= MID_MAX and Kd >= 4096
             and Kd % 64 == 0 and N % 4 == 0 and (n <= 64 or relu2 or 2048 <= N < Kd) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
             and weight.stride(0) < (1 << 22) and weight.data_ptr() % 16 == 0)
+
+
+def large_takes(x, weight, relu2=False) -> bool:
+    """Products of a long prompt that the persistent GEMM (tv_gemm_bf16_fwd) runs faster than the library: its 256 x 256 tiles are two
+    rounds of the compute units or more and fill them, and the output is wide (22 656 x 4 480, us, library | here: 1 500 rows, 70 % full, 355 | 275; 2 048: 445 |
+    319, 4 096: 726 | 617, 10 007: 1 494 | 1 464), the contraction long (4 480 x 10 240: 6 011 rows 481 | 408, 10 007: 937 | 718; 75 % full, 8 000 rows: 579 |
+    591; one round, 3 000: 191 | 195) or the squared ReLU saves its own pass (15 680 x 4 480, 2 048 rows 198 + 24 | 207, 10 007: 974 + 102 | 1 028).  The rest
+    stays the library's (15 680 x 4 480 alone; 12 288 x 4 096, 8 000 rows: 553 | 595)."""
+    N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
+    rows = x.numel() // max(x.shape[-1], 1)
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and rows > MID_MAX and Kd >= 4096
+            and Kd % 128 == 0 and N % 8 == 0 and N >= 256 and x.is_contiguous() and weight.is_contiguous()
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        return False
+    cus = 256                                                  # of an MI355X
+    tiles = -(-rows // 256) * -(-N // 256)
+    fill = tiles / (-(-tiles // cus) * cus)
+    if tiles <= cus:
+        return False
+    return fill >= 0.75 and Kd <= 8192 if relu2 else fill >= (0.69 if N >= 20480 else 0.8) and (N >= 20480 or Kd >= 8192)
 
 
 def mid_linear(x, weight, bias=None, relu2=False):

@@ -313,15 +313,17 @@ def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
 
 
 def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torch.Tensor:
-    """mod(x), or its squared ReLU.  A short prompt's rows (2..256) run on tv_gemm_rows_fwd / tv_gemm_mid_fwd where those are faster than the
-    library; what a caller may have put around the module (hooks, a subclass, autocast) sees it called as ever."""
-    if (x.is_cuda and x.dim() == 3 and x.shape[0] * x.shape[1] <= K.MID_MAX and x.shape[1] > 1 and not torch.is_grad_enabled()
-            and type(mod) is nn.Linear and not mod._forward_hooks and not mod._forward_pre_hooks and not torch.is_autocast_enabled()
-            and (mod.bias is None or (mod.bias.dtype == x.dtype and mod.bias.is_contiguous()))):
+    """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256) or tv_gemm_bf16_fwd where those
+    are faster than the library; what a caller may have put around the module (hooks, a subclass, autocast) sees it called as ever."""
+    if (x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and type(mod) is nn.Linear and not mod._forward_hooks
+            and not mod._forward_pre_hooks and not torch.is_autocast_enabled()
+            and (mod.bias is None or (mod.bias.dtype == x.dtype and mod.bias.is_contiguous() and mod.bias.data_ptr() % 16 == 0))):
         if K.rows_take(x, mod.weight):
             return K.rows_linear(x, mod.weight, mod.bias, relu2=relu2)
         if K.mid_takes(x, mod.weight, relu2):
             return K.mid_linear(x, mod.weight, mod.bias, relu2)
+        if K.large_takes(x, mod.weight, relu2):
+            return K.linear_fused(x, mod.weight, mod.bias, epilogue=K.GEMM_BIAS_RELU2 if relu2 else K.GEMM_BIAS)
     y = mod(x)
     return K.relu2(y, inplace=True) if relu2 else y
 

@@ -143,13 +143,13 @@ class Attention(nn.Module):
         return o.reshape(B, N, C)
 
     def _own_qkv(self, x) -> bool:
-        """qkv projection + bias on the hand-written persistent GEMM instead of hipBLASLt: where its 256 x 256 tiles are two to eight
+        """qkv projection + bias on the hand-written persistent GEMM instead of hipBLASLt: where its 256 x 256 tiles are two to six
         rounds of the compute units (library on the padded copy | persistent, us, SigLIP so400m: 9 frames 68 | 58, 16: 107 | 96, 24: 142 | 128, 33: 213 |
-        181, 41: 208 | 214, 48: 254 | 246; one round: 5 frames 31 | 33; more than eight: 64 frames 326 | 333, and 0.5 % of a 10 240-frame
+        181; one round: 5 frames 31 | 33; more than six: 41 frames 208 | 214, 48: 254 | 246, 64: 326 | 333, and 0.5 % of a 10 240-frame
         forward), or everywhere with TV_VIT_OWN_QKV=1.  bf16 on the GPU, inference, K a multiple of 128, N of 8."""
         w, rows = self.qkv.weight, x.numel() // x.shape[-1]
         rounds = -(-_tiles(rows, w.shape[0]) // CUS)
-        own = rows >= 65536 if os.environ.get("TV_VIT_OWN_QKV", "0") == "1" else 2 <= rounds <= 8
+        own = rows >= 65536 if os.environ.get("TV_VIT_OWN_QKV", "0") == "1" else 2 <= rounds <= 6
         return (own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
                 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0)
 
