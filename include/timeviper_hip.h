@@ -614,6 +614,18 @@ size_t tv_gemm_mid_workspace_bytes(int M, int N, int K);
 int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
                     int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Between the layers of a decoded token and the next one (csrc/decode_glue.hip).
+ * tv_kv_append: k / v, one row of row_bytes per sequence, to position *pos (device) of the caches; all strides in bytes, everything a
+ *   multiple of 16; a position outside [0, capacity) writes nothing.
+ * tv_count_up: pos[0] += 1, lens[0..n) += 1.
+ * tv_argmax_rows: out[r] = position of the largest of n fp32 values (NaN above all, the lowest of equals: torch.argmax). */
+int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* pos, int batch, int64_t capacity,
+                 int row_bytes, int64_t k_stride_b, int64_t v_stride_b, int64_t kc_stride_b, int64_t kc_stride_l, int64_t vc_stride_b,
+                 int64_t vc_stride_l, void* stream);
+int tv_count_up(int64_t* pos, int* lens, int n, void* stream);
+size_t tv_argmax_rows_workspace_bytes(int rows);
+int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int64_t stride, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Linear attention with one constant decay per head, ragged batches:
  *   S_t = decay[h] S_(t-1) + k_t v_t^T,  o_t = S_t^T q_t

@@ -87,6 +87,10 @@ SIGNATURES = {
     "tv_gemm_rows_pair_fwd": (_i, [_p] * 6 + [_i] * 4 + [_l] * 5 + [_p]),
     "tv_gemm_mid_workspace_bytes": (_z, [_i] * 3),
     "tv_gemm_mid_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l] * 3 + [_i, _p, _z, _p]),
+    "tv_kv_append": (_i, [_p] * 5 + [_i, _l, _i] + [_l] * 6 + [_p]),
+    "tv_count_up": (_i, [_p, _p, _i, _p]),
+    "tv_argmax_rows_workspace_bytes": (_z, [_i]),
+    "tv_argmax_rows": (_i, [_p, _p, _i, _i, _l, _p, _z, _p]),
     "tv_lightning_workspace_bytes": (_z, [_i] * 6),
     "tv_lightning_fwd": (_i, [_p] * 8 + [_i, _i, _p, _z] + [_i] * 3 + [_l] * 4 + [_i, _i, _p]),
     "tv_attn_generic_fwd": (_i, [_p] * 8 + [_i, _l] + [_i] * 4 + [_l] * 10 + [_f] + [_i] * 3 + [_p, _l, _l, _i, _p]),

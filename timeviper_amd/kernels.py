@@ -762,6 +762,47 @@ def mid_linear(x, weight, bias=None, relu2=False):
     return y
 
 
+def kv_append(k, v, k_cache, v_cache, pos) -> None:
+    """k_cache[:, pos] = k[:, 0], v_cache[:, pos] = v[:, 0] for (B, 1, H, D) keys and values and an int64 position on the device (both
+    caches' `index_copy_` in one launch)."""
+    B, one, H, D = k.shape
+    size = k.element_size()
+    ok = (k.is_cuda and one == 1 and k.dtype == v.dtype == k_cache.dtype == v_cache.dtype and k.shape == v.shape and k_cache.shape == v_cache.shape
+          and k_cache.shape[0] == B and k_cache.shape[2:] == k.shape[2:] and (H * D * size) % 16 == 0 and pos.dtype == torch.int64 and pos.numel() == 1
+          and all([t.stride(3) == 1 and t.stride(2) == D and not (t.data_ptr() | t.stride(0) * size | t.stride(1) * size) % 16
+                   for t in (k, v, k_cache, v_cache)]))
+    if not ok:
+        k_cache.index_copy_(1, pos, k)
+        v_cache.index_copy_(1, pos, v)
+        return
+    _gpu(k, v, k_cache, v_cache, pos)
+    st = lambda t, d: t.stride(d) * size
+    check(_capi.lib().tv_kv_append(_p(k), _p(v), _p(k_cache), _p(v_cache), _p(pos), B, k_cache.shape[1], H * D * size, st(k, 0), st(v, 0), st(k_cache, 0),
+                                   st(k_cache, 1), st(v_cache, 0), st(v_cache, 1), _stream()), "tv_kv_append")
+
+
+def count_up(pos, lens) -> None:
+    """pos += 1 (int64, one entry), lens += 1 (int32), in one launch on the GPU"""
+    if not (pos.is_cuda and lens.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1 and lens.dtype == torch.int32 and lens.is_contiguous()):
+        pos += 1
+        lens += 1
+        return
+    _gpu(pos, lens)
+    check(_capi.lib().tv_count_up(_p(pos), _p(lens), lens.numel(), _stream()), "tv_count_up")
+
+
+def argmax_rows(x):
+    """x.argmax(-1); the fp32 logits of up to 65 535 rows by 64 work-groups a row."""
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] < (1 << 31)):
+        return x.argmax(-1)
+    _gpu(x)
+    lib, B = _capi.lib(), x.shape[0]
+    out = torch.empty((B,), dtype=torch.int64, device=x.device)
+    ws = torch.empty((int(lib.tv_argmax_rows_workspace_bytes(B)),), dtype=torch.uint8, device=x.device)
+    check(lib.tv_argmax_rows(_p(x), _p(out), B, x.shape[1], x.stride(0), _p(ws), ws.numel(), _stream()), "tv_argmax_rows")
+    return out
+
+
 def _decode_attn_takes(q, k, v) -> bool:
     """Shapes tv_attn_decode_fwd is written for (the rest stays on tv_flash_attn_fwd with one query row)."""
     return (q.dtype == torch.bfloat16 and q.shape[-1] == 128 and k.shape[1] >= 256

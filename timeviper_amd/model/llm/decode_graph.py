@@ -23,6 +23,8 @@ import warnings
 
 import torch
 
+from ... import kernels as K
+
 __all__ = ["GraphedDecodeStep"]
 
 
@@ -50,7 +52,7 @@ class GraphedDecodeStep:
     def _run(self):
         logits = self.step_fn(self.ids)
         logits = logits[:, -1] if logits.dim() == 3 else logits
-        nxt = logits.argmax(-1)
+        nxt = K.argmax_rows(logits)
         self.cache.advance_static_device()
         return logits, nxt
 

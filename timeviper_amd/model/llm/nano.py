@@ -211,8 +211,7 @@ class HybridMambaAttentionDynamicCache(StaticDecode):
             if new != 1:
                 raise RuntimeError("static decode takes one token per step")
             pos = self._static_of[layer_idx][0]
-            kb.index_copy_(1, pos, key_states)
-            vb.index_copy_(1, pos, value_states)
+            K.kv_append(key_states, value_states, kb, vb, pos)
         else:
             kb[:, have:have + new], vb[:, have:have + new] = key_states, value_states
         self._kv_len[layer_idx] = have + new
@@ -251,8 +250,7 @@ class HybridMambaAttentionDynamicCache(StaticDecode):
     def advance_static_device(self):
         """Device side of one finished step (part of the captured graph)."""
         for pos, lens in self._static.values():
-            pos += 1
-            lens += 1
+            K.count_up(pos, lens)
 
     def decode_lens(self, layer_idx):
         return self._static_of[layer_idx][1]
