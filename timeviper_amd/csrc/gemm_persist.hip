@@ -47,8 +47,9 @@ enum { KT_FIRST = 0, KT_MID = 1, KT_LAST = 2 };
 struct PArgs {
   GemmArgs g;
   int ntiles;
-  int dbg;       // dev switches (TV_GEMM_DBG): 1 = no epilogue, 2 = epilogue arithmetic without stores
+  int dbg;       // dev switches (TV_GEMM_DBG): 1 = no epilogue, 2 = epilogue arithmetic without stores; PF_RELU2: squared ReLU of the rounded sum
 };
+constexpr int PF_RELU2 = 4;
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4e __attribute__((ext_vector_type(4)));
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
 #pragma unroll
           for (int r = 0; r < 8; ++r) v[r] = gelu_erf_f((float)(bf16_t)v[r]);       // the GEMM's own bf16 rounding first
         }
-        if (EPI == EPI_BIAS_RELU2) {
+        if (EPI == EPI_BIAS && (pa.dbg & PF_RELU2)) {
 #pragma unroll
           for (int r = 0; r < 8; ++r) {
             const float p = fmaxf((float)(bf16_t)v[r], 0.f);
@@ -432,11 +433,13 @@ int launch_persist(const GemmArgs& a, int epilogue, hipStream_t st) {
   pa.g = a;
   pa.ntiles = a.tiles_m * a.tiles_n;
   static const int dbg_env = [] { const char* e = getenv("TV_GEMM_DBG"); return e ? atoi(e) : 0; }();
-  pa.dbg = dbg_env;
+  pa.dbg = dbg_env & 3;
   const int grid = grid_size();
   switch (epilogue) {
     case EPI_BIAS: return launch<EPI_BIAS>(pa, grid, st);
-    case EPI_BIAS_RELU2: return launch<EPI_BIAS_RELU2>(pa, grid, st);
+    case EPI_BIAS_RELU2:                         // a uniform branch of the plain kernel, not a third copy of it
+      pa.dbg |= PF_RELU2;
+      return launch<EPI_BIAS>(pa, grid, st);
     default: return launch<EPI_BIAS_GELU>(pa, grid, st);
   }
 }
