@@ -12,6 +12,9 @@
 //       work-group folds its own predecessors — at most 63 states of P x N floats from L2 — so no chain of launches or
 //       work-groups exists);  y_t += exp(cs_t) C_t . S_in(c)   (Y_off);  the last chunk writes the final state and the
 //       total decay.
+// Bound by latency and LDS reads (0.3 MB of data): all of a work-group's rows are loaded at once, operands that are the same for all lanes
+// come four at a time, M and Y_off's sums keep 16 tokens a lane in registers, and LDS and registers are small enough for all 1 024
+// work-groups of 1 024 tokens x 32 heads to run at once.  There, launch 1 33.6 -> 24.0 us and launch 2 24.6 -> 15.1.
 // fp32 arithmetic throughout (every exponent is <= 0: decays only), y in the caller's dtype (a bf16 / f16 y is rounded once
 // per launch: the generic path's tolerance).  Takes d_state <= 64, head_dim <= 128, 2 .. 64 chunks; everything else stays on
 // the token recurrence.
@@ -58,90 +61,119 @@ __device__ __forceinline__ void chunk_decays(const ChArgs& a, int b, int h, int 
   }
 }
 
+// LDS of the local kernel: x, then B | C and, once these are used up, M transposed in their place: four work-groups fit a compute unit, so
+// that 1 024 of them (1 024 tokens, 32 heads) run at once
+constexpr int MTS = 68;         // row stride of M^T (four tokens of one source token in one read)
+__host__ __device__ __forceinline__ int local_region(int N) {
+  const int NC = (N + 3) & ~3, bc = CQ * (N | 1) + CQ * NC + 4;
+  return bc > CQ * MTS ? bc : CQ * MTS;
+}
+
 template <typename T>
 __global__ __launch_bounds__(CH_THREADS) void ssd_chunk_local_kernel(ChArgs a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  const int N = a.N, P = a.P, PP = (P + 3) & ~3, NS = N | 1;      // (odd row stride of B / C: a wave reads 64 rows at one n)
+  const int N = a.N, P = a.P, PP = (P + 3) & ~3, NS = N | 1, NC = (N + 3) & ~3;      // (odd row stride of B: a wave reads 64 rows at one n)
   float* sX = smem;                    // [64][PP]
   float* sB = sX + CQ * PP;            // [64][NS]
-  float* sC = sB + CQ * NS;            // [64][NS]
-  float* sM = sC + CQ * NS;            // [64][65]
-  float* sD = sM + CQ * 65;            // [64]
+  float* sC = sB + ((CQ * NS + 3) & ~3);      // [64][NC]
+  float* sM = sB;                      // [64 s][MTS]: M[t][s] at s MTS + t, over B and C
+  float* sD = sB + local_region(N);    // [64]
   float* sCs = sD + CQ;                // [64]
   float* sW = sCs + CQ;                // [64]: exp(cs_end - cs_s) dt_s
   // two work-groups per chunk: the even one computes M and Y_diag, the odd one the chunk's state (both need x and B; the
-  // problem is too small to fill the chip otherwise: 512 work-groups of ~10 us each)
+  // problem is too small to fill the chip otherwise)
   const int c = blockIdx.x >> 1, part = blockIdx.x & 1, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
   const int t0 = c * CQ, tt = min(CQ, a.L - t0);
   const int g = a.group_map ? (h % a.G) : (h / (a.H / a.G));
   const T* xb = (const T*)a.x + (int64_t)b * a.xsb + (int64_t)h * P;
   const T* Bb = (const T*)a.Bm + (int64_t)b * a.bsb + (int64_t)g * a.bsg;
   const T* Cb = (const T*)a.Cm + (int64_t)b * a.csb + (int64_t)g * a.csg;
-  chunk_decays<T>(a, b, h, t0, tt, sD, sCs);
-  // Staging.  Wave w takes the rows w, w + 4, ..., lane = column; eight rows' loads are issued before the first LDS store
+  // Staging.  Wave w takes the rows w, w + 4, ..., lane = column; all loads of the 16 rows are issued before the first LDS store
   // (clamped addresses + a select instead of a branch around the load, no integer division by run-time sizes: written as
   // one element per loop pass, hipcc waited for every load before issuing the next — 20 round trips a work-group)
   {
     const int w = tid >> 6, lane = tid & 63;
-    const int nc = min(lane, N - 1);
-    for (int kb = 0; kb < CQ / 4; kb += 8) {
-      float bv[8], cv[8];
+    const int nc = min(lane, N - 1), px = min(lane, P - 1);
+    float bv[CQ / 4], cv[CQ / 4], xv[CQ / 4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int tc = min(w + 4 * (kb + k), tt - 1);
-        bv[k] = to_f32(Bb[(int64_t)(t0 + tc) * a.bsl + nc]);
-        cv[k] = to_f32(Cb[(int64_t)(t0 + tc) * a.csl + nc]);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int t = w + 4 * (kb + k);
-        if (lane < N) {
-          sB[t * NS + lane] = t < tt ? bv[k] : 0.f;
-          sC[t * NS + lane] = t < tt ? cv[k] : 0.f;
-        }
-      }
+    for (int k = 0; k < CQ / 4; ++k) {
+      const int64_t t = t0 + min(w + 4 * k, tt - 1);
+      bv[k] = to_f32(Bb[t * a.bsl + nc]);
+      cv[k] = part == 0 ? to_f32(Cb[t * a.csl + nc]) : 0.f;
+      xv[k] = to_f32(xb[t * a.xsl + px]);
     }
-    for (int p0 = 0; p0 < PP; p0 += 64) {
+    chunk_decays<T>(a, b, h, t0, tt, sD, sCs);
+#pragma unroll
+    for (int k = 0; k < CQ / 4; ++k) {
+      const int t = w + 4 * k;
+      if (lane < N) {
+        sB[t * NS + lane] = t < tt ? bv[k] : 0.f;
+        sC[t * NC + lane] = t < tt ? cv[k] : 0.f;
+      } else if (lane < NC) {
+        sC[t * NC + lane] = 0.f;
+      }
+      if (lane < PP) sX[t * PP + lane] = (t < tt && lane < P) ? xv[k] : 0.f;
+    }
+    for (int p0 = 64; p0 < PP; p0 += 64) {
       const int p = p0 + lane, pc = min(p, P - 1);
-      for (int kb = 0; kb < CQ / 4; kb += 8) {
-        float xv[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) xv[k] = to_f32(xb[(int64_t)(t0 + min(w + 4 * (kb + k), tt - 1)) * a.xsl + pc]);
+      for (int k = 0; k < CQ / 4; ++k) xv[k] = to_f32(xb[(int64_t)(t0 + min(w + 4 * k, tt - 1)) * a.xsl + pc]);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int t = w + 4 * (kb + k);
-          if (p < PP) sX[t * PP + p] = (t < tt && p < P) ? xv[k] : 0.f;
-        }
+      for (int k = 0; k < CQ / 4; ++k) {
+        const int t = w + 4 * k;
+        if (p < PP) sX[t * PP + p] = (t < tt && p < P) ? xv[k] : 0.f;
       }
     }
   }
   __syncthreads();
   if (part == 1) {
-    // the chunk's state from a zero start, and its decay
+    // the chunk's state from a zero start, and its decay: four columns of x and one n a thread
     if (tid < CQ) sW[tid] = __expf(sCs[CQ - 1] - sCs[tid]) * sD[tid];
     __syncthreads();
     const float cend = sCs[CQ - 1];                        // (tokens past the end add 0: cs stays at the last real value)
     float* So = ws_state(a, b, h, c);
-    for (int idx = tid; idx < P * N; idx += CH_THREADS) {
-      const int p = idx / N, n = idx - p * N;
-      float acc = 0.f;
+    const int tiles = (PP >> 2) * N;
+    for (int tile = tid; tile < tiles; tile += CH_THREADS) {
+      const int pq = tile / N, n = tile - pq * N;
+      float acc[4] = {};
 #pragma unroll 8
-      for (int s = 0; s < tt; ++s) acc = fmaf(sW[s] * sX[s * PP + p], sB[s * NS + n], acc);
-      So[idx] = acc;
+      for (int s = 0; s < CQ; ++s) {                       // (rows past the end: w 0, x 0, B 0)
+        const f32x4 xq = *(const f32x4*)(sX + s * PP + 4 * pq);
+        const float wv = sW[s], bn = sB[s * NS + n];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = fmaf(wv * xq[j], bn, acc[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * pq + j < P) So[(4 * pq + j) * N + n] = acc[j];
     }
     if (tid == 0) ws_decay(a, b, h)[c] = cend;
     return;
   }
-  // M[t][s]: causal, decayed, dt-weighted C.B^T of the chunk
-  for (int i = tid; i < CQ * CQ; i += CH_THREADS) {
-    const int t = i >> 6, s = i & 63;
-    float v = 0.f;
-    if (s <= t) {
-      float dot = 0.f;
-      for (int n = 0; n < N; ++n) dot = fmaf(sC[t * NS + n], sB[s * NS + n], dot);
-      v = __expf(sCs[t] - sCs[s]) * sD[s] * dot;
+  // M[t][s]: causal, decayed, dt-weighted C.B^T of the chunk.  Lane = s, wave w: t = w, w + 4, ...; B by lane, C the same for all lanes
+  {
+    const int w = tid >> 6, sl = tid & 63;
+    float acc[CQ / 4] = {};
+    for (int n = 0; n < N; n += 4) {
+      float bn[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bn[j] = n + j < N ? sB[sl * NS + n + j] : 0.f;
+#pragma unroll
+      for (int k = 0; k < CQ / 4; ++k) {
+        const f32x4 cq = *(const f32x4*)(sC + (w + 4 * k) * NC + n);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[k] = fmaf(cq[j], bn[j], acc[k]);
+      }
     }
-    sM[t * 65 + s] = v;
+    const float cs = sCs[sl], ds = sD[sl];
+#pragma unroll
+    for (int k = 0; k < CQ / 4; ++k) {
+      const int t = w + 4 * k;
+      acc[k] = sl <= t ? __expf(sCs[t] - cs) * ds * acc[k] : 0.f;
+    }
+    __syncthreads();                                       // (B and C are used up)
+#pragma unroll
+    for (int k = 0; k < CQ / 4; ++k) sM[sl * MTS + w + 4 * k] = acc[k];
   }
   __syncthreads();
   // Y_diag: 4 x 4 (token, column) tiles
@@ -153,15 +185,13 @@ __global__ __launch_bounds__(CH_THREADS) void ssd_chunk_local_kernel(ChArgs a) {
       const int tq = tile / ptiles, pq = tile - tq * ptiles;
       const int tb = 4 * tq, pb = 4 * pq;
       float acc[4][4] = {};
-      const int send = min(tb + 3, tt - 1);
-      for (int s = 0; s <= send; ++s) {
-        const f32x4 xv = *(const f32x4*)(sX + s * PP + pb);
+#pragma unroll 4
+      for (int s = 0; s < tb + 4; ++s) {                   // (rows past the end are zeros)
+        const f32x4 xv = *(const f32x4*)(sX + s * PP + pb), m = *(const f32x4*)(sM + s * MTS + tb);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float m = sM[(tb + i) * 65 + s];
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(m, xv[j], acc[i][j]);
-        }
+          for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(m[i], xv[j], acc[i][j]);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -178,12 +208,13 @@ __global__ __launch_bounds__(CH_THREADS) void ssd_chunk_local_kernel(ChArgs a) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(CH_THREADS) void ssd_chunk_carry_kernel(ChArgs a) {
+__global__ __launch_bounds__(CH_THREADS, 4) void ssd_chunk_carry_kernel(ChArgs a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int N = a.N, P = a.P;
   float* sS = smem;                    // [P][N + 1]
-  float* sC = sS + P * (N + 1);        // [64][N]
-  float* sD = sC + CQ * N;             // [64]
+  const int NC = (N + 3) & ~3;
+  float* sC = sS + ((P * (N + 1) + 3) & ~3);      // [64][NC]
+  float* sD = sC + CQ * NC;            // [64]
   float* sCs = sD + CQ;                // [64]
   float* sE = sCs + CQ;                // [CH_MAXCHUNKS]: exp(decay of chunk j)
   // two work-groups per chunk, each with half of the head's columns [p_lo, p_hi)
@@ -195,19 +226,17 @@ __global__ __launch_bounds__(CH_THREADS) void ssd_chunk_carry_kernel(ChArgs a) {
   const float* dec = ws_decay(a, b, h);
   const bool last = c == a.nch - 1;
   if (c == 0 && !a.init && !last) return;                 // nothing enters the first chunk
-  chunk_decays<T>(a, b, h, t0, tt, sD, sCs);
   {
     const int w = tid >> 6, lane = tid & 63;
     const int nc = min(lane, N - 1);
-    for (int kb = 0; kb < CQ / 4; kb += 8) {
-      float cv[8];
+    float cv[CQ / 4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) cv[k] = to_f32(Cb[(int64_t)(t0 + min(w + 4 * (kb + k), tt - 1)) * a.csl + nc]);
+    for (int k = 0; k < CQ / 4; ++k) cv[k] = to_f32(Cb[(int64_t)(t0 + min(w + 4 * k, tt - 1)) * a.csl + nc]);
+    chunk_decays<T>(a, b, h, t0, tt, sD, sCs);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int t = w + 4 * (kb + k);
-        if (lane < N) sC[t * N + lane] = t < tt ? cv[k] : 0.f;
-      }
+    for (int k = 0; k < CQ / 4; ++k) {
+      const int t = w + 4 * k;
+      if (lane < NC) sC[t * NC + lane] = t < tt && lane < N ? cv[k] : 0.f;
     }
   }
   // the state that enters chunk c: the recurrence over the chunks before it
@@ -261,21 +290,28 @@ __global__ __launch_bounds__(CH_THREADS) void ssd_chunk_carry_kernel(ChArgs a) {
   __syncthreads();
   // Y_off: y_t += exp(cs_t) C_t . S_in
   T* yb = (T*)a.y + (int64_t)b * a.ysb + (int64_t)h * P;
-  // wave w takes the rows w, w + 4, ..., lane = column of this work-group's half; eight rows' old values are loaded together
+  // wave w takes the rows w, w + 4, ..., lane = column of this work-group's half; all rows' old values are loaded together
   {
     const int w = tid >> 6, lane = tid & 63;
     const int p = p_lo + min(lane, PH - 1);
-    for (int kb = 0; kb < CQ / 4; kb += 8) {
-      float yo[8];
+    float yo[CQ / 4], acc[CQ / 4] = {};
 #pragma unroll
-      for (int k = 0; k < 8; ++k) yo[k] = to_f32(yb[(int64_t)(t0 + min(w + 4 * (kb + k), tt - 1)) * a.ysl + p]);
+    for (int k = 0; k < CQ / 4; ++k) yo[k] = to_f32(yb[(int64_t)(t0 + min(w + 4 * k, tt - 1)) * a.ysl + p]);
+    for (int n = 0; n < N; n += 4) {                       // four entries of the lane's state row, then C, the same for all lanes
+      float sn[4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int t = w + 4 * (kb + k);
-        float s_ = 0.f;
-        for (int n = 0; n < N; ++n) s_ = fmaf(sC[t * N + n], sS[p * (N + 1) + n], s_);
-        if (t < tt && lane < PH) yb[(int64_t)(t0 + t) * a.ysl + p] = from_f32<T>(fmaf(__expf(sCs[t]), s_, yo[k]));
+      for (int j = 0; j < 4; ++j) sn[j] = n + j < N ? sS[p * (N + 1) + n + j] : 0.f;
+#pragma unroll
+      for (int k = 0; k < CQ / 4; ++k) {
+        const f32x4 cq = *(const f32x4*)(sC + (w + 4 * k) * NC + n);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[k] = fmaf(cq[j], sn[j], acc[k]);
       }
+    }
+#pragma unroll
+    for (int k = 0; k < CQ / 4; ++k) {
+      const int t = w + 4 * k;
+      if (t < tt && lane < PH) yb[(int64_t)(t0 + t) * a.ysl + p] = from_f32<T>(fmaf(__expf(sCs[t]), acc[k], yo[k]));
     }
   }
 }
@@ -284,8 +320,8 @@ template <typename T>
 int launch_chunked(const ChArgs& a, int B, hipStream_t st) {
   const dim3 grid((unsigned)(2 * a.nch), (unsigned)a.H, (unsigned)B);
   const int PP = (a.P + 3) & ~3;
-  const size_t lds1 = (size_t)(CQ * PP + 2 * CQ * (a.N | 1) + CQ * 65 + 3 * CQ) * sizeof(float);
-  const size_t lds2 = (size_t)(a.P * (a.N + 1) + CQ * a.N + 2 * CQ + CH_MAXCHUNKS) * sizeof(float);
+  const size_t lds1 = (size_t)(CQ * PP + local_region(a.N) + 3 * CQ) * sizeof(float);
+  const size_t lds2 = (size_t)(((a.P * (a.N + 1) + 3) & ~3) + CQ * ((a.N + 3) & ~3) + 2 * CQ + CH_MAXCHUNKS) * sizeof(float);
   hipError_t e = hipFuncSetAttribute((const void*)ssd_chunk_local_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1);
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)ssd_chunk_carry_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2);
