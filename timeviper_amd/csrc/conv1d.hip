@@ -144,8 +144,8 @@ __global__ __launch_bounds__(CONV_THREADS) void conv1d_xbc_kernel(ConvArgs a) {
 // (same fp32 operations in the same order), group-major stores — and, while the chunk's 64 x 128 B and C tiles are
 // still on the chip (LDS), the causal part of C.B^T in the fragment order the scan kernel's mask waves read
 // (ssd_slice.hip: 6 fragments of 512 bf16 per (chunk, group); fragment (ti, sp), lane (lc, kq) holds
-// CB[16 ti + lc][32 sp + 8 kq + 0..7]).  Round 2 recomputed it in a pre-pass of the scan that read B and C back from
-// memory (0.8 GB and ~100 us per layer at 164 k tokens).
+// CB[16 ti + lc][32 sp + 8 kq + 0..7]).  A pre-pass of the scan that reads B and C back from
+// memory costs 0.8 GB and ~100 us per layer at 164 k tokens.
 // 256 threads: thread = (strip of 8 tokens, 16 bytes of the group's 256 B / C channels).
 constexpr int CBQ = 64, CBN = 128, CB_FRAGS = 6;
 template <int K>
