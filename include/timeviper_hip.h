@@ -296,6 +296,8 @@ int tv_gemm_bf16_fwd(const void* A, const void* W, const void* bias, void* C, in
  * (default), 0: never, 1: wherever the shape allows (tests); grid: work-groups of the persistent kernels, 0 = one per
  * compute unit. */
 void tv_gemm_set_persist(int mode, int grid);
+/* 0 where the persistent kernels are switched off (mode 0, or TV_GEMM_PERSIST=0 with mode -1): epilogue 3 is refused then. */
+int tv_gemm_persist_on(void);
 /* Of the persistent kernels the first choice is csrc/gemm_drip.hip: 256 x 192 tiles (the ViT's widths 1 152 / 3 456 /
  * 4 352 are multiples of 192, not of 256) whose finished tile leaves during the NEXT tile's K loop — half of it parked in
  * LDS, half in accumulator registers, stored one 1 KiB piece per phase with the GELU applied on the way out.  Takes

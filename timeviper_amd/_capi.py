@@ -45,6 +45,7 @@ SIGNATURES = {
     "tv_selective_state_update_rows": (_i, [_p] * 9 + [_i] * 5 + [_l] * 4 + [_i, _i, _p]),
     "tv_gemm_bf16_fwd": (_i, [_p, _p, _p, _p, _l, _i, _i, _l, _l, _l, _i, _i, _p]),
     "tv_gemm_set_persist": (None, [_i, _i]),
+    "tv_gemm_persist_on": (_i, []),
     "tv_gemm_set_drip": (None, [_i]),
     "tv_flash_attn_fwd": (_i, [_p] * 5 + [_i] * 6 + [_l] * 12 + [_f, _i, _i, _p]),
     "tv_flash_attn_sink_fwd": (_i, [_p] * 5 + [_i] * 7 + [_l] * 12 + [_f, _i, _p]),
@@ -111,7 +112,7 @@ class TimeViperHipError(RuntimeError):
     pass
 
 
-ABI_VERSION = 15      # tv_abi_version() of the library these SIGNATURES describe (csrc/capi.cpp)
+ABI_VERSION = 16      # tv_abi_version() of the library these SIGNATURES describe (csrc/capi.cpp)
 
 
 def lib_path() -> Path:

@@ -55,6 +55,7 @@ int launch_grouped(const GemmArgs& a, int64_t max_rows, int epilogue, hipStream_
 
 // gemm_persist.hip: returns TV_ERR_UNSUPPORTED (without setting the error text) when the shape is not one the persistent
 // kernel takes; the caller then runs the per-tile kernel.
+bool persist_on();         // not switched off (tv_gemm_set_persist, TV_GEMM_PERSIST=0)
 bool persist_takes(const GemmArgs& a, int epilogue);
 int launch_persist(const GemmArgs& a, int epilogue, hipStream_t st);
 int persist_grid();        // work-groups of the persistent kernels (one per compute unit unless tv_gemm_set_persist says otherwise)

@@ -417,9 +417,12 @@ int grid_size() {
 // Shapes the persistent kernel takes: the bias epilogues, whole 16-byte pieces everywhere, at least one full tile in both
 // directions (edge tiles are shifted back, not clamped).  Few tiles do not change that: N 4 304 with GELU, per-tile kernel | this: 2 916 rows (204
 // tiles) 42 | 41 us, 5 832: 80 | 74, 17 496: 201 | 189.
-bool persist_takes(const GemmArgs& a, int epilogue) {
+bool persist_on() {
   static const int off = [] { const char* e = getenv("TV_GEMM_PERSIST"); return e && atoi(e) == 0; }();
-  if (g_mode == 0 || (g_mode < 0 && off)) return false;
+  return g_mode > 0 || (g_mode < 0 && !off);
+}
+bool persist_takes(const GemmArgs& a, int epilogue) {
+  if (!persist_on()) return false;
   const int nkt = a.K / BK;
   if (epilogue == EPI_ACCUM || a.K % (2 * BK) || nkt < 4) return false;
   if (a.M < BM || a.N < BN || a.N % 8 || a.ldc % 8 || ((uintptr_t)a.C & 15)) return false;
@@ -450,3 +453,4 @@ int persist_grid() { return grid_size(); }
 }  // namespace tvgemm
 
 extern "C" void tv_gemm_set_persist(int mode, int grid) { tvgemm::set_persist(mode, grid); }
+extern "C" int tv_gemm_persist_on(void) { return tvgemm::persist_on(); }

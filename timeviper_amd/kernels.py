@@ -263,7 +263,7 @@ GEMM_BIAS, GEMM_BIAS_GELU, GEMM_ACCUM, GEMM_BIAS_RELU2 = 0, 1, 2, 3
 def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
     """F.linear(x, weight, bias) on the hand-written bf16 GEMM (csrc/gemm.hip) with the epilogue fused:
     GEMM_BIAS (plain), GEMM_BIAS_GELU (exact GELU of the bf16-rounded result: the timm Mlp's fc1 + act), GEMM_BIAS_RELU2 (its squared
-    ReLU; at least 256 rows and columns) or GEMM_ACCUM (out += x @ weight.T, `out` required, bias ignored).  x (..., K) bf16 with dense rows,
+    ReLU; at least 256 rows and columns, on the persistent kernel alone) or GEMM_ACCUM (out += x @ weight.T, `out` required, bias ignored).  x (..., K) bf16 with dense rows,
     weight (N, K) bf16; K % 128 == 0, N % 4 == 0."""
     _gpu(x, weight, bias, out)
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
@@ -308,6 +308,11 @@ def gemm_set_persist(mode: int = -1, grid: int = 0) -> None:
     work-groups of the persistent kernel (0 = one per compute unit; tests use 8 so that small problems still give
     every work-group several tiles)."""
     _capi.lib().tv_gemm_set_persist(int(mode), int(grid))
+
+
+def gemm_persist_on() -> bool:
+    """Whether `linear_fused` may take the persistent kernel (`gemm_set_persist`, TV_GEMM_PERSIST)."""
+    return bool(_capi.lib().tv_gemm_persist_on())
 
 
 # zero-padded inference copies of weights (model/vit/siglip.py): storage address -> (useful rows, useful columns), so that a
@@ -729,13 +734,13 @@ def large_takes(x, weight, relu2=False) -> bool:
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     rows = x.numel() // max(x.shape[-1], 1)
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and rows > MID_MAX and Kd >= 4096
-            and Kd % 128 == 0 and N % 8 == 0 and N >= 256 and x.is_contiguous() and weight.is_contiguous()
+            and Kd % 128 == 0 and N % 8 == 0 and 256 <= N < (1 << 22) and x.is_contiguous() and weight.is_contiguous()
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
         return False
     cus = 256                                                  # of an MI355X
     tiles = -(-rows // 256) * -(-N // 256)
     fill = tiles / (-(-tiles // cus) * cus)
-    if tiles <= cus:
+    if tiles <= cus or not gemm_persist_on():
         return False
     return fill >= 0.75 and Kd <= 8192 if relu2 else fill >= (0.69 if N >= 20480 else 0.8) and (N >= 20480 or Kd >= 8192)
 
