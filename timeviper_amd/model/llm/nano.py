@@ -27,6 +27,7 @@ import torch.nn.functional as F
 
 from ... import kernels as K
 from .cache import StaticDecode
+from ..plain_linear import plain_linear, unhooked
 from .pdrop import PdropMixin
 
 
@@ -305,17 +306,15 @@ def _rows_decode(x: torch.Tensor) -> bool:
 def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     if _fused_decode(x) and K.gemv_takes(x, mod.weight):
         return K.gemv_fused(x, mod.weight, mod.bias)
-    if _rows_decode(x) and K.rows_take(x, mod.weight):
+    if _rows_decode(x) and plain_linear(mod, x) and K.rows_take(x, mod.weight):
         return K.rows_linear(x, mod.weight, mod.bias)
     return _prompt_linear(mod, x)
 
 
 def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torch.Tensor:
     """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256) or tv_gemm_bf16_fwd where those
-    are faster than the library; what a caller may have put around the module (hooks, a subclass, autocast) sees it called as ever."""
-    if (x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and type(mod) is nn.Linear and not mod._forward_hooks
-            and not mod._forward_pre_hooks and not torch.is_autocast_enabled()
-            and (mod.bias is None or (mod.bias.dtype == x.dtype and mod.bias.is_contiguous() and mod.bias.data_ptr() % 16 == 0))):
+    are faster than the library (`plain_linear`: a module with anything around it is called)."""
+    if x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and plain_linear(mod, x):
         if K.rows_take(x, mod.weight):
             return K.rows_linear(x, mod.weight, mod.bias, relu2=relu2)
         if K.mid_takes(x, mod.weight, relu2):
@@ -463,6 +462,10 @@ class NemotronHMamba2Mixer(nn.Module):
         return out
 
 
+    def rows_fused(self, x) -> bool:
+        """decode_fused for more than four sequences: nothing may stand around the modules whose weights it reads"""
+        return type(self) is NemotronHMamba2Mixer and unhooked(self) and plain_linear(self.in_proj, x) and plain_linear(self.out_proj, x)
+
     def decode_fused(self, hidden, delta, norm, cache_params):
         """One decode token with the block's RMSNorm (+ residual add) inside in_proj and the gated norm inside out_proj:
         in_proj (+ conv update in its epilogue) -> state update -> out_proj, 3 launches.  Returns (residual stream, mixer output).
@@ -521,6 +524,9 @@ class NemotronHMLP(nn.Module):
     def forward(self, x):
         # `act_fn` stays for the module tree; the activation runs as one in-place HIP pass
         return _prompt_linear(self.down_proj, _prompt_linear(self.up_proj, x, relu2=True))
+
+    def rows_fused(self, x) -> bool:
+        return type(self) is NemotronHMLP and unhooked(self) and plain_linear(self.up_proj, x) and plain_linear(self.down_proj, x)
 
     def decode_fused(self, hidden, delta, norm):
         """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches (more than four sequences: 3,
@@ -587,6 +593,9 @@ class NemotronHAttention(nn.Module):
             self._qkv_cat = torch.cat([w.detach() for w in ws], dim=0).contiguous()
             self._qkv_key = key
         return self._qkv_cat
+
+    def rows_fused(self, x) -> bool:
+        return type(self) is NemotronHAttention and unhooked(self) and all(plain_linear(m, x) for m in (self.q_proj, self.k_proj, self.v_proj))
 
     def decode_fused(self, hidden, delta, norm, cache):
         """One decode token: the block's RMSNorm (+ residual add) in the prologue of ONE q / k / v product, cache append,
@@ -805,7 +814,8 @@ class NemotronHModel(PdropMixin, nn.Module):
         self.last_pdrop_trace = []
         delta = None  # pending mixer output, added inside the next fused norm
         c = self.config
-        fused_step = ((_fused_decode(hidden) or (_rows_decode(hidden) and all(n % 64 == 0 for n in (
+        rows = _rows_decode(hidden)
+        fused_step = ((_fused_decode(hidden) or (rows and all(n % 64 == 0 for n in (
                           c.hidden_size, c.intermediate_size, c.mamba_num_heads * c.mamba_head_dim)))) and past_key_values is not None and cache_position is not None
                       and int(cache_position[0]) > 0 and not output_hidden_states and not self.check_nan
                       and hidden.shape[-1] % 8 == 0 and hidden.shape[-1] <= 8192
@@ -833,7 +843,7 @@ class NemotronHModel(PdropMixin, nn.Module):
             if output_hidden_states:
                 all_hidden += ((hidden if delta is None else hidden + delta),)
             # x_{i+1} = x_i + mixer(norm(x_i)); the add of layer i-1 is fused into this norm
-            if fused_step and (block.block_type != "attention" or attn_fused):
+            if fused_step and (block.block_type != "attention" or attn_fused) and (not rows or block.mixer.rows_fused(hidden)):
                 # decode token: the norm (+ add) runs in the prologue of the block's first matrix-vector product
                 if block.block_type == "mlp":
                     hidden, delta = block.mixer.decode_fused(hidden, delta, block.norm)
