@@ -81,3 +81,19 @@ def test_autocast_reaches_the_modules(monkeypatch):
     with torch.autocast("cuda", torch.bfloat16):
         decode(m)
     assert not calls
+
+
+def test_operands_the_products_do_not_take(monkeypatch):
+    """A convolution kept in fp32, and weights off 16-byte alignment: the general operators, as with one sequence's worth of them"""
+    m = model()
+    m.backbone.layers[0].mixer.conv1d.float()
+    for mod in (m.backbone.layers[0].mixer.out_proj, m.backbone.layers[1].mixer.up_proj, m.backbone.layers[2].mixer.o_proj, m.lm_head):
+        w = torch.empty(mod.weight.numel() + 4, dtype=torch.bfloat16, device=DEV)[4:].view(mod.weight.shape)
+        assert w.data_ptr() % 16 == 8
+        w.copy_(mod.weight.detach())
+        mod.weight = torch.nn.Parameter(w, requires_grad=False)
+    got, conv = decode(m)
+    monkeypatch.setenv("TV_DECODE_FUSED", "0")
+    want, conv0 = decode(m)
+    rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
+    assert rel(got, want) < 2e-2 and rel(conv, conv0) < 2e-2

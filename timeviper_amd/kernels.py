@@ -644,13 +644,17 @@ def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=Non
 ROWS_MAX = 32
 
 
+def rows_weight(weight: torch.Tensor) -> bool:
+    """Weights tv_gemm_rows_fwd reads: bf16 (N, K), K a multiple of 64, 16-byte aligned rows."""
+    return (weight.dtype == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] % 64 == 0 and weight.shape[1] > 0 and weight.stride(1) == 1
+            and weight.stride(0) % 8 == 0 and weight.stride(0) < (1 << 24) and weight.data_ptr() % 16 == 0)
+
+
 def rows_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Shapes tv_gemm_rows_fwd is written for: 2..32 rows of bf16 against a bf16 (N, K) weight, K a multiple of 64."""
+    """Shapes tv_gemm_rows_fwd is written for: 2..32 rows of bf16 against such a weight."""
     Kd = x.shape[-1]
     n = x.numel() // max(Kd, 1)
-    return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2 and 2 <= n <= ROWS_MAX
-            and Kd % 64 == 0 and Kd > 0 and weight.stride(1) == 1 and weight.stride(0) % 8 == 0 and weight.stride(0) < (1 << 24)
-            and weight.data_ptr() % 16 == 0)
+    return x.is_cuda and x.dtype == torch.bfloat16 and 2 <= n <= ROWS_MAX and Kd % 64 == 0 and Kd > 0 and rows_weight(weight)
 
 
 def _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd):

@@ -463,8 +463,9 @@ class NemotronHMamba2Mixer(nn.Module):
 
 
     def rows_fused(self, x) -> bool:
-        """decode_fused for more than four sequences: nothing may stand around the modules whose weights it reads"""
-        return type(self) is NemotronHMamba2Mixer and unhooked(self) and plain_linear(self.in_proj, x) and plain_linear(self.out_proj, x)
+        """decode_fused for more than four sequences: nothing may stand around the modules whose weights it reads, and rows_linear takes them"""
+        return (type(self) is NemotronHMamba2Mixer and unhooked(self)
+                and all(plain_linear(m, x) and K.rows_weight(m.weight) for m in (self.in_proj, self.out_proj)))
 
     def decode_fused(self, hidden, delta, norm, cache_params):
         """One decode token with the block's RMSNorm (+ residual add) inside in_proj and the gated norm inside out_proj:
@@ -480,10 +481,12 @@ class NemotronHMamba2Mixer(nn.Module):
         d_in = self.intermediate_size
         conv_state = cache_params.conv_states[self.layer_idx]
         w = self.conv1d.weight.squeeze(1)
-        # the conv update rides in the product's epilogue where the kernel offers it (width 4, SiLU, K < 8192)
+        # the conv update rides in the product's epilogue where the kernel offers it (width 4, SiLU, K < 8192, parameters of the rows' dtype)
+        cb = self.conv1d.bias
         conv_in = (self.conv_kernel_size == 4 and self.activation in ("silu", "swish") and (rows or hidden.shape[-1] < 8192)
-                   and conv_state.dtype == hidden.dtype and conv_state.is_contiguous() and w.is_contiguous())
-        conv = (conv_state, w, self.conv1d.bias, d_in) if conv_in else None
+                   and conv_state.dtype == w.dtype == hidden.dtype and conv_state.is_contiguous() and w.is_contiguous()
+                   and (conv_state.data_ptr() | w.data_ptr()) % 8 == 0 and (cb is None or (cb.dtype == hidden.dtype and cb.is_contiguous())))
+        conv = (conv_state, w, cb, d_in) if conv_in else None
         if rows:
             proj = K.rows_linear(normed, self.in_proj.weight, self.in_proj.bias, conv=conv)
         else:
@@ -492,7 +495,7 @@ class NemotronHMamba2Mixer(nn.Module):
                                 eps=norm.variance_epsilon, conv=conv)
         gate, xBC, dt = proj.split([d_in, self.conv_dim, self.num_heads], dim=-1)
         negA, D32, dtb32 = self._consts()
-        xBC = xBC[:, 0] if conv_in else K.causal_conv1d_update(xBC[:, 0], conv_state, w, self.conv1d.bias, self.activation)
+        xBC = xBC[:, 0] if conv_in else K.causal_conv1d_update(xBC[:, 0], conv_state, w, cb, self.activation)
         x, Bm, Cm = torch.split(xBC, [d_in, gts, gts], dim=-1)
         y = K.selective_state_update(
             cache_params.ssm_states[self.layer_idx], x.unflatten(1, (self.num_heads, self.head_dim)), dt[:, 0], negA,
@@ -526,7 +529,8 @@ class NemotronHMLP(nn.Module):
         return _prompt_linear(self.down_proj, _prompt_linear(self.up_proj, x, relu2=True))
 
     def rows_fused(self, x) -> bool:
-        return type(self) is NemotronHMLP and unhooked(self) and plain_linear(self.up_proj, x) and plain_linear(self.down_proj, x)
+        return (type(self) is NemotronHMLP and unhooked(self)
+                and all(plain_linear(m, x) and K.rows_weight(m.weight) for m in (self.up_proj, self.down_proj)))
 
     def decode_fused(self, hidden, delta, norm):
         """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches (more than four sequences: 3,
@@ -595,7 +599,8 @@ class NemotronHAttention(nn.Module):
         return self._qkv_cat
 
     def rows_fused(self, x) -> bool:
-        return type(self) is NemotronHAttention and unhooked(self) and all(plain_linear(m, x) for m in (self.q_proj, self.k_proj, self.v_proj))
+        return (type(self) is NemotronHAttention and unhooked(self) and self.hidden_size % 64 == 0      # (rows_linear reads a stacked copy)
+                and all(plain_linear(m, x) and m.weight.dtype == x.dtype for m in (self.q_proj, self.k_proj, self.v_proj)))
 
     def decode_fused(self, hidden, delta, norm, cache):
         """One decode token: the block's RMSNorm (+ residual add) in the prologue of ONE q / k / v product, cache append,
@@ -813,10 +818,8 @@ class NemotronHModel(PdropMixin, nn.Module):
         train_pdrop_args = kwargs.get("train_pdrop_args")
         self.last_pdrop_trace = []
         delta = None  # pending mixer output, added inside the next fused norm
-        c = self.config
         rows = _rows_decode(hidden)
-        fused_step = ((_fused_decode(hidden) or (rows and all(n % 64 == 0 for n in (
-                          c.hidden_size, c.intermediate_size, c.mamba_num_heads * c.mamba_head_dim)))) and past_key_values is not None and cache_position is not None
+        fused_step = ((_fused_decode(hidden) or rows) and past_key_values is not None and cache_position is not None
                       and int(cache_position[0]) > 0 and not output_hidden_states and not self.check_nan
                       and hidden.shape[-1] % 8 == 0 and hidden.shape[-1] <= 8192
                       and self._all_matrices_bf16())
