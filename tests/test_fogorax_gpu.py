@@ -433,6 +433,28 @@ def test_batched_decoding_fused_and_general(B, tmp_path, monkeypatch):
         assert float(err.max()) < lim(BF), (fused, err.flatten().topk(5))
 
 
+@pytest.mark.parametrize("which", ["inp", "out", "gate", "proj"])
+def test_batched_decoding_with_a_weight_off_its_alignment(which, tmp_path, monkeypatch):
+    """8-byte aligned weights of one layer: the general operators, whatever the batch"""
+    from timeviper_amd.model.llm import TextEngine
+    cfg, _, llm = C.build("large", BF, DEV, tmp_path, seed=12)
+    layer = llm.backbone.layers[1]
+    owner = layer.side if which in ("gate", "proj") else layer
+    w = getattr(owner, which)
+    off = torch.empty(w.numel() + 4, dtype=BF, device=DEV)[4:].view(w.shape)
+    off.copy_(w.detach())
+    setattr(owner, which, torch.nn.Parameter(off, requires_grad=False))
+    assert off.data_ptr() % 16 == 8
+    toks = [C.prompt(cfg, 9 + i, 400 + i) for i in range(6)]
+    got = []
+    for fused in ("1", "0"):
+        monkeypatch.setenv("TV_DECODE_FUSED", fused)
+        eng = TextEngine(llm, slots=2)
+        eng.step([(i, t[:-1], [len(t) - 2]) for i, t in enumerate(toks)])
+        got.append(eng.step([(i, t[-1:], [0]) for i, t in enumerate(toks)]))
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("graph", ["1", "0"])
 @pytest.mark.parametrize("name,dtype", [("odd", torch.float32), ("tiles", torch.float32), ("tiles", BF), ("large", BF)])
 def test_greedy_generation_through_the_scheduler(name, dtype, graph, tmp_path, monkeypatch):

@@ -89,8 +89,9 @@ class ParallelLayer(nn.Module):
         return x, (self.side(h, ids, side_rows), self.side.norm)
 
     def decode_takes(self, rows, dtype):
-        if 4 < rows <= K.ROWS_MAX:               # the products on the matrix cores: a multiple of 64 columns each
-            return dtype == torch.bfloat16 and self.k1 % 8 == 0 and all(n % 64 == 0 for n in (self.shift.numel(), self.out.shape[1], self.side.dim))
+        if 4 < rows <= K.ROWS_MAX:               # the products on the matrix cores (gate and up rows of one work-group at 32-bit offsets)
+            return (dtype == torch.bfloat16 and self.k1 % 8 == 0 and all(K.rows_weight(w) for w in (self.inp, self.out, self.side.gate, self.side.proj))
+                    and (self.inp.shape[0] + 32) * self.inp.stride(0) * 2 < (1 << 31))
         return all(K.gemv_rows_take(rows, n, dtype) for n in (self.shift.numel(), self.out.shape[1], self.side.dim)) and self.k1 % 8 == 0
 
     def decode(self, x, pending, ids, side_rows, state, kv_rows, plan):
