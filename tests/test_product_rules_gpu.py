@@ -32,3 +32,18 @@ def test_persistent_kernel_switched_off(K, N, relu2):
             ops.gemm_set_persist(-1)
         want = lin(x)
         assert torch.equal(got, ops.relu2(want, inplace=True) if relu2 else want)
+
+
+@pytest.mark.parametrize("rows", [5, 32])
+def test_output_layer_keeps_its_gradient(rows):
+    """logits of 5..32 rows of a packed model: differentiable in the table where gradients are enabled"""
+    from timeviper_amd.model.llm.packed import vocabulary_logits
+    h = torch.randn(rows, 128, device=DEV).to(BF)
+    table = torch.nn.Parameter(torch.randn(300, 128, device=DEV).to(BF))
+    up = torch.randn(rows, 300, device=DEV).to(BF).float()
+    vocabulary_logits(h, table).backward(up)
+    want = up.double().T @ h.double()                               # fp32 sums of `rows` products, rounded to bf16
+    assert (table.grad.double() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+    with torch.no_grad():
+        got = vocabulary_logits(h, table)
+    assert got.dtype == torch.float32 and (got.double() - h.double() @ table.double().T).abs().max() < 1e-3
