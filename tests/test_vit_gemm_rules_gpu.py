@@ -84,3 +84,25 @@ def test_long_prompts(rows, N, K, relu2, own, monkeypatch):
     assert bool(calls) == own
     # 2^-8 a rounding of bf16: one, or a squared one (twice) and another; 5 % for the fp32 sums
     assert (got[0, sel].double() - ref).abs().max() <= 1.05 * (3 if relu2 else 1) * 2.0 ** -8 * ref.abs().max()
+
+
+def test_weights_off_their_alignment_are_the_librarys(monkeypatch):
+    """qkv, proj and fc2 weights at an address that is no multiple of 16 bytes: the block runs, and none of them on the hand-written kernels"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.vit.siglip import Block
+    torch.manual_seed(0)
+    blk = Block(1152, 16, 4352).to(DEV, BF).eval().requires_grad_(False)
+    x = torch.randn(10, 729, 1152, device=DEV).to(BF)
+    with torch.no_grad():
+        want = blk.forward_stream(x.clone(), None)[0]
+    for mod in (blk.attn.qkv, blk.attn.proj, blk.mlp.fc1, blk.mlp.fc2):
+        w = torch.empty(mod.weight.numel() + 4, dtype=BF, device=DEV)[4:].view(mod.weight.shape)
+        w.copy_(mod.weight)
+        mod.weight = torch.nn.Parameter(w, requires_grad=False)
+        assert w.data_ptr() % 16 == 8
+    calls, real = [], ops.linear_fused
+    monkeypatch.setattr(ops, "linear_fused", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        got = blk.forward_stream(x.clone(), None)[0]
+    assert not calls
+    assert ((got.float() - want.float()).norm() / want.float().norm()) < 1e-2

@@ -71,6 +71,11 @@ def _tiles(rows: int, n: int, width: int = 256) -> int:
     return -(-rows // 256) * -(-n // width)
 
 
+def _gemm_reads(*ts) -> bool:
+    """Rows that tv_gemm_bf16_fwd reads and writes in 16-byte pieces"""
+    return all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and (t.dim() == 1 or t.stride(-2) % 8 == 0) for t in ts)
+
+
 def _aligned(n: int) -> int:
     return -(-n // GEMM_ALIGN) * GEMM_ALIGN
 
@@ -151,7 +156,7 @@ class Attention(nn.Module):
         rounds = -(-_tiles(rows, w.shape[0]) // CUS)
         own = rows >= 65536 if os.environ.get("TV_VIT_OWN_QKV", "0") == "1" else 2 <= rounds <= 6
         return (own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
-                and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0)
+                and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and _gemm_reads(x, w, self.qkv.bias))
 
     def forward(self, x):
         return self.proj(self.heads(x))
@@ -173,25 +178,25 @@ class Mlp(nn.Module):
             w1, b1, w2 = self._padded.get((self.fc1.weight, self.fc1.bias, self.fc2.weight), lambda: (
                 _pad_rows(self.fc1.weight.detach(), _aligned(Hd)), _pad_rows(self.fc1.bias.detach(), _aligned(Hd)),
                 _pad_cols(self.fc2.weight.detach(), _aligned(Hd))))
-            if self._fused_fc1(x, w1):
+            if self._fused_fc1(x, w1, b1):
                 return K.linear_fused(x, w1, b1, epilogue=K.GEMM_BIAS_GELU), w2
             h = F.linear(x, w1, b1)
         else:
             w2 = self.fc2.weight
-            if self._fused_fc1(x, self.fc1.weight):
+            if self._fused_fc1(x, self.fc1.weight, self.fc1.bias):
                 return K.linear_fused(x, self.fc1.weight, self.fc1.bias, epilogue=K.GEMM_BIAS_GELU), w2
             h = self.fc1(x)
         h = K.gelu(h, inplace=True) if self.exact_gelu else self.act(h)
         return h, w2
 
-    def _fused_fc1(self, x, w1) -> bool:
+    def _fused_fc1(self, x, w1, b1) -> bool:
         """fc1 + bias + exact GELU in ONE kernel (csrc/gemm_persist.hip from 4 tiles per compute unit on, csrc/gemm.hip
         below: the activation is applied to the accumulators, same rounding points as GEMM-then-GELU): 14.0 ms
         (persistent) / 14.8 ms (per tile) against 16.7 ms for hipBLASLt + tv_gelu_fwd per 2 048 SigLIP frames.  bf16 on the GPU, inference, K
         a multiple of 128, tiles for three quarters of the compute units (4 frames, 204 tiles: library + GELU 42 us, fused 41; 3 frames, 153:
         34 and 39); TV_VIT_FUSED_FC1=0 switches it off."""
         return (self.exact_gelu and x.is_cuda and x.dtype == torch.bfloat16 and w1.dtype == torch.bfloat16
-                and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0
+                and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0 and _gemm_reads(x, w1, b1)
                 and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
 
     def forward(self, x):
@@ -218,7 +223,7 @@ def _accumulate(x2: torch.Tensor, h2: torch.Tensor, w: torch.Tensor, role: str) 
     rows, n = x2.shape
     if ((_own_accumulate(rows, n) or (role in _OWN_ACCUM and rows >= 65536)) and x2.is_cuda and x2.dtype == torch.bfloat16
             and h2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0
-            and w.shape[1] >= 1152 and n % 8 == 0 and h2.stride(1) == 1 and w.stride(1) == 1):
+            and w.shape[1] >= 1152 and n % 8 == 0 and _gemm_reads(x2, h2, w)):
         K.linear_fused(h2, w, None, epilogue=K.GEMM_ACCUM, out=x2)
     else:
         torch.addmm(x2, h2, w.t(), out=x2)
