@@ -106,3 +106,14 @@ def test_weights_off_their_alignment_are_the_librarys(monkeypatch):
         got = blk.forward_stream(x.clone(), None)[0]
     assert not calls
     assert ((got.float() - want.float()).norm() / want.float().norm()) < 1e-2
+
+
+# (width, tokens a frame, frames) -> the qkv projection is faster on the persistent kernel: padded widths alone, rounds that are full, ragged rows
+@pytest.mark.parametrize("width,heads,tokens,frames,own", [(1152, 16, 729, 15, True), (1152, 16, 729, 33, True), (1152, 16, 729, 8, False),
+                                                           (1152, 16, 729, 14, False), (1152, 16, 729, 41, False), (1152, 16, 256, 32, False),
+                                                           (768, 12, 576, 16, False), (1024, 16, 261, 24, False)])
+def test_qkv_rule(width, heads, tokens, frames, own):
+    from timeviper_amd.model.vit.siglip import Attention
+    attn = Attention(width, heads).to(DEV, BF).requires_grad_(False)
+    with torch.no_grad():
+        assert attn._own_qkv(torch.empty(frames, tokens, width, device=DEV, dtype=BF)) is own
