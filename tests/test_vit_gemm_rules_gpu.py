@@ -117,3 +117,9 @@ def test_qkv_rule(width, heads, tokens, frames, own):
     attn = Attention(width, heads).to(DEV, BF).requires_grad_(False)
     with torch.no_grad():
         assert attn._own_qkv(torch.empty(frames, tokens, width, device=DEV, dtype=BF)) is own
+
+
+@pytest.mark.parametrize("rows,n,own", [(7290, 1152, True), (34992, 1152, True), (13122, 1152, False), (10368, 768, False), (73728, 768, False)])
+def test_accumulate_rule(rows, n, own):
+    from timeviper_amd.model.vit.siglip import _own_accumulate
+    assert _own_accumulate(rows, n) is own
