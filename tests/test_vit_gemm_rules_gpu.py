@@ -123,3 +123,24 @@ def test_qkv_rule(width, heads, tokens, frames, own):
 def test_accumulate_rule(rows, n, own):
     from timeviper_amd.model.vit.siglip import _own_accumulate
     assert _own_accumulate(rows, n) is own
+
+
+def test_hook_on_fc1_of_a_short_clip(monkeypatch):
+    """3 654 rows of the 1 024 wide tower: fused as it stands, called with a hook on it"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.vit.siglip import Mlp
+    torch.manual_seed(0)
+    mlp = Mlp(1024, 4096).to(DEV, BF).requires_grad_(False)
+    x = torch.randn(14, 261, 1024, device=DEV).to(BF)
+    calls, real = [], ops.linear_fused
+    monkeypatch.setattr(ops, "linear_fused", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        plain = mlp(x)
+        assert calls == [1]
+        handle = mlp.fc1.register_forward_hook(lambda m, a, y: 2 * y)
+        got = mlp(x)
+        handle.remove()
+        want = F.linear(F.gelu(2 * F.linear(x, mlp.fc1.weight, mlp.fc1.bias)), mlp.fc2.weight, mlp.fc2.bias)
+    assert calls == [1]
+    rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
+    assert rel(got, want) < 1e-2 < rel(plain, want)

@@ -23,6 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ... import kernels as K
+from ..plain_linear import plain_linear
 
 TIMM_VIT_CONFIGS = {
     # public timm model definitions (not in the reference tree)
@@ -189,7 +190,8 @@ class Mlp(nn.Module):
             h = F.linear(x, w1, b1)
         else:
             w2 = self.fc2.weight
-            if self._fused_fc1(x, self.fc1.weight, self.fc1.bias):
+            # (below 4 096 rows fc1 is called if anything stands around it)
+            if (x.numel() // x.shape[-1] >= 4096 or plain_linear(self.fc1, x)) and self._fused_fc1(x, self.fc1.weight, self.fc1.bias):
                 return K.linear_fused(x, self.fc1.weight, self.fc1.bias, epilogue=K.GEMM_BIAS_GELU), w2
             h = self.fc1(x)
         h = K.gelu(h, inplace=True) if self.exact_gelu else self.act(h)
