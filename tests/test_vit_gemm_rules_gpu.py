@@ -144,3 +144,15 @@ def test_hook_on_fc1_of_a_short_clip(monkeypatch):
     assert calls == [1]
     rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
     assert rel(got, want) < 1e-2 < rel(plain, want)
+
+
+def test_qkv_switch(monkeypatch):
+    """TV_VIT_OWN_QKV: 0 never, unset by the rule, 1 by the rule and from 65 536 rows on"""
+    from timeviper_amd.model.vit.siglip import Attention
+    attn = Attention(1152, 16).to(DEV, BF).requires_grad_(False)
+    got = {}
+    for switch in ("0", None, "1"):
+        monkeypatch.setenv("TV_VIT_OWN_QKV", switch) if switch else monkeypatch.delenv("TV_VIT_OWN_QKV")
+        with torch.no_grad():
+            got[switch] = [attn._own_qkv(torch.empty(n, 729, 1152, device=DEV, dtype=BF)) for n in (2, 20, 60, 90)]
+    assert got == {"0": [False] * 4, None: [False, True, False, False], "1": [False, True, False, True]}

@@ -155,13 +155,14 @@ class Attention(nn.Module):
         frame: 15 frames 106 | 89, 18: 112 | 98, 20: 149 | 118, 24: 145 | 128, 33: 211 | 181, 38: 204 | 192; the library's choice of a kernel varies, so that some in
         between lose 1 - 6 % (11: 59 | 63, 23: 122 | 126, 28: 149 | 155).  Fewer tiles in the last round: 8 frames (63 %) 51 | 57, 14 (73 %) 81 | 87.  One round: 5
         frames 31 | 33; more than six: 41 211 | 216, 64 326 | 333, and 0.5 % of a 10 240-frame forward.  256 tokens a frame: 32 frames 59 | 62, 96 175 | 181.  Whole
-        tiles of columns: 2 304 (K 768), 9 216 rows 39 | 42; 3 072 (K 1 024), 6 264 rows 43 | 52.  Or everywhere with TV_VIT_OWN_QKV=1.  bf16 on the GPU, inference, K
-        a multiple of 128, N of 8."""
+        tiles of columns: 2 304 (K 768), 9 216 rows 39 | 42; 3 072 (K 1 024), 6 264 rows 43 | 52.  TV_VIT_OWN_QKV=1: also from 65 536 rows
+        on; 0: never.  bf16 on the GPU, inference, K a multiple of 128, N of 8."""
         w, rows = self.qkv.weight, x.numel() // x.shape[-1]
         tiles = _tiles(rows, w.shape[0])
         rounds = -(-tiles // CUS)
-        own = rows >= 65536 if os.environ.get("TV_VIT_OWN_QKV", "0") == "1" else (
-            2 <= rounds <= 6 and 4 * tiles >= 3 * rounds * CUS and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on())
+        switch = os.environ.get("TV_VIT_OWN_QKV", "")
+        own = switch != "0" and ((switch == "1" and rows >= 65536) or (
+            2 <= rounds <= 6 and 4 * tiles >= 3 * rounds * CUS and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
         return bool(own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
                 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and _gemm_reads(x, w, self.qkv.bias))
 
