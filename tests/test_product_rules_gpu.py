@@ -47,3 +47,13 @@ def test_output_layer_keeps_its_gradient(rows):
     with torch.no_grad():
         got = vocabulary_logits(h, table)
     assert got.dtype == torch.float32 and (got.double() - h.double() @ table.double().T).abs().max() < 1e-3
+
+
+# (4 480 wide stack: in_proj, out_proj, up_proj + squared ReLU) x rows on either side of each line
+@pytest.mark.parametrize("N,K,relu2,rows,own", [(22656, 4480, False, 10007, True), (22656, 4480, False, 14000, False), (22656, 4480, False, 163940, False),
+                                                (4480, 10240, False, 28000, True), (4480, 10240, False, 40000, False), (4480, 10240, False, 163940, False),
+                                                (15680, 4480, True, 163940, True), (15680, 4480, False, 10007, False)])
+def test_large_rule(N, K, relu2, rows, own):
+    from timeviper_amd import kernels as ops
+    x, w = torch.empty(1, rows, K, device=DEV, dtype=BF), torch.empty(N, K, device=DEV, dtype=BF)
+    assert ops.large_takes(x, w, relu2) is own

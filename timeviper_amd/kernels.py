@@ -731,10 +731,13 @@ def mid_takes(x, weight, relu2=False) -> bool:
 
 def large_takes(x, weight, relu2=False) -> bool:
     """Products of a long prompt that the persistent GEMM (tv_gemm_bf16_fwd) runs faster than the library: its 256 x 256 tiles are two
-    rounds of the compute units or more and fill them, and the output is wide (22 656 x 4 480, us, library | here: 1 500 rows, 70 % full, 355 | 275; 2 048: 445 |
-    319, 4 096: 726 | 617, 10 007: 1 494 | 1 464), the contraction long (4 480 x 10 240: 6 011 rows 481 | 408, 10 007: 937 | 718; 75 % full, 8 000 rows: 579 |
-    591; one round, 3 000: 191 | 195) or the squared ReLU saves its own pass (15 680 x 4 480, 2 048 rows 198 + 24 | 207, 10 007: 974 + 102 | 1 028).  The rest
-    stays the library's (15 680 x 4 480 alone; 12 288 x 4 096, 8 000 rows: 553 | 595)."""
+    rounds of the compute units or more and fill them, and
+      - the output is wide, up to 12 288 rows (22 656 x 4 480, us, library | here: 1 500 rows, 70 % full, 355 | 275; 2 048: 445 | 319, 4 096: 726 | 617, 10 007: 1 494 |
+        1 464; from there on the library's longer K loop wins: 14 000: 1 980 | 2 067, 80 000: 10 964 | 11 645, 163 940: 22 528 | 23 831),
+      - the contraction is long, up to 32 768 rows (4 480 x 10 240: 6 011 rows 473 | 429, 10 007: 934 | 701, 28 000: 1 997 | 1 860, 40 000: 2 647 | 2 706, 163 940:
+        10 637 | 10 797; 75 % full, 8 000 rows: 575 | 616; one round, 3 000: 191 | 195), or
+      - the squared ReLU saves its own pass (15 680 x 4 480, with that pass: 2 048 rows 222 | 207, 10 007: 1 103 | 1 034, 163 940: 17 722 | 16 798).
+    The rest stays the library's (15 680 x 4 480 alone; 12 288 x 4 096, 8 000 rows: 553 | 595)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     rows = x.numel() // max(x.shape[-1], 1)
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and rows > MID_MAX and Kd >= 4096
@@ -746,7 +749,9 @@ def large_takes(x, weight, relu2=False) -> bool:
     fill = tiles / (-(-tiles // cus) * cus)
     if tiles <= cus or not gemm_persist_on():
         return False
-    return fill >= 0.75 and Kd <= 8192 if relu2 else fill >= (0.69 if N >= 20480 else 0.8) and (N >= 20480 or Kd >= 8192)
+    if relu2:
+        return fill >= 0.75 and Kd <= 8192
+    return (N >= 20480 and rows <= 12288 and fill >= 0.69) or (N < 20480 and Kd >= 8192 and rows <= 32768 and fill >= 0.8)
 
 
 def mid_linear(x, weight, bias=None, relu2=False):
