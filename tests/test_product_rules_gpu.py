@@ -57,3 +57,29 @@ def test_large_rule(N, K, relu2, rows, own):
     from timeviper_amd import kernels as ops
     x, w = torch.empty(1, rows, K, device=DEV, dtype=BF), torch.empty(N, K, device=DEV, dtype=BF)
     assert ops.large_takes(x, w, relu2) is own
+
+
+@pytest.mark.parametrize("M", [1, 2, 4])
+def test_decode_products_refuse_and_take_what_one_row_does(M):
+    """gemv_fused: rows off their alignment, a convolution behind 8 192 inputs and groups of more than 2 048 channels are refused whatever the
+    number of rows; a norm weight at an 8-byte address is taken"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV).to(BF)
+    w = r(96, 8192)
+    with pytest.raises(ops.TimeViperHipError):
+        ops.gemv_fused(r(M, 8192 + 8)[:, 4:-4], w)
+    with pytest.raises(ops.TimeViperHipError):
+        ops.gemv_fused(r(M, 8192), w, conv=(r(M, 32, 4), r(32, 4), None, 16))
+    with pytest.raises(ops.TimeViperHipError):
+        ops.gemv_fused(r(M, 8192), w, prologue=ops.GEMV_GATED, gate=r(M, 8192), norm_weight=r(8192), group_size=4096, eps=1e-5)
+    x, nw = r(M, 512), 1 + 0.1 * r(516)
+    off = nw[4:]
+    assert off.data_ptr() % 16 == 8
+    w = r(96, 512)
+    got = ops.gemv_fused(x, w, prologue=ops.GEMV_RMSNORM, norm_weight=off, eps=1e-5)
+    f = (x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5) * off.double())
+    want = f @ w.double().T
+    # two roundings of the 512 normed values (2^-8 each, at random signs) and one of the sum
+    bound = 2.0 ** -7 * torch.sqrt(f.square() @ w.double().square().T) * 2 + 2.0 ** -8 * want.abs()
+    assert ((got.double() - want).abs() <= bound).all()

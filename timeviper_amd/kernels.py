@@ -627,7 +627,11 @@ def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=Non
         if (cst.dtype != x.dtype or cw.dtype != x.dtype or not cst.is_contiguous() or not cw.is_contiguous()
                 or cst.shape != (M, nch, 4) or cw.shape != (nch, 4) or (cb is not None and (cb.dtype != x.dtype or not cb.is_contiguous()))):
             raise TimeViperHipError("gemv_fused: conv needs a contiguous (rows, C, 4) state and (C, 4) weight of x's dtype")
-    if M <= 4 and rows_take(x2, weight) and M * K * 2 <= 128 * 1024:
+    # (what the matrix-vector kernel refuses for one row it refuses for several: its bounds, not those of the launches that stand in for it)
+    as_one = (M <= 4 and M * K * 2 <= 128 * 1024 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (conv is None or K < 8192)
+              and (prologue != GEMV_RMSNORM or K <= 8192) and (prologue != GEMV_GATED or 0 < group_size <= 2048)
+              and (norm_weight is None or norm_weight.data_ptr() % 16 == 0) and GEMV_NONE <= prologue <= GEMV_GATED)
+    if as_one and rows_take(x2, weight):
         # several rows: the operator in front as its own launch and the product on the matrix cores (22 656 x 4 480, four rows: 42.8 us with
         # the prologue in the matrix-vector kernel, 30.5 + 5); same rounding points
         f = _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd=K)
