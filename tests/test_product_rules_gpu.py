@@ -83,3 +83,17 @@ def test_decode_products_refuse_and_take_what_one_row_does(M):
     # two roundings of the 512 normed values (2^-8 each, at random signs) and one of the sum
     bound = 2.0 ** -7 * torch.sqrt(f.square() @ w.double().square().T) * 2 + 2.0 ** -8 * want.abs()
     assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K,normed,rows", [(2, 1024, 1024, True, False), (2, 1024, 1024, False, True), (3, 1024, 1024, True, True), (2, 4096, 1024, True, True),
+                                               (2, 4480, 4480, True, True), (1, 4480, 4480, True, False)])
+def test_two_rows_of_a_small_matrix_are_one_launch(M, N, K, normed, rows, monkeypatch):
+    from timeviper_amd import kernels as ops
+    calls, real = [], ops._rows_product
+    monkeypatch.setattr(ops, "_rows_product", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    x, w = torch.randn(M, K, device=DEV).to(BF), torch.randn(N, K, device=DEV).to(BF)
+    kw = dict(prologue=ops.GEMV_RMSNORM, norm_weight=torch.ones(K, device=DEV), eps=1e-5) if normed else {}
+    got = ops.gemv_fused(x, w, **kw)
+    f = ops.rms_norm(x, torch.ones(K, device=DEV), 1e-5) if normed else x
+    want = f.double() @ w.double().T
+    assert bool(calls) is rows and ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + (f.double().abs() @ w.double().abs().T) * K * 2.0 ** -24).all()

@@ -631,9 +631,11 @@ def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=Non
     as_one = (M <= 4 and M * K * 2 <= 128 * 1024 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (conv is None or K < 8192)
               and (prologue != GEMV_RMSNORM or K <= 8192) and (prologue != GEMV_GATED or 0 < group_size <= 2048)
               and (norm_weight is None or norm_weight.data_ptr() % 16 == 0) and GEMV_NONE <= prologue <= GEMV_GATED)
-    if as_one and rows_take(x2, weight):
-        # several rows: the operator in front as its own launch and the product on the matrix cores (22 656 x 4 480, four rows: 42.8 us with
-        # the prologue in the matrix-vector kernel, 30.5 + 5); same rounding points
+    if as_one and rows_take(x2, weight) and (M > 2 or prologue == GEMV_NONE or N > K or N * K >= (1 << 23)):
+        # several rows: the operator in front as its own launch and the product on the matrix cores, same rounding points.  us with the prologue
+        # in the matrix-vector kernel | so, 2, 3 and 4 rows: 22 656 x 4 480, RMSNorm 37 41 45 | 35 35 35; 4 480 x 15 680, ReLU^2 30 43 49 | 25 25 25; 6 144 x
+        # 2 048, RMSNorm 10.5 12.8 15.0 | 9.6 9.7 9.8; 1 024 x 1 024 without one 4.6 5.0 5.3 | 3.6 3.7 3.7.  Two rows of a small matrix
+        # with few outputs do not pay for the launch (2 048 x 2 048, RMSNorm 7.0 | 7.1; 1 024 x 4 096, ReLU^2 6.5 | 7.0; 4 096 x 1 024, RMSNorm 7.2 | 6.7).
         f = _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd=K)
         _rows_product(f, weight, bias, y, 0, cst, cw, cb, row0, nch)
         return y
