@@ -97,3 +97,19 @@ def test_two_rows_of_a_small_matrix_are_one_launch(M, N, K, normed, rows, monkey
     f = ops.rms_norm(x, torch.ones(K, device=DEV), 1e-5) if normed else x
     want = f.double() @ w.double().T
     assert bool(calls) is rows and ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + (f.double().abs() @ w.double().abs().T) * K * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("rows,N,K,own", [(17, 131072, 1024, True), (24, 131072, 1024, False), (32, 32768, 1024, True), (20, 131072, 1024, True)])
+def test_output_layer_of_many_sequences(rows, N, K, own, monkeypatch):
+    """more than 20 rows of the largest matrices are the library's: a step's output layer, and a packed model's"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    from timeviper_amd.model.llm.packed import vocabulary_logits
+    lin, x = linear(K, N), torch.randn(rows, 1, K, device=DEV).to(BF)
+    calls, real = [], ops.rows_linear
+    monkeypatch.setattr(ops, "rows_linear", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    want = x[:, 0, :].double() @ lin.weight[-500:].double().T
+    with torch.no_grad():
+        for got in (nano._linear(lin, x)[:, 0], vocabulary_logits(x[:, 0], lin.weight)):
+            assert (got[:, -500:].double() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+    assert len(calls) == (2 if own else 0)

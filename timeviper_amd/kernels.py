@@ -663,6 +663,13 @@ def rows_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return x.is_cuda and x.dtype == torch.bfloat16 and 2 <= n <= ROWS_MAX and Kd % 64 == 0 and Kd > 0 and rows_weight(weight)
 
 
+def rows_pay(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Shapes of `rows_take` on which tv_gemm_rows_fwd is faster than the library: more than 20 rows of a matrix of over 96 million entries
+    are not (x, read again by every work-group, is then as many bytes as W; us, library | here: 131 072 x 4 480, 17 rows 198 | 189, 24: 199 | 207, 32: 198 |
+    235; 65 536 x 4 480, 20: 102 | 98, 28: 102 | 108; 22 656 x 4 480, 24: 39 | 38, 32: 40 | 42; 15 680 x 4 480, 32: 37 | 29; 32 768 x 2 048, 32: 34 | 29)."""
+    return rows_take(x, weight) and (x.numel() <= 20 * x.shape[-1] or weight.numel() <= 96_000_000)
+
+
 def _rows_prologue(x2, prologue, d2, s2, norm_weight, nw_dt, eps, g2, group_size, Kd):
     """f(x) of gemv_fused for several rows, by the stand-alone kernels"""
     if prologue == GEMV_NONE:

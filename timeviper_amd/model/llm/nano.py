@@ -306,7 +306,7 @@ def _rows_decode(x: torch.Tensor) -> bool:
 def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     if _fused_decode(x) and K.gemv_takes(x, mod.weight):
         return K.gemv_fused(x, mod.weight, mod.bias)
-    if _rows_decode(x) and plain_linear(mod, x) and K.rows_take(x, mod.weight):
+    if _rows_decode(x) and plain_linear(mod, x) and K.rows_pay(x, mod.weight):
         return K.rows_linear(x, mod.weight, mod.bias)
     return _prompt_linear(mod, x)
 
@@ -315,7 +315,7 @@ def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torc
     """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256) or tv_gemm_bf16_fwd where those
     are faster than the library (`plain_linear`: a module with anything around it is called)."""
     if x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and plain_linear(mod, x):
-        if K.rows_take(x, mod.weight):
+        if K.rows_pay(x, mod.weight):
             return K.rows_linear(x, mod.weight, mod.bias, relu2=relu2)
         if K.mid_takes(x, mod.weight, relu2):
             return K.mid_linear(x, mod.weight, mod.bias, relu2)

@@ -19,7 +19,7 @@ def vocabulary_logits(h, table):
     """fp32 logits of rows in the model's dtype against a (vocab, width) matrix"""
     if K.gemv_post_takes(h.shape[0], h.shape[1], h.dtype):
         return K.gemv_post(h, table, out_dtype=torch.float32)
-    if K.rows_take(h, table) and not (torch.is_grad_enabled() and (h.requires_grad or table.requires_grad)):
+    if K.rows_pay(h, table) and not (torch.is_grad_enabled() and (h.requires_grad or table.requires_grad)):
         return K.rows_linear(h, table, out_dtype=torch.float32)
     return F.linear(h, table).float()
 
