@@ -40,8 +40,9 @@ def test_layers_take_them(tokens, monkeypatch):
     from timeviper_amd import kernels as ops
     from timeviper_amd.model.llm import nano
     torch.manual_seed(tokens)
-    lin = torch.nn.Linear(4096, 2048, bias=True, device=DEV, dtype=BF).requires_grad_(False)
-    x = torch.randn(1, tokens, 4096, device=DEV, dtype=BF)
+    # (a size that the rule takes up to 256 rows; 4 096 -> 2 048 is faster in the library from 65 on)
+    lin = torch.nn.Linear(8192, 4096, bias=True, device=DEV, dtype=BF).requires_grad_(False)
+    x = torch.randn(1, tokens, 8192, device=DEV, dtype=BF)
     calls = []
     for name in ("mid_linear", "rows_linear"):
         real = getattr(ops, name)

@@ -731,14 +731,18 @@ MID_MAX = 256
 
 
 def mid_takes(x, weight, relu2=False) -> bool:
-    """Products of up to 256 rows that tv_gemm_mid_fwd runs faster than the library: a long contraction into fewer outputs (4 480 x 15 680, 203
-    rows: 131 us in the library, 52 here), any of at most 64 rows (15 680 x 4 480, 64 rows: 42, 32), and the squared ReLU of up to 256 (its own pass
-    saved; without it 128 rows 42 and 44, 203: 50 and 51).  Shorter contractions and a thousand outputs are the library's (6 144 x 2 048, 128 rows: 12
-    and 20 us; 1 024 x 4 480, 256: 14.5 and 16)."""
+    """Products of up to 256 rows that tv_gemm_mid_fwd runs faster than the library (us, library | here):
+      - any of at most 64 rows (15 680 x 4 480, 64 rows: 42 | 32; 1 024 x 4 480, 64: 21 | 10) but for 1, 2 or 3 x 4 096 outputs of a contraction no longer
+        than they are (4 096 x 4 096, 48 rows: 13.5 | 14.3; 8 192 x 8 192: 32 | 36; 12 288 x 4 096: 25 | 29),
+      - a long contraction into fewer outputs, 4 096 of them or more (4 480 x 15 680, 203 rows: 131 | 52; 4 480 x 5 120: 43 | 31; not 2 048 x 4 096, 96 rows:
+        12.6 | 14.1, 256: 16 | 21),
+      - the squared ReLU of more than 160 rows (its own pass saved; 15 680 x 4 480, with that pass, 96 rows 36 | 39, 160: 48 | 49, 203: 53 | 52, 256: 61 | 55).
+    Shorter contractions are the library's (6 144 x 2 048, 128 rows: 12 | 20)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     n = x.numel() // max(x.shape[-1], 1)
-    return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and 2 <= n <= MID_MAX and Kd >= 4096
-            and Kd % 64 == 0 and N % 4 == 0 and (n <= 64 or relu2 or 2048 <= N < Kd) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
+    pays = (not (N % 4096 == 0 and Kd <= N <= 12288) if n <= 64 else 4096 <= N < Kd or (relu2 and n > 160 and N >= 4096))
+    return (pays and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and 2 <= n <= MID_MAX
+            and Kd >= 4096 and Kd % 64 == 0 and N % 4 == 0 and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
             and weight.stride(0) < (1 << 22) and weight.data_ptr() % 16 == 0)
 
 
