@@ -620,7 +620,7 @@ int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int
  * tv_kv_append: k / v, one row of row_bytes per sequence, to position *pos (device) of the caches; all strides in bytes, everything a
  *   multiple of 16; a position outside [0, capacity) writes nothing.
  * tv_count_up: pos[0] += 1, lens[0..n) += 1.
- * tv_argmax_rows: out[r] = position of the largest of n fp32 values (NaN above all, the lowest of equals: torch.argmax). */
+ * tv_argmax_rows: out[r] = position of the largest of n <= 2^30 fp32 values (NaN above all, the lowest of equals: torch.argmax). */
 int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* pos, int batch, int64_t capacity,
                  int row_bytes, int64_t k_stride_b, int64_t v_stride_b, int64_t kc_stride_b, int64_t kc_stride_l, int64_t vc_stride_b,
                  int64_t vc_stride_l, void* stream);

@@ -39,6 +39,15 @@ def test_bad_arguments_fail_loudly_without_gpu():
     assert st == -2  # kernel width 7 unsupported
 
 
+def test_argmax_refuses_rows_beyond_its_positions():
+    """a row of nearly 2^31 values would step past the largest 32-bit position and read in front of the row"""
+    from timeviper_amd import _capi
+    lib = _capi.lib()
+    for n in ((1 << 30) + 1, (1 << 31) - 1):
+        st = lib.tv_argmax_rows(16, 16, 1, n, n, 16, 1 << 20, None)
+        assert st == -2 and b"2^30" in lib.tv_last_error()
+
+
 def test_product_path_has_no_cpu_fallback():
     import torch
     from timeviper_amd import kernels

@@ -93,6 +93,7 @@ extern "C" size_t tv_argmax_rows_workspace_bytes(int rows) { return rows > 0 ? (
 extern "C" int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int64_t stride, void* workspace, size_t workspace_bytes, void* stream) {
   TV_CHECK_ARG(x && out && workspace, "argmax_rows: null pointer");
   TV_CHECK_ARG(rows > 0 && rows <= 65535 && n > 0 && stride >= 0, "argmax_rows: rows %d, %d elements", rows, n);
+  if (n > (1 << 30)) TV_UNSUPPORTED("argmax_rows: %d elements a row, at most 2^30 (positions and the step behind the last share are 32-bit)", n);
   TV_CHECK_ARG(workspace_bytes >= tv_argmax_rows_workspace_bytes(rows) && ((uintptr_t)workspace & 7) == 0, "argmax_rows: workspace too small");
   const int wide = n % 4 == 0 && stride % 4 == 0 && ((uintptr_t)x & 15) == 0;
   argmax_part_kernel<<<dim3(ARG_BLOCKS, (unsigned)rows), 256, 0, (hipStream_t)stream>>>(x, (Best*)workspace, n, stride, wide);

@@ -825,7 +825,7 @@ def count_up(pos, lens) -> None:
 
 def argmax_rows(x):
     """x.argmax(-1); the fp32 logits of up to 65 535 rows by 64 work-groups a row."""
-    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] < (1 << 31)):
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] <= (1 << 30)):
         return x.argmax(-1)
     _gpu(x)
     lib, B = _capi.lib(), x.shape[0]
