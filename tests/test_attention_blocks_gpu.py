@@ -71,3 +71,13 @@ def test_packed_sequences_share_a_launch(K, counts, starts, window, keep):
         k, v = cache[s, :a + c].split([G * d, G * e], 1)
         want = reference(q[r:r + c], k.unflatten(1, (G, d)), v.unflatten(1, (G, e)), 0.11, a, window, keep)
         close(o[r:r + c], want * torch.sigmoid(gate[r:r + c].float()))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_more_query_blocks_than_a_grid_dimension(K, causal):
+    """20 480 000 (batch, head) pairs of one query: a key of its own is all that each sees"""
+    q, v = rnd((20000, 1, 1024, 8), 1), rnd((20000, 1, 1024, 8), 2)
+    o, lse = K.flash_attn_func(q, q, v, causal=causal, return_lse=True)
+    assert torch.equal(o, v)
+    want = (q[:, 0].float() ** 2).sum(-1) * 8 ** -0.5
+    assert (lse[:, :, 0] - want).abs().max() <= 1e-5 * want.abs().max()

@@ -78,7 +78,7 @@ struct AttnArgs {
   int64_t qsb, qsl, qsh, ksb, ksl, ksh, vsb, vsl, vsh, osb, osl, osh;
   float scale_log2;  // softmax_scale * log2(e)
   int causal;
-  int nqb, nb;       // nqb > 0: 1-D XCD-aware grid, nqb query blocks per (batch, head), nb batches; 0: 3-D grid
+  int nqb, nb;       // nqb > 0: many short sequences, nqb query blocks per (batch, head); 0: blocks dealt out by block_of; nb batches
   int ppx;           // streaming kernel: (batch, head) pairs per XCD
   int o16;           // streaming kernel: o rows are 16-byte aligned (wide epilogue stores)
   int Dv;            // value head dim (D unless the caller says otherwise)
@@ -986,6 +986,20 @@ int launch_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) 
 
 template <typename T>
 int launch_fa(const AttnArgs& a, int B, hipStream_t st) {
+  // One grid dimension takes fewer than 2^32 work-items: a batch with more query blocks than that goes in slices
+  const int64_t blocks = (int64_t)(a.Lq > 128 ? (a.Lq + 255) / 256 : 1) * a.Hq;      // of a batch entry, at most 512 work-items each
+  const int64_t most = blocks < (1 << 22) ? ((1 << 23) - 64) / blocks : 1;           // (pairs are padded to a multiple of 8 in one form)
+  if (B > most) {
+    for (int64_t b = 0; b < B; b += most) {
+      AttnArgs s = a;
+      s.q = (const T*)a.q + b * a.qsb; s.k = (const T*)a.k + b * a.ksb; s.v = (const T*)a.v + b * a.vsb; s.o = (T*)a.o + b * a.osb;
+      if (a.lse) s.lse = a.lse + b * a.Hq * a.Lq;
+      s.nb = (int)(B - b < most ? B - b : most);
+      const int rc = launch_fa<T>(s, s.nb, st);
+      if (rc != TV_OK) return rc;
+    }
+    return TV_OK;
+  }
   const int D = a.D > a.Dv ? a.D : a.Dv;
   if (D <= 64) return launch_fa_d<T, 4, 2>(a, B, st);
   if (D <= 80) return launch_fa_d<T, 5, 3>(a, B, st);
