@@ -104,6 +104,12 @@ def test_state_update_reads_slices_in_place(K, dtype, P, N):
     assert torch.equal(y, y2) and torch.equal(st, st2)
 
 
+def test_state_update_refuses_an_empty_batch(K):
+    z = lambda *s: torch.zeros(s, device=DEV)
+    with pytest.raises(K.TimeViperHipError):
+        K.selective_state_update(z(0, 2, 16, 16), z(0, 2, 16), z(0, 2), z(2), z(0, 1, 16), z(0, 1, 16))
+
+
 @pytest.mark.parametrize("B", [5, 17])
 def test_decode_step_of_many_sequences_is_the_general_one(K, B, monkeypatch):
     """5..32 sequences on tv_gemm_rows_fwd against torch.nn.Linear and the stand-alone operators: same rounding points"""

@@ -447,8 +447,7 @@ def selective_state_update(state, x, dt, A, B, C, D=None, z=None, dt_bias=None,
         (t if t.dim() == nd else t[(..., *([0] * (t.dim() - nd)))]).to(torch.float32).contiguous()
     A1, D1, b1 = head(A, 1), head(D, 1), head(dt_bias, 1)
     # slices of the mixer's projection are read in place (one row per sequence, dense behind the batch dimension)
-    rows = lambda t: t if all(t.stride(d) == t[0].numel() // math.prod(t.shape[1:d + 1]) for d in range(1, t.dim())) and t.data_ptr() % 16 == 0 \
-        and t.stride(0) % 8 == 0 else t.contiguous()
+    rows = lambda t: t if t.stride(1) == t.shape[2] and t.stride(2) == 1 and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 else t.contiguous()
     dt1 = (dt if dt.dim() == 2 else dt[..., 0]).to(x.dtype)
     dt1 = dt1 if dt1.stride(1) == 1 else dt1.contiguous()
     xc, Bc, Cc = rows(x), rows(B.to(x.dtype)), rows(C.to(x.dtype))
