@@ -40,6 +40,7 @@ HBM_PEAK_GBS = 8000.0                                      # MI355X_MICROARCH.md
 
 
 MFMA_BF16_PEAK_TFLOPS = 2500.0                             # dense bf16, MI355X_MICROARCH.md
+OWN_EPILOGUE = {0: "", 1: " + GELU", 2: " (+=)", 3: " + squared ReLU"}      # of kernels.linear_fused
 SCAN_SOURCES = ("ssd_head.hip", "ssd_head_step.inc", "ssd_slice.hip", "ssd_correct.hip", "ssd_scan.hip", "ssd_common.hpp", "conv1d.hip")
 
 
@@ -186,10 +187,10 @@ class OpTimers:
             return ("gelu", 2 * x.numel() * x.element_size())
         def gemm(x, weight, bias=None, epilogue=0, out=None):
             rows = x.numel() // x.shape[-1]
-            # USEFUL flops: zero-padded weight rows (so400m's fc1: 4 352 rows for 4 304 outputs) are not counted, nor is
-            # the activation.  (The padded rows are all-zero by construction: ZeroPaddedLinears.)
-            n_useful = getattr(weight, "_tv_useful_rows", weight.shape[0])
-            return ("gemm_fused", 2.0 * rows * n_useful * weight.shape[1])
+            # USEFUL flops: zero-padded weight rows (so400m's fc1: 4 352 rows for 4 304 outputs) and columns are not counted, nor is
+            # the activation.  (The padding is all-zero by construction: ZeroPaddedLinears.)
+            n, k = self._useful(weight)
+            return ("own:" + self._lib_role(weight) + OWN_EPILOGUE[epilogue], 2.0 * rows * n * k)
         self._wrap("linear_fused", gemm)
         self._wrap("mamba_chunk_scan_combined", scan)
         self._wrap("flash_attn_func", attn)
@@ -242,8 +243,8 @@ class OpTimers:
         # MI355X_MICROARCH.md) on this op, committed under profiles/ (PMC cannot be collected from
         # here).  The file names the kernel sources it was taken on: a ratio from other kernels is
         # refused, not silently reused.
-        traffic, src = None, "no profiles/r*_ssd_scan_traffic.json"
-        files = sorted((ROOT / "profiles").glob("r*_ssd_scan_traffic.json"))
+        traffic, src = None, "no profiles/*ssd_scan_traffic.json"
+        files = sorted((ROOT / "profiles").glob("*ssd_scan_traffic.json"))
         if files:
             tf = json.loads(files[-1].read_text())
             if tf.get("scan_source_id") == scan_source_id():
@@ -315,11 +316,11 @@ class OpTimers:
         out = [self.scan_roofline(bytes_per_token),
                self.mfma_roofline("attn_vit", "flash_fwd_vit_kernel (generated tile loop; other dtypes: flash_fwd_stream_kernel), ViT frames (non-causal, head_dim 72; useful FLOPs)"),
                self.mfma_roofline("attn_causal", "flash_fwd_kernel, causal GQA (LLM attention layers; useful FLOPs)")]
-        out.append(self.mfma_roofline("gemm_fused", "gemm_persist_kernel<bias + erf-GELU> (tv_gemm_bf16_fwd: ViT fc1 with the activation in "
-                                                    "the epilogue, persistent work-groups; useful GEMM FLOPs only: 4 304 of the "
-                                                    "4 352 zero-padded columns)"))
+        # hand-written GEMMs by role (useful FLOPs, as for the library's below)
+        for key in sorted(k for k in self.rec if k.startswith("own:")):
+            out.append(self.mfma_roofline(key, f"tv_gemm_bf16_fwd, role {key[4:]} (persistent work-groups; useful GEMM FLOPs only)"))
         out += self.patch_rooflines()
-        out += [self.hbm_roofline("conv", "conv1d_xbc_kernel + conv1d_bc_cb_kernel (tv_causal_conv1d_xbc_cb_fwd: conv + SiLU + "
+        out += [self.hbm_roofline("conv", "conv1d_xbc_cb_kernel (tv_causal_conv1d_xbc_cb_fwd: conv + SiLU + "
                                           "x|B|C split + causal C.B^T fragments; bytes: xBC read, x|B|C written)"),
                 self.hbm_roofline("gated_norm", "rmsnorm_gated_kernel (tv_rmsnorm_gated_fwd; bytes: y, gate read, out written)"),
                 self.mixer_trio_roofline(cfg) if cfg is not None else None,

@@ -1,6 +1,6 @@
-"""Dev tool: profiles/<tag>_ssd_scan_pmc.md and profiles/<tag>_ssd_scan_traffic.json from the rocprofv3 --pmc
+"""Dev tool: profiles/ssd_scan_pmc.md and profiles/ssd_scan_traffic.json from the rocprofv3 --pmc
 passes of pmc_scan.sh (gpurun_out/pmc_slice*/**/p_counter_collection.csv).
-usage: python timeviper_amd/devtools/summarize_pmc_scan.py r02 4 [tokens=163940]"""
+usage: python timeviper_amd/devtools/summarize_pmc_scan.py 0 [tokens=163940]"""
 import collections
 import csv
 import glob
@@ -13,8 +13,8 @@ ROOT = Path(__file__).resolve().parent.parent.parent
 sys.path.insert(0, str(ROOT))
 from bench import scan_source_id  # noqa: E402
 
-tag, impl = sys.argv[1], int(sys.argv[2])
-tokens = int(sys.argv[3]) if len(sys.argv) > 3 else 163940
+impl = int(sys.argv[1])
+tokens = int(sys.argv[2]) if len(sys.argv) > 2 else 163940
 KERNELS = ["ssd_head_asm_kernel", "ssd_head_kernel<5, 4, 2>", "ssd_slice_kernel", "ssd_cb_kernel",
            "ssd_correct_list_kernel", "ssd_correct_kernel", "ssd_chain_prefix_kernel", "ssd_seg_chain_kernel", "ssd_seg_combine_kernel", "ssd_chunk_decay_kernel",
            "ssd_decay_prefix_kernel", "ssd_dt_transpose_kernel"]
@@ -46,7 +46,7 @@ for k, m in mean.items():
         hbm[f"{k}_write"] = m["WRITE_SIZE"] * 1024
 hbm["total"] = sum(hbm.values())
 out = [f"# rocprofv3 --pmc passes on `python3 timeviper_amd/devtools/bench_ops.py --ops scan --model-dt --dt-std 1.3 --impl {impl}` "
-       f"({tokens} tokens, Nano-9B dims), {tag}\n",
+       f"({tokens} tokens, Nano-9B dims)\n",
        "One counter set per pass, no tracing (`timeviper_amd/devtools/pmc_scan.sh`); mean per launch, summed over the rows "
        "rocprofv3 reports per dispatch (`timeviper_amd/devtools/summarize_pmc_scan.py`).\n"]
 for k in KERNELS:
@@ -65,8 +65,8 @@ for k in KERNELS:
 out.append(f"\n## HBM traffic per tv_ssd_scan_fwd call\n\nalgorithmic bytes {alg / 1e9:.3f} GB; FETCH_SIZE (KiB) x 2 "
            f"(gfx950 correction, MI355X_MICROARCH.md) + WRITE_SIZE (KiB): {hbm['total'] / 1e9:.3f} GB = "
            f"**{hbm['total'] / alg:.3f} x algorithmic**.")
-(ROOT / "profiles" / f"{tag}_ssd_scan_pmc.md").write_text("\n".join(out) + "\n")
-(ROOT / "profiles" / f"{tag}_ssd_scan_traffic.json").write_text(json.dumps({
+(ROOT / "profiles" / "ssd_scan_pmc.md").write_text("\n".join(out) + "\n")
+(ROOT / "profiles" / "ssd_scan_traffic.json").write_text(json.dumps({
     "kernel": " + ".join(names[k] for k in KERNELS if k in names), "scan_impl": impl, "scan_source_id": scan_source_id(),
     "tokens": tokens, "algorithmic_bytes": alg, "hbm_bytes": hbm, "hbm_over_algorithmic": hbm["total"] / alg,
     "how": "rocprofv3 --pmc FETCH_SIZE / --pmc WRITE_SIZE (separate passes, timeviper_amd/devtools/pmc_scan.sh) on "
