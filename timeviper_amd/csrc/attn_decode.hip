@@ -293,20 +293,9 @@ __global__ __launch_bounds__(AD_D) void attn_decode_merge_kernel(DecArgs a) {
     a.lse[(int64_t)b * a.Hq + h] = nvalid > 0 ? (M + __log2f(L)) * 0.6931471805599453f : -INFINITY;
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 int pick_splits(int batch, int nheads_kv, int hblocks, int seqlen_k) {
   const int per = batch * nheads_kv * hblocks;
-  int want = (cu_count() + per - 1) / per;                          // one work-group per CU
+  int want = (tv_cu_count() + per - 1) / per;                          // one work-group per CU
   const int most = (seqlen_k + AD_NW * AD_STEP - 1) / (AD_NW * AD_STEP);          // >= one step per wave
   if (want > most) want = most;
   if (want > AD_MAX_SPLIT) want = AD_MAX_SPLIT;

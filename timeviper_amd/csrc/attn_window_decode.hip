@@ -258,17 +258,6 @@ __global__ __launch_bounds__(WD_MERGE) void attn_window_merge_kernel(WdArgs a) {
   }
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 // query heads a work-group serves (16 fill the columns of a product; at wide values their sums would not fit the LDS)
 int heads_per_group(int gq, int v_dim) { return gq > 8 && v_dim <= 128 ? 16 : gq > 4 ? 8 : gq > 2 ? 4 : gq; }
 
@@ -277,7 +266,7 @@ int pick_splits(int batch, int nheads_kv, int gq, int v_dim, int capacity, int w
   const int hpg = heads_per_group(gq, v_dim);
   const int64_t per = (int64_t)batch * nheads_kv * ((gq + hpg - 1) / hpg);
   const int64_t vis = (int64_t)window + keep < capacity ? (int64_t)window + keep : capacity;
-  int64_t rounds = vis * per / (WD_KEYS * 8ll * cu_count());
+  int64_t rounds = vis * per / (WD_KEYS * 8ll * tv_cu_count());
   const int64_t least = (vis + (int64_t)WD_KEYS * WD_MAX_SPLIT - 1) / ((int64_t)WD_KEYS * WD_MAX_SPLIT);
   if (rounds < least) rounds = least;
   return (int)((vis + WD_KEYS * rounds - 1) / (WD_KEYS * rounds));

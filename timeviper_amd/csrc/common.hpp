@@ -18,6 +18,17 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 
 #define TV_WAVE 64
 
+// compute units of the device (work-groups of one round)
+inline int tv_cu_count() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
+      cus = 256;                               // MI355X
+    return cus;
+  }();
+  return n;
+}
+
 // 16-byte vector of T (bf16/f16: 8 lanes, f32: 4 lanes).
 template <typename T> struct Vec16;
 template <> struct Vec16<float> { enum { N = 4 }; typedef f32x4 type; };

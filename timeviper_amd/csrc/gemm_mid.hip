@@ -289,17 +289,6 @@ int launch_one(const GmArgs& a, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 struct GmPlan {
   int ni, splits, xt;
 };
@@ -308,7 +297,7 @@ struct GmPlan {
 // fill and epilogue, per split 4 M N bytes written and read at 5 TB/s and a second launch.
 GmPlan plan(int M, int N, int K) {
   GmPlan best{4, 1, M <= 64 ? 2 : M <= 128 ? 4 : 8};
-  const int cus = cu_count(), nst = K / GM_KC;
+  const int cus = tv_cu_count(), nst = K / GM_KC;
   double least = 1e30;
   for (int ni = 4; ni >= 2; --ni)
     for (int s = 1; s <= 16 && s * 8 <= nst; ++s) {

@@ -391,23 +391,13 @@ int launch(const PArgs& pa, int grid, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
-    return cus;
-  }();
-  return n;
-}
-
 // tv_gemm_set_persist: mode -1 automatic (default; TV_GEMM_PERSIST=0 in the environment switches it off), 0 never, 1
 // wherever the shape allows it (tests: a few tiles per work-group on a small grid); grid 0 = one work-group per CU.
 int g_mode = -1, g_grid = 0;
 
 int grid_size() {
   static const int grid_env = [] { const char* e = getenv("TV_GEMM_PERSIST_GRID"); return e ? atoi(e) : 0; }();   // dev tool
-  int grid = g_grid > 0 ? g_grid : (grid_env > 0 ? grid_env : cu_count());
+  int grid = g_grid > 0 ? g_grid : (grid_env > 0 ? grid_env : tv_cu_count());
   grid = (grid / 8) * 8;
   return grid < 8 ? 8 : grid;
 }

@@ -215,21 +215,10 @@ int launch_xi(const SkArgs& a, int wi, int wgs, bool one, hipStream_t st) {
 #undef SK_GO
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 // Rows of W per work-group: the fewest rounds of one work-group per compute unit whose share is at most 32 rows, all shares alike
 // (4 480 rows: 18 in 249 work-groups; 9 in 498 read x twice as often, 24.0 against 22.7 us at K = 15 680).
 int rows_share(int64_t n, bool& one) {
-  const int cus = cu_count();
+  const int cus = tv_cu_count();
   const int64_t rounds = (n + 32ll * cus - 1) / (32ll * cus);
   one = rounds == 1;
   return (int)((n + rounds * cus - 1) / (rounds * cus));

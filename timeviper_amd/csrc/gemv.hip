@@ -798,17 +798,6 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_splitk_reg_kernel(GemvArgs a)
   }
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 // dev switches (A/B runs): TV_GEMV_NT = 0 plain loads of W; TV_GEMV_WGS = work-groups per CU (default 2)
 int gemv_nt() { static const int v = [] { const char* e = getenv("TV_GEMV_NT"); return e ? atoi(e) : 1; }(); return v; }
 int gemv_wgs() { static const int v = [] { const char* e = getenv("TV_GEMV_WGS"); return e ? atoi(e) : 2; }(); return v < 1 ? 1 : v; }
@@ -824,7 +813,7 @@ int launch_gemv_r(const GemvArgs& a, hipStream_t st) {
   }
   // two work-groups per CU; fewer when there are not R rows for each
   int wgs = (a.N + R - 1) / R;
-  const int most = gemv_wgs() * cu_count();
+  const int most = gemv_wgs() * tv_cu_count();
   if (wgs > most) wgs = most;
   gemv_bf16_kernel<PRO, MT, R, NB, NT, PF><<<dim3((unsigned)wgs), GV_THREADS, lds, st>>>(a);
   TV_LAUNCH_CHECK();
@@ -839,7 +828,7 @@ int launch_gemv_rows(const GemvArgs& a, hipStream_t st) {
     return TV_ERR_LAUNCH;
   }
   int wgs = (a.N + R * GV_WAVES - 1) / (R * GV_WAVES);            // >= one row group per wave, two work-groups per CU
-  const int most = gemv_wgs() * cu_count();
+  const int most = gemv_wgs() * tv_cu_count();
   if (wgs > most) wgs = most;
   gemv_rows_kernel<PRO, MT, NT, R, NB><<<dim3((unsigned)wgs), GV_THREADS, lds, st>>>(a);
   TV_LAUNCH_CHECK();
@@ -847,7 +836,7 @@ int launch_gemv_rows(const GemvArgs& a, hipStream_t st) {
 template <int PRO, bool NT>
 int launch_splitk_reg(const GemvArgs& a, hipStream_t st) {
   int wgs = (a.N + 1) / 2;
-  const int most = gemv_wgs() * cu_count();
+  const int most = gemv_wgs() * tv_cu_count();
   if (wgs > most) wgs = most;
   const int pw = a.K / 8 / GV_WAVES;                 // (reg_takes: K / 8 is a multiple of the four waves)
   if (pw == 64 * 5) gemv_splitk_reg_kernel<PRO, 2, 5, NT, true><<<dim3((unsigned)wgs), GV_THREADS, 0, st>>>(a);          // K = 10 240
@@ -869,7 +858,7 @@ template <int PRO, int MT>
 int launch_gemv_m(const GemvArgs& a, hipStream_t st) {
   static const int force = [] { const char* e = getenv("TV_GEMV_SPLITK"); return e ? atoi(e) : -1; }();    // (dev: 0 / 1)
   // (few long rows: a row per wave would leave half of the waves idle)
-  const bool few = PRO == PRO_NONE && a.K >= 4096 && a.N <= 2 * GV_WAVES * gemv_wgs() * cu_count();
+  const bool few = PRO == PRO_NONE && a.K >= 4096 && a.N <= 2 * GV_WAVES * gemv_wgs() * tv_cu_count();
   const bool splitk = a.conv_state ? false : (force >= 0 ? force != 0 : a.K >= 8192 || few);
   if constexpr (MT == 1 && (PRO == PRO_NONE || PRO == PRO_RELU2 || PRO == PRO_GATED)) {
     if (splitk && !a.y32 && reg_takes<PRO>(a)) return gemv_nt() ? launch_splitk_reg<PRO, true>(a, st) : launch_splitk_reg<PRO, false>(a, st);
@@ -1031,7 +1020,7 @@ extern "C" int tv_gemv_pair_fwd(const void* x, const void* x2, const void* W, co
   PairArgs a{(const bf16_t*)x, (const bf16_t*)x2, (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)y, (bf16_t*)act, M, n1, ff, K, 0,
              x_stride, x2_stride, ldw, y_stride, act_stride};
   // two work-groups per CU, shared out by rows; no more than there are groups for the waves
-  const int most = gemv_wgs() * cu_count(), g1 = (n1 + 1) / 2, need1 = (g1 + GV_WAVES - 1) / GV_WAVES, need2 = (ff + GV_WAVES - 1) / GV_WAVES;
+  const int most = gemv_wgs() * tv_cu_count(), g1 = (n1 + 1) / 2, need1 = (g1 + GV_WAVES - 1) / GV_WAVES, need2 = (ff + GV_WAVES - 1) / GV_WAVES;
   int w1 = need1, w2 = need2;
   if (w1 + w2 > most) {
     w1 = (int)((int64_t)most * g1 / (g1 + ff));

@@ -314,18 +314,8 @@ __global__ __launch_bounds__(LD_THREADS) void latent_out_kernel(LdArgs a) {
   }
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 int pick_splits(int batch, int groups, int capacity) {
-  int want = (2 * cu_count() + batch * groups - 1) / (batch * groups);       // two work-groups a compute unit
+  int want = (2 * tv_cu_count() + batch * groups - 1) / (batch * groups);       // two work-groups a compute unit
   const int most = (capacity + 2 * LD_TILE - 1) / (2 * LD_TILE);             // of at least two tiles: a split writes 2 H R floats
   if (want > most) want = most;
   if (want > LD_MAXSPLIT) want = LD_MAXSPLIT;

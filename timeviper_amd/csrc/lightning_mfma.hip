@@ -295,22 +295,12 @@ int launch_dims(const LmArgs& a, int nseq, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 }  // namespace
 
 // segments per sequence: one work-group per compute unit, at least 4 chunks each
 void tv_lightning_segments(int nseq, int nheads, int max_len, int* nseg, int* seglen) {
   const int chunks = (max_len + LM_Q - 1) / LM_Q;
-  int want = cu_count() / (nseq * nheads > 0 ? nseq * nheads : 1);
+  int want = tv_cu_count() / (nseq * nheads > 0 ? nseq * nheads : 1);
   if (want > (chunks + 3) / 4) want = (chunks + 3) / 4;
   if (want < 1) want = 1;
   const int per = (chunks + want - 1) / want;

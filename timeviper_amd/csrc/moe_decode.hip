@@ -156,16 +156,6 @@ __global__ __launch_bounds__(MD_THREADS) void moe_decode_down_kernel(MdArgs a) {
   }
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 }  // namespace
 }  // namespace tvmoe
 
@@ -185,7 +175,7 @@ extern "C" int tv_moe_decode_fwd(const float* logits, const void* correction, co
   hipStream_t st = (hipStream_t)stream;
   // about two work-groups a compute unit over all choices; at least two rows a wave
   auto wgs = [&](int rows, int groups) {
-    int w = (2 * cu_count() + groups - 1) / groups;
+    int w = (2 * tv_cu_count() + groups - 1) / groups;
     const int most = (rows + 2 * MD_WAVES - 1) / (2 * MD_WAVES);
     if (w > most) w = most;
     return w < 1 ? 1 : w;

@@ -1233,24 +1233,13 @@ int pick_segments(int batch, int nheads, int nchunks) {
   return nseg < 1 ? 1 : nseg;
 }
 
-int cu_count() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-      cus = 256;                               // MI355X
-    return cus;
-  }();
-  return n;
-}
-
 // Short sequences: column slices (ssd_cols.hip) while their work-groups (4 slices) all run at once and the march over them is no longer than
 // segments would make it.  128 heads x 80, 8 groups, whole operator, one segment | best number of segments | slices: 203 tokens 35 | 51 |
 // 17 us, 512: 56 | 59 | 29, 1 501: 146 | 89 | 83 - 93, 2 048: 180 | 98 | 107, 3 000: 244 | 113 | 128.
 bool use_cols(int batch, int nheads, int headdim, int ngroups, int nchunks) {
   if (ngroups < 1 || nchunks < 1) return false;
   const int slices = nheads / ngroups * (headdim / 16);        // of a group
-  return nchunks <= 24 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= cu_count();
+  return nchunks <= 24 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= tv_cu_count();
 }
 
 struct HeadLayout {
