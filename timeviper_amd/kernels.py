@@ -257,6 +257,7 @@ def rmsnorm_fn(x, weight, bias=None, z=None, eps=1e-6, group_size=None,
 
 
 # ------------------------------------------------------------------- linears with fused epilogues
+CUS = 256            # compute units of an MI355X: work-groups of one round
 GEMM_BIAS, GEMM_BIAS_GELU, GEMM_ACCUM, GEMM_BIAS_RELU2 = 0, 1, 2, 3
 
 
@@ -587,7 +588,8 @@ def gemv_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=None, norm_weight=None, eps=0.0,
                gate=None, group_size=0, conv=None):
     """y = f(x) @ weight.T (+ bias) for 1..4 rows — the linear layers of a decode step (torch.nn.Linear at q_len 1) with
-    the single-row operator in front of them computed in the kernel's prologue: GEMV_RMSNORM (NemotronHRMSNorm with the
+    the operator in front of them computed in the kernel's prologue (several rows: mostly as a launch in front of a product on the matrix cores,
+    see below): GEMV_RMSNORM (NemotronHRMSNorm with the
     block's residual add: `delta` is added to x first, the sum goes to `sum_out`), GEMV_RELU2 (the MLP activation),
     GEMV_GATED (MambaRMSNormGated with `gate`), rounding where the stand-alone operators round.
     `conv=(conv_state, weight, bias, row0)`: the outputs [row0, row0 + C) go through `causal_conv1d_update` (width 4,
@@ -761,10 +763,9 @@ def large_takes(x, weight, relu2=False) -> bool:
             and Kd % 128 == 0 and N % 8 == 0 and 256 <= N < (1 << 22) and x.is_contiguous() and weight.is_contiguous()
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
         return False
-    cus = 256                                                  # of an MI355X
     tiles = -(-rows // 256) * -(-N // 256)
-    fill = tiles / (-(-tiles // cus) * cus)
-    if tiles <= cus or not gemm_persist_on():
+    fill = tiles / (-(-tiles // CUS) * CUS)
+    if tiles <= CUS or not gemm_persist_on():
         return False
     if relu2:
         return fill >= 0.75 and Kd <= 8192

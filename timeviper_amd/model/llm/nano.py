@@ -291,8 +291,8 @@ class HybridMambaAttentionDynamicCache(StaticDecode):
 
 # ------------------------------------------------------------------ decode-step helpers
 def _fused_decode(x: torch.Tensor) -> bool:
-    """The linear layers of a decode step (1..4 rows) run on tv_gemv_bf16_fwd with the operator in front of them in
-    the prologue; TV_DECODE_FUSED=0 keeps torch.nn.Linear + the stand-alone kernels (same arithmetic, library GEMV)."""
+    """The linear layers of a decode step (1..4 rows) run through `gemv_fused` with the operator in front of them (one row: in
+    the prologue); TV_DECODE_FUSED=0 keeps torch.nn.Linear + the stand-alone kernels (same arithmetic, library GEMV)."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 4
             and not torch.is_grad_enabled() and os.environ.get("TV_DECODE_FUSED", "1") != "0")
 
@@ -468,9 +468,9 @@ class NemotronHMamba2Mixer(nn.Module):
                 and all(plain_linear(m, x) and K.rows_weight(m.weight) for m in (self.in_proj, self.out_proj)))
 
     def decode_fused(self, hidden, delta, norm, cache_params):
-        """One decode token with the block's RMSNorm (+ residual add) inside in_proj and the gated norm inside out_proj:
-        in_proj (+ conv update in its epilogue) -> state update -> out_proj, 3 launches.  Returns (residual stream, mixer output).
-        More than four sequences: the norms as launches of their own."""
+        """One decode token: in_proj (+ conv update in its epilogue) -> state update -> out_proj.  One sequence: the block's RMSNorm
+        (+ residual add) inside in_proj and the gated norm inside out_proj, 3 launches.  More: the norms as launches of their own (up to four
+        inside `gemv_fused`).  Returns (residual stream, mixer output)."""
         B = hidden.shape[0]
         rows = B > 4
         if rows:
@@ -533,8 +533,8 @@ class NemotronHMLP(nn.Module):
                 and all(plain_linear(m, x) and K.rows_weight(m.weight) for m in (self.up_proj, self.down_proj)))
 
     def decode_fused(self, hidden, delta, norm):
-        """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches (more than four sequences: 3,
-        relu^2 behind up_proj)."""
+        """One decode token: RMSNorm (+ residual add) inside up_proj, relu^2 inside down_proj — 2 launches.  Two to four sequences: each as a
+        launch of its own inside `gemv_fused`; more: 3 launches, relu^2 behind up_proj."""
         if hidden.shape[0] > 4:
             normed, new_hidden = _norm_add(norm, hidden, delta)
             u = K.rows_linear(normed, self.up_proj.weight, self.up_proj.bias, relu2=True)
@@ -603,8 +603,8 @@ class NemotronHAttention(nn.Module):
                 and all(plain_linear(m, x) and m.weight.dtype == x.dtype for m in (self.q_proj, self.k_proj, self.v_proj)))
 
     def decode_fused(self, hidden, delta, norm, cache):
-        """One decode token: the block's RMSNorm (+ residual add) in the prologue of ONE q / k / v product, cache append,
-        split-KV attention, o_proj — 4 launches + the cache writes, against 7."""
+        """One decode token: the block's RMSNorm (+ residual add) in the prologue of ONE q / k / v product (several sequences: in front of
+        it), cache append, split-KV attention, o_proj — 5 launches, against 9."""
         B = hidden.shape[0]
         nq, nkv = self.num_heads * self.head_dim, self.num_key_value_heads * self.head_dim
         if B > 4:

@@ -95,7 +95,7 @@ class ParallelLayer(nn.Module):
         return all(K.gemv_rows_take(rows, n, dtype) for n in (self.shift.numel(), self.out.shape[1], self.side.dim)) and self.k1 % 8 == 0
 
     def decode(self, x, pending, ids, side_rows, state, kv_rows, plan):
-        """The same for a few single tokens on matrix-vector kernels: both input products and the activation in one launch, the residual
+        """The same for a few single tokens (one: matrix-vector kernels; up to 32: the matrix cores): both input products and the activation in one launch, the residual
         add behind the output product."""
         y, w = pending or (None, None)
         x, h, hs = K.norm_shift(x, self.gain, self.eps, y, w, self.shift, state, plan, need_h=self.mlp is not None)

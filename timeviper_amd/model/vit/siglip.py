@@ -64,9 +64,6 @@ class PatchEmbed(nn.Module):
 GEMM_ALIGN = 256     # hipBLASLt's bf16 macro-tile on gfx950
 
 
-CUS = 256            # compute units of an MI355X: work-groups of one round
-
-
 def _tiles(rows: int, n: int, width: int = 256) -> int:
     """256-row output tiles of a (rows, n) product"""
     return -(-rows // 256) * -(-n // width)
@@ -133,8 +130,7 @@ class Attention(nn.Module):
         """qkv projection + attention, without the output projection"""
         B, N, C = x.shape
         if self._own_qkv(x):
-            # the persistent GEMM (csrc/gemm_persist.hip) on the weights as stored: 3 456 columns are 13 tiles and one
-            # shifted back — no padded copies, and the bias is added in the kernel's epilogue
+            # on the weights as stored: 3 456 columns are 13 tiles and one shifted back — no padded copies
             qkv = K.linear_fused(x, self.qkv.weight, self.qkv.bias, epilogue=K.GEMM_BIAS)
             qkv = qkv.view(B, N, 3, self.num_heads, self.head_dim)
         elif ZeroPaddedLinears.wanted(x, 3 * C):
@@ -159,10 +155,10 @@ class Attention(nn.Module):
         on; 0: never.  bf16 on the GPU, inference, K a multiple of 128, N of 8."""
         w, rows = self.qkv.weight, x.numel() // x.shape[-1]
         tiles = _tiles(rows, w.shape[0])
-        rounds = -(-tiles // CUS)
+        rounds = -(-tiles // K.CUS)
         switch = os.environ.get("TV_VIT_OWN_QKV", "")
         own = switch != "0" and ((switch == "1" and rows >= 65536) or (
-            2 <= rounds <= 6 and 4 * tiles >= 3 * rounds * CUS and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
+            2 <= rounds <= 6 and 4 * tiles >= 3 * rounds * K.CUS and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
         return bool(own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
                 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and _gemm_reads(x, w, self.qkv.bias))
 
@@ -199,14 +195,13 @@ class Mlp(nn.Module):
         return h, w2
 
     def _fused_fc1(self, x, w1, b1) -> bool:
-        """fc1 + bias + exact GELU in ONE kernel (csrc/gemm_persist.hip from 4 tiles per compute unit on, csrc/gemm.hip
-        below: the activation is applied to the accumulators, same rounding points as GEMM-then-GELU): 14.0 ms
-        (persistent) / 14.8 ms (per tile) against 16.7 ms for hipBLASLt + tv_gelu_fwd per 2 048 SigLIP frames.  bf16 on the GPU, inference, K
+        """fc1 + bias + exact GELU in ONE kernel (csrc/gemm_persist.hip: the activation is applied to the accumulators, same
+        rounding points as GEMM-then-GELU): 14.0 ms against 16.7 ms for hipBLASLt + tv_gelu_fwd per 2 048 SigLIP frames.  bf16 on the GPU, inference, K
         a multiple of 128, tiles for three quarters of the compute units (4 frames, 204 tiles: library + GELU 42 us, fused 41; 3 frames, 153:
-        34 and 39); TV_VIT_FUSED_FC1=0 switches it off."""
+        34 and 39; 1 024 x 4 096: 192 tiles 37 and 38, 240: 42 and 40); TV_VIT_FUSED_FC1=0 switches it off."""
         return (self.exact_gelu and x.is_cuda and x.dtype == torch.bfloat16 and w1.dtype == torch.bfloat16
                 and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0 and _gemm_reads(x, w1, b1)
-                and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
+                and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * K.CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
 
     def forward(self, x):
         h, w2 = self.hidden(x)
@@ -222,7 +217,7 @@ def _own_accumulate(rows: int, n: int) -> bool:
     of a kernel; of 40 clip lengths in the range five lose, 2 - 5 %)."""
     if rows > 131072 or n % GEMM_ALIGN == 0:
         return False
-    fill = max(t / (-(-t // CUS) * CUS) for t in (_tiles(rows, n), _tiles(rows, n, 192)))
+    fill = max(t / (-(-t // K.CUS) * K.CUS) for t in (_tiles(rows, n), _tiles(rows, n, 192)))
     return fill >= 0.63
 
 
