@@ -58,6 +58,15 @@ def test_subclasses_of_the_module_and_of_its_tensors():
     assert not plain_linear(lin, X)
 
 
+def test_tensors_that_are_no_longer_its_parameters():
+    for name in ("weight", "bias"):
+        lin = linear()
+        t = getattr(lin, name).detach()
+        delattr(lin, name)
+        setattr(lin, name, t)
+        assert not plain_linear(lin, X)
+
+
 def test_biases_of_another_dtype():
     lin = linear()
     lin.bias = nn.Parameter(lin.bias.detach().double())
