@@ -146,19 +146,17 @@ class Attention(nn.Module):
 
     def _own_qkv(self, x) -> bool:
         """qkv projection + bias on the hand-written persistent GEMM instead of hipBLASLt: widths that the library needs a padded copy
-        for, where the 256 x 256 tiles are two to six rounds of the compute units and fill them to three quarters, and the rows are no
-        multiple of 256 (the library's own tile: it does not lose there).  Library on the padded copy | persistent, us, SigLIP so400m of 729 tokens a
-        frame: 15 frames 106 | 89, 18: 112 | 98, 20: 149 | 118, 24: 145 | 128, 33: 211 | 181, 38: 204 | 192; the library's choice of a kernel varies, so that some in
-        between lose 1 - 6 % (11: 59 | 63, 23: 122 | 126, 28: 149 | 155).  Fewer tiles in the last round: 8 frames (63 %) 51 | 57, 14 (73 %) 81 | 87.  One round: 5
-        frames 31 | 33; more than six: 41 211 | 216, 64 326 | 333, and 0.5 % of a 10 240-frame forward.  256 tokens a frame: 32 frames 59 | 62, 96 175 | 181.  Whole
-        tiles of columns: 2 304 (K 768), 9 216 rows 39 | 42; 3 072 (K 1 024), 6 264 rows 43 | 52.  TV_VIT_OWN_QKV=1: also from 65 536 rows
-        on; 0: never.  bf16 on the GPU, inference, K a multiple of 128, N of 8."""
+        for, where the 256 x 256 tiles are two to six rounds of the compute units and the rows are no multiple of 256 (the library's own tile).  Inside the
+        SigLIP so400m forward, 729 tokens a frame, us a layer won (all in turn on one box): 7 frames 6, 9: 11, 13: 9, 15: 16, 20: 54, 24: 25, 32: 25, 36: 12; level at 10
+        - 14, 19, 21, 26; lost at 8 (3) and 28 (6), as the library's choice of a kernel varies.  One round: 5 frames level, 6 1; more than six: 39 to 42 lost 12 - 18,
+        and 0.5 % of a 10 240-frame forward.  Alone, library on the padded copy | persistent: 256 tokens a frame, 32 frames 59 | 62, 96 175 | 181; whole tiles of
+        columns: 2 304 (K 768), 9 216 rows 39 | 42; 3 072 (K 1 024), 6 264 rows 43 | 52.  TV_VIT_OWN_QKV=1: also from 65 536 rows on; 0: never.  bf16 on the
+        GPU, inference, K a multiple of 128, N of 8."""
         w, rows = self.qkv.weight, x.numel() // x.shape[-1]
-        tiles = _tiles(rows, w.shape[0])
-        rounds = -(-tiles // K.CUS)
+        rounds = -(-_tiles(rows, w.shape[0]) // K.CUS)
         switch = os.environ.get("TV_VIT_OWN_QKV", "")
         own = switch != "0" and ((switch == "1" and rows >= 65536) or (
-            2 <= rounds <= 6 and 4 * tiles >= 3 * rounds * K.CUS and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
+            2 <= rounds <= 6 and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
         return bool(own and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.qkv.bias is not None
                 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and _gemm_reads(x, w, self.qkv.bias))
 
