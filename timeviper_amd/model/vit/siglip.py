@@ -211,8 +211,8 @@ def _own_accumulate(rows: int, n: int) -> bool:
     the compute units to 63 % or more, up to 131 072 rows, and the width is no multiple of the library's 256 (768, K 3 072: 10 368 rows 48 | 56,
     73 728 313 | 339).  us, library | own, SigLIP so400m, proj (K 1 152): 9 frames 26 | 27 (61 %), 10: 34 | 28
     (68 %), 16: 50 | 37, 18: 46 | 53 (61 %), 26: 93 | 58, 33: 96 | 79, 48: 156 | 111, 128: 335 | 273; fc2 (K 4 352): 10: 79 | 75, 16: 112 | 101, 18: 127 |
-    153, 26: 228 | 169, 33: 220 | 212, 45: 301 | 320, 48: 404 | 323, 88: 549 | 568, 128: 847 | 836, 256: 1 599 | 1 663 (the library's times jump with its choice
-    of a kernel; of 40 clip lengths in the range five lose, 2 - 5 %)."""
+    153, 26: 228 | 169, 33: 220 | 212, 45: 301 | 320, 48: 404 | 323, 88: 549 | 568, 128: 847 | 836, 256: 1 599 | 1 663   The library's times jump with its choice
+    of a kernel: inside the forward fc2 wins 3.5 - 4 % of it at 46, 47, 64 and 72 frames and loses 1 - 2.5 % at 43 - 45, 56, 80 and 88."""
     if rows > 131072 or n % GEMM_ALIGN == 0:
         return False
     fill = max(t / (-(-t // K.CUS) * K.CUS) for t in (_tiles(rows, n), _tiles(rows, n, 192)))
