@@ -62,7 +62,7 @@ __device__ __forceinline__ bool conv_place(const ConvArgs& a, int block, int c_e
 }
 
 // One lane's strip of CONV_TL rows from t0 on, of a sequence of L: all its rows and the K-1 in front of it are in flight before the
-// arithmetic; rows past the end repeat the last one and are not stored.  FAST: SiLU with the reciprocal instruction (the mixer's convolution).
+// arithmetic; rows past the end repeat the last one and are left out of it.  FAST: SiLU with the reciprocal instruction (the mixer's convolution).
 template <typename T, int K, bool FAST>
 __device__ __forceinline__ void conv_strip(const ConvArgs& a, int c0, int t0, int b, T* __restrict__ yb, int64_t ysl) {
   constexpr int V = Vec16<T>::N;
@@ -88,6 +88,7 @@ __device__ __forceinline__ void conv_strip(const ConvArgs& a, int c0, int t0, in
     for (int i = 0; i < V; ++i) win[j][i] = to_f32(v[j][i]);
 #pragma unroll
   for (int u = 0; u < CONV_TL; ++u) {
+    if (t0 + u >= a.L) break;                      // (the same for all lanes; one row of 4 096 channels 5.3 us with all eight computed)
     vec_t ov;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
@@ -100,7 +101,7 @@ __device__ __forceinline__ void conv_strip(const ConvArgs& a, int c0, int t0, in
 #pragma unroll
       for (int j = 0; j < K - 1; ++j) win[j][i] = win[j + 1][i];
     }
-    if (t0 + u < a.L) *(vec_t*)(yb + (int64_t)(t0 + u) * ysl) = ov;
+    *(vec_t*)(yb + (int64_t)(t0 + u) * ysl) = ov;
   }
 }
 
