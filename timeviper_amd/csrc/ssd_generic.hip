@@ -197,8 +197,8 @@ __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restri
                                                                         const T* __restrict__ Bm, const T* __restrict__ Cm,
                                                                         const float* __restrict__ D,
                                                                         const float* __restrict__ dt_bias, T* __restrict__ y,
-                                                                        int H, int P, int G, int64_t xs, int64_t ds, int64_t bs,
-                                                                        int64_t cs, int softplus, int rows_total) {
+                                                                        int H, int P, int G, int xd, int dd, int bd,
+                                                                        int cd, int softplus, int rows_total) {
   constexpr int N = 4 * LPR, RPW = 64 / LPR, IT = 1, WAVES = 4;      // IT: state rows per lane group in flight
   typedef typename std::conditional<std::is_same<T, float>::value, f32x4, typename std::conditional<std::is_same<T, bf16_t>::value, bf16x4, f16x4>::type>::type vec4_t;
   const int lane = threadIdx.x & 63;
@@ -218,13 +218,15 @@ __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restri
     const int h = bh - b * H;
     const int g = (int)((unsigned)h / (unsigned)hpg);
     sv[it] = __builtin_nontemporal_load((const f32x4*)(state + (int64_t)rc * N) + ln);
-    dtv[it] = to_f32(dt[b * ds + h]);
-    xr[it] = to_f32(x[b * xs + (rc - b * H * P)]);
+    // xd, dd, bd, cd: how much further apart than dense the sequences lie (32-bit offsets: launcher)
+    const int bc = (b * G + g) * N + 4 * ln;
+    dtv[it] = to_f32(dt[bh + b * dd]);
+    xr[it] = to_f32(x[rc + b * xd]);
     av[it] = A[h];
     bv[it] = dt_bias ? dt_bias[h] : 0.f;
     dv[it] = D ? D[h] : 0.f;
-    Bv[it] = *(const vec4_t*)(Bm + b * bs + g * N + 4 * ln);
-    Cv[it] = *(const vec4_t*)(Cm + b * cs + g * N + 4 * ln);
+    Bv[it] = *(const vec4_t*)(Bm + bc + b * bd);
+    Cv[it] = *(const vec4_t*)(Cm + bc + b * cd);
   }
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -295,15 +297,23 @@ extern "C" int tv_selective_state_update_rows(void* state, const void* x, const 
   hipStream_t s = (hipStream_t)stream;
   // d_state 16 / 32 / 64 / 128 / 256 with 16-byte aligned rows: lanes share a row (coalesced); anything else: a thread per row
   const int lpr = dstate / 4;
+  // a sequence's row (`dense` elements) and every offset up to it in 32 bits
+  auto near = [&](int64_t stride, int64_t dense) {
+    const int64_t far = stride < 0 ? -stride : stride;
+    return (int64_t)batch * (far > dense ? far : dense) < (1ll << 30);
+  };
   if (dstate % 4 == 0 && (lpr == 4 || lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64) && (((uintptr_t)state) & 15) == 0 &&
-      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && b_stride % 4 == 0 && c_stride % 4 == 0 && (int64_t)batch * nheads * headdim < (1ll << 31)) {
+      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && b_stride % 4 == 0 && c_stride % 4 == 0 && (int64_t)batch * nheads * headdim < (1ll << 31) &&
+      near(x_stride, (int64_t)nheads * headdim) && near(dt_stride, nheads) && near(b_stride, (int64_t)ngroups * dstate) &&
+      near(c_stride, (int64_t)ngroups * dstate)) {
     const int64_t rows = (int64_t)batch * nheads * headdim;
     const int64_t rows_per_block = 4 * (64 / lpr);              // 4 waves x rows per wave-instruction
     const dim3 rgrid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
 #define TV_SUR(T, LPR)                                                                                        \
     state_update_chain_kernel<T, LPR><<<rgrid, 256, 0, s>>>((float*)state, (const T*)x, (const T*)dt,         \
         (const float*)A, (const T*)Bm, (const T*)Cm, (const float*)D, (const float*)dt_bias, (T*)y, nheads,   \
-        headdim, ngroups, x_stride, dt_stride, b_stride, c_stride, dt_softplus, (int)rows)
+        headdim, ngroups, (int)(x_stride - (int64_t)nheads * headdim), (int)(dt_stride - nheads),                   \
+        (int)(b_stride - (int64_t)ngroups * dstate), (int)(c_stride - (int64_t)ngroups * dstate), dt_softplus, (int)rows)
 #define TV_SUR_T(T)                                                                                           \
     switch (lpr) { case 4: TV_SUR(T, 4); break; case 8: TV_SUR(T, 8); break; case 16: TV_SUR(T, 16); break;     \
                    case 32: TV_SUR(T, 32); break; default: TV_SUR(T, 64); break; }
