@@ -100,8 +100,11 @@ struct NoSeqs {};
 // grows with its position, so the blocks of all heads are dealt out by falling cost (a grid that finishes one head after
 // the other ends with the last heads' heaviest blocks running alone: 40 heads x 5 003 tokens 402 us, dealt out 309; 10 007 tokens: 1 475, 1 215).
 // An XCD (id % 8) gets a contiguous range of the pairs in every round, about the same one: heads that share K / V share an L2.
+// SCALAR: the quotient, and with it all addresses, in scalar registers (a division leaves it in a vector register): 64 rows against 4 064 keys, 16
+// heads on 4 x 128, windowed: 58.4 us, so 57.2; the plain kernels have no scalar registers to spare (16 x 16 000: 461, so 472).
+template <bool SCALAR>
 __device__ __forceinline__ void block_of(int id, int pairs, int& t, int& pair) {
-  t = id / pairs;
+  t = SCALAR ? __builtin_amdgcn_readfirstlane(id / pairs) : id / pairs;
   const int p = id - t * pairs, q = pairs >> 3, rem = pairs & 7;
   const int x0 = (id - p) & 7, x = id & 7;             // XCD of the round's first work-group, and of this one
   // an XCD gets q pairs of a round, the `rem` XCDs from x0 on (modulo 8) one more: those in front of XCD x
@@ -140,14 +143,14 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 31, hh = lane >> 5;
-  // 1-D grid.  Few sequences: `block_of` (causal: the heaviest query blocks of all heads first).  Many short sequences (ViT
+  // 1-D grid (but for NW = 4).  Few sequences: `block_of` (causal: the heaviest query blocks of all heads first).  Many short sequences (ViT
   // frames): ids walk the query blocks of ONE (batch, head) on one XCD (id % 8): the blocks that
   // share K / V then share an L2 instead of pulling the same keys into three of them
   int qblk, h, b, Lq = a.Lq, Lk = a.Lk;
   int64_t row0 = 0;                             // WIN: the sequence's first row of q, o and gate
   if constexpr (WIN) {
     int t;
-    block_of(blockIdx.x, a.Hq, t, h);
+    block_of<true>(blockIdx.x, a.Hq, t, h);
     int s = 0, nblk;
     for (;; ++s) {                              // (t is below the sum of the sequences' blocks: launcher)
       nblk = (sq.len_q[s] + QB - 1) / QB;
@@ -168,15 +171,19 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     h = pair % a.Hq;
     b = pair / a.Hq;
     if (b >= a.nb) return;                    // (batch, head) pairs are padded to a multiple of 8
+  } else if constexpr (NW == 4) {               // up to 128 query rows: one block, a 3-D grid with heads and batch entries
+    qblk = a.causal ? (gridDim.x - 1 - blockIdx.x) : blockIdx.x;
+    h = blockIdx.y;
+    b = blockIdx.z;
   } else {
     const int pairs = a.nb * a.Hq;
     int pair;
-    block_of(blockIdx.x, pairs, qblk, pair);
+    block_of<false>(blockIdx.x, pairs, qblk, pair);
     if (a.causal) qblk = (a.Lq + QB - 1) / QB - 1 - qblk;
     b = a.nb == 1 ? 0 : pair / a.Hq;           // (a division is 30 instructions of a short call)
     h = pair - b * a.Hq;
   }
-  const int hk = h / (a.Hq / a.Hkv);
+  const int hk = WIN ? __builtin_amdgcn_readfirstlane(h / (a.Hq / a.Hkv)) : h / (a.Hq / a.Hkv);
   const int q0 = qblk * QB + wave * FA_QW;      // first query row of this wave
   const int qrow = q0 + r;                      // this lane's query row
   const int D = a.D;
@@ -933,7 +940,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e == hipSuccess) {
-      flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3((unsigned)((int64_t)((a.Lq + 127) / 128) * a.Hq * B)), 256, lds, st>>>(a, NoSeqs{});
+      flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
     }
   }
   if (e != hipSuccess) {
@@ -976,9 +983,9 @@ int launch_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) 
 template <typename T>
 int launch_fa(const AttnArgs& a, int B, hipStream_t st) {
   // One grid dimension takes fewer than 2^32 work-items: a batch with more query blocks than that goes in slices
-  const int64_t blocks = (int64_t)(a.Lq > 128 ? (a.Lq + 255) / 256 : 1) * a.Hq;      // of a batch entry, at most 512 work-items each
+  const int64_t blocks = (int64_t)((a.Lq + 255) / 256) * a.Hq;                        // of a batch entry, 512 work-items each
   const int64_t most = blocks < (1 << 22) ? ((1 << 23) - 64) / blocks : 1;           // (pairs are padded to a multiple of 8 in one form)
-  if (B > most) {
+  if (a.Lq > 128 && B > most) {
     for (int64_t b = 0; b < B; b += most) {
       AttnArgs s = a;
       s.q = (const T*)a.q + b * a.qsb; s.k = (const T*)a.k + b * a.ksb; s.v = (const T*)a.v + b * a.vsb; s.o = (T*)a.o + b * a.osb;
