@@ -104,6 +104,21 @@ def test_state_update_reads_slices_in_place(K, dtype, P, N):
     assert torch.equal(y, y2) and torch.equal(st, st2)
 
 
+@pytest.mark.parametrize("B,far", [(1, (0, 1, 2, 3)), (3, (0,)), (3, (1,)), (3, (2,)), (3, (3,))])
+def test_state_update_of_one_sequence_and_of_single_operands_apart(K, B, far):
+    """x, dt, B, C (by number) with sequences further apart than dense, the others dense; one sequence has no distance"""
+    H, G, P, N = 6, 2, 80, 128
+    g = torch.Generator(device=DEV).manual_seed(2)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    widths = (H * P, H, G * N, G * N)
+    flat = [r(B, n + 8 * (i in far)).bfloat16()[:, :n] for i, n in enumerate(widths)]
+    A, D, bias, st = -torch.rand(H, generator=g, device=DEV) - 0.1, r(H), r(H), r(B, H, P, N)
+    st2 = st.clone()
+    step = lambda s, t: K.selective_state_update(s, t[0].unflatten(1, (H, P)), t[1], A, t[2].unflatten(1, (G, N)), t[3].unflatten(1, (G, N)), D,
+                                                 dt_bias=bias, dt_softplus=True)
+    assert torch.equal(step(st, flat), step(st2, [t.contiguous() for t in flat])) and torch.equal(st, st2)
+
+
 def test_state_update_refuses_an_empty_batch(K):
     z = lambda *s: torch.zeros(s, device=DEV)
     with pytest.raises(K.TimeViperHipError):

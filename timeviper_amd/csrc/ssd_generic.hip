@@ -191,7 +191,9 @@ __device__ __forceinline__ float group_sum_dpp(float v) {      // valid in the l
   return v;
 }
 
-template <typename T, int LPR>
+// DENSE: the sequences lie one behind the other (or there is one): no distances to add in front of the loads (100 sequences of 128 heads x 80 x 128
+// 205.9 -> 202.3 us, 4: 10.64 -> 10.48, 100 of 32 x 64 x 16 7.92 -> 7.81)
+template <typename T, int LPR, bool DENSE>
 __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restrict__ state, const T* __restrict__ x,
                                                                         const T* __restrict__ dt, const float* __restrict__ A,
                                                                         const T* __restrict__ Bm, const T* __restrict__ Cm,
@@ -220,13 +222,13 @@ __global__ __launch_bounds__(256) void state_update_chain_kernel(float* __restri
     sv[it] = __builtin_nontemporal_load((const f32x4*)(state + (int64_t)rc * N) + ln);
     // xd, dd, bd, cd: how much further apart than dense the sequences lie (32-bit offsets: launcher)
     const int bc = (b * G + g) * N + 4 * ln;
-    dtv[it] = to_f32(dt[bh + b * dd]);
-    xr[it] = to_f32(x[rc + b * xd]);
+    dtv[it] = to_f32(dt[bh + (DENSE ? 0 : b * dd)]);
+    xr[it] = to_f32(x[rc + (DENSE ? 0 : b * xd)]);
     av[it] = A[h];
     bv[it] = dt_bias ? dt_bias[h] : 0.f;
     dv[it] = D ? D[h] : 0.f;
-    Bv[it] = *(const vec4_t*)(Bm + bc + b * bd);
-    Cv[it] = *(const vec4_t*)(Cm + bc + b * cd);
+    Bv[it] = *(const vec4_t*)(Bm + bc + (DENSE ? 0 : b * bd));
+    Cv[it] = *(const vec4_t*)(Cm + bc + (DENSE ? 0 : b * cd));
   }
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -297,23 +299,27 @@ extern "C" int tv_selective_state_update_rows(void* state, const void* x, const 
   hipStream_t s = (hipStream_t)stream;
   // d_state 16 / 32 / 64 / 128 / 256 with 16-byte aligned rows: lanes share a row (coalesced); anything else: a thread per row
   const int lpr = dstate / 4;
-  // a sequence's row (`dense` elements) and every offset up to it in 32 bits
-  auto near = [&](int64_t stride, int64_t dense) {
+  const int64_t xn = (int64_t)nheads * headdim, bn = (int64_t)ngroups * dstate;         // a sequence's elements
+  const bool dense = batch == 1 || (x_stride == xn && dt_stride == nheads && b_stride == bn && c_stride == bn);
+  // every offset in 32 bits
+  auto near = [&](int64_t stride, int64_t n) {
     const int64_t far = stride < 0 ? -stride : stride;
-    return (int64_t)batch * (far > dense ? far : dense) < (1ll << 30);
+    return (int64_t)batch * (far > n ? far : n) < (1ll << 30);
   };
+  const bool fits = dense ? batch * xn < (1ll << 31) && batch * bn < (1ll << 31)
+                          : near(x_stride, xn) && near(dt_stride, nheads) && near(b_stride, bn) && near(c_stride, bn);
   if (dstate % 4 == 0 && (lpr == 4 || lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64) && (((uintptr_t)state) & 15) == 0 &&
-      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && b_stride % 4 == 0 && c_stride % 4 == 0 && (int64_t)batch * nheads * headdim < (1ll << 31) &&
-      near(x_stride, (int64_t)nheads * headdim) && near(dt_stride, nheads) && near(b_stride, (int64_t)ngroups * dstate) &&
-      near(c_stride, (int64_t)ngroups * dstate)) {
-    const int64_t rows = (int64_t)batch * nheads * headdim;
+      (((uintptr_t)Bm | (uintptr_t)Cm) & 15) == 0 && (dense || (b_stride % 4 == 0 && c_stride % 4 == 0)) && fits) {
+    const int64_t rows = batch * xn;
     const int64_t rows_per_block = 4 * (64 / lpr);              // 4 waves x rows per wave-instruction
     const dim3 rgrid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
-#define TV_SUR(T, LPR)                                                                                        \
-    state_update_chain_kernel<T, LPR><<<rgrid, 256, 0, s>>>((float*)state, (const T*)x, (const T*)dt,         \
+    const int xd = dense ? 0 : (int)(x_stride - xn), dd = dense ? 0 : (int)(dt_stride - nheads), bd = dense ? 0 : (int)(b_stride - bn),
+              cd = dense ? 0 : (int)(c_stride - bn);
+#define TV_SUR_D(T, LPR, DENSE)                                                                               \
+    state_update_chain_kernel<T, LPR, DENSE><<<rgrid, 256, 0, s>>>((float*)state, (const T*)x, (const T*)dt,  \
         (const float*)A, (const T*)Bm, (const T*)Cm, (const float*)D, (const float*)dt_bias, (T*)y, nheads,   \
-        headdim, ngroups, (int)(x_stride - (int64_t)nheads * headdim), (int)(dt_stride - nheads),                   \
-        (int)(b_stride - (int64_t)ngroups * dstate), (int)(c_stride - (int64_t)ngroups * dstate), dt_softplus, (int)rows)
+        headdim, ngroups, xd, dd, bd, cd, dt_softplus, (int)rows)
+#define TV_SUR(T, LPR) if (dense) TV_SUR_D(T, LPR, true); else TV_SUR_D(T, LPR, false)
 #define TV_SUR_T(T)                                                                                           \
     switch (lpr) { case 4: TV_SUR(T, 4); break; case 8: TV_SUR(T, 8); break; case 16: TV_SUR(T, 16); break;     \
                    case 32: TV_SUR(T, 32); break; default: TV_SUR(T, 64); break; }
@@ -325,6 +331,7 @@ extern "C" int tv_selective_state_update_rows(void* state, const void* x, const 
     }
 #undef TV_SUR_T
 #undef TV_SUR
+#undef TV_SUR_D
     TV_LAUNCH_CHECK();
   }
   dim3 grid((headdim + 63) / 64, nheads, batch);
