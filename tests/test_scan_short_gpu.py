@@ -86,3 +86,23 @@ def test_segments_that_rounding_up_leaves_without_chunks(K, monkeypatch):
     rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
     # x~ is rounded to bf16 in another frame on each side (2^-8 each), the carried-in states enter y as a product of their own
     assert torch.isfinite(y).all() and rel(y, y1) < 2.0 ** -7 and rel(fin, fin1) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("L", [1, 63, 64, 150])
+@pytest.mark.parametrize("which", ["x", "B", "C"])
+def test_operands_expanded_over_the_tokens(K, L, which):
+    """rows that lie on top of each other: copied row by row below 64 tokens, the general recurrence from there on (one token has no distance)"""
+    H, P, G, N = 8, 80, 2, 128
+    g = torch.Generator(device=DEV).manual_seed(L)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV).bfloat16()
+    ops = {"x": r(1, L, H, P), "B": 0.3 * r(1, L, G, N), "C": 0.3 * r(1, L, G, N)}
+    ops[which] = ops[which][:, :1].expand(-1, L, -1, -1)
+    assert L == 1 or ops[which].stride(1) == 0
+    x, Bm, Cm = ops.values()
+    dt, A, bias, D = r(1, L, H), -torch.linspace(0.01, 16, H, device=DEV), torch.full((H,), -4.0, device=DEV), torch.ones(H, device=DEV)
+    y, fin = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
+    assert (K.ssd_scan_last_impl() == 6) == (L < 64)
+    yr, Sr, ym, Sm = recurrence(x[0].double(), F.softplus(dt[0].double() + bias.double()), A.double(), Bm[0].double(), Cm[0].double(), D.double(),
+                                torch.zeros(H, P, N, dtype=torch.float64, device=DEV), torch.arange(H, device=DEV) // (H // G))
+    assert ((y[0].double() - yr).abs() <= 1.05 * (2.0 ** -7 * ym + 2.0 ** -8 * yr.abs()) + 1e-30).all()       # (as above)
+    assert ((fin[0].double() - Sr).abs() <= 1.05 * 2.0 ** -8 * Sm + 1e-30).all()

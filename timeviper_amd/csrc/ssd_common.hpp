@@ -36,9 +36,15 @@ __device__ __forceinline__ void glds16(const void* sbase, unsigned voff, unsigne
                "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_dst) : "memory");
 }
+// Rows of x, B and C that the scan's copies may take: whole chunks of 64 move the global and the LDS address by one instruction offset, and
+// the lane offsets that make up for it wrap (4 GiB off) where rows overlap, as those of a tensor expanded over the tokens do.  Shorter
+// sequences are copied row by row.
+inline bool scan_rows_apart(int seqlen, int64_t xsl, int64_t bsl, int64_t csl, int headdim, int dstate) {
+  return seqlen < 64 ? xsl >= 0 && bsl >= 0 && csl >= 0 : xsl >= headdim && bsl >= dstate && csl >= dstate;
+}
 // Four 1 KiB pieces with ONE M0 set-up: piece j copies *(sbase + vj + 1024 j) to LDS[lds_dst + 1024 j + 16*lane].
 // The instruction offset moves the global and the LDS address alike, so the caller passes vj = (source offset of
-// piece j) - 1024 j (never negative for rows of >= 256 bytes taken in order).
+// piece j) - 1024 j (never negative for rows of >= 256 bytes taken in order: scan_rows_apart).
 __device__ __forceinline__ void glds16x4(const void* sbase, unsigned v0, unsigned v1, unsigned v2, unsigned v3,
                                          unsigned lds_dst) {
   unsigned keep;

@@ -1303,6 +1303,7 @@ bool tv_ssd_head_supported(int seqlen, int nheads, int headdim, int ngroups, int
   if (dtype != TV_BF16 || dstate != HN || seqlen < 1) return false;
   if (headdim != 32 && headdim != 64 && headdim != 80) return false;
   if (xsl % 8 || bsl % 8 || csl % 8 || bsg % 8 || csg % 8 || ysl % 8) return false;
+  if (!ssdk::scan_rows_apart(seqlen, xsl, bsl, csl, headdim, dstate)) return false;
   if (((uintptr_t)x & 15) || ((uintptr_t)Bm & 15) || ((uintptr_t)Cm & 15) || ((uintptr_t)y & 15)) return false;
   if (64 * xsl * 2 >= (1ll << 31) || 64 * bsl * 2 >= (1ll << 31) || 64 * csl * 2 >= (1ll << 31) ||
       64 * ysl * 2 >= (1ll << 31))
