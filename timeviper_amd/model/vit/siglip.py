@@ -71,7 +71,10 @@ def _tiles(rows: int, n: int, width: int = 256) -> int:
 
 def _gemm_reads(*ts) -> bool:
     """Rows that tv_gemm_bf16_fwd reads and writes in 16-byte pieces"""
-    return all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and (t.dim() == 1 or t.stride(-2) % 8 == 0) for t in ts)
+    for t in ts:
+        if t.stride(-1) != 1 or t.data_ptr() % 16 or (t.dim() > 1 and t.stride(-2) % 8):
+            return False
+    return True
 
 
 def _aligned(n: int) -> int:
@@ -154,6 +157,8 @@ class Attention(nn.Module):
         GPU, inference, K a multiple of 128, N of 8."""
         w, rows = self.qkv.weight, x.numel() // x.shape[-1]
         rounds = -(-_tiles(rows, w.shape[0]) // K.CUS)
+        if not 2 <= rounds <= 6 and rows < 65536:
+            return False
         switch = os.environ.get("TV_VIT_OWN_QKV", "")
         own = switch != "0" and ((switch == "1" and rows >= 65536) or (
             2 <= rounds <= 6 and rows % 256 and ZeroPaddedLinears.wanted(x, w.shape[0]) and K.gemm_persist_on()))
@@ -198,8 +203,9 @@ class Mlp(nn.Module):
         a multiple of 128, tiles for three quarters of the compute units (4 frames, 204 tiles: library + GELU 42 us, fused 41; 3 frames, 153:
         34 and 39; 1 024 x 4 096: 192 tiles 37 and 38, 240: 42 and 40); TV_VIT_FUSED_FC1=0 switches it off."""
         return (self.exact_gelu and x.is_cuda and x.dtype == torch.bfloat16 and w1.dtype == torch.bfloat16
-                and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0 and _gemm_reads(x, w1, b1)
-                and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * K.CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0")
+                and not torch.is_grad_enabled() and w1.shape[1] % 128 == 0 and w1.shape[0] % 4 == 0
+                and 4 * _tiles(x.numel() // x.shape[-1], w1.shape[0]) >= 3 * K.CUS and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0"
+                and _gemm_reads(x, w1, b1))
 
     def forward(self, x):
         h, w2 = self.hidden(x)
