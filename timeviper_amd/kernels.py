@@ -759,17 +759,17 @@ def large_takes(x, weight, relu2=False) -> bool:
     The rest stays the library's (15 680 x 4 480 alone; 12 288 x 4 096, 8 000 rows: 553 | 595)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     rows = x.numel() // max(x.shape[-1], 1)
-    if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and rows > MID_MAX and Kd >= 4096
-            and Kd % 128 == 0 and N % 8 == 0 and 256 <= N < (1 << 22) and x.is_contiguous() and weight.is_contiguous()
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
-        return False
     tiles = -(-rows // 256) * -(-N // 256)
-    fill = tiles / (-(-tiles // CUS) * CUS)
-    if tiles <= CUS or not gemm_persist_on():
+    if tiles <= CUS or rows <= MID_MAX or Kd < 4096:
         return False
+    fill = tiles / (-(-tiles // CUS) * CUS)
     if relu2:
-        return fill >= 0.75 and Kd <= 8192
-    return (N >= 20480 and rows <= 12288 and fill >= 0.69) or (N < 20480 and Kd >= 8192 and rows <= 32768 and fill >= 0.8)
+        pays = fill >= 0.75 and Kd <= 8192
+    else:
+        pays = (N >= 20480 and rows <= 12288 and fill >= 0.69) or (N < 20480 and Kd >= 8192 and rows <= 32768 and fill >= 0.8)
+    return (pays and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 128 == 0
+            and N % 8 == 0 and 256 <= N < (1 << 22) and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0 and gemm_persist_on())
 
 
 def mid_linear(x, weight, bias=None, relu2=False):
