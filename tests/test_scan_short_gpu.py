@@ -106,3 +106,36 @@ def test_operands_expanded_over_the_tokens(K, L, which):
                                 torch.zeros(H, P, N, dtype=torch.float64, device=DEV), torch.arange(H, device=DEV) // (H // G))
     assert ((y[0].double() - yr).abs() <= 1.05 * (2.0 ** -7 * ym + 2.0 ** -8 * yr.abs()) + 1e-30).all()       # (as above)
     assert ((fin[0].double() - Sr).abs() <= 1.05 * 2.0 ** -8 * Sm + 1e-30).all()
+
+
+# csrc/ssd_par.hip: a head per work-group, segments that start from the state their predecessors leave.  Chunk and segment edges, one segment (many heads, or slices
+# that column work-groups cannot take), head dims with and without a single tile; decays that take a chunk as it is, raised, or with the true mask
+@pytest.mark.parametrize("B,H,P,G,group_map,L", [
+    (1, 8, 80, 2, "block", 512), (1, 8, 80, 2, "tile", 577), (2, 8, 80, 2, "block", 1089), (1, 4, 32, 1, "block", 705), (2, 8, 64, 4, "tile", 640),
+    (1, 2, 80, 2, "block", 1), (1, 2, 80, 2, "block", 63), (1, 2, 80, 2, "tile", 130), (1, 6, 64, 2, "block", 513),
+    (3, 128, 80, 8, "block", 65), (2, 128, 32, 8, "block", 200)])
+@pytest.mark.parametrize("decay", ["slow", "mixed", "fast"])
+def test_heads_in_segments(K, B, H, P, G, group_map, L, decay):
+    N = 128
+    g = torch.Generator(device=DEV).manual_seed(L * 7 + H)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    proj = (1.3 * r(B, L, H * P + H + 16 - H % 8)).bfloat16()  # x and dt as slices of a wider row
+    proj = proj[..., :proj.shape[-1] // 8 * 8].contiguous()
+    x, dt = proj[..., :H * P].unflatten(-1, (H, P)), proj[..., H * P:H * P + H]
+    bc = (0.3 * r(B, 2 * G, L, N)).bfloat16()
+    Bm, Cm = bc[:, :G].transpose(1, 2), bc[:, G:].transpose(1, 2)
+    A = -{"slow": torch.linspace(0.01, 1, H, device=DEV), "mixed": torch.linspace(0.01, 16, H, device=DEV),
+          "fast": torch.linspace(8, 60, H, device=DEV)}[decay]
+    bias, D = torch.linspace(-6, -1, H, device=DEV), r(H)
+    init = r(B, H, P, N)
+    y, fin, dec = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
+                                              group_map=group_map, return_total_decay=True)
+    assert K.ssd_scan_last_impl() == 6
+    h = torch.arange(H, device=DEV)
+    of = h % G if group_map == "tile" else h // (H // G)
+    for b in range(B):
+        d = F.softplus(dt[b].double() + bias.double())
+        yr, Sr, ym, Sm = recurrence(x[b].double(), d, A.double(), Bm[b].double(), Cm[b].double(), D.double(), init[b].double(), of)
+        assert ((y[b].double() - yr).abs() <= 1.05 * (2.0 ** -7 * ym + 2.0 ** -8 * yr.abs()) + 1e-30).all()       # (as above)
+        assert ((fin[b].double() - Sr).abs() <= 1.05 * 2.0 ** -8 * Sm + 1e-30).all()
+        assert torch.allclose(dec[b].double(), (d * A.double()).sum(0), rtol=1e-4, atol=1e-4)

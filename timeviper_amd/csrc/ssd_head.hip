@@ -47,6 +47,13 @@ int tv_ssd_cols_launch(const void* x, const void* dt, const void* A, const void*
                        int headdim, int ngroups, int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg,
                        int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map,
                        hipStream_t st);
+// ssd_par.hip: a head per work-group, segments that start from the true state
+size_t tv_ssd_par_workspace_bytes(int batch, int nheads, int headdim, int nseg);
+int tv_ssd_par_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* cb, const void* D,
+                      const void* dt_bias, const void* init_state, void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads,
+                      int headdim, int ngroups, int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg,
+                      int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map,
+                      int nseg, int seg_chunks, void* workspace, hipStream_t st);
 // ssd_correct.hip
 size_t tv_ssd_correct_all_workspace_bytes(int batch, int nheads, int nchunks, int nseg, int headdim);
 unsigned* tv_ssd_correct_all_counters(void* workspace, int batch, int nheads, int nchunks, int nseg, int headdim);
@@ -1233,18 +1240,32 @@ int pick_segments(int batch, int nheads, int nchunks) {
   return nseg < 1 ? 1 : nseg;
 }
 
-// Short sequences: column slices (ssd_cols.hip) while their work-groups (4 slices) all run at once and the march over them is no longer than
-// segments would make it.  128 heads x 80, 8 groups, whole operator, one segment | best number of segments | slices: 203 tokens 35 | 51 |
-// 17 us, 512: 56 | 59 | 29, 1 501: 146 | 89 | 83 - 93, 2 048: 180 | 98 | 107, 3 000: 244 | 113 | 128.
+// Short sequences: column slices (ssd_cols.hip) while their work-groups (4 slices) all run at once and a segment's first pass would cost more
+// than it takes off the chain.  128 heads x 80, 8 groups, whole operator, slices | heads in segments (ssd_par.hip): 203 tokens 17.4 | 20.6 us, 390: 23.1 | 26.7,
+// 512: 36.2 | 30.3, 1 501: 90 | 54; 64 heads: 390 tokens 19.2 | 20.8, 512: 22.7 | 23.0, 700: 27.2 | 25.9.
 bool use_cols(int batch, int nheads, int headdim, int ngroups, int nchunks) {
   if (ngroups < 1 || nchunks < 1) return false;
   const int slices = nheads / ngroups * (headdim / 16);        // of a group
-  return nchunks <= 24 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= tv_cu_count();
+  return nchunks < 8 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= tv_cu_count();
+}
+
+// Segments of ssd_par.hip, 0: not its case.  Its work-groups (one a head and segment, two a compute unit) fill one round, a segment has two chunks or more (twelve, where the
+// heads alone give more than half of the compute units their work) and at most 24: beyond, the march's pass over y for what later segments carry in costs less than reading x and B twice.
+// 128 heads x 80 (4 segments), march | this: 2 048 tokens 99.9 | 61.5 us, 4 200: 147 | 118, 6 000: 170 | 156, 8 000: 198 | 210; 64 heads (8): 4 200: 112 | 69, 10 007: 167 |
+// 147; 256 heads (2): 64 tokens 23.5 | 12.6, 1 024: 95 | 57, 3 000: 167 | 161, 4 200: 206 | 224; 512 heads (1): 203: 48 | 29, 1 501: 158 | 112.
+int par_segments(int batch, int nheads, int nchunks) {
+  const int64_t heads = (int64_t)batch * nheads, round = 2 * (int64_t)tv_cu_count();
+  if (heads < 1 || heads > round || nchunks < 1) return 0;
+  int nseg = (int)(round / heads);
+  if (nseg > 16) nseg = 16;
+  const int least = 2 * heads > tv_cu_count() ? 12 : 2;        // (256 heads, one | two segments: 203 tokens 24 | 28 us, 1 024: 57 | 59, 1 501: 94 | 90)
+  if (nseg > nchunks / least) nseg = nchunks > least ? nchunks / least : 1;
+  return (nchunks + nseg - 1) / nseg <= 24 ? nseg : 0;
 }
 
 struct HeadLayout {
-  size_t cb, seg_state, seg_decay, ctot, corr, dtt, total;
-  int nseg, seg_chunks;
+  size_t cb, par, seg_state, seg_decay, ctot, corr, dtt, total;
+  int nseg, seg_chunks, par_nseg, par_chunks;  // of the march; of ssd_par.hip (0: not its case)
   bool cols;
 };
 HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngroups) {
@@ -1252,11 +1273,15 @@ HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngrou
   const size_t nchunks = (size_t)(seqlen + HQ - 1) / HQ;
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   l.cols = use_cols(batch, nheads, headdim, ngroups, (int)nchunks);
-  l.nseg = l.cols ? 1 : pick_segments(batch, nheads, (int)nchunks);
+  l.par_nseg = l.cols ? 0 : par_segments(batch, nheads, (int)nchunks);
+  l.par_chunks = l.par_nseg ? (int)((nchunks + l.par_nseg - 1) / l.par_nseg) : 0;
+  if (l.par_nseg) l.par_nseg = (int)((nchunks + l.par_chunks - 1) / l.par_chunks);
+  l.nseg = l.cols || l.par_nseg ? 1 : pick_segments(batch, nheads, (int)nchunks);
   l.seg_chunks = (int)((nchunks + l.nseg - 1) / l.nseg);
   if (l.seg_chunks > 0) l.nseg = (int)((nchunks + l.seg_chunks - 1) / l.seg_chunks);      // no segment is empty (the march reads its first chunk)
   l.cb = 0;
-  l.seg_state = up((size_t)batch * ngroups * nchunks * CBE * sizeof(bf16_t));
+  l.par = up((size_t)batch * ngroups * nchunks * CBE * sizeof(bf16_t));
+  l.seg_state = l.par + up(tv_ssd_par_workspace_bytes(batch, nheads, headdim, l.par_nseg));
   const size_t st = (size_t)batch * nheads * headdim * HN * sizeof(float);
   l.seg_decay = l.seg_state + (l.nseg > 1 ? up(l.nseg * st) : 0);
   l.ctot = l.seg_decay + (l.nseg > 1 ? up((size_t)l.nseg * batch * nheads * sizeof(float)) : 0);
@@ -1339,11 +1364,15 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
   a.seg_state = lay.nseg > 1 ? (float*)(wsb + lay.seg_state) : nullptr;
   a.seg_decay = lay.nseg > 1 ? (float*)(wsb + lay.seg_decay) : nullptr;
   a.chunk_tot = lay.nseg > 1 ? (float*)(wsb + lay.ctot) : nullptr;
-  if (lay.cols && dsl < (1 << 24)) {           // (64 rows of dt at 32-bit offsets)
+  if ((lay.cols || lay.par_nseg) && dsl < (1 << 24)) {         // (64 rows of dt at 32-bit offsets)
     if (!cb_pre) {
       const int rc = tv_ssd_cb_prepass_launch(Bm, Cm, workspace, batch, seqlen, ngroups, bsb, bsl, bsg, csb, csl, csg, st);
       if (rc != TV_OK) return rc;
     }
+    if (lay.par_nseg)
+      return tv_ssd_par_launch(x, dt, A, Bm, Cm, a.cb, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups,
+                               xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, lay.par_nseg,
+                               lay.par_chunks, wsb + lay.par, st);
     return tv_ssd_cols_launch(x, dt, A, Bm, Cm, a.cb, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups,
                               xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, st);
   }
