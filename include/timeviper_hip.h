@@ -608,6 +608,14 @@ int tv_gemm_rows_pair_fwd(const void* x, const void* x2, const void* W, const vo
                           int ff, int K, int64_t x_stride, int64_t x2_stride, int64_t ldw, int64_t y_stride,
                           int64_t act_stride, void* stream);
 
+/* y = x W^T + bias on tiles of 256 x 256 outputs (csrc/gemm.hip) whose contraction is split over `splits` work-groups (1..64; each takes at
+ * least two steps of 64 columns, K % 64 == 0, N % 4 == 0): fp32 partial sums to the workspace (tv_gemm_split_workspace_bytes, 0 for one
+ * split; 16-byte aligned, not shared by launches that may run at once), added in order by a second launch, one rounding.  bias fp32 or bf16
+ * or NULL, 16-byte aligned; epilogue 0, or 3: the squared ReLU of the rounded sum. */
+size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits);
+int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
+                      int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Products of a short prompt's rows (csrc/gemm_mid.hip): y = x W^T + bias for 1..TV_GEMM_MID_MAX bf16 rows, K % 64 == 0, N % 4 == 0,
  * bias bf16 or NULL, fp32 sums, one rounding; epilogue 0 or TV_GEMM_ROWS_RELU2.  workspace: partial sums where K is split
  * (tv_gemm_mid_workspace_bytes, 0 where it is not), 16-byte aligned, not shared by launches that may run at once. */

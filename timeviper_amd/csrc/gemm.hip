@@ -42,8 +42,12 @@ constexpr int LDS_BYTES = RING_BYTES;
 
 // GROUPED (mixture of experts): the tile belongs to one expert — its rows of C, its W — and the rows of A are gathered by the
 // copies' per-lane offsets.  The number of row tiles is only known on the device: the grid covers the largest possible one.
-template <int EPI, bool GROUPED>
-__global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
+// SPLIT: `a.splits` work-groups share a tile, each with its own K-tiles (any number from two on, odd ones too), their fp32 sums go to
+// a.part and gemm_split_sum_kernel adds them; with one split the tile is written as ever.  A few hundred rows against a few thousand outputs are 36 - 126
+// tiles for 256 compute units; the library's answer, smaller tiles, reads LDS more often.  A split costs 64 MB of partial sums at most (one round of
+// tiles), 6 us to write and 10 to add: 4 480 x 15 680, 512 rows 137 | 75 us (library | here), 4 480 x 10 240, 1 000 rows 110 | 89; kernels.split_takes has more.
+template <int EPI, bool GROUPED, bool SPLIT>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -57,8 +61,14 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
   int id = blockIdx.x;
   if (GROUPED && id >= ntiles) return;
   {
-    const int q = ntiles / 8, r = ntiles % 8, x = id % 8;
+    const int all = SPLIT ? ntiles * a.splits : ntiles;
+    const int q = all / 8, r = all % 8, x = id % 8;
     id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + id / 8;
+  }
+  int split = 0;
+  if (SPLIT) {                                 // (neighbours of an XCD share a split: the same k-slabs)
+    split = __builtin_amdgcn_readfirstlane(id / ntiles);
+    id -= split * ntiles;
   }
   // ... in bands of `gm` m-tiles, m fastest: the ~32 work-groups an XCD runs at a time cover gm x (32 / gm) tiles and
   // share each A / W k-slab through its L2 while they march through K together
@@ -94,8 +104,13 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
       voffA[h][j] = (unsigned)((ra * a.lda + ch * 8) * 2);
       voffW[h][j] = (unsigned)((rw * a.ldw + ch * 8) * 2);
     }
-  const bf16_t* Ag = GROUPED ? a.A : a.A + (int64_t)m0 * a.lda;
-  const bf16_t* Wg = a.W + (GROUPED ? (int64_t)e * a.w_group : 0) + (int64_t)n0 * a.ldw;
+  int nkt = a.K / BK, kt0 = 0;
+  if (SPLIT) {
+    kt0 = (int)((int64_t)nkt * split / a.splits);
+    nkt = (int)((int64_t)nkt * (split + 1) / a.splits) - kt0;       // (>= 2: launcher)
+  }
+  const bf16_t* Ag = (GROUPED ? a.A : a.A + (int64_t)m0 * a.lda) + kt0 * BK;
+  const bf16_t* Wg = a.W + (GROUPED ? (int64_t)e * a.w_group : 0) + (int64_t)n0 * a.ldw + kt0 * BK;
   const unsigned piece0 = (unsigned)(2 * wave * 1024);
   // X: 0 = A, 1 = W;  h: half;  t: K-tile
   auto stage = [&](int X, int h, int t) __attribute__((always_inline)) {
@@ -132,7 +147,6 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
   bf16x8 af[4][2];                          // A rows of the current m-half: [m-tile][k-step]
   bf16x8 wf0[2][2][2], wf1[2][2];           // W0 of the current and of the next K-tile (by K-tile parity), W1
 
-  const int nkt = a.K / BK;
   const int nitems = 4 * nkt;               // half-tiles in issue order: item 4 t + {0: W0, 1: A0, 2: W1, 3: A1} of K-tile t
 
   // Copy schedule (ONE half-tile per phase, each 6 phases ahead of its read): phase g = 4 t + p (p = 1..4) READS item g —
@@ -253,11 +267,31 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
       ktile(t, integral_constant<int, 0>{}, integral_constant<bool, false>{});
       ktile(t + 1, integral_constant<int, 1>{}, integral_constant<bool, false>{});
     }
-    // the last two K-tiles (the launcher takes an even number of K-tiles: t is even here)
+    // the last two K-tiles, three of an odd number (t is even here; without SPLIT the launcher takes even numbers only)
     ktile(t, integral_constant<int, 0>{}, integral_constant<bool, true>{});
     ktile(t + 1, integral_constant<int, 1>{}, integral_constant<bool, true>{});
+    if (SPLIT && t + 2 < nkt) ktile(t + 2, integral_constant<int, 0>{}, integral_constant<bool, true>{});
   }
   if (wr == 0) __builtin_amdgcn_s_barrier();          // barrier counts match again
+
+  if (SPLIT && a.part) {                              // 16 rows x 64 bytes an instruction
+    float* const P = a.part + (int64_t)split * a.M * a.N;
+#pragma unroll
+    for (int mh = 0; mh < 2; ++mh)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int row = m0 + 128 * mh + 64 * wr + 16 * m + lc;
+        if (row >= mend) continue;
+#pragma unroll
+        for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            const int col = n0 + 128 * nh + 32 * wc + 16 * n + 4 * kq;
+            if (col < a.N) *(f32x4*)(P + (int64_t)row * a.N + col) = acc[mh][nh][m][n];
+          }
+      }
+    return;
+  }
 
   // ---- epilogue.  A lane holds, for (mh, nh, m-tile, n-tile), columns .. + 4 kq + 0..3 of row .. + lc.  Two m-tiles at a
   // time: v_permlane16_swap exchanges the odd 16-lane rows of one register with the even rows of the other, after which a
@@ -328,6 +362,13 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) v[r] = gelu_erf_f((float)(bf16_t)v[r]);       // the GEMM's own bf16 rounding first
           }
+          if (SPLIT && a.relu2) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+              const float p = fmaxf((float)(bf16_t)v[r], 0.f);
+              v[r] = p * p;
+            }
+          }
           u32x4e o;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -342,6 +383,58 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) {
           }
         }
     }
+}
+
+template <int EPI, bool GROUPED>
+__global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) { gemm_tile<EPI, GROUPED, false>(a); }
+__global__ __launch_bounds__(512) void gemm_split_kernel(GemmArgs a) { gemm_tile<EPI_BIAS, false, true>(a); }
+
+// the splits of four neighbouring outputs, added in order; bias, one rounding, squared ReLU of what was rounded
+__global__ __launch_bounds__(256) void gemm_split_sum_kernel(GemmArgs a) {
+  const int nq = a.N / 4;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)a.M * nq) return;
+  const int row = (int)(i / nq), col = 4 * (int)(i - (int64_t)row * nq);
+  const float* p = a.part + (int64_t)row * a.N + col;
+  const int64_t step = (int64_t)a.M * a.N;
+  f32x4 s = *(const f32x4*)p;
+  for (int j = 1; j < a.splits; j += 4) {             // (a split that is not there repeats the last one, weighted 0 by not being added)
+    f32x4 t[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t[u] = *(const f32x4*)(p + min(j + u, a.splits - 1) * step);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (j + u < a.splits) s += t[u];
+  }
+  if (a.bias) {
+    if (a.bias_f32) s += *(const f32x4*)((const float*)a.bias + col);
+    else {
+      const bf16x4 b = *(const bf16x4*)((const bf16_t*)a.bias + col);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] += (float)b[r];
+    }
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    o[r] = (bf16_t)s[r];
+    if (a.relu2) {
+      const float f = fmaxf((float)o[r], 0.f);
+      o[r] = (bf16_t)(f * f);
+    }
+  }
+  *(bf16x4*)(a.C + (int64_t)row * a.ldc + col) = o;
+}
+
+int launch_split(const GemmArgs& a, hipStream_t st) {
+  hipError_t e = hipFuncSetAttribute((const void*)gemm_split_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+  if (e != hipSuccess) {
+    tv_set_error("gemm_split: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+    return TV_ERR_LAUNCH;
+  }
+  gemm_split_kernel<<<dim3((unsigned)(a.tiles_m * a.tiles_n * a.splits)), 512, LDS_BYTES, st>>>(a);
+  if (a.part) gemm_split_sum_kernel<<<dim3((unsigned)(((int64_t)a.M * (a.N / 4) + 255) / 256)), 256, 0, st>>>(a);
+  TV_LAUNCH_CHECK();
 }
 
 template <int EPI>
@@ -432,4 +525,37 @@ extern "C" int tv_gemm_bf16_fwd(const void* A, const void* W, const void* bias, 
     case EPI_BIAS_GELU: return launch_gemm<EPI_BIAS_GELU>(a, st);
     default: return launch_gemm<EPI_ACCUM>(a, st);
   }
+}
+
+extern "C" size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits) {
+  return M <= 0 || N <= 0 || splits <= 1 ? 0 : (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
+}
+
+extern "C" int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
+                                 int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(M > 0 && N > 0 && K > 0, "gemm_split: bad sizes (M %lld N %d K %d)", (long long)M, N, K);
+  TV_CHECK_ARG(A && W && C, "gemm_split: null pointer");
+  TV_CHECK_ARG(epilogue == 0 || epilogue == 3, "gemm_split: epilogue %d", epilogue);
+  TV_CHECK_ARG(bias == nullptr || bias_dtype == TV_F32 || bias_dtype == TV_BF16, "gemm_split: bias dtype %d", bias_dtype);
+  TV_CHECK_ARG(splits >= 1 && splits <= 64, "gemm_split: %d splits", splits);
+  if (K % BK || K / BK < 2 * splits || N % 4 || lda % 8 || ldw % 8 || ldc % 4 || lda < 0 || ldw < 0 || ldc < 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) ||
+      ((uintptr_t)C & 7) || ((uintptr_t)bias & 15))
+    TV_UNSUPPORTED("gemm_split: K must be a multiple of %d (two of them a split), N of 4, rows 16-byte aligned (K %d N %d lda %lld ldw %lld ldc %lld)", BK, K,
+                   N, (long long)lda, (long long)ldw, (long long)ldc);
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (M > (1ll << 31) - BM || 256 * lda * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31) || tiles * splits >= (1ll << 31) || M * (N / 4) >= (1ll << 38))
+    TV_UNSUPPORTED("gemm_split: sizes beyond the 32-bit offsets of the copies");
+  const size_t need = tv_gemm_split_workspace_bytes(M, N, splits);
+  TV_CHECK_ARG(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
+               "gemm_split: workspace of %zu bytes (16-byte aligned) needed, got %zu", need, workspace_bytes);
+  GemmArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.bias = bias; a.C = (bf16_t*)C;
+  a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc;
+  a.tiles_m = (int)((M + BM - 1) / BM); a.tiles_n = (N + BN - 1) / BN;
+  a.bias_f32 = bias_dtype == TV_F32;
+  a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
+  a.part = splits > 1 ? (float*)workspace : nullptr;
+  a.splits = splits;
+  a.relu2 = epilogue == 3;
+  return launch_split(a, (hipStream_t)stream);
 }

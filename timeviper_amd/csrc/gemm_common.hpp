@@ -29,6 +29,9 @@ struct GemmArgs {
   const int *offsets, *row_token;
   int groups;
   int64_t w_group;
+  // products whose contraction is split over work-groups: partial sums [splits][M][N], NULL where splits is 1 (tv_gemm_split_fwd)
+  float* part;
+  int splits, relu2;       // relu2: squared ReLU of the rounded sum
 };
 
 // same formula as norms.hip's gelu_erf (A&S 7.1.26): the fused and the two-pass path agree bit for bit

@@ -772,6 +772,58 @@ def large_takes(x, weight, relu2=False) -> bool:
             and weight.data_ptr() % 16 == 0 and gemm_persist_on())
 
 
+def split_takes(x, weight, relu2=False) -> int:
+    """Products of more than 256 rows that tv_gemm_split_fwd runs faster than the library: work-groups a tile of 256 x 256 outputs, 0 where the product is not one
+    of them (us, library | here):
+      - a long contraction into fewer outputs whose tiles leave half of the compute units idle: as many work-groups a tile as fit one round, if they fill 80 % of
+        it (4 480 x 10 240: 300 rows 59 | 52, 512: 85 | 59, 1 024: 108 | 90, 1 536: 137 | 124; 4 480 x 15 680: 300: 92 | 67, 512: 137 | 75, 1 400: 349 | 177; 75 % full,
+        600 rows of 8 192 x 28 672: 254 | 287),
+      - a contraction longer than the outputs whose last round is 80 % full: one work-group a tile, where `large_takes` does not have it, and in a first round
+        only widths that the library's 256 columns do not divide (4 096 x 11 008, 3 900 rows: 227 | 237) (4 480 x 15 680, an odd
+        number of steps: 3 000 rows 532 | 306, 10 007: 1 382 | 999, 14 000: 1 728 | 1 360; 4 480 x 10 240: 3 000: 219 | 203; 4 480 x 5 120: 3 000: 117 | 107, 6 011: 224 |
+        207; 84 % full and the library in step, 7 000 x 15 680: 654 | 680; 75 %, 8 192 x 5 120: 292 | 314),
+      - more than 12 288 columns in up to one and a half rounds: two work-groups a tile (4 480 x 15 680: 4 096 rows 855 | 514, 5 000: 966 | 564),
+      - the squared ReLU in a single round that is 72 % full (15 680 x 4 480, with the pass that it saves: 700 rows 101 | 90, 1 024: 122 | 103)."""
+    N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
+    rows = x.numel() // max(x.shape[-1], 1)
+    tiles = -(-rows // 256) * -(-N // 256)
+    if rows <= MID_MAX or N < 4096 or Kd < 4096 or rows > 32768:
+        return 0
+    fill = tiles / (-(-tiles // CUS) * CUS)
+    splits = 0
+    if relu2:
+        splits = int(Kd <= 8192 and tiles <= CUS and fill >= 0.72)
+    elif N <= Kd:
+        fit = CUS // tiles
+        if fit >= 2:
+            splits = fit if Kd >= 8192 and fit <= 8 and tiles * fit >= 0.8 * CUS else 0
+        elif fill >= 0.8:
+            splits = int(N % 256 != 0 if tiles <= CUS else N < Kd < 8192 or Kd % 128 != 0)
+        elif Kd > 12288 and CUS < tiles <= CUS * 3 // 2:
+            splits = 2
+    takes = (splits and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 64 == 0 and N % 4 == 0
+             and Kd < (1 << 22) and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+    return splits if takes else 0
+
+
+def split_linear(x, weight, bias=None, relu2=False, splits=1):
+    """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) on tiles of 256 x 256 outputs, `splits` work-groups a tile."""
+    _gpu(x, weight, bias)
+    N, Kd = weight.shape
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[-1] != Kd or weight.stride(1) != 1:
+        raise TimeViperHipError(f"split_linear: bf16 rows of {Kd} elements, got {tuple(x.shape)} {x.dtype} against {weight.dtype}")
+    if bias is not None and (bias.dtype not in (torch.float32, torch.bfloat16) or not bias.is_contiguous() or bias.numel() != N):
+        raise TimeViperHipError("split_linear: bias must be contiguous, fp32 or bf16")
+    x2 = _rows2d(x)
+    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    lib, M = _capi.lib(), x2.shape[0]
+    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib.tv_gemm_split_fwd(_p(x2), _p(weight), _p(bias), _p(y), M, N, Kd, x2.stride(0), weight.stride(0), N, 3 if relu2 else 0,
+                                TV_F32 if bias is None else _dt(bias), splits, _p(ws), need, _stream()), "tv_gemm_split_fwd")
+    return y
+
+
 def mid_linear(x, weight, bias=None, relu2=False):
     """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) for up to 256 bf16 rows (a short prompt)."""
     _gpu(x, weight, bias)

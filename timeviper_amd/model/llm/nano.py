@@ -312,8 +312,8 @@ def _linear(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
 
 
 def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torch.Tensor:
-    """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256) or tv_gemm_bf16_fwd where those
-    are faster than the library (`plain_linear`: a module with anything around it is called)."""
+    """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256), tv_gemm_split_fwd or tv_gemm_bf16_fwd where
+    those are faster than the library (`plain_linear`: a module with anything around it is called)."""
     if x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and plain_linear(mod, x):
         rows, w = x.shape[0] * x.shape[1], mod.weight
         if rows <= K.ROWS_MAX and K.rows_pay(x, w):
@@ -321,6 +321,8 @@ def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torc
         if rows <= K.MID_MAX:
             if K.mid_takes(x, w, relu2):
                 return K.mid_linear(x, w, mod.bias, relu2)
+        elif splits := K.split_takes(x, w, relu2):
+            return K.split_linear(x, w, mod.bias, relu2, splits)
         elif K.large_takes(x, w, relu2):
             return K.linear_fused(x, w, mod.bias, epilogue=K.GEMM_BIAS_RELU2 if relu2 else K.GEMM_BIAS)
     y = mod(x)
