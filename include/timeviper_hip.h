@@ -616,6 +616,22 @@ size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits);
 int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
                       int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same with the residual stream behind it: residual_out = residual + (x W^T + bias) in fp32 (rows of N, 16-byte aligned; in place where residual_out is
+ * residual) and y (rows of N), its bf16 copy. */
+int tv_gemm_split_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N,
+                          int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream);
+
+/* C = gelu_tanh(A Wg^T + bg) * (A Wu^T + bu), Wg the first N rows of W and Wu the next N, bg | bu the bf16 bias (csrc/gemm_persist.hip): fp32 until the one
+ * rounding.  M >= 256, N >= 128 and a multiple of 8, K a multiple of 128 and at least 256, everything 16-byte aligned. */
+int tv_gemm_glu_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                    void* stream);
+
+/* y = P (gelu_tanh(G h) * e), e the table's row of each token (csrc/token_side.hip): h (rows, width) bf16, G (dim, width), P (width, dim), table (table_rows,
+ * dim) with a row stride of its own; ids outside the table count as rows of zeros.  width % 32 == 0, dim 128. */
+int tv_token_side_fwd(const void* h, const int64_t* ids, const void* table, const void* gate, const void* proj, void* y, int64_t rows, int width,
+                      int dim, int64_t table_rows, int64_t h_stride, int64_t table_stride, int64_t gate_stride, int64_t proj_stride,
+                      int64_t y_stride, void* stream);
+
 /* Products of a short prompt's rows (csrc/gemm_mid.hip): y = x W^T + bias for 1..TV_GEMM_MID_MAX bf16 rows, K % 64 == 0, N % 4 == 0,
  * bias bf16 or NULL, fp32 sums, one rounding; epilogue 0 or TV_GEMM_ROWS_RELU2.  workspace: partial sums where K is split
  * (tv_gemm_mid_workspace_bytes, 0 where it is not), 16-byte aligned, not shared by launches that may run at once. */

@@ -1,0 +1,85 @@
+"""The products of a parallel layer's prompt with what stands behind them: gated pair, residual stream, token side."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+def rand(seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return lambda *s: torch.randn(s, generator=g, device=DEV)
+
+
+# edges of tiles (256 rows, 128 outputs), one tile and more than one round of them, an even number of steps from four on
+@pytest.mark.parametrize("M,N,K", [(256, 128, 256), (257, 136, 384), (511, 264, 512), (2100, 5632, 256)])
+def test_gated_pair(M, N, K):
+    from timeviper_amd import kernels as ops
+    r = rand(M)
+    x, w, b = r(M, K).to(BF), (K ** -0.5 * r(2 * N, K)).to(BF), r(2 * N).to(BF)
+    wide = torch.full((M, N + 24), 7.0, device=DEV, dtype=BF)
+    out = wide[:, 8:8 + N]
+    ops.glu_linear(x, w, b, out)
+    g, u = (x.double() @ w.double().T + b.double()).split(N, 1)
+    want = F.gelu(g, approximate="tanh") * u
+    # fp32 sums and functions (1e-5 of the factors; the slope of the activation is below 1.13) and one rounding
+    bound = 2.0 ** -8 * want.abs() + 2e-5 * (g.abs() + 1) * (u.abs() + 1)
+    assert ((out.double() - want).abs() <= bound).all()
+    assert (wide[:, :8] == 7).all() and (wide[:, 8 + N:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(1, 4, 192, 1), (300, 516, 1088, 1), (255, 260, 640, 3), (513, 1024, 7680, 16)])
+def test_onto_the_stream(M, N, K, splits):
+    from timeviper_amd import kernels as ops
+    r = rand(N)
+    x, w, b, res = r(M, K).to(BF), (K ** -0.5 * r(N, K)).to(BF), r(N).to(BF), r(M, N)
+    got, h = ops.split_add_linear(x, w, res, b, splits)
+    want = res.double() + x.double() @ w.double().T + b.double()
+    assert ((got.double() - want).abs() <= (x.double().abs() @ w.double().abs().T + want.abs() + 4) * K * 2.0 ** -24).all()
+    assert torch.equal(h, got.to(BF))
+
+
+# tiles of 32 rows, units of 32 columns: fewer than the eight waves, no multiple of them; ids on both ends of the table, a slice of a wider one
+@pytest.mark.parametrize("T,D", [(1, 32), (31, 96), (33, 288), (64, 2048), (515, 2080)])
+def test_token_side(T, D):
+    from timeviper_amd import kernels as ops
+    r = rand(T)
+    h, g, p, table = r(T, D + 8).to(BF)[:, :D], (D ** -0.5 * r(128, D)).to(BF), (128 ** -0.5 * r(D, 128)).to(BF), r(50, 384).to(BF)[:, 132:260]
+    ids = torch.randint(0, 50, (T,), device=DEV)
+    ids[0], ids[-1] = 0, 49
+    got = ops.token_side(h, ids, table, g, p).double()
+    s = h.double() @ g.double().T
+    z = F.gelu(s, approximate="tanh") * table[ids].double()
+    want = z @ p.double().T
+    # roundings of the 128 sums, of z (2^-8 each, the first through a slope below 1.13) and of the result
+    dz = (1.13 * 2.0 ** -8 * s.abs() + 1e-5) * table[ids].double().abs() + 2.0 ** -8 * z.abs()
+    assert ((got - want).abs() <= 1.02 * dz @ p.double().abs().T + 2.0 ** -8 * want.abs()).all()
+    ids[T // 2] = 50
+    got, want[T // 2] = ops.token_side(h, ids, table, g, p), 0
+    assert (got[T // 2] == 0).all()
+
+
+def test_refused():
+    from timeviper_amd import kernels as ops
+    z = lambda *s: torch.zeros(s, device=DEV, dtype=BF)
+    for x, w, n in ((z(255, 256), z(256, 256), 128), (z(256, 320), z(256, 320), 128), (z(256, 256), z(240, 256), 120)):
+        with pytest.raises(ops.TimeViperHipError):
+            ops.glu_linear(x, w, z(2 * n), z(x.shape[0], n))
+    with pytest.raises(ops.TimeViperHipError):
+        ops.token_side(z(4, 64), torch.zeros(4, dtype=torch.long, device=DEV), z(9, 64), z(64, 64), z(64, 64))
+    with pytest.raises(ops.TimeViperHipError):
+        ops.split_add_linear(z(4, 100), z(64, 100), torch.zeros(4, 64, device=DEV))
+
+
+# both sides of each line
+@pytest.mark.parametrize("rows,glu,add", [(255, False, 16), (512, False, 16), (700, True, 10), (1300, False, 5), (1800, True, 4), (4096, True, 2), (6011, True, 0)])
+def test_rules(rows, glu, add):
+    from timeviper_amd import kernels as ops
+    h, u = torch.empty(rows, 2048, device=DEV, dtype=BF), torch.empty(rows, 7680, device=DEV, dtype=BF)
+    inp, out = torch.empty(16384, 2048, device=DEV, dtype=BF)[5120:], torch.empty(2048, 7680, device=DEV, dtype=BF)
+    with torch.no_grad():
+        assert ops.glu_takes(h, inp) is glu and ops.split_add_takes(u, out) == add
+        assert not ops.glu_takes(h[:, 4:], inp[:, 4:]) and not ops.split_add_takes(u[:, 4:], out[:, 4:])
+    assert not ops.glu_takes(h, inp) and not ops.split_add_takes(u, out)       # gradients enabled

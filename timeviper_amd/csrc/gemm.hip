@@ -362,6 +362,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) v[r] = gelu_erf_f((float)(bf16_t)v[r]);       // the GEMM's own bf16 rounding first
           }
+          if (SPLIT && a.res) {
+            const int64_t at = (int64_t)row * a.N + col;
+            const bool more = col + 4 < a.N;
+            const f32x4 r0 = *(const f32x4*)(a.res + at), r1 = more ? *(const f32x4*)(a.res + at + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { v[r] += r0[r]; v[4 + r] += r1[r]; }
+            *(f32x4*)(a.res_out + at) = f32x4{v[0], v[1], v[2], v[3]};
+            if (more) *(f32x4*)(a.res_out + at + 4) = f32x4{v[4], v[5], v[6], v[7]};
+          }
           if (SPLIT && a.relu2) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
@@ -413,6 +422,11 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[r] += (float)b[r];
     }
+  }
+  if (a.res) {
+    const int64_t at = (int64_t)row * a.N + col;
+    s += *(const f32x4*)(a.res + at);
+    *(f32x4*)(a.res_out + at) = s;
   }
   bf16x4 o;
 #pragma unroll
@@ -531,8 +545,8 @@ extern "C" size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits) {
   return M <= 0 || N <= 0 || splits <= 1 ? 0 : (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
 }
 
-extern "C" int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
-                                 int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+static int split_fwd(const void* A, const void* W, const void* bias, const float* res, float* res_out, void* C, int64_t M, int N, int K, int64_t lda,
+                     int64_t ldw, int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
   TV_CHECK_ARG(M > 0 && N > 0 && K > 0, "gemm_split: bad sizes (M %lld N %d K %d)", (long long)M, N, K);
   TV_CHECK_ARG(A && W && C, "gemm_split: null pointer");
   TV_CHECK_ARG(epilogue == 0 || epilogue == 3, "gemm_split: epilogue %d", epilogue);
@@ -557,5 +571,18 @@ extern "C" int tv_gemm_split_fwd(const void* A, const void* W, const void* bias,
   a.part = splits > 1 ? (float*)workspace : nullptr;
   a.splits = splits;
   a.relu2 = epilogue == 3;
+  a.res = res; a.res_out = res_out;
   return launch_split(a, (hipStream_t)stream);
+}
+
+extern "C" int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
+                                 int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  return split_fwd(A, W, bias, nullptr, nullptr, C, M, N, K, lda, ldw, ldc, epilogue, bias_dtype, splits, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tv_gemm_split_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N,
+                                     int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(residual && residual_out, "gemm_split_add: null pointer");
+  if (((uintptr_t)residual & 15) || ((uintptr_t)residual_out & 15)) TV_UNSUPPORTED("gemm_split_add: the residual rows must be 16-byte aligned");
+  return split_fwd(A, W, bias, residual, residual_out, C, M, N, K, lda, ldw, N, 0, bias_dtype, splits, workspace, workspace_bytes, stream);
 }

@@ -9,7 +9,7 @@
 namespace tvgemm {
 using namespace ssdk;
 
-enum { EPI_BIAS = 0, EPI_BIAS_GELU = 1, EPI_ACCUM = 2, EPI_RELU2 = 3, EPI_BIAS_RELU2 = 4 };      // EPI_RELU2: of the fp32 sum (moe); EPI_BIAS_RELU2: of the rounded one
+enum { EPI_BIAS = 0, EPI_BIAS_GELU = 1, EPI_ACCUM = 2, EPI_RELU2 = 3, EPI_BIAS_RELU2 = 4, EPI_GLU = 5 };      // EPI_RELU2: of the fp32 sum (moe); EPI_BIAS_RELU2: of the rounded one
 
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int HALF_BYTES = 128 * BK * 2;          // one half-tile: 128 rows x 128 bytes
@@ -32,6 +32,8 @@ struct GemmArgs {
   // products whose contraction is split over work-groups: partial sums [splits][M][N], NULL where splits is 1 (tv_gemm_split_fwd)
   float* part;
   int splits, relu2;       // relu2: squared ReLU of the rounded sum
+  const float* res;        // res_out = res + sum (fp32, rows of N) and C, its bf16 copy, in the sum's place (tv_gemm_split_add_fwd); NULL: none
+  float* res_out;
 };
 
 // same formula as norms.hip's gelu_erf (A&S 7.1.26): the fused and the two-pass path agree bit for bit

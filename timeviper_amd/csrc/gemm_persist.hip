@@ -56,8 +56,13 @@ typedef unsigned u32x4e __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
 typedef __attribute__((address_space(3))) const f32x4 lds_f32x4;
 
+// EPI_GLU: a tile is 128 outputs gelu_tanh(g + bias) * (u + bias) of 256 rows; half-tile W0 holds the rows of g, W1 those of u, N further down (a.N: outputs),
+// so that a lane's quadrants (mh, 0) and (mh, 1) are the two factors of the same outputs.  g and u enter unrounded.  Saves the product's 2 N columns on the way
+// to memory and back (6 011 rows, N 5 632, K 2 048: library and gating pass 301 us, here 230).
 template <int EPI>
-__global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
+__device__ __forceinline__ void persist_tiles(const PArgs& pa) {
+  constexpr bool GLU = EPI == EPI_GLU;
+  constexpr int BNO = GLU ? BN / 2 : BN;         // outputs of a tile
   const GemmArgs& a = pa.g;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -84,7 +89,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
     const int rows = min(a.group_m, a.tiles_m - band * a.group_m);
     const int tn = in_band / rows, tm = band * a.group_m + (in_band - tn * rows);
     m0 = __builtin_amdgcn_readfirstlane(min(tm * BM, a.M - BM));
-    n0 = __builtin_amdgcn_readfirstlane(min(tn * BN, a.N - BN));
+    n0 = __builtin_amdgcn_readfirstlane(min(tn * BNO, a.N - BNO));
   };
 
   const unsigned lds0 = lds_addr_of(smem_raw);
@@ -157,7 +162,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
       const bf16_t* b = Ais + (int64_t)(tk * BK) + (int64_t)(128 * h) * lda;
       dma2(uniform_ptr(b), voffA[0], voffA[1], dst);
     } else {
-      const bf16_t* b = Wis + (int64_t)(tk * BK) + (int64_t)(128 * h) * ldw;
+      const bf16_t* b = Wis + (int64_t)(tk * BK) + (int64_t)((GLU ? a.N : 128) * h) * ldw;
       dma2(uniform_ptr(b), voffW[0], voffW[1], dst);
     }
   };
@@ -228,6 +233,45 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
     }
   };
 
+  // ---- EPI_GLU: both factors of the wave's 64 x 32 outputs in row half MH
+  auto epi_glu = [&](auto MHT, int m0, int n0, unsigned bias_lds) __attribute__((always_inline)) {
+    constexpr int MH = decltype(MHT)::value;
+    bf16_t* Cb = c_base(m0, n0);
+    const int skr = (-m0) & (BM - 1), skc = (-n0) & (BNO - 1);
+    const int lx = opaque_lane();
+    const int lane_r = 64 * wr + 16 * ((lx >> 4) & 1) + (lx & 15), lane_c = 32 * wc + 8 * (lx >> 5);
+    const unsigned lane_coff = (unsigned)((lane_r * ldc + lane_c) * 2);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int col_t = 16 * n + lane_c;
+      const bf16x8 bg = *(lds_bf16x8*)(size_t)(bias_lds + (unsigned)(col_t * 2)), bu = *(lds_bf16x8*)(size_t)(bias_lds + (unsigned)(col_t * 2 + BNO * 2));
+#pragma unroll
+      for (int mp = 0; mp < 4; mp += 2) {
+        float v[8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[MH][0][mp][n][r]), __float_as_uint(acc[MH][0][mp + 1][n][r]), false, false);
+          const auto su = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[MH][1][mp][n][r]), __float_as_uint(acc[MH][1][mp + 1][n][r]), false, false);
+          v[r] = gelu_tanh_f(__uint_as_float(sw[0]) + (float)bg[r]) * (__uint_as_float(su[0]) + (float)bu[r]);
+          v[4 + r] = gelu_tanh_f(__uint_as_float(sw[1]) + (float)bg[4 + r]) * (__uint_as_float(su[1]) + (float)bu[4 + r]);
+        }
+        u32x4e o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bf16x2 pk = {(bf16_t)v[2 * r], (bf16_t)v[2 * r + 1]};
+          o[r] = __builtin_bit_cast(unsigned, pk);
+        }
+        unsigned char* cp = (unsigned char*)(Cb + (int64_t)(128 * MH + 16 * mp) * ldc + 16 * n) + lane_coff;
+        if (128 * MH + 16 * mp + lane_r >= skr && col_t >= skc) *(u32x4e*)cp = o;
+      }
+    }
+  };
+  // quadrant (MH, NH) has become final; EPI_GLU takes both of a row half behind the second one (Q01, Q10)
+  auto epi = [&](auto MHT, auto NHT, int m0, int n0, unsigned bias_lds) __attribute__((always_inline)) {
+    if constexpr (!GLU) epi_quadrant(MHT, NHT, m0, n0, bias_lds);
+    else if constexpr (decltype(MHT)::value != decltype(NHT)::value) epi_glu(MHT, m0, n0, bias_lds);
+  };
+
   // ---- prologue: items 0 .. 6 of the first tile; W0(0) and A0(0) have landed behind vmcnt(10)
   {
     using std::integral_constant;
@@ -291,7 +335,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
     // segment — the same interval
     auto tail = [&](auto MHT, auto NHT) __attribute__((always_inline)) {
       mma_end();
-      if (KIND == KT_LAST && wr == 1) epi_quadrant(MHT, NHT, cm0, cn0, bias_cur);
+      if (KIND == KT_LAST && wr == 1) epi(MHT, NHT, cm0, cn0, bias_cur);
       __builtin_amdgcn_s_barrier();
     };
     // ---- phase 1: A0(t)
@@ -310,7 +354,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
       tsub = nkt;
     }
     if (KIND == KT_FIRST && have_prev && wr == 0)
-      epi_quadrant(I1{}, I0{}, pm0, pn0, bias_lds0 + (unsigned)((jpar ^ 1) * BIAS_SLOT));
+      epi(I1{}, I0{}, pm0, pn0, bias_lds0 + (unsigned)((jpar ^ 1) * BIAS_SLOT));
     wait();
     mma_quadrant(I0{}, I0{}, integral_constant<bool, Z>{}, wf0[DB]);
     tail(I0{}, I0{});
@@ -324,10 +368,10 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
     if (KIND == KT_FIRST && has_bias) {
       // the current tile's bias row: 1 KiB (fp32) / 512 B (bf16) into slot jpar, the same copy from every wave
       const unsigned char* bp = (const unsigned char*)a.bias + (int64_t)cn0 * (a.bias_f32 ? 4 : 2);
-      const unsigned bl = a.bias_f32 ? (unsigned)(lane * 16) : (unsigned)((lane & 31) * 16);
+      const unsigned bl = GLU ? (unsigned)((lane & 15) * 16 + (lane & 16 ? a.N * 2 : 0)) : a.bias_f32 ? (unsigned)(lane * 16) : (unsigned)((lane & 31) * 16);
       glds16(uniform_ptr(bp), bl, (unsigned)__builtin_amdgcn_readfirstlane((int)bias_cur));
     }
-    if (KIND == KT_LAST && wr == 0) epi_quadrant(I0{}, I0{}, cm0, cn0, bias_cur);
+    if (KIND == KT_LAST && wr == 0) epi(I0{}, I0{}, cm0, cn0, bias_cur);
     wait();
     mma_quadrant(I0{}, I1{}, integral_constant<bool, Z>{}, wf1);
     tail(I0{}, I1{});
@@ -338,7 +382,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
       af[m][1] = PG_LD(a_b1, TB + HALF_BYTES + m * 2048);
     }
     copy(integral_constant<int, 3>{});
-    if (KIND == KT_LAST && wr == 0) epi_quadrant(I0{}, I1{}, cm0, cn0, bias_cur);
+    if (KIND == KT_LAST && wr == 0) epi(I0{}, I1{}, cm0, cn0, bias_cur);
     wait();
     mma_quadrant(I1{}, I1{}, integral_constant<bool, Z>{}, wf1);
     tail(I1{}, I1{});
@@ -349,7 +393,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
       wf0[DB ^ 1][n][1] = PG_LD(w_b1, (TILE_BYTES - TB) + 2 * HALF_BYTES + n * 2048);
     }
     copy(integral_constant<int, 4>{});
-    if (KIND == KT_LAST && wr == 0) epi_quadrant(I1{}, I1{}, cm0, cn0, bias_cur);
+    if (KIND == KT_LAST && wr == 0) epi(I1{}, I1{}, cm0, cn0, bias_cur);
     wait();
     mma_quadrant(I1{}, I0{}, integral_constant<bool, Z>{}, wf0[DB]);
     tail(I1{}, I0{});
@@ -374,11 +418,15 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) {
   }
   if (wr == 0) {
     __builtin_amdgcn_s_barrier();          // barrier counts match again
-    epi_quadrant(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, cm0, cn0,
+    epi(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, cm0, cn0,
                  bias_lds0 + (unsigned)(jpar * BIAS_SLOT));
   }
   GEMM_WAIT_VM(0);        // the copies issued for a tile that does not exist must not land in another work-group's LDS
 }
+
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_persist_kernel(PArgs pa) { persist_tiles<EPI>(pa); }
+__global__ __launch_bounds__(512) void gemm_glu_kernel(PArgs pa) { persist_tiles<EPI_GLU>(pa); }
 
 template <int EPI>
 int launch(const PArgs& pa, int grid, hipStream_t st) {
@@ -444,3 +492,30 @@ int persist_grid() { return grid_size(); }
 
 extern "C" void tv_gemm_set_persist(int mode, int grid) { tvgemm::set_persist(mode, grid); }
 extern "C" int tv_gemm_persist_on(void) { return tvgemm::persist_on(); }
+
+extern "C" int tv_gemm_glu_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                               void* stream) {
+  using namespace tvgemm;
+  TV_CHECK_ARG(A && W && bias && C, "gemm_glu: null pointer");
+  TV_CHECK_ARG(M > 0 && N > 0 && K > 0, "gemm_glu: bad sizes (M %lld N %d K %d)", (long long)M, N, K);
+  if (K % (2 * BK) || K / BK < 4 || M < BM || N < BN / 2 || N % 8 || lda % 8 || ldw % 8 || ldc % 8 || lda < 64 || ldw < 64 || ((uintptr_t)A & 15) ||
+      ((uintptr_t)W & 15) || ((uintptr_t)C & 15) || ((uintptr_t)bias & 15))
+    TV_UNSUPPORTED("gemm_glu: K must be a multiple of %d, %d at least, M at least %d, N %d and a multiple of 8, rows 16-byte aligned", 2 * BK, 4 * BK, BM, BN / 2);
+  if (M > (1ll << 31) - BM || N > (1 << 29) || 256 * lda * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31) || 256 * ldc * 2 >= (1ll << 31))
+    TV_UNSUPPORTED("gemm_glu: sizes beyond the 32-bit offsets of the copies");
+  PArgs pa{};
+  GemmArgs& a = pa.g;
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.bias = bias; a.C = (bf16_t*)C;
+  a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc;
+  a.tiles_m = (int)((M + BM - 1) / BM); a.tiles_n = (N + BN / 2 - 1) / (BN / 2);
+  a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
+  if ((int64_t)a.tiles_m * a.tiles_n >= (1ll << 30)) TV_UNSUPPORTED("gemm_glu: too many tiles");
+  pa.ntiles = a.tiles_m * a.tiles_n;
+  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_glu_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+  if (attr != hipSuccess) {
+    tv_set_error("gemm_glu: hipFuncSetAttribute failed: %s", hipGetErrorString(attr));
+    return TV_ERR_LAUNCH;
+  }
+  gemm_glu_kernel<<<dim3((unsigned)grid_size()), 512, LDS_BYTES, (hipStream_t)stream>>>(pa);
+  TV_LAUNCH_CHECK();
+}

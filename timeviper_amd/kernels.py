@@ -1298,6 +1298,86 @@ def residual_add(x, u):
 ACT_SIGMOID, ACT_GELU_TANH = 0, 1
 
 
+def products_take(x, *weights) -> bool:
+    """What the products below need of a layer's rows and matrices: bf16 on the GPU, whole 16-byte rows, no gradients, no autocast, plain tensors."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and x.shape[0] > 0
+            and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and all(type(w) in (torch.Tensor, torch.nn.Parameter) and w.dtype == torch.bfloat16 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 8 == 0
+                    and 64 <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights))
+
+
+def glu_takes(x, weight) -> bool:
+    """Rows on which tv_gemm_glu_fwd is faster than the library's product and the pass over it: its tiles (256 rows x 128 outputs) fill half of a first round, or
+    65 % of several (us, two launches | here, 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800,
+    69 %: 95 | 90; 3 000: 146 | 136, 4 000: 186 | 146, 6 011: 301 | 230, 8 192: 405 | 285)."""
+    N, Kd = weight.shape[0] // 2, weight.shape[1]
+    tiles = -(-x.shape[0] // 256) * -(-N // 128)
+    return (x.shape[0] >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2
+            and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS)) and products_take(x, weight))
+
+
+def glu_linear(x, weight, bias, out):
+    """out = gelu_tanh(x @ Wg.T + bg) * (x @ Wu.T + bu) for the two halves of weight's rows and of the bias, on tv_gemm_glu_fwd; fp32 until the one rounding."""
+    _gpu(x, weight, bias, out)
+    N, Kd = weight.shape[0] // 2, weight.shape[1]
+    if (x.dtype != torch.bfloat16 or weight.dtype != x.dtype or out.dtype != x.dtype or weight.shape[0] % 2 or x.shape[1] != Kd or x.stride(1) != 1
+            or weight.stride(1) != 1 or out.stride(1) != 1 or out.shape != (x.shape[0], N)):
+        raise TimeViperHipError(f"glu_linear: {tuple(x.shape)} bf16 against {tuple(weight.shape)} into {tuple(out.shape)}")
+    _bf16_bias(bias, 2 * N, "glu_linear")
+    check(_capi.lib().tv_gemm_glu_fwd(_p(x), _p(weight), _p(bias), _p(out), x.shape[0], N, Kd, x.stride(0), weight.stride(0), out.stride(0), _stream()),
+          "tv_gemm_glu_fwd")
+    return out
+
+
+def split_add_takes(x, weight) -> int:
+    """Work-groups a tile with which tv_gemm_split_add_fwd is faster than the library's product and the pass that adds it, 0 where it is not: a contraction of 4 096
+    columns or more whose tiles, shared, fill 75 % of one round, 16 work-groups a tile at most (us, two launches | here, 2 048 x 7 680: 40 rows 30 | 20, 256: 30 | 30,
+    700: 42 | 41, 1 000: 51 | 47, 2 100: 82 | 74, 4 000: 124 | 115; whole tiles, 6 011: 160 | 168)."""
+    N, Kd = weight.shape
+    tiles = -(-x.shape[0] // 256) * -(-N // 256)
+    splits = min(CUS // tiles, 16, Kd // 192) if tiles else 0
+    pays = splits >= 2 and (tiles * splits >= 0.75 * CUS or splits == 16) and Kd >= 4096 and Kd % 64 == 0 and N >= 1024 and N % 4 == 0
+    return splits if pays and products_take(x, weight) else 0
+
+
+def split_add_linear(x, weight, residual, bias=None, splits=1):
+    """(residual + x @ weight.T (+ bias) in fp32, its bf16 copy): `split_linear` with the residual stream behind it"""
+    _gpu(x, weight, residual, bias)
+    N, Kd = weight.shape
+    if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[1] != Kd or x.stride(1) != 1 or weight.stride(1) != 1 or residual.dtype != torch.float32
+            or residual.shape != (x.shape[0], N) or not residual.is_contiguous()):
+        raise TimeViperHipError(f"split_add_linear: {tuple(x.shape)} bf16 against {tuple(weight.shape)} onto {tuple(residual.shape)} fp32")
+    if bias is not None:
+        _bf16_bias(bias, N, "split_add_linear")
+    lib, M = _capi.lib(), x.shape[0]
+    res, h = torch.empty_like(residual), torch.empty((M, N), dtype=x.dtype, device=x.device)
+    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib.tv_gemm_split_add_fwd(_p(x), _p(weight), _p(bias), _p(residual), _p(res), _p(h), M, N, Kd, x.stride(0), weight.stride(0), TV_BF16, splits,
+                                    _p(ws), need, _stream()), "tv_gemm_split_add_fwd")
+    return res, h
+
+
+def side_takes(h, table, gate, proj) -> bool:
+    """Shapes tv_token_side_fwd is written for: a side of 128 columns."""
+    return gate.shape[0] == 128 and gate.shape[1] % 32 == 0 and table.stride(0) % 4 == 0 and products_take(h, gate, proj) and table.data_ptr() % 8 == 0 \
+        and table.dtype == torch.bfloat16 and table.stride(1) == 1
+
+
+def token_side(h, ids, table, gate, proj):
+    """proj @ (gelu_tanh(gate @ h) * table[ids]) for the rows of h in one launch (tv_token_side_fwd); ids are checked where the step was planned"""
+    _gpu(h, ids, table, gate, proj)
+    T, D = h.shape
+    S = gate.shape[0]
+    if (any(t.dtype != torch.bfloat16 or t.stride(1) != 1 for t in (h, table, gate, proj)) or gate.shape != (S, D) or proj.shape != (D, S) or table.shape[1] != S
+            or ids.dtype != torch.int64 or ids.numel() != T or not ids.is_contiguous()):
+        raise TimeViperHipError(f"token_side: rows {tuple(h.shape)} with {tuple(gate.shape)}, {tuple(proj.shape)} and a table {tuple(table.shape)}")
+    y = torch.empty((T, D), dtype=h.dtype, device=h.device)
+    check(_capi.lib().tv_token_side_fwd(_p(h), _p(ids), _p(table), _p(gate), _p(proj), _p(y), T, D, S, table.shape[0], h.stride(0), table.stride(0),
+                                        gate.stride(0), proj.stride(0), D, _stream()), "tv_token_side_fwd")
+    return y
+
+
 def gated_mul(a, b, act, ids=None, out=None):
     """f(a) * b over rows, f = sigmoid or the tanh form of gelu; `ids` (int64): row r meets b[ids[r]].  `out`: rows to write to."""
     _gpu(a, b, ids, out)

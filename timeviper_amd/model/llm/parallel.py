@@ -49,6 +49,8 @@ class TokenSide(nn.Module):
 
     def forward(self, h, ids, rows):
         """h: the stream in the model's dtype; rows (vocab, dim): this layer's slice of the table"""
+        if K.side_takes(h, rows, self.gate, self.proj):
+            return K.token_side(h, ids, rows, self.gate, self.proj)
         return F.linear(K.gated_mul(F.linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
 
     def decode(self, h, ids, rows):
@@ -84,8 +86,13 @@ class ParallelLayer(nn.Module):
         u = torch.empty((x.shape[0], self.out.shape[1]), dtype=hs.dtype, device=hs.device)
         self.mixer.attend(F.linear(hs, self.inp[:self.n1]), kv_rows, plan, out=u[:, :self.k1])
         if self.mlp is not None:
-            K.gated_mul(*self.mlp.split(F.linear(h, self.inp[self.n1:], self.inp_bias)), K.ACT_GELU_TANH, out=u[:, self.k1:])
-        x, h = K.residual_add(x, F.linear(u, self.out, self.out_bias))
+            w, act = self.inp[self.n1:], u[:, self.k1:]
+            if K.glu_takes(h, w) and self.k1 % 8 == 0:
+                K.glu_linear(h, w, self.inp_bias, act)
+            else:
+                K.gated_mul(*self.mlp.split(F.linear(h, w, self.inp_bias)), K.ACT_GELU_TANH, out=act)
+        splits = K.split_add_takes(u, self.out)
+        x, h = K.split_add_linear(u, self.out, x, self.out_bias, splits) if splits else K.residual_add(x, F.linear(u, self.out, self.out_bias))
         return x, (self.side(h, ids, side_rows), self.side.norm)
 
     def decode_takes(self, rows, dtype):
