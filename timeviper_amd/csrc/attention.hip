@@ -1,7 +1,7 @@
 // A1 / T3 / ViT: fused softmax attention forward on CDNA4 MFMA tiles.
 //
 // Structure (wave64, v_mfma_f32_32x32x16): a workgroup of 8 waves owns 256 query
-// rows of one (batch, q-head) (4 waves / 128 rows for short queries); each wave keeps
+// rows of one (batch, q-head) (128 with half of the keys a wave where those are too few work-groups); each wave keeps
 // its 32 query rows as MFMA B fragments in registers for the whole kernel.  K/V tiles
 // of 96 keys arrive by LDS-DMA into a 3-stage ring shared by the waves, two tiles ahead
 // of the math (counted vmcnt, one barrier per tile).  The score tile is computed
@@ -120,20 +120,24 @@ __device__ __forceinline__ void block_of(int id, int pairs, int& t, int& pair) {
 // XOR-swizzled on the DMA source address so that the row reads of K (ds_read_b128, chunk ^
 // row%16) and the transposing reads of V (ds_read_b64_tr_b16, chunk ^ 4(row%4)) are bank
 // conflict free.  Chunks past head_dim are never copied (the K ones QK^T reads are zeroed once).
+// KG 2: the first four waves and the last four hold the same 128 query rows and take every second tile of 32 KT keys each; two tiles are a step, two stages a
+// ring, and the halves (maximum, sum, accumulators) meet in LDS at the end.  A short grid is a chain of steps that lasts as long as the longest row of keys: this
+// halves it with the same two waves a SIMD (1 000 tokens, 40 heads: 41.0 -> 31.2 us).  Long grids lose by it: K and V go into LDS once per 128 rows.
 // WIN: causal with a sliding window and kept first keys.  The work-group visits the tiles that hold kept keys, then jumps to the
 // first tile of its first row's window: ring, copies and waits count the visited tiles.  All sequences of a packed step share the
 // launch (a launch per prompt leaves most of the chip idle: six prompts, 6 011 tokens, 16 heads on 4 x 128, window 1 024: 265 us, in one launch 95).
-template <typename T, int KS, int DT, int NW, int KT, bool WIN = false>
+template <typename T, int KS, int DT, int NW, int KT, bool WIN = false, int KG = 1>
 __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename std::conditional<WIN, AttnSeqs, NoSeqs>::type sq) {
   constexpr int FA_KB = 32 * KT;     // keys per tile
-  constexpr int NPK = FA_KB / 4;     // 1 KiB DMA pieces (4 key rows) of K per tile; as many of V
+  constexpr int TPK = FA_KB / 4;     // 1 KiB DMA pieces (4 key rows) of K per tile
+  constexpr int NPK = KG * TPK;      // ... and per step; as many of V
   typedef typename Frag<T>::v8 v8;
   typedef typename Frag<T>::v4 v4;
-  constexpr int QB = NW * FA_QW;     // query rows per workgroup
+  constexpr int QB = NW / KG * FA_QW;     // query rows per workgroup
   constexpr int ROWB = 256;          // LDS bytes per key row
-  constexpr int TILEB = FA_KB * ROWB;
-  constexpr int NS = 3;              // ring stages
-  constexpr int PPW = 2 * NPK / NW;  // DMA pieces per wave and tile
+  constexpr int TILEB = KG * FA_KB * ROWB;      // of a step
+  constexpr int NS = KG == 1 ? 3 : 2;           // ring stages
+  constexpr int PPW = 2 * NPK / NW;  // DMA pieces per wave and step
   static_assert(2 * NPK % NW == 0, "pieces must divide over the waves");
   extern __shared__ __attribute__((aligned(16))) unsigned char fa_smem[];
   unsigned char* const sK = fa_smem;
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 31, hh = lane >> 5;
-  // 1-D grid (but for NW = 4).  Few sequences: `block_of` (causal: the heaviest query blocks of all heads first).  Many short sequences (ViT
+  // 1-D grid.  Few sequences: `block_of` (causal: the heaviest query blocks of all heads first).  Many short sequences (ViT
   // frames): ids walk the query blocks of ONE (batch, head) on one XCD (id % 8): the blocks that
   // share K / V then share an L2 instead of pulling the same keys into three of them
   int qblk, h, b, Lq = a.Lq, Lk = a.Lk;
@@ -171,10 +175,6 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     h = pair % a.Hq;
     b = pair / a.Hq;
     if (b >= a.nb) return;                    // (batch, head) pairs are padded to a multiple of 8
-  } else if constexpr (NW == 4) {               // up to 128 query rows: one block, a 3-D grid with heads and batch entries
-    qblk = a.causal ? (gridDim.x - 1 - blockIdx.x) : blockIdx.x;
-    h = blockIdx.y;
-    b = blockIdx.z;
   } else {
     const int pairs = a.nb * a.Hq;
     int pair;
@@ -184,7 +184,8 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     h = pair - b * a.Hq;
   }
   const int hk = WIN ? __builtin_amdgcn_readfirstlane(h / (a.Hq / a.Hkv)) : h / (a.Hq / a.Hkv);
-  const int q0 = qblk * QB + wave * FA_QW;      // first query row of this wave
+  const int grp = KG == 1 ? 0 : wave / (NW / KG);                        // which of a step's tiles this wave takes
+  const int q0 = qblk * QB + (wave - grp * (NW / KG)) * FA_QW;      // first query row of this wave
   const int qrow = q0 + r;                      // this lane's query row
   const int D = a.D;
   const int shift = Lk - Lq;                // bottom-right causal alignment
@@ -199,8 +200,8 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   if (D < 16 * KS) {
     const v8 z = {};
     const int c0 = D / 8, nc = 2 * KS - c0;
-    for (int i = tid; i < NS * FA_KB * nc; i += NW * 64) {
-      const int row = (i / nc) % FA_KB, st = i / (nc * FA_KB), c = c0 + i % nc;
+    for (int i = tid; i < NS * KG * FA_KB * nc; i += NW * 64) {
+      const int row = (i / nc) % (KG * FA_KB), st = i / (nc * KG * FA_KB), c = c0 + i % nc;
       *reinterpret_cast<v8*>(sK + st * TILEB + row * ROWB + ((c ^ (row & 15)) << 4)) = z;
     }
   }
@@ -234,6 +235,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     ntiles -= tskip;
   }
   auto key_of_tile = [&](int kt) __attribute__((always_inline)) { return (WIN && kt >= tkeep ? kt + tskip : kt) * FA_KB; };
+  const int nsteps = (ntiles + KG - 1) / KG;
 
   // ---- DMA pieces of this wave: piece id pc = wave + NW*i; pc < 16 -> K rows 4pc..4pc+3,
   // else V rows 4(pc-16)..; lane l carries row 4(pc%16) + l/16, LDS slot l%16 ----
@@ -244,17 +246,18 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   for (int i = 0; i < PPW; ++i) {
     const int pc = wave + NW * i;
     const bool isK = pc < NPK;
-    const int row = 4 * (isK ? pc : pc - NPK) + (lane >> 4);
+    const int row = 4 * ((isK ? pc : pc - NPK) % TPK) + (lane >> 4);
     const int c = (lane & 15) ^ (isK ? (row & 15) : 4 * (row & 3));
     p_row[i] = row;
     p_chunk[i] = c < (isK ? a.D : a.Dv) / 8 ? c : 255;
     p_off[i] = (unsigned)(((int64_t)row * (isK ? a.ksl : a.vsl) + c * 8) * (int)sizeof(T));
   }
-  auto issue_piece = [&](int kt, int i) {          // piece i (0..PPW-1) of tile kt
-    const int kbase = key_of_tile(kt);
+  auto issue_piece = [&](int kt, int i) {          // piece i (0..PPW-1) of step kt
     const int stage = kt % NS;
     const int pc = wave + NW * i;
     const bool isK = pc < NPK;           // wave-uniform
+    // (a step's second tile may not exist: the last one again, nobody reads it)
+    const int kbase = key_of_tile(KG == 1 ? kt : min(kt * KG + (isK ? pc : pc - NPK) / TPK, ntiles - 1));
     const void* tb = ssdk::uniform_ptr(isK ? (const void*)(kp + (int64_t)kbase * a.ksl)
                                            : (const void*)(vp + (int64_t)kbase * a.vsl));
     const int left = Lk - kbase;          // rows of this tile that exist
@@ -286,9 +289,9 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   }
 
   __syncthreads();                 // LDS zeroed before the first copy lands
-  if (ntiles > 0) issue_tile(0);
-  if (ntiles > 1) issue_tile(1);
-  if (ntiles > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
+  if (nsteps > 0) issue_tile(0);
+  if (NS > 2 && nsteps > 1) issue_tile(1);
+  if (NS > 2 && nsteps > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -298,18 +301,19 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     qf[ks] = (qrow < Lq && ks * 16 + hh * 8 < D) ? __builtin_bit_cast(v8, qraw[ks]) : z;
   }
 
-  for (int kt = 0; kt < ntiles; ++kt) {
-    const int kbase = key_of_tile(kt);
-    const bool ahead = kt + 2 < ntiles;
+  for (int kt = 0; kt < nsteps; ++kt) {
+    const int kbase = key_of_tile(KG == 1 ? kt : kt * KG + grp);
+    const bool ahead = kt + NS - 1 < nsteps;
     // stage bases as LDS byte offsets (scalar), folded into one base register per fragment family
-    const unsigned stage_off = (unsigned)((kt % NS) * TILEB);
+    const unsigned stage_off = (unsigned)((kt % NS) * TILEB + grp * (FA_KB * ROWB));
     const unsigned cK = sK_off + stage_off, cV = sV_off + stage_off;
 
     // wave-uniform skip of tiles entirely above this wave's causal diagonal
     const int wave_q_last = q0 + FA_QW - 1;
     bool active = !(a.causal && kbase > wave_q_last + shift);
     if constexpr (WIN) active = active && (kbase < a.keep || kbase + FA_KB > q0 + shift - a.window + 1);
-    if (!active && ahead) issue_tile(kt + 2);
+    if (KG > 1) active = active && kt * KG + grp < ntiles;
+    if (!active && ahead) issue_tile(kt + NS - 1);
     if (active) {
       // ---- S^T = K . Q^T  (2 key sub-tiles of 32); all K fragment reads ahead of the MFMAs;
       // the copies of tile kt+2 are issued between the MFMAs, whose pipe time hides them ----
@@ -333,12 +337,12 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
           // PPW pieces spread over the 2*KS MFMAs
           constexpr int every = (KT * KS) / PPW > 0 ? (KT * KS) / PPW : 1;
           const int idx = t * KS + ks;
-          if (ahead && idx % every == 0 && idx / every < PPW) issue_piece(kt + 2, idx / every);
+          if (ahead && idx % every == 0 && idx / every < PPW) issue_piece(kt + NS - 1, idx / every);
         }
       }
       if (ahead) {      // pieces that did not fit the spacing (PPW > 2*KS)
 #pragma unroll
-        for (int i = (KT * KS) / ((KT * KS) / PPW > 0 ? (KT * KS) / PPW : 1); i < PPW; ++i) issue_piece(kt + 2, i);
+        for (int i = (KT * KS) / ((KT * KS) / PPW > 0 ? (KT * KS) / PPW : 1); i < PPW; ++i) issue_piece(kt + NS - 1, i);
       }
       // ---- mask, running max on the raw scores (the scale is positive, so it commutes with
       // max), then p = 2^(s*scale - m) as one FMA + v_exp per score; packed fp32 math ----
@@ -428,7 +432,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
       }
     }
     // tile kt+1 (issued an iteration ago) must have landed; this iteration's copies stay in flight
-    if (ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
+    if (NS > 2 && ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -436,6 +440,37 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
 
   // ---- epilogue: normalise and store O[q][d] ----
   float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  // KG 2: the two waves of a row meet over the ring; the first keeps the first half of the d-tiles, the second the rest
+  constexpr int DH = (DT + 1) / 2;
+  if constexpr (KG == 2) {
+    f32x4* const xo = (f32x4*)fa_smem;                    // [wave][d-tile of the partner][4][lane]
+    float* const xm = (float*)(fa_smem + NW * DH * 4 * 64 * 16);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      if ((dt < DH) == (grp == 1)) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          xo[((wave * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + lane] = f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+      }
+    xm[(wave * 2 + 0) * 64 + lane] = m_run;
+    xm[(wave * 2 + 1) * 64 + lane] = l_tot;
+    __syncthreads();
+    const int other = wave ^ (NW / 2);
+    const float m_o = xm[(other * 2 + 0) * 64 + lane], l_o = xm[(other * 2 + 1) * 64 + lane], m_all = fmaxf(m_run, m_o);
+    const float f = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_all), f_o = m_o == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_o - m_all);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      if ((dt < DH) == (grp == 0)) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 v = xo[((other * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + lane];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) oacc[dt][4 * g + j] = oacc[dt][4 * g + j] * f + v[j] * f_o;
+        }
+      }
+    l_tot = l_tot * f + l_o * f_o;
+    m_run = m_all;
+  }
   if (a.sink) l_tot += __builtin_amdgcn_exp2f(a.sink[h] * 1.4426950408889634f - m_run);      // (not scaled; inf: the keys weigh nothing)
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (qrow < Lq) {
@@ -445,6 +480,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int d0 = dt * 32 + 8 * g + 4 * hh;
+        if (KG == 2 && (dt < DH) != (grp == 0)) continue;
         if (d0 < a.Dv) {
           v4 pk;
           if constexpr (WIN) {
@@ -459,7 +495,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
           *(v4*)(op + d0) = pk;
         }
       }
-    if (!WIN && a.lse && hh == 0) {
+    if (!WIN && a.lse && hh == 0 && grp == 0) {
       const float lse = l_tot > 0.f ? (m_run * 0.6931471805599453f + logf(l_tot)) : -INFINITY;
       a.lse[((int64_t)b * a.Hq + h) * Lq + qrow] = lse;
     }
@@ -885,18 +921,31 @@ __global__ __launch_bounds__(512) void flash_fwd_stream_kernel(AttnArgs a) {
 
 std::atomic<int> g_fa_variant{[] { const char* v = getenv("TV_FA_W64"); return v ? atoi(v) : 0; }()};
 
+// Whether two waves share 32 query rows (KG 2): up to 128 rows (64 against 4 096 keys, 40 heads: 131 us with one wave a SIMD, 88; 128: 14.7, 11.7), while 128-row
+// blocks are one round of the compute units (40 heads x 700: 31.8 | 24.2), and twice as many where they grow from nothing, since the short ones share
+// (40 x 1 400: 51.7 | 46.7, 28 x 2 000: 66.4 | 58.3; 40 x 2 000, 320 blocks of 256: 70.4 | 84.7; 48 whole rows of 729, 288 of 128: 27.1 | 39.5).
+bool two_waves_a_row(int Lq, int64_t blocks256, int64_t blocks128, bool triangle) {
+  return Lq <= 128 || blocks128 <= tv_cu_count() || (triangle && blocks256 <= tv_cu_count());
+}
+constexpr int FA_LDS2 = 2 * 2 * 2 * 64 * 256;    // K and V of two steps of 128 keys
+
 template <typename T, int KS, int DT>
 int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   constexpr int KT = FA_KT;
   constexpr int lds = 2 * 3 * 32 * KT * 256;   // K and V rings: 3 stages x 32 KT rows x 256 B
   hipError_t e;
-  if (a.Lq > 128) {
+  const int64_t all = (int64_t)a.Hq * B;
+  const int nqb = (a.Lq + 255) / 256;
+  static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
+  const bool frames = a.Lq > 128 && xcd_ && !a.causal && nqb <= 8 && all >= 64;
+  if (!frames && two_waves_a_row(a.Lq, nqb * all, (a.Lq + 127) / 128 * all, a.causal && a.Lk - a.Lq <= a.Lq / 4)) {
+    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS2);
+    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 8, 2, false, 2><<<dim3((unsigned)((a.Lq + 127) / 128 * all)), 512, FA_LDS2, st>>>(a, NoSeqs{});
+  } else {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, KT>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e == hipSuccess) {
-      const int nqb = (a.Lq + 255) / 256;
-      static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
-      if (xcd_ && !a.causal && nqb <= 8 && (int64_t)B * a.Hq >= 64) {
+      if (frames) {
         AttnArgs ax = a;
         ax.nqb = nqb;
         ax.nb = B;
@@ -933,14 +982,8 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
           flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax, NoSeqs{});
         }
       } else {
-        flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)((int64_t)nqb * a.Hq * B)), 512, lds, st>>>(a, NoSeqs{});
+        flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(nqb * all)), 512, lds, st>>>(a, NoSeqs{});
       }
-    }
-  } else {
-    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e == hipSuccess) {
-      flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
     }
   }
   if (e != hipSuccess) {
@@ -950,26 +993,33 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-// windowed form: bf16, one query block of 256 (or, if no sequence has more than 128 rows, 128) rows a work-group; 64-key tiles at head dim
-// 128 (the bounds of the window do not fit beside 96 keys' fragments)
+// windowed form: bf16, 64-key tiles at head dim 128 (the bounds of the window do not fit beside 96 keys' fragments).  Blocks of 256 rows, or of 128 with two waves a
+// row: if no sequence is longer, while those are one round, and for more where the sequences start from nothing, the more the more of them there are (one
+// prompt, 16 heads, window 1 024: 1 200 rows 54 | 37 us, 2 560: 65 | 54, 3 200: 64 | 75; two, 3 000 together: 63 | 53, 3 500: 63 | 66; four, 3 000: 61 | 45, 4 000: 64 | 61;
+// six, 4 500: 65 | 68; 32 x 100 rows behind 1 000 keys 116 | 81).
 template <int KS, int DT>
 int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) {
   constexpr int KT = KS > 6 ? 2 : FA_KT, lds = 2 * 3 * 32 * KT * 256;
   int most = 0;
-  for (int s = 0; s < nseq; ++s) most = sq.len_q[s] > most ? sq.len_q[s] : most;
-  const bool big = most > 128;
-  const int qb = big ? 256 : 128;
-  int64_t blocks = 0;
-  for (int s = 0; s < nseq; ++s) blocks += (sq.len_q[s] + qb - 1) / qb;
-  const void* f = big ? (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true> : (const void*)flash_fwd_kernel<bf16_t, KS, DT, 4, KT, true>;
-  const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  int64_t blocks = 0, blocks128 = 0;
+  bool triangle = true;
+  for (int s = 0; s < nseq; ++s) {
+    most = sq.len_q[s] > most ? sq.len_q[s] : most;
+    blocks += (sq.len_q[s] + 255) / 256;
+    blocks128 += (sq.len_q[s] + 127) / 128;
+    triangle = triangle && sq.len_k[s] - sq.len_q[s] <= sq.len_q[s] / 4;
+  }
+  const int64_t cus = tv_cu_count();
+  const bool two = most <= 128 || blocks128 * a.Hq <= cus || (triangle && blocks * a.Hq * 6 <= cus * (nseq < 3 ? 3 + nseq : 6));
+  const void* f = two ? (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2> : (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true>;
+  const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, two ? FA_LDS2 : lds);
   if (e != hipSuccess) {
     tv_set_error("flash_attn: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     return TV_ERR_LAUNCH;
   }
-  const dim3 grid((unsigned)(blocks * a.Hq));
-  if (big) flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<grid, 512, lds, st>>>(a, sq);
-  else flash_fwd_kernel<bf16_t, KS, DT, 4, KT, true><<<grid, 256, lds, st>>>(a, sq);
+  const dim3 grid((unsigned)((two ? blocks128 : blocks) * a.Hq));
+  if (two) flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2><<<grid, 512, FA_LDS2, st>>>(a, sq);
+  else flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<grid, 512, lds, st>>>(a, sq);
   TV_LAUNCH_CHECK();
 }
 
@@ -985,7 +1035,7 @@ int launch_fa(const AttnArgs& a, int B, hipStream_t st) {
   // One grid dimension takes fewer than 2^32 work-items: a batch with more query blocks than that goes in slices
   const int64_t blocks = (int64_t)((a.Lq + 255) / 256) * a.Hq;                        // of a batch entry, 512 work-items each
   const int64_t most = blocks < (1 << 22) ? ((1 << 23) - 64) / blocks : 1;           // (pairs are padded to a multiple of 8 in one form)
-  if (a.Lq > 128 && B > most) {
+  if (B > most) {
     for (int64_t b = 0; b < B; b += most) {
       AttnArgs s = a;
       s.q = (const T*)a.q + b * a.qsb; s.k = (const T*)a.k + b * a.ksb; s.v = (const T*)a.v + b * a.vsb; s.o = (T*)a.o + b * a.osb;
