@@ -1,0 +1,56 @@
+"""The fp32 scan on the matrix cores (csrc/ssd_f32.hip) against chunks in 64 bits: ends of chunks and of segments, segments of one chunk and of several, operands that
+keep the general kernels."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def reference(x, d, A, Bm, Cm, D, S, of):
+    """(y, final state, magnitudes of both): x (B, L, H, P) ... in 64 bits, 32 tokens at a time"""
+    L, H = x.shape[1:3]
+    y, mag, Sm = torch.empty_like(x), torch.empty_like(x), S.abs()
+    for t in range(0, L, 32):
+        xt, dt, b, c = (v[:, t:t + 32].transpose(1, 2).contiguous() for v in (x, d, Bm[:, :, of], Cm[:, :, of]))
+        cs = torch.cumsum(dt * A[:, None], 2)
+        M = torch.exp((cs[..., :, None] - cs[..., None, :]).masked_fill(~torch.ones(cs.shape[2], cs.shape[2], dtype=torch.bool, device=DEV).tril(), -float("inf")))
+        xd, bt, e, w = xt * dt[..., None], b.transpose(2, 3).contiguous(), torch.exp(cs)[..., None], torch.exp(cs[..., -1:] - cs)[..., None]
+        for o, f, s in ((y, lambda v: v, S), (mag, torch.abs, Sm)):
+            o[:, t:t + 32] = (torch.matmul(M * torch.matmul(f(c), f(bt)), f(xd)) + e * torch.matmul(f(c), s.transpose(2, 3).contiguous())
+                              + f(D)[:, None, None] * f(xt)).transpose(1, 2)
+        step = lambda f, s: torch.exp(cs[..., -1])[..., None, None] * s + torch.matmul((f(xd) * w).transpose(2, 3).contiguous(), f(b))
+        S, Sm = step(lambda v: v, S), step(torch.abs, Sm)
+    return y, S, mag, Sm
+
+
+@pytest.mark.parametrize("B,L,H,P,G,group_map,init", [(1, 65, 2, 16, 1, "block", True), (2, 128, 4, 48, 2, "tile", False), (1, 129, 4, 64, 4, "block", True),
+                                                      (2, 1000, 32, 128, 2, "block", True), (1, 4096, 32, 64, 2, "tile", False)])
+@pytest.mark.parametrize("form", ["dense", "rows", "general"])
+def test_against_64_bits(B, L, H, P, G, group_map, init, form):
+    """rows: operands as slices of wider rows; general: rows off the 16-byte pieces"""
+    from timeviper_amd import kernels as ops
+    N = 16
+    g = torch.Generator(device=DEV).manual_seed(L + P)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    off = {"dense": 0, "rows": 8, "general": 3}[form]
+    wide = lambda *s: r(*s[:2], s[2] * s[3] + off)[..., off:].unflatten(2, s[2:])
+    x, Bm, Cm = wide(B, L, H, P), 0.3 * r(B, G, L, N + off)[..., off:].transpose(1, 2), wide(B, L, G, N)
+    dt, A, bias, D = r(B, L, H), -torch.linspace(0.01, 8, H, device=DEV), torch.linspace(-4, 0, H, device=DEV), r(H)
+    S0 = r(B, H, P, N) if init else None
+    y, fin, dec = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=S0, return_final_states=True,
+                                                return_total_decay=True, group_map=group_map)
+    assert ops.ssd_scan_last_impl() == 8
+    of = torch.arange(H, device=DEV) % G if group_map == "tile" else torch.arange(H, device=DEV) // (H // G)
+    d = F.softplus(dt.double() + bias.double())
+    want, S, mag, Sm = reference(x.double(), d, A.double(), Bm.double(), Cm.double(), D.double(), torch.zeros(B, H, P, N, device=DEV, dtype=torch.float64)
+                                 if S0 is None else S0.double(), of)
+    # a few hundred rounded terms (2^-18 of their magnitudes) and exponents that are differences of prefix sums of 64 tokens (2^-21 of the sum)
+    rel = 2.0 ** -18 + 2.0 ** -21 * 64 * (d * A.double()).abs().mean(1).max().item()
+    assert ((y.double() - want).abs() <= mag * rel + 1e-9).all()
+    assert ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
+    assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5, atol=1e-6)
+    if form == "dense":
+        only = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=S0, group_map=group_map)
+        assert torch.equal(only, y)

@@ -1,0 +1,211 @@
+// S3 (fp32, d_state 16, head_dim a multiple of 16): the chunked scan of ssd_chunked.hip on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: fp32 products
+// and sums, 4 columns of contraction a step).
+//
+// ssd_chunked.hip's work-groups were LDS reads: an operand a fused multiply-add from LDS, x and M through it, y written, read back and written again.  Here a WAVE takes
+// 16 columns of a head through a segment of chunks of 64 tokens, and nothing but the tokens' decays passes LDS, because the operands chain:
+//   * G^T = B C^T puts, in a lane, four source tokens of one output token (rows 4 (lane / 16) + r, column lane % 16); numbering the four steps of a
+//     contraction of 16 tokens the same way (step r, quarter q: token 4 q + r), M^T = decays x dt x G^T is the operand of Y^T += x^T M^T as it leaves G;
+//   * the state S^T += (w B)^T x leaves, in a lane, four entries n of one column p: the operand of Y^T = S C^T as it is, and 16-byte rows in memory;
+//   * Y^T leaves four neighbouring columns of one token: 16-byte stores.
+// Two launches: the state that every segment but the last leaves from a zero start; then a segment folds its predecessors' (in order, as the recurrence) and
+// marches, writing y once.  Segments are as long as leaves two waves a SIMD; the fold reads 1 KB a predecessor and wave.
+// Products for a wave and chunk: 40 for G (again by each of a head's P / 16 waves), 40 + 16 for Y, 16 for S, 32 cycles each.
+// Measured (32 heads x 64, 2 groups; ssd_chunked.hip's kernels -> here): 1 024 tokens 38 -> 21 us, 4 096: 128 -> 52, 2 x 4 096: 226 -> 91,
+// 2 x 128: 23 -> 13.  Error of the final state against 64 bits 1.3e-7 (5e-7 .. 3e-6 with weights of differences of sums), of y 1.6e-7 (1.9e-7).
+#include "ssd_common.hpp"
+
+namespace {
+using namespace ssdk;
+
+constexpr int FQ = 64, FN = 16;       // tokens a chunk, d_state
+
+struct F3Args {
+  const float *x, *dt, *Bm, *Cm, *A, *D, *dt_bias, *init;
+  float *y, *final_state, *total_decay;
+  float *loc, *segdec;                // [segment][batch][head][P][16] local states, [segment][batch][head] sums of dt A
+  int L, H, P, G, nch, nseg, seg_chunks;
+  int64_t xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl;
+  int softplus, group_map;
+  float dt_min, dt_max;
+};
+
+__device__ __forceinline__ float rdlane(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+__device__ __forceinline__ float from_lane(float v, int l) { return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * l, __float_as_int(v))); }
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// OUT: the second launch
+template <bool OUT>
+__global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
+  __shared__ __attribute__((aligned(16))) float sv[4][3][FQ];         // a wave's own: cs, dt, weights of the state
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lc = lane & 15, q = lane >> 4;
+  const int pt_n = a.P >> 4, unit = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
+  const int seg = unit / pt_n, pt = unit - seg * pt_n;
+  if (seg >= (OUT ? a.nseg : a.nseg - 1)) return;                     // (no barrier in this kernel)
+  const int c0 = seg * a.seg_chunks, c1 = min(c0 + a.seg_chunks, a.nch);
+  const int g = a.group_map ? h % a.G : h / (a.H / a.G);
+  const float* const xb = a.x + (int64_t)b * a.xsb + (int64_t)h * a.P + 16 * pt;
+  const float* const Bb = a.Bm + (int64_t)b * a.bsb + (int64_t)g * a.bsg;
+  const float* const Cb = a.Cm + (int64_t)b * a.csb + (int64_t)g * a.csg;
+  const float* const db = a.dt + (int64_t)b * a.dsb + h;
+  const float Ah = a.A[h], bias = a.dt_bias ? a.dt_bias[h] : 0.f, Dh = OUT && a.D ? a.D[h] : 0.f;
+  const int64_t bh = (int64_t)b * a.H + h, nbh = (int64_t)gridDim.z * a.H, PN = (int64_t)a.P * FN;
+  const int64_t mine = bh * PN + (16 * pt + lc) * FN + 4 * q;         // this lane's four state entries: column 16 pt + lc, n = 4 q ..
+
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  float before = 0.f;
+  if constexpr (OUT) {
+    if (a.init) S = *(const f32x4*)(a.init + mine);
+    if (seg > 0) {
+      const float sd = lane < seg ? a.segdec[lane * nbh + bh] : 0.f, e = __expf(sd);
+      for (int j0 = 0; j0 < seg; j0 += 8) {
+        f32x4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = *(const f32x4*)(a.loc + min(j0 + j, seg - 1) * (nbh * PN) + mine);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (j0 + j < seg) {
+            const float f = rdlane(e, j0 + j);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[r] = fmaf(f, S[r], v[j][r]);
+          }
+      }
+      if (seg == a.nseg - 1) for (int j = 0; j < seg; ++j) before += rdlane(sd, j);
+    }
+  }
+  float own = 0.f;
+  for (int c = c0; c < c1; ++c) {
+    const int t0 = c * FQ, tt = min(FQ, a.L - t0);
+    const bool next = !OUT || c + 1 < c1 || (c + 1 == a.nch && a.final_state);        // the state behind this chunk is wanted
+    const float raw = db[(int64_t)(t0 + min(lane, tt - 1)) * a.dsl];
+    float xa[4][4], bn[4][4];
+    f32x4 ba[4], ca[4], xd[4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t t = t0 + min(16 * st + 4 * q + r, tt - 1);
+        xa[st][r] = xb[t * a.xsl + lc];
+        bn[st][r] = Bb[t * a.bsl + lc];
+      }
+    if constexpr (OUT) {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const int64_t t = t0 + min(16 * st + lc, tt - 1);
+        ba[st] = *(const f32x4*)(Bb + t * a.bsl + 4 * q);
+        ca[st] = *(const f32x4*)(Cb + t * a.csl + 4 * q);
+        xd[st] = *(const f32x4*)(xb + t * a.xsl + 4 * q);
+      }
+    }
+    float d = raw + bias;
+    if (a.softplus) d = softplus_f(d);
+    d = lane < tt ? fminf(fmaxf(d, a.dt_min), a.dt_max) : 0.f;
+    const float da = d * Ah, cs = wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
+    // what decays behind a token, summed from the end: cend - cs would carry the rounding of the whole chunk's sum into the tokens that weigh most
+    const float back = from_lane(wave_incl_scan_dpp(from_lane(da, 63 - lane)), 62 - lane);
+    own += cend;
+    sv[wave][0][lane] = cs;
+    sv[wave][1][lane] = d;
+    sv[wave][2][lane] = lane == 63 ? d : __expf(back) * d;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (a wave's own LDS: in order)
+    if (tt < FQ) {                                                    // rows past the end are zeros, as tokens that are not there
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * st + 4 * q + r >= tt) xa[st][r] = bn[st][r] = 0.f;
+        if (OUT && 16 * st + lc >= tt) ba[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    if constexpr (OUT) {
+      f32x4 css[4], ds[4];
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        css[st] = *(const f32x4*)&sv[wave][0][16 * st + 4 * q];
+        ds[st] = *(const f32x4*)&sv[wave][1][16 * st + 4 * q];
+      }
+#pragma unroll
+      for (int ot = 0; ot < 4; ++ot) {                                // 16 output tokens
+        const float cst = sv[wave][0][16 * ot + lc], et = __expf(cst);
+        f32x4 Y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) Y = mfma4(S[k], ca[ot][k], Y);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Y[r] *= et;
+#pragma unroll
+        for (int st = 0; st <= ot; ++st) {
+          f32x4 M = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) M = mfma4(ba[st][k], ca[ot][k], M);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float m = __expf(cst - css[st][r]) * ds[st][r] * M[r];
+            M[r] = st < ot || 4 * q + r <= lc ? m : 0.f;
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) Y = mfma4(xa[st][r], M[r], Y);
+        }
+        if (16 * ot + lc < tt) {
+          f32x4 o;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = fmaf(Dh, xd[ot][r], Y[r]);
+          *(f32x4*)(a.y + (int64_t)b * a.ysb + (int64_t)(t0 + 16 * ot + lc) * a.ysl + (int64_t)h * a.P + 16 * pt + 4 * q) = o;
+        }
+      }
+    }
+    if (next) {
+      const float ec = __expf(cend);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[r] *= ec;
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const f32x4 w = *(const f32x4*)&sv[wave][2][16 * st + 4 * q];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S = mfma4(w[r] * bn[st][r], xa[st][r], S);
+      }
+    }
+    asm volatile("" ::: "memory");                                    // (the next chunk's vectors are written behind this one's reads)
+  }
+  if constexpr (!OUT) {
+    *(f32x4*)(a.loc + seg * (nbh * PN) + mine) = S;
+    if (pt == 0 && lane == 0) a.segdec[seg * nbh + bh] = own;
+  } else if (seg == a.nseg - 1) {
+    if (a.final_state) *(f32x4*)(a.final_state + mine) = S;
+    if (a.total_decay && pt == 0 && lane == 0) a.total_decay[bh] = before + own;
+  }
+}
+
+}  // namespace
+
+// called from ssd_chunked.hip: fp32 shapes whose rows are read and written in 16-byte pieces
+bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
+                          int64_t ysb, int64_t ysl, const void* x, const void* Bm, const void* Cm, const void* y, const void* init,
+                          const void* final_state) {
+  const int64_t strides = xsb | xsl | bsb | bsl | bsg | csb | csl | csg | ysb | ysl;
+  const uintptr_t at = (uintptr_t)x | (uintptr_t)Bm | (uintptr_t)Cm | (uintptr_t)y | (uintptr_t)init | (uintptr_t)final_state;
+  return dstate == FN && headdim % 16 == 0 && strides % 4 == 0 && at % 16 == 0;
+}
+
+int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias,
+                      const void* init_state, void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups,
+                      int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
+                      int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map, void* workspace, hipStream_t st) {
+  F3Args a;
+  a.x = (const float*)x; a.dt = (const float*)dt; a.Bm = (const float*)Bm; a.Cm = (const float*)Cm; a.A = (const float*)A; a.D = (const float*)D;
+  a.dt_bias = (const float*)dt_bias; a.init = (const float*)init_state; a.y = (float*)y; a.final_state = (float*)final_state;
+  a.total_decay = (float*)total_decay;
+  a.L = seqlen; a.H = nheads; a.P = headdim; a.G = ngroups; a.nch = (seqlen + FQ - 1) / FQ;
+  const int64_t waves = (int64_t)batch * nheads * (headdim / 16) * a.nch;
+  int64_t len = waves / (8ll * tv_cu_count());                        // (two waves a SIMD; one: 2 x 4 096 tokens 92 | 105 us, four: 93, 2 x 1 024: 31 | 35, 36)
+  if (len < (a.nch + 63) / 64) len = (a.nch + 63) / 64;               // (the fold keeps a segment's decay a lane)
+  a.seg_chunks = (int)(len < 1 ? 1 : len > a.nch ? a.nch : len);
+  a.nseg = (a.nch + a.seg_chunks - 1) / a.seg_chunks;
+  a.loc = (float*)workspace;
+  a.segdec = a.loc + (int64_t)a.nseg * batch * nheads * headdim * FN;
+  a.xsb = xsb; a.xsl = xsl; a.dsb = dsb; a.dsl = dsl; a.bsb = bsb; a.bsl = bsl; a.bsg = bsg; a.csb = csb; a.csl = csl; a.csg = csg; a.ysb = ysb; a.ysl = ysl;
+  a.softplus = dt_softplus; a.group_map = group_map; a.dt_min = dt_min; a.dt_max = dt_max;
+  const int units = headdim / 16 * a.nseg;
+  if (a.nseg > 1) ssd_f32_kernel<false><<<dim3((unsigned)((units - headdim / 16 + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
+  ssd_f32_kernel<true><<<dim3((unsigned)((units + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
+  TV_LAUNCH_CHECK();
+}
