@@ -38,9 +38,9 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _gpu(*ts: Optional[torch.Tensor]) -> None:
-    cur = None
+    cur = -1
     for t in ts:
-        if t is None:
+        if t is None or (cur >= 0 and t.get_device() == cur):
             continue
         if not t.is_cuda:
             raise TimeViperHipError(
@@ -48,18 +48,18 @@ def _gpu(*ts: Optional[torch.Tensor]) -> None:
                 "there is no CPU fallback in the product path"
             )
         # the launch goes to the CURRENT device's stream (`_stream`): a tensor of another device
-        # would hand that stream foreign pointers.  One process drives one GPU here (SURVEY 8e).
-        if cur is None:
-            cur = torch.cuda.current_device()
-        if t.device.index != cur:
+        # would hand that stream foreign pointers.  One process drives one GPU here.
+        # (a GPU tensor exists: torch.cuda.current_device()'s look at the initialisation is half of its time)
+        cur = torch._C._cuda_getDevice()
+        if t.get_device() != cur:
             raise TimeViperHipError(
-                f"tensor on cuda:{t.device.index} but the current device is cuda:{cur}: "
+                f"tensor on cuda:{t.get_device()} but the current device is cuda:{cur}: "
                 "call torch.cuda.set_device() (one process per GPU)")
 
 
 def _stream() -> int:
     # the handle alone: a torch.cuda.Stream object around it takes 6 us of every launch
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -69,6 +69,14 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
 def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """t, dense and of `dtype` (two calls into torch saved where it is both)"""
     return t if t.dtype is dtype and t.is_contiguous() else t.to(dtype).contiguous()
+
+
+def _like_rows(t: torch.Tensor):
+    """(rows, row stride, empty tensor of t's shape) of dense t, without the views that `_rows2d` makes; else None"""
+    D = t.shape[-1]
+    if D == 0 or not t.is_contiguous():
+        return None
+    return t.numel() // D, D, torch.empty_like(t, memory_format=torch.contiguous_format)
 
 
 def _rows2d(t: torch.Tensor) -> torch.Tensor:
@@ -129,13 +137,15 @@ def causal_conv1d_xbc(xBC, weight, bias, d_inner: int, ngroups: int, dstate: int
     if xBC.stride(2) != 1:
         xBC = xBC.contiguous()
     K = weight.shape[-1]
-    w = weight.reshape(Cc, K).to(xBC.dtype).contiguous()
-    b = None if bias is None else bias.to(xBC.dtype).contiguous()
+    w = _as(weight if weight.dim() == 2 else weight.reshape(Cc, K), xBC.dtype)
+    if w.shape[0] != Cc:
+        w = w.reshape(Cc, K)
+    b = None if bias is None else _as(bias, xBC.dtype)
     if halo is not None:
-        halo = halo.to(xBC.dtype).contiguous()
-    yx = torch.empty((Bsz, L, d_inner), dtype=xBC.dtype, device=xBC.device)
-    yb = torch.empty((Bsz, ngroups, L, dstate), dtype=xBC.dtype, device=xBC.device)
-    yc = torch.empty((Bsz, ngroups, L, dstate), dtype=xBC.dtype, device=xBC.device)
+        halo = _as(halo, xBC.dtype)
+    yx = xBC.new_empty((Bsz, L, d_inner))
+    yb = xBC.new_empty((Bsz, ngroups, L, dstate))
+    yc = torch.empty_like(yb)
     lib = _capi.lib()
     if return_cb and xBC.dtype == torch.bfloat16 and dstate == 128 and L > 0:
         cb = torch.empty(lib.tv_ssd_cb_bytes(Bsz, L, ngroups) // 2, dtype=torch.bfloat16, device=xBC.device)
@@ -176,12 +186,18 @@ def rms_norm(x, weight, eps, residual=None, return_sum=False):
     s = x + residual (rounded to x.dtype like the reference's bf16 add, :966) and
     can return s too."""
     _gpu(x, weight, residual)
+    w = weight if weight.dtype in (torch.float32, x.dtype) else weight.to(torch.float32)
+    w = w.contiguous()
+    dense = _like_rows(x) if residual is None or (residual.is_contiguous() and residual.shape == x.shape) else None
+    if dense:
+        (n, D, y), s = dense, torch.empty_like(x) if return_sum and residual is not None else None
+        check(_capi.lib().tv_rmsnorm_fwd(_p(x), _p(residual), _p(w), _p(s), _p(y), n, D, D, 0 if residual is None else D, 0 if s is None else D, D, float(eps),
+                                         _dt(x), _dt(w), _stream()), "tv_rmsnorm_fwd")
+        return (y, x if s is None else s) if return_sum else y
     x2 = _rows2d(x)
     r2 = None if residual is None else _rows2d(residual)
     y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
     s = torch.empty_like(y) if (return_sum and residual is not None) else None
-    w = weight if weight.dtype in (torch.float32, x.dtype) else weight.to(torch.float32)
-    w = w.contiguous()
     check(_capi.lib().tv_rmsnorm_fwd(
         _p(x2), _p(r2), _p(w), _p(s), _p(y), x2.shape[0], x2.shape[1], x2.stride(0),
         0 if r2 is None else r2.stride(0), 0 if s is None else s.stride(0), y.stride(0),
@@ -198,13 +214,18 @@ def layer_norm(x, weight, bias, eps, residual=None, return_sum=False, row_bias=N
     `row_bias` (D,) fp32: a constant row added to every s before the statistics (not to the
     returned sum): the projection biases a caller carries beside a stream its GEMMs accumulate into."""
     _gpu(x, weight, bias, residual, row_bias)
+    w = _as(weight, x.dtype)
+    b = None if bias is None else _as(bias, x.dtype)
+    rb = None if row_bias is None else _as(row_bias, torch.float32)
+    dense = _like_rows(x) if residual is None else None
+    if dense:
+        n, D, y = dense
+        check(_capi.lib().tv_layernorm_fwd(_p(x), None, _p(w), _p(b), _p(rb), None, _p(y), n, D, D, 0, 0, D, float(eps), _dt(x), _stream()), "tv_layernorm_fwd")
+        return (y, x) if return_sum else y
     x2 = _rows2d(x)
     r2 = None if residual is None else _rows2d(residual)
     y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
     s = torch.empty_like(y) if (return_sum and residual is not None) else None
-    w = _as(weight, x.dtype)
-    b = None if bias is None else _as(bias, x.dtype)
-    rb = None if row_bias is None else _as(row_bias, torch.float32)
     check(_capi.lib().tv_layernorm_fwd(
         _p(x2), _p(r2), _p(w), _p(b), _p(rb), _p(s), _p(y), x2.shape[0], x2.shape[1], x2.stride(0),
         0 if r2 is None else r2.stride(0), 0 if s is None else s.stride(0), y.stride(0), float(eps),
@@ -242,13 +263,21 @@ def rmsnorm_fn(x, weight, bias=None, z=None, eps=1e-6, group_size=None,
     if z is not None and norm_before_gate:
         raise TimeViperHipError("rmsnorm_fn: only norm_before_gate=False is on the path")
     _gpu(x, weight, z)
-    x2 = _rows2d(x)
-    z2 = None if z is None else _rows2d(z)
-    D = x2.shape[1]
+    D = x.shape[-1]
     gs = D if group_size is None else int(group_size)
-    y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
     w = weight if weight.dtype in (torch.float32, x.dtype) else weight.to(torch.float32)
     w = w.contiguous()
+    # (z: a slice of a wider projection, whose rows of one batch entry lie one distance apart)
+    if z is None or (z.dim() == 3 and z.shape == x.shape and z.stride(2) == 1 and (z.shape[0] == 1 or z.stride(0) == z.shape[1] * z.stride(1))):
+        dense = _like_rows(x)
+        if dense:
+            n, _, y = dense
+            check(_capi.lib().tv_rmsnorm_gated_fwd(_p(x), _p(z), _p(w), _p(y), n, D, gs, D, 0 if z is None else z.stride(1), D, float(eps), _dt(x), _dt(w),
+                                                   _stream()), "tv_rmsnorm_gated_fwd")
+            return y
+    x2 = _rows2d(x)
+    z2 = None if z is None else _rows2d(z)
+    y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
     check(_capi.lib().tv_rmsnorm_gated_fwd(
         _p(x2), _p(z2), _p(w), _p(y), x2.shape[0], D, gs, x2.stride(0),
         0 if z2 is None else z2.stride(0), y.stride(0), float(eps), _dt(x), _dt(w), _stream()),
@@ -332,6 +361,8 @@ def _row_view(t: torch.Tensor, inner: int):
     """(B, L, ...) tensor whose trailing dims are contiguous with `inner`
     elements per row: return (tensor, stride_b, stride_l) without copying when
     the rows are dense (slices of a wider projection keep their row stride)."""
+    if t.is_contiguous():
+        return t, t.stride(0), t.stride(1)
     ok = t.stride(-1) == 1
     exp = 1
     for d in range(t.dim() - 1, 1, -1):
@@ -375,9 +406,9 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size=None, D=None, z=None, d
         C = C.contiguous()
     bsb, bsl, bsg = B.stride(0), B.stride(1), B.stride(2)
     csb, csl, csg = C.stride(0), C.stride(1), C.stride(2)
-    f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
+    f32 = lambda t: None if t is None else _as(t, torch.float32)
     A, D, dt_bias, initial_states = f32(A), f32(D), f32(dt_bias), f32(initial_states)
-    y = torch.empty((Bsz, L, H, P), dtype=x.dtype, device=x.device)
+    y = x.new_empty((Bsz, L, H, P))
     final = torch.empty((Bsz, H, P, N), dtype=torch.float32, device=x.device) \
         if return_final_states else None
     decay = torch.empty((Bsz, H), dtype=torch.float32, device=x.device) \
