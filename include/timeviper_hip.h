@@ -626,6 +626,12 @@ int tv_gemm_split_add_fwd(const void* A, const void* W, const void* bias, const 
 int tv_gemm_glu_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                     void* stream);
 
+/* C = epilogue(A W^T) for a few hundred to a few thousand rows (csrc/gemm_small.hip), epilogue 0 (bias), 1 (bias, exact GELU of the rounded sum), 2 (C += the sum) as
+ * tv_gemm_bf16_fwd, or 5: tv_gemm_glu_fwd's (bf16 bias of 2 N, N outputs).  tile: 0, 1: 128 x 128 outputs a work-group (ring of four stages, of two), 2: 64 x 128, 3:
+ * 64 x 64 (half as many outputs with epilogue 5).  K % 64 == 0, N % 8 == 0, everything 16-byte aligned. */
+int tv_gemm_small_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                      int epilogue, int bias_dtype, int tile, void* stream);
+
 /* y = P (gelu_tanh(G h) * e), e the table's row of each token (csrc/token_side.hip): h (rows, width) bf16, G (dim, width), P (width, dim), table (table_rows,
  * dim) with a row stride of its own; ids outside the table count as rows of zeros.  width % 32 == 0, dim 128. */
 int tv_token_side_fwd(const void* h, const int64_t* ids, const void* table, const void* gate, const void* proj, void* y, int64_t rows, int width,

@@ -1,0 +1,90 @@
+"""Products on small tiles (tv_gemm_small_fwd): edges of the three tiles, one to many stages of 64 columns, every epilogue; where they replace the library's."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (63, 72, 128), (65, 64, 192), (128, 128, 256), (129, 136, 320), (300, 264, 1152)])
+def test_against_64_bits(M, N, K, tile):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, w, b, c = r(M, K + 16).to(BF)[:, 8:8 + K], (K ** -0.5 * r(N, K)).to(BF), r(N), r(M, N).to(BF)
+    s = x.double() @ w.double().T
+    sums = (x.double().abs() @ w.double().abs().T + 4) * K * 2.0 ** -24       # fp32 sums in any order
+    one = lambda v, e: e + 2.0 ** -8 * (v.abs() + e)                           # ... and one rounding
+    for bias in (None, b, b.to(BF)):
+        want = s if bias is None else s + bias.double()
+        got = ops.small_linear(x, w, bias, tile=tile).double()
+        assert ((got - want).abs() <= one(want, sums)).all()
+        got = ops.small_linear(x, w, bias, ops.GEMM_BIAS_GELU, tile=tile).double()
+        want, e = F.gelu(want), 1.13 * one(want, sums) + 1e-6                 # the GELU of the rounded sum: its slope is below 1.13
+        assert ((got - want).abs() <= one(want, e)).all()
+    wide = torch.full((M, N + 16), 7.0, device=DEV, dtype=BF)
+    out = wide[:, 8:8 + N]
+    out.copy_(c)
+    ops.small_linear(x, w, None, ops.GEMM_ACCUM, out=out, tile=tile)
+    assert ((out.double() - (s + c.double())).abs() <= one(s + c.double(), sums)).all() and (wide[:, :8] == 7).all() and (wide[:, 8 + N:] == 7).all()
+    w2, b2 = (K ** -0.5 * r(2 * N, K)).to(BF), r(2 * N).to(BF)
+    f, u = (x.double() @ w2.double().T + b2.double()).split(N, 1)
+    want = F.gelu(f, approximate="tanh") * u
+    got = ops.small_linear(x, w2, b2, ops.GEMM_GLU, tile=tile).double()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * (f.abs() + 1) * (u.abs() + 1)).all()
+
+
+def test_refused():
+    from timeviper_amd import kernels as ops
+    z = lambda *s: torch.zeros(s, device=DEV, dtype=BF)
+    for x, w, kw in ((z(9, 96), z(64, 96), {}), (z(9, 64), z(60, 64), {}), (z(9, 68)[:, 4:], z(64, 64), {}), (z(9, 64), z(64, 64), dict(epilogue=ops.GEMM_ACCUM)),
+                     (z(9, 64), z(64, 64), dict(epilogue=ops.GEMM_GLU)), (z(9, 64), z(64, 64), dict(tile=4)), (z(9, 64), z(64, 64), dict(epilogue=3))):
+        with pytest.raises(ops.TimeViperHipError):
+            ops.small_linear(x, w, **kw)
+
+
+# rows x outputs x columns: both sides of each line
+@pytest.mark.parametrize("rows,n,k,glu,tile", [(1, 1152, 1152, False, -1), (2, 1152, 1152, False, 3), (729, 1152, 1152, False, 3), (1458, 1152, 1152, False, 2), (729, 3456, 1152, False, 2),
+                                               (1458, 3456, 1152, False, 1), (2304, 3456, 1152, False, 1), (2305, 3456, 1152, False, -1), (2187, 4352, 1152, False, -1),
+                                               (1458, 1152, 4352, False, 3), (2187, 1152, 4352, False, -1), (729, 1152, 8192, False, -1), (200, 5632, 2048, True, 0),
+                                               (512, 5632, 2048, True, 1), (700, 5632, 2048, True, -1), (729, 504, 1152, False, -1), (729, 1152, 1120, False, -1)])
+def test_rule(rows, n, k, glu, tile):
+    from timeviper_amd import kernels as ops
+    x, w = torch.empty(rows, k, device=DEV, dtype=BF), torch.empty(n * (2 if glu else 1), k, device=DEV, dtype=BF)
+    assert ops.small_tile(rows, n, k, glu) == tile and ops.small_takes(x, w, glu) == -1       # gradients enabled
+    with torch.no_grad():
+        assert ops.small_takes(x, w, glu) == tile and ops.small_takes(x, w, glu, most=rows - 1) == -1
+        assert ops.small_takes(x[:, 4:], w[:, 4:], glu) == -1 and ops.small_takes(x.float(), w.float(), glu) == -1
+
+
+@pytest.mark.parametrize("frames", [1, 3])
+def test_short_clips(frames, monkeypatch):
+    """a block of a short clip on small tiles, and on the library where something stands around its layers"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.vit.siglip import Block
+    torch.manual_seed(frames)
+    blk = Block(1152, 16, 4304).to(DEV, BF).requires_grad_(False)
+    x = torch.randn(frames, 729, 1152, device=DEV, dtype=BF)
+    calls, real = [], ops.small_linear
+    monkeypatch.setattr(ops, "small_linear", lambda x, w, *a, **k: (calls.append(w.shape[0]), real(x, w, *a, **k))[1])
+    with torch.no_grad():
+        got = [blk.forward_stream(x.clone(), None)]
+        assert calls == ([3456, 1152, 4352, 1152] if frames == 1 else [3456, 1152])
+        hooks = [m.register_forward_hook(lambda *a: None) for m in (blk.attn.qkv, blk.mlp.fc1)]
+        calls.clear()
+        got.append(blk.forward_stream(x.clone(), None))
+        assert 3456 not in calls and 4352 not in calls
+        for h in hooks:
+            h.remove()
+        z = x.double()
+        f = lambda m: torch.nn.functional.linear if m is None else (lambda t: F.linear(t, m.weight.double(), m.bias.double()))
+        n = lambda m, t: F.layer_norm(t, (1152,), m.weight.double(), m.bias.double(), m.eps)
+        q, k, v = (t.transpose(1, 2).contiguous() for t in f(blk.attn.qkv)(n(blk.norm1, z)).view(frames, 729, 3, 16, 72).unbind(2))
+        a = torch.softmax(torch.matmul(q, k.transpose(2, 3).contiguous()) * 72 ** -0.5, -1)
+        z = z + f(blk.attn.proj)(torch.matmul(a, v).transpose(1, 2).reshape(frames, 729, 1152))
+        z = z + f(blk.mlp.fc2)(F.gelu(f(blk.mlp.fc1)(n(blk.norm2, z))))
+    for y, pend in got:
+        assert ((y.double() + pend.double() - z).norm() / z.norm()) < 6e-3    # (bf16 between the operators)

@@ -1,0 +1,257 @@
+// bf16 products of a few hundred to a few thousand rows, C = epilogue(A W^T), on small tiles: 128 x 128, 64 x 128 or 64 x 64 outputs a work-group of four waves.
+//
+// gemm.hip's 256 x 256 tiles are a quarter of a round there, and each takes its whole contraction (729 rows: 42 - 51 tiles, 26 us however short it is).  Small tiles
+// fill the compute units; what bounds them is the way into the compute unit (a stage of 64 columns is 16 - 32 KB, at about 70 bytes a ns), so the tile is the
+// largest that still gives the chip a round (kernels.small_tile).
+//   * a wave holds a quarter of the tile; both operands arrive by LDS-DMA (8 rows x 128 bytes an instruction, 16-byte pieces exchanged on the source side so that
+//     fragment reads meet no bank twice) in a ring of NS stages, NS - 1 ahead of the products behind counted waits, one barrier a stage;
+//   * v_mfma_f32_16x16x32_bf16 with W on the A side: two tiles of rows joined by v_permlane16_swap are 16-byte stores, as gemm.hip;
+//   * EPI_GLU: half of a tile's rows of W are those of the gate, half those of the factor N rows further down: a lane holds both of an output.
+// fp32 sums, one rounding; the GELU is that of the rounded sum (what the library's product would have written).
+// Measured (us, library -> here, on the device): 729 x 3 456 x 1 152 15.0 -> 13.8, 729 x 1 152 x 1 152 9.5 -> 7.5, 729 x 1 152 x 4 352 18.7 -> 19.4, 200 x (2 x 5 632) x 2 048 with the
+// gate 26 + 5 -> 23; with the library's 19 us of host time gone: SigLIP so400m, 1 frame 4.1 -> 2.8 ms, 2 frames 4.1 -> 3.3.
+#include "gemm_common.hpp"
+
+namespace tvgemm {
+namespace {
+
+typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
+
+// WM, WN: a wave's 16-row tiles of A and of W
+template <int WM, int WN, int NS, int EPI>
+__global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
+  constexpr int TM = 32 * WM, TN = 32 * WN, STAGE = (TM + TN) * 128, PA = TM / 8, PW = (TM + TN) / 32;
+  constexpr bool GLU = EPI == EPI_GLU;
+  constexpr int TO = GLU ? TN / 2 : TN;                    // outputs a tile
+  extern __shared__ __attribute__((aligned(16))) unsigned char gs_smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 1, wc = wave & 1, lc = lane & 15, kq = lane >> 4;
+
+  // ---- tile: ids of an XCD (id % 8) walk neighbouring tiles, bands of group_m tiles of rows
+  int id = blockIdx.x;
+  {
+    const int nt = a.tiles_m * a.tiles_n, q = nt / 8, r = nt % 8, x = id % 8;
+    id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + id / 8;
+  }
+  const int band = id / (a.group_m * a.tiles_n), in_band = id % (a.group_m * a.tiles_n), rows_in_band = min(a.group_m, a.tiles_m - band * a.group_m);
+  const int m0 = (band * a.group_m + in_band % rows_in_band) * TM, n0 = in_band / rows_in_band * TO;
+
+  // ---- copies: this wave's pieces of a stage, the rows of A first.  Rows past the end repeat the last one (never stored)
+  const unsigned lds0 = lds_addr_of(gs_smem);
+  const bf16_t* src[PW];
+  unsigned off[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int pc = wave * PW + i;
+    const bool isA = pc < PA;
+    const int row = 8 * (isA ? pc : pc - PA) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+    int64_t r;
+    if (isA) r = min(row, a.M - 1 - m0);
+    else if (GLU) r = row < TO ? min(row, a.N - 1 - n0) : (int64_t)a.N + min(row - TO, a.N - 1 - n0);
+    else r = min(row, a.N - 1 - n0);
+    src[i] = (const bf16_t*)uniform_ptr(isA ? a.A + (int64_t)m0 * a.lda : a.W + (int64_t)n0 * a.ldw);
+    off[i] = (unsigned)((r * (isA ? a.lda : a.ldw) + ch * 8) * 2);
+  }
+  const int nkt = a.K / BK;
+  auto issue = [&](int t, int S) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) glds16(uniform_ptr(src[i] + t * BK), off[i], lds0 + (unsigned)(S * STAGE + (wave * PW + i) * 1024));
+  };
+
+  f32x4 acc[WM][WN];
+#pragma unroll
+  for (int m = 0; m < WM; ++m)
+#pragma unroll
+    for (int n = 0; n < WN; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned frag = lds0 + (unsigned)(lc * 128 + ((kq ^ (lc >> 1)) << 4));
+  const unsigned fa = frag + (unsigned)(wr * WM * 2048), fw = frag + (unsigned)(TM * 128);
+  // row of the tile's rows of W at which a wave's tile n starts
+  auto w_row = [&](int n) __attribute__((always_inline)) {
+    return GLU ? (n < WN / 2 ? 0 : TO) + 16 * (wc * (WN / 2) + n % (WN / 2)) : 16 * (wc * WN + n);
+  };
+#pragma unroll
+  for (int j = 0; j < NS - 1; ++j)
+    if (j < nkt) issue(j, j);
+  // fragments of stage t, in slot S, both k-steps
+  bf16x8 af[2][2][WM], wf[2][2][WN];
+  auto read = [&](int S, auto BT) __attribute__((always_inline)) {
+    constexpr int B = decltype(BT)::value;
+    const unsigned st = (unsigned)(S * STAGE);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int m = 0; m < WM; ++m) af[B][ks][m] = *(lds_bf16x8*)(size_t)((fa + st + (unsigned)(m * 2048)) ^ (unsigned)(ks * 64));
+#pragma unroll
+      for (int n = 0; n < WN; ++n) wf[B][ks][n] = *(lds_bf16x8*)(size_t)((fw + st + (unsigned)(w_row(n) * 128)) ^ (unsigned)(ks * 64));
+    }
+  };
+  auto multiply = [&](auto BT) __attribute__((always_inline)) {
+    constexpr int B = decltype(BT)::value;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int m = 0; m < WM; ++m)
+#pragma unroll
+        for (int n = 0; n < WN; ++n) acc[m][n] = mfma16(wf[B][ks][n], af[B][ks][m], acc[m][n]);
+  };
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, 1> I1;
+  if constexpr (NS < 4) {
+    int S = 0;
+    for (int t = 0; t < nkt; ++t) {
+      if (t + NS - 2 < nkt) GEMM_WAIT_VM(PW * (NS - 2));
+      else GEMM_WAIT_VM(0);
+      __builtin_amdgcn_s_barrier();                        // stage t is there for all waves, and all have read stage t - 1
+      asm volatile("" ::: "memory");
+      if (t + NS - 1 < nkt) issue(t + NS - 1, S == 0 ? NS - 1 : S - 1);
+      read(S, I0{});
+      multiply(I0{});
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      S = S == NS - 1 ? 0 : S + 1;
+    }
+  } else {
+    // four stages: the fragments of stage t + 1 are read while stage t is multiplied; the wait and the barrier of a step are for the stage behind (4 352
+    // columns on 64 x 64 tiles 23.6 -> 19.4 us, on 128 x 128 48 -> 40; with three stages the fragments' second set costs more than it hides, 31 -> 39)
+    int S = 0;                                             // slot of stage t
+    auto step = [&](int t, auto BT) __attribute__((always_inline)) {
+      constexpr int B = decltype(BT)::value;
+      const int S1 = S == NS - 1 ? 0 : S + 1;
+      if (t + 1 < nkt) {
+        if (t + NS - 2 < nkt) GEMM_WAIT_VM(PW * (NS - 3));
+        else GEMM_WAIT_VM(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave has read stage t, and so stage t - 1, whose slot is filled next
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t + NS - 1 < nkt) issue(t + NS - 1, S == 0 ? NS - 1 : S - 1);
+        read(S1, std::integral_constant<int, B ^ 1>{});
+      }
+      multiply(BT);
+      S = S1;
+    };
+    if (nkt > NS - 2) GEMM_WAIT_VM(PW * (NS - 2));
+    else GEMM_WAIT_VM(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, I0{});
+    int t = 0;
+    for (; t + 1 < nkt; t += 2) {
+      step(t, I0{});
+      step(t + 1, I1{});
+    }
+    if (t < nkt) step(t, I0{});
+  }
+
+  // ---- epilogue: a lane holds, of two joined tiles of rows, 8 columns 16 n + 8 (kq >> 1) .. of row 16 (m + (kq & 1)) + lc
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned u32x4e __attribute__((ext_vector_type(4)));
+  constexpr int NO = GLU ? WN / 2 : WN;
+#pragma unroll
+  for (int n = 0; n < NO; ++n) {
+    const int col = n0 + 16 * (wc * NO + n) + 8 * (kq >> 1);
+    float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, bu[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (EPI != EPI_ACCUM && a.bias && col < a.N) {         // (N is a multiple of 8)
+      if (a.bias_f32) {
+        const f32x4 b0 = *(const f32x4*)((const float*)a.bias + col), b1 = *(const f32x4*)((const float*)a.bias + col + 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { bv[r] = b0[r]; bv[4 + r] = b1[r]; }
+      } else {
+        const bf16x8 b8 = *(const bf16x8*)((const bf16_t*)a.bias + col);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) bv[r] = (float)b8[r];
+        if (GLU) {
+          const bf16x8 u8 = *(const bf16x8*)((const bf16_t*)a.bias + a.N + col);
+#pragma unroll
+          for (int r = 0; r < 8; ++r) bu[r] = (float)u8[r];
+        }
+      }
+    }
+#pragma unroll
+    for (int mp = 0; mp < WM; mp += 2) {
+      float v[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[mp][n][r]), __float_as_uint(acc[mp + 1][n][r]), false, false);
+        v[r] = __uint_as_float(sw[0]) + bv[r];
+        v[4 + r] = __uint_as_float(sw[1]) + bv[4 + r];
+        if constexpr (GLU) {
+          const auto su = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[mp][n + NO][r]), __float_as_uint(acc[mp + 1][n + NO][r]), false, false);
+          v[r] = gelu_tanh_f(v[r]) * (__uint_as_float(su[0]) + bu[r]);
+          v[4 + r] = gelu_tanh_f(v[4 + r]) * (__uint_as_float(su[1]) + bu[4 + r]);
+        }
+      }
+      const int row = m0 + 16 * (wr * WM + mp + (kq & 1)) + lc;
+      if (row >= a.M || col >= a.N) continue;
+      bf16_t* cp = a.C + (int64_t)row * a.ldc + col;
+      if (EPI == EPI_ACCUM) {
+        const bf16x8 c8 = *(const bf16x8*)cp;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[r] += (float)c8[r];
+      }
+      if (EPI == EPI_BIAS_GELU) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[r] = gelu_erf_f((float)(bf16_t)v[r]);
+      }
+      u32x4e o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bf16x2 pk = {(bf16_t)v[2 * r], (bf16_t)v[2 * r + 1]};
+        o[r] = __builtin_bit_cast(unsigned, pk);
+      }
+      *(u32x4e*)cp = o;
+    }
+  }
+}
+
+template <int WM, int WN, int NS, int EPI>
+int go_epi(GemmArgs& a, hipStream_t st) {
+  constexpr int TM = 32 * WM, TO = EPI == EPI_GLU ? 16 * WN : 32 * WN, LDS = NS * (TM + 32 * WN) * 128;
+  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_small_kernel<WM, WN, NS, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (attr != hipSuccess) {
+    tv_set_error("gemm_small: cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr));
+    return TV_ERR_LAUNCH;
+  }
+  a.tiles_m = (a.M + TM - 1) / TM;
+  a.tiles_n = (a.N + TO - 1) / TO;
+  a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
+  gemm_small_kernel<WM, WN, NS, EPI><<<dim3((unsigned)(a.tiles_m * a.tiles_n)), 256, LDS, st>>>(a);
+  TV_LAUNCH_CHECK();
+}
+template <int WM, int WN, int NS>
+int go(GemmArgs& a, int epilogue, hipStream_t st) {
+  switch (epilogue) {
+    case EPI_BIAS: return go_epi<WM, WN, NS, EPI_BIAS>(a, st);
+    case EPI_BIAS_GELU: return go_epi<WM, WN, NS, EPI_BIAS_GELU>(a, st);
+    case EPI_ACCUM: return go_epi<WM, WN, NS, EPI_ACCUM>(a, st);
+    default: return go_epi<WM, WN, NS, EPI_GLU>(a, st);
+  }
+}
+
+}  // namespace
+}  // namespace tvgemm
+
+extern "C" int tv_gemm_small_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                                 int epilogue, int bias_dtype, int tile, void* stream) {
+  using namespace tvgemm;
+  TV_CHECK_ARG(A && W && C, "gemm_small: null pointer");
+  TV_CHECK_ARG(M > 0 && N > 0 && K > 0 && tile >= 0 && tile <= 3, "gemm_small: bad sizes (M %lld N %d K %d, tile %d)", (long long)M, N, K, tile);
+  TV_CHECK_ARG(epilogue == EPI_BIAS || epilogue == EPI_BIAS_GELU || epilogue == EPI_ACCUM || epilogue == EPI_GLU, "gemm_small: epilogue %d", epilogue);
+  TV_CHECK_ARG(bias ? bias_dtype == TV_BF16 || (bias_dtype == TV_F32 && epilogue != EPI_GLU) : epilogue != EPI_GLU, "gemm_small: bias dtype %d", bias_dtype);
+  if (K % BK || N % 8 || lda % 8 || ldw % 8 || ldc % 8 || lda < 0 || ldw < 0 || ldc < 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) || ((uintptr_t)C & 15) ||
+      ((uintptr_t)bias & 15))
+    TV_UNSUPPORTED("gemm_small: K must be a multiple of %d, N of 8, rows 16-byte aligned (K %d N %d lda %lld ldw %lld ldc %lld)", BK, K, N, (long long)lda,
+                   (long long)ldw, (long long)ldc);
+  if (M > (1ll << 24) || 128 * lda * 2 >= (1ll << 31) || ((epilogue == EPI_GLU ? (int64_t)N : 0) + 128) * ldw * 2 >= (1ll << 31) ||
+      ((M + 63) / 64) * ((N + 31) / 32) >= (1ll << 31))
+    TV_UNSUPPORTED("gemm_small: sizes beyond the 32-bit offsets of the copies");
+  GemmArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.bias = bias; a.C = (bf16_t*)C;
+  a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc;
+  a.bias_f32 = bias_dtype == TV_F32;
+  hipStream_t st = (hipStream_t)stream;
+  switch (tile) {
+    case 0: return go<4, 4, 4>(a, epilogue, st);
+    case 1: return go<4, 4, 2>(a, epilogue, st);
+    case 2: return go<2, 4, 3>(a, epilogue, st);
+    default: return go<2, 2, 4>(a, epilogue, st);
+  }
+}

@@ -803,6 +803,51 @@ def large_takes(x, weight, relu2=False) -> bool:
             and weight.data_ptr() % 16 == 0 and gemm_persist_on())
 
 
+GEMM_GLU = 5
+
+
+def small_linear(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None, tile: int = 0):
+    """`linear_fused` on small tiles (tv_gemm_small_fwd): x (rows, K) bf16, weight (N, K); GEMM_GLU: the two halves of weight's rows, `glu_linear`'s result"""
+    _gpu(x, weight, bias, out)
+    N, Kd = weight.shape
+    if epilogue == GEMM_GLU:
+        N //= 2
+    if x.dtype != torch.bfloat16 or weight.dtype != x.dtype or x.dim() != 2 or x.shape[1] != Kd or x.stride(1) != 1 or weight.stride(1) != 1:
+        raise TimeViperHipError(f"small_linear: {tuple(x.shape)} {x.dtype} against {tuple(weight.shape)}")
+    if out is None:
+        if epilogue == GEMM_ACCUM:
+            raise TimeViperHipError("small_linear: GEMM_ACCUM needs `out`")
+        out = x.new_empty((x.shape[0], N))
+    if out.shape != (x.shape[0], N) or out.dtype != x.dtype or out.stride(1) != 1:
+        raise TimeViperHipError("small_linear: `out` must be (rows, N) of x's dtype")
+    if bias is not None and (bias.dtype not in (torch.float32, torch.bfloat16) or not bias.is_contiguous() or bias.numel() != weight.shape[0]):
+        raise TimeViperHipError("small_linear: bias must be contiguous, fp32 or bf16")
+    check(_capi.lib().tv_gemm_small_fwd(_p(x), _p(weight), None if epilogue == GEMM_ACCUM else _p(bias), _p(out), x.shape[0], N, Kd, x.stride(0),
+                                        weight.stride(0), out.stride(0), int(epilogue), TV_F32 if bias is None else _dt(bias), tile, _stream()),
+          "tv_gemm_small_fwd")
+    return out
+
+
+def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
+    """The tile of tv_gemm_small_fwd for rows x n outputs (of either factor with `glu`) where it replaces a library call of a short forward, -1 where it does not.
+    Such a forward waits for the host, which a library call takes 19 us of and this one 8, so the product may take as long as the library's, not longer (us on the
+    device, library | here): 64 x 64 where they are one round of the compute units or less (1 152 x 1 152, 729 rows: 9.5 | 7.5, 1 458: 10.7 | 9.6; 5 120 x 2 048, 100: 10.8 | 10.5; 1
+    152 x 4 352, 729: 18.7 | 19.4), 64 x 128 up to 1.3 rounds (3 456 x 1 152, 729: 15.0 | 13.8), 128 x 128 up to two (1 458: 17.1 | 21; with the GELU 20.7 + 4 | 22; 2 187:
+    26 | 24), and not contractions of more than 2 048 columns on more than a few hundred rows (1 152 x 4 352, 2 187 rows: 31 | 43)."""
+    if not 2 <= rows <= 2304 or n < 512 or k % 64 or (k > 2048 and (k > 4608 or rows > 1536)):
+        return -1
+    over = lambda tm, tn: -(-rows // tm) * -(-n * (2 if glu else 1) // tn)
+    if over(64, 64) <= CUS * 6 // 5:
+        return 3
+    if k > 2048:
+        return 3 if over(64, 64) <= CUS * 2 else -1
+    if over(64, 128) <= CUS * 4 // 3:
+        return 2
+    if over(128, 128) <= CUS:
+        return 0
+    return 1 if over(128, 128) <= CUS * 2 else -1
+
+
 def split_takes(x, weight, relu2=False) -> int:
     """Products of more than 256 rows that tv_gemm_split_fwd runs faster than the library: work-groups a tile of 256 x 256 outputs, 0 where the product is not one
     of them (us, library | here):
@@ -1335,6 +1380,13 @@ def products_take(x, *weights) -> bool:
             and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
             and all(type(w) in (torch.Tensor, torch.nn.Parameter) and w.dtype == torch.bfloat16 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 8 == 0
                     and 64 <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights))
+
+
+def small_takes(x, weight, glu: bool = False, most: int = 2304) -> int:
+    """`small_tile` of x (rows, K) against weight, -1 where the rows are more than `most` or the operands are not what the kernel reads"""
+    n = weight.shape[0] // 2 if glu else weight.shape[0]
+    tile = small_tile(x.shape[0], n, x.shape[1], glu) if x.shape[0] <= most else -1
+    return tile if tile >= 0 and n % 8 == 0 and products_take(x, weight) else -1
 
 
 def glu_takes(x, weight) -> bool:

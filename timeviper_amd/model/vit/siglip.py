@@ -77,6 +77,14 @@ def _gemm_reads(*ts) -> bool:
     return True
 
 
+def _small(x: torch.Tensor, mod: nn.Linear, weight: Optional[torch.Tensor] = None) -> int:
+    """The small tile (`kernels.small_tile`) on which mod(x), or the product with a padded copy of mod's weight, runs in a clip of a few frames; -1: none.  Such a
+    clip waits for its launches (26 blocks of so400m, 1 to 3 frames: 4.0 ms)."""
+    if x.dim() != 3 or x.shape[0] * x.shape[1] > 2304 or not x.is_contiguous() or not plain_linear(mod, x) or mod.bias is None or mod.bias.data_ptr() % 16:
+        return -1
+    return K.small_takes(x.view(-1, x.shape[-1]), mod.weight if weight is None else weight)
+
+
 def _aligned(n: int) -> int:
     return -(-n // GEMM_ALIGN) * GEMM_ALIGN
 
@@ -132,7 +140,10 @@ class Attention(nn.Module):
     def heads(self, x):
         """qkv projection + attention, without the output projection"""
         B, N, C = x.shape
-        if self._own_qkv(x):
+        tile = _small(x, self.qkv)
+        if tile >= 0:
+            qkv = K.small_linear(x.view(-1, C), self.qkv.weight, self.qkv.bias, tile=tile).view(B, N, 3, self.num_heads, self.head_dim)
+        elif self._own_qkv(x):
             # on the weights as stored: 3 456 columns are 13 tiles and one shifted back — no padded copies
             qkv = K.linear_fused(x, self.qkv.weight, self.qkv.bias, epilogue=K.GEMM_BIAS)
             qkv = qkv.view(B, N, 3, self.num_heads, self.head_dim)
@@ -185,11 +196,15 @@ class Mlp(nn.Module):
             w1, b1, w2 = self._padded.get((self.fc1.weight, self.fc1.bias, self.fc2.weight), lambda: (
                 _pad_rows(self.fc1.weight.detach(), _aligned(Hd)), _pad_rows(self.fc1.bias.detach(), _aligned(Hd)),
                 _pad_cols(self.fc2.weight.detach(), _aligned(Hd))))
+            if self.exact_gelu and (tile := _small(x, self.fc1, w1)) >= 0:
+                return K.small_linear(x.view(-1, x.shape[-1]), w1, b1, K.GEMM_BIAS_GELU, tile=tile).view(*x.shape[:-1], -1), w2
             if self._fused_fc1(x, w1, b1):
                 return K.linear_fused(x, w1, b1, epilogue=K.GEMM_BIAS_GELU), w2
             h = F.linear(x, w1, b1)
         else:
             w2 = self.fc2.weight
+            if self.exact_gelu and (tile := _small(x, self.fc1)) >= 0:
+                return K.small_linear(x.view(-1, x.shape[-1]), self.fc1.weight, self.fc1.bias, K.GEMM_BIAS_GELU, tile=tile).view(*x.shape[:-1], -1), w2
             # (below 4 096 rows fc1 is called if anything stands around it)
             if (x.numel() // x.shape[-1] >= 4096 or plain_linear(self.fc1, x)) and self._fused_fc1(x, self.fc1.weight, self.fc1.bias):
                 return K.linear_fused(x, self.fc1.weight, self.fc1.bias, epilogue=K.GEMM_BIAS_GELU), w2
@@ -231,7 +246,10 @@ def _accumulate(x2: torch.Tensor, h2: torch.Tensor, w: torch.Tensor, role: str) 
     TV_VIT_OWN_ACCUM, comma separated: proj, fc2) and the shape allows (bf16, K a multiple of 128 and >= 1 152), else hipBLASLt
     (`torch.addmm`, beta = 1)."""
     rows, n = x2.shape
-    if ((_own_accumulate(rows, n) or (role in _OWN_ACCUM and rows >= 65536)) and x2.is_cuda and x2.dtype == torch.bfloat16
+    tile = K.small_takes(h2, w)
+    if tile >= 0 and _gemm_reads(x2) and x2.dtype == h2.dtype:
+        K.small_linear(h2, w, None, K.GEMM_ACCUM, out=x2, tile=tile)
+    elif ((_own_accumulate(rows, n) or (role in _OWN_ACCUM and rows >= 65536)) and x2.is_cuda and x2.dtype == torch.bfloat16
             and h2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and not torch.is_grad_enabled() and w.shape[1] % 128 == 0
             and w.shape[1] >= 1152 and n % 8 == 0 and _gemm_reads(x2, h2, w)):
         K.linear_fused(h2, w, None, epilogue=K.GEMM_ACCUM, out=x2)
