@@ -140,7 +140,7 @@ class Attention(nn.Module):
     def heads(self, x):
         """qkv projection + attention, without the output projection"""
         B, N, C = x.shape
-        tile = _small(x, self.qkv)
+        tile = _small(x, self.qkv) if os.environ.get("TV_VIT_OWN_QKV", "") != "0" else -1
         if tile >= 0:
             qkv = K.small_linear(x.view(-1, C), self.qkv.weight, self.qkv.bias, tile=tile).view(B, N, 3, self.num_heads, self.head_dim)
         elif self._own_qkv(x):
@@ -196,14 +196,14 @@ class Mlp(nn.Module):
             w1, b1, w2 = self._padded.get((self.fc1.weight, self.fc1.bias, self.fc2.weight), lambda: (
                 _pad_rows(self.fc1.weight.detach(), _aligned(Hd)), _pad_rows(self.fc1.bias.detach(), _aligned(Hd)),
                 _pad_cols(self.fc2.weight.detach(), _aligned(Hd))))
-            if self.exact_gelu and (tile := _small(x, self.fc1, w1)) >= 0:
+            if self._fuse() and (tile := _small(x, self.fc1, w1)) >= 0:
                 return K.small_linear(x.view(-1, x.shape[-1]), w1, b1, K.GEMM_BIAS_GELU, tile=tile).view(*x.shape[:-1], -1), w2
             if self._fused_fc1(x, w1, b1):
                 return K.linear_fused(x, w1, b1, epilogue=K.GEMM_BIAS_GELU), w2
             h = F.linear(x, w1, b1)
         else:
             w2 = self.fc2.weight
-            if self.exact_gelu and (tile := _small(x, self.fc1)) >= 0:
+            if self._fuse() and (tile := _small(x, self.fc1)) >= 0:
                 return K.small_linear(x.view(-1, x.shape[-1]), self.fc1.weight, self.fc1.bias, K.GEMM_BIAS_GELU, tile=tile).view(*x.shape[:-1], -1), w2
             # (below 4 096 rows fc1 is called if anything stands around it)
             if (x.numel() // x.shape[-1] >= 4096 or plain_linear(self.fc1, x)) and self._fused_fc1(x, self.fc1.weight, self.fc1.bias):
@@ -211,6 +211,9 @@ class Mlp(nn.Module):
             h = self.fc1(x)
         h = K.gelu(h, inplace=True) if self.exact_gelu else self.act(h)
         return h, w2
+
+    def _fuse(self) -> bool:
+        return self.exact_gelu and os.environ.get("TV_VIT_FUSED_FC1", "1") != "0"
 
     def _fused_fc1(self, x, w1, b1) -> bool:
         """fc1 + bias + exact GELU in ONE kernel (csrc/gemm_persist.hip: the activation is applied to the accumulators, same
