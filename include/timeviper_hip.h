@@ -608,18 +608,18 @@ int tv_gemm_rows_pair_fwd(const void* x, const void* x2, const void* W, const vo
                           int ff, int K, int64_t x_stride, int64_t x2_stride, int64_t ldw, int64_t y_stride,
                           int64_t act_stride, void* stream);
 
-/* y = x W^T + bias on tiles of 256 x 256 outputs (csrc/gemm.hip) whose contraction is split over `splits` work-groups (1..64; each takes at
- * least two steps of 64 columns, K % 64 == 0, N % 4 == 0): fp32 partial sums to the workspace (tv_gemm_split_workspace_bytes, 0 for one
+/* y = x W^T + bias on tiles of 256 x 256 outputs (csrc/gemm.hip); the first `full` of them are a work-group's each, the contraction of the others is split over
+ * `splits` work-groups (1..64; each takes at least two steps of 64 columns, K % 64 == 0, N % 4 == 0): fp32 partial sums to the workspace (tv_gemm_split_workspace_bytes, 0 for one
  * split; 16-byte aligned, not shared by launches that may run at once), added in order by a second launch, one rounding.  bias fp32 or bf16
  * or NULL, 16-byte aligned; epilogue 0, or 3: the squared ReLU of the rounded sum. */
-size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits);
+size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits, int full);
 int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
-                      int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream);
+                      int64_t ldc, int epilogue, int bias_dtype, int splits, int full, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same with the residual stream behind it: residual_out = residual + (x W^T + bias) in fp32 (rows of N, 16-byte aligned; in place where residual_out is
  * residual) and y (rows of N), its bf16 copy. */
 int tv_gemm_split_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N,
-                          int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream);
+                          int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, int full, void* workspace, size_t workspace_bytes, void* stream);
 
 /* C = gelu_tanh(A Wg^T + bg) * (A Wu^T + bu), Wg the first N rows of W and Wu the next N, bg | bu the bf16 bias (csrc/gemm_persist.hip): fp32 until the one
  * rounding.  M >= 256, N >= 128 and a multiple of 8, K a multiple of 128 and at least 256, everything 16-byte aligned. */

@@ -44,26 +44,43 @@ def test_refused():
         ops.split_linear(torch.zeros(300, 196, device=DEV, dtype=BF)[:, 4:], w)
 
 
+# whole tiles in front of the split ones, none and all of them; bands of fewer than four tiles of rows
+@pytest.mark.parametrize("M,N,K,splits,full", [(300, 700, 320, 2, 5), (1300, 516, 384, 3, 8), (1300, 516, 384, 2, 17), (520, 300, 448, 3, 6), (520, 300, 448, 2, 1)])
+def test_whole_tiles_in_front(M, N, K, splits, full):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + full)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, w, b = r(M, K).to(BF), (K ** -0.5 * r(N, K)).to(BF), r(N)
+    want, mag = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    got = ops.split_linear(x, w, b, False, splits, full).double()
+    sums = mag * K * 2.0 ** -24
+    assert ((got - want).abs() <= sums + 2.0 ** -8 * (want.abs() + sums)).all()
+    with pytest.raises(ops.TimeViperHipError):
+        ops.split_linear(x, w, b, False, splits, 1000)
+
+
 # both sides of each line of the rule, and the route
-@pytest.mark.parametrize("N,K,relu2,rows,splits", [(4480, 10240, False, 256, 0), (4480, 10240, False, 257, 7), (4480, 10240, False, 1000, 3), (4480, 10240, False, 1700, 2),
-                                                   (4480, 10240, False, 2000, 0), (8192, 28672, False, 600, 0), (4096, 11008, False, 3900, 0), (4096, 4096, False, 12000, 0), (4480, 10240, False, 3000, 1), (4480, 10240, False, 6011, 0), (4480, 15680, False, 5000, 2),
-                                                   (4480, 15680, False, 8192, 0), (4480, 15680, False, 10007, 1), (15680, 4480, True, 512, 0), (15680, 4480, True, 1000, 1),
-                                                   (15680, 4480, False, 1000, 0), (4480, 5120, False, 512, 0), (4480, 5120, False, 3000, 1), (1024, 4480, False, 3000, 0)])
-def test_rule(N, K, relu2, rows, splits, monkeypatch):
+@pytest.mark.parametrize("N,K,relu2,rows,plan", [
+    (4480, 10240, False, 256, None), (4480, 10240, False, 257, (7, 0)), (4480, 10240, False, 1000, (3, 0)), (4480, 10240, False, 1700, (2, 0)), (4480, 10240, False, 2000, None),
+    (8192, 28672, False, 600, None), (4096, 11008, False, 3900, None), (4096, 4096, False, 12000, None), (4480, 10240, False, 3000, (1, 0)), (4480, 10240, False, 6011, None),
+    (4480, 10240, False, 4096, (8, 256)), (4480, 10240, False, 5600, None), (4480, 15680, False, 5000, (2, 256)), (4480, 15680, False, 5600, (1, 0)),
+    (4480, 15680, False, 8192, (4, 512)), (4480, 15680, False, 10007, (1, 0)), (15680, 4480, True, 512, None), (15680, 4480, True, 1000, (1, 0)), (15680, 4480, True, 1400, (2, 256)),
+    (15680, 4480, True, 2048, None), (15680, 4480, False, 1400, None), (15680, 4480, False, 1000, None), (4480, 5120, False, 512, None), (4480, 5120, False, 3000, (1, 0)),
+    (5120, 4480, False, 7000, (5, 512)), (22656, 4480, False, 768, (16, 256)), (22656, 4480, False, 1400, None), (1024, 4480, False, 3000, None)])
+def test_rule(N, K, relu2, rows, plan, monkeypatch):
     from timeviper_amd import kernels as ops
     from timeviper_amd.model.llm import nano
     with torch.device("meta"):
         lin = torch.nn.Linear(K, N, bias=False, dtype=BF)
     lin = lin.to_empty(device=DEV).requires_grad_(False)
     x = torch.empty(1, rows, K, device=DEV, dtype=BF)
-    assert ops.split_takes(x, lin.weight, relu2) == splits
-    assert ops.split_takes(x[:, :, 1:], lin.weight[:, 1:], relu2) == 0
+    assert ops.split_takes(x, lin.weight, relu2) == plan
+    assert ops.split_takes(x[:, :, 1:], lin.weight[:, 1:], relu2) is None
     calls = []
-    monkeypatch.setattr(ops, "split_linear", lambda x, w, b, r, s: calls.append((r, s)))
-    monkeypatch.setattr(ops, "linear_fused", lambda *a, **k: None)
-    monkeypatch.setattr(ops, "mid_linear", lambda *a, **k: None)
-    if splits:
+    monkeypatch.setattr(ops, "split_linear", lambda x, w, b, r, *p: calls.append((r, *p)))
+    if plan or ops.large_takes(x, lin.weight, relu2):
+        plan = plan or ops.tail_plan(rows, N, K)              # (linear_fused: the persistent kernel, or whole tiles in front of split ones)
         with torch.no_grad():
             nano._prompt_linear(lin, x, relu2)
         nano._prompt_linear(lin, x[:, :300])                  # gradients enabled: the module
-    assert calls == ([(relu2, splits)] if splits else [])
+    assert calls == ([(relu2, *plan)] if plan else [])

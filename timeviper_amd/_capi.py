@@ -44,9 +44,9 @@ SIGNATURES = {
     "tv_selective_state_update": (_i, [_p] * 9 + [_i] * 7 + [_p]),
     "tv_selective_state_update_rows": (_i, [_p] * 9 + [_i] * 5 + [_l] * 4 + [_i, _i, _p]),
     "tv_gemm_bf16_fwd": (_i, [_p, _p, _p, _p, _l, _i, _i, _l, _l, _l, _i, _i, _p]),
-    "tv_gemm_split_workspace_bytes": (_z, [_l, _i, _i]),
-    "tv_gemm_split_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _i, _i, _i, _p, _z, _p]),
-    "tv_gemm_split_add_fwd": (_i, [_p] * 6 + [_l, _i, _i, _l, _l, _i, _i, _p, _z, _p]),
+    "tv_gemm_split_workspace_bytes": (_z, [_l, _i, _i, _i]),
+    "tv_gemm_split_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _i, _i, _i, _i, _p, _z, _p]),
+    "tv_gemm_split_add_fwd": (_i, [_p] * 6 + [_l, _i, _i, _l, _l, _i, _i, _i, _p, _z, _p]),
     "tv_gemm_glu_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _p]),
     "tv_token_side_fwd": (_i, [_p] * 6 + [_l, _i, _i] + [_l] * 6 + [_p]),
     "tv_gemm_small_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _i, _i, _i, _p]),

@@ -60,15 +60,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
   const int ntiles = tiles_m * a.tiles_n;
   int id = blockIdx.x;
   if (GROUPED && id >= ntiles) return;
+  const int ntail = SPLIT ? ntiles - a.full : 0;       // (the whole tiles' work-groups come first)
+  const bool tail = SPLIT && id >= a.full;
   {
-    const int all = SPLIT ? ntiles * a.splits : ntiles;
-    const int q = all / 8, r = all % 8, x = id % 8;
-    id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + id / 8;
+    const int first = tail ? a.full : 0, all = !SPLIT ? ntiles : tail ? ntail * a.splits : a.full;
+    const int i = id - first, q = all / 8, r = all % 8, x = i % 8;
+    id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i / 8;
   }
-  int split = 0;
-  if (SPLIT) {                                 // (neighbours of an XCD share a split: the same k-slabs)
-    split = __builtin_amdgcn_readfirstlane(id / ntiles);
-    id -= split * ntiles;
+  int split = 0, in_tail = 0;
+  if (tail) {                                  // (neighbours of an XCD share a split: the same k-slabs)
+    split = __builtin_amdgcn_readfirstlane(id / ntail);
+    in_tail = id - split * ntail;
+    id = a.full + in_tail;
   }
   // ... in bands of `gm` m-tiles, m fastest: the ~32 work-groups an XCD runs at a time cover gm x (32 / gm) tiles and
   // share each A / W k-slab through its L2 while they march through K together
@@ -105,7 +108,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
       voffW[h][j] = (unsigned)((rw * a.ldw + ch * 8) * 2);
     }
   int nkt = a.K / BK, kt0 = 0;
-  if (SPLIT) {
+  if (tail) {
     kt0 = (int)((int64_t)nkt * split / a.splits);
     nkt = (int)((int64_t)nkt * (split + 1) / a.splits) - kt0;       // (>= 2: launcher)
   }
@@ -274,8 +277,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
   }
   if (wr == 0) __builtin_amdgcn_s_barrier();          // barrier counts match again
 
-  if (SPLIT && a.part) {                              // 16 rows x 64 bytes an instruction
-    float* const P = a.part + (int64_t)split * a.M * a.N;
+  if (tail && a.splits > 1) {                         // 16 rows x 64 bytes an instruction
+    float* const P = a.part + (int64_t)(split * ntail + in_tail) * (BM * BN);
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh)
 #pragma unroll
@@ -287,7 +290,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a) {
 #pragma unroll
           for (int n = 0; n < 2; ++n) {
             const int col = n0 + 128 * nh + 32 * wc + 16 * n + 4 * kq;
-            if (col < a.N) *(f32x4*)(P + (int64_t)row * a.N + col) = acc[mh][nh][m][n];
+            if (col < a.N) *(f32x4*)(P + (row - m0) * BN + (col - n0)) = acc[mh][nh][m][n];
           }
       }
     return;
@@ -398,16 +401,17 @@ template <int EPI, bool GROUPED>
 __global__ __launch_bounds__(512) void gemm_bf16_kernel(GemmArgs a) { gemm_tile<EPI, GROUPED, false>(a); }
 __global__ __launch_bounds__(512) void gemm_split_kernel(GemmArgs a) { gemm_tile<EPI_BIAS, false, true>(a); }
 
-// the splits of four neighbouring outputs, added in order; bias, one rounding, squared ReLU of what was rounded
+// the splits of four neighbouring outputs, added in order; bias, one rounding, squared ReLU of what was rounded.  64 work-groups a split tile, four rows each
 __global__ __launch_bounds__(256) void gemm_split_sum_kernel(GemmArgs a) {
-  const int nq = a.N / 4;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (int64_t)a.M * nq) return;
-  const int row = (int)(i / nq), col = 4 * (int)(i - (int64_t)row * nq);
-  const float* p = a.part + (int64_t)row * a.N + col;
-  const int64_t step = (int64_t)a.M * a.N;
+  const int ntail = a.tiles_m * a.tiles_n - a.full, in_tail = blockIdx.x >> 6, id = a.full + in_tail;
+  const int band = id / (a.group_m * a.tiles_n), in_band = id % (a.group_m * a.tiles_n), rows_in_band = min(a.group_m, a.tiles_m - band * a.group_m);
+  const int r = 4 * (blockIdx.x & 63) + (threadIdx.x >> 6), c = 4 * (threadIdx.x & 63);
+  const int row = (band * a.group_m + in_band % rows_in_band) * BM + r, col = in_band / rows_in_band * BN + c;
+  if (row >= a.M || col >= a.N) return;
+  const float* p = a.part + (int64_t)in_tail * (BM * BN) + r * BN + c;
+  const int64_t step = (int64_t)ntail * (BM * BN);
   f32x4 s = *(const f32x4*)p;
-  for (int j = 1; j < a.splits; j += 4) {             // (a split that is not there repeats the last one, weighted 0 by not being added)
+  for (int j = 1; j < a.splits; j += 4) {             // (a split that is not there repeats the last one and is not added)
     f32x4 t[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) t[u] = *(const f32x4*)(p + min(j + u, a.splits - 1) * step);
@@ -446,8 +450,9 @@ int launch_split(const GemmArgs& a, hipStream_t st) {
     tv_set_error("gemm_split: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     return TV_ERR_LAUNCH;
   }
-  gemm_split_kernel<<<dim3((unsigned)(a.tiles_m * a.tiles_n * a.splits)), 512, LDS_BYTES, st>>>(a);
-  if (a.part) gemm_split_sum_kernel<<<dim3((unsigned)(((int64_t)a.M * (a.N / 4) + 255) / 256)), 256, 0, st>>>(a);
+  const int tail = a.tiles_m * a.tiles_n - a.full;
+  gemm_split_kernel<<<dim3((unsigned)(a.full + tail * a.splits)), 512, LDS_BYTES, st>>>(a);
+  if (a.part) gemm_split_sum_kernel<<<dim3((unsigned)(tail * 64)), 256, 0, st>>>(a);
   TV_LAUNCH_CHECK();
 }
 
@@ -541,12 +546,14 @@ extern "C" int tv_gemm_bf16_fwd(const void* A, const void* W, const void* bias, 
   }
 }
 
-extern "C" size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits) {
-  return M <= 0 || N <= 0 || splits <= 1 ? 0 : (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
+extern "C" size_t tv_gemm_split_workspace_bytes(int64_t M, int N, int splits, int full) {
+  if (M <= 0 || N <= 0 || splits <= 1 || full < 0) return 0;
+  const int64_t tail = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) - full;
+  return tail > 0 ? (size_t)splits * (size_t)tail * (BM * BN) * sizeof(float) : 0;
 }
 
 static int split_fwd(const void* A, const void* W, const void* bias, const float* res, float* res_out, void* C, int64_t M, int N, int K, int64_t lda,
-                     int64_t ldw, int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+                     int64_t ldw, int64_t ldc, int epilogue, int bias_dtype, int splits, int full, void* workspace, size_t workspace_bytes, void* stream) {
   TV_CHECK_ARG(M > 0 && N > 0 && K > 0, "gemm_split: bad sizes (M %lld N %d K %d)", (long long)M, N, K);
   TV_CHECK_ARG(A && W && C, "gemm_split: null pointer");
   TV_CHECK_ARG(epilogue == 0 || epilogue == 3, "gemm_split: epilogue %d", epilogue);
@@ -557,9 +564,10 @@ static int split_fwd(const void* A, const void* W, const void* bias, const float
     TV_UNSUPPORTED("gemm_split: K must be a multiple of %d (two of them a split), N of 4, rows 16-byte aligned (K %d N %d lda %lld ldw %lld ldc %lld)", BK, K,
                    N, (long long)lda, (long long)ldw, (long long)ldc);
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  if (M > (1ll << 31) - BM || 256 * lda * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31) || tiles * splits >= (1ll << 31) || M * (N / 4) >= (1ll << 38))
+  if (M > (1ll << 31) - BM || 256 * lda * 2 >= (1ll << 31) || 256 * ldw * 2 >= (1ll << 31) || tiles * (splits > 64 ? splits : 64) >= (1ll << 31))
     TV_UNSUPPORTED("gemm_split: sizes beyond the 32-bit offsets of the copies");
-  const size_t need = tv_gemm_split_workspace_bytes(M, N, splits);
+  TV_CHECK_ARG(full >= 0 && full <= tiles, "gemm_split: %d whole tiles of %lld", full, (long long)tiles);
+  const size_t need = tv_gemm_split_workspace_bytes(M, N, splits, full);
   TV_CHECK_ARG(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
                "gemm_split: workspace of %zu bytes (16-byte aligned) needed, got %zu", need, workspace_bytes);
   GemmArgs a{};
@@ -568,21 +576,22 @@ static int split_fwd(const void* A, const void* W, const void* bias, const float
   a.tiles_m = (int)((M + BM - 1) / BM); a.tiles_n = (N + BN - 1) / BN;
   a.bias_f32 = bias_dtype == TV_F32;
   a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
-  a.part = splits > 1 ? (float*)workspace : nullptr;
+  a.part = need ? (float*)workspace : nullptr;
   a.splits = splits;
+  a.full = full;
   a.relu2 = epilogue == 3;
   a.res = res; a.res_out = res_out;
   return launch_split(a, (hipStream_t)stream);
 }
 
 extern "C" int tv_gemm_split_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw,
-                                 int64_t ldc, int epilogue, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
-  return split_fwd(A, W, bias, nullptr, nullptr, C, M, N, K, lda, ldw, ldc, epilogue, bias_dtype, splits, workspace, workspace_bytes, stream);
+                                 int64_t ldc, int epilogue, int bias_dtype, int splits, int full, void* workspace, size_t workspace_bytes, void* stream) {
+  return split_fwd(A, W, bias, nullptr, nullptr, C, M, N, K, lda, ldw, ldc, epilogue, bias_dtype, splits, full, workspace, workspace_bytes, stream);
 }
 
 extern "C" int tv_gemm_split_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N,
-                                     int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+                                     int K, int64_t lda, int64_t ldw, int bias_dtype, int splits, int full, void* workspace, size_t workspace_bytes, void* stream) {
   TV_CHECK_ARG(residual && residual_out, "gemm_split_add: null pointer");
   if (((uintptr_t)residual & 15) || ((uintptr_t)residual_out & 15)) TV_UNSUPPORTED("gemm_split_add: the residual rows must be 16-byte aligned");
-  return split_fwd(A, W, bias, residual, residual_out, C, M, N, K, lda, ldw, N, 0, bias_dtype, splits, workspace, workspace_bytes, stream);
+  return split_fwd(A, W, bias, residual, residual_out, C, M, N, K, lda, ldw, N, 0, bias_dtype, splits, full, workspace, workspace_bytes, stream);
 }

@@ -29,9 +29,9 @@ struct GemmArgs {
   const int *offsets, *row_token;
   int groups;
   int64_t w_group;
-  // products whose contraction is split over work-groups: partial sums [splits][M][N], NULL where splits is 1 (tv_gemm_split_fwd)
+  // products whose contraction is split over work-groups (tv_gemm_split_fwd): the tiles from `full` on, partial sums [split][tile][256][256]
   float* part;
-  int splits, relu2;       // relu2: squared ReLU of the rounded sum
+  int full, splits, relu2;       // relu2: squared ReLU of the rounded sum
   const float* res;        // res_out = res + sum (fp32, rows of N) and C, its bf16 copy, in the sum's place (tv_gemm_split_add_fwd); NULL: none
   float* res_out;
 };

@@ -302,6 +302,11 @@ def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
     N, Kd = weight.shape
     if weight.stride(1) != 1:
         weight = weight.contiguous()
+    if out is None and epilogue in (GEMM_BIAS, GEMM_BIAS_RELU2) and Kd >= 4096 and x.shape[-1] == Kd and x2.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 \
+            and (x2.data_ptr() | weight.data_ptr()) % 16 == 0 and bias is None and N % 8 == 0 and gemm_persist_on():
+        plan = tail_plan(x2.shape[0], N, Kd)
+        if plan:
+            return split_linear(x, weight, None, epilogue == GEMM_BIAS_RELU2, *plan)
     if epilogue == GEMM_ACCUM:
         if out is None:
             raise TimeViperHipError("linear_fused: GEMM_ACCUM needs `out`")
@@ -848,42 +853,59 @@ def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
     return 1 if over(128, 128) <= CUS * 2 else -1
 
 
-def split_takes(x, weight, relu2=False) -> int:
-    """Products of more than 256 rows that tv_gemm_split_fwd runs faster than the library: work-groups a tile of 256 x 256 outputs, 0 where the product is not one
-    of them (us, library | here):
+def tail_plan(rows: int, n: int, k: int):
+    """(work-groups a tile, whole tiles in front) for a product whose last round of 256 x 256 tiles is at most 46 % full (half from 12 288 columns on): those tiles
+    share the compute units, as many work-groups each as fit (us, one work-group a tile | here: 22 656 x 4 480, 1 400 rows, 2.09 rounds, 276 | 237, 3 000: 475 | 457,
+    2 500, 48 %: 386 | 393; 4 480 x 15 680, 4 096: 569 | 409, 5 000: 592 | 508); None where it is fuller, or where there is a single round or a short contraction."""
+    tiles = -(-rows // 256) * -(-n // 256)
+    last = tiles % CUS
+    if tiles <= CUS or not 0 < last <= (CUS // 2 if k > 12288 else CUS * 46 // 100) or k < 4096 or k % 64 or n % 4:
+        return None
+    return min(CUS // last, 16), tiles - last
+
+
+def split_takes(x, weight, relu2=False):
+    """Products of more than 256 rows that tv_gemm_split_fwd runs faster than the library, and that `large_takes` does not have: (work-groups a tile, whole tiles in
+    front of those), None where the product is not one of them (us, library | here):
       - a long contraction into fewer outputs whose tiles leave half of the compute units idle: as many work-groups a tile as fit one round, if they fill 80 % of
         it (4 480 x 10 240: 300 rows 59 | 52, 512: 85 | 59, 1 024: 108 | 90, 1 536: 137 | 124; 4 480 x 15 680: 300: 92 | 67, 512: 137 | 75, 1 400: 349 | 177; 75 % full,
         600 rows of 8 192 x 28 672: 254 | 287),
-      - a contraction longer than the outputs whose last round is 80 % full: one work-group a tile, where `large_takes` does not have it, and in a first round
-        only widths that the library's 256 columns do not divide (4 096 x 11 008, 3 900 rows: 227 | 237) (4 480 x 15 680, an odd
-        number of steps: 3 000 rows 532 | 306, 10 007: 1 382 | 999, 14 000: 1 728 | 1 360; 4 480 x 10 240: 3 000: 219 | 203; 4 480 x 5 120: 3 000: 117 | 107, 6 011: 224 |
-        207; 84 % full and the library in step, 7 000 x 15 680: 654 | 680; 75 %, 8 192 x 5 120: 292 | 314),
-      - more than 12 288 columns in up to one and a half rounds: two work-groups a tile (4 480 x 15 680: 4 096 rows 855 | 514, 5 000: 966 | 564),
-      - the squared ReLU in a single round that is 72 % full (15 680 x 4 480, with the pass that it saves: 700 rows 101 | 90, 1 024: 122 | 103)."""
+      - a contraction longer than the outputs whose last round is 80 % full (75 from 12 288 columns on): one work-group a tile, in a first round only at widths that the
+        library's 256 columns do not divide (4 096 x 11 008, 3 900 rows: 227 | 237) (4 480 x 15 680, an odd number of steps: 3 000 rows 532 | 306, 10 007: 1 382 |
+        999, 14 000: 1 728 | 1 360; 4 480 x 10 240: 3 000: 219 | 203; 4 480 x 5 120: 3 000: 117 | 107, 6 011: 224 | 207; 84 % full and the library in step, 7 000 x
+        15 680: 654 | 680),
+      - several rounds of which the last is nearly empty (`tail_plan`), of outputs up to 1.25 times as wide as the contraction is long, or of 20 480 and more up to
+        12 288 rows (22 656 x 4 480: 768 rows 182 | 132, 2 200: 378 | 339; 4 480 x 10 240: 3 700: 464 | 248, 8 192: 561 | 527; 5 120 x 4 480: 3 400: 149 | 130, 7 000:
+        382 | 241; 4 480 x 5 120, 4 096: 167 | 148, 5 000: 184 | 182),
+      - the squared ReLU in a single round that is 72 % full, or in several with such a last one (15 680 x 4 480, with the pass that it saves: 700 rows 101 | 90, 1 024:
+        122 | 103, 1 400: 185 | 170, 2 200: 266 | 243)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     rows = x.numel() // max(x.shape[-1], 1)
     tiles = -(-rows // 256) * -(-N // 256)
     if rows <= MID_MAX or N < 4096 or Kd < 4096 or rows > 32768:
-        return 0
+        return None
     fill = tiles / (-(-tiles // CUS) * CUS)
-    splits = 0
-    if relu2:
-        splits = int(Kd <= 8192 and tiles <= CUS and fill >= 0.72)
-    elif N <= Kd:
-        fit = CUS // tiles
-        if fit >= 2:
-            splits = fit if Kd >= 8192 and fit <= 8 and tiles * fit >= 0.8 * CUS else 0
-        elif fill >= 0.8:
-            splits = int(N % 256 != 0 if tiles <= CUS else N < Kd < 8192 or Kd % 128 != 0)
-        elif Kd > 12288 and CUS < tiles <= CUS * 3 // 2:
-            splits = 2
-    takes = (splits and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 64 == 0 and N % 4 == 0
+    fit = CUS // tiles
+    plan = None
+    if fit >= 2:
+        plan = (fit, 0) if not relu2 and N <= Kd and Kd >= 8192 and fit <= 8 and tiles * fit >= 0.8 * CUS else None
+    elif tiles <= CUS:
+        pays = fill >= 0.72 and Kd <= 8192 if relu2 else fill >= 0.8 and N <= Kd and N % 256 != 0
+        plan = (1, 0) if pays else None
+    elif relu2:
+        plan = tail_plan(rows, N, Kd) if Kd <= 8192 else None
+    else:
+        if 4 * N <= 5 * Kd or (N >= 20480 and rows <= 12288):
+            plan = tail_plan(rows, N, Kd)
+        if plan is None and N < Kd and fill >= (0.75 if Kd > 12288 else 0.8) and (Kd < 8192 or Kd % 128 != 0):
+            plan = (1, 0)
+    takes = (plan and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 64 == 0 and N % 4 == 0
              and Kd < (1 << 22) and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
-    return splits if takes else 0
+    return plan if takes and not large_takes(x, weight, relu2) else None
 
 
-def split_linear(x, weight, bias=None, relu2=False, splits=1):
-    """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) on tiles of 256 x 256 outputs, `splits` work-groups a tile."""
+def split_linear(x, weight, bias=None, relu2=False, splits=1, full=0):
+    """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) on tiles of 256 x 256 outputs, `splits` work-groups a tile but for the first `full`."""
     _gpu(x, weight, bias)
     N, Kd = weight.shape
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[-1] != Kd or weight.stride(1) != 1:
@@ -893,10 +915,10 @@ def split_linear(x, weight, bias=None, relu2=False, splits=1):
     x2 = _rows2d(x)
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
     lib, M = _capi.lib(), x2.shape[0]
-    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits))
+    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits, full))
     ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
     check(lib.tv_gemm_split_fwd(_p(x2), _p(weight), _p(bias), _p(y), M, N, Kd, x2.stride(0), weight.stride(0), N, 3 if relu2 else 0,
-                                TV_F32 if bias is None else _dt(bias), splits, _p(ws), need, _stream()), "tv_gemm_split_fwd")
+                                TV_F32 if bias is None else _dt(bias), splits, full, _p(ws), need, _stream()), "tv_gemm_split_fwd")
     return y
 
 
@@ -1434,9 +1456,9 @@ def split_add_linear(x, weight, residual, bias=None, splits=1):
         _bf16_bias(bias, N, "split_add_linear")
     lib, M = _capi.lib(), x.shape[0]
     res, h = torch.empty_like(residual), torch.empty((M, N), dtype=x.dtype, device=x.device)
-    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits))
+    need = int(lib.tv_gemm_split_workspace_bytes(M, N, splits, 0))
     ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-    check(lib.tv_gemm_split_add_fwd(_p(x), _p(weight), _p(bias), _p(residual), _p(res), _p(h), M, N, Kd, x.stride(0), weight.stride(0), TV_BF16, splits,
+    check(lib.tv_gemm_split_add_fwd(_p(x), _p(weight), _p(bias), _p(residual), _p(res), _p(h), M, N, Kd, x.stride(0), weight.stride(0), TV_BF16, splits, 0,
                                     _p(ws), need, _stream()), "tv_gemm_split_add_fwd")
     return res, h
 

@@ -321,8 +321,8 @@ def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torc
         if rows <= K.MID_MAX:
             if K.mid_takes(x, w, relu2):
                 return K.mid_linear(x, w, mod.bias, relu2)
-        elif splits := K.split_takes(x, w, relu2):
-            return K.split_linear(x, w, mod.bias, relu2, splits)
+        elif plan := K.split_takes(x, w, relu2):
+            return K.split_linear(x, w, mod.bias, relu2, *plan)
         elif K.large_takes(x, w, relu2):
             return K.linear_fused(x, w, mod.bias, epilogue=K.GEMM_BIAS_RELU2 if relu2 else K.GEMM_BIAS)
     y = mod(x)
