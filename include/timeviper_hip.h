@@ -587,18 +587,23 @@ int tv_gemv_pair_fwd(const void* x, const void* x2, const void* W, const void* b
                      void* stream);
 int tv_gemv_add_fwd(const void* x, const void* W, const void* bias, const float* residual, float* residual_out, void* h_out,
                     int M, int N, int K, int64_t x_stride, int64_t ldw, void* stream);
+/* y (fp32) = bf16(f(x) W^T + bias): the logits of 1..4 bf16 rows.  f(x) = x, or for one row (norm_weight not NULL) the RMS norm of bf16(x + delta) as in
+ * tv_gemv_bf16_fwd (delta may be NULL; K <= 8192).  Same alignment. */
+int tv_gemv_logits_fwd(const void* x, const void* W, const void* bias, float* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
+                       int64_t y_stride, const void* delta, const void* norm_weight, int norm_weight_dtype, float eps, void* stream);
 int tv_gemv_glu_fwd(const void* z, const void* u, const int64_t* u_ids, int64_t u_rows, const void* W, void* y, int M, int N,
                     int K, int64_t z_stride, int64_t u_stride, int64_t ldw, int64_t y_stride, void* stream);
 
 /* ------------------------------------------------------------------------
  * Products of a few rows (csrc/gemm_skinny.hip; M = 2..TV_GEMM_ROWS_MAX bf16 rows, K % 64 == 0, rows 16-byte aligned), on the
  * matrix cores: y = x W^T + bias (bias bf16 or NULL), fp32 sums, one rounding.
- * tv_gemm_rows_fwd: y bf16, or fp32 without epilogue; epilogue TV_GEMM_ROWS_RELU2: y = relu(bf16(.))^2; conv_state not NULL: the
+ * tv_gemm_rows_fwd: y bf16, or fp32 without epilogue or with TV_GEMM_ROWS_ROUND (the bf16 values, stored as fp32); epilogue TV_GEMM_ROWS_RELU2: y = relu(bf16(.))^2; conv_state not NULL: the
  *   outputs [conv_row0, conv_row0 + conv_channels) pass through tv_causal_conv1d_update (width 4, SiLU) on conv_state
  *   (M, conv_channels, 4), as in tv_gemv_bf16_fwd.
  * tv_gemm_rows_add_fwd, tv_gemm_rows_pair_fwd: tv_gemv_add_fwd and tv_gemv_pair_fwd for these rows.                        */
 #define TV_GEMM_ROWS_MAX 32
 #define TV_GEMM_ROWS_RELU2 1
+#define TV_GEMM_ROWS_ROUND 2
 int tv_gemm_rows_fwd(const void* x, const void* W, const void* bias, void* y, int y_dtype, int M, int N, int K, int64_t x_stride,
                      int64_t ldw, int64_t y_stride, int epilogue, void* conv_state, const void* conv_weight,
                      const void* conv_bias, int conv_row0, int conv_channels, void* stream);
@@ -650,13 +655,16 @@ int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int
  * tv_kv_append: k / v, one row of row_bytes per sequence, to position *pos (device) of the caches; all strides in bytes, everything a
  *   multiple of 16; a position outside [0, capacity) writes nothing.
  * tv_count_up: pos[0] += 1, lens[0..n) += 1.
- * tv_argmax_rows: out[r] = position of the largest of n <= 2^30 fp32 values (NaN above all, the lowest of equals: torch.argmax). */
+ * tv_argmax_rows: out[r] = position of the largest of n <= 2^30 fp32 values (NaN above all, the lowest of equals: torch.argmax).
+ * tv_argmax_rows_count: the same, and tv_count_up in its last launch (pos NULL: nothing is counted). */
 int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* pos, int batch, int64_t capacity,
                  int row_bytes, int64_t k_stride_b, int64_t v_stride_b, int64_t kc_stride_b, int64_t kc_stride_l, int64_t vc_stride_b,
                  int64_t vc_stride_l, void* stream);
 int tv_count_up(int64_t* pos, int* lens, int n, void* stream);
 size_t tv_argmax_rows_workspace_bytes(int rows);
 int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int64_t stride, void* workspace, size_t workspace_bytes, void* stream);
+int tv_argmax_rows_count(const float* x, int64_t* out, int rows, int n, int64_t stride, int64_t* pos, int* lens, int nlens,
+                         void* workspace, size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Linear attention with one constant decay per head, ragged batches:

@@ -98,6 +98,7 @@ SIGNATURES = {
     "tv_count_up": (_i, [_p, _p, _i, _p]),
     "tv_argmax_rows_workspace_bytes": (_z, [_i]),
     "tv_argmax_rows": (_i, [_p, _p, _i, _i, _l, _p, _z, _p]),
+    "tv_argmax_rows_count": (_i, [_p, _p, _i, _i, _l, _p, _p, _i, _p, _z, _p]),
     "tv_lightning_workspace_bytes": (_z, [_i] * 6),
     "tv_lightning_fwd": (_i, [_p] * 8 + [_i, _i, _p, _z] + [_i] * 3 + [_l] * 4 + [_i, _i, _p]),
     "tv_attn_generic_fwd": (_i, [_p] * 8 + [_i, _l] + [_i] * 4 + [_l] * 10 + [_f] + [_i] * 3 + [_p, _l, _l, _i, _p]),
@@ -106,6 +107,7 @@ SIGNATURES = {
     "tv_latent_decode_workspace_bytes": (_z, [_i] * 4),
     "tv_latent_decode_fwd": (_i, [_p] * 6 + [_f] + [_p] * 5 + [_i] * 6 + [_l] * 3 + [_f, _p, _z, _p]),
     "tv_gemv_post_fwd": (_i, [_p] * 3 + [_i] * 4 + [_l] * 3 + [_i] + [_p] * 4 + [_i] + [_f] * 3 + [_p, _l, _p]),
+    "tv_gemv_logits_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l] * 3 + [_p, _p, _i, _f, _p]),
     "tv_moe_decode_fwd": (_i, [_p] * 10 + [_i] * 6 + [_p]),
     "tv_moe_router_fwd": (_i, [_p] * 5 + [_l] + [_i] * 3 + [_l, _i, _i, _p]),
     "tv_moe_plan": (_i, [_p] * 5 + [_l, _i, _i, _p]),

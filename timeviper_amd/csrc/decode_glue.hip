@@ -1,7 +1,8 @@
 // What stands between the layers of a decoded token and the next one: the new keys and values into the cache, the counters, the greedy choice.
 // A launch of these takes 4 - 5 us however little it does, so what counts is how many there are, and how many compute units read the logits.
 // Measured (one sequence, in a replayed graph): index_copy_ twice 9.2 -> 4.7 us, += 1 twice 8.4 -> 3.9, argmax of 131 072 logits (one work-group
-// a row) 12.8 -> 4.8 + 4.6; a token 433 -> 421 us with the gaps that went.
+// a row) 12.8 -> 4.8 + 4.6; a token 433 -> 421 us with the gaps that went.  The counters in the greedy
+// choice's last launch, the logits as fp32 and their norm in the product (gemv.hip): 422 -> 415 of the 13 us that those launches take alone.
 #include "common.hpp"
 
 namespace {
@@ -61,9 +62,15 @@ __global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restric
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.y * ARG_BLOCKS + blockIdx.x] = better(better(s[0], s[1]), better(s[2], s[3]));
 }
-__global__ __launch_bounds__(ARG_BLOCKS) void argmax_rows_kernel(const Best* __restrict__ part, int64_t* __restrict__ out) {
+// ... and (pos not NULL) the counters that count_up_kernel moves, by the first row's work-group (3.9 us as a launch of its own)
+__global__ __launch_bounds__(ARG_BLOCKS) void argmax_rows_kernel(const Best* __restrict__ part, int64_t* __restrict__ out, int64_t* __restrict__ pos,
+                                                                 int* __restrict__ lens, int nlens) {
   const Best b = wave_best(part[blockIdx.x * ARG_BLOCKS + threadIdx.x]);
   if (threadIdx.x == 0) out[blockIdx.x] = (int64_t)b.i;
+  if (pos && blockIdx.x == 0) {
+    if (threadIdx.x == 0) pos[0] += 1;
+    for (int i = threadIdx.x; i < nlens; i += ARG_BLOCKS) lens[i] += 1;
+  }
 }
 
 }  // namespace
@@ -91,6 +98,12 @@ extern "C" int tv_count_up(int64_t* pos, int* lens, int n, void* stream) {
 extern "C" size_t tv_argmax_rows_workspace_bytes(int rows) { return rows > 0 ? (size_t)rows * ARG_BLOCKS * sizeof(Best) : 0; }
 
 extern "C" int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int64_t stride, void* workspace, size_t workspace_bytes, void* stream) {
+  return tv_argmax_rows_count(x, out, rows, n, stride, nullptr, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tv_argmax_rows_count(const float* x, int64_t* out, int rows, int n, int64_t stride, int64_t* pos, int* lens, int nlens, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(nlens >= 0 && (lens || nlens == 0), "argmax_rows: %d counters", nlens);
   TV_CHECK_ARG(x && out && workspace, "argmax_rows: null pointer");
   TV_CHECK_ARG(rows > 0 && rows <= 65535 && n > 0 && stride >= 0, "argmax_rows: rows %d, %d elements", rows, n);
   if (n > (1 << 30)) TV_UNSUPPORTED("argmax_rows: %d elements a row, at most 2^30 (positions and the step behind the last share are 32-bit)", n);
@@ -102,6 +115,6 @@ extern "C" int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int
     tv_set_error("argmax_rows: %s", hipGetErrorString(e));
     return TV_ERR_LAUNCH;
   }
-  argmax_rows_kernel<<<(unsigned)rows, ARG_BLOCKS, 0, (hipStream_t)stream>>>((const Best*)workspace, out);
+  argmax_rows_kernel<<<(unsigned)rows, ARG_BLOCKS, 0, (hipStream_t)stream>>>((const Best*)workspace, out, pos, lens, nlens);
   TV_LAUNCH_CHECK();
 }

@@ -29,7 +29,7 @@ struct SkArgs {
   bf16_t *y, *h_out, *act;
   float *y32, *res_out;
   const float* res;
-  int epi;
+  int epi, round;                                  // round: SK_F32 of the bf16 rounding
   int M, N, K, rw;                                 // rw: rows of W per work-group (SK_PAIR, second part: gate rows per work-group)
   int64_t xs, x2s, ldw, ys, as;
   int n1, ff, wg1, rw1;                            // SK_PAIR: work-groups [0, wg1) take rw1 rows each of the first n1
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_stream_kernel(SkArgs a) {
         const int o = n0 + 4 * q + j;
         float v = s[j];
         if (!two && a.bias) v += (float)a.bias[o];
-        if (a.epi == SK_F32) a.y32[(int64_t)m * a.ys + o] = v;
+        if (a.epi == SK_F32) a.y32[(int64_t)m * a.ys + o] = a.round ? (float)(bf16_t)v : v;
         else if (a.epi == SK_ADD) {
           v += a.res[(int64_t)m * a.N + o];
           a.res_out[(int64_t)m * a.N + o] = v;
@@ -276,14 +276,15 @@ extern "C" int tv_gemm_rows_fwd(const void* x, const void* W, const void* bias, 
                                 int conv_row0, int conv_channels, void* stream) {
   TV_CHECK_ARG(x && W && y, "gemm_rows: null pointer");
   TV_CHECK_ARG(M >= 2 && M <= TV_GEMM_ROWS_MAX && N >= 1 && K >= 1, "gemm_rows: M %d must be 2..%d, N %d and K %d positive", M, TV_GEMM_ROWS_MAX, N, K);
-  TV_CHECK_ARG(y_dtype == TV_BF16 || (y_dtype == TV_F32 && epilogue == 0 && !conv_state), "gemm_rows: y dtype %d", y_dtype);
-  TV_CHECK_ARG(epilogue == 0 || (epilogue == TV_GEMM_ROWS_RELU2 && !conv_state), "gemm_rows: epilogue %d", epilogue);
+  TV_CHECK_ARG(y_dtype == TV_BF16 || (y_dtype == TV_F32 && (epilogue == 0 || epilogue == TV_GEMM_ROWS_ROUND) && !conv_state), "gemm_rows: y dtype %d", y_dtype);
+  TV_CHECK_ARG(epilogue == 0 || (epilogue == TV_GEMM_ROWS_RELU2 && !conv_state) || (epilogue == TV_GEMM_ROWS_ROUND && y_dtype == TV_F32), "gemm_rows: epilogue %d", epilogue);
   if (!tv_skinny_takes(x, W, M, K, x_stride, ldw, 0))
     TV_UNSUPPORTED("gemm_rows: K must be a multiple of %d, the row strides of x and W of 8 elements, x and W 16-byte aligned", SK_KC);
   SkArgs a{};
   a.x = (const bf16_t*)x; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias;
   if (y_dtype == TV_F32) a.y32 = (float*)y; else a.y = (bf16_t*)y;
   a.M = M; a.N = N; a.K = K; a.xs = x_stride; a.ldw = ldw; a.ys = y_stride;
+  a.round = epilogue == TV_GEMM_ROWS_ROUND;
   a.epi = y_dtype == TV_F32 ? SK_F32 : epilogue == TV_GEMM_ROWS_RELU2 ? SK_RELU2 : SK_BF16;
   if (conv_state) {
     TV_CHECK_ARG(conv_weight && conv_row0 >= 0 && conv_channels > 0 && conv_row0 + conv_channels <= N,

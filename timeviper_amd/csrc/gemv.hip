@@ -45,6 +45,7 @@ struct GemvArgs {
   const bf16_t *conv_w, *conv_b;   // (channels, 4), (channels) or NULL
   int conv_lo, conv_hi;
   float* y32;                      // the outputs in fp32 instead of bf16 (router logits)
+  int y32_round;                   // ... rounded to bf16 first (a language model's logits: the conversion behind the product is a launch of 4.6 us)
   const float* res;                // PRO_POSTNORM; PRO_NONE: the outputs are added to it (fp32 res_out, bf16 h_out instead of y)
   float* res_out;
   bf16_t* h_out;
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_bf16_kernel(GemvArgs a) {
             const float v = sm + (a.bias ? (float)a.bias[n] : 0.f) + a.res[(int64_t)m * a.N + n];
             a.res_out[(int64_t)m * a.N + n] = v;
             if (a.h_out) a.h_out[(int64_t)m * a.N + n] = (bf16_t)v;
-          } else if (a.y32) a.y32[(int64_t)m * a.ys + n] = sm;
+          } else if (a.y32) a.y32[(int64_t)m * a.ys + n] = a.y32_round ? (float)(bf16_t)(sm + (a.bias ? (float)a.bias[n] : 0.f)) : sm;
           else a.y[(int64_t)m * a.ys + n] = (bf16_t)(sm + (a.bias ? (float)a.bias[n] : 0.f));
         }
       }
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_rows_kernel(GemvArgs a) {
             v += bs + a.res[(int64_t)m * a.N + nmine];
             a.res_out[(int64_t)m * a.N + nmine] = v;
             if (a.h_out) a.h_out[(int64_t)m * a.N + nmine] = (bf16_t)v;
-          } else if (a.y32) a.y32[(int64_t)m * a.ys + nmine] = v;
+          } else if (a.y32) a.y32[(int64_t)m * a.ys + nmine] = a.y32_round ? (float)out : v;
           else a.y[(int64_t)m * a.ys + nmine] = out;
         }
     }
@@ -960,6 +961,26 @@ extern "C" int tv_gemv_post_fwd(const void* x, const void* W, void* y, int y_dty
   TV_CHECK_ARG(gate, "gemv_post: gate needed");
   a.gate = (const bf16_t*)gate; a.gs = gate_stride;
   return launch_gemv<PRO_NORMGATE>(a, st);
+}
+
+// The logits of a decoded token: fp32, of the values that a bf16 product holds.  The norm in front belongs to one row; several rows go to the matrix cores.
+extern "C" int tv_gemv_logits_fwd(const void* x, const void* W, const void* bias, float* y, int M, int N, int K, int64_t x_stride, int64_t ldw, int64_t y_stride,
+                                  const void* delta, const void* norm_weight, int norm_weight_dtype, float eps, void* stream) {
+  TV_CHECK_ARG(x && W && y, "gemv_logits: null pointer");
+  TV_CHECK_ARG(M >= 1 && M <= GV_MAXM && N >= 1 && K >= 8, "gemv_logits: M %d must be 1..%d, N %d >= 1, K %d >= 8", M, GV_MAXM, N, K);
+  TV_CHECK_ARG(!norm_weight || norm_weight_dtype == TV_F32 || norm_weight_dtype == TV_BF16, "gemv_logits: norm weight dtype %d", norm_weight_dtype);
+  TV_CHECK_ARG(norm_weight ? M == 1 : !delta, "gemv_logits: the norm is that of one row, and what is added to x belongs to it");
+  if (K % 8 || ldw % 8 || x_stride % 8 || ((uintptr_t)x & 15) || ((uintptr_t)W & 15) || ((uintptr_t)delta & 15) || ((uintptr_t)norm_weight & 15))
+    TV_UNSUPPORTED("gemv_logits: K and the row strides must be multiples of 8 elements, operands 16-byte aligned");
+  if ((size_t)M * K * 2 > 128 * 1024) TV_UNSUPPORTED("gemv_logits: M x K = %d x %d does not fit the 128 KiB of LDS f(x) is held in", M, K);
+  if (norm_weight && K > 8 * GV_THREADS * 4) TV_UNSUPPORTED("gemv_logits: the norm holds a row of <= %d channels", 8 * GV_THREADS * 4);
+  if (!norm_weight && tv_skinny_takes(x, W, M, K, x_stride, ldw, 0))
+    return tv_gemm_rows_fwd(x, W, bias, y, TV_F32, M, N, K, x_stride, ldw, y_stride, TV_GEMM_ROWS_ROUND, nullptr, nullptr, nullptr, 0, 0, stream);
+  GemvArgs a{};
+  a.x = (const bf16_t*)x; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.y32 = y; a.y32_round = 1;
+  a.M = M; a.N = N; a.K = K; a.group = K; a.xs = x_stride; a.ldw = ldw; a.ys = y_stride; a.eps = eps;
+  a.delta = (const bf16_t*)delta; a.norm_w = norm_weight; a.norm_w_f32 = norm_weight_dtype == TV_F32;
+  return norm_weight ? launch_gemv<PRO_RMSNORM>(a, (hipStream_t)stream) : launch_gemv<PRO_NONE>(a, (hipStream_t)stream);
 }
 
 // residual + x W^T + bias in fp32 (residual_out) and its bf16 rounding (h_out): the output side of a layer on a 32-bit stream.

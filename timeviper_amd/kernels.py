@@ -622,14 +622,23 @@ def gemv_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def gemv_fused(x, weight, bias=None, prologue=GEMV_NONE, delta=None, sum_out=None, norm_weight=None, eps=0.0,
-               gate=None, group_size=0, conv=None):
+               gate=None, group_size=0, conv=None, out_dtype=None):
     """y = f(x) @ weight.T (+ bias) for 1..4 rows — the linear layers of a decode step (torch.nn.Linear at q_len 1) with
     the operator in front of them computed in the kernel's prologue (several rows: mostly as a launch in front of a product on the matrix cores,
     see below): GEMV_RMSNORM (NemotronHRMSNorm with the
     block's residual add: `delta` is added to x first, the sum goes to `sum_out`), GEMV_RELU2 (the MLP activation),
     GEMV_GATED (MambaRMSNormGated with `gate`), rounding where the stand-alone operators round.
     `conv=(conv_state, weight, bias, row0)`: the outputs [row0, row0 + C) go through `causal_conv1d_update` (width 4,
-    SiLU) on conv_state (B, C, 4) before they are stored — the mixer's in_proj -> conv pair as one launch (K < 8192)."""
+    SiLU) on conv_state (B, C, 4) before they are stored — the mixer's in_proj -> conv pair as one launch (K < 8192).
+    out_dtype fp32: the same values as fp32, from the product itself (GEMV_NONE, or one row's GEMV_RMSNORM without sum_out: a model's logits)."""
+    if out_dtype is not None and out_dtype != x.dtype:
+        if out_dtype != torch.float32 or gate is not None or conv is not None or sum_out is not None or prologue not in (GEMV_NONE, GEMV_RMSNORM):
+            raise TimeViperHipError("gemv_fused: fp32 outputs of GEMV_NONE, or GEMV_RMSNORM without sum_out, only")
+        if prologue == GEMV_NONE:
+            delta = norm_weight = None
+        elif norm_weight is None or x.numel() != x.shape[-1]:
+            raise TimeViperHipError("gemv_fused: the norm in front of fp32 outputs is that of one row, with a weight")
+        return _gemv_logits(x, weight, bias, delta, norm_weight, eps)
     _gpu(x, weight, bias, delta, sum_out, norm_weight, gate)
     K = x.shape[-1]
     x2 = _rows2d(x)
@@ -740,10 +749,30 @@ def _rows_product(f, weight, bias, y, epilogue=0, cst=None, cw=None, cb=None, ro
                                        y2.stride(0), int(epilogue), _p(cst), _p(cw), _p(cb), int(row0), int(nch), _stream()), "tv_gemm_rows_fwd")
 
 
-def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None):
+def _gemv_logits(x, weight, bias, delta, norm_weight, eps):
+    _gpu(x, weight, bias, delta, norm_weight)
+    x2 = _rows2d(x)
+    N, Kd = weight.shape
+    if not gemv_takes(x2, weight) or x2.shape[1] != Kd:
+        raise TimeViperHipError(f"gemv_fused: 1..4 bf16 rows, got {tuple(x.shape)} {x.dtype} against {tuple(weight.shape)} {weight.dtype}")
+    if bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous() or bias.numel() != N):
+        raise TimeViperHipError("gemv_fused: bias must be contiguous, of x's dtype")
+    if x2.shape[0] > 1 and (x2.stride(0) % 8 or x2.data_ptr() % 16):
+        x2 = x2.contiguous()
+    if (delta is not None and (delta.dtype != x.dtype or delta.shape != x.shape or not delta.is_contiguous())) or (
+            norm_weight is not None and (norm_weight.numel() != Kd or not norm_weight.is_contiguous())):
+        raise TimeViperHipError("gemv_fused: a contiguous delta of x's shape and dtype, a contiguous norm weight")
+    y = torch.empty(x.shape[:-1] + (N,), dtype=torch.float32, device=x.device)
+    check(_capi.lib().tv_gemv_logits_fwd(_p(x2), _p(weight), _p(bias), _p(y), x2.shape[0], N, Kd, x2.stride(0), weight.stride(0), N, _p(delta), _p(norm_weight),
+                                         0 if norm_weight is None else _dt(norm_weight), float(eps), _stream()), "tv_gemv_logits_fwd")
+    return y
+
+
+def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None, rounded=False):
     """x @ weight.T (+ bias) for 2..32 bf16 rows on the matrix cores (a decoded token for each of several sequences).  `relu2`: the squared
     ReLU of the bf16 product; `conv=(conv_state, weight, bias, row0)`: the outputs [row0, row0 + C) go through
-    `causal_conv1d_update` (width 4, SiLU) on conv_state (rows, C, 4), as in `gemv_fused`.  out_dtype: bf16, or fp32 without either."""
+    `causal_conv1d_update` (width 4, SiLU) on conv_state (rows, C, 4), as in `gemv_fused`.  out_dtype: bf16, or fp32 without either
+    (`rounded`: of the bf16 values)."""
     _gpu(x, weight, bias)
     if not rows_take(x, weight) or weight.shape[1] != x.shape[-1]:
         raise TimeViperHipError(f"rows_linear: 2..{ROWS_MAX} bf16 rows of a multiple of 64 elements, got {tuple(x.shape)} against {tuple(weight.shape)}")
@@ -760,7 +789,7 @@ def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None):
                 or cw.shape != (nch, 4) or (cb is not None and (cb.dtype != x.dtype or not cb.is_contiguous()))):
             raise TimeViperHipError("rows_linear: conv needs a contiguous (rows, C, 4) state and (C, 4) weight of x's dtype")
     y = torch.empty(x.shape[:-1] + (weight.shape[0],), dtype=out_dtype or x.dtype, device=x.device)
-    _rows_product(x2, weight, bias, y, 1 if relu2 else 0, cst, cw, cb, row0, nch)
+    _rows_product(x2, weight, bias, y, 1 if relu2 else 2 if rounded else 0, cst, cw, cb, row0, nch)
     return y
 
 
@@ -973,15 +1002,22 @@ def count_up(pos, lens) -> None:
     check(_capi.lib().tv_count_up(_p(pos), _p(lens), lens.numel(), _stream()), "tv_count_up")
 
 
-def argmax_rows(x):
-    """x.argmax(-1); the fp32 logits of up to 65 535 rows by 64 work-groups a row."""
-    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] <= (1 << 30)):
+def argmax_rows(x, count=None):
+    """x.argmax(-1); the fp32 logits of up to 65 535 rows by 64 work-groups a row.  count=(pos, lens): `count_up` of them in the same launches."""
+    pos, lens = count or (None, None)
+    takes = x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] <= (1 << 30)
+    if count and not (takes and lens.dtype == torch.int32 and lens.is_contiguous() and lens.is_cuda and pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1):
+        out = argmax_rows(x)
+        count_up(pos, lens)
+        return out
+    if not takes:
         return x.argmax(-1)
-    _gpu(x)
+    _gpu(x, pos, lens)
     lib, B = _capi.lib(), x.shape[0]
     out = torch.empty((B,), dtype=torch.int64, device=x.device)
     ws = torch.empty((int(lib.tv_argmax_rows_workspace_bytes(B)),), dtype=torch.uint8, device=x.device)
-    check(lib.tv_argmax_rows(_p(x), _p(out), B, x.shape[1], x.stride(0), _p(ws), ws.numel(), _stream()), "tv_argmax_rows")
+    check(lib.tv_argmax_rows_count(_p(x), _p(out), B, x.shape[1], x.stride(0), _p(pos), _p(lens), lens.numel() if count else 0, _p(ws), ws.numel(), _stream()),
+          "tv_argmax_rows_count")
     return out
 
 

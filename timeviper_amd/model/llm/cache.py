@@ -35,6 +35,10 @@ class StaticDecode:
         """Device side of one finished step (part of the captured graph)."""
         raise NotImplementedError
 
+    def static_counters(self):
+        """(an int64 counter, int32 counters) that `advance_static_device` adds one to, for a launch that does it on its way; None: call it."""
+        return None
+
     def advance_static_host(self):
         """Host side of one REPLAYED step (an eager or captured step does it by itself)."""
         raise NotImplementedError

@@ -52,8 +52,11 @@ class GraphedDecodeStep:
     def _run(self):
         logits = self.step_fn(self.ids)
         logits = logits[:, -1] if logits.dim() == 3 else logits
-        nxt = K.argmax_rows(logits)
-        self.cache.advance_static_device()
+        counters = getattr(self.cache, "static_counters", None)
+        count = counters() if counters is not None else None
+        nxt = K.argmax_rows(logits, count)
+        if count is None:
+            self.cache.advance_static_device()
         return logits, nxt
 
     @torch.inference_mode()
