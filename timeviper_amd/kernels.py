@@ -322,10 +322,35 @@ def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
             bias = bias.float()
         bias = bias.contiguous()
         bd = _dt(bias)
-    check(_capi.lib().tv_gemm_bf16_fwd(_p(x2), _p(weight), _p(bias), _p(o2), x2.shape[0], N, Kd, x2.stride(0),
-                                       weight.stride(0), o2.stride(0), int(epilogue), bd, _stream()),
+    lib, rows = _capi.lib(), x2.shape[0]
+    lead = lead_rows(rows, N, Kd, epilogue)
+    if lead and ((x2.data_ptr() | weight.data_ptr() | o2.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 or x2.stride(1) != 1
+                 or (x2.stride(0) | weight.stride(0) | o2.stride(0)) % 8 or x2.shape[1] != Kd or max(x2.stride(0), weight.stride(0)) >= (1 << 22)
+                 or not gemm_persist_on()):
+        lead = 0
+    check(lib.tv_gemm_bf16_fwd(_p(x2), _p(weight), _p(bias), _p(o2), lead or rows, N, Kd, x2.stride(0), weight.stride(0), o2.stride(0), int(epilogue), bd, _stream()),
           "tv_gemm_bf16_fwd")
+    if lead:
+        check(lib.tv_gemm_small_fwd(_p(x2[lead:]), _p(weight), _p(bias), _p(o2[lead:]), rows - lead, N, Kd, x2.stride(0), weight.stride(0), o2.stride(0),
+                                    int(epilogue), bd, 0, _stream()), "tv_gemm_small_fwd")
     return out
+
+
+def lead_rows(rows: int, n: int, k: int, epilogue: int) -> int:
+    """The rows in front of a product of short contraction that fill whole rounds of 256 x 256 tiles, where the rows behind them are one 128 x 128 tile a compute
+    unit or less: such a launch (csrc/gemm_small.hip) takes 15 us where a round that is nearly empty takes a full one's 26 - 35; 0: all rows in one launch.
+    us, one launch | two, n x k 4 352 x 1 152 with the GELU: 4 374 rows, 1.2 rounds, 67 | 56, 8 180: 108 | 94, 12 320: 143 | 132, 20 000, 5.3: 221 | 207, 35 060:
+    364 | 359; 4 096 x 1 024: 4 896: 63 | 54; 3 072 x 768: 11 552: 85 | 77; 8 192 x 2 048: 2 548: 99 | 85, 10 740: 311 | 302; plain, up to three rounds, 3 456 x 1 152:
+    5 103: 52 | 47, 10 016: 86 | 81, 23 552: 168 | 173; 6 144 x 2 048: 3 060: 84 | 75.  With 270 small tiles and more (10 416 rows: 85 | 87) the second
+    round of them costs what it saves."""
+    if epilogue not in (GEMM_BIAS, GEMM_BIAS_GELU) or not 768 <= k <= 2048 or n < 2048 or n % 8 or k % 128:
+        return 0
+    wide = -(-n // 256)
+    rounds = -(-rows // 256) * wide // CUS
+    lead = rounds * CUS // wide * 256
+    if rounds < 1 or lead >= rows or (epilogue == GEMM_BIAS and rounds > 3) or -(-(rows - lead) // 128) * -(-n // 128) > CUS:
+        return 0
+    return lead
 
 
 def param_key(params):
