@@ -2,7 +2,7 @@
 // A launch of these takes 4 - 5 us however little it does, so what counts is how many there are, and how many compute units read the logits.
 // Measured (one sequence, in a replayed graph): index_copy_ twice 9.2 -> 4.7 us, += 1 twice 8.4 -> 3.9, argmax of 131 072 logits (one work-group
 // a row) 12.8 -> 4.8 + 4.6; a token 433 -> 421 us with the gaps that went.  The counters in the greedy
-// choice's last launch, the logits as fp32 and their norm in the product (gemv.hip): 422 -> 415 of the 13 us that those launches take alone.
+// choice's last launch, and the logits as fp32 with their norm out of the product (gemv.hip): 420 -> 413 (three launches of 4 - 5 us when traced alone).
 #include "common.hpp"
 
 namespace {

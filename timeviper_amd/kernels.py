@@ -326,7 +326,7 @@ def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
     lead = lead_rows(rows, N, Kd, epilogue)
     if lead and ((x2.data_ptr() | weight.data_ptr() | o2.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 or x2.stride(1) != 1
                  or (x2.stride(0) | weight.stride(0) | o2.stride(0)) % 8 or x2.shape[1] != Kd or max(x2.stride(0), weight.stride(0)) >= (1 << 22)
-                 or not gemm_persist_on()):
+                 or (bias is not None and bd == TV_F32) or not gemm_persist_on()):         # (an fp32 bias may take launches of many tiles to another kernel)
         lead = 0
     check(lib.tv_gemm_bf16_fwd(_p(x2), _p(weight), _p(bias), _p(o2), lead or rows, N, Kd, x2.stride(0), weight.stride(0), o2.stride(0), int(epilogue), bd, _stream()),
           "tv_gemm_bf16_fwd")
