@@ -1,4 +1,4 @@
-"""linear_fused where whole rounds of large tiles take the leading rows and small tiles the rest (kernels.lead_rows), against fp32."""
+"""linear_fused and glu_linear where whole rounds of large tiles take the leading rows and small tiles the rest (kernels.lead_rows, glu_lead), against fp32."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -41,3 +41,32 @@ def test_against_fp32(rows, gelu, form):
     assert bool((err <= 1.63 * 2 ** -7 * want.abs() + 4.1e-3).all()), err.max()
     if form == "rows":
         assert bool((room[rows:] == 7).all()) and bool((room[:, n:] == 7).all())
+
+
+# one small tile a compute unit, two on some, too many; a single large tile's rows missing, a full last round, less than a round
+@pytest.mark.parametrize("rows,n,lead,tile", [(6011, 5632, 5888, 0), (3196, 5632, 2816, 1), (4750, 5632, 4750, -1), (1281, 5632, 1280, 0), (2048, 4096, 2048, -1), (1000, 5632, 1000, -1),
+                                              (300, 40000, 300, -1)])
+def test_pair_rule(rows, n, lead, tile):
+    from timeviper_amd import kernels as K
+    assert K.glu_lead(rows, n) == (lead, tile)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,tile", [(2049, 0), (2176, 0), (2177, 0), (2400, 0), (2600, 1)])
+@pytest.mark.parametrize("sliced", [True, False])
+def test_pair_against_fp64(rows, tile, sliced):
+    from timeviper_amd import kernels as K
+    n, k = 4096, 384
+    assert K.glu_lead(rows, n) == (2048, tile)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, k + 64 * sliced, generator=g, device=DEV).bfloat16()[:, :k]
+    w, b = (torch.randn(2 * n, k, generator=g, device=DEV) * k ** -0.5).bfloat16(), torch.randn(2 * n, generator=g, device=DEV).bfloat16()
+    room = torch.full((rows + 1, n + 24), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = room[:rows, 8:8 + n]
+    with torch.inference_mode():
+        K.glu_linear(x, w, b, out)
+    gate, up = (x.double() @ w.double().T + b.double()).split(n, 1)
+    want = F.gelu(gate, approximate="tanh") * up
+    # fp32 sums and functions (1e-5 of the factors; the slope of the activation is below 1.13) and one rounding
+    assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * (gate.abs() + 1) * (up.abs() + 1)).all()
+    assert (room[rows:] == 7).all() and (room[:, :8] == 7).all() and (room[:, 8 + n:] == 7).all()

@@ -1473,25 +1473,45 @@ def small_takes(x, weight, glu: bool = False, most: int = 2304) -> int:
 
 
 def glu_takes(x, weight) -> bool:
-    """Rows on which tv_gemm_glu_fwd is faster than the library's product and the pass over it: its tiles (256 rows x 128 outputs) fill half of a first round, or
-    65 % of several (us, two launches | here, 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800,
+    """Rows on which `glu_linear` is faster than the library's product and the pass over it: its tiles (256 rows x 128 outputs) fill half of a first round, or
+    65 % of several, or they leave a few rows behind rounds that are nine tenths full to small tiles (`glu_lead`), in contractions of 2 048 or less (2 x 7 680 x 2 048,
+    1 147 rows: 96 | 74; 2 x 4 096 x 1 024, 2 098: 53 | 47; 86 % full, 2 x 5 632 x 2 048, 1 403: 73 | 72; 2 x 11 008 x 4 096, 635: 129 | 133) (us, two launches | here, 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800,
     69 %: 95 | 90; 3 000: 146 | 136, 4 000: 186 | 146, 6 011: 301 | 230, 8 192: 405 | 285)."""
     N, Kd = weight.shape[0] // 2, weight.shape[1]
     tiles = -(-x.shape[0] // 256) * -(-N // 128)
     return (x.shape[0] >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2
-            and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS)) and products_take(x, weight))
+            and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS) or (Kd <= 2048 and glu_lead(x.shape[0], N)[1] == 0 and
+                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight))
+
+
+def glu_lead(rows: int, n: int):
+    """(rows in front that fill whole rounds of tv_gemm_glu_fwd's tiles, the tile of tv_gemm_small_fwd for the rows behind them); (rows, -1): one launch for all.
+    128 x 128 small tiles: one a compute unit, or two to a third of them (us, one launch | two, 2 x 5 632 x 2 048: 1 536 rows 90 | 73, 2 939: 138 | 123, 3 196, 264 small
+    tiles, 139 | 131, 6 011: 235 | 222; 2 x 4 096 x 1 024: 4 476: 85 | 78, 4 736, 320: 84 | 83; 2 x 11 008 x 4 096: 2 171: 341 | 307, 3 072, 344: 433 | 424)."""
+    wide = -(-n // 128)
+    rounds = -(-rows // 256) * wide // CUS
+    lead = rounds * CUS // wide * 256
+    small = -(-(rows - lead) // 128) * -(-n // 64)
+    if rounds < 1 or not 256 <= lead < rows or small > CUS * 4 // 3:
+        return rows, -1
+    return lead, 0 if small <= CUS else 1
 
 
 def glu_linear(x, weight, bias, out):
-    """out = gelu_tanh(x @ Wg.T + bg) * (x @ Wu.T + bu) for the two halves of weight's rows and of the bias, on tv_gemm_glu_fwd; fp32 until the one rounding."""
+    """out = gelu_tanh(x @ Wg.T + bg) * (x @ Wu.T + bu) for the two halves of weight's rows and of the bias, on tv_gemm_glu_fwd, the rows behind its whole
+    rounds on tv_gemm_small_fwd (`glu_lead`); fp32 until the one rounding."""
     _gpu(x, weight, bias, out)
     N, Kd = weight.shape[0] // 2, weight.shape[1]
     if (x.dtype != torch.bfloat16 or weight.dtype != x.dtype or out.dtype != x.dtype or weight.shape[0] % 2 or x.shape[1] != Kd or x.stride(1) != 1
             or weight.stride(1) != 1 or out.stride(1) != 1 or out.shape != (x.shape[0], N)):
         raise TimeViperHipError(f"glu_linear: {tuple(x.shape)} bf16 against {tuple(weight.shape)} into {tuple(out.shape)}")
     _bf16_bias(bias, 2 * N, "glu_linear")
-    check(_capi.lib().tv_gemm_glu_fwd(_p(x), _p(weight), _p(bias), _p(out), x.shape[0], N, Kd, x.stride(0), weight.stride(0), out.stride(0), _stream()),
+    lead, tile = glu_lead(x.shape[0], N) if (N + 128) * weight.stride(0) < (1 << 30) else (x.shape[0], -1)       # (the small tiles reach both halves at 32-bit offsets)
+    check(_capi.lib().tv_gemm_glu_fwd(_p(x), _p(weight), _p(bias), _p(out), lead, N, Kd, x.stride(0), weight.stride(0), out.stride(0), _stream()),
           "tv_gemm_glu_fwd")
+    if tile >= 0:
+        check(_capi.lib().tv_gemm_small_fwd(_p(x[lead:]), _p(weight), _p(bias), _p(out[lead:]), x.shape[0] - lead, N, Kd, x.stride(0), weight.stride(0),
+                                            out.stride(0), GEMM_GLU, _dt(bias), tile, _stream()), "tv_gemm_small_fwd")
     return out
 
 
