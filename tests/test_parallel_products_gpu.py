@@ -83,3 +83,35 @@ def test_rules(rows, glu, add):
         assert ops.glu_takes(h, inp) is glu and ops.split_add_takes(u, out) == add
         assert not ops.glu_takes(h[:, 4:], inp[:, 4:]) and not ops.split_add_takes(u[:, 4:], out[:, 4:])
     assert not ops.glu_takes(h, inp) and not ops.split_add_takes(u, out)       # gradients enabled
+
+
+# a prompt on small tiles, one on the gated pair and on shared tiles, one on the library; biases that are slices of a larger tensor
+@pytest.mark.parametrize("rows", [40, 700, 1400])
+@pytest.mark.parametrize("off", [0, 1, 4])
+def test_biases_at_any_address(rows, off):
+    """a layer's biases off 16 bytes: the library's product, as for any other operand that the kernels do not read"""
+    from timeviper_amd.model.llm.fogorax import FogoraxConfig, FogoraxForCausalLM
+    mix = {"heads": 16, "kv_heads": 4, "dim": 128, "vdim": 128, "scale": 128 ** -0.5, "mask": {"size": 1024, "keep_first": 64}}
+    with torch.device("meta"):
+        llm = FogoraxForCausalLM(FogoraxConfig(vocab_size=320, hidden_size=2048, side_dim=128, max_positions=2048,
+                                               layers=[{"type": "attention", "mixer": mix, "mlp": {"kind": "dense", "ff": 5632}}]))
+    llm = llm.to(BF).to_empty(device=DEV).requires_grad_(False)
+    r = rand(5)
+    for p in llm.parameters():
+        p.copy_(0.02 * r(*p.shape))
+    ids = torch.randint(0, 320, (rows,), generator=torch.Generator(device=DEV).manual_seed(rows), device=DEV)
+
+    def logits():
+        cache = llm.new_cache(1, capacity=rows)
+        return llm.step(ids, cache, cache.plan(cache.default_slots, [rows]))
+    with torch.inference_mode():
+        want = logits()
+        for layer in llm.backbone.layers:
+            for name in ("inp_bias", "out_bias"):
+                b = getattr(layer, name)
+                moved = torch.empty(b.numel() + 8, device=DEV, dtype=BF)[off:off + b.numel()].copy_(b)
+                assert moved.data_ptr() % 16 == 2 * off
+                layer._parameters[name] = torch.nn.Parameter(moved, requires_grad=False)
+        got = logits()
+    # the same products with other roundings: gate and factor are rounded, the sum is rounded before it meets the stream
+    assert torch.equal(got, want) if off == 0 else (got - want).norm() < 2.0 ** -6 * want.norm()

@@ -1465,14 +1465,19 @@ def products_take(x, *weights) -> bool:
                     and 64 <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights))
 
 
-def small_takes(x, weight, glu: bool = False, most: int = 2304) -> int:
+def bias_takes(b) -> bool:
+    """What the products below need of a bias: bf16 in whole 16-byte pieces, or none (the library takes any address)"""
+    return b is None or (type(b) in (torch.Tensor, torch.nn.Parameter) and b.dtype == torch.bfloat16 and b.is_contiguous() and b.data_ptr() % 16 == 0)
+
+
+def small_takes(x, weight, glu: bool = False, most: int = 2304, bias=None) -> int:
     """`small_tile` of x (rows, K) against weight, -1 where the rows are more than `most` or the operands are not what the kernel reads"""
     n = weight.shape[0] // 2 if glu else weight.shape[0]
     tile = small_tile(x.shape[0], n, x.shape[1], glu) if x.shape[0] <= most else -1
-    return tile if tile >= 0 and n % 8 == 0 and products_take(x, weight) else -1
+    return tile if tile >= 0 and n % 8 == 0 and products_take(x, weight) and bias_takes(bias) else -1
 
 
-def glu_takes(x, weight) -> bool:
+def glu_takes(x, weight, bias=None) -> bool:
     """Rows on which `glu_linear` is faster than the library's product and the pass over it: its tiles (256 rows x 128 outputs) fill half of a first round, or
     65 % of several, or they leave a few rows behind rounds that are nine tenths full to small tiles (`glu_lead`), in contractions of 2 048 or less (2 x 7 680 x 2 048,
     1 147 rows: 96 | 74; 2 x 4 096 x 1 024, 2 098: 53 | 47; 86 % full, 2 x 5 632 x 2 048, 1 403: 73 | 72; 2 x 11 008 x 4 096, 635: 129 | 133) (us, two launches | here, 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800,
@@ -1481,7 +1486,7 @@ def glu_takes(x, weight) -> bool:
     tiles = -(-x.shape[0] // 256) * -(-N // 128)
     return (x.shape[0] >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2
             and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS) or (Kd <= 2048 and glu_lead(x.shape[0], N)[1] == 0 and
-                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight))
+                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight) and bias_takes(bias))
 
 
 def glu_lead(rows: int, n: int):
@@ -1515,7 +1520,7 @@ def glu_linear(x, weight, bias, out):
     return out
 
 
-def split_add_takes(x, weight) -> int:
+def split_add_takes(x, weight, bias=None) -> int:
     """Work-groups a tile with which tv_gemm_split_add_fwd is faster than the library's product and the pass that adds it, 0 where it is not: a contraction of 4 096
     columns or more whose tiles, shared, fill 75 % of one round, 16 work-groups a tile at most (us, two launches | here, 2 048 x 7 680: 40 rows 30 | 20, 256: 30 | 30,
     700: 42 | 41, 1 000: 51 | 47, 2 100: 82 | 74, 4 000: 124 | 115; whole tiles, 6 011: 160 | 168)."""
@@ -1523,7 +1528,7 @@ def split_add_takes(x, weight) -> int:
     tiles = -(-x.shape[0] // 256) * -(-N // 256)
     splits = min(CUS // tiles, 16, Kd // 192) if tiles else 0
     pays = splits >= 2 and (tiles * splits >= 0.75 * CUS or splits == 16) and Kd >= 4096 and Kd % 64 == 0 and N >= 1024 and N % 4 == 0
-    return splits if pays and products_take(x, weight) else 0
+    return splits if pays and products_take(x, weight) and bias_takes(bias) else 0
 
 
 def split_add_linear(x, weight, residual, bias=None, splits=1):

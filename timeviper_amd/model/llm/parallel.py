@@ -92,13 +92,13 @@ class ParallelLayer(nn.Module):
         self.mixer.attend(F.linear(hs, w) if tile < 0 else K.small_linear(hs, w, tile=tile), kv_rows, plan, out=u[:, :self.k1])
         if self.mlp is not None:
             w, act = self.inp[self.n1:], u[:, self.k1:]
-            if self.k1 % 8 == 0 and K.glu_takes(h, w):
+            if self.k1 % 8 == 0 and K.glu_takes(h, w, self.inp_bias):
                 K.glu_linear(h, w, self.inp_bias, act)
-            elif self.k1 % 8 == 0 and (tile := K.small_takes(h, w, glu=True, most=HOST_BOUND_ROWS)) >= 0:
+            elif self.k1 % 8 == 0 and (tile := K.small_takes(h, w, glu=True, most=HOST_BOUND_ROWS, bias=self.inp_bias)) >= 0:
                 K.small_linear(h, w, self.inp_bias, K.GEMM_GLU, out=act, tile=tile)
             else:
                 K.gated_mul(*self.mlp.split(F.linear(h, w, self.inp_bias)), K.ACT_GELU_TANH, out=act)
-        splits = K.split_add_takes(u, self.out)
+        splits = K.split_add_takes(u, self.out, self.out_bias)
         x, h = K.split_add_linear(u, self.out, x, self.out_bias, splits) if splits else K.residual_add(x, F.linear(u, self.out, self.out_bias))
         return x, (self.side(h, ids, side_rows), self.side.norm)
 
