@@ -34,6 +34,38 @@ def test_persistent_kernel_switched_off(K, N, relu2):
         assert torch.equal(got, ops.relu2(want, inplace=True) if relu2 else want)
 
 
+# shared tiles, tiles of an odd number of steps, shared last rounds (which `large_takes` has too, or not), the squared ReLU of a single round
+@pytest.mark.parametrize("K,N,relu2,rows", [(15680, 4480, False, 512), (15680, 4480, False, 3000), (4480, 22656, False, 2200), (10240, 4480, False, 8192),
+                                            (4480, 15680, True, 700)])
+def test_shared_tiles_switched_off(K, N, relu2, rows):
+    """the same switch: the products that the split kernel has are the library's as well, and do not take the place of those that the persistent one gave up"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    lin, x = linear(K, N), torch.randn(1, rows, K, device=DEV).to(BF)
+    with torch.no_grad():
+        assert ops.split_takes(x, lin.weight, relu2) or ops.large_takes(x, lin.weight, relu2)
+        ops.gemm_set_persist(0)
+        try:
+            assert ops.split_takes(x, lin.weight, relu2) is None
+            got = nano._prompt_linear(lin, x, relu2)
+        finally:
+            ops.gemm_set_persist(-1)
+        want = lin(x)
+        assert torch.equal(got, ops.relu2(want, inplace=True) if relu2 else want)
+
+
+def test_gated_pair_switched_off():
+    from timeviper_amd import kernels as ops
+    h, w = torch.empty(6011, 2048, device=DEV, dtype=BF), torch.empty(2 * 5632, 2048, device=DEV, dtype=BF)
+    with torch.no_grad():
+        assert ops.glu_takes(h, w)
+        ops.gemm_set_persist(0)
+        try:
+            assert not ops.glu_takes(h, w)
+        finally:
+            ops.gemm_set_persist(-1)
+
+
 @pytest.mark.parametrize("rows", [5, 32])
 def test_output_layer_keeps_its_gradient(rows):
     """logits of 5..32 rows of a packed model: differentiable in the table where gradients are enabled"""

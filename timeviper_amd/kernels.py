@@ -955,7 +955,7 @@ def split_takes(x, weight, relu2=False):
             plan = (1, 0)
     takes = (plan and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 64 == 0 and N % 4 == 0
              and Kd < (1 << 22) and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
-    return plan if takes and not large_takes(x, weight, relu2) else None
+    return plan if takes and gemm_persist_on() and not large_takes(x, weight, relu2) else None
 
 
 def split_linear(x, weight, bias=None, relu2=False, splits=1, full=0):
@@ -1486,7 +1486,8 @@ def glu_takes(x, weight, bias=None) -> bool:
     tiles = -(-x.shape[0] // 256) * -(-N // 128)
     return (x.shape[0] >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2
             and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS) or (Kd <= 2048 and glu_lead(x.shape[0], N)[1] == 0 and
-                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight) and bias_takes(bias))
+                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight) and bias_takes(bias)
+            and gemm_persist_on())
 
 
 def glu_lead(rows: int, n: int):
