@@ -54,3 +54,28 @@ def test_against_64_bits(B, L, H, P, G, group_map, init, form):
     if form == "dense":
         only = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=S0, group_map=group_map)
         assert torch.equal(only, y)
+
+
+# the infinity or NaN in the first, an inner and the last token of a 16-token tile; whole and partial chunks, one segment and several
+@pytest.mark.parametrize("L,at", [(65, 0), (130, 21), (130, 129), (512, 303), (500, 495)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_tokens_in_front_of_an_infinity(L, at, value):
+    """an x that is no number is not seen by the tokens in front of it, nor by the head's other columns"""
+    from timeviper_amd import kernels as ops
+    B, H, P, G, N, h, p = 1, 4, 32, 2, 16, 2, 19
+    g = torch.Generator(device=DEV).manual_seed(L + at)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, Bm, Cm, dt = r(B, L, H, P), 0.3 * r(B, L, G, N), r(B, L, G, N), r(B, L, H)
+    A, bias, D = -torch.linspace(0.01, 2, H, device=DEV), torch.linspace(-4, 0, H, device=DEV), r(H)
+    f = lambda: ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
+    clean, S = f()
+    x[0, at, h, p] = value
+    y, fin = f()
+    assert ops.ssd_scan_last_impl() == 8
+    hit = torch.zeros(B, L, H, P, dtype=torch.bool, device=DEV)
+    hit[0, at:, h, p] = True
+    # (the tile is summed in another order: 16 terms, each within 2^-24 of the magnitudes, which are below 100 here)
+    assert (y[~hit] - clean[~hit]).abs().max() < 1e-3 and not torch.isfinite(y[0, at, h, p]) and not torch.isfinite(fin[0, h, p]).any()
+    keep = torch.ones(B, H, P, dtype=torch.bool, device=DEV)
+    keep[0, h, p] = False
+    assert torch.equal(fin[keep], S[keep])

@@ -118,6 +118,12 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
       }
     }
     if constexpr (OUT) {
+      float zero = 0.f;                                               // NaN if one of this wave's columns holds anything but numbers
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zero = fmaf(xa[st][r], 0.f, zero);
+      const bool odd = __ballot(zero != 0.f) != 0;
       f32x4 css[4], ds[4];
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
@@ -142,8 +148,21 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
             const float m = __expf(cst - css[st][r]) * ds[st][r] * M[r];
             M[r] = st < ot || 4 * q + r <= lc ? m : 0.f;
           }
+          if (st == ot && odd) {
+            // (a factor of 0 does not hide an infinity or a NaN from the tokens in front of it: term by term)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) Y = mfma4(xa[st][r], M[r], Y);
+            for (int t = 0; t < 16; ++t) {
+              const float m = from_lane(M[t & 3], 16 * (t >> 2) + lc);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const float xt = from_lane(xd[ot][r], 16 * q + t);
+                if (t <= lc) Y[r] = fmaf(xt, m, Y[r]);
+              }
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Y = mfma4(xa[st][r], M[r], Y);
+          }
         }
         if (16 * ot + lc < tt) {
           f32x4 o;
