@@ -601,16 +601,21 @@ def _realshape_model(tag, group_map):
 def test_realshape_prefill_bf16_vs_reference_golden():
     """Model-level parity at Nano-9B's real head shapes against numbers the REFERENCE produced (tests/golden/
     toy_realshape_g2.npz; the toy goldens above stop at the generic scan kernel and the small attention instance): the
-    bf16 prefill runs ssd_head_kernel<5,4,2> (asserted) and the d-128 causal attention.  group_map "tile" = the
+    bf16 prefill runs the column slices and, forced, the head-per-wave march (asserted) and the d-128 causal attention.  group_map "tile" = the
     reference CPU prefill's h % G (modeling_nano.py:781-782)."""
     from timeviper_amd import kernels as K
     cfg, model, g, L, _ = _realshape_model("g2", "tile")
     emb = torch.from_numpy(g["embeds"]).to(DEV).bfloat16()
-    with torch.no_grad():
-        out = model(inputs_embeds=emb, logits_to_keep=0).logits
-    assert K.ssd_scan_last_impl() == 6, "the prefill did not run on the head-per-wave march"
-    assert out.shape == (1, L, 96)
-    assert relerr(out, g["logits"]) < 3e-2, relerr(out, g["logits"])
+    for impl, kernel in ((0, 9), (6, 6)):      # (short: column slices by themselves)
+        K.ssd_scan_set_impl(impl)
+        try:
+            with torch.no_grad():
+                out = model(inputs_embeds=emb, logits_to_keep=0).logits
+        finally:
+            K.ssd_scan_set_impl(0)
+        assert K.ssd_scan_last_kernel() == kernel
+        assert out.shape == (1, L, 96)
+        assert relerr(out, g["logits"]) < 3e-2, relerr(out, g["logits"])
 
 
 def test_realshape_prefill_plus_graphed_fused_decode_vs_reference_golden(monkeypatch):
@@ -630,7 +635,7 @@ def test_realshape_prefill_plus_graphed_fused_decode_vs_reference_golden(monkeyp
         cache = HybridMambaAttentionDynamicCache(cfg, 1, dtype=torch.bfloat16, device=DEV)
         pre = model(inputs_embeds=emb[:, :L], past_key_values=cache, use_cache=True,
                     cache_position=torch.zeros(1, dtype=torch.long), logits_to_keep=0).logits
-        assert K.ssd_scan_last_impl() == 6
+        assert K.ssd_scan_last_kernel() == 9
         assert relerr(pre, ref[:, :L]) < 3e-2, relerr(pre, ref[:, :L])
         cache.begin_static_decode(ndec)
         cur = {}
@@ -679,7 +684,7 @@ def test_true_width_slice_vs_oracle():
           "is_interleaved": False}
     with torch.no_grad():
         out = model(inputs_embeds=emb.to(DEV), train_pdrop_args=pa).logits
-    assert K.ssd_scan_last_impl() == 6, "the prefill did not run on the head-per-wave march"
+    assert K.ssd_scan_last_kernel() == 10, "the prefill did not run on heads in segments"
     assert out.shape == (1, 1, 2048) and torch.isfinite(out).all()
     tr = [t["kept"].cpu() for t in model.backbone.last_pdrop_trace]
     assert [len(t) for t in tr] == [int(nv * 0.75), int(nv * 0.5)]

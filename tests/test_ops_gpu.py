@@ -174,7 +174,10 @@ def test_ssd_scan(K, impl, dtype, B, L, H, P, G, N):
         y_ref, fin_ref, dec_ref = R.ssd_recurrence_ref(*f[:5], D=f[5], dt_bias=f[6])
         y, fin, dec = run_scan(K, *ins)
         if impl == 8 or (impl == 0 and N <= 64 and L > 64):
-            assert K.ssd_scan_last_impl() == 8, "the chunk-parallel generic kernel did not run"
+            matrix = impl == 0 and dtype is torch.float32 and N == 16 and P % 16 == 0
+            assert K.ssd_scan_last_kernel() == (11 if matrix else 8), "the chunk-parallel generic kernel did not run"
+        if impl == 6:
+            assert K.ssd_scan_last_kernel() == 6, "the head-per-wave march did not run"
         rt, at = TOL[dtype]
         close(y, y_ref, rt, at * 2, "y")
         close(fin, fin_ref, rt, at, "final state")
@@ -195,8 +198,8 @@ def test_ssd_scan_nano_geometry_vs_oracle(K):
     four work-groups of the head march — share one B / C group, modeling_nano.py:639-653), d_state 128, 4 200 tokens (two
     sequence segments and the carried-in correction), A = 1 .. 128 and a raw dt of standard deviation 1.3 as in the
     synthetic 9B model (floating, re-basing, reset and standard steps all occur).  x, B, C come out of the conv + split +
-    C.B^T kernel at d_inner 10 240 / G 8 and are checked against the oracle's conv first; the scan then runs on the
-    default path with those fragments (head march, asserted)."""
+    C.B^T kernel at d_inner 10 240 / G 8 and are checked against the oracle's conv first; the scan then runs with those
+    fragments on the default path (heads in segments) and on the head march, both asserted."""
     B, L, H, P, G, N = 1, 4200, 128, 80, 8, 128
     d_in, conv_dim = H * P, H * P + 2 * G * N
     g = torch.Generator().manual_seed(4200)
@@ -215,18 +218,25 @@ def test_ssd_scan_nano_geometry_vs_oracle(K):
     close(Bm, ref[..., d_in:d_in + G * N].view(B, L, G, N), *TOL[torch.bfloat16], "conv B")
     close(Cm, ref[..., d_in + G * N:].view(B, L, G, N), *TOL[torch.bfloat16], "conv C")
     xh = x.view(B, L, H, P)
-    y, fin, dec = K.mamba_chunk_scan_combined(xh, dt.to(DEV), A.to(DEV), Bm, Cm, chunk_size=128, D=D.to(DEV),
-                                              dt_bias=dt_bias.to(DEV), dt_softplus=True, return_final_states=True,
-                                              return_total_decay=True, cb=cb)
-    assert K.ssd_scan_last_impl() == 6, "the scan did not run on the head-per-wave march"
+    outs = []
+    for impl, kernel in ((0, 10), (6, 6)):
+        K.ssd_scan_set_impl(impl)
+        try:
+            outs.append(K.mamba_chunk_scan_combined(xh, dt.to(DEV), A.to(DEV), Bm, Cm, chunk_size=128, D=D.to(DEV),
+                                                    dt_bias=dt_bias.to(DEV), dt_softplus=True, return_final_states=True,
+                                                    return_total_decay=True, cb=cb))
+        finally:
+            K.ssd_scan_set_impl(0)
+        assert K.ssd_scan_last_kernel() == kernel
     # the oracle on the SAME bf16 x / B / C the kernel read
     y_ref, fin_ref, dec_ref = R.ssd_recurrence_ref(xh.float().cpu(), dt.float(), A, Bm.float().cpu(), Cm.float().cpu(), D=D,
                                                    dt_bias=dt_bias)
-    close(y, y_ref, 2e-2, 4e-2, "y")
-    close(fin, fin_ref, 2e-2, 2e-2, "final state")
-    close(dec, dec_ref, 1e-4, 1e-3, "total decay")
-    rel = float((y.float().cpu().double() - y_ref).norm() / y_ref.norm())
-    assert rel < 6e-3, rel            # bf16 outputs of fp32 sums: the error is the rounding of y
+    for y, fin, dec in outs:
+        close(y, y_ref, 2e-2, 4e-2, "y")
+        close(fin, fin_ref, 2e-2, 2e-2, "final state")
+        close(dec, dec_ref, 1e-4, 1e-3, "total decay")
+        rel = float((y.float().cpu().double() - y_ref).norm() / y_ref.norm())
+        assert rel < 6e-3, rel            # bf16 outputs of fp32 sums: the error is the rounding of y
 
 
 @pytest.mark.parametrize("dtype,H,P,G,N", [(torch.float32, 8, 16, 2, 16), (torch.bfloat16, 16, 80, 8, 128)])
@@ -249,7 +259,9 @@ def test_ssd_scan_initial_state_and_sharding(K, dtype, H, P, G, N):
 
 
 _MARCH_SHAPES = [(1, 1000, 16, 80, 8), (2, 449, 8, 64, 2), (1, 64, 4, 48, 1), (1, 2049, 8, 80, 4), (1, 130, 4, 128, 2),
-                 (1, 65, 6, 24, 3), (1, 5000, 8, 80, 8), (1, 4100, 4, 72, 2), (2, 2500, 4, 56, 1)]
+                 (1, 65, 6, 24, 3), (1, 5000, 8, 80, 8), (1, 4100, 4, 72, 2), (2, 2500, 4, 56, 1),
+                 # head march: work-groups of one and of two heads at head dims 64 and 32, of four at 32
+                 (1, 900, 4, 64, 4), (1, 500, 4, 64, 2), (1, 700, 6, 32, 2), (2, 1400, 4, 32, 2), (1, 600, 8, 32, 2)]
 
 
 @pytest.mark.parametrize("B,L,H,P,G", _MARCH_SHAPES)
@@ -272,6 +284,7 @@ def test_ssd_scan_march_kernels(K, B, L, H, P, G):
                 y, fin, dec = run_scan(K, *ins, initial_states=init.to(DEV), group_map=gmap)
             finally:
                 K.ssd_scan_set_impl(0)
+            assert impl != 6 or K.ssd_scan_last_kernel() == (6 if P in (32, 64, 80) else K.ssd_scan_last_impl())
             close(y, y_ref, 2e-2, 4e-2, f"y {gmap} impl {impl}")
             close(fin, fin_ref, 2e-2, 2e-2, f"final state {gmap} impl {impl}")
             close(dec, dec_ref, 1e-4, 1e-4, f"total decay impl {impl}")
@@ -309,6 +322,7 @@ def test_ssd_scan_decay_regimes(K, regime, a_lo, a_hi, dt_mean, dt_std):
             y, fin, dec = run_scan(K, *ins, initial_states=init.to(DEV))
         finally:
             K.ssd_scan_set_impl(0)
+        assert K.ssd_scan_last_kernel() == impl
         assert torch.isfinite(y.float()).all() and torch.isfinite(fin).all()
         # y is bf16 and its terms are products of bf16-rounded operands (x~ = bf16(w x), C.B^T in bf16 — the reference's
         # chunked kernels round the same way) summed with cancellation: the error is judged against the row's magnitude.
@@ -350,7 +364,7 @@ def test_ssd_head_generated_step_is_bit_identical_to_the_cpp_step(K, regime, a_l
         for on in (1, 0):
             K.ssd_head_set_asm(on)
             y, fin, dec = run_scan(K, *ins, initial_states=init)
-            assert K.ssd_scan_last_impl() == 6
+            assert K.ssd_scan_last_kernel() == 6
             outs.append((y.clone(), fin.clone(), dec.clone()))
     finally:
         K.ssd_head_set_asm(-1)
@@ -396,6 +410,7 @@ def test_ssd_correction_walker_list_matches_the_grid(K, monkeypatch, a_lo, a_hi,
         y_list, fin_list, _ = run_scan(K, *ins)
         monkeypatch.setenv("TV_CORR_SLOTS", "3")
         y_grid, fin_grid, _ = run_scan(K, *ins)
+        assert K.ssd_scan_last_kernel() == 6
     finally:
         K.ssd_scan_set_impl(0)
     assert torch.equal(y_list, y_grid), (y_list.float() - y_grid.float()).abs().max().item()

@@ -19,9 +19,13 @@ def test_chunked(L, P, N, dtype):
     x, Bm, Cm = r(B, L, H, P).to(dtype), (0.3 * r(B, L, G, N)).to(dtype), (0.3 * r(B, L, G, N)).to(dtype)
     dt, A, bias, D = r(B, L, H).to(dtype), -torch.linspace(0.01, 8, H, device=DEV), torch.linspace(-4, 0, H, device=DEV), r(H)
     init = r(B, H, P, N)
-    y, fin, dec = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
-                                                return_total_decay=True)
-    assert ops.ssd_scan_last_impl() == 8
+    ops.ssd_scan_set_impl(8)                                   # (some of these have a form on the matrix cores, csrc/ssd_f32.hip)
+    try:
+        y, fin, dec = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
+                                                    return_total_decay=True)
+    finally:
+        ops.ssd_scan_set_impl(0)
+    assert ops.ssd_scan_last_kernel() == 8
     of = torch.arange(H, device=DEV) // (H // G)
     d = F.softplus(dt.double() + bias.double())
     S, want, mag = init.double(), torch.empty(B, L, H, P, device=DEV, dtype=torch.float64), torch.empty(B, L, H, P, device=DEV, dtype=torch.float64)

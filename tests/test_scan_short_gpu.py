@@ -45,7 +45,7 @@ def test_short_scan(K, L, B, H, P, G, group_map, decay):
     init = r(B, H, P, N)
     y, fin, dec = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
                                               group_map=group_map, return_total_decay=True)
-    assert K.ssd_scan_last_impl() == 6
+    assert K.ssd_scan_last_kernel() == 9
     h = torch.arange(H, device=DEV)
     of = h % G if group_map == "tile" else h // (H // G)
     for b in range(B):
@@ -58,18 +58,30 @@ def test_short_scan(K, L, B, H, P, G, group_map, decay):
         assert torch.allclose(dec[b].double(), (d * A.double()).sum(0), rtol=1e-4, atol=1e-4)
 
 
-def test_segments_and_slices_agree(K):
-    """either side of the rule's line: 24 chunks in one pass, 25 in segments"""
-    H, P, G, N = 16, 80, 2, 128
+# slices up to 7 chunks, heads in segments from 8 on; those up to 24 chunks a segment (here one: 512 heads), the march beyond
+@pytest.mark.parametrize("B,H,G,chunks,kernels", [(1, 16, 2, 8, (9, 10)), (4, 128, 8, 25, (10, 6))])
+def test_either_side_of_a_line_agrees(K, B, H, G, chunks, kernels):
+    P, N = 80, 128
     g = torch.Generator(device=DEV).manual_seed(3)
     r = lambda *s: torch.randn(s, generator=g, device=DEV)
-    L = 25 * 64
-    x, dt, Bm, Cm = r(1, L, H, P).bfloat16(), r(1, L, H).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16()
+    L = chunks * 64
+    x, dt, Bm, Cm = r(B, L, H, P).bfloat16(), r(B, L, H).bfloat16(), (0.3 * r(B, L, G, N)).bfloat16(), (0.3 * r(B, L, G, N)).bfloat16()
     A, bias, D = -torch.linspace(0.02, 16, H, device=DEV), torch.full((H,), -4.0, device=DEV), r(H)
-    f = lambda n: K.mamba_chunk_scan_combined(x[:, :n], dt[:, :n], A, Bm[:, :n], Cm[:, :n], D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
-    (long, _), (short, _) = f(L), f(L - 64)
-    rel = (long[:, :L - 64].float() - short.float()).norm() / short.float().norm()
-    assert rel < 5e-3, rel
+
+    def f(n):
+        y, S = K.mamba_chunk_scan_combined(x[:, :n], dt[:, :n], A, Bm[:, :n], Cm[:, :n], D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
+        return y, S, K.ssd_scan_last_kernel()
+    (long, _, b), (short, fin, a) = f(L), f(L - 64)
+    assert (a, b) == kernels
+    K.ssd_scan_set_impl(6)
+    try:
+        march, Sm, six = f(L - 64)
+    finally:
+        K.ssd_scan_set_impl(0)
+    assert six == 6
+    rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
+    # (x~ is rounded to bf16 in another frame on each side, 2^-9 at most each)
+    assert rel(long[:, :L - 64], short) < 5e-3 and rel(march, short) < 5e-3 and rel(Sm, fin) < 5e-3
 
 
 def test_segments_that_rounding_up_leaves_without_chunks(K, monkeypatch):
@@ -80,9 +92,15 @@ def test_segments_that_rounding_up_leaves_without_chunks(K, monkeypatch):
     x, dt, Bm, Cm = r(1, L, H, P).bfloat16(), r(1, L, H).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16(), (0.3 * r(1, L, G, N)).bfloat16()
     A, bias, D, init = -torch.linspace(0.02, 16, H, device=DEV), torch.full((H,), -4.0, device=DEV), r(H), r(1, H, P, N)
     f = lambda: K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True)
-    y, fin = f()
-    monkeypatch.setenv("TV_SSD_NSEG", "1")
+    K.ssd_scan_set_impl(6)
+    try:
+        y, fin = f()
+        assert K.ssd_scan_last_kernel() == 6
+    finally:
+        K.ssd_scan_set_impl(0)
+    monkeypatch.setenv("TV_SSD_NSEG", "1")                     # (asks for the march by itself)
     y1, fin1 = f()
+    assert K.ssd_scan_last_kernel() == 6 and not torch.equal(y, y1)
     rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())
     # x~ is rounded to bf16 in another frame on each side (2^-8 each), the carried-in states enter y as a product of their own
     assert torch.isfinite(y).all() and rel(y, y1) < 2.0 ** -7 and rel(fin, fin1) < 2.0 ** -7
@@ -101,7 +119,7 @@ def test_operands_expanded_over_the_tokens(K, L, which):
     x, Bm, Cm = ops.values()
     dt, A, bias, D = r(1, L, H), -torch.linspace(0.01, 16, H, device=DEV), torch.full((H,), -4.0, device=DEV), torch.ones(H, device=DEV)
     y, fin = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, return_final_states=True)
-    assert (K.ssd_scan_last_impl() == 6) == (L < 64)
+    assert K.ssd_scan_last_kernel() == (9 if L < 64 else 1)
     yr, Sr, ym, Sm = recurrence(x[0].double(), F.softplus(dt[0].double() + bias.double()), A.double(), Bm[0].double(), Cm[0].double(), D.double(),
                                 torch.zeros(H, P, N, dtype=torch.float64, device=DEV), torch.arange(H, device=DEV) // (H // G))
     assert ((y[0].double() - yr).abs() <= 1.05 * (2.0 ** -7 * ym + 2.0 ** -8 * yr.abs()) + 1e-30).all()       # (as above)
@@ -113,7 +131,7 @@ def test_operands_expanded_over_the_tokens(K, L, which):
 @pytest.mark.parametrize("B,H,P,G,group_map,L", [
     (1, 8, 80, 2, "block", 512), (1, 8, 80, 2, "tile", 577), (2, 8, 80, 2, "block", 1089), (1, 4, 32, 1, "block", 705), (2, 8, 64, 4, "tile", 640),
     (1, 2, 80, 2, "block", 1), (1, 2, 80, 2, "block", 63), (1, 2, 80, 2, "tile", 130), (1, 6, 64, 2, "block", 513),
-    (3, 128, 80, 8, "block", 65), (2, 128, 32, 8, "block", 200)])
+    (3, 128, 80, 8, "block", 65), (2, 128, 32, 8, "block", 500)])
 @pytest.mark.parametrize("decay", ["slow", "mixed", "fast"])
 def test_heads_in_segments(K, B, H, P, G, group_map, L, decay):
     N = 128
@@ -130,7 +148,7 @@ def test_heads_in_segments(K, B, H, P, G, group_map, L, decay):
     init = r(B, H, P, N)
     y, fin, dec = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=True,
                                               group_map=group_map, return_total_decay=True)
-    assert K.ssd_scan_last_impl() == 6
+    assert K.ssd_scan_last_kernel() == 10
     h = torch.arange(H, device=DEV)
     of = h % G if group_map == "tile" else h // (H // G)
     for b in range(B):

@@ -40,6 +40,7 @@ SIGNATURES = {
     "tv_ssd_state_correction": (_i, [_p] * 6 + [_i] * 6 + [_l] * 7 + [_i, _i, _f, _f, _i, _p, _z, _p]),
     "tv_ssd_scan_set_impl": (None, [_i]),
     "tv_ssd_scan_last_impl": (_i, []),
+    "tv_ssd_scan_last_kernel": (_i, []),
     "tv_ssd_head_set_asm": (None, [_i]),
     "tv_selective_state_update": (_i, [_p] * 9 + [_i] * 7 + [_p]),
     "tv_selective_state_update_rows": (_i, [_p] * 9 + [_i] * 5 + [_l] * 4 + [_i, _i, _p]),

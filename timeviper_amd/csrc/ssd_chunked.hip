@@ -358,12 +358,14 @@ int tv_ssd_chunked_launch(const void* x, const void* dt, const void* A, const vo
                           int batch, int seqlen, int nheads, int headdim, int ngroups, int dstate, int64_t xsb, int64_t xsl,
                           int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl,
                           int64_t csg, int64_t ysb, int64_t ysl, int dtype, int dt_softplus, float dt_min, float dt_max,
-                          int group_map, void* workspace, hipStream_t st) {
+                          int group_map, void* workspace, bool vector_only, int* ran, hipStream_t st) {
   // fp32, d_state 16: on the matrix cores (ssd_f32.hip)
-  if (dtype == TV_F32 && (uintptr_t)workspace % 16 == 0 &&
-      tv_ssd_f32_supported(headdim, dstate, xsb, xsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, x, Bm, Cm, y, init_state, final_state))
+  if (!vector_only && dtype == TV_F32 && (uintptr_t)workspace % 16 == 0 &&
+      tv_ssd_f32_supported(headdim, dstate, xsb, xsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, x, Bm, Cm, y, init_state, final_state)) {
+    *ran = 11;
     return tv_ssd_f32_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups, xsb, xsl, dsb, dsl,
                              bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, workspace, st);
+  }
   ChArgs a;
   a.x = x; a.dt = dt; a.Bm = Bm; a.Cm = Cm;
   a.A = (const float*)A; a.D = (const float*)D; a.dt_bias = (const float*)dt_bias;

@@ -1268,12 +1268,13 @@ struct HeadLayout {
   int nseg, seg_chunks, par_nseg, par_chunks;  // of the march; of ssd_par.hip (0: not its case)
   bool cols;
 };
-HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngroups) {
+// march_only: neither slices nor segments of ssd_par.hip (tv_ssd_scan_set_impl(6)); a number of the march's segments in the environment asks for the march too
+HeadLayout head_layout(int batch, int seqlen, int nheads, int headdim, int ngroups, bool march_only) {
   HeadLayout l;
   const size_t nchunks = (size_t)(seqlen + HQ - 1) / HQ;
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-  l.cols = use_cols(batch, nheads, headdim, ngroups, (int)nchunks);
-  l.par_nseg = l.cols ? 0 : par_segments(batch, nheads, (int)nchunks);
+  l.cols = !march_only && use_cols(batch, nheads, headdim, ngroups, (int)nchunks);
+  l.par_nseg = march_only || l.cols || getenv("TV_SSD_NSEG") ? 0 : par_segments(batch, nheads, (int)nchunks);
   l.par_chunks = l.par_nseg ? (int)((nchunks + l.par_nseg - 1) / l.par_nseg) : 0;
   if (l.par_nseg) l.par_nseg = (int)((nchunks + l.par_chunks - 1) / l.par_chunks);
   l.nseg = l.cols || l.par_nseg ? 1 : pick_segments(batch, nheads, (int)nchunks);
@@ -1337,8 +1338,8 @@ bool tv_ssd_head_supported(int seqlen, int nheads, int headdim, int ngroups, int
   return true;
 }
 
-size_t tv_ssd_head_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int ngroups) {
-  return head_layout(batch, seqlen, nheads, headdim, ngroups).total;
+size_t tv_ssd_head_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int ngroups, bool march_only) {
+  return head_layout(batch, seqlen, nheads, headdim, ngroups, march_only).total;
 }
 
 int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm,
@@ -1347,8 +1348,8 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
                        int ngroups, int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb,
                        int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg, int64_t ysb,
                        int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map,
-                       void* workspace, size_t workspace_bytes, const void* cb_pre, hipStream_t st) {
-  const HeadLayout lay = head_layout(batch, seqlen, nheads, headdim, ngroups);
+                       void* workspace, size_t workspace_bytes, const void* cb_pre, bool march_only, int* ran, hipStream_t st) {
+  const HeadLayout lay = head_layout(batch, seqlen, nheads, headdim, ngroups, march_only);
   TV_CHECK_ARG(workspace && workspace_bytes >= lay.total && (((uintptr_t)workspace) & 15) == 0,
                "ssd_head: workspace of %zu bytes (16-byte aligned) required, got %zu", lay.total, workspace_bytes);
   unsigned char* wsb = (unsigned char*)workspace;
@@ -1369,6 +1370,7 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
       const int rc = tv_ssd_cb_prepass_launch(Bm, Cm, workspace, batch, seqlen, ngroups, bsb, bsl, bsg, csb, csl, csg, st);
       if (rc != TV_OK) return rc;
     }
+    *ran = lay.par_nseg ? 10 : 9;
     if (lay.par_nseg)
       return tv_ssd_par_launch(x, dt, A, Bm, Cm, a.cb, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups,
                                xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, lay.par_nseg,

@@ -36,20 +36,20 @@ int tv_ssd_chunked_launch(const void* x, const void* dt, const void* A, const vo
                           int batch, int seqlen, int nheads, int headdim, int ngroups, int dstate, int64_t xsb, int64_t xsl,
                           int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl,
                           int64_t csg, int64_t ysb, int64_t ysl, int dtype, int dt_softplus, float dt_min, float dt_max,
-                          int group_map, void* workspace, hipStream_t st);
+                          int group_map, void* workspace, bool vector_only, int* ran, hipStream_t st);
 
 // ssd_head.hip
 bool tv_ssd_head_supported(int seqlen, int nheads, int headdim, int ngroups, int dstate, int dtype,
                            int64_t xsl, int64_t bsl, int64_t bsg, int64_t csl, int64_t csg, int64_t ysl,
                            const void* x, const void* Bm, const void* Cm, const void* y);
-size_t tv_ssd_head_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int ngroups);
+size_t tv_ssd_head_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int ngroups, bool march_only);
 int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm,
                        const void* D, const void* dt_bias, const void* init_state, void* y,
                        void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim,
                        int ngroups, int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb,
                        int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg, int64_t ysb,
                        int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map,
-                       void* workspace, size_t workspace_bytes, const void* cb_pre, hipStream_t st);
+                       void* workspace, size_t workspace_bytes, const void* cb_pre, bool march_only, int* ran, hipStream_t st);
 
 // 0 auto, 1 generic token recurrence (ssd_generic.hip: the definition), 3 slice march, two or more work-groups per head
 // (ssd_slice.hip: the fallback for head dims that split into <= 40-column slices), 4 slice march, whole-head work-groups
@@ -57,6 +57,8 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
 // 6 head-per-wave march (ssd_head.hip: a wave owns a head, a work-group the heads of one B/C group, up to 16 sequence
 // segments + correction; head_dim 32 / 64 / 80), 8 the generic path in chunk-parallel form (ssd_chunked.hip: small
 // d_state, 2 .. 64 chunks) — what automatic selection takes where no march applies.
+// Automatic selection has three more kernels, by its own rules and not to be forced, each of the family whose shapes it takes: 9 column slices (ssd_cols.hip) and
+// 10 heads in segments (ssd_par.hip), both of family 6, 11 the matrix cores' form of 8 (ssd_f32.hip).  Forced, 6 is the march and 8 is ssd_chunked.hip.
 // Removed, docs/history.md: 2 (round 1's chunk march; the number now means 3), 5 (round 3's 12-wave whole-head layout; now
 // means 4), 7 (round 4's two-waves-per-SIMD head march; now means 6).
 // process-wide override for tests / dev tools; atomic so that concurrent callers never race on it
@@ -64,10 +66,15 @@ static std::atomic<int> g_ssd_impl{0};
 static const int kAutoImpl = 6;   // head-per-wave march; falls back to 4, 3, the generic path
 
 extern "C" void tv_ssd_scan_set_impl(int impl) { g_ssd_impl.store(impl, std::memory_order_relaxed); }
-// which kernel family the most recent tv_ssd_scan_fwd / _cb_fwd of this process ran on (the numbers above; tests assert
-// that a shape reached the kernel they mean to check)
-static std::atomic<int> g_ssd_last{0};
+// which kernel family (0 .. 8 above), and which kernel (9 .. 11 as well), the most recent tv_ssd_scan_fwd / _cb_fwd of this process ran on; tests assert
+// that a shape reached the kernel they mean to check
+static std::atomic<int> g_ssd_last{0}, g_ssd_kernel{0};
 extern "C" int tv_ssd_scan_last_impl(void) { return g_ssd_last.load(std::memory_order_relaxed); }
+extern "C" int tv_ssd_scan_last_kernel(void) { return g_ssd_kernel.load(std::memory_order_relaxed); }
+static void ran_on(int impl, int kernel) {
+  g_ssd_last.store(impl, std::memory_order_relaxed);
+  g_ssd_kernel.store(kernel, std::memory_order_relaxed);
+}
 
 extern "C" size_t tv_ssd_scan_workspace_bytes(int batch, int seqlen, int nheads, int headdim,
                                               int ngroups, int dstate, int dtype) {
@@ -75,7 +82,8 @@ extern "C" size_t tv_ssd_scan_workspace_bytes(int batch, int seqlen, int nheads,
     return (tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate) + 255) / 256 * 256;
   const size_t narrow = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 0);
   const size_t wide = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 1);
-  const size_t head = tv_ssd_head_workspace_bytes(batch, seqlen, nheads, headdim, ngroups);
+  const int forced = g_ssd_impl.load(std::memory_order_relaxed);
+  const size_t head = tv_ssd_head_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, forced == 6 || forced == 7);
   size_t m = narrow > wide ? narrow : wide;             // any variant may be selected (tv_ssd_scan_set_impl)
   return ((m > head ? m : head) + 255) / 256 * 256;
 }
@@ -118,19 +126,21 @@ static int scan_impl(const void* x, const void* dt, const void* A, const void* B
   if (mfma_ok && impl == 6 &&
       tv_ssd_head_supported(seqlen, nheads, headdim, ngroups, dstate, dtype, x_stride_l, b_stride_l, b_stride_g,
                             c_stride_l, c_stride_g, y_stride_l, x, Bm, Cm, y)) {
-    g_ssd_last.store(6, std::memory_order_relaxed);
     // the head-per-wave march takes every chunk itself (floating, reset and standard steps in the one kernel)
-    return tv_ssd_head_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen,
+    int ran = 6;
+    const int rc = tv_ssd_head_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen,
                               nheads, headdim, ngroups, x_stride_b, x_stride_l, dt_stride_b, dt_stride_l, b_stride_b,
                               b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b, y_stride_l,
-                              dt_softplus, dt_min, dt_max, group_map, workspace, workspace_bytes, cb, st);
+                              dt_softplus, dt_min, dt_max, group_map, workspace, workspace_bytes, cb, forced == 6, &ran, st);
+    ran_on(6, ran);
+    return rc;
   }
   for (int wide = 1; wide >= 0; --wide) {       // impl 4 (and 6 where it does not apply): whole-head work-groups first, then slices of a head
     if (wide == 1 && impl != 4 && impl != 6) continue;
     if (mfma_ok && impl >= 3 &&
         tv_ssd_slice_supported(seqlen, nheads, headdim, ngroups, dstate, dtype, x_stride_l, b_stride_l,
                                b_stride_g, c_stride_l, c_stride_g, y_stride_l, x, Bm, Cm, y, wide)) {
-      g_ssd_last.store(wide == 1 ? 4 : 3, std::memory_order_relaxed);
+      ran_on(wide == 1 ? 4 : 3, wide == 1 ? 4 : 3);
       return tv_ssd_slice_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state,
                                  total_decay, batch, seqlen, nheads, headdim, ngroups, dstate,
                                  x_stride_b, x_stride_l, dt_stride_b, dt_stride_l, b_stride_b,
@@ -143,14 +153,16 @@ static int scan_impl(const void* x, const void* dt, const void* A, const void* B
     TV_UNSUPPORTED("ssd_scan: MFMA march kernel forced but shape / dtype / alignment unsupported or no workspace given");
   if ((forced == 0 || forced == 8) && workspace && tv_ssd_chunked_supported(seqlen, headdim, dstate) &&
       workspace_bytes >= tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate)) {
-    g_ssd_last.store(8, std::memory_order_relaxed);
-    return tv_ssd_chunked_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen,
+    int ran = 8;
+    const int rc = tv_ssd_chunked_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen,
                                  nheads, headdim, ngroups, dstate, x_stride_b, x_stride_l, dt_stride_b, dt_stride_l,
                                  b_stride_b, b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b,
-                                 y_stride_l, dtype, dt_softplus, dt_min, dt_max, group_map, workspace, st);
+                                 y_stride_l, dtype, dt_softplus, dt_min, dt_max, group_map, workspace, forced == 8, &ran, st);
+    ran_on(8, ran);
+    return rc;
   }
   if (forced == 8) TV_UNSUPPORTED("ssd_scan: chunk-parallel generic kernel forced but shape unsupported");
-  g_ssd_last.store(1, std::memory_order_relaxed);
+  ran_on(1, 1);
   return tv_ssd_generic_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state,
                                total_decay, batch, seqlen, nheads, headdim, ngroups, dstate,
                                x_stride_b, x_stride_l, dt_stride_b, dt_stride_l, b_stride_b,

@@ -76,8 +76,8 @@ def run(n, seed, verbose=False):
                 y, fin, dec = K.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, chunk_size=64, D=D, dt_bias=bias, dt_softplus=softplus,
                                                           dt_limit=limit, initial_states=init, return_final_states=True,
                                                           return_total_decay=True, group_map=gmap)
-                impl = K.ssd_scan_last_impl()
-                assert impl == 6, f"the fuzz case ran on scan implementation {impl}, not on the head march (6)"
+                impl = K.ssd_scan_last_kernel()
+                assert impl == 6, f"the fuzz case ran on scan kernel {impl}, not on the head march (6)"
                 outs.append((y.clone(), fin.clone(), dec.clone()))
         finally:
             K.ssd_head_set_asm(-1)

@@ -524,7 +524,7 @@ def selective_state_update(state, x, dt, A, B, C, D=None, z=None, dt_bias=None,
 def ssd_scan_set_impl(impl: int) -> None:
     """0 auto (= 6 where it applies, else 4, 3; other dtypes / d_state: 8, else 1), 1 generic fp32 token recurrence, 3 MFMA
     slice march on <= 40-column slices of a head, 4 whole-head slice march x sequence segments, 6 head-per-wave march
-    (ssd_head.hip), 8 chunk-parallel fp32 form (ssd_chunked.hip); 2 / 5 / 7 (removed kernels) select 3 / 4 / 6.
+    (ssd_head.hip, at every length), 8 chunk-parallel fp32 form (ssd_chunked.hip); 2 / 5 / 7 (removed kernels) select 3 / 4 / 6.
     Process-global (dev tools and tests)."""
     _capi.lib().tv_ssd_scan_set_impl(int(impl))
 
@@ -538,6 +538,12 @@ def ssd_head_set_asm(on: int) -> None:
 def ssd_scan_last_impl() -> int:
     """Kernel family (the numbers of `ssd_scan_set_impl`) the most recent scan call of this process ran on."""
     return int(_capi.lib().tv_ssd_scan_last_impl())
+
+
+def ssd_scan_last_kernel() -> int:
+    """The kernel of that call: the same numbers, and those that only automatic selection takes: 9 column slices (ssd_cols.hip) and 10 a head per work-group in
+    segments (ssd_par.hip), of family 6; 11 chunks on the fp32 matrix instruction (ssd_f32.hip), of family 8."""
+    return int(_capi.lib().tv_ssd_scan_last_kernel())
 
 
 # ------------------------------------------------------------------ attention
