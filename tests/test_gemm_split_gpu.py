@@ -66,7 +66,11 @@ def test_whole_tiles_in_front(M, N, K, splits, full):
     (4480, 10240, False, 4096, (8, 256)), (4480, 10240, False, 5600, None), (4480, 15680, False, 5000, (2, 256)), (4480, 15680, False, 5600, (1, 0)),
     (4480, 15680, False, 8192, (4, 512)), (4480, 15680, False, 10007, (1, 0)), (15680, 4480, True, 512, None), (15680, 4480, True, 1000, (1, 0)), (15680, 4480, True, 1400, (2, 256)),
     (15680, 4480, True, 2048, None), (15680, 4480, False, 1400, None), (15680, 4480, False, 1000, None), (4480, 5120, False, 512, None), (4480, 5120, False, 3000, (1, 0)),
-    (5120, 4480, False, 7000, (5, 512)), (22656, 4480, False, 768, (16, 256)), (22656, 4480, False, 1400, None), (1024, 4480, False, 3000, None)])
+    (5120, 4480, False, 7000, (5, 512)), (22656, 4480, False, 768, (16, 256)), (22656, 4480, False, 1400, None), (1024, 4480, False, 3000, None),
+    (8192, 8192, False, 400, (4, 0)), (8192, 8192, False, 1000, None), (12288, 4096, True, 800, None), (12288, 4096, True, 1000, (1, 0)), (4480, 15680, False, 7000, None),
+    (4096, 4096, False, 5000, None), (4480, 4544, False, 4096, (8, 256)), (28672, 8192, False, 600, None), (28672, 8192, False, 700, (3, 256)), (5376, 5632, False, 8835, None),
+    (5248, 5632, False, 8835, (1, 0)), (21440, 11840, False, 9244, None), (7680, 8064, False, 9993, None), (9088, 12800, False, 1335, None), (9088, 12800, False, 1500, (1, 0)),
+    (13312, 18432, False, 280, None), (13312, 18432, False, 500, (2, 0))])
 def test_rule(N, K, relu2, rows, plan, monkeypatch):
     from timeviper_amd import kernels as ops
     from timeviper_amd.model.llm import nano

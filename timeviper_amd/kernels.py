@@ -926,38 +926,46 @@ def tail_plan(rows: int, n: int, k: int):
 
 def split_takes(x, weight, relu2=False):
     """Products of more than 256 rows that tv_gemm_split_fwd runs faster than the library, and that `large_takes` does not have: (work-groups a tile, whole tiles in
-    front of those), None where the product is not one of them (us, library | here):
+    front of those), None where the product is not one of them.  Over 260 drawn sizes that the rule takes (outputs 4 096 - 30 000, columns 4 096 - 24 000, multiples of 64, rows 257 -
+    16 000, weights out of cache) a factor of 1.30 in the mean; the library's own times jump with its choice of a kernel, and 2 in 100 of the sizes lose 4 - 6 % to a
+    good one (us, library | here):
       - a long contraction into fewer outputs whose tiles leave half of the compute units idle: as many work-groups a tile as fit one round, if they fill 80 % of
-        it (4 480 x 10 240: 300 rows 59 | 52, 512: 85 | 59, 1 024: 108 | 90, 1 536: 137 | 124; 4 480 x 15 680: 300: 92 | 67, 512: 137 | 75, 1 400: 349 | 177; 75 % full,
-        600 rows of 8 192 x 28 672: 254 | 287),
-      - a contraction longer than the outputs whose last round is 80 % full (75 from 12 288 columns on): one work-group a tile, in a first round only at widths that the
-        library's 256 columns do not divide (4 096 x 11 008, 3 900 rows: 227 | 237) (4 480 x 15 680, an odd number of steps: 3 000 rows 532 | 306, 10 007: 1 382 |
-        999, 14 000: 1 728 | 1 360; 4 480 x 10 240: 3 000: 219 | 203; 4 480 x 5 120: 3 000: 117 | 107, 6 011: 224 | 207; 84 % full and the library in step, 7 000 x
-        15 680: 654 | 680),
-      - several rounds of which the last is nearly empty (`tail_plan`), of outputs up to 1.25 times as wide as the contraction is long, or of 20 480 and more up to
-        12 288 rows (22 656 x 4 480: 768 rows 182 | 132, 2 200: 378 | 339; 4 480 x 10 240: 3 700: 464 | 248, 8 192: 561 | 527; 5 120 x 4 480: 3 400: 149 | 130, 7 000:
-        382 | 241; 4 480 x 5 120, 4 096: 167 | 148, 5 000: 184 | 182),
-      - the squared ReLU in a single round that is 72 % full, or in several with such a last one (15 680 x 4 480, with the pass that it saves: 700 rows 101 | 90, 1 024:
-        122 | 103, 1 400: 185 | 170, 2 200: 266 | 243)."""
+        it, more than two up to 8 192 columns (4 480 x 10 240: 300 rows 59 | 52, 512: 85 | 59, 1 024: 108 | 90, 1 536: 137 | 124; 4 480 x 15 680: 300: 92 | 67, 512: 137 | 75,
+        1 400: 349 | 177; 75 % full, 600 rows of 8 192 x 28 672: 254 | 287; two of 8 192 x 8 192: 800: 107 | 113, 1 024: 117 | 120; two, 44 % without the padding, 13 312 x 18 432, 280: 186 | 200),
+      - a contraction longer than the outputs whose last round is 80 % full (75 from 12 288 columns on): one work-group a tile; in a first round (75 % without the
+        padding: 9 088 x 12 800, 1 335 rows, 72: 238 | 259) and in contractions of less than 8 192 only at widths that the library's 256 columns do not divide (4 096 x 11 008, 3 900 rows:
+        227 | 237; 5 376 x 5 632, 8 835: 354 | 364; 7 680 x 8 064, 9 993: 817 | 889; 4 480 x 15 680, an
+        odd number of steps: 3 000 rows 532 | 306, 10 007: 1 382 | 999, 14 000: 1 728 | 1 360; 4 480 x 10 240: 3 000: 219 | 203; 4 480 x 5 120: 3 000: 117 | 107, 6 011:
+        224 | 207), not two rounds that are full, where the library is in step (7 000 x 15 680: 654 | 680),
+      - several rounds of which the last is nearly empty (`tail_plan`), of outputs up to 1.25 times as wide as the contraction is long, from more than 4 096 columns on (4 096 x 4 096,
+        5 000 rows: 135 | 139), or of 20 480 and more up to 12 288 rows and eight rounds (21 440 x 11 840, 9 244, twelve: 3 191 | 3 327), unless a fifth of the rows would be padding
+        (28 672 x 8 192, 600: 259 | 268) (22 656 x 4 480: 768 rows 182 | 132, 2 200: 378 | 339; 4 480 x 10 240: 3 700: 464 | 248, 8 192: 561 | 527; 5 120 x 4 480: 3 400:
+        149 | 130, 7 000: 382 | 241; 4 480 x 5 120, 4 096: 167 | 148, 5 000: 184 | 182),
+      - the squared ReLU in a single round that is 72 % full, 63 without the padding (12 288 x 4 096, 800 rows, 59: 77 | 84; 28 672 x 8 192, 300, 51: 157 | 179), or in several with such
+        a last one (15 680 x 4 480, with the pass that it saves: 700 rows 101 | 90, 1 024: 122 | 103, 1 400: 185 | 170, 2 200: 266 | 243)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     rows = x.numel() // max(x.shape[-1], 1)
     tiles = -(-rows // 256) * -(-N // 256)
     if rows <= MID_MAX or N < 4096 or Kd < 4096 or rows > 32768:
         return None
     fill = tiles / (-(-tiles // CUS) * CUS)
-    fit = CUS // tiles
+    fit, useful = CUS // tiles, rows * N / 65536           # (useful: tiles without the padding)
     plan = None
     if fit >= 2:
-        plan = (fit, 0) if not relu2 and N <= Kd and Kd >= 8192 and fit <= 8 and tiles * fit >= 0.8 * CUS else None
+        pays = not relu2 and N <= Kd and Kd >= 8192 and fit <= 8 and tiles * fit >= 0.8 * CUS and (fit > 2 or (Kd > 8192 and 2 * useful >= 0.65 * CUS))
+        plan = (fit, 0) if pays else None
     elif tiles <= CUS:
-        pays = fill >= 0.72 and Kd <= 8192 if relu2 else fill >= 0.8 and N <= Kd and N % 256 != 0
+        pays = fill >= 0.72 and useful >= 0.63 * CUS and Kd <= 8192 if relu2 else fill >= 0.8 and useful >= 0.75 * CUS and N <= Kd and N % 256 != 0
         plan = (1, 0) if pays else None
     elif relu2:
         plan = tail_plan(rows, N, Kd) if Kd <= 8192 else None
     else:
-        if 4 * N <= 5 * Kd or (N >= 20480 and rows <= 12288):
+        padded = rows < 0.8 * 256 * -(-rows // 256) and tiles % CUS > CUS // 8
+        if (4 * N <= 5 * Kd and Kd > 4096) or (N >= 20480 and rows <= 12288 and tiles <= 8 * CUS and not padded):
             plan = tail_plan(rows, N, Kd)
-        if plan is None and N < Kd and fill >= (0.75 if Kd > 12288 else 0.8) and (Kd < 8192 or Kd % 128 != 0):
+        in_step = tiles <= 2 * CUS and fill > 0.96
+        if plan is None and N < Kd and fill >= (0.75 if Kd > 12288 else 0.8) and (
+                (Kd % 128 != 0 and not in_step) if Kd >= 8192 else N % 256 != 0):
             plan = (1, 0)
     takes = (plan and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and Kd % 64 == 0 and N % 4 == 0
              and Kd < (1 << 22) and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
