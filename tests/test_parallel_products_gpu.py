@@ -115,3 +115,16 @@ def test_biases_at_any_address(rows, off):
         got = logits()
     # the same products with other roundings: gate and factor are rounded, the sum is rounded before it meets the stream
     assert torch.equal(got, want) if off == 0 else (got - want).norm() < 2.0 ** -6 * want.norm()
+
+
+# a caller that does not wait for its launches: both sides of each line
+@pytest.mark.parametrize("rows,D,ff,glu,add,side", [(300, 3072, 8192, False, 0, False), (400, 3072, 8192, False, 10, False), (700, 3072, 8192, True, 7, False), (203, 4096, 11008, False, 16, False),
+                                                    (40, 4096, 11008, False, 0, False), (1400, 3072, 8192, False, 3, False), (1800, 2048, 5632, True, 4, False), (6011, 2048, 5632, True, 0, True),
+                                                    (1800, 1024, 4096, True, 0, True), (6011, 4096, 11008, True, 0, True), (6011, 8192, 28672, False, 0, False)])
+def test_rules_of_a_busy_device(rows, D, ff, glu, add, side):
+    from timeviper_amd import kernels as ops
+    z = lambda *s: torch.empty(s, device=DEV, dtype=BF)
+    h, u, inp, out = z(rows, D), z(rows, D + ff), z(2 * ff, D), z(D, D + ff)
+    with torch.no_grad():
+        assert bool(ops.glu_takes(h, inp, None, False)) is glu and ops.split_add_takes(u, out, None, False) == add
+        assert ops.side_takes(h, z(9, 128), z(128, D), z(D, 128), False) is side and ops.side_takes(h, z(9, 128), z(128, D), z(D, 128))

@@ -1491,17 +1491,27 @@ def small_takes(x, weight, glu: bool = False, most: int = 2304, bias=None) -> in
     return tile if tile >= 0 and n % 8 == 0 and products_take(x, weight) and bias_takes(bias) else -1
 
 
-def glu_takes(x, weight, bias=None) -> bool:
-    """Rows on which `glu_linear` is faster than the library's product and the pass over it: its tiles (256 rows x 128 outputs) fill half of a first round, or
-    65 % of several, or they leave a few rows behind rounds that are nine tenths full to small tiles (`glu_lead`), in contractions of 2 048 or less (2 x 7 680 x 2 048,
-    1 147 rows: 96 | 74; 2 x 4 096 x 1 024, 2 098: 53 | 47; 86 % full, 2 x 5 632 x 2 048, 1 403: 73 | 72; 2 x 11 008 x 4 096, 635: 129 | 133) (us, two launches | here, 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800,
-    69 %: 95 | 90; 3 000: 146 | 136, 4 000: 186 | 146, 6 011: 301 | 230, 8 192: 405 | 285)."""
-    N, Kd = weight.shape[0] // 2, weight.shape[1]
-    tiles = -(-x.shape[0] // 256) * -(-N // 128)
-    return (x.shape[0] >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2
-            and (tiles <= CUS or tiles >= 0.65 * CUS * -(-tiles // CUS) or (Kd <= 2048 and glu_lead(x.shape[0], N)[1] == 0 and
-                 glu_lead(x.shape[0], N)[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS))) and products_take(x, weight) and bias_takes(bias)
-            and gemm_persist_on())
+def glu_takes(x, weight, bias=None, waits: bool = True) -> bool:
+    """Rows on which `glu_linear` takes the place of the library's product and the pass over it.  waits: the caller waits for its launches, which is worth 20 us of the
+    device: tiles (256 rows x 128 outputs) for half of a first round, or 65 % of several, or a few rows behind rounds that are nine tenths full that go to small tiles
+    (`glu_lead`), in contractions of 2 048 or less.  Else it has to be the faster one: 60 % of a round without the padding, 70 % of several
+    (60 in contractions of 2 048 or less), up to 6 144 columns.
+    us, two launches | here: 2 x 5 632 x 2 048: 512 rows, 34 % full, 38 | 44; 600: 39 | 45, 700: 51 | 45, 1 000: 62 | 49; 1 300, 52 % of two rounds: 75 | 89; 1 800, 69 %: 95 | 90;
+    3 000: 146 | 136, 4 000: 186 | 146, 6 011: 301 | 230, 8 192: 405 | 285; with small tiles, 1 403: 73 | 72; 2 x 7 680 x 2 048, 1 147: 96 | 74; 2 x 4 096 x 1 024, 2 098: 53 | 47;
+    2 x 8 192 x 3 072: 300, half full, 47 | 69, 600: 66 | 72, 1 400: 135 | 140; 2 x 11 008 x 4 096: 300: 75 | 89, 900: 170 | 173; 2 x 14 336 x 4 096, 700: 165 | 174; 2 x 28 672 x 8 192, 1 800:
+    1 269 | 1 306, 6 011: 3 870 | 3 978."""
+    N, Kd, rows = weight.shape[0] // 2, weight.shape[1], x.shape[0]
+    tiles = -(-rows // 256) * -(-N // 128)
+    if not (rows >= 256 and N >= 2048 and N % 8 == 0 and Kd >= 1024 and Kd % 128 == 0 and tiles >= CUS // 2):
+        return False
+    rounds, lead = -(-tiles // CUS), (rows, -1)
+    pays = tiles <= CUS or tiles >= 0.65 * CUS * rounds
+    if pays and not waits:
+        pays = rows * N >= (0.6 if rounds == 1 or Kd <= 2048 else 0.7) * 32768 * CUS * rounds and Kd <= 6144
+    if not pays and Kd <= 2048:
+        lead = glu_lead(rows, N)
+        pays = lead[1] == 0 and lead[0] // 256 * -(-N // 128) >= 0.9 * CUS * (tiles // CUS)
+    return pays and products_take(x, weight) and bias_takes(bias) and gemm_persist_on()
 
 
 def glu_lead(rows: int, n: int):
@@ -1535,14 +1545,21 @@ def glu_linear(x, weight, bias, out):
     return out
 
 
-def split_add_takes(x, weight, bias=None) -> int:
-    """Work-groups a tile with which tv_gemm_split_add_fwd is faster than the library's product and the pass that adds it, 0 where it is not: a contraction of 4 096
-    columns or more whose tiles, shared, fill 75 % of one round, 16 work-groups a tile at most (us, two launches | here, 2 048 x 7 680: 40 rows 30 | 20, 256: 30 | 30,
-    700: 42 | 41, 1 000: 51 | 47, 2 100: 82 | 74, 4 000: 124 | 115; whole tiles, 6 011: 160 | 168)."""
+def split_add_takes(x, weight, bias=None, waits: bool = True) -> int:
+    """Work-groups a tile with which tv_gemm_split_add_fwd takes the place of the library's product and the pass that adds it, 0 where it does not.  waits: the caller
+    waits for its launches: a contraction of 4 096 columns or more whose tiles, shared, fill 75 % of one round, 16 work-groups a tile at most.  Else it has to be the
+    faster one: contractions of 7 168 columns or more, shares of more than 768, 65 % of the round without the padding; or a single row of tiles (64 rows
+    or more of 256) in 16 shares of 704 columns or more.
+    us, two launches | here: 2 048 x 7 680: 40 rows 17 | 20, 256: 26 | 30, 512: 30 | 39, 700: 41 | 42, 1 100: 55 | 53, 1 400: 55 | 58, 2 500: 92 | 84, 4 000: 130 | 121; whole
+    tiles, 6 011: 160 | 168; 1 024 x 5 120: 256: 16 | 28, 1 800: 38 | 41, 6 011: 72 | 77; 1 536 x 5 632, 1 800: 45 | 51; 3 072 x 11 264: 70: 40 | 28, 203: 40 | 37, 300, 55 % full, 42 | 47, 400: 59 | 49,
+    1 100: 111 | 86; 4 096 x 15 104: 17: 28 | 32, 203: 62 | 47, 700: 115 | 93, 1 800: 218 | 195; 8 192 x 36 864, 600, 59 % full: 344 | 379."""
     N, Kd = weight.shape
-    tiles = -(-x.shape[0] // 256) * -(-N // 256)
+    rows = x.shape[0]
+    tiles = -(-rows // 256) * -(-N // 256)
     splits = min(CUS // tiles, 16, Kd // 192) if tiles else 0
     pays = splits >= 2 and (tiles * splits >= 0.75 * CUS or splits == 16) and Kd >= 4096 and Kd % 64 == 0 and N >= 1024 and N % 4 == 0
+    if pays and not waits:
+        pays = Kd >= 7168 and ((Kd > 768 * splits and rows * N * splits >= 0.65 * 65536 * CUS) or (splits == 16 and 64 <= rows <= 256 and Kd >= 704 * 16))
     return splits if pays and products_take(x, weight) and bias_takes(bias) else 0
 
 
@@ -1564,10 +1581,15 @@ def split_add_linear(x, weight, residual, bias=None, splits=1):
     return res, h
 
 
-def side_takes(h, table, gate, proj) -> bool:
-    """Shapes tv_token_side_fwd is written for: a side of 128 columns."""
-    return gate.shape[0] == 128 and gate.shape[1] % 32 == 0 and table.stride(0) % 4 == 0 and products_take(h, gate, proj) and table.data_ptr() % 8 == 0 \
-        and table.dtype == torch.bfloat16 and table.stride(1) == 1
+def side_takes(h, table, gate, proj, waits: bool = True) -> bool:
+    """Shapes tv_token_side_fwd is written for: a side of 128 columns.  Where the caller does not wait for its launches, rows on which it is faster than the three of
+    them, too: its work-groups read both matrices whole, so that few rows of a wide model take as long as thousands (us, three launches | here, 512 wide: 17 to
+    8 192 rows 12 - 18 | 8 - 11; 1 024: 12 - 23 | 11 - 16; 2 048: 40 rows 12 | 17, 1 100: 16 | 19, 2 500: 22 | 23, 3 300: 25 | 23, 6 011: 29 | 26; 3 072: 4 000: 30 | 34, 6 011: 46 | 35;
+    4 096: 203: 15 | 30, 5 000: 42 | 44, 6 011: 50 | 45; 8 192: 203: 16 | 76, 6 011: 69 | 79)."""
+    rows, width = h.shape[0], gate.shape[1]
+    return (gate.shape[0] == 128 and width % 32 == 0 and table.stride(0) % 4 == 0
+            and (waits or width <= 1024 or (width <= 2048 and rows >= 3072) or (width <= 4096 and rows >= 6000))
+            and products_take(h, gate, proj) and table.data_ptr() % 8 == 0 and table.dtype == torch.bfloat16 and table.stride(1) == 1)
 
 
 def token_side(h, ids, table, gate, proj):

@@ -20,7 +20,12 @@ from ... import kernels as K
 from .mixers import _weight
 
 
-HOST_BOUND_ROWS = 768      # up to here a prompt of eight layers of width 2 048 waits for its launches (700 tokens 1.65 ms, 100: 1.58), not for its products
+# A prompt of a few hundred rows waits for its launches, not for its products: 225 us of host time a layer on library calls (150 on the kernels below), which
+# 768 rows of a layer with 50 million entries keep the device busy for.  Up to there a kernel that saves a call may take somewhat longer than what it stands in
+# for; wider layers come to that line with fewer rows (us a prompt of eight layers, on library calls | without the bound on the work: width 2 048, 768
+# rows: 1 824 | 1 582; 3 072, 203: 1 815 | 1 548, 400: 1 860 | 1 923; 4 096, 203: 1 948 | 2 071).
+HOST_BOUND_ROWS = 768
+HOST_BOUND_WORK = HOST_BOUND_ROWS * 50_000_000
 
 
 class GatedFeedForward:
@@ -50,9 +55,9 @@ class TokenSide(nn.Module):
     def checkpoint_tensors(self):
         return [("gate", self.gate), ("proj", self.proj), ("norm", self.norm)]
 
-    def forward(self, h, ids, rows):
-        """h: the stream in the model's dtype; rows (vocab, dim): this layer's slice of the table"""
-        if K.side_takes(h, rows, self.gate, self.proj):
+    def forward(self, h, ids, rows, waits=True):
+        """h: the stream in the model's dtype; rows (vocab, dim): this layer's slice of the table; waits: the caller waits for its launches"""
+        if K.side_takes(h, rows, self.gate, self.proj, waits):
             return K.token_side(h, ids, rows, self.gate, self.proj)
         return F.linear(K.gated_mul(F.linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
 
@@ -87,20 +92,21 @@ class ParallelLayer(nn.Module):
         y, w = pending or (None, None)
         x, h, hs = K.norm_shift(x, self.gain, self.eps, y, w, self.shift, state, plan, need_h=self.mlp is not None)
         u = torch.empty((x.shape[0], self.out.shape[1]), dtype=hs.dtype, device=hs.device)
-        w = self.inp[:self.n1]
-        tile = K.small_takes(hs, w, most=HOST_BOUND_ROWS)
+        w, waits = self.inp[:self.n1], x.shape[0] * (self.inp.numel() + self.out.numel()) <= HOST_BOUND_WORK
+        most = HOST_BOUND_ROWS if waits else 0
+        tile = K.small_takes(hs, w, most=most)
         self.mixer.attend(F.linear(hs, w) if tile < 0 else K.small_linear(hs, w, tile=tile), kv_rows, plan, out=u[:, :self.k1])
         if self.mlp is not None:
             w, act = self.inp[self.n1:], u[:, self.k1:]
-            if self.k1 % 8 == 0 and K.glu_takes(h, w, self.inp_bias):
+            if self.k1 % 8 == 0 and K.glu_takes(h, w, self.inp_bias, waits):
                 K.glu_linear(h, w, self.inp_bias, act)
-            elif self.k1 % 8 == 0 and (tile := K.small_takes(h, w, glu=True, most=HOST_BOUND_ROWS, bias=self.inp_bias)) >= 0:
+            elif self.k1 % 8 == 0 and (tile := K.small_takes(h, w, glu=True, most=most, bias=self.inp_bias)) >= 0:
                 K.small_linear(h, w, self.inp_bias, K.GEMM_GLU, out=act, tile=tile)
             else:
                 K.gated_mul(*self.mlp.split(F.linear(h, w, self.inp_bias)), K.ACT_GELU_TANH, out=act)
-        splits = K.split_add_takes(u, self.out, self.out_bias)
+        splits = K.split_add_takes(u, self.out, self.out_bias, waits)
         x, h = K.split_add_linear(u, self.out, x, self.out_bias, splits) if splits else K.residual_add(x, F.linear(u, self.out, self.out_bias))
-        return x, (self.side(h, ids, side_rows), self.side.norm)
+        return x, (self.side(h, ids, side_rows, waits), self.side.norm)
 
     def decode_takes(self, rows, dtype):
         if 4 < rows <= K.ROWS_MAX:               # the products on the matrix cores (gate and up rows of one work-group at 32-bit offsets)
