@@ -1,10 +1,11 @@
 // A1 / T3 / ViT: fused softmax attention forward on CDNA4 MFMA tiles.
 //
 // Structure (wave64, v_mfma_f32_32x32x16): a workgroup of 8 waves owns 256 query
-// rows of one (batch, q-head) (128 with half of the keys a wave where those are too few work-groups); each wave keeps
+// rows of one (batch, q-head) (128 with half of the keys a wave where those are too few work-groups; 4 waves for 128 rows of many short ones); each wave keeps
 // its 32 query rows as MFMA B fragments in registers for the whole kernel.  K/V tiles
 // of 96 keys arrive by LDS-DMA into a 3-stage ring shared by the waves, two tiles ahead
-// of the math (counted vmcnt, one barrier per tile).  The score tile is computed
+// of the math (counted vmcnt, one barrier per tile); with two waves a row, steps of two tiles
+// of 64 keys into a ring of two stages, one step ahead.  The score tile is computed
 // TRANSPOSED, S^T = K . Q^T, so every lane owns one query column: the softmax
 // row statistics are per-lane scalars (one cross-half shuffle per tile), and the
 // P^T accumulator registers are, after a bf16 pack, directly the B operand of
@@ -115,7 +116,7 @@ __device__ __forceinline__ void block_of(int id, int pairs, int& t, int& pair) {
 // KS = ceil(D/16) k-steps of QK^T, DT = ceil(D/32) d-tiles of PV, NW waves per workgroup.
 // K/V tiles of 32*KT keys go global -> LDS by LDS-DMA (global_load_lds_dwordx4, 16 bytes per
 // lane, no VGPR round trip: staging through registers cost a third of the kernel) into a
-// ring of 3 stages, two tiles ahead of the math, with counted vmcnt waits and one barrier
+// ring of 3 stages (KG 2: two), two tiles (one step) ahead of the math, with counted vmcnt waits and one barrier
 // per tile.  LDS rows are 256 bytes (128 elements); the 16-byte chunks of a row are
 // XOR-swizzled on the DMA source address so that the row reads of K (ds_read_b128, chunk ^
 // row%16) and the transposing reads of V (ds_read_b64_tr_b16, chunk ^ 4(row%4)) are bank
@@ -175,6 +176,10 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     h = pair % a.Hq;
     b = pair / a.Hq;
     if (b >= a.nb) return;                    // (batch, head) pairs are padded to a multiple of 8
+  } else if constexpr (NW == 4) {               // short sequences: one block each, a grid of heads and batch entries
+    qblk = 0;
+    h = blockIdx.y;
+    b = blockIdx.z;
   } else {
     const int pairs = a.nb * a.Hq;
     int pair;
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     if (!active && ahead) issue_tile(kt + NS - 1);
     if (active) {
       // ---- S^T = K . Q^T  (2 key sub-tiles of 32); all K fragment reads ahead of the MFMAs;
-      // the copies of tile kt+2 are issued between the MFMAs, whose pipe time hides them ----
+      // the copies of tile kt+2 (KG 2: of step kt+1) are issued between the MFMAs, whose pipe time hides them ----
       f32x16 sacc[KT];
       v8 kf[KT][KS];
       unsigned kb[KS];
@@ -431,7 +436,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
         }
       }
     }
-    // tile kt+1 (issued an iteration ago) must have landed; this iteration's copies stay in flight
+    // tile kt+1 (issued an iteration ago) must have landed; this iteration's copies stay in flight (KG 2: step kt+1 is this iteration's, and is waited for)
     if (NS > 2 && ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -927,6 +932,11 @@ std::atomic<int> g_fa_variant{[] { const char* v = getenv("TV_FA_W64"); return v
 bool two_waves_a_row(int Lq, int64_t blocks256, int64_t blocks128, bool triangle) {
   return Lq <= 128 || blocks128 <= tv_cu_count() || (triangle && blocks256 <= tv_cu_count());
 }
+// ... but not for more than a round of such short rows whose keys are one tile of 96: the second wave has nothing to do, or a masked step where one wave's tile has none.  Head
+// dims up to 64, and non-causal rows against 96 keys, against 65 and more at head dim 128 (16 heads, us, two waves | one, 320 and 16 384 pairs: 64 wide, causal,
+// 65 x 65: 14.9 | 13.9, 433 | 396; 48 x 48: 13.7 | 13.4, 384 | 382; 80 wide, 96 x 96: 16.7 | 14.5, 499 | 452; 128 wide: 19.7 | 16.5, 603 | 535, 80 x 80 19.1 | 18.3, 572 | 567; 80
+// wide: 80 x 80 476 | 482, causal 96 x 96 501 | 517).  Those start by head and batch entry: the division of a 1-D grid is 6 % of them (65 x 65: 428 | 396).
+bool one_tile(int ks, int Lk, int tile, bool causal) { return Lk <= tile && (ks <= 4 || (!causal && (Lk == tile || (ks > 6 && Lk > 64)))); }
 constexpr int FA_LDS2 = 2 * 2 * 2 * 64 * 256;    // K and V of two steps of 128 keys
 
 template <typename T, int KS, int DT>
@@ -938,7 +948,10 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   const int nqb = (a.Lq + 255) / 256;
   static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
   const bool frames = a.Lq > 128 && xcd_ && !a.causal && nqb <= 8 && all >= 64;
-  if (!frames && two_waves_a_row(a.Lq, nqb * all, (a.Lq + 127) / 128 * all, a.causal && a.Lk - a.Lq <= a.Lq / 4)) {
+  if (a.Lq <= 128 && all > tv_cu_count() && one_tile(KS, a.Lk, 32 * KT, a.causal) && B <= 65535 && a.Hq <= 65535) {
+    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
+  } else if (!frames && two_waves_a_row(a.Lq, nqb * all, (a.Lq + 127) / 128 * all, a.causal && a.Lk - a.Lq <= a.Lq / 4)) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS2);
     if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 8, 2, false, 2><<<dim3((unsigned)((a.Lq + 127) / 128 * all)), 512, FA_LDS2, st>>>(a, NoSeqs{});
   } else {
