@@ -63,3 +63,53 @@ def test_a_cache_that_counts_otherwise_is_asked():
         assert c.static_counters() is want
         c._static = {3: pair, 4: pair}
         assert c.static_counters() is None
+
+
+def _last_norm(llm, how):
+    """what a caller may have put in the way of the norm in front of the logits; returns a list of the norm's calls that a hook saw"""
+    seen, norm, head = [], llm.backbone.norm_f, llm.lm_head
+    if how == "hook":
+        norm.register_forward_hook(lambda *a: seen.append(1))
+    elif how == "half":
+        norm.weight = torch.nn.Parameter(norm.weight.detach().half(), requires_grad=False)
+    elif how == "strided":
+        norm.weight = torch.nn.Parameter(norm.weight.detach().repeat_interleave(2)[::2], requires_grad=False)
+    elif how == "fp32":
+        norm.weight = torch.nn.Parameter(norm.weight.detach().float(), requires_grad=False)
+    elif how == "subclass":
+        head.__class__ = type("Mine", (torch.nn.Linear,), {})
+    elif how == "bias":
+        head.bias = torch.nn.Parameter(torch.zeros(head.out_features, device=DEV, dtype=torch.bfloat16), requires_grad=False)
+    return seen
+
+
+# the norm goes with the product, or is called, with the same logits either way
+@pytest.mark.parametrize("how,inside", [("plain", True), ("fp32", True), ("bias", True), ("hook", False), ("half", False), ("strided", False), ("subclass", False), ("hidden", False),
+                                        ("two", False)])
+def test_a_model_of_which_one_token_is_decoded(how, inside, monkeypatch):
+    from timeviper_amd import kernels as K
+    from timeviper_amd.model.llm.nano import HybridMambaAttentionDynamicCache, NemotronHConfig, NemotronHForCausalLM
+    cfg = NemotronHConfig(vocab_size=1000, hidden_size=256, intermediate_size=512, num_hidden_layers=3, hybrid_override_pattern="M*-", num_attention_heads=4, head_dim=128,
+                          num_key_value_heads=2, ssm_state_size=128, mamba_num_heads=8, mamba_n_groups=2, mamba_head_dim=80)
+    torch.manual_seed(3)
+    llm = NemotronHForCausalLM(cfg).to(DEV).bfloat16().eval().requires_grad_(False)
+    llm.backbone.norm_f.weight.copy_(1 + 0.1 * _mk(256))
+    B, ids = 2 if how == "two" else 1, torch.arange(40, device=DEV).view(1, 40)
+    calls, real = [], K.gemv_fused
+    monkeypatch.setattr(K, "gemv_fused", lambda *a, **k: (calls.append(k.get("norm_weight") is not None and k.get("out_dtype") is torch.float32), real(*a, **k))[1])
+
+    def decode():
+        cache = HybridMambaAttentionDynamicCache(cfg, B, dtype=torch.bfloat16, device=DEV)
+        llm(input_ids=ids[:, :-1].expand(B, -1), past_key_values=cache, use_cache=True, cache_position=torch.arange(39))
+        calls.clear()
+        return llm(input_ids=ids[:, -1:].expand(B, -1).contiguous(), past_key_values=cache, use_cache=True, cache_position=torch.tensor([39]), output_hidden_states=how == "hidden")
+    with torch.inference_mode():
+        seen = _last_norm(llm, how)
+        out = decode()
+        assert any(calls) is inside and len(seen) == (2 if how == "hook" else 0)
+        monkeypatch.setattr("timeviper_amd.model.llm.nano._norm_and_head", lambda bb, head: False)
+        want = decode()
+        assert not any(calls)
+    if how == "hidden":
+        assert out.hidden_states[-1].shape == (1, 1, 256)
+    assert out.logits.dtype == torch.float32 and torch.equal(out.logits, want.logits)

@@ -324,6 +324,17 @@ def _logits(mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     return _linear(mod, x).float()
 
 
+def _norm_and_head(bb: nn.Module, head: nn.Module) -> bool:
+    """Whether the product of one decoded token's logits may take the model's last norm with it: both as they are here, and operands that it reads as they lie (what
+    norm_f copies or converts, and what the plain product does, stays with them)"""
+    if not (type(bb) is NemotronHModel and unhooked(bb) and type(bb.norm_f) is NemotronHRMSNorm and unhooked(bb.norm_f) and type(head) is nn.Linear and unhooked(head)):
+        return False
+    w, nw, b = head.weight, bb.norm_f.weight, head.bias
+    return (w.dtype == torch.bfloat16 and w.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and w.stride(1) == 1
+            and nw.dtype in (torch.float32, torch.bfloat16) and nw.is_contiguous() and nw.data_ptr() % 16 == 0
+            and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous())))
+
+
 def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torch.Tensor:
     """mod(x), or its squared ReLU, for a prompt's rows: on tv_gemm_rows_fwd (2..32), tv_gemm_mid_fwd (up to 256), tv_gemm_split_fwd or tv_gemm_bf16_fwd where
     those are faster than the library (`plain_linear`: a module with anything around it is called)."""
@@ -875,7 +886,8 @@ class NemotronHModel(PdropMixin, nn.Module):
             else:
                 normed, hidden = block.norm(hidden, residual=delta, return_sum=True)
             delta = block.mix(normed, past_key_values, cache_position, None, position_ids)
-        if fused_step and kwargs.get("norm_in_head", False) and hidden.shape[0] == 1 and delta is not None:
+        if (fused_step and kwargs.get("norm_in_head", False) and hidden.shape[0] == 1 and delta is not None and delta.dtype == hidden.dtype
+                and delta.shape == hidden.shape and delta.is_contiguous()):
             hidden = (hidden, delta)           # (the head's product norms the sum)
         else:
             hidden = self.norm_f(hidden, residual=delta) if delta is not None else self.norm_f(hidden)
@@ -953,8 +965,7 @@ class NemotronHForCausalLM(nn.Module):
                 use_cache=None, cache_position=None, attention_mask=None, logits_to_keep=None,
                 **kwargs):
         bb, head = self.backbone, self.lm_head
-        if type(bb) is NemotronHModel and unhooked(bb) and type(bb.norm_f) is NemotronHRMSNorm and unhooked(bb.norm_f) and head.weight.dtype == torch.bfloat16 \
-                and type(head) is nn.Linear and unhooked(head) and head.weight.data_ptr() % 16 == 0 and head.weight.stride(0) % 8 == 0 and head.weight.stride(1) == 1:
+        if _norm_and_head(bb, head):
             kwargs["norm_in_head"] = True      # one decoded token (4.6 us of 422: the norm as a launch)
         out = self.backbone(input_ids, past_key_values=past_key_values, inputs_embeds=inputs_embeds,
                             position_ids=position_ids, output_hidden_states=output_hidden_states,
