@@ -88,3 +88,16 @@ def test_rule(N, K, relu2, rows, plan, monkeypatch):
             nano._prompt_linear(lin, x, relu2)
         nano._prompt_linear(lin, x[:, :300])                  # gradients enabled: the module
     assert calls == ([(relu2, *plan)] if plan else [])
+
+
+def test_linear_fused_takes_what_it_took():
+    """shared last rounds inside linear_fused: an odd number of steps stays refused, rows with strides are copied once and keep their leading shape"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(1)
+    w = (0.02 * torch.randn(4480, 4224, generator=g, device=DEV)).to(BF)
+    x = torch.randn(2, 2048, 2 * 4224, generator=g, device=DEV).to(BF)[:, :, ::2]
+    assert ops.tail_plan(4096, 4480, 4224) and ops.tail_plan(4096, 4480, 4160)
+    got = ops.linear_fused(x, w)
+    assert got.shape == (2, 2048, 4480) and torch.equal(got.view(4096, 4480), ops.linear_fused(x.reshape(4096, 4224), w))
+    with pytest.raises(ops.TimeViperHipError):
+        ops.linear_fused(x[..., :4160].contiguous(), w[:, :4160].contiguous())

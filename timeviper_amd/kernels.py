@@ -302,11 +302,11 @@ def linear_fused(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None):
     N, Kd = weight.shape
     if weight.stride(1) != 1:
         weight = weight.contiguous()
-    if out is None and epilogue in (GEMM_BIAS, GEMM_BIAS_RELU2) and Kd >= 4096 and x.shape[-1] == Kd and x2.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 \
-            and (x2.data_ptr() | weight.data_ptr()) % 16 == 0 and bias is None and N % 8 == 0 and gemm_persist_on():
+    if out is None and epilogue in (GEMM_BIAS, GEMM_BIAS_RELU2) and Kd >= 4096 and Kd % 128 == 0 and x.shape[-1] == Kd and x2.stride(0) % 8 == 0 \
+            and weight.stride(0) % 8 == 0 and (x2.data_ptr() | weight.data_ptr()) % 16 == 0 and bias is None and N % 8 == 0 and gemm_persist_on():
         plan = tail_plan(x2.shape[0], N, Kd)
         if plan:
-            return split_linear(x, weight, None, epilogue == GEMM_BIAS_RELU2, *plan)
+            return split_linear(x2.view(x.shape), weight, None, epilogue == GEMM_BIAS_RELU2, *plan)
     if epilogue == GEMM_ACCUM:
         if out is None:
             raise TimeViperHipError("linear_fused: GEMM_ACCUM needs `out`")
