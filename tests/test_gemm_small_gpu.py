@@ -60,6 +60,18 @@ def test_rule(rows, n, k, glu, tile):
         assert ops.small_takes(x[:, 4:], w[:, 4:], glu) == -1 and ops.small_takes(x.float(), w.float(), glu) == -1
 
 
+def test_rows_far_apart():
+    """what the copies' 32-bit offsets do not reach is not taken (and refused by the kernel)"""
+    from timeviper_amd import kernels as ops
+    flat, out = torch.empty(1024 * 1_700_000 + 64, device=DEV, dtype=BF), torch.empty(17, 512, device=DEV, dtype=BF)
+    x, w = flat[:17 * 64].view(17, 64), flat.as_strided((1024, 64), (1_700_000 // 8 * 8, 1))
+    with torch.no_grad():
+        assert ops.small_takes(x, w.contiguous(), True) == 3 and ops.small_takes(x, w, True) == -1 and ops.small_takes(x, w[:512]) == 3
+        assert ops.small_takes(flat.as_strided((17, 64), (1 << 22, 1)), w[:512]) == -1 and ops.small_takes(flat.as_strided((17, 64), ((1 << 22) - 8, 1)), w[:512]) == 3
+    with pytest.raises(ops.TimeViperHipError):
+        ops.small_linear(x, w, torch.zeros(1024, device=DEV, dtype=BF), ops.GEMM_GLU, out=out)
+
+
 @pytest.mark.parametrize("frames", [1, 3])
 def test_short_clips(frames, monkeypatch):
     """a block of a short clip on small tiles, and on the library where something stands around its layers"""

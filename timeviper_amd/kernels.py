@@ -1473,8 +1473,8 @@ ACT_SIGMOID, ACT_GELU_TANH = 0, 1
 
 def products_take(x, *weights) -> bool:
     """What the products below need of a layer's rows and matrices: bf16 on the GPU, whole 16-byte rows, no gradients, no autocast, plain tensors."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and x.shape[0] > 0
-            and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) < (1 << 22) and x.data_ptr() % 16 == 0
+            and x.shape[0] > 0 and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
             and all(type(w) in (torch.Tensor, torch.nn.Parameter) and w.dtype == torch.bfloat16 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 8 == 0
                     and 64 <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights))
 
@@ -1488,7 +1488,8 @@ def small_takes(x, weight, glu: bool = False, most: int = 2304, bias=None) -> in
     """`small_tile` of x (rows, K) against weight, -1 where the rows are more than `most` or the operands are not what the kernel reads"""
     n = weight.shape[0] // 2 if glu else weight.shape[0]
     tile = small_tile(x.shape[0], n, x.shape[1], glu) if x.shape[0] <= most else -1
-    return tile if tile >= 0 and n % 8 == 0 and products_take(x, weight) and bias_takes(bias) else -1
+    reach = ((n if glu else 0) + 128) * weight.stride(0) < (1 << 30)             # (both halves of a gated pair at 32-bit offsets)
+    return tile if tile >= 0 and n % 8 == 0 and reach and products_take(x, weight) and bias_takes(bias) else -1
 
 
 def glu_takes(x, weight, bias=None, waits: bool = True) -> bool:
