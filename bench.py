@@ -10,7 +10,7 @@ the frame/token sequence is sharded over the ranks (timeviper_amd.distributed; f
 that causal attention does not leave the last rank behind) and the total work is fixed
 ("scaling": "strong").  Rank 0 prints ONE JSON line.
 
-roofline: the SSD selective-scan kernel — algorithmic bytes (SURVEY §8d: 45 312 B per
+roofline: the SSD selective-scan kernel — algorithmic bytes (45 312 B per
 token per Mamba layer at Nano dims, bf16) / its launch durations measured live with
 events on the launch stream inside the timed steps.  rooflines: the same for the ViT
 attention, the causal LLM attention (useful FLOPs against the dense bf16 MFMA peak) and the
@@ -36,10 +36,10 @@ sys.path.insert(0, str(ROOT))
 
 PDROP = "uni_14_0.8-attn_21_0.6-attn_30_0.4-attn_39_0.2"   # evaluate.py:170 defaults
 TOK_PER_FRAME = 16                                         # arch_specifier tome_mlp-16
-HBM_PEAK_GBS = 8000.0                                      # MI355X_MICROARCH.md
+HBM_PEAK_GBS = 8000.0                                      # nominal
 
 
-MFMA_BF16_PEAK_TFLOPS = 2500.0                             # dense bf16, MI355X_MICROARCH.md
+MFMA_BF16_PEAK_TFLOPS = 2500.0                             # dense bf16, nominal
 OWN_EPILOGUE = {0: "", 1: " + GELU", 2: " (+=)", 3: " + squared ReLU"}      # of kernels.linear_fused
 SCAN_SOURCES = ("ssd_head.hip", "ssd_head_step.inc", "ssd_slice.hip", "ssd_correct.hip", "ssd_scan.hip", "ssd_common.hpp", "conv1d.hip")
 
@@ -166,7 +166,7 @@ class OpTimers:
             flops = 2.0 * F_ * n * Cin * pp * pp * weight.shape[0]
             byts = F_ * (Cin * Hh * Ww + n * weight.shape[0]) * pixels.element_size()
             return ("patch_embed", (flops, byts))
-        # HBM-bound companions of the scan (SURVEY 8d: bytes per token and Mamba layer) and the ViT's element-wise passes:
+        # HBM-bound companions of the scan (bytes per token and Mamba layer) and the ViT's element-wise passes:
         # key[1] = algorithmic bytes of the call
         def conv(xBC, weight, bias, d_inner, ngroups, dstate, *a, **kw):
             return ("conv", xBC.shape[0] * xBC.shape[1] * 2 * xBC.shape[2] * xBC.element_size())   # xBC read, x|B|C written
@@ -239,8 +239,8 @@ class OpTimers:
             return None
         tokens = sum(n for _, _, n in r)
         gbs = tokens * bytes_per_token / (ms * 1e-3) / 1e9
-        # HBM bytes actually moved per algorithmic byte: rocprofv3 PMC passes (FETCH_SIZE x2, WRITE_SIZE,
-        # MI355X_MICROARCH.md) on this op, committed under profiles/ (PMC cannot be collected from
+        # HBM bytes actually moved per algorithmic byte: rocprofv3 PMC passes (FETCH_SIZE x2, WRITE_SIZE) on
+        # this op, committed under profiles/ (PMC cannot be collected from
         # here).  The file names the kernel sources it was taken on: a ratio from other kernels is
         # refused, not silently reused.
         traffic, src = None, "no profiles/*ssd_scan_traffic.json"
@@ -296,7 +296,7 @@ class OpTimers:
                 "avg_launch_us": round(ms * 1e3 / len(r), 1)}
 
     def mixer_trio_roofline(self, cfg):
-        """conv + scan + gated norm of the Mamba layers as ONE operator against SURVEY 8d's fused lower bound: read
+        """conv + scan + gated norm of the Mamba layers as ONE operator against the fused lower bound: read
         xBC + dt + gate, write the normed y (65 792 B per token and layer at Nano dims).  Work that moves between the
         three kernels (C.B^T into the conv, the carried-in correction into the norm, ...) stays inside this entry."""
         ms = sum(self._ms(k)[0] for k in ("conv", "scan", "gated_norm"))

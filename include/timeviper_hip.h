@@ -5,7 +5,7 @@
  * The reference (xiaomi-research/timeviper) is pure Python; its accelerated
  * operators are calls into un-vendored wheels (mamba_ssm 2.2.5, causal_conv1d
  * 1.5.2, flash_attn 2.8.0.post2, timm).  Each entry point below replaces one of
- * those call sites.  A maintainer binds them with ctypes (see INTEGRATION.md);
+ * those call sites.  A maintainer binds them with ctypes;
  * `timeviper_amd/kernels.py` is exactly that binding, exposing the reference's
  * Python operator names.
  *
@@ -212,7 +212,7 @@ int tv_ssd_scan_cb_fwd(const void* x, const void* dt, const void* A,
                        float dt_max, int group_map, void* workspace,
                        size_t workspace_bytes, void* stream);
 
-/* Carried-in state correction ("sequence sharding"; the Y_off term of
+/* Carried-in state correction (sequence sharding; the Y_off term of
  * modeling_nano.py:833-836 with the decay taken from the range start): a shard — another GPU's
  * tokens, or a later segment of one GPU's sequence — is scanned from a ZERO state by
  * tv_ssd_scan_fwd; once the state entering it is known its outputs are completed in place,
@@ -249,7 +249,7 @@ int tv_ssd_state_correction(void* y, const void* dt, const void* A, const void* 
  * 8 = the generic path in chunk-parallel form (csrc/ssd_chunked.hip: any dtype, d_state <= 64, head_dim <= 128, 65 ..
  *     4 096 tokens; fp32 arithmetic, needs the workspace).
  * 3 / 4 / 6 fall back (6 -> 4 -> 3) where the shape does not fit and fail with TV_ERR_UNSUPPORTED where none does.
- * 2, 5 and 7 named kernels that measured slower and were removed (docs/history.md); they select 3, 4 and 6. */
+ * 2, 5 and 7 named kernels that measured slower and were removed; they select 3, 4 and 6. */
 void tv_ssd_scan_set_impl(int impl);
 /* kernel family (same numbers) the most recent scan call of this process ran on; 0 before the first call */
 int tv_ssd_scan_last_impl(void);
@@ -281,7 +281,7 @@ int tv_selective_state_update_rows(void* state, const void* x, const void* dt,
                                    int dt_softplus, void* stream);
 
 /* ------------------------------------------------------------------------
- * ViT linears with fused epilogues (SURVEY 8f-4): C = epilogue(A . W^T), A (M,K), W (N,K) =
+ * ViT linears with fused epilogues: C = epilogue(A . W^T), A (M,K), W (N,K) =
  * nn.Linear.weight as stored, C (M,N), all bf16 row-major with element row strides lda / ldw / ldc.
  *   epilogue 0  C = acc + bias
  *            1  C = gelu(bf16(acc + bias)), exact (erf) GELU — timm Mlp fc1 + act
@@ -336,19 +336,18 @@ int tv_flash_attn_fwd(const void* q, const void* k, const void* v, void* o,
 /* Kernel variant for many short non-causal sequences of head_dim 65..80 (the SigLIP ViT frames; testing /
  * benchmarking, process-global): 0 = auto — bf16, >= 193 keys: the kernel with the key-tile loop as generated instruction
  * streams (csrc/attention_vit.hpp: one wave per SIMD, 64 query rows a wave, the softmax of tile i beside P.V of tile i - 1
- * and Q.K^T of tile i + 1, a lazy running maximum; round 6), otherwise the compiled streaming kernel (8 waves x 32 query
+ * and Q.K^T of tile i + 1, a lazy running maximum), otherwise the compiled streaming kernel (8 waves x 32 query
  * rows, two waves per SIMD); 4 = the same choice as 0; 5 = always the compiled streaming kernel (P's row sums out of the
  * P.V MFMAs through a ones column in the V ring); 3 = the compiled kernel with the row sums on the vector pipe (`l` summed
  * in fp32 before P is rounded) — 3 and 5 for A/B runs and tests.  The generated kernel's results equal the compiled one's
  * within the bf16 rounding of P (not bit for bit: P is rounded relative to another maximum).  (1 / 2 named two
- * measured-slower kernels removed in round 6: docs/history.md; the values are accepted and mean 0.)  Initial value: env
+ * measured-slower kernels, since removed; the values are accepted and mean 0.)  Initial value: env
  * TV_FA_W64. */
 void tv_flash_attn_set_variant(int variant);
 
 /* The same operator with the QK^T and PV products on the FP8 matrix path of CDNA4
- * (v_mfma_f32_32x32x64_f8f6f4, OCP e4m3 operands, fp32 accumulation, fp32 softmax): BASELINE
- * config 5 ("fp8 MFMA attention path"; call sites modeling_qwen2.py:196-244,
- * modeling_nano.py:1198-1209).  The reference's arithmetic is bf16, so this variant is opt-in and
+ * (v_mfma_f32_32x32x64_f8f6f4, OCP e4m3 operands, fp32 accumulation, fp32 softmax)
+ * (call sites modeling_qwen2.py:196-244, modeling_nano.py:1198-1209).  The reference's arithmetic is bf16, so this variant is opt-in and
  * judged by tolerance: q, k, v are quantised per (batch, head) to max |x| = 440, P per row to
  * 2^8 p; inputs, output and lse keep the layout, dtype and meaning of tv_flash_attn_fwd.
  * headdim <= 128 (multiple of 8).  workspace: tv_flash_attn_fp8_workspace_bytes() bytes,
@@ -426,7 +425,7 @@ int tv_attn_rank_scores(const void* q, const void* k, void* scores,
                         int64_t k_stride_l, int64_t k_stride_h,
                         int vis_start, int n_vis, float scale, int dtype,
                         void* workspace, size_t workspace_bytes, void* stream);
-/* The two halves of tv_attn_rank_scores for a sequence-sharded caller (SURVEY 8e-3): every rank
+/* The two halves of tv_attn_rank_scores for a sequence-sharded caller: every rank
  * computes the logits of ITS keys, logits (n_keys, Hq) fp32 key-major — per-shard pieces
  * concatenate along dim 0 — with the reference's roundings (q.K^T and the 1/sqrt(d) scaling
  * rounded to `dtype`, modeling_nano.py:1923-1927); after an all-gather every rank runs the
@@ -452,7 +451,7 @@ int tv_gather_rows(const void* src, const int64_t* index, void* dst,
                    int64_t dst_stride, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------
- * Qwen2 backbone ("next" row).
+ * Qwen2 backbone.
  * tv_rope_fwd: rotary embedding in place on x (rows, heads, headdim) with element
  *   strides (x_stride_l, x_stride_h); cos / sin (rows, headdim) contiguous in x's
  *   dtype (the tables Qwen2RotaryEmbedding returns, modeling_qwen2.py:362-385):

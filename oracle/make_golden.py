@@ -2,9 +2,8 @@
 
     python oracle/make_golden.py            # writes tests/golden/*.npz
 
-/root/reference (xiaomi-research/timeviper) is imported with the stub recipe of
-SURVEY.md Appendix B: the third-party wheels it needs (mamba_ssm, timm,
-flash_attn, causal_conv1d) are absent here, so `is_fast_path_available` is False
+/root/reference (xiaomi-research/timeviper) is imported with stubs: the
+third-party wheels it needs (mamba_ssm, timm, flash_attn, causal_conv1d) are absent here, so `is_fast_path_available` is False
 and every module runs the reference's own pure-PyTorch path (`torch_forward`,
 SDPA).  The only stand-in arithmetic is mamba_ssm's `rmsnorm_fn` (gated RMSNorm),
 which the reference does not vendor: that operator stays "parity unpinned".
@@ -192,7 +191,7 @@ def main():
         cfg = tiny_config(nano, use_pdrop=pd is not None, pdrop_type=pd, merge_module=merge)
         model = nano.NemotronHForCausalLM(cfg).eval()
         randomize(model, 4)
-        model.config._attn_implementation = "flash_attention_2"  # mask-free path (SURVEY §8c)
+        model.config._attn_implementation = "flash_attention_2"  # mask-free path
         n_vis, t_before, t_after = 40, 5, 9
         Ltot = t_before + n_vis + t_after
         emb = torch.randn(1, Ltot, cfg.hidden_size)
@@ -435,7 +434,7 @@ def make_multi_projector_golden():
     """G13: the two-encoder projectors of the reference (projector/tome.py:180-231,
     projector/mlp.py:37-68) on dict inputs keyed by backbone id: an image encoder (frame-wise ToMe)
     beside a 4-frame-tube video encoder (local_num_frames=4) — the reshape + token interleave of
-    BASELINE config 4 — and the unequal-token-count case (concatenation)."""
+    the two-encoder model — and the unequal-token-count case (concatenation)."""
     import_reference()
     tome = importlib.import_module("timeviper.model.projector.tome")
     mlp = importlib.import_module("timeviper.model.projector.mlp")
@@ -482,7 +481,7 @@ def make_realshape_golden():
                           ssm_state_size=128, mamba_num_heads=8, mamba_n_groups=G, mamba_head_dim=80, mamba_chunk_size=64)
         model = nano.NemotronHForCausalLM(cfg).eval()
         randomize(model, 21 + G)
-        model.config._attn_implementation = "flash_attention_2"   # mask-free path, SDPA modules stay (SURVEY 8c)
+        model.config._attn_implementation = "flash_attention_2"   # mask-free path, SDPA modules stay
         emb = torch.randn(1, L + ndec, cfg.hidden_size)
         n = L if G == 2 else L + ndec
         out = model(inputs_embeds=emb[:, :n])

@@ -187,7 +187,7 @@ def attention_ref(q, k, v, causal, scale=None):
 
 
 def fp8_quantise_ref(x, qmax: float = 440.0):
-    """What the fp8 attention variant (BASELINE config 5; tv_flash_attn_fp8_fwd) does to q, k and
+    """What the fp8 attention variant (tv_flash_attn_fp8_fwd) does to q, k and
     v before the MFMAs: one scale per (batch, head) so that max |x| -> qmax, rounding to OCP
     e4m3 (torch.float8_e4m3fn, round to nearest even), and the matching dequantisation.
     x (B, L, H, D) -> fp32 tensor of the values the kernel multiplies.  The reference has no fp8

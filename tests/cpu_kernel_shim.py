@@ -45,7 +45,7 @@ def _scan(x, dt, A, B, C, chunk_size=None, D=None, z=None, dt_bias=None, initial
 
 def _state_corr(y, dt, A, C, state_in, dt_bias=None, dt_softplus=False, dt_limit=(0.0, float("inf")),
                 group_map="block"):
-    """y_t += exp(cs_t) C_t . S_in (SURVEY Appendix A), from the definition"""
+    """y_t += exp(cs_t) C_t . S_in, from the definition"""
     Bsz, L, H, P = y.shape
     G = C.shape[2]
     d = dt.float() + (0.0 if dt_bias is None else dt_bias.float())

@@ -1,4 +1,4 @@
-"""FP8 (e4m3) MFMA attention variant — BASELINE config 5, `tv_flash_attn_fp8_fwd`.
+"""FP8 (e4m3) MFMA attention variant, `tv_flash_attn_fp8_fwd`.
 
 The reference's attention arithmetic is bf16, so this opt-in variant is judged by stated tolerances:
   (a) against the oracle attention evaluated ON THE QUANTISED INPUTS (oracle.ops.fp8_quantise_ref:

@@ -6,7 +6,7 @@ Several kernels issue global loads from inline asm that the compiler does not tr
 `s_waitcnt vmcnt(N)` (ssdk::gload16_async for the Q fragments of the attention kernels; the C.B^T and dt loads of the
 head-per-wave scan).  That is only sound while the compiler never saves or copies the destination registers between the
 load and the wait — i.e. while the kernel SPILLS NOTHING: a spilled register with a load in flight is stored before its
-data arrives and reloaded stale (this happened in round 3's spilling 'complete' scan kernel, since removed).
+data arrives and reloaded stale (this happened in a spilling scan kernel, since removed).
 So every kernel that uses the idiom must have zero scratch; a compiler upgrade or a source edit that introduces a spill
 fails here instead of producing silently wrong numbers on the GPU."""
 import re

@@ -1,4 +1,4 @@
-"""BASELINE config 5 at its named sizes: "TimeViper-Qwen2.5 backbone, DINOv2+InternVideo2 dual encoder,
+"""The Qwen2.5 model at full size: "TimeViper-Qwen2.5 backbone, DINOv2+InternVideo2 dual encoder,
 4096 frames, fp8 MFMA attention path" = 4 096 frames x 32 tokens + 100 text tokens = 131 172 tokens of a
 28 q / 4 kv x 128 causal RoPE attention, and a 4 096-frame dual-encoder vision path.
 

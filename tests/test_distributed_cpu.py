@@ -150,7 +150,7 @@ def worker(rank, world, port, merge, T, q, family="nano", rebalance=None):
     ("CrossAttention", 2, 5, "nano", 1.0), ("CrossAttention", 4, 9, "nano", 1.0), ("CrossAttention", 4, 9, "qwen2", 1.0)])
 def test_sequence_parallel_matches_single_process(merge, world, T, family, rebalance):
     """world 8 = the node size the driver scales to: eight ranks, unequal frame ranges; qwen2 = the
-    decoder-only family of BASELINE config 5 (every layer gathers rotated K and V)"""
+    decoder-only family (every layer gathers rotated K and V)"""
     ctx = mp.get_context("spawn")
     q = ctx.Queue()
     port = free_port()

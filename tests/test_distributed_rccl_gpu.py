@@ -5,7 +5,7 @@ exercises: `init_process_group(device_id=...)`, `all_gather_into_tensor(async_op
 stream overlapped with q_proj, `broadcast` of the ranking query, the `_attention` /
 `_run_layers_qwen2` data paths without any stand-in, and K.layer_norm's row_bias path under the
 sharded ViT.  Sharded logits and pdrop traces must equal the single-GPU forward
-(SURVEY.md §8e; reference semantics modeling_nano.py:1134-1220, :1929-1942)."""
+(reference semantics modeling_nano.py:1134-1220, :1929-1942)."""
 import os
 
 import pytest

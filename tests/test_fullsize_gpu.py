@@ -1,4 +1,4 @@
-"""BASELINE.json's full sizes (10 240 frames -> 163 940 tokens, Nemotron-Nano-9B-v2 dims) through
+"""Full sizes (10 240 frames -> 163 940 tokens, Nemotron-Nano-9B-v2 dims) through
 size-independent properties: the oracle cannot run here in seconds, so the HIP kernels are checked
 against themselves (shard chaining, exact power-of-two linearity, two independent kernels) and
 against the definition on sampled rows."""
@@ -57,7 +57,7 @@ def test_scan_full_length_properties(K):
     assert ((y2.float() - 2 * y.float()).abs() <= 2.0 ** -7 * (2 * y.float()).abs() + 1e-30).all()      # one bf16 step
     assert rel(fin2, fin * 2) < 1e-6
     del y2, fin2, ne
-    # (2) shard chaining (SURVEY 8e): two shards with the state handed over == one pass
+    # (2) shard chaining: two shards with the state handed over == one pass
     s = 81 * 1000 + 37                                   # not a multiple of the chunk length
     ya, fa, da = run(K, x[:, :s], dt[:, :s], A, Bm[:, :s], Cm[:, :s], D, bias)
     yb, fb, db = run(K, x[:, s:], dt[:, s:], A, Bm[:, s:], Cm[:, s:], D, bias, initial_states=fa)
@@ -214,7 +214,7 @@ def test_pdrop_token_ops_full_length(K):
     # The kernel rounds where the reference rounds (bf16 logits after the fp32-accumulated dot, bf16 after "/ sqrt(d)",
     # fp32 softmax -> bf16, fp32 head sum / H -> bf16): the bf16 SCORE VECTORS are equal except where an fp32
     # difference that no two implementations share — exp's last bit, the order of the 163 940-term fp32 sum — meets a
-    # bf16 rounding boundary (DESIGN.md section 4): a handful of scores, each exactly one bf16 step away
+    # bf16 rounding boundary: a handful of scores, each exactly one bf16 step away
     sb, pb = sc.bfloat16(), p.bfloat16()
     assert torch.equal(sb.float(), sc.float()) and torch.equal(pb.float(), p)        # both ARE bf16 values
     steps = (sb.view(torch.int16).int() - pb.view(torch.int16).int()).abs()

@@ -257,7 +257,7 @@ def test_evaluate_py_call_sequence_on_a_saved_checkpoint(tmp_path):
     with pytest.raises(RuntimeError):
         HybridTimeViperVLM.from_pretrained(tmp_path / "bad.pt", "m", vb2, llm2, arch_specifier="tome_mlp-16")
 
-    # attributes evaluate.py / vllm_infer.py read (SURVEY 8b)
+    # attributes evaluate.py / vllm_infer.py read
     assert model.llm_tokenizer is tokenizer and model.config is model.llm_backbone.llm.config
     assert model.arch_specifier == "tome_mlp-16" and model.llm_backbone.half_precision_dtype == torch.bfloat16
     T, tok = 4, model.default_token_id

@@ -296,7 +296,7 @@ def test_vlm_with_internvideo2_backbone_runs_and_matches_parts():
 
 
 def test_vlm_with_qwen2_backbone_vs_oracle_and_generate():
-    """BASELINE config 5's LM family behind the same VLM wiring: pixels -> ViT -> ToMe+MLP -> fusion ->
+    """The Qwen2.5 LM family behind the same VLM wiring: pixels -> ViT -> ToMe+MLP -> fusion ->
     Qwen2 with uniform pdrop + TransV (llm_registry.py:65-77 ids), against the pinned Qwen2 oracle on
     the same visual embeddings; greedy `generate` must continue from the prefill's argmax."""
     from oracle import qwen2 as oq
@@ -331,7 +331,7 @@ def test_vlm_with_qwen2_backbone_vs_oracle_and_generate():
 
 
 def test_vlm_dual_encoder_qwen2_matches_parts():
-    """BASELINE config 4's wiring at toy size: DINOv2-L (frame-wise) + InternVideo2 (4-frame tubes)
+    """The two-encoder wiring at toy size: DINOv2-L (frame-wise) + InternVideo2 (4-frame tubes)
     -> MultiToMe (16 + 16 tokens per frame, interleaved token-wise) -> fusion -> Qwen2 with pdrop +
     TransV.  The end-to-end forward must equal the same members run one by one, the interleave must
     be the reference's rule (projector/tome.py:214-231) and the LM stage must match the oracle."""
@@ -429,7 +429,7 @@ def test_qwen2_bf16_vs_oracle_well_conditioned(merge):
     assert out.logits.shape == ref.shape
     e16 = relerr(out.logits, ref)
     assert e16 < 3e-2
-    # The same forward with EVERY attention call on the e4m3 MFMA path (BASELINE config 5's switch, forced down to these
+    # The same forward with EVERY attention call on the e4m3 MFMA path (`fp8_attention`, forced down to these
     # short sequences): pinned against the same fp32 oracle.  e4m3 carries 3 mantissa bits on q, k, v and P, so the bound
     # is wider than bf16's — stated here: logits within 8e-2 relative L2 (2.7 x the bf16 bound), the arg-max token of
     # every position whose oracle margin exceeds the fp8 error the same as the oracle's.

@@ -153,7 +153,7 @@ def run_scan(K, x, dt, A, Bm, Cm, D, dt_bias, **kw):
 
 @pytest.mark.parametrize("impl", [1, 0, 6, 8])      # (3 / 4, the slice marches: test_ssd_scan_march_kernels)
 @pytest.mark.parametrize("dtype,B,L,H,P,G,N", [
-    (torch.float32, 1, 1024, 32, 64, 1, 16),
+    (torch.float32, 1, 1024, 32, 64, 1, 16),      # the fp32 scan of 32 heads x 64
     (torch.float32, 2, 77, 8, 8, 2, 16),
     (torch.float32, 1, 5, 4, 24, 4, 40),
     (torch.float32, 2, 1000, 6, 50, 3, 24),       # ragged last chunk, head_dim not a multiple of 4, 16 chunks
@@ -241,7 +241,7 @@ def test_ssd_scan_nano_geometry_vs_oracle(K):
 
 @pytest.mark.parametrize("dtype,H,P,G,N", [(torch.float32, 8, 16, 2, 16), (torch.bfloat16, 16, 80, 8, 128)])
 def test_ssd_scan_initial_state_and_sharding(K, dtype, H, P, G, N):
-    """shard chaining through initial_states == single pass (SURVEY §8e)."""
+    """shard chaining through initial_states == single pass."""
     L, s = 333, 140
     ins = scan_inputs(1, L, H, P, G, N, 11, dtype)
     x, dt, A, Bm, Cm, D, dt_bias = ins
@@ -301,7 +301,7 @@ def test_ssd_scan_march_kernels(K, B, L, H, P, G):
 ])
 def test_ssd_scan_decay_regimes(K, regime, a_lo, a_hi, dt_mean, dt_std):
     """Every step kind of the head-per-wave march (floating frame, re-base, reset, standard) and the hand-overs between
-    them, against the fp32 recurrence; impl 4 (round 2's slice march) takes the same inputs.  Heads of one work-group
+    them, against the fp32 recurrence; impl 4 (the slice march) takes the same inputs.  Heads of one work-group
     get different A, so the kinds mix inside a work-group; 2 600 tokens = 2 - 4 sequence segments with carried-in
     corrections."""
     B, L, H, P, G, N = 1, 2600, 16, 80, 2, 128
@@ -476,7 +476,7 @@ def test_selective_state_update(K, B, H, P, G, N):
 @pytest.mark.parametrize("L,H,P,G,slow", [(300, 8, 40, 2, False), (1000, 16, 80, 8, True), (64, 4, 64, 1, True),
                                           (5, 8, 80, 4, False), (2000, 8, 80, 8, False)])
 def test_ssd_state_correction_completes_a_zero_state_scan(K, L, H, P, G, slow):
-    """y(scan from S_in) = y(scan from 0) + exp(cs_t) C_t . S_in (SURVEY Appendix A): the in-place
+    """y(scan from S_in) = y(scan from 0) + exp(cs_t) C_t . S_in: the in-place
     correction on top of the zero-state scan against the oracle recurrence started from S_in.
     `slow`: heads that barely decay (the term stays alive over the whole range); otherwise most heads
     forget within a few chunks and the kernel's early exit is what runs."""
@@ -903,7 +903,7 @@ def test_uniform_keep_indices_bit_exact(K):
         got = K.uniform_keep_indices(n, keep).cpu()
         assert torch.equal(got, R.uniform_keep_indices_ref(n, keep)), (n, keep)
         assert torch.equal(got, torch.linspace(0, n - 1, keep, dtype=torch.long)), (n, keep)
-    # BASELINE full sizes, with the vision offset
+    # full sizes, with the vision offset
     for n, keep in [(163840, 131072), (160000, 128000), (131072, 98304), (32768, 26214)]:
         got = K.uniform_keep_indices(n, keep, offset=20).cpu()
         assert torch.equal(got, torch.linspace(0, n - 1, keep, dtype=torch.long) + 20)

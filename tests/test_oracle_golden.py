@@ -71,7 +71,7 @@ def test_group_map_block_differs_from_tile_when_grouped():
 
 
 def test_scan_initial_state_chaining():
-    """two shards chained through (final, total_decay) == one pass (SURVEY Appendix A)."""
+    """two shards chained through (final, total_decay) == one pass."""
     g = load_golden("mixer_g1")
     sd = golden_state_dict(g)
     A = -torch.exp(sd["A_log"])

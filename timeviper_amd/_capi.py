@@ -1,6 +1,6 @@
 """ctypes binding of libtimeviper_hip.so — the C ABI declared in include/timeviper_hip.h.
 
-This is the stub a reference maintainer would add (INTEGRATION.md): plain pointers
+This is the stub a reference maintainer would add: plain pointers
 and sizes, no torch types cross the boundary.  There is NO fallback: if the
 library is missing, `lib()` raises, and every operator in `kernels.py` fails
 loudly rather than silently running eager PyTorch.

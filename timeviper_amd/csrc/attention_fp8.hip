@@ -1,7 +1,7 @@
-// A1 (BASELINE config 5): fused softmax attention forward with FP8 (OCP e4m3) MFMA operands.
+// A1: fused softmax attention forward with FP8 (OCP e4m3) MFMA operands.
 //
 // The reference's attention arithmetic is bf16 (flash-attn / SDPA: modeling_qwen2.py:196-244,
-// modeling_nano.py:1198-1209); BASELINE.json's fifth configuration asks for the QK^T / PV
+// modeling_nano.py:1198-1209); the Qwen2.5 model with two vision encoders can have its QK^T / PV
 // products on the fp8 matrix path of CDNA4, v_mfma_f32_32x32x64_f8f6f4 (K = 64 per instruction,
 // twice the bf16 rate).  This is that variant: opt-in, fp32 accumulation and fp32 softmax,
 // inputs and output stay bf16 at the boundary.

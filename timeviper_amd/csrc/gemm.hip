@@ -1,4 +1,4 @@
-// bf16 GEMM with fused epilogues for the ViT linears ("fused beyond patch-embed"):
+// bf16 GEMM with fused epilogues for the ViT linears:
 //
 //     C[M][N] = epilogue( A[M][K] . W[N][K]^T )          A, W, C bf16 row-major (W = nn.Linear.weight as stored)
 //

@@ -1,10 +1,10 @@
-// Persistent bf16 GEMM on 256 x 192 tiles whose finished tile LEAVES SLOWLY ("drips"): the ViT linears of SURVEY 8f-4 (timm
+// Persistent bf16 GEMM on 256 x 192 tiles whose finished tile LEAVES SLOWLY ("drips"): the ViT linears (timm
 // block via base_vision.py:146-170,274-278; InternVideo2 Attention / Mlp vit_scale_clean.py:188-320),
 //     C[M][N] = epilogue( A[M][K] . W[N][K]^T ),   epilogues of gemm.hip (bias / bias + exact GELU / C += ...).
 //
 // Why a third kernel.  (1) The ViT's widths are multiples of 192, not of 256: 1 152 = 6 x 192 (4.5 x 256: the output
 // projections burn 10 % of their MFMAs on a half-empty tile column, here and in the library's 256 x 256 macro-tile alike),
-// 3 456 = 18 x 192, 4 352 = 22.7 x 192.  (2) gemm_persist.hip measured where the rest goes:
+// 3 456 = 18 x 192, 4 352 = 22.7 x 192.  (2) gemm_persist.hip showed where the rest goes:
 // the K loop runs at 1.5 PFLOP/s, but a tile's 128 KB of C cost 2.8 us in the CU's memory pipeline in front of the
 // copies, whoever issues them and whoever waits, and the GELU is vector-pipe work in a burst — 20 % of the qkv launch,
 // 44 % of fc1.  Both can only be hidden by SPREADING them over the next tile's K loop, which needs the packed tile to

@@ -1,10 +1,10 @@
-// Persistent bf16 GEMM for the ViT linears (SURVEY 8f-4; timm block via base_vision.py:146-170,274-278, InternVideo2
+// Persistent bf16 GEMM for the ViT linears (timm block via base_vision.py:146-170,274-278, InternVideo2
 // Attention / Mlp vit_scale_clean.py:188-320):  C[M][N] = epilogue( A[M][K] . W[N][K]^T ) for the bias epilogues of gemm.hip
 // (EPI_BIAS: the qkv projection; EPI_BIAS_GELU: fc1 + exact GELU; EPI_BIAS_RELU2: the hybrid stack's up projection + squared ReLU).
 //
 // Why a second kernel.  The linears of a SigLIP block have K = 1 152: 18 K-tiles of 64.  With one work-group per output
 // tile every tile pays, outside its K loop, the pipeline fill, the conversion of 256 x 256 accumulators (with the
-// GELU: ~1 700 vector instructions a wave) and 128 KB of C stores: 24 - 32 % of a launch (DESIGN.md, K sweep).  Here a
+// GELU: ~1 700 vector instructions a wave) and 128 KB of C stores: 24 - 32 % of a launch (K from 768 to 4 352).  Here a
 // work-group stays on its CU and walks a list of tiles:
 //   * the copy pipeline (one half-tile per phase, six phases ahead, gemm.hip's schedule) never stops: the last two
 //     K-tiles of a tile already issue the first copies of the next one;

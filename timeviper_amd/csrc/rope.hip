@@ -1,4 +1,4 @@
-// Qwen2 ("next" row): rotary position embedding applied in place to the q
+// Qwen2: rotary position embedding applied in place to the q
 // and k projections, and the SwiGLU gate  silu(gate) * up.  Elementwise, HBM-bound.
 // Reference: apply_rotary_pos_emb / rotate_half (llm_repo/qwen2/modeling_qwen2.py:82-113,
 // called :211-214), Qwen2MLP.forward (:78-80).

@@ -1,5 +1,5 @@
 // S3 (generic path, chunk-parallel): the selective scan for shapes the MFMA marches do not take — any dtype, small d_state
-// (fp32, 32 heads x 64, d_state 16, L = 1 024) — in the CHUNKED form the reference's CPU path states
+// (fp32, 32 heads x 64, d_state 16, 1 024 tokens) — in the CHUNKED form the reference's CPU path states
 // (NemotronHMamba2Mixer.torch_forward, modeling_nano.py:775-851: chunk-local decays :792-806, diagonal blocks Y_diag
 // :808-818, per-chunk states :820-824, the recurrence over chunk states :826-832, off-diagonal Y_off :833-836) instead of
 // ssd_generic.hip's token recurrence: that kernel walks L dependent steps per head (1 024 x ~0.3 us = 331 us for 0.3 MB of

@@ -2,7 +2,7 @@
 //
 //   y_t += exp(cs_t) * C_t . S_in        cs_t = sum_{j <= t} dt_j A_h  (inclusive, from the range start)
 //
-// — SURVEY.md Appendix A's "sequence sharding" identity: a shard (another GPU's, or the second
+// — the identity behind sequence sharding: a shard (another GPU's, or the second
 // segment of one GPU's sequence) scans from a zero state, and once the state that enters it is
 // known the outputs are completed by this term.  It is the Y_off term of modeling_nano.py:833-836
 // with the chunk-local decay replaced by the decay from the range start.
@@ -35,7 +35,7 @@ constexpr int CSLOTS = 64;        // work-groups per (batch, head): a head that 
                                   // (measured with 8: the slowest heads set the launch time, 808 us in the 9B model)
 // The walk of a head ends where the factor 2^(cs_t log2 e) has fallen below 2^-32: the term is then < 2.5e-10 of
 // |C_t . S_in| — two orders of magnitude under the fp32 rounding of the sum it would be added to and seven
-// under a bf16 ulp of y; round 2 walked on to 2^-160 (exactly 0 in fp32), five times the distance.
+// under a bf16 ulp of y; walking on to 2^-160 (exactly 0 in fp32) is five times the distance.
 constexpr float C_UNDERFLOW = -32.f;
 
 struct CorrArgs {
@@ -156,8 +156,8 @@ __device__ __forceinline__ void correct_walk(const CorrArgs& a, const int h, con
 
   // One chunk per iteration; the C rows, the dt value and the prefix of the NEXT chunk of this work-group and the y
   // rows of the current one are requested before the current chunk's arithmetic, so an iteration waits for one
-  // round trip to memory instead of three in a row (C -> MFMA -> y read -> y write; round 2: 80 % of the
-  // wave-cycles of this kernel were parked).
+  // round trip to memory instead of three in a row (C -> MFMA -> y read -> y write, with which 80 % of
+  // the wave-cycles of this kernel were parked).
   constexpr int NY = (CQ * 2 * PT + 255) / 256;      // y pieces per thread (rows of at most 16 PT columns)
   auto fetch = [&](int c, bf16x8 (&cf)[4], bf16x8 (&yv)[NY], float& draw, float& p0) {
     const int t0 = c * CQ;
@@ -426,7 +426,7 @@ int tv_ssd_correct_all_launch(void* y, const void* dt, const void* A, const void
                                                                                       nseg, bh, per_head, nb_chain, a, npairs);
   if (nsegc > 0) {
     // walkers: one per CPW chunks of a (head, boundary)'s horizon (at most MAXW), listed by the prefix kernel, taken off the list by
-    // persistent work-groups (4 per CU).  TV_CORR_SLOTS = n (dev tool): the round-3 grid of n work-groups per (head, boundary)
+    // persistent work-groups (4 per CU).  TV_CORR_SLOTS = n (dev tool): a grid of n work-groups per (head, boundary)
     // instead (whole scan at 163 940 / 32 868 tokens, bench-like dt, on that grid: 1: 2 560 / 754 us, 4: 2 454 / 694, 6: 2 458 / 681,
     // 8: 2 499 / 699, 16: 2 613 / 785, 32: 2 827 / 961).
     int slots = 0;

@@ -1,6 +1,6 @@
 // S3 (generic path): Mamba-2 selective scan as the exact fp32 token recurrence
 //   S_t = exp(dt_t A_h) S_{t-1} + dt_t x_t (x) B_t ;  y_t = S_t . C_t + D_h x_t
-// for any dtype / head_dim / d_state (fp32, N=16).  One
+// for any dtype / head_dim / d_state (fp32, d_state 16, for one).  One
 // workgroup owns (batch, head, 16 columns of P); a thread owns one column and
 // every 16th state index n, keeps its state slice in registers for the whole
 // sequence, and the 16 n-lanes of a column reduce y with DPP shuffles.  Token
@@ -172,9 +172,9 @@ __global__ void state_update_kernel(float* __restrict__ state, const T* __restri
 
 // Decode step for d_state = 4 LPR (16 .. 256): LPR lanes share a state row (16 bytes = 4 fp32 each), a wave covers
 // 64 / LPR rows per load — coalesced 512-byte rows instead of one thread walking its row with 4-byte loads at a 512-byte
-// lane stride (36.7 us for the 2 x 5.2 MB of a Nano layer, round 4).  The launch is a latency chain, not a stream (a Nano
+// lane stride (36.7 us for the 2 x 5.2 MB of a Nano layer).  The launch is a latency chain, not a stream (a Nano
 // layer is 10 240 rows = 5.2 MB, 20 KB a CU; an empty launch of this grid inside the decode graph takes 1.85 us):
-// round 6 keeps ONE state row per lane group in flight per wave (5 120 waves; two and four rows a wave measured 4.7 and
+// it keeps ONE state row per lane group in flight per wave (5 120 waves; two and four rows a wave measured 4.7 and
 // 5.6 us against 4.3), requests every scalar of the row (dt, dt_bias, A, D, x) and its B / C pieces in front of the state,
 // reads and writes the state non-temporally (nothing re-reads it before the next token, 16.6 GB of weights later) and sums
 // over d_state on DPP (row_shr inside a 16-lane row, row_bcast across rows: the group's last lane holds the sum) instead

@@ -25,7 +25,7 @@
 //     serves the state update and Ydiag alike.  Every factor formed lies within 2^(+-2 RMAX); when E + cs_Q
 //     would leave [-RMAX, RMAX] the frame is re-based (X' *= 2^(E - RMAX), E = RMAX: one pass over the state,
 //     every ~120 log2 units of decay), and a single chunk that decays by more than 2^(2 RMAX) (dt |A| > 1.3 per
-//     token) runs round 2's standard step: true mask 2^(cs_t - cs_s) dt_s, X' *= 2^(E + cs_Q) mid-step, E = 0 —
+//     token) runs a standard step: true mask 2^(cs_t - cs_s) dt_s, X' *= 2^(E + cs_Q) mid-step, E = 0 —
 //     only factors 2^(a - b), a >= b, like the reference's segment_sum form (modeling_nano.py:159-186);
 //   * D x is added in fp32 from x in the accumulator layout.
 // x reaches the MFMA operand layout through a wave-private LDS tile (register-staged: loaded one chunk
@@ -78,9 +78,9 @@ int tv_ssd_correct_all_launch(void* y, const void* dt, const void* A, const void
 #define TV_HEAD_RESET 1
 #endif
 // Standard steps (a chunk that decays by more than 2^(2 RMAX)) are taken by the one kernel itself, as three side blocks of
-// the one step body (scaled accumulators, per-head mask built into the C.B^T registers, raw x fragments).  Round 3's first
+// the one step body (scaled accumulators, per-head mask built into the C.B^T registers, raw x fragments).  Another
 // scheme — a flag per work-group + a second, complete kernel, or a device-side check that sent such calls to the slice
-// march — was measured (7.5 ms / 2.92 ms against 2.50 ms at 164 k tokens) and removed in round 4.
+// march — was measured (7.5 ms / 2.92 ms against 2.50 ms at 164 k tokens) and is gone.
 // TV_HEAD_UNTRACKED: 1 = the C.B^T / dt loads of the 4-wave fast kernels are inline asm with counted waits (needs a
 // kernel without scratch), 0 = ordinary loads
 #ifndef TV_HEAD_UNTRACKED

@@ -59,8 +59,8 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
 // d_state, 2 .. 64 chunks) — what automatic selection takes where no march applies.
 // Automatic selection has three more kernels, by its own rules and not to be forced, each of the family whose shapes it takes: 9 column slices (ssd_cols.hip) and
 // 10 heads in segments (ssd_par.hip), both of family 6, 11 the matrix cores' form of 8 (ssd_f32.hip).  Forced, 6 is the march and 8 is ssd_chunked.hip.
-// Removed, docs/history.md: 2 (round 1's chunk march; the number now means 3), 5 (round 3's 12-wave whole-head layout; now
-// means 4), 7 (round 4's two-waves-per-SIMD head march; now means 6).
+// Removed as the slower ones: 2 (a chunk march; the number now means 3), 5 (a 12-wave whole-head layout; now
+// means 4), 7 (a head march with two waves a SIMD; now means 6).
 // process-wide override for tests / dev tools; atomic so that concurrent callers never race on it
 static std::atomic<int> g_ssd_impl{0};
 static const int kAutoImpl = 6;   // head-per-wave march; falls back to 4, 3, the generic path

@@ -1,8 +1,8 @@
 // S3 (fast path, v2): Mamba-2 SSD selective scan as a "slice march" on CDNA4.
 //
 // A single pass over HBM (x, dt, B, C read once, y written once, the running state never leaves the
-// chip), organised around what bounded round 1's chunk march (state published to LDS, a barrier and a
-// re-read every chunk; removed in round 6, docs/history.md): LDS operand traffic and that round trip.
+// chip), organised around what bounds a chunk march that publishes its state to LDS (a barrier and a
+// re-read every chunk): LDS operand traffic and that round trip.
 //
 //   * A workgroup = (batch, head, <=48-column slice of head_dim), 12 waves, one barrier per
 //     64-token chunk.
@@ -38,18 +38,18 @@ int tv_ssd_correct_launch(void* y, const void* dt, const void* A, const void* Cm
                           hipStream_t st);
 
 // TV_BSCALE (wide layouts): 1 = the B/C waves scale the B tile in place (B~ = w_t B) and the slice-waves run the
-// state update on raw x fragments; 0 = the slice-waves form x~ = w_t x on their own fragments (round 2)
+// state update on raw x fragments; 0 = the slice-waves form x~ = w_t x on their own fragments
 #ifndef TV_BSCALE
 #define TV_BSCALE 0
 #endif
 // TV_YDIRECT (wide layouts): 1 = the slice-waves store y from their registers (no y tiles in LDS: room for a B/C ring
-// of 3); 0 = y tiles in LDS, stored by the B/C waves, B/C ring of 2 (round 2)
+// of 3); 0 = y tiles in LDS, stored by the B/C waves, B/C ring of 2
 #ifndef TV_YDIRECT
 #define TV_YDIRECT 0
 #endif
 // TV_YDIAG_FIRST (wide layouts): 1 = a step OPENS with Ydiag + D x (M and the raw x fragments are the first reads after the
 // barrier; their twelve MFMAs run while the C / B fragments of quarter 0 arrive) and ends with y = e^{cs_t} Yoff + that,
-// vector work only; 0 = Ydiag accumulates onto the scaled Yoff at the end of the step (round 2)
+// vector work only; 0 = Ydiag accumulates onto the scaled Yoff at the end of the step
 #ifndef TV_YDIAG_FIRST
 #define TV_YDIAG_FIRST 0
 #endif
@@ -66,7 +66,7 @@ constexpr int SQ = 64;           // tokens per chunk
 constexpr int SN = 128;          // d_state
 constexpr int NV = 3;            // cs / ecs / dt / weight vector buffers
 // Two layouts of a work-group.
-//   narrow (slices of <= 48 columns, two work-groups per head at Nano dims; round 1): 12 waves, one
+//   narrow (slices of <= 48 columns, two work-groups per head at Nano dims): 12 waves, one
 //     16-column tile per slice-wave, B/C ring of 3 (prefetch distance 2), x issued 4 chunks ahead,
 //     x~ built by helper waves.
 //   wide (a whole head, <= 80 columns): 8 waves with up to 256 registers each; a slice-wave owns TWO
@@ -224,8 +224,7 @@ __device__ __forceinline__ int xad(int a, int k, int b) {
 //   narrow: 0-2 slices, 3 x/dt/y, 4-6 + 11 B/C (+ one x~ piece each), 7-8 mask, 9 prep, 10 x~ pieces —
 //     the two mask waves, the heaviest VALU helpers, sit on different SIMDs; SIMD 3 has no slice-wave;
 //   wide:   0-2 slices (two column tiles each), 3 x/dt copies + prep, 4-5 B/C copies + y stores, 6-7 mask.
-//   (round 3's 12-wave whole-head layout with one column tile per slice-wave, "impl 5", measured slower than this one and was
-//   removed in round 6: docs/history.md.)
+//   (A 12-wave whole-head layout with one column tile per slice-wave measured slower than this one.)
 template <int PW> struct Roles {
   static constexpr bool WIDE = PW > 48;
   static constexpr int NWAVES = WIDE ? 8 : 12;
@@ -417,7 +416,7 @@ __global__ __launch_bounds__((Roles<PW>::NWAVES * 64)) void ssd_slice_kernel(Sli
       }
     };
     // Wide layout: y leaves the wave straight from these registers — 8 bytes per lane and (tile, t-tile),
-    // NC * 4 global_store_dwordx2 per step, nobody waits for them (round 3; the y tiles in LDS, their
+    // NC * 4 global_store_dwordx2 per step, nobody waits for them (the y tiles in LDS, their
     // ds_write_b64 / ds_read_b128 round trip and the helper waves' stores are gone, and the 20 KiB they
     // took hold the third B/C ring slot).  The 32-byte pieces of a row that the five tiles write meet in L2.
     bf16_t* const ygs = a.y + (int64_t)b * a.ysb + (int64_t)t_first * a.ysl + (int64_t)h * a.P + p_base;

@@ -1,6 +1,6 @@
 """Dev tool (GPU box): a plain 16-byte-per-lane copy of 3.36 GB (the size of the scan's x at 163 840 tokens) at full occupancy —
 grid sizes x loads in flight per lane x default / non-temporal — against torch's copy_: the practical roof of a read + write stream
-on THIS box (MI355X_MICROARCH.md records 6.29 TB/s for a tuned float4 copy; bytes = read + written).
+on THIS box (a tuned float4 copy: 6.29 TB/s; bytes = read + written).
     python timeviper_amd/devtools/membench_copy.py"""
 import ctypes
 import subprocess

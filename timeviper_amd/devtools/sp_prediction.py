@@ -1,6 +1,6 @@
 """Dev tool: the per-rank critical path of the sequence-sharded 10 240-frame forward at N = 2 / 4 / 8 ranks, priced from
 single-GPU measurements and xGMI link rates, written as profiles/rNN_sp_prediction.json — a FALSIFIABLE artefact: the
-first SCALE run on a multi-GPU node can be judged against it component by component (DESIGN.md section 6).
+first SCALE run on a multi-GPU node can be judged against it component by component.
 
     python timeviper_amd/devtools/sp_prediction.py [--round 6] [--step-ms 8084] [--out profiles/r06_sp_prediction.json]
 
@@ -13,7 +13,7 @@ import json
 import math
 
 FRAMES, TOKENS = 10240, 163940
-SCAN_BYTES = 45312           # per token and layer
+SCAN_BYTES = 45312           # per token and layer (algorithmic)
 N_MAMBA, N_ATTN = 27, 4
 STATE_BYTES = 128 * 80 * 128 * 4 + 512
 LINK = 153e9                 # bytes/s per link and direction

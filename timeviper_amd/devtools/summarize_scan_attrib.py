@@ -32,7 +32,7 @@ for dbg, name in NAMES.items():
     f = per_launch(f"attrib_{dbg}_FET", "FETCH_SIZE")
     if f is None:
         continue
-    rd = f * 1024 * 2                      # KiB; x2: gfx950 counts 128-B requests at 64 B (MI355X_MICROARCH.md)
+    rd = f * 1024 * 2                      # KiB; x2: gfx950 counts 128-B requests at 64 B
     hit, req = per_launch(f"attrib_{dbg}_TCC", "TCC_HIT_sum"), per_launch(f"attrib_{dbg}_TCC", "TCC_REQ_sum")
     out["runs"][str(dbg)] = {"what": name, "hbm_read_bytes": rd, "l2_requests": req, "l2_hit_rate": (hit / req if req else None)}
     if dbg == 0:

@@ -1,8 +1,8 @@
-"""Sequence-sharded TimeViper forward over the GPUs of one node (SURVEY.md §8e).
+"""Sequence-sharded TimeViper forward over the GPUs of one node.
 
-The reference has no collective anywhere (multi-GPU is delegated to DeepSpeed / vLLM,
-SURVEY §2a); this is new design for the north star's "frame/token sequence shards across
-the 8 GPUs with RCCL all-gather of the SSM states over xGMI".  One process per GPU,
+The reference has no collective anywhere (multi-GPU is delegated to DeepSpeed / vLLM);
+this is new design: frame / token sequence shards across the GPUs of a node, with an RCCL
+all-gather of the SSM states over xGMI.  One process per GPU,
 `torch.distributed` backend "nccl" (= RCCL on ROCm); every rank holds the full weights.
 
   * ViT + ToMe + projector: frames are independent -> rank r encodes its contiguous frame
@@ -26,7 +26,7 @@ the 8 GPUs with RCCL all-gather of the SSM states over xGMI".  One process per G
     After a token-drop stage the shards can be moved back to an even split (`rebalance_rows`: ONE
     all_to_all_single of contiguous row ranges, order kept; option `rebalance` / env TV_SP_REBALANCE,
     off by default: uniform and synthetic "attn" stages leave the shards within a few percent of even;
-    the kept tokens of a real checkpoint may cluster, DESIGN.md section 6).
+    the kept tokens of a real checkpoint may cluster).
 Collectives per Mamba layer: two — the conv halo (needed BEFORE the conv, whose output feeds the scan)
 and ONE gather of [S_r | L_r] packed in a single fp32 buffer (after the scan); the dependency
 in_proj -> halo -> conv -> scan -> state leaves no way to merge the two.
@@ -99,8 +99,8 @@ def rebalance_rows(x: torch.Tensor, lens: List[int], group=None, target: Optiona
     """Move the shard boundaries of a row-sharded sequence without changing its order: rank r holds rows
     [sum(lens[:r]), sum(lens[:r+1])) in `x` (dim 0) and ends up with [sum(target[:r]), sum(target[:r+1]))
     (default: `balanced_lens`).  One all-to-all of row ranges — a rank only exchanges rows with the ranks whose new
-    range overlaps its old one (after an "attn" token-drop stage whose kept tokens cluster on a few ranks, §6 of
-    DESIGN.md); every split size is a host integer derived from `lens`, no size exchange.  Returns (x', target)."""
+    range overlaps its old one (after an "attn" token-drop stage whose kept tokens cluster on a few
+    ranks); every split size is a host integer derived from `lens`, no size exchange.  Returns (x', target)."""
     world = dist.get_world_size(group)
     rank = dist.get_rank(group)
     total = sum(lens)
@@ -183,7 +183,7 @@ def split_frames(n_frames: int, world: int, causal_skew: float = 0.0, align: int
     return out
 
 
-# effective rates behind `estimate_causal_skew` (measured on MI355X, DESIGN.md section 5): the whole
+# effective rates behind `estimate_causal_skew` (measured on MI355X): the whole
 # forward without the LLM attention sustains ~0.95 PFLOP/s of its linear-layer FLOPs, the causal
 # attention kernel 0.86 PFLOP/s
 _LINEAR_RATE, _ATTN_RATE = 0.95e15, 0.86e15
@@ -211,7 +211,7 @@ def estimate_causal_skew(vlm, tokens_per_frame: int) -> float:
     if flops_lin <= 0.0:
         return 0.0
     # TV_SP_RATES="<linear TFLOP/s>,<causal-attention TFLOP/s>": the two kernel rates of the GPU at hand (the module
-    # constants are this repo's MI355X measurements, DESIGN.md §5); TV_SP_CAUSAL_SKEW=<k> overrides the estimate
+    # constants are this repo's MI355X measurements); TV_SP_CAUSAL_SKEW=<k> overrides the estimate
     if os.environ.get("TV_SP_CAUSAL_SKEW"):
         return float(os.environ["TV_SP_CAUSAL_SKEW"])
     lin_rate, attn_rate = _LINEAR_RATE, _ATTN_RATE
@@ -353,7 +353,7 @@ class SequenceParallelTimeViper:
         d_all = both[:, nS:].view((self.world,) + tuple(dec.shape))
         if self.rank > 0 and L > 0:
             # the state entering this shard, then the carried-in term y_t += exp(cs_t) C_t . In_r added
-            # in place (SURVEY Appendix A) — not a second scan: the term dies out after each head's
+            # in place — not a second scan: the term dies out after each head's
             # decay horizon and the kernel stops there
             inc = chain_states(S_all, d_all, self.rank)
             dtl = {} if "dt_limit" not in kw else {"dt_limit": kw["dt_limit"]}

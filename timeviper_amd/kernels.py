@@ -1,7 +1,7 @@
 """Operator API of the TimeViper hot path, bound to the gfx950 kernels.
 
 Each function keeps the NAME and ARGUMENT MEANING of the third-party operator
-the reference calls (SURVEY.md §8b "inner boundary"), so `NemotronHMamba2Mixer`
+the reference calls (the boundary to the wheels it does not ship), so `NemotronHMamba2Mixer`
 and friends read like the reference's:
 
     causal_conv1d_fn / causal_conv1d_update      modeling_nano.py:619-624 / :495-501
@@ -467,8 +467,8 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size=None, D=None, z=None, d
 def ssd_state_correction(y, dt, A, C, state_in, dt_bias=None, dt_softplus=False,
                          dt_limit=(0.0, float("inf")), group_map="block"):
     """In place: y_t += exp(sum_{j<=t} dt_j A_h) C_t . state_in[h] — completes the outputs of a scan
-    that started from a zero state once the state entering it is known (sequence shards, SURVEY
-    Appendix A).  y (B,L,H,P), dt (B,L,H) raw, C (B,L,G,N), state_in (B,H,P,N) fp32.  Returns y."""
+    that started from a zero state once the state entering it is known (sequence
+    shards).  y (B,L,H,P), dt (B,L,H) raw, C (B,L,G,N), state_in (B,H,P,N) fp32.  Returns y."""
     _gpu(y, dt, A, C, state_in, dt_bias)
     Bsz, L, H, P = y.shape
     G, N = C.shape[2], C.shape[3]
@@ -559,7 +559,7 @@ _ATTN_FP8 = {"on": False, "min_keys": 4096, "min_queries": 64}
 
 class fp8_attention:
     """Context manager / switch: inside it `flash_attn_func` (and everything built on it) runs the
-    QK^T / PV products on the FP8 MFMA path (`tv_flash_attn_fp8_fwd`) — BASELINE config 5.  Off by
+    QK^T / PV products on the FP8 MFMA path (`tv_flash_attn_fp8_fwd`).  Off by
     default: the reference's attention arithmetic is bf16.  Key sequences shorter than `min_keys`
     stay on the bf16 kernel: the ViT towers (<= 1 025 keys per frame / tube; measured 2.3 ms fp8
     against 1.5 ms bf16 per 256 SigLIP frames — the quantisation pre-pass and head_dim 72 -> 128

@@ -50,7 +50,7 @@ def build_synthetic_timeviper(llm_config=None,
                               vision_config=None, llm_backbone_id: str = "nanov2-9b",
                               member_kwargs=None):
     """Random-init TimeViper (there are no checkpoints offline): weights N(0, 0.02),
-    A_log = log U[1,16], dt_bias = softplus^-1(U[1e-3,1e-1]), D = 1 (SURVEY §8d)."""
+    A_log = log U[1,16], dt_bias = softplus^-1(U[1e-3,1e-1]), D = 1."""
     torch.manual_seed(seed)
     with torch.device("meta"):
         vtype = get_vision_backbone_config(vision_backbone_id)["type"]

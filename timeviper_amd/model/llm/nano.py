@@ -1,11 +1,11 @@
 """Host-side mirror of the reference's NemotronH hybrid LM
 (`timeviper/model/llm/llm_repo/nano/{configuration_nano,modeling_nano}.py`): same
-class names, module tree, parameter names / shapes (state-dict compatible,
-SURVEY.md §8b) and forward() signatures — with every hot operator bound to the
+class names, module tree, parameter names / shapes (state-dict
+compatible) and forward() signatures — with every hot operator bound to the
 gfx950 kernels in `timeviper_amd.kernels` instead of mamba_ssm / causal_conv1d /
 flash_attn.  GEMMs stay on torch (hipBLASLt).  Inference (prefill + decode) only.
 
-What is deliberately different from the reference (SURVEY.md §3.2 notes):
+What is deliberately different from the reference:
   * no per-layer `torch.isnan(...).any()` host sync (:1690) — `check_nan=True`
     restores it;
   * `lm_head` is applied to the positions asked for by `logits_to_keep`
@@ -115,7 +115,7 @@ class NemotronHConfig:
 
     @classmethod
     def nemotron_nano_9b_v2(cls, **over):
-        """NVIDIA-Nemotron-Nano-9B-v2 dims (SURVEY.md Appendix C; public config.json)."""
+        """NVIDIA-Nemotron-Nano-9B-v2 dims (public config.json)."""
         kw = dict(vocab_size=131072, hidden_size=4480, intermediate_size=15680,
                   num_hidden_layers=56,
                   hybrid_override_pattern="M-M-M-MM-M-M-M*-M-M-M*-M-M-M-M*-M-M-M-M*-M-MM-M-M-M-M-M-",

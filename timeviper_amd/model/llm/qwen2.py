@@ -1,6 +1,5 @@
 """Qwen2 / Qwen2.5 backbone with pdrop + TransV (reference
-timeviper/model/llm/llm_repo/qwen2/modeling_qwen2.py:59-1197, configuration_qwen2.py) —
-SURVEY §8f "next" row, needed by BASELINE config 5.
+timeviper/model/llm/llm_repo/qwen2/modeling_qwen2.py:59-1197, configuration_qwen2.py).
 
 Inference paths only (prefill and single-token decode, batch 1, no padding mask), same module
 tree / parameter names as the reference (`model.embed_tokens`, `model.layers.{i}.{self_attn.

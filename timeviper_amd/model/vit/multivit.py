@@ -1,4 +1,4 @@
-"""`MultiViTBackbone`: several vision encoders over the same frames (BASELINE config 4: DINOv2-L +
+"""`MultiViTBackbone`: several vision encoders over the same frames (DINOv2-L +
 InternVideo2-1B).
 
 The reference imports this class from `timeviper/model/vit/multivit_backbones.py`

@@ -26,7 +26,7 @@ from ... import kernels as K
 from ..plain_linear import plain_linear
 
 TIMM_VIT_CONFIGS = {
-    # public timm model definitions (not in the reference tree; SURVEY Appendix C)
+    # public timm model definitions (not in the reference tree)
     "vit_so400m_patch14_siglip_384": dict(img_size=384, patch_size=14, embed_dim=1152, depth=27,
                                           num_heads=16, mlp_hidden=4304, class_token=False,
                                           reg_tokens=0, pool="map"),
