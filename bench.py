@@ -245,7 +245,10 @@ class OpTimers:
         # refused, not silently reused.
         traffic, src = None, "no profiles/*ssd_scan_traffic.json"
         files = sorted((ROOT / "profiles").glob("*ssd_scan_traffic.json"))
-        if files:
+        kernel = getattr(self.K, "ssd_scan_last_kernel", lambda: 6)()
+        if kernel != 6:
+            src = "the passes are of the head-per-wave march, which this length does not run"
+        elif files:
             tf = json.loads(files[-1].read_text())
             if tf.get("scan_source_id") == scan_source_id():
                 ratio = tf["hbm_over_algorithmic"]
@@ -254,10 +257,12 @@ class OpTimers:
             else:
                 src = (f"profiles/{files[-1].name} was taken on other scan kernels (source id "
                        f"{tf.get('scan_source_id')}, tree {scan_source_id()}): re-run devtools/pmc_scan.sh")
-        return {"bound": "hbm", "kernel": "ssd_scan (tv_ssd_scan_cb_fwd: ssd_head_asm_kernel — head-per-wave march, the 64-token step one "
-                                          "generated, hand-scheduled instruction stream (csrc/ssd_head_step.inc) — x 8-16 sequence "
-                                          "segments (floating, reset and standard steps) + ssd_dt_transpose + ssd_chain_prefix + "
-                                          "ssd_correct_list kernels)",
+        return {"bound": "hbm", "kernel": {10: "ssd_scan (tv_ssd_scan_cb_fwd: ssd_par_kernel, a head per work-group in segments)",
+                                           9: "ssd_scan (tv_ssd_scan_cb_fwd: ssd_cols_kernel, column slices)"}.get(
+                                               kernel, "ssd_scan (tv_ssd_scan_cb_fwd: ssd_head_asm_kernel — head-per-wave march, the 64-token step one "
+                                                       "generated, hand-scheduled instruction stream (csrc/ssd_head_step.inc) — x 8-16 sequence "
+                                                       "segments (floating, reset and standard steps) + ssd_dt_transpose + ssd_chain_prefix + "
+                                                       "ssd_correct_list kernels)"),
                 "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "traffic_source": src, "launches": len(r),
                 "avg_launch_us": round(ms * 1e3 / len(r), 1), "bytes_per_token": bytes_per_token}
@@ -402,7 +407,7 @@ def cpu_baseline(cfg, frames_sample=256, vit_frames=16):
 def config1_scan(args):
     """one Mamba-2 selective scan, B=1 L=1024, 32 heads x 64, d_state 16, fp32 — the one configuration
     the reference's eager CPU path runs as it is.  Prints one JSON line: the HIP kernels' time (tv_ssd_scan_fwd picks the
-    generic path's chunk-parallel form for this dtype / d_state), the oracle's time on the host cores, and the largest
+    chunk-parallel form on the fp32 matrix instruction for this dtype / d_state), the oracle's time on the host cores, and the largest
     deviation of the HIP result from the oracle and of the oracle from the reference's golden fixture."""
     import numpy as np
     from timeviper_amd.build import ensure_built
@@ -436,7 +441,7 @@ def config1_scan(args):
     for _ in range(max(args.warmup, 1)):
         y, fin = fn2()
     torch.cuda.synchronize()
-    impl = K.ssd_scan_last_impl()
+    impl = K.ssd_scan_last_kernel()
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     steps = max(args.steps, 20)
     e0.record()
@@ -475,11 +480,11 @@ def config1_scan(args):
         "ms_per_step": round(us / 1e3, 4), "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "tv_ssd_scan_fwd (d_state 16 is not an MFMA shape: the generic path, chunk-parallel form — "
-                               "ssd_chunk_local_kernel + ssd_chunk_carry_kernel, csrc/ssd_chunked.hip), "
-                               f"tokens {L}, heads {H} x {P}, groups {G}, d_state {N}; scan implementation {impl}",
+                               "on the fp32 matrix instruction, ssd_f32_kernel twice, csrc/ssd_f32.hip), "
+                               f"tokens {L}, heads {H} x {P}, groups {G}, d_state {N}; scan kernel {impl}",
                    "timing": f"{steps} scans captured in one hipGraph and replayed; the eager Python loop takes "
                              f"{us_eager:.1f} us per scan (host-paced)"},
-        "roofline": {"bound": "hbm", "kernel": "ssd_chunk_local_kernel + ssd_chunk_carry_kernel" if impl == 8 else "ssd_generic_kernel",
+        "roofline": {"bound": "hbm", "kernel": {11: "ssd_f32_kernel (local states, outputs)", 8: "ssd_chunk_local_kernel + ssd_chunk_carry_kernel"}.get(impl, "ssd_generic_kernel"),
                      "achieved": round(bytes_alg / us / 1e3, 2),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(bytes_alg / us / 1e3 / HBM_PEAK_GBS, 5),
                      "traffic": None, "note": "0.3 MB per scan: a launch-latency-sized problem, not a bandwidth one"},

@@ -44,3 +44,12 @@ def test_bench_job_propagates_a_failing_rank():
     r = run(2, {"TV_BENCH_DRYRUN_FAIL_RANK": "1"})
     assert r.returncode != 0
     assert not [l for l in r.stdout.splitlines() if l.strip().startswith("{")], "a failed job must not print a result line"
+
+
+@pytest.mark.parametrize("where", ["sources", pytest.param("GPU", marks=pytest.mark.gpu)])
+def test_traffic_of_the_scan_is_at_hand_and_of_its_sources(where):
+    """the PMC passes that the bench line's `roofline.traffic` rests on are there, here and where the bench runs, and were taken on these scan kernels"""
+    sys.path.insert(0, str(ROOT))
+    import bench
+    files = sorted((ROOT / "profiles").glob("*ssd_scan_traffic.json"))
+    assert files and json.loads(files[-1].read_text())["scan_source_id"] == bench.scan_source_id()
