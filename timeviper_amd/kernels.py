@@ -895,10 +895,13 @@ def small_linear(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None, tile
 
 def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
     """The tile of tv_gemm_small_fwd for rows x n outputs (of either factor with `glu`) where it replaces a library call of a short forward, -1 where it does not.
-    Such a forward waits for the host, which a library call takes 19 us of and this one 8, so the product may take as long as the library's, not longer (us on the
-    device, library | here): 64 x 64 where they are one round of the compute units or less (1 152 x 1 152, 729 rows: 9.5 | 7.5, 1 458: 10.7 | 9.6; 5 120 x 2 048, 100: 10.8 | 10.5; 1
-    152 x 4 352, 729: 18.7 | 19.4), 64 x 128 up to 1.3 rounds (3 456 x 1 152, 729: 15.0 | 13.8), 128 x 128 up to two (1 458: 17.1 | 21; with the GELU 20.7 + 4 | 22; 2 187:
-    26 | 24), and not contractions of more than 2 048 columns on more than a few hundred rows (1 152 x 4 352, 2 187 rows: 31 | 43)."""
+    Such a forward waits for the host, which a library call takes 19 us of and this one 8: some sizes take longer on the device than the library's, which shows where
+    the device is busy with other work or the calls are captured.  64 x 64 up to 1.2 rounds of the compute units (two of them run on one), up to two in contractions of more
+    than 2 048 columns (at most 4 608, at most 1 536 rows), else 64 x 128 up to 1.3, 128 x 128 up to two.
+    us on the device, library | here: 64 x 64: 1 152 x 1 152, 729 rows: 9.5 | 7.5; 5 120 x 2 048, 100: 10.8 | 10.5; 1 152 x 4 352, 196: 11.9 | 18.3, 729: 18.7 | 19.4, 1 024: 22 | 28;
+    64 x 128: 3 456 x 1 152, 588: 13.0 | 14.4, 729: 15.0 | 13.8; 128 x 128: 1 024: 14.4 | 16.1, 1 458: 17.8 | 22.8, with the GELU, 4 352 columns, 1 024: 21.6 | 24.5, 1 458:
+    20.7 + 4 | 22; 1 152 x 4 352, 2 187 rows, left: 31 | 43.  SigLIP so400m, whole forwards | captured: 1 frame of 729: 4 055 -> 2 784 | 2 956 -> 2 631, 3: 4 065 -> 3 883 |
+    3 940 -> 3 928, 1 of 256: 4 014 -> 2 750 | 2 262 -> 2 181, 4: 3 984 -> 3 194 | 2 838 -> 3 195, 8: 4 016 -> 3 887 | 3 724 -> 3 908."""
     if not 2 <= rows <= 2304 or n < 512 or k % 64 or (k > 2048 and (k > 4608 or rows > 1536)):
         return -1
     over = lambda tm, tn: -(-rows // tm) * -(-n * (2 if glu else 1) // tn)
