@@ -344,6 +344,9 @@ int tv_flash_attn_fwd(const void* q, const void* k, const void* v, void* o,
  * measured-slower kernels, since removed; the values are accepted and mean 0.)  Initial value: env
  * TV_FA_W64. */
 void tv_flash_attn_set_variant(int variant);
+/* Whether a grid of `pairs` (batch entry, query head) pairs without a window has two waves on each query row (128-row blocks, two key tiles a step) instead
+ * of one (256-row blocks); ViT frames and grids of one-tile sequences are outside this rule. */
+int tv_flash_attn_two_waves(int seqlen_q, int seqlen_k, int64_t pairs, int headdim, int causal);
 
 /* The same operator with the QK^T and PV products on the FP8 matrix path of CDNA4
  * (v_mfma_f32_32x32x64_f8f6f4, OCP e4m3 operands, fp32 accumulation, fp32 softmax)

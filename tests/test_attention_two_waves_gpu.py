@@ -30,6 +30,8 @@ def close(got, want, mag):
     (1, 4, 2, 128, 1, 1, True), (1, 4, 2, 128, 2, 63, True), (2, 4, 4, 128, 31, 64, True), (1, 8, 2, 128, 33, 65, True), (1, 4, 1, 128, 127, 128, True),
     (1, 4, 1, 128, 128, 129, False), (1, 2, 2, 128, 129, 129, True), (1, 2, 1, 128, 257, 191, True), (1, 2, 1, 128, 100, 20, True), (1, 3, 3, 72, 255, 193, False),
     (2, 3, 3, 64, 300, 300, True), (1, 2, 2, 96, 140, 1000, True), (1, 2, 2, 80, 64, 513, False), (70, 1, 1, 64, 100, 100, False), (1, 16, 4, 128, 1000, 1000, True),
+    # more than a round of 128-row blocks: where the longest ones' time is filled up, and where not
+    (1, 44, 11, 64, 1100, 1100, True), (50, 4, 1, 128, 129, 130, True), (32, 4, 2, 80, 257, 257, True), (20, 5, 1, 64, 400, 490, True),
     # more than a round of short sequences: one wave a row where the keys are one tile of 96
     (300, 2, 2, 128, 96, 96, False), (150, 4, 1, 128, 70, 65, False), (150, 4, 1, 128, 70, 64, False), (600, 1, 1, 80, 1, 1, True), (300, 2, 1, 64, 65, 65, True), (200, 3, 3, 72, 96, 96, False), (130, 4, 2, 96, 128, 96, True), (513, 1, 1, 64, 33, 20, True),
     (513, 1, 1, 64, 100, 97, True)])
@@ -49,7 +51,7 @@ def test_against_64_bits(B, H, G, D, Lq, Lk, causal, dtype):
 
 # windows that end inside a tile, kept keys, sequences in one launch; chunks behind a cache
 @pytest.mark.parametrize("counts,starts,window,keep", [([1, 64, 127], [0, 0, 0], 50, 0), ([128, 33], [70, 500], 100, 7), ([300], [0], 128, 64), ([257, 1], [0, 640], 191, 65),
-                                                       ([130], [400], 2 ** 31 - 1, 0)])
+                                                       ([130], [400], 2 ** 31 - 1, 0), ([1400] * 6, [0] * 6, 1024, 64), ([520] * 14, [0] * 14, 200, 1)])
 def test_windows(counts, starts, window, keep):
     from timeviper_amd import kernels as ops
     from timeviper_amd.model.llm.cache import SlotStateCache

@@ -60,3 +60,13 @@ def test_product_path_has_no_cpu_fallback():
     # and nothing under timeviper_amd/ imports the oracle
     for p in (ROOT / "timeviper_amd").rglob("*.py"):
         assert "oracle" not in p.read_text().replace("# oracle", ""), p
+
+
+@pytest.mark.parametrize("rows,keys,pairs,D,causal,two", [
+    (128, 5000, 400, 64, 0, 1), (700, 700, 40, 128, 1, 1), (729, 729, 40, 72, 0, 1), (129, 129, 128, 64, 1, 1),       # up to 128 rows; a round of 128-row blocks
+    (729, 729, 48, 72, 0, 0), (1400, 3000, 40, 128, 1, 0), (2000, 2000, 40, 128, 1, 0),             # more, every row against all keys; 256-row blocks beyond a round
+    (1000, 1000, 40, 128, 1, 1), (1400, 1400, 40, 128, 1, 1), (2000, 2000, 28, 96, 1, 1), (4096, 5120, 16, 128, 1, 1),  # triangles whose short blocks fill up the long ones' time
+    (129, 129, 200, 64, 1, 0), (200, 200, 200, 128, 1, 0), (300, 300, 100, 64, 1, 0), (256, 256, 129, 128, 1, 0), (256, 64, 200, 64, 1, 0)])     # ... and whose do not
+def test_two_waves_a_row_where_its_grid_ends_first(rows, keys, pairs, D, causal, two):
+    from timeviper_amd import _capi
+    assert _capi.lib().tv_flash_attn_two_waves(rows, keys, pairs, D, causal) == two

@@ -18,6 +18,7 @@
 // cross_attention.py:310-317 non-causal), flash_attn_varlen_qkvpacked_func
 // (flash_attention_class.py:59-66).
 #include "ssd_common.hpp"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -926,11 +927,44 @@ __global__ __launch_bounds__(512) void flash_fwd_stream_kernel(AttnArgs a) {
 
 std::atomic<int> g_fa_variant{[] { const char* v = getenv("TV_FA_W64"); return v ? atoi(v) : 0; }()};
 
+// When the last of a grid's work-groups ends, one of them a compute unit at a time, each starting where a unit is free first: runs of equal ones in grid order.  Its
+// unit of time is a quarter of a step of 128 keys by two waves a row, which a step of 96 by one wave takes as well; a block's start and end take 10.
+struct Dealt {
+  struct Run { int64_t end; int n; } runs[512];     // (every run is a compute unit or more: never more runs than those)
+  int size = 1;
+  int64_t last = 0;
+  Dealt() { runs[0] = {0, std::max(1, std::min(tv_cu_count(), 512))}; }
+  void add(int64_t cost, int64_t n) {
+    const auto later = [](const Run& a, const Run& b) { return a.end > b.end; };
+    while (n > 0) {
+      std::pop_heap(runs, runs + size, later);
+      Run& first = runs[size - 1];
+      const Run taken{first.end + cost, (int)std::min<int64_t>(first.n, n)};
+      n -= taken.n;
+      last = std::max(last, taken.end);
+      if ((first.n -= taken.n) == 0) first = taken;
+      else { std::push_heap(runs, runs + size, later); runs[size++] = taken; }
+      std::push_heap(runs, runs + size, later);
+    }
+  }
+};
+// Blocks of 256 rows are at most a round (their longest ends last): whether those of 128 rows, more than one, end before .94 of it, and before .99 at head dim 128, where a
+// step of one wave takes a little more than the estimate (16 heads, 4 096 rows against 5 120 keys: 159 | 145 us, estimated alike)
+bool dealt_out_pays(const Dealt& two, int64_t one, bool wide) { return two.last * 100 < one * (wide ? 99 : 94); }
+
 // Whether two waves share 32 query rows (KG 2): up to 128 rows (64 against 4 096 keys, 40 heads: 131 us with one wave a SIMD, 88; 128: 14.7, 11.7), while 128-row
-// blocks are one round of the compute units (40 heads x 700: 31.8 | 24.2), and twice as many where they grow from nothing, since the short ones share
-// (40 x 1 400: 51.7 | 46.7, 28 x 2 000: 66.4 | 58.3; 40 x 2 000, 320 blocks of 256: 70.4 | 84.7; 48 whole rows of 729, 288 of 128: 27.1 | 39.5).
-bool two_waves_a_row(int Lq, int64_t blocks256, int64_t blocks128, bool triangle) {
-  return Lq <= 128 || blocks128 <= tv_cu_count() || (triangle && blocks256 <= tv_cu_count());
+// blocks are one round of the compute units (40 heads x 700: 31.8 | 24.2), and for more of them where causal blocks grow from nothing and the short ones, dealt out last,
+// fill up the long ones' time (40 x 1 400: 51.7 | 46.7, 28 x 2 000: 66.4 | 58.3; not 40 x 2 000, 320 blocks of 256: 70.4 | 84.7; nor 48 whole rows of 729: 27.1 | 39.5).
+// The line is the estimate above: it takes .095 of the .097 (logarithms, in the mean over 450 triangles beyond a round, head dim 64) and .122 of the .123 (128) that the better
+// form of each would give.  Two waves on all of them were slower on the short and the many (us, one | two: head dim 64, 256 rows against 320, 224 pairs 18.3 | 24.6; 384 x 480, 93:
+// 18.1 | 24.8; 128: 256 x 320, 167: 24.7 | 30.7; 768 x 960, 81: 41.0 | 48.2).
+bool two_waves_a_row(int Lq, int Lk, int64_t pairs, bool causal, bool wide) {
+  const int cus = tv_cu_count(), rows = (Lq + 127) / 128;
+  if (Lq <= 128 || rows * pairs <= cus) return true;
+  if (!causal || Lk - Lq > Lq / 4 || (Lq + 255) / 256 * pairs > cus) return false;
+  Dealt two;
+  for (int q = rows; q > 0; --q) two.add(10 + 4 * ((std::max<int64_t>(0, std::min<int64_t>(Lk, q * 128ll + Lk - Lq)) + 127) / 128), pairs);
+  return dealt_out_pays(two, 10 + 4 * ((Lk + 95ll) / 96), wide);
 }
 // ... but not for more than a round of such short rows whose keys are one tile of 96: the second wave has nothing to do, or a masked step where one wave's tile has none.  Head
 // dims up to 64, and non-causal rows against 96 keys, against 65 and more at head dim 128 (16 heads, us, two waves | one, 320 and 16 384 pairs: 64 wide, causal,
@@ -951,7 +985,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   if (a.Lq <= 128 && all > tv_cu_count() && one_tile(KS, a.Lk, 32 * KT, a.causal) && B <= 65535 && a.Hq <= 65535) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
-  } else if (!frames && two_waves_a_row(a.Lq, nqb * all, (a.Lq + 127) / 128 * all, a.causal && a.Lk - a.Lq <= a.Lq / 4)) {
+  } else if (!frames && two_waves_a_row(a.Lq, a.Lk, all, a.causal, KS > 6)) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS2);
     if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 8, 2, false, 2><<<dim3((unsigned)((a.Lq + 127) / 128 * all)), 512, FA_LDS2, st>>>(a, NoSeqs{});
   } else {
@@ -1006,10 +1040,10 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-// windowed form: bf16, 64-key tiles at head dim 128 (the bounds of the window do not fit beside 96 keys' fragments).  Blocks of 256 rows, or of 128 with two waves a
-// row: if no sequence is longer, while those are one round, and for more where the sequences start from nothing, the more the more of them there are (one
-// prompt, 16 heads, window 1 024: 1 200 rows 54 | 37 us, 2 560: 65 | 54, 3 200: 64 | 75; two, 3 000 together: 63 | 53, 3 500: 63 | 66; four, 3 000: 61 | 45, 4 000: 64 | 61;
-// six, 4 500: 65 | 68; 32 x 100 rows behind 1 000 keys 116 | 81).
+// windowed form: bf16, 64-key tiles at head dim 128 (the bounds of the window do not fit beside 96 keys' fragments; a step of 64 takes 3 of the estimate's units, the
+// rest of a block 13).  Blocks of 256 rows, or of 128 with two waves a row: if no sequence is longer, while those are one round, and for more where the sequences start
+// from nothing and the estimate of both grids says so (one prompt, 16 heads, window 1 024: 1 200 rows 54 | 37 us, 2 560: 65 | 54, 3 200: 64 | 75; four, 3 000 together:
+// 61 | 45; 32 x 100 rows behind 1 000 keys 116 | 81; but eight of 425, 16 heads 28 | 39, sixteen of 162, window 256 19 | 27).
 template <int KS, int DT>
 int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) {
   constexpr int KT = KS > 6 ? 2 : FA_KT, lds = 2 * 3 * 32 * KT * 256;
@@ -1023,7 +1057,21 @@ int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t s
     triangle = triangle && sq.len_k[s] - sq.len_q[s] <= sq.len_q[s] / 4;
   }
   const int64_t cus = tv_cu_count();
-  const bool two = most <= 128 || blocks128 * a.Hq <= cus || (triangle && blocks * a.Hq * 6 <= cus * (nseq < 3 ? 3 + nseq : 6));
+  bool two = most <= 128 || blocks128 * a.Hq <= cus;
+  if (!two && triangle && blocks * a.Hq * 6 <= cus * (nseq < 3 ? 3 + nseq : 6)) {
+    Dealt of128;
+    int64_t longest = 0;
+    for (int s = 0; s < nseq; ++s) {
+      const int64_t start = sq.len_k[s] - sq.len_q[s];
+      const auto steps = [&](int64_t q, int rows, int tile) {                     // tiles of keys that block q of the sequence visits
+        const int64_t hi = std::min<int64_t>(sq.len_k[s], (q + 1) * rows + start), lo = std::max<int64_t>(0, q * rows + start - a.window + 1) / tile;
+        return (hi + tile - 1) / tile - lo + std::min((std::min<int64_t>(a.keep, hi) + tile - 1) / tile, lo);
+      };
+      for (int64_t q = (sq.len_q[s] + 127) / 128; q-- > 0;) of128.add(10 + 4 * steps(q, 128, 128), a.Hq);
+      for (int64_t q = (sq.len_q[s] + 255) / 256; q-- > 0;) longest = std::max(longest, KT == 2 ? 13 + 3 * steps(q, 256, 64) : 10 + 4 * steps(q, 256, 96));
+    }
+    two = dealt_out_pays(of128, longest, KS > 6);
+  }
   const void* f = two ? (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2> : (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true>;
   const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, two ? FA_LDS2 : lds);
   if (e != hipSuccess) {
@@ -1074,6 +1122,10 @@ extern "C" int tv_fa_debug_stamps(unsigned long long* out) {
   return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_fa_stamps), sizeof(g_fa_stamps));
 }
 #endif
+
+extern "C" int tv_flash_attn_two_waves(int seqlen_q, int seqlen_k, int64_t pairs, int headdim, int causal) {
+  return two_waves_a_row(seqlen_q, seqlen_k, pairs, causal != 0, headdim > 96);
+}
 
 extern "C" void tv_flash_attn_set_variant(int variant) { g_fa_variant.store(variant, std::memory_order_relaxed); }
 
