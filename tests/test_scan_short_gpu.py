@@ -58,10 +58,11 @@ def test_short_scan(K, L, B, H, P, G, group_map, decay):
         assert torch.allclose(dec[b].double(), (d * A.double()).sum(0), rtol=1e-4, atol=1e-4)
 
 
-# slices up to 7 chunks, heads in segments from 8 on; those up to 24 chunks a segment (here one: 512 heads), the march beyond
-@pytest.mark.parametrize("B,H,G,chunks,kernels", [(1, 16, 2, 8, (9, 10)), (4, 128, 8, 25, (10, 6))])
-def test_either_side_of_a_line_agrees(K, B, H, G, chunks, kernels):
-    P, N = 80, 128
+# slices up to 7 chunks, 9 at head dim 80 and 24 of more than 128 heads; heads in segments from there on; those up to 24 chunks a segment (here one: 512 heads), the march beyond
+@pytest.mark.parametrize("B,H,P,G,chunks,kernels", [(1, 16, 64, 2, 8, (9, 10)), (1, 16, 80, 2, 10, (9, 10)), (1, 160, 80, 8, 25, (9, 10)), (1, 160, 32, 8, 8, (9, 10)),
+                                                    (4, 128, 80, 8, 25, (10, 6))])
+def test_either_side_of_a_line_agrees(K, B, H, P, G, chunks, kernels):
+    N = 128
     g = torch.Generator(device=DEV).manual_seed(3)
     r = lambda *s: torch.randn(s, generator=g, device=DEV)
     L = chunks * 64
@@ -129,7 +130,7 @@ def test_operands_expanded_over_the_tokens(K, L, which):
 # csrc/ssd_par.hip: a head per work-group, segments that start from the state their predecessors leave.  Chunk and segment edges, one segment (many heads, or slices
 # that column work-groups cannot take), head dims with and without a single tile; decays that take a chunk as it is, raised, or with the true mask
 @pytest.mark.parametrize("B,H,P,G,group_map,L", [
-    (1, 8, 80, 2, "block", 512), (1, 8, 80, 2, "tile", 577), (2, 8, 80, 2, "block", 1089), (1, 4, 32, 1, "block", 705), (2, 8, 64, 4, "tile", 640),
+    (1, 8, 80, 2, "block", 640), (1, 8, 80, 2, "tile", 577), (2, 8, 80, 2, "block", 1089), (1, 4, 32, 1, "block", 705), (2, 8, 64, 4, "tile", 640),
     (1, 2, 80, 2, "block", 1), (1, 2, 80, 2, "block", 63), (1, 2, 80, 2, "tile", 130), (1, 6, 64, 2, "block", 513),
     (3, 128, 80, 8, "block", 65), (2, 128, 32, 8, "block", 500)])
 @pytest.mark.parametrize("decay", ["slow", "mixed", "fast"])

@@ -1242,11 +1242,15 @@ int pick_segments(int batch, int nheads, int nchunks) {
 
 // Short sequences: column slices (ssd_cols.hip) while their work-groups (4 slices) all run at once and a segment's first pass would cost more
 // than it takes off the chain.  128 heads x 80, 8 groups, whole operator, slices | heads in segments (ssd_par.hip): 203 tokens 17.4 | 20.6 us, 390: 23.1 | 26.7,
-// 512: 36.2 | 30.3, 1 501: 90 | 54; 64 heads: 390 tokens 19.2 | 20.8, 512: 22.7 | 23.0, 700: 27.2 | 25.9.
+// 1 501: 90 | 54; 64 heads: 390 tokens 19.2 | 20.8, 700: 27.2 | 25.9.  A step of the slices costs up to twice as much where heads decay by more than 2^199 a chunk, so
+// the line depends on the data.  Slices | segments, times relative to the segments', slow decays and those of a fresh Mamba-2 layer: 128 heads x 80, 8 chunks .78, 1.2; 10: .81,
+// 1.25; 24: .93, 1.65; 32 heads, 9: .91, 1.1, 10: 1.06 and more; x 64, up to 128 heads, 8: .87 - 1.1, 1.4; over 128 heads, which are two or three segments, x 80 .66 - .78,
+// .7 - 1.1 up to 24 chunks, x 64 .76 - .88, 1.05 - 1.3; x 32 from 8 chunks on 1.05 and more.
 bool use_cols(int batch, int nheads, int headdim, int ngroups, int nchunks) {
   if (ngroups < 1 || nchunks < 1) return false;
   const int slices = nheads / ngroups * (headdim / 16);        // of a group
-  return nchunks < 8 && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= tv_cu_count();
+  const int most = headdim >= 64 && (int64_t)batch * nheads > 128 ? 24 : headdim == 80 ? 9 : 7;
+  return nchunks <= most && nheads % 2 == 0 && slices % 4 == 0 && (int64_t)batch * ngroups * (slices / 4) <= tv_cu_count();
 }
 
 // Segments of ssd_par.hip, 0: not its case.  Its work-groups (one a head and segment, two a compute unit) fill one round, a segment has two chunks or more (twelve, where the
