@@ -32,7 +32,8 @@ def close(got, want, mag):
     (2, 3, 3, 64, 300, 300, True), (1, 2, 2, 96, 140, 1000, True), (1, 2, 2, 80, 64, 513, False), (70, 1, 1, 64, 100, 100, False), (1, 16, 4, 128, 1000, 1000, True),
     # more than a round of 128-row blocks: where the longest ones' time is filled up, and where not
     (1, 44, 11, 64, 1100, 1100, True), (50, 4, 1, 128, 129, 130, True), (32, 4, 2, 80, 257, 257, True), (20, 5, 1, 64, 400, 490, True),
-    # more than a round of short sequences: one wave a row where the keys are one tile of 96
+    # short sequences: one wave a row where the keys are one tile of 96, up to a round of them and beyond
+    (1, 2, 1, 64, 96, 96, False), (1, 2, 1, 72, 1, 96, True), (2, 4, 2, 80, 128, 96, True), (1, 4, 1, 128, 100, 66, True), (1, 2, 2, 64, 64, 64, False), (3, 2, 1, 96, 3, 90, False),
     (300, 2, 2, 128, 96, 96, False), (150, 4, 1, 128, 70, 65, False), (150, 4, 1, 128, 70, 64, False), (600, 1, 1, 80, 1, 1, True), (300, 2, 1, 64, 65, 65, True), (200, 3, 3, 72, 96, 96, False), (130, 4, 2, 96, 128, 96, True), (513, 1, 1, 64, 33, 20, True),
     (513, 1, 1, 64, 100, 97, True)])
 def test_against_64_bits(B, H, G, D, Lq, Lk, causal, dtype):

@@ -966,11 +966,17 @@ bool two_waves_a_row(int Lq, int Lk, int64_t pairs, bool causal, bool wide) {
   for (int q = rows; q > 0; --q) two.add(10 + 4 * ((std::max<int64_t>(0, std::min<int64_t>(Lk, q * 128ll + Lk - Lq)) + 127) / 128), pairs);
   return dealt_out_pays(two, 10 + 4 * ((Lk + 95ll) / 96), wide);
 }
-// ... but not for more than a round of such short rows whose keys are one tile of 96: the second wave has nothing to do, or a masked step where one wave's tile has none.  Head
-// dims up to 64, and non-causal rows against 96 keys, against 65 and more at head dim 128 (16 heads, us, two waves | one, 320 and 16 384 pairs: 64 wide, causal,
-// 65 x 65: 14.9 | 13.9, 433 | 396; 48 x 48: 13.7 | 13.4, 384 | 382; 80 wide, 96 x 96: 16.7 | 14.5, 499 | 452; 128 wide: 19.7 | 16.5, 603 | 535, 80 x 80 19.1 | 18.3, 572 | 567; 80
-// wide: 80 x 80 476 | 482, causal 96 x 96 501 | 517).  Those start by head and batch entry: the division of a 1-D grid is 6 % of them (65 x 65: 428 | 396).
-bool one_tile(int ks, int Lk, int tile, bool causal) { return Lk <= tile && (ks <= 4 || (!causal && (Lk == tile || (ks > 6 && Lk > 64)))); }
+// ... but not for short rows whose keys are one tile of 96, where the second wave has nothing to do, or a masked step where one wave's tile has none (us, two waves | one).
+// Every row against all 96 keys: any grid (96 x 96, 16 heads, 256 and 320 pairs: 64 wide 9.1 | 7.4, 128 wide 12.2 | 10.4; 80 wide, 320: 16.7 | 14.5).  Two masked steps against
+// one, 65 keys and more: up to a round (80 x 80, 4 pairs 1.02 to 1.06 times by head dim), and beyond it at head dims up to 64 (65 x 65, 320 and 16 384 pairs: 14.9 | 13.9, 433 | 396)
+// and of 128 (causal 96 x 96: 1.04 - 1.07; 80 x 80 19.1 | 18.3, 572 | 567), not between (72 and 80 wide, 1 024 pairs: 32.5 | 37.0; 16 384: 476 | 482).  One step each, 64 keys
+// and fewer: beyond a round at head dims up to 64 (48 x 48: 13.7 | 13.4; 64 keys, 4 pairs: 7.1 | 7.6; 72 to 96 wide .81 to .97).
+// One wave's form starts by head and batch entry: the division of a 1-D grid is 6 % of such a call (65 x 65: 428 | 396).
+bool one_tile(int ks, int Lq, int Lk, int tile, bool causal, bool round) {
+  if (Lk > tile) return false;
+  if (Lk == tile && (!causal || Lq == 1)) return true;
+  return ks <= 4 ? !round || Lk > 64 : Lk > 64 && (ks > 6 || round);
+}
 constexpr int FA_LDS2 = 2 * 2 * 2 * 64 * 256;    // K and V of two steps of 128 keys
 
 template <typename T, int KS, int DT>
@@ -982,7 +988,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   const int nqb = (a.Lq + 255) / 256;
   static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
   const bool frames = a.Lq > 128 && xcd_ && !a.causal && nqb <= 8 && all >= 64;
-  if (a.Lq <= 128 && all > tv_cu_count() && one_tile(KS, a.Lk, 32 * KT, a.causal) && B <= 65535 && a.Hq <= 65535) {
+  if (a.Lq <= 128 && one_tile(KS, a.Lq, a.Lk, 32 * KT, a.causal, all <= tv_cu_count()) && B <= 65535 && a.Hq <= 65535) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
   } else if (!frames && two_waves_a_row(a.Lq, a.Lk, all, a.causal, KS > 6)) {
