@@ -13,7 +13,7 @@
 // Two barriers a step: k's inputs are complete | last readers of the two buffers with one copy (state copy, y tile) are done.
 // Arithmetic, frames and modes are ssd_head.hip's (floating frame, reset and standard steps; see there); a standard step takes its
 // mask factors one by one.
-// 7 to 9 chunks come here, 24 where the heads are too many for more than three segments (use_cols in ssd_head.hip); beyond, the chain is cut (ssd_par.hip).
+// Up to 7 chunks come here, 9 at head dim 80, 24 where the heads are too many for more than three segments (use_cols in ssd_head.hip); beyond, the chain is cut (ssd_par.hip).
 // What is left is instruction issue — three waves a SIMD with about 350 vector and 38 matrix instructions a step, 1.6 us — and, in heads that
 // decay by more than 2^199 a chunk, the mask factors of a standard step (2.6 us).
 // Measured (128 heads x 80, 8 groups, whole operator, against a wave per head): 203 tokens 35 -> 17 us, 390: 46 -> 23.
