@@ -3,9 +3,9 @@
 // Structure (wave64, v_mfma_f32_32x32x16): a workgroup of 8 waves owns 256 query
 // rows of one (batch, q-head) (128 with half of the keys a wave where those are too few work-groups; 4 waves for 128 rows of many short ones); each wave keeps
 // its 32 query rows as MFMA B fragments in registers for the whole kernel.  K/V tiles
-// of 96 keys arrive by LDS-DMA into a 3-stage ring shared by the waves, two tiles ahead
-// of the math (counted vmcnt, one barrier per tile); with two waves a row, steps of two tiles
-// of 64 keys into a ring of two stages, one step ahead.  The score tile is computed
+// of 64 keys arrive by LDS-DMA into rings of four shared by the waves, a step of two tiles
+// ahead of the math, one barrier a step.  A wave's loop is pipelined over its tiles: the
+// next tile's scores are multiplied beside the present one's exponentials.  The score tile is computed
 // TRANSPOSED, S^T = K . Q^T, so every lane owns one query column: the softmax
 // row statistics are per-lane scalars (one cross-half shuffle per tile), and the
 // P^T accumulator registers are, after a bf16 pack, directly the B operand of
@@ -25,9 +25,7 @@
 namespace {
 
 constexpr int FA_QW = 32;                  // query rows per wave
-#ifndef FA_KT
-#define FA_KT 3                            // key sub-tiles of 32 per LDS tile (96 keys: +7 % causal d=128 vs 64)
-#endif
+constexpr int FA_KT = 3;                   // key sub-tiles of 32 per LDS tile of the streaming kernels and of rows that see one tile
 
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -43,9 +41,17 @@ using ssdk::u32x4;
 using ssdk::gload16_async;
 using ssdk::settle;
 
+// f(integral_constant) for FROM .. TO - 1: indices into register arrays have to be constants
+template <int FROM, int TO, typename F> __device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (FROM < TO) {
+    f(std::integral_constant<int, FROM>{});
+    static_for<FROM + 1, TO>(f);
+  }
+}
+
 template <typename T> struct Frag;
 template <> struct Frag<bf16_t> {
-  typedef bf16x8 v8; typedef bf16x4 v4;
+  typedef bf16x8 v8; typedef bf16x4 v4; typedef bf16_t v2 __attribute__((ext_vector_type(2)));
   static constexpr bool is_bf16 = true;
   static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -58,7 +64,7 @@ template <> struct Frag<bf16_t> {
   }
 };
 template <> struct Frag<f16_t> {
-  typedef f16x8 v8; typedef f16x4 v4;
+  typedef f16x8 v8; typedef f16x4 v4; typedef f16_t v2 __attribute__((ext_vector_type(2)));
   static constexpr bool is_bf16 = false;
   static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -114,37 +120,50 @@ __device__ __forceinline__ void block_of(int id, int pairs, int& t, int& pair) {
   pair = x * q + more + (p >> 3);
 }
 
+// ssdk::glds16 for the lanes of `live` only (a wave-uniform mask): the other lanes' 16 LDS bytes keep what they hold.
+__device__ __forceinline__ void glds16_lanes(const void* sbase, unsigned voff, unsigned lds_dst, unsigned long long live) {
+  unsigned keep;
+  unsigned long long ex;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_mov_b64 %1, exec\n\ts_mov_b64 exec, %5\n\t"
+               "global_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %1\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep), "=&s"(ex) : "v"(voff), "s"(sbase), "s"(lds_dst), "s"(live) : "memory");
+}
+
 // KS = ceil(D/16) k-steps of QK^T, DT = ceil(D/32) d-tiles of PV, NW waves per workgroup.
 // K/V tiles of 32*KT keys go global -> LDS by LDS-DMA (global_load_lds_dwordx4, 16 bytes per
-// lane, no VGPR round trip: staging through registers cost a third of the kernel) into a
-// ring of 3 stages (KG 2: two), two tiles (one step) ahead of the math, with counted vmcnt waits and one barrier
-// per tile.  LDS rows are 256 bytes (128 elements); the 16-byte chunks of a row are
+// lane, no VGPR round trip: staging through registers cost a third of the kernel) into
+// rings of four tiles, a step of two tiles ahead of the math, one copy instruction every few MFMAs (a step's 64 in a row hold up every wave: 5 003 tokens, 40 heads: 330 us,
+// spread 304).  One barrier a step: with one per tile of 64 keys and rings of three 345 us.
+// What bounds it: long grids the chip's power (16 384 tokens: the matrix pipe is busy .62 of the time at 1.83 GHz, where one phase behind the other, all waves between
+// the same barriers, it was .48 at 2.09), short ones the chain of steps.  us, before and with this loop, causal, 40 heads on 8 x 128: 1 400 tokens 53 | 45, 5 003 308 | 280,
+// 16 384 2 725 | 2 455; 16 heads of 64, 4 096: 81 | 61; of 80: 94 | 70; windows of 256 - 8 192 in 2 - 16 prompts: 1.07 - 1.5 times.
+// LDS rows are 256 bytes (128 elements); the 16-byte chunks of a row are
 // XOR-swizzled on the DMA source address so that the row reads of K (ds_read_b128, chunk ^
 // row%16) and the transposing reads of V (ds_read_b64_tr_b16, chunk ^ 4(row%4)) are bank
 // conflict free.  Chunks past head_dim are never copied (the K ones QK^T reads are zeroed once).
-// KG 2: the first four waves and the last four hold the same 128 query rows and take every second tile of 32 KT keys each; two tiles are a step, two stages a
-// ring, and the halves (maximum, sum, accumulators) meet in LDS at the end.  A short grid is a chain of steps that lasts as long as the longest row of keys: this
-// halves it with the same two waves a SIMD (1 000 tokens, 40 heads: 41.0 -> 31.2 us).  Long grids lose by it: K and V go into LDS once per 128 rows.
+// KG 2: the first four waves and the last four hold the same 128 query rows and take every second tile of 32 KT keys each, one of a step's two; the halves (maximum, sum, accumulators) meet in LDS at the end.  A short grid is a chain of steps that lasts as long as the longest row of keys: this
+// halves it with the same two waves a SIMD (1 100 tokens, 40 heads: 35.2 -> 31.2 us).  Long grids lose by it: K and V go into LDS once per 128 rows.
 // WIN: causal with a sliding window and kept first keys.  The work-group visits the tiles that hold kept keys, then jumps to the
 // first tile of its first row's window: ring, copies and waits count the visited tiles.  All sequences of a packed step share the
 // launch (a launch per prompt leaves most of the chip idle: six prompts, 6 011 tokens, 16 heads on 4 x 128, window 1 024: 265 us, in one launch 95).
+constexpr int fa_slots(int kt) { return kt == 2 ? 4 : 1; }                       // (KT 3: keys of one tile)
+constexpr int fa_lds(int kt) { return 2 * fa_slots(kt) * 32 * kt * 256; }      // K and V rings, rows of 256 bytes
 template <typename T, int KS, int DT, int NW, int KT, bool WIN = false, int KG = 1>
 __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename std::conditional<WIN, AttnSeqs, NoSeqs>::type sq) {
   constexpr int FA_KB = 32 * KT;     // keys per tile
   constexpr int TPK = FA_KB / 4;     // 1 KiB DMA pieces (4 key rows) of K per tile
-  constexpr int NPK = KG * TPK;      // ... and per step; as many of V
   typedef typename Frag<T>::v8 v8;
   typedef typename Frag<T>::v4 v4;
+  typedef typename Frag<T>::v2 v2;
   constexpr int QB = NW / KG * FA_QW;     // query rows per workgroup
   constexpr int ROWB = 256;          // LDS bytes per key row
-  constexpr int TILEB = KG * FA_KB * ROWB;      // of a step
-  constexpr int NS = KG == 1 ? 3 : 2;           // ring stages
-  constexpr int PPW = 2 * NPK / NW;  // DMA pieces per wave and step
-  static_assert(2 * NPK % NW == 0, "pieces must divide over the waves");
+  constexpr int TILEB = FA_KB * ROWB;
+  constexpr int SLOTS = fa_slots(KT);           // tiles of the rings
+  static_assert(SLOTS == 1 || (SLOTS == 4 && TILEB == 16384), "a ring's halves are bit 15 of an LDS address");
+  constexpr int TPS = KG == 1 ? 2 : 1;          // tiles of a step that one wave takes: a step is two tiles
   extern __shared__ __attribute__((aligned(16))) unsigned char fa_smem[];
   unsigned char* const sK = fa_smem;
-  unsigned char* const sV = fa_smem + NS * TILEB;
-  const unsigned sK_off = (unsigned)(uintptr_t)(lds_u8*)fa_smem, sV_off = sK_off + NS * TILEB;
+  const unsigned sK_off = (unsigned)(uintptr_t)(lds_u8*)fa_smem, sV_off = sK_off + SLOTS * TILEB;      // (sK_off is 0: all LDS is dynamic)
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -206,9 +225,9 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   if (D < 16 * KS) {
     const v8 z = {};
     const int c0 = D / 8, nc = 2 * KS - c0;
-    for (int i = tid; i < NS * KG * FA_KB * nc; i += NW * 64) {
-      const int row = (i / nc) % (KG * FA_KB), st = i / (nc * KG * FA_KB), c = c0 + i % nc;
-      *reinterpret_cast<v8*>(sK + st * TILEB + row * ROWB + ((c ^ (row & 15)) << 4)) = z;
+    for (int i = tid; i < SLOTS * FA_KB * nc; i += NW * 64) {
+      const int row = i / nc, c = c0 + i % nc;
+      *reinterpret_cast<v8*>(sK + row * ROWB + ((c ^ (row & 15)) << 4)) = z;
     }
   }
 
@@ -241,205 +260,271 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     ntiles -= tskip;
   }
   auto key_of_tile = [&](int kt) __attribute__((always_inline)) { return (WIN && kt >= tkeep ? kt + tskip : kt) * FA_KB; };
-  const int nsteps = (ntiles + KG - 1) / KG;
 
-  // ---- DMA pieces of this wave: piece id pc = wave + NW*i; pc < 16 -> K rows 4pc..4pc+3,
-  // else V rows 4(pc-16)..; lane l carries row 4(pc%16) + l/16, LDS slot l%16 ----
-  int p_row[PPW];
-  unsigned p_off[PPW];            // byte offset from the tile's first key (full tiles)
-  int p_chunk[PPW];               // source 16-byte chunk of the row (255: past the head dim, nothing to copy)
-#pragma unroll
-  for (int i = 0; i < PPW; ++i) {
-    const int pc = wave + NW * i;
-    const bool isK = pc < NPK;
-    const int row = 4 * ((isK ? pc : pc - NPK) % TPK) + (lane >> 4);
-    const int c = (lane & 15) ^ (isK ? (row & 15) : 4 * (row & 3));
-    p_row[i] = row;
-    p_chunk[i] = c < (isK ? a.D : a.Dv) / 8 ? c : 255;
-    p_off[i] = (unsigned)(((int64_t)row * (isK ? a.ksl : a.vsl) + c * 8) * (int)sizeof(T));
-  }
-  auto issue_piece = [&](int kt, int i) {          // piece i (0..PPW-1) of step kt
-    const int stage = kt % NS;
-    const int pc = wave + NW * i;
-    const bool isK = pc < NPK;           // wave-uniform
-    // (a step's second tile may not exist: the last one again, nobody reads it)
-    const int kbase = key_of_tile(KG == 1 ? kt : min(kt * KG + (isK ? pc : pc - NPK) / TPK, ntiles - 1));
-    const void* tb = ssdk::uniform_ptr(isK ? (const void*)(kp + (int64_t)kbase * a.ksl)
-                                           : (const void*)(vp + (int64_t)kbase * a.vsl));
-    const int left = Lk - kbase;          // rows of this tile that exist
-    unsigned off = p_off[i];
-    if (left < FA_KB) {                  // last tile: rows past the end repeat the last key (masked later)
-      const int rr = min(p_row[i], left - 1);
-      off = (unsigned)(((int64_t)rr * (isK ? a.ksl : a.vsl) + p_chunk[i] * 8) * (int)sizeof(T));
-    }
-    const unsigned dst = ssdk::lds_addr_of((isK ? sK : sV) + stage * TILEB + (isK ? pc : pc - NPK) * 1024);
-    if (p_chunk[i] < 16) ssdk::glds16(tb, off, dst);     // EXEC masks the pad chunks
+  // ---- copies: a tile is TPK pieces of 4 key rows (lane l: row l / 16, LDS slot l % 16), piece wave + NW j of it this wave's; the rows of a wave's pieces are
+  // 4 NW apart, a multiple of 16, so that one lane offset an operand serves all of them (the source pointer moves instead)
+  constexpr int PPT = TPK / NW;                 // pieces of a tile this wave copies
+  static_assert(TPK % NW == 0 && 4 * NW % 16 == 0, "pieces must divide over the waves");
+  const int c_row = 4 * wave + (lane >> 4);
+  const int ck = (lane & 15) ^ (c_row & 15), cv = (lane & 15) ^ (4 * (c_row & 3));      // source chunks
+  const unsigned long long k_live = __builtin_amdgcn_ballot_w64(ck < a.D / 8), v_live = __builtin_amdgcn_ballot_w64(cv < a.Dv / 8);      // (chunks past the head dim: nothing to copy)
+  const unsigned k_row = (unsigned)a.ksl * (unsigned)sizeof(T), v_row = (unsigned)a.vsl * (unsigned)sizeof(T);      // (below 2^24: launcher)
+  auto copy_piece = [&](bool isK, int tile, int j) __attribute__((always_inline)) {      // (no branch: a tile that does not exist has no lanes)
+    const int kbase = key_of_tile(tile);
+    const void* src = ssdk::uniform_ptr(isK ? kp + (int64_t)kbase * a.ksl : vp + (int64_t)kbase * a.vsl);
+    const int row = min(c_row + 4 * NW * j, Lk - kbase - 1);                                // rows past the end repeat the last key (masked later)
+    const unsigned off = __umul24((unsigned)row, isK ? k_row : v_row) + (unsigned)((isK ? ck : cv) * 16);
+    glds16_lanes(src, off, __builtin_amdgcn_readfirstlane((isK ? sK_off : sV_off) + (unsigned)(tile % SLOTS * TILEB + (wave + NW * j) * 1024)), tile < ntiles ? isK ? k_live : v_live : 0ull);
   };
-  auto issue_tile = [&](int kt) {
+  auto copy_tile = [&](bool isK, int tile) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < PPW; ++i) issue_piece(kt, i);
+    for (int j = 0; j < PPT; ++j) copy_piece(isK, tile, j);
+  };
+  // what the step that starts with this wave's tile kt copies: the next one's tiles, piece c of 4 PPT
+  auto copy_ahead = [&](int kt, int c) __attribute__((always_inline)) {
+    const int t = c / PPT, tile = kt * KG + (t & 1);
+    copy_piece(t < 2, tile + (t < 2 ? KG + 2 : 2), c % PPT);
   };
 
-  // fragment read offsets inside a stage
-  int k_rd[KS];                   // K row fragment: row t*32 + r, chunk (2ks + hh) ^ (r % 16)
-  const int kz = (hh ^ (r & 15)) << 4;
+  // fragment reads: LDS addresses in the ring's present half (bit 15; KG 2: in this wave's tile of it); tile and sub-tile are instruction offsets
+  unsigned k_rd[KS], v_rd[DT];
+  constexpr unsigned HALF = SLOTS == 4 ? 2 * TILEB : 0;
+  auto set_reads = [&](unsigned half) __attribute__((always_inline)) {
+    const int kz = (hh ^ (r & 15)) << 4;      // K row fragment: row t*32 + r, chunk (2ks + hh) ^ (r % 16)
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) k_rd[ks] = r * ROWB + ((32 * ks) ^ kz);
-  const int q4 = (lane & 15) >> 2, p4 = lane & 3;
-  int v_rd[DT];                   // V^T fragment: row 16s + 4hh + q4 (+8), chunk (4dt + cc) ^ 4 q4
-  {
-    const int cc = 2 * ((lane >> 4) & 1) + (p4 >> 1);
+    for (int ks = 0; ks < KS; ++ks) k_rd[ks] = sK_off + half + (unsigned)(grp * TILEB + r * ROWB + ((32 * ks) ^ kz));
+    const int q4 = (lane & 15) >> 2, p4 = lane & 3, cc = 2 * ((lane >> 4) & 1) + (p4 >> 1);      // V^T fragment: row 16s + 4hh + q4 (+8), chunk (4dt + cc) ^ 4 q4
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      v_rd[dt] = (4 * hh + q4) * ROWB + ((4 * (dt ^ q4) + cc) << 4) + (p4 & 1) * 8;
+    for (int dt = 0; dt < DT; ++dt) v_rd[dt] = sV_off + half + (unsigned)(grp * TILEB + (4 * hh + q4) * ROWB + ((4 * (dt ^ q4) + cc) << 4) + (p4 & 1) * 8);
+  };
+
+  // ---- the steps this wave works in: of the visited tiles [0, n_seen) start below the last key its rows see; a window leaves out those between the kept keys and
+  // its first row's window
+  const int wave_q_last = q0 + FA_QW - 1;
+  int n_seen = ntiles, keep_to = 0, win_from = 0;
+  if (a.causal) {
+    const int whole = wave_q_last + shift < 0 ? 0 : (wave_q_last + shift) / FA_KB + 1;       // tiles of the sequence that start at or below it
+    n_seen = min(ntiles, WIN ? (whole <= tkeep ? whole : max(tkeep, whole - tskip)) : whole);
   }
+  if (q0 >= Lq) n_seen = 0;
+  if constexpr (WIN) {
+    keep_to = min(tkeep, n_seen);
+    win_from = max(keep_to, min(n_seen, max(0, q0 + shift - a.window + 1) / FA_KB - tskip));
+  }
+  // a wave's own count of tiles: with two waves a row every second one is its own
+  auto own = [&](int tile) __attribute__((always_inline)) { return KG == 1 ? tile : (max(tile - grp, 0) + KG - 1) / KG; };
+  const int nown = (ntiles + KG - 1) / KG;
 
   __syncthreads();                 // LDS zeroed before the first copy lands
-  if (nsteps > 0) issue_tile(0);
-  if (NS > 2 && nsteps > 1) issue_tile(1);
-  if (NS > 2 && nsteps > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // K of the first tile (of both halves) has landed, and Q, older, behind the first wait; the rest of the first step may be in flight
+  copy_tile(true, 0);
+  if (KG == 2) copy_tile(true, 1);
+  if constexpr (SLOTS > 1) { copy_tile(true, KG); copy_tile(true, KG + 1); }
+  copy_tile(false, 0);
+  if constexpr (SLOTS > 1) copy_tile(false, 1);
+  if (SLOTS > 1 && ntiles > KG + 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * PPT) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (copies without lanes are not counted on)
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {      // the Q loads are older than every copy: landed
+  for (int ks = 0; ks < KS; ++ks) {
     settle(qraw[ks]);
     const v8 z = {};
     qf[ks] = (qrow < Lq && ks * 16 + hh * 8 < D) ? __builtin_bit_cast(v8, qraw[ks]) : z;
   }
 
-  for (int kt = 0; kt < nsteps; ++kt) {
-    const int kbase = key_of_tile(KG == 1 ? kt : kt * KG + grp);
-    const bool ahead = kt + NS - 1 < nsteps;
-    // stage bases as LDS byte offsets (scalar), folded into one base register per fragment family
-    const unsigned stage_off = (unsigned)((kt % NS) * TILEB + grp * (FA_KB * ROWB));
-    const unsigned cK = sK_off + stage_off, cV = sV_off + stage_off;
-
-    // wave-uniform skip of tiles entirely above this wave's causal diagonal
-    const int wave_q_last = q0 + FA_QW - 1;
-    bool active = !(a.causal && kbase > wave_q_last + shift);
-    if constexpr (WIN) active = active && (kbase < a.keep || kbase + FA_KB > q0 + shift - a.window + 1);
-    if (KG > 1) active = active && kt * KG + grp < ntiles;
-    if (!active && ahead) issue_tile(kt + NS - 1);
-    if (active) {
-      // ---- S^T = K . Q^T  (2 key sub-tiles of 32); all K fragment reads ahead of the MFMAs;
-      // the copies of tile kt+2 (KG 2: of step kt+1) are issued between the MFMAs, whose pipe time hides them ----
-      f32x16 sacc[KT];
-      v8 kf[KT][KS];
-      unsigned kb[KS];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kb[ks] = cK + (unsigned)k_rd[ks];
+  // ---- a step: the scores of the wave's next tile (Q.K^T, matrix pipe) beside the weights of the present one (exponentials, vector pipe), then its P.V beside the
+  // next tile's maximum.  Every MFMA (32 cycles) gets its share of vector work in the source order, which the scheduling barriers pin: a wave keeps both pipes
+  // busy by itself, and its partner on the SIMD fills what is left.  (Multiplying first and exponentiating behind it, all waves between the same two barriers:
+  // 7 000 cycles a tile of 96 keys where the matrix pipe needs 3 072.)
+  // The accumulators are rescaled whenever some row's maximum has moved: a maximum that follows only when it has grown by 2^8 saves nearly all of that (5 003 tokens,
+  // 40 heads: 329 -> 305 us), but then a row's largest weight is no longer exactly 1 in bf16, and the error against 64 bits grows from .0019 to .0022.
+  constexpr int NQK = KT * KS, NPV = 2 * KT * DT, NE = 16 * KT;
+  constexpr int NE1 = NE * 5 / 8 / 2 * 2;       // weights formed beside Q.K^T, the rest beside P.V, each in front of the k-step that needs it
+  constexpr int LEAD = 4;                       // ... of them ahead of the first MFMA, whose operands are still on their way from LDS
+  constexpr int KAHEAD = 4;                     // K fragments read ahead
+  float neg_m = 0.f;                            // - maximum, 0 while there is none
+  typedef f32x16 Scores[KT];
+  Scores s0, s1;
+  auto tile_key = [&](int kt) __attribute__((always_inline)) { return key_of_tile(KG == 1 ? kt : kt * KG + grp); };
+  auto mask = [&](int kt, Scores& S) __attribute__((always_inline)) {
+    const int kbase = tile_key(kt);
+    bool need = (kbase + FA_KB > Lk) || (a.causal && kbase + FA_KB - 1 > q0 + shift);
+    if constexpr (WIN) need = need || (kbase <= wave_q_last + shift - a.window && kbase + FA_KB > a.keep);
+    if (need) {
 #pragma unroll
       for (int t = 0; t < KT; ++t)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) kf[t][ks] = Frag<T>::row_read(lds_at(kb[ks]) + t * (32 * ROWB));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < KT; ++t) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[t][i] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          sacc[t] = Frag<T>::mfma(kf[t][ks], qf[ks], sacc[t]);
-          // PPW pieces spread over the 2*KS MFMAs
-          constexpr int every = (KT * KS) / PPW > 0 ? (KT * KS) / PPW : 1;
-          const int idx = t * KS + ks;
-          if (ahead && idx % every == 0 && idx / every < PPW) issue_piece(kt + NS - 1, idx / every);
+        for (int i = 0; i < 16; ++i) {
+          const int key = kbase + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh;
+          bool ok = key < Lk && (!a.causal || key <= qrow + shift);
+          if constexpr (WIN) ok = ok && (key > qrow + shift - a.window || key < a.keep);
+          S[t][i] = ok ? S[t][i] : -INFINITY;
         }
-      }
-      if (ahead) {      // pieces that did not fit the spacing (PPW > 2*KS)
+    }
+  };
+  auto new_max = [&](float tmax) __attribute__((always_inline)) {       // of a tile: both halves of the wave hold keys of the same row
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+    const float mt = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * a.scale_log2;
+    if (__builtin_amdgcn_ballot_w64(mt > m_run)) {
+      const float m_new = fmaxf(m_run, mt);
+      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;       // (nothing visible yet)
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);    // m_run = -inf -> 0
+      l_run *= alpha;
 #pragma unroll
-        for (int i = (KT * KS) / ((KT * KS) / PPW > 0 ? (KT * KS) / PPW : 1); i < PPW; ++i) issue_piece(kt + NS - 1, i);
-      }
-      // ---- mask, running max on the raw scores (the scale is positive, so it commutes with
-      // max), then p = 2^(s*scale - m) as one FMA + v_exp per score; packed fp32 math ----
-      typedef float f32x2 __attribute__((ext_vector_type(2)));
-      bool need_mask = (kbase + FA_KB > Lk) || (a.causal && kbase + FA_KB - 1 > q0 + shift);
-      if constexpr (WIN) need_mask = need_mask || (kbase <= wave_q_last + shift - a.window && kbase + FA_KB > a.keep);
-      if (need_mask) {
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = kbase + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh;
-            bool ok = key < Lk && (!a.causal || key <= qrow + shift);
-            if constexpr (WIN) ok = ok && (key > qrow + shift - a.window || key < a.keep);
-            sacc[t][i] = ok ? sacc[t][i] : -INFINITY;
-          }
-      }
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < KT; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) tmax = fmaxf(fmaxf(tmax, sacc[t][i]), sacc[t][i + 1]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float m_new = fmaxf(m_run, tmax * a.scale_log2);
-      // rows with nothing visible yet keep m=-inf: use 0 as the exponent base
-      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);  // m_run=-inf -> 0
-      const f32x2 sc2 = {a.scale_log2, a.scale_log2}, nm2 = {-m_use, -m_use};
-      f32x2 ps2 = {0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < KT; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-          const f32x2 e = __builtin_elementwise_fma(f32x2{sacc[t][i], sacc[t][i + 1]}, sc2, nm2);
-          const f32x2 pp = {__builtin_amdgcn_exp2f(e[0]), __builtin_amdgcn_exp2f(e[1])};
-          sacc[t][i] = pp[0];
-          sacc[t][i + 1] = pp[1];
-          ps2 += pp;
-        }
-      l_run = l_run * alpha + (ps2[0] + ps2[1]);
-      // the accumulators only need rescaling when some row's maximum moved (wave-uniform test)
-      if (__builtin_amdgcn_ballot_w64(m_new > m_run)) {
-        const f32x2 al2 = {alpha, alpha};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; i += 2) {
-            const f32x2 v = f32x2{oacc[dt][i], oacc[dt][i + 1]} * al2;
-            oacc[dt][i] = v[0];
-            oacc[dt][i + 1] = v[1];
-          }
-      }
+        for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
       m_run = m_new;
-
-      // ---- O^T += V^T . P^T over 4 k-steps of 16 keys; the V^T fragments of k-step s+1 are in
-      // flight while k-step s multiplies ----
-      {
-        unsigned vb[DT];
+      neg_m = -m_use;
+    }
+  };
+  // CUR: S holds tile kt's masked scores; NEXT: the wave works in tile kt + 1 too; ODD: kt is odd (one wave a row: the second tile of a step)
+  auto step = [&](int kt, auto CURT, auto NEXTT, auto ODDT, Scores& S, Scores& SN) __attribute__((always_inline)) {
+    constexpr bool CUR = decltype(CURT)::value, NEXT = decltype(NEXTT)::value, ODD = decltype(ODDT)::value;
+    constexpr int KOFF = KG == 1 && !ODD && CUR ? TILEB : 0, VOFF = KG == 1 && ODD ? TILEB : 0;      // (without CUR: the first tile of a step)
+    constexpr bool COPIES = SLOTS > 1 && CUR && (TPS == 1 || !ODD);        // the first tile of a step: the next one's copies, spread (64 of them at once hold up every wave)
+    constexpr int CEVERY = (NQK + NPV) / (4 * PPT);
+    static_assert(!COPIES || (NQK + NPV) % (4 * PPT) == 0 || CEVERY * 4 * PPT <= NQK + NPV, "");
+    if constexpr (COPIES && !NEXT)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vb[dt] = cV + (unsigned)v_rd[dt];
-        auto read_v = [&](int s_, v4 (&lo)[DT], v4 (&hi)[DT]) {
-          // element j of this lane is key row 16s + 8(j>>2) + 4hh + (j&3) of the tile
+      for (int c = 0; c < 4 * PPT; ++c) copy_ahead(kt, c);
+    if constexpr (NEXT && CUR && (KG == 2 || ODD)) {             // tile kt + 1 is in the ring's other half
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            lo[dt] = Frag<T>::tr_read(lds_at(vb[dt]) + s_ * (16 * ROWB));
-            hi[dt] = Frag<T>::tr_read(lds_at(vb[dt]) + s_ * (16 * ROWB) + 8 * ROWB);
-          }
-        };
-        v4 vlo[2][DT], vhi[2][DT];
-        read_v(0, vlo[0], vhi[0]);
+      for (int ks = 0; ks < KS; ++ks) k_rd[ks] ^= HALF;
+    }
+    float ps0 = 0.f, ps1 = 0.f;
+    u32x4 pf[2 * KT];
+    auto weights = [&](auto FROM, auto TO) __attribute__((always_inline)) {
+      static_for<decltype(FROM)::value / 2, decltype(TO)::value / 2>([&](auto E) __attribute__((always_inline)) {
+        constexpr int e = 2 * decltype(E)::value;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][e & 15], a.scale_log2, neg_m));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][(e & 15) + 1], a.scale_log2, neg_m));
+        ps0 += p0;
+        ps1 += p1;
+        const v2 pair = {from_f32<T>(p0), from_f32<T>(p1)};
+        pf[e >> 3][(e & 7) >> 1] = __builtin_bit_cast(unsigned, pair);
+        // (formed HERE: the compiler would sink all of it behind the next branch, where the matrix pipe has nothing to do)
+        asm volatile("" : "+v"(pf[e >> 3][(e & 7) >> 1]), "+v"(ps0), "+v"(ps1));
+      });
+    };
+    auto largest = [&](auto FROM, auto TO, float m) __attribute__((always_inline)) {
+      static_for<decltype(FROM)::value, decltype(TO)::value>([&](auto E) __attribute__((always_inline)) {
+        constexpr int e = 2 * decltype(E)::value;
+        m = fmaxf(fmaxf(m, SN[e >> 4][e & 15]), SN[e >> 4][(e & 15) + 1]);
+      });
+      return m;
+    };
+    v4 vlo[2][DT], vhi[2][DT];
+    auto read_v = [&](int s_, int dt) __attribute__((always_inline)) {
+      // element j of this lane is key row 16s + 8(j>>2) + 4hh + (j&3) of the tile
+      const lds_u8* at = lds_at(v_rd[dt]) + VOFF;
+      vlo[s_ & 1][dt] = Frag<T>::tr_read(at + s_ * (16 * ROWB));
+      vhi[s_ & 1][dt] = Frag<T>::tr_read(at + s_ * (16 * ROWB) + 8 * ROWB);
+    };
+    using std::integral_constant;
+    if constexpr (NEXT) {
+      v8 kf[NQK];
+      auto read_k = [&](int i) __attribute__((always_inline)) { kf[i] = Frag<T>::row_read(lds_at(k_rd[i % KS]) + KOFF + (i / KS) * (32 * ROWB)); };
 #pragma unroll
-        for (int s_ = 0; s_ < 2 * KT; ++s_) {
-          if (s_ < 2 * KT - 1) read_v(s_ + 1, vlo[(s_ + 1) & 1], vhi[(s_ + 1) & 1]);
-          const int t = s_ >> 1, rb = (s_ & 1) * 8;
-          v8 pf;
+      for (int i = 0; i < KAHEAD; ++i) read_k(i);
+      if constexpr (CUR) weights(integral_constant<int, 0>{}, integral_constant<int, LEAD>{});
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, NQK>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (i + KAHEAD < NQK) read_k(i + KAHEAD);
+        if constexpr (CUR && i >= NQK - DT) read_v(0, i - (NQK - DT));
+        if constexpr (i % KS == 0)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) pf[j] = from_f32<T>(sacc[t][rb + j]);
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            v8 vf;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { vf[j] = vlo[s_ & 1][dt][j]; vf[4 + j] = vhi[s_ & 1][dt][j]; }
-            oacc[dt] = Frag<T>::mfma(vf, pf, oacc[dt]);
-          }
-          __builtin_amdgcn_sched_barrier(0);
+          for (int j = 0; j < 16; ++j) SN[i / KS][j] = 0.f;
+        SN[i / KS] = Frag<T>::mfma(kf[i], qf[i % KS], SN[i / KS]);
+        if constexpr (CUR && COPIES) {
+          if constexpr (i % CEVERY == CEVERY / 2) copy_ahead(kt, i / CEVERY);
         }
+        if constexpr (CUR) weights(integral_constant<int, LEAD + 2 * ((NE1 - LEAD) / 2 * i / NQK)>{}, integral_constant<int, LEAD + 2 * ((NE1 - LEAD) / 2 * (i + 1) / NQK)>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      mask(kt + 1, SN);
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) read_v(0, dt);
+      weights(integral_constant<int, 0>{}, integral_constant<int, NE1>{});
+    }
+    float tmax = -INFINITY;
+    if constexpr (CUR) {
+      __builtin_amdgcn_s_setprio(1);            // P.V first where both waves of a SIMD want the matrix pipe (16 384 tokens, 40 heads: 2 467 -> 2 445 us)
+      constexpr int NP1 = NPV - DT;             // (the last k-step needs all of them)
+      static_assert(NE1 >= 8 && NE1 % 2 == 0, "the first k-step's weights come first");
+      static_for<0, NPV>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value, s_ = i / DT, dt = i % DT;
+        if constexpr (s_ + 1 < 2 * KT) read_v(s_ + 1, dt);
+        v8 vf;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { vf[j] = vlo[s_ & 1][dt][j]; vf[4 + j] = vhi[s_ & 1][dt][j]; }
+        oacc[dt] = Frag<T>::mfma(vf, __builtin_bit_cast(v8, pf[s_]), oacc[dt]);
+        if constexpr (i < NP1) weights(integral_constant<int, NE1 + 2 * ((NE - NE1) / 2 * i / NP1)>{}, integral_constant<int, NE1 + 2 * ((NE - NE1) / 2 * (i + 1) / NP1)>{});
+        if constexpr (NEXT && COPIES) {
+          if constexpr ((NQK + i) % CEVERY == CEVERY / 2) copy_ahead(kt, (NQK + i) / CEVERY);
+        }
+        constexpr int M0 = 2;                   // (the scores' last MFMA ends behind the first of these)
+        if constexpr (NEXT && i >= M0) tmax = largest(integral_constant<int, NE / 2 * (i - M0) / (NPV - M0)>{}, integral_constant<int, NE / 2 * (i + 1 - M0) / (NPV - M0)>{}, tmax);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      __builtin_amdgcn_s_setprio(0);
+      l_run += ps0 + ps1;
+    } else {
+      tmax = largest(integral_constant<int, 0>{}, integral_constant<int, NE / 2>{}, tmax);
+    }
+    if constexpr (CUR && (KG == 2 || ODD)) {                    // tile kt + 1's V is in the other half
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) v_rd[dt] ^= HALF;
+    }
+    if constexpr (NEXT) new_max(tmax);
+  };
+  // The step that starts with this wave's tile kt: its V and the K of the tiles behind each are there for every wave, and nobody reads the other two places of a ring
+  // any more, which the next step's copies take.  (One barrier for two tiles.)
+  auto turn = [&](int kt, bool idle) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (SLOTS > 1 && idle)
+#pragma unroll
+      for (int c = 0; c < 4 * PPT; ++c) copy_ahead(kt, c);
+  };
+  {
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    int kt = 0;
+    // (a run starts with the first tile of a step)
+    const int run2 = TPS == 2 ? win_from & ~1 : own(win_from);
+    const bool one = !WIN || run2 <= own(keep_to);                  // nothing left out: one run of tiles
+#pragma unroll 1
+    for (int run = one ? 1 : 0; run < 2; ++run) {
+      const int from = one || !run ? 0 : run2, to = own(one || run ? n_seen : keep_to);
+      if (from >= to) continue;
+      for (; kt + TPS < from; kt += TPS) turn(kt, true);
+      if (kt < from) { turn(kt, true); kt += TPS; }
+      set_reads(HALF & (unsigned)-(int)((from * KG >> 1) & 1));
+      step(from - 1, no, yes, no, s1, s0);
+      if constexpr (SLOTS > 1) {
+#pragma unroll 1
+        for (; kt + 2 < to; kt += 2) {
+          turn(kt, false);
+          step(kt, yes, yes, no, s0, s1);
+          if (TPS == 1) turn(kt + 1, false);
+          step(kt + 1, yes, yes, yes, s1, s0);
+        }
+      }
+      turn(kt, false);
+      if (SLOTS > 1 && kt + 1 < to) {
+        step(kt, yes, yes, no, s0, s1);
+        if (TPS == 1) turn(kt + 1, false);
+        step(kt + 1, yes, no, yes, s1, s0);
+        kt += 2;
+      } else {
+        step(kt, yes, no, no, s0, s1);
+        kt += TPS;
       }
     }
-    // tile kt+1 (issued an iteration ago) must have landed; this iteration's copies stay in flight (KG 2: step kt+1 is this iteration's, and is waited for)
-    if (NS > 2 && ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (; kt < nown; kt += TPS) turn(kt, true);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
   }
@@ -508,15 +593,6 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   }
 }
 
-
-// ssdk::glds16 for the lanes of `live` only (a wave-uniform mask): the other lanes' 16 LDS bytes keep what they hold.
-__device__ __forceinline__ void glds16_lanes(const void* sbase, unsigned voff, unsigned lds_dst, unsigned long long live) {
-  unsigned keep;
-  unsigned long long ex;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_mov_b64 %1, exec\n\ts_mov_b64 exec, %5\n\t"
-               "global_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %1\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep), "=&s"(ex) : "v"(voff), "s"(sbase), "s"(lds_dst), "s"(live) : "memory");
-}
 
 // -DTV_FA_STAMP (dev): waves 0 and 4 of work-group 0 of the streaming kernel sum the cycles of each phase
 // of tile kt (s_memtime): g_fa_stamps[wave/4][kt < 16][phase < 8]; tv_fa_debug_stamps() copies them out.
@@ -928,7 +1004,7 @@ __global__ __launch_bounds__(512) void flash_fwd_stream_kernel(AttnArgs a) {
 std::atomic<int> g_fa_variant{[] { const char* v = getenv("TV_FA_W64"); return v ? atoi(v) : 0; }()};
 
 // When the last of a grid's work-groups ends, one of them a compute unit at a time, each starting where a unit is free first: runs of equal ones in grid order.  Its
-// unit of time is a quarter of a step of 128 keys by two waves a row, which a step of 96 by one wave takes as well; a block's start and end take 10.
+// unit of time is a quarter of a step of 128 keys by two waves a row, which 96 keys by one wave take as well; a block's start and end take 10.
 struct Dealt {
   struct Run { int64_t end; int n; } runs[512];     // (every run is a compute unit or more: never more runs than those)
   int size = 1;
@@ -952,12 +1028,11 @@ struct Dealt {
 // step of one wave takes a little more than the estimate (16 heads, 4 096 rows against 5 120 keys: 159 | 145 us, estimated alike)
 bool dealt_out_pays(const Dealt& two, int64_t one, bool wide) { return two.last * 100 < one * (wide ? 99 : 94); }
 
-// Whether two waves share 32 query rows (KG 2): up to 128 rows (64 against 4 096 keys, 40 heads: 131 us with one wave a SIMD, 88; 128: 14.7, 11.7), while 128-row
-// blocks are one round of the compute units (40 heads x 700: 31.8 | 24.2), and for more of them where causal blocks grow from nothing and the short ones, dealt out last,
-// fill up the long ones' time (40 x 1 400: 51.7 | 46.7, 28 x 2 000: 66.4 | 58.3; not 40 x 2 000, 320 blocks of 256: 70.4 | 84.7; nor 48 whole rows of 729: 27.1 | 39.5).
-// The line is the estimate above: it takes .095 of the .097 (logarithms, in the mean over 450 triangles beyond a round, head dim 64) and .122 of the .123 (128) that the better
-// form of each would give.  Two waves on all of them were slower on the short and the many (us, one | two: head dim 64, 256 rows against 320, 224 pairs 18.3 | 24.6; 384 x 480, 93:
-// 18.1 | 24.8; 128: 256 x 320, 167: 24.7 | 30.7; 768 x 960, 81: 41.0 | 48.2).
+// Whether two waves share 32 query rows (KG 2): up to 128 rows, while 128-row blocks are one round of the compute units (us, one wave | two: 40 heads x 128, 700 tokens
+// 24.9 | 18.6, 28 x 1 100 33.8 | 24.3; 64 wide, 40 x 700 18.5 | 13.3), and for more of them where causal blocks grow from nothing and the short ones, dealt out last,
+// fill up the long ones' time (40 x 1 400: 42.1 | 38.8, 28 x 2 000: 56.6 | 47.0; not 40 x 2 000, 320 blocks of 256: 60.3 | 67.1; nor whole rows).
+// The line is the estimate above: over 707 shapes of 130 to 4 000 rows (head dims 64, 80, 128; 4 to 160 pairs; triangles, triangles behind earlier keys, whole rows) what it
+// takes is .5 % slower in the mean than the better form of each; one wave always is 20 % slower, two 4 %.
 bool two_waves_a_row(int Lq, int Lk, int64_t pairs, bool causal, bool wide) {
   const int cus = tv_cu_count(), rows = (Lq + 127) / 128;
   if (Lq <= 128 || rows * pairs <= cus) return true;
@@ -977,26 +1052,26 @@ bool one_tile(int ks, int Lq, int Lk, int tile, bool causal, bool round) {
   if (Lk == tile && (!causal || Lq == 1)) return true;
   return ks <= 4 ? !round || Lk > 64 : Lk > 64 && (ks > 6 || round);
 }
-constexpr int FA_LDS2 = 2 * 2 * 2 * 64 * 256;    // K and V of two steps of 128 keys
 
 template <typename T, int KS, int DT>
 int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   constexpr int KT = FA_KT;
   constexpr int lds = 2 * 3 * 32 * KT * 256;   // K and V rings: 3 stages x 32 KT rows x 256 B
+  constexpr int lds1 = fa_lds(KT), lds2 = fa_lds(2);
   hipError_t e;
   const int64_t all = (int64_t)a.Hq * B;
   const int nqb = (a.Lq + 255) / 256;
   static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
   const bool frames = a.Lq > 128 && xcd_ && !a.causal && nqb <= 8 && all >= 64;
   if (a.Lq <= 128 && one_tile(KS, a.Lq, a.Lk, 32 * KT, a.causal, all <= tv_cu_count()) && B <= 65535 && a.Hq <= 65535) {
-    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds, st>>>(a, NoSeqs{});
+    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
+    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds1, st>>>(a, NoSeqs{});
   } else if (!frames && two_waves_a_row(a.Lq, a.Lk, all, a.causal, KS > 6)) {
-    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, FA_LDS2);
-    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 8, 2, false, 2><<<dim3((unsigned)((a.Lq + 127) / 128 * all)), 512, FA_LDS2, st>>>(a, NoSeqs{});
+    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2, false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
+    if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 8, 2, false, 2><<<dim3((unsigned)((a.Lq + 127) / 128 * all)), 512, lds2, st>>>(a, NoSeqs{});
   } else {
-    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, KT>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 8, 2>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
     if (e == hipSuccess) {
       if (frames) {
         AttnArgs ax = a;
@@ -1008,7 +1083,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
         static const int stream_ = [] { const char* v = getenv("TV_FA_STREAM"); return v ? atoi(v) : 1; }();
         const int64_t slots = (int64_t)ax.ppx * nqb;          // query blocks per XCD
         if constexpr (KS > 6) {                                // head_dim 128: the second Q set does not fit the registers
-          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax, NoSeqs{});
+          flash_fwd_kernel<T, KS, DT, 8, 2><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds2, st>>>(ax, NoSeqs{});
         } else if (stream_ && a.Lk > 32 * KT && slots > tv_cu_count() / 8) {
           // one resident work-group per CU streams its share of the query blocks
           static const int ones_ = [] { const char* v = getenv("TV_FA_ONES"); return v ? atoi(v) : 1; }();
@@ -1032,10 +1107,10 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
             if (e == hipSuccess) flash_fwd_stream_kernel<T, KS, DT, KT, false><<<grid_s, 512, lds, st>>>(ax);
           }
         } else {
-          flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds, st>>>(ax, NoSeqs{});
+          flash_fwd_kernel<T, KS, DT, 8, 2><<<dim3((unsigned)(pairs * nqb), 1, 1), 512, lds2, st>>>(ax, NoSeqs{});
         }
       } else {
-        flash_fwd_kernel<T, KS, DT, 8, KT><<<dim3((unsigned)(nqb * all)), 512, lds, st>>>(a, NoSeqs{});
+        flash_fwd_kernel<T, KS, DT, 8, 2><<<dim3((unsigned)(nqb * all)), 512, lds2, st>>>(a, NoSeqs{});
       }
     }
   }
@@ -1046,13 +1121,12 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   TV_LAUNCH_CHECK();
 }
 
-// windowed form: bf16, 64-key tiles at head dim 128 (the bounds of the window do not fit beside 96 keys' fragments; a step of 64 takes 3 of the estimate's units, the
-// rest of a block 13).  Blocks of 256 rows, or of 128 with two waves a row: if no sequence is longer, while those are one round, and for more where the sequences start
+// windowed form: bf16 (64 keys by one wave take 3 of the estimate's units, the rest of a block 13).  Blocks of 256 rows, or of 128 with two waves a row: if no sequence is longer, while those are one round, and for more where the sequences start
 // from nothing and the estimate of both grids says so (one prompt, 16 heads, window 1 024: 1 200 rows 54 | 37 us, 2 560: 65 | 54, 3 200: 64 | 75; four, 3 000 together:
 // 61 | 45; 32 x 100 rows behind 1 000 keys 116 | 81; but eight of 425, 16 heads 28 | 39, sixteen of 162, window 256 19 | 27).
 template <int KS, int DT>
 int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t st) {
-  constexpr int KT = KS > 6 ? 2 : FA_KT, lds = 2 * 3 * 32 * KT * 256;
+  constexpr int KT = 2, lds2 = fa_lds(KT);
   int most = 0;
   int64_t blocks = 0, blocks128 = 0;
   bool triangle = true;
@@ -1074,19 +1148,19 @@ int launch_fa_win(const AttnArgs& a, const AttnSeqs& sq, int nseq, hipStream_t s
         return (hi + tile - 1) / tile - lo + std::min((std::min<int64_t>(a.keep, hi) + tile - 1) / tile, lo);
       };
       for (int64_t q = (sq.len_q[s] + 127) / 128; q-- > 0;) of128.add(10 + 4 * steps(q, 128, 128), a.Hq);
-      for (int64_t q = (sq.len_q[s] + 255) / 256; q-- > 0;) longest = std::max(longest, KT == 2 ? 13 + 3 * steps(q, 256, 64) : 10 + 4 * steps(q, 256, 96));
+      for (int64_t q = (sq.len_q[s] + 255) / 256; q-- > 0;) longest = std::max(longest, 13 + 3 * steps(q, 256, 64));
     }
     two = dealt_out_pays(of128, longest, KS > 6);
   }
   const void* f = two ? (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2> : (const void*)flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true>;
-  const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, two ? FA_LDS2 : lds);
+  const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
   if (e != hipSuccess) {
     tv_set_error("flash_attn: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     return TV_ERR_LAUNCH;
   }
   const dim3 grid((unsigned)((two ? blocks128 : blocks) * a.Hq));
-  if (two) flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2><<<grid, 512, FA_LDS2, st>>>(a, sq);
-  else flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<grid, 512, lds, st>>>(a, sq);
+  if (two) flash_fwd_kernel<bf16_t, KS, DT, 8, 2, true, 2><<<grid, 512, lds2, st>>>(a, sq);
+  else flash_fwd_kernel<bf16_t, KS, DT, 8, KT, true><<<grid, 512, lds2, st>>>(a, sq);
   TV_LAUNCH_CHECK();
 }
 
