@@ -203,12 +203,13 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   } else {
     const int pairs = a.nb * a.Hq;
     int pair;
-    block_of<false>(blockIdx.x, pairs, qblk, pair);
+    block_of<KG == 2>(blockIdx.x, pairs, qblk, pair);
     if (a.causal) qblk = (a.Lq + QB - 1) / QB - 1 - qblk;
     b = a.nb == 1 ? 0 : pair / a.Hq;           // (a division is 30 instructions of a short call)
+    if (KG == 2) b = __builtin_amdgcn_readfirstlane(b);
     h = pair - b * a.Hq;
   }
-  const int hk = WIN ? __builtin_amdgcn_readfirstlane(h / (a.Hq / a.Hkv)) : h / (a.Hq / a.Hkv);
+  const int hk = WIN || KG == 2 ? __builtin_amdgcn_readfirstlane(h / (a.Hq / a.Hkv)) : h / (a.Hq / a.Hkv);
   const int grp = KG == 1 ? 0 : wave / (NW / KG);                        // which of a step's tiles this wave takes
   const int q0 = qblk * QB + (wave - grp * (NW / KG)) * FA_QW;      // first query row of this wave
   const int qrow = q0 + r;                      // this lane's query row
@@ -261,6 +262,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   }
   auto key_of_tile = [&](int kt) __attribute__((always_inline)) { return (WIN && kt >= tkeep ? kt + tskip : kt) * FA_KB; };
 
+  constexpr bool FEW = KS > 6 && WIN;           // no registers left: lane constants of the loop are formed where they are used
   // ---- copies: a tile is TPK pieces of 4 key rows (lane l: row l / 16, LDS slot l % 16), piece wave + NW j of it this wave's; the rows of a wave's pieces are
   // 4 NW apart, a multiple of 16, so that one lane offset an operand serves all of them (the source pointer moves instead)
   constexpr int PPT = TPK / NW;                 // pieces of a tile this wave copies
@@ -272,8 +274,15 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   auto copy_piece = [&](bool isK, int tile, int j) __attribute__((always_inline)) {      // (no branch: a tile that does not exist has no lanes)
     const int kbase = key_of_tile(tile);
     const void* src = ssdk::uniform_ptr(isK ? kp + (int64_t)kbase * a.ksl : vp + (int64_t)kbase * a.vsl);
-    const int row = min(c_row + 4 * NW * j, Lk - kbase - 1);                                // rows past the end repeat the last key (masked later)
-    const unsigned off = __umul24((unsigned)row, isK ? k_row : v_row) + (unsigned)((isK ? ck : cv) * 16);
+    int cr = c_row, cc = isK ? ck : cv;
+    if constexpr (FEW) {
+      int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("" : "+v"(l));
+      cr = 4 * wave + (l >> 4);
+      cc = (l & 15) ^ (isK ? cr & 15 : 4 * (cr & 3));
+    }
+    const int row = min(cr + 4 * NW * j, Lk - kbase - 1);                                   // rows past the end repeat the last key (masked later)
+    const unsigned off = __umul24((unsigned)row, isK ? k_row : v_row) + (unsigned)(cc * 16);
     glds16_lanes(src, off, __builtin_amdgcn_readfirstlane((isK ? sK_off : sV_off) + (unsigned)(tile % SLOTS * TILEB + (wave + NW * j) * 1024)), tile < ntiles ? isK ? k_live : v_live : 0ull);
   };
   auto copy_tile = [&](bool isK, int tile) __attribute__((always_inline)) {
@@ -287,15 +296,16 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   };
 
   // fragment reads: LDS addresses in the ring's present half (bit 15; KG 2: in this wave's tile of it); tile and sub-tile are instruction offsets
-  unsigned k_rd[KS], v_rd[DT];
+  constexpr int NK = FEW ? 1 : KS, NV = FEW ? 1 : DT;
+  unsigned k_rd[NK], v_rd[NV];
   constexpr unsigned HALF = SLOTS == 4 ? 2 * TILEB : 0;
   auto set_reads = [&](unsigned half) __attribute__((always_inline)) {
     const int kz = (hh ^ (r & 15)) << 4;      // K row fragment: row t*32 + r, chunk (2ks + hh) ^ (r % 16)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) k_rd[ks] = sK_off + half + (unsigned)(grp * TILEB + r * ROWB + ((32 * ks) ^ kz));
+    for (int ks = 0; ks < NK; ++ks) k_rd[ks] = sK_off + half + (unsigned)(grp * TILEB + r * ROWB + ((32 * ks) ^ kz));
     const int q4 = (lane & 15) >> 2, p4 = lane & 3, cc = 2 * ((lane >> 4) & 1) + (p4 >> 1);      // V^T fragment: row 16s + 4hh + q4 (+8), chunk (4dt + cc) ^ 4 q4
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) v_rd[dt] = sV_off + half + (unsigned)(grp * TILEB + (4 * hh + q4) * ROWB + ((4 * (dt ^ q4) + cc) << 4) + (p4 & 1) * 8);
+    for (int dt = 0; dt < NV; ++dt) v_rd[dt] = sV_off + half + (unsigned)(grp * TILEB + (4 * hh + q4) * ROWB + ((4 * (dt ^ q4) + cc) << 4) + (p4 & 1) * 8);
   };
 
   // ---- the steps this wave works in: of the visited tiles [0, n_seen) start below the last key its rows see; a window leaves out those between the kept keys and
@@ -341,7 +351,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   constexpr int NQK = KT * KS, NPV = 2 * KT * DT, NE = 16 * KT;
   constexpr int NE1 = NE * 5 / 8 / 2 * 2;       // weights formed beside Q.K^T, the rest beside P.V, each in front of the k-step that needs it
   constexpr int LEAD = 4;                       // ... of them ahead of the first MFMA, whose operands are still on their way from LDS
-  constexpr int KAHEAD = 4;                     // K fragments read ahead
+  constexpr int KAHEAD = FEW && KG == 2 ? 2 : 4;                     // K fragments read ahead
   float neg_m = 0.f;                            // - maximum, 0 while there is none
   typedef f32x16 Scores[KT];
   Scores s0, s1;
@@ -390,15 +400,16 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
       for (int c = 0; c < 4 * PPT; ++c) copy_ahead(kt, c);
     if constexpr (NEXT && CUR && (KG == 2 || ODD)) {             // tile kt + 1 is in the ring's other half
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) k_rd[ks] ^= HALF;
+      for (int ks = 0; ks < NK; ++ks) k_rd[ks] ^= HALF;
     }
-    float ps0 = 0.f, ps1 = 0.f;
+    float ps0 = 0.f, ps1 = 0.f, nm = neg_m;
+    asm volatile("" : "+v"(nm));             // (the exponents of all forms of a step would be formed in front of the branch between them)
     u32x4 pf[2 * KT];
     auto weights = [&](auto FROM, auto TO) __attribute__((always_inline)) {
       static_for<decltype(FROM)::value / 2, decltype(TO)::value / 2>([&](auto E) __attribute__((always_inline)) {
         constexpr int e = 2 * decltype(E)::value;
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][e & 15], a.scale_log2, neg_m));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][(e & 15) + 1], a.scale_log2, neg_m));
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][e & 15], a.scale_log2, nm));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e >> 4][(e & 15) + 1], a.scale_log2, nm));
         ps0 += p0;
         ps1 += p1;
         const v2 pair = {from_f32<T>(p0), from_f32<T>(p1)};
@@ -417,14 +428,14 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     v4 vlo[2][DT], vhi[2][DT];
     auto read_v = [&](int s_, int dt) __attribute__((always_inline)) {
       // element j of this lane is key row 16s + 8(j>>2) + 4hh + (j&3) of the tile
-      const lds_u8* at = lds_at(v_rd[dt]) + VOFF;
+      const lds_u8* at = lds_at(FEW ? v_rd[0] ^ (unsigned)(dt << 6) : v_rd[FEW ? 0 : dt]) + VOFF;
       vlo[s_ & 1][dt] = Frag<T>::tr_read(at + s_ * (16 * ROWB));
       vhi[s_ & 1][dt] = Frag<T>::tr_read(at + s_ * (16 * ROWB) + 8 * ROWB);
     };
     using std::integral_constant;
     if constexpr (NEXT) {
       v8 kf[NQK];
-      auto read_k = [&](int i) __attribute__((always_inline)) { kf[i] = Frag<T>::row_read(lds_at(k_rd[i % KS]) + KOFF + (i / KS) * (32 * ROWB)); };
+      auto read_k = [&](int i) __attribute__((always_inline)) { kf[i] = Frag<T>::row_read(lds_at(FEW ? k_rd[0] ^ (unsigned)(32 * (i % KS)) : k_rd[FEW ? 0 : i % KS]) + KOFF + (i / KS) * (32 * ROWB)); };
 #pragma unroll
       for (int i = 0; i < KAHEAD; ++i) read_k(i);
       if constexpr (CUR) weights(integral_constant<int, 0>{}, integral_constant<int, LEAD>{});
@@ -476,7 +487,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     }
     if constexpr (CUR && (KG == 2 || ODD)) {                    // tile kt + 1's V is in the other half
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) v_rd[dt] ^= HALF;
+      for (int dt = 0; dt < NV; ++dt) v_rd[dt] ^= HALF;
     }
     if constexpr (NEXT) new_max(tmax);
   };
@@ -530,6 +541,8 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   }
 
   // ---- epilogue: normalise and store O[q][d] ----
+  const int le = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));      // the lane, anew: what hangs on it would be carried through the loop and spilled
+  const int hh_e = le >> 5, qrow_e = q0 + (le & 31);
   float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   // KG 2: the two waves of a row meet over the ring; the first keeps the first half of the d-tiles, the second the rest
   constexpr int DH = (DT + 1) / 2;
@@ -541,20 +554,20 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
       if ((dt < DH) == (grp == 1)) {
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          xo[((wave * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + lane] = f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+          xo[((wave * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + le] = f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
       }
-    xm[(wave * 2 + 0) * 64 + lane] = m_run;
-    xm[(wave * 2 + 1) * 64 + lane] = l_tot;
+    xm[(wave * 2 + 0) * 64 + le] = m_run;
+    xm[(wave * 2 + 1) * 64 + le] = l_tot;
     __syncthreads();
     const int other = wave ^ (NW / 2);
-    const float m_o = xm[(other * 2 + 0) * 64 + lane], l_o = xm[(other * 2 + 1) * 64 + lane], m_all = fmaxf(m_run, m_o);
+    const float m_o = xm[(other * 2 + 0) * 64 + le], l_o = xm[(other * 2 + 1) * 64 + le], m_all = fmaxf(m_run, m_o);
     const float f = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_all), f_o = m_o == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_o - m_all);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
       if ((dt < DH) == (grp == 0)) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const f32x4 v = xo[((other * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + lane];
+          const f32x4 v = xo[((other * DH + (dt < DH ? dt : dt - DH)) * 4 + g) * 64 + le];
 #pragma unroll
           for (int j = 0; j < 4; ++j) oacc[dt][4 * g + j] = oacc[dt][4 * g + j] * f + v[j] * f_o;
         }
@@ -564,19 +577,19 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
   }
   if (a.sink) l_tot += __builtin_amdgcn_exp2f(a.sink[h] * 1.4426950408889634f - m_run);      // (not scaled; inf: the keys weigh nothing)
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (qrow < Lq) {
-    T* op = (T*)a.o + (WIN ? 0 : (int64_t)b * a.osb) + (row0 + qrow) * a.osl + (int64_t)h * a.osh;
+  if (qrow_e < Lq) {
+    T* op = (T*)a.o + (WIN ? 0 : (int64_t)b * a.osb) + (row0 + qrow_e) * a.osl + (int64_t)h * a.osh;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int d0 = dt * 32 + 8 * g + 4 * hh;
+        const int d0 = dt * 32 + 8 * g + 4 * hh_e;
         if (KG == 2 && (dt < DH) != (grp == 0)) continue;
         if (d0 < a.Dv) {
           v4 pk;
           if constexpr (WIN) {
             if (a.gate) {
-              const v4 gt = *(const v4*)((const T*)a.gate + (row0 + qrow) * a.gsl + (int64_t)h * a.gsh + d0);
+              const v4 gt = *(const v4*)((const T*)a.gate + (row0 + qrow_e) * a.gsl + (int64_t)h * a.gsh + d0);
 #pragma unroll
               for (int j = 0; j < 4; ++j) oacc[dt][4 * g + j] *= sigmoid_f((float)gt[j]);
             }
@@ -586,9 +599,9 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
           *(v4*)(op + d0) = pk;
         }
       }
-    if (!WIN && a.lse && hh == 0 && grp == 0) {
+    if (!WIN && a.lse && hh_e == 0 && grp == 0) {
       const float lse = l_tot > 0.f ? (m_run * 0.6931471805599453f + logf(l_tot)) : -INFINITY;
-      a.lse[((int64_t)b * a.Hq + h) * Lq + qrow] = lse;
+      a.lse[((int64_t)b * a.Hq + h) * Lq + qrow_e] = lse;
     }
   }
 }
@@ -1041,17 +1054,10 @@ bool two_waves_a_row(int Lq, int Lk, int64_t pairs, bool causal, bool wide) {
   for (int q = rows; q > 0; --q) two.add(10 + 4 * ((std::max<int64_t>(0, std::min<int64_t>(Lk, q * 128ll + Lk - Lq)) + 127) / 128), pairs);
   return dealt_out_pays(two, 10 + 4 * ((Lk + 95ll) / 96), wide);
 }
-// ... but not for short rows whose keys are one tile of 96, where the second wave has nothing to do, or a masked step where one wave's tile has none (us, two waves | one).
-// Every row against all 96 keys: any grid (96 x 96, 16 heads, 256 and 320 pairs: 64 wide 9.1 | 7.4, 128 wide 12.2 | 10.4; 80 wide, 320: 16.7 | 14.5).  Two masked steps against
-// one, 65 keys and more: up to a round (80 x 80, 4 pairs 1.02 to 1.06 times by head dim), and beyond it at head dims up to 64 (65 x 65, 320 and 16 384 pairs: 14.9 | 13.9, 433 | 396)
-// and of 128 (causal 96 x 96: 1.04 - 1.07; 80 x 80 19.1 | 18.3, 572 | 567), not between (72 and 80 wide, 1 024 pairs: 32.5 | 37.0; 16 384: 476 | 482).  One step each, 64 keys
-// and fewer: beyond a round at head dims up to 64 (48 x 48: 13.7 | 13.4; 64 keys, 4 pairs: 7.1 | 7.6; 72 to 96 wide .81 to .97).
-// One wave's form starts by head and batch entry: the division of a 1-D grid is 6 % of such a call (65 x 65: 428 | 396).
-bool one_tile(int ks, int Lq, int Lk, int tile, bool causal, bool round) {
-  if (Lk > tile) return false;
-  if (Lk == tile && (!causal || Lq == 1)) return true;
-  return ks <= 4 ? !round || Lk > 64 : Lk > 64 && (ks > 6 || round);
-}
+// ... but not for short rows whose keys are one tile of 96: four waves, no ring, a third of the LDS, so that several such work-groups run on a compute unit; by head and
+// batch entry, without a division (us, two waves a row | this, causal: 16 heads of 64: 1 x 1 5.7 | 5.5, 64 x 64 6.2 | 5.8, 96 x 96 7.0 | 6.1; of 128: 8.2 | 6.6, 9.6 | 7.3; 4 000 pairs
+// 64 wide, 33 x 33 83 | 35, 128 x 96 107 | 46; 128 wide, 111 | 41, 173 | 84; the worst of 80 forms, 16 heads of 64, 64 x 64 without a mask: 5.7 | 5.9).
+bool one_tile(int Lk, int tile) { return Lk <= tile; }
 
 template <typename T, int KS, int DT>
 int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
@@ -1063,7 +1069,7 @@ int launch_fa_d(const AttnArgs& a, int B, hipStream_t st) {
   const int nqb = (a.Lq + 255) / 256;
   static const int xcd_ = [] { const char* v = getenv("TV_FA_XCD"); return v ? atoi(v) : 1; }();
   const bool frames = a.Lq > 128 && xcd_ && !a.causal && nqb <= 8 && all >= 64;
-  if (a.Lq <= 128 && one_tile(KS, a.Lq, a.Lk, 32 * KT, a.causal, all <= tv_cu_count()) && B <= 65535 && a.Hq <= 65535) {
+  if (a.Lq <= 128 && one_tile(a.Lk, 32 * KT) && B <= 65535 && a.Hq <= 65535) {
     e = hipFuncSetAttribute((const void*)flash_fwd_kernel<T, KS, DT, 4, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
     if (e == hipSuccess) flash_fwd_kernel<T, KS, DT, 4, KT><<<dim3(1, (unsigned)a.Hq, (unsigned)B), 256, lds1, st>>>(a, NoSeqs{});
   } else if (!frames && two_waves_a_row(a.Lq, a.Lk, all, a.causal, KS > 6)) {
