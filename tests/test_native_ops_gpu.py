@@ -1,0 +1,193 @@
+"""The operators' native host side: the same kernels on the same operands, so the same bits as the way through Python, over the forms that both take; what it does not take."""
+import threading
+
+import pytest
+import torch
+
+from timeviper_amd import kernels as ops
+from timeviper_amd._native import ops as native
+
+DEV = "cuda"
+BF, F32, F16 = torch.bfloat16, torch.float32, torch.float16
+NAMES = ("rms_norm", "layer_norm", "gated_norm", "conv_xbc", "scan", "flash", "mid_linear", "split_linear", "rows_linear", "small_linear", "residual_add", "split_add_linear",
+         "token_side", "norm_shift", "gated_mul", "scatter_rows", "attention_window")
+
+
+class Asked:
+    """The native operators (or none of them), with a count of the calls that they took"""
+    def __init__(self, on):
+        self.on, self.took = on, 0
+
+    def __getattr__(self, name):
+        def call(*a):
+            r = getattr(native, name)(*a) if self.on else None
+            self.took += r is not None
+            return r
+        return call
+
+
+def r(*s, dtype=BF, seed=0):
+    return torch.randn(s, generator=torch.Generator(device=DEV).manual_seed(seed + sum(s)), device=DEV).to(dtype)
+
+
+class Own(torch.Tensor):
+    pass
+
+
+def plan(counts, starts, slots, cap):
+    from timeviper_amd.model.llm.cache import StepPlan
+    i = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    cu = [sum(counts[:j]) for j in range(len(counts) + 1)]
+    return StepPlan(slots=tuple(slots), counts=tuple(counts), starts=tuple(starts), cu=i(cu), start=i(starts), slot=i(slots),
+                    rows=i([s * cap + a + j for s, a, n in zip(slots, starts, counts) for j in range(n)]), seq=i([b for b, n in enumerate(counts) for _ in range(n)]), keys=None, moving=None,
+                    decode=False)
+
+
+def norms(t):
+    for x, res in ((r(7, 96, dtype=t), None), (r(2, 3, 4096, dtype=t), r(2, 3, 4096, dtype=t, seed=1)), (r(5, 64, dtype=t), r(5, 64, dtype=t, seed=2))):
+        D = x.shape[-1]
+        for w in {t: r(D, dtype=t), F32: r(D, dtype=F32)}.values():
+            for sums in (False, True):
+                yield lambda: ops.rms_norm(x, w, 1e-5, res, sums), 1
+        for b in (None, r(D, dtype=t, seed=3)):
+            for rb in (None, r(D, dtype=F32, seed=4)):
+                yield lambda: ops.layer_norm(x, r(D, dtype=t), b, 1e-6, None, True, rb), 1
+    z = r(2, 9, 704, dtype=t)                                                            # gates: columns of a wider projection
+    for z_, group in ((None, 64), (z[..., 64:320], 64), (z[..., :256].contiguous(), None)):
+        yield lambda: ops.rmsnorm_fn(r(2, 9, 256, dtype=t), r(256, dtype=F32), None, z_, 1e-5, group, norm_before_gate=False), 1
+    yield lambda: ops.rms_norm(r(6, 96, dtype=t)[::2], r(96, dtype=t), 1e-5), 0           # a copy is needed
+    yield lambda: ops.rms_norm(r(6, 96, dtype=t).as_subclass(Own), r(96, dtype=t), 1e-5), 0
+
+
+def mixer(t):
+    for B, L, cols in ((1, 1, 0), (2, 63, 40), (1, 300, 8)):
+        H, P, G, N = 16, 64, 2, 128
+        di = H * P
+        wide = r(B, L, cols + di + 2 * G * N + H, dtype=t)
+        xBC, dt = wide[..., cols:cols + di + 2 * G * N], wide[..., cols + di + 2 * G * N:]
+        w, b = r(di + 2 * G * N, 1, 4, dtype=t), r(di + 2 * G * N, dtype=t)
+        A, D, bias = -torch.rand(H, device=DEV) - .1, r(H, dtype=F32), r(H, dtype=F32)
+        for cb in (False, True):
+            yield lambda: ops.causal_conv1d_xbc(xBC, w.squeeze(1), b if cb else None, di, G, N, return_cb=cb), 1
+        x, Bm, Cm = ops.causal_conv1d_xbc(xBC, w.squeeze(1), b, di, G, N)[:3]
+        for init in (None, r(B, H, P, N, dtype=F32)):
+            for final in (False, True):
+                yield lambda: ops.mamba_chunk_scan_combined(x.view(B, L, H, P), dt, A, Bm, Cm, chunk_size=256, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=final), 1
+
+
+def attention(t):
+    for D, Lq, Lk in ((128, 5, 5), (72, 130, 130), (64, 33, 100)):
+        wide = r(2, max(Lq, Lk), 8 * D, dtype=t)
+        q, k, v = wide[:, :Lq, :4 * D].unflatten(2, (4, D)), wide[:, :Lk, 4 * D:6 * D].unflatten(2, (2, D)), wide[:, :Lk, 6 * D:].unflatten(2, (2, D))
+        for causal in (False, True):
+            for scale in (None, .3):
+                yield lambda: ops.flash_attn_func(q, k, v, softmax_scale=scale, causal=causal, return_lse=causal), 1
+    yield lambda: ops.flash_attn_func(r(2, 9, 4, 128, dtype=t)[..., ::2], r(2, 9, 2, 64, dtype=t), r(2, 9, 2, 64, dtype=t)), 0       # a copy is needed
+
+
+def products(t):
+    for M in (33, 100, 256):
+        wide = r(640, 520)
+        for w in (wide[:, :512], wide[:, :512].contiguous()):
+            for b in (None, r(640)):
+                yield lambda: ops.mid_linear(r(M, 512), w, b, relu2=b is None), 1
+                yield lambda: ops.split_linear(r(M, 512), w, b, splits=2), 1
+                yield lambda: ops.small_linear(r(M, 512), w, b, 1 if b is None else 0), 1
+                yield lambda: ops.split_add_linear(r(M, 512), w, r(M, 640, dtype=F32), b, splits=2), 1
+    for M in (2, 17, 32):
+        yield lambda: ops.rows_linear(r(1, M, 512), r(640, 512), r(640) if M == 2 else None, relu2=M == 17), 1
+
+
+def packed(t):
+    dk, G, H, cap = 64, 2, 6, 200
+    cache, p = r(3, cap, G * 2 * dk), plan([5, 1, 120], [0, 30, 80], [2, 0, 1], cap)
+    T, D = 126, 96
+    wide = r(T, 2 * H * dk)
+    q, gate = wide[:, :H * dk].unflatten(1, (H, dk)), wide[:, H * dk:].unflatten(1, (H, dk))
+    for g in (None, gate):
+        for window in (7, 1 << 30):
+            yield lambda: ops.attention_window(q, cache, p, G, .125, window=window, keep_first=4, gate=g), 1
+    yield lambda: ops.attention_window(q, cache, p, G, .125, gate=gate, out=torch.empty(T, H, dk + 8, dtype=BF, device=DEV)[..., :dk]), 1
+    x, y = r(T, D, dtype=F32), r(T, 2 * D)[:, D:]
+    for pending in (None, y):
+        yield lambda: ops.norm_shift(x, r(1), 1e-5, pending, None if pending is None else r(D)), 1
+        state = r(3, 5, 2, D, dtype=F32)
+        yield lambda: (ops.norm_shift(x, r(1), 1e-5, pending, None if pending is None else r(D), r(D), (s := state.clone())[:, 3], p, need_h=pending is None), s), 1
+    yield lambda: ops.residual_add(x, y), 1
+    ids = torch.arange(T, device=DEV).flip(0)
+    for i, b in ((None, r(T, D, seed=5)), (ids, r(T, D, seed=6))):
+        for act in (0, 1):
+            yield lambda: ops.gated_mul(y, b, act, i), 1
+    yield lambda: ops.gated_mul(y, r(T, D), 0, None, torch.empty(T, 2 * D, dtype=BF, device=DEV)[:, :D]), 1
+    def scatter():
+        dst = torch.zeros(3 * cap, D, dtype=BF, device=DEV)
+        ops.scatter_rows(y, p.rows, dst)
+        return dst
+    yield scatter, 1
+
+
+def flat(v):
+    return [t for u in v for t in flat(u)] if isinstance(v, (tuple, list)) else [v]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("forms,dtype", [(norms, BF), (norms, F32), (norms, F16), (mixer, BF), (mixer, F32), (attention, BF), (attention, F16), (products, BF), (packed, BF)])
+def test_same_bits(forms, dtype, monkeypatch):
+    for call, taken in forms(dtype):
+        got = []
+        for on in (True, False):
+            asked = Asked(on)
+            monkeypatch.setattr(ops, "_n", asked)
+            got.append(flat(call()))
+            assert asked.took == (taken if on else 0)
+        monkeypatch.setattr(ops, "_n", native)
+        assert len(got[0]) == len(got[1])
+        for a, b in zip(*got):
+            if not isinstance(a, torch.Tensor):
+                assert a is b is None
+                continue
+            assert type(a) is type(b) and a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+            bits = lambda t: t.contiguous().view(torch.uint8)
+            assert torch.equal(bits(a), bits(b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", [
+    lambda: ops.flash_attn_func(r(2, 9, 4, 68)[..., :64], r(2, 9, 2, 64), r(2, 9, 2, 64)), lambda: ops.rms_norm(r(3, 64), torch.ones(64), 1e-5), lambda: ops.flash_attn_func(r(1, 4, 3, 64), r(1, 4, 2, 64), r(1, 4, 2, 64)),
+    lambda: ops.residual_add(r(3, 64), r(3, 64)), lambda: ops.gated_mul(r(3, 64), r(4, 64), 0), lambda: ops.mid_linear(r(300, 512), r(640, 512)),
+    lambda: ops.attention_window(r(4, 2, 64), r(1, 3, 256), plan([4], [0], [0], 3), 2, .1), lambda: ops.scatter_rows(r(4, 64), torch.zeros(3, dtype=torch.int32, device=DEV), r(9, 64))])
+def test_refused_as_before(call, monkeypatch):
+    told = []
+    for on in (True, False):
+        monkeypatch.setattr(ops, "_n", Asked(on))
+        with pytest.raises(Exception) as e:
+            call()
+        told.append((type(e.value), str(e.value)))
+    assert told[0] == told[1]
+
+
+@pytest.mark.gpu
+def test_threads_on_streams_of_their_own():
+    x, w = [r(64 + i, 1024, seed=i) for i in range(4)], r(1024)
+    want = [ops.rms_norm(v, w, 1e-5) for v in x]
+    torch.cuda.synchronize()
+    ok = [False] * 4
+
+    def go(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(50):
+                y = ops.rms_norm(x[i], w, 1e-5)
+            torch.cuda.current_stream().synchronize()
+            ok[i] = torch.equal(y, want[i])
+    threads = [threading.Thread(target=go, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert all(ok)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_nothing_but_gpu_tensors(name):
+    """CPU tensors, no tensors, too few arguments: None, and no error left behind"""
+    f = getattr(native, name)
+    t = torch.ones(2, 4, 8, 8, dtype=torch.bfloat16)
+    assert f() is None and all(f(*[v] * n) is None for v in (t, None, 1, "a") for n in range(1, 18))

@@ -23,6 +23,9 @@ CSRC = ROOT / "csrc"
 OBJ = ROOT / "lib" / "obj"
 LIB = ROOT / "lib" / "libtimeviper_hip.so"
 LIB_ID = ROOT / "lib" / "libtimeviper_hip.id"
+NATIVE = ROOT / "lib" / "_tv_native.so"          # the operators' host side: a Python extension on torch's headers, no device code
+NATIVE_ID = ROOT / "lib" / "_tv_native.id"
+NATIVE_SRC = CSRC / "host" / "native_ops.cpp"
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off",
@@ -102,7 +105,39 @@ def build(force: bool = False, jobs: int = 0) -> Path:
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
         LIB_ID.write_text(bid)
+    build_native(force)
     return LIB
+
+
+def _native_flags():
+    import sysconfig
+    import torch
+    t = Path(torch.__file__).resolve().parent
+    rocm = Path(HIPCC).resolve().parent.parent if Path(HIPCC).is_absolute() else Path("/opt/rocm")
+    inc = [ROOT.parent / "include", t / "include", t / "include" / "torch" / "csrc" / "api" / "include", "/opt/rocm/include", rocm / "include", sysconfig.get_paths()["include"]]
+    return (["-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"] + [f"-I{p}" for p in inc],
+            [f"-L{t / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], torch.__version__)
+
+
+def native_id() -> str:
+    """Hash of the host operators' source, the C ABI's header and torch's version"""
+    import torch
+    return _hash([NATIVE_SRC, ROOT.parent / "include" / "timeviper_hip.h"], torch.__version__)
+
+
+def native_is_current() -> bool:
+    return NATIVE.exists() and NATIVE_ID.exists() and NATIVE_ID.read_text() == native_id()
+
+
+def build_native(force: bool = False) -> Path:
+    if force or not native_is_current():
+        flags, libs, _ = _native_flags()
+        NATIVE.parent.mkdir(parents=True, exist_ok=True)
+        r = subprocess.run([os.environ.get("CXX", "g++"), *flags, str(NATIVE_SRC), "-o", str(NATIVE), *libs], capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"host operators: {r.stdout}\n{r.stderr}")
+        NATIVE_ID.write_text(native_id())
+    return NATIVE
 
 
 def ensure_built() -> Path:
@@ -111,7 +146,7 @@ def ensure_built() -> Path:
     This is a BUILD step, not a fallback: without a working hipcc it raises, and the operators
     keep failing loudly.  (`_capi.lib()` checks `tv_build_id()` of the loaded library against the
     same hash, so a stale binary cannot be used silently either.)"""
-    if LIB.exists() and LIB_ID.exists() and LIB_ID.read_text() == source_id():
+    if LIB.exists() and LIB_ID.exists() and LIB_ID.read_text() == source_id() and native_is_current():
         return LIB
     return build()
 

@@ -26,6 +26,7 @@ import torch
 
 from . import _capi
 from ._capi import TV_BF16, TV_F16, TV_F32, TimeViperHipError, check
+from ._native import ops as _n
 
 _DT = {torch.float32: TV_F32, torch.bfloat16: TV_BF16, torch.float16: TV_F16}
 
@@ -131,6 +132,8 @@ def causal_conv1d_xbc(xBC, weight, bias, d_inner: int, ngroups: int, dstate: int
     `return_cb`: also return the causal C.B^T fragments of every (chunk, group) for
     `mamba_chunk_scan_combined(..., cb=...)` (an opaque bf16 tensor; None where the scan would
     not use them: other dtypes / d_state), computed while the B / C tiles are on the chip."""
+    if halo is None and xBC.is_cuda and (r := _n.conv_xbc(xBC, weight, bias, d_inner, ngroups, dstate, activation in ("silu", "swish"), return_cb)) is not None:
+        return r
     _gpu(xBC, weight, bias, halo)
     Bsz, L, Cc = xBC.shape
     assert Cc == d_inner + 2 * ngroups * dstate
@@ -185,6 +188,8 @@ def rms_norm(x, weight, eps, residual=None, return_sum=False):
     """NemotronHRMSNorm (modeling_nano.py:897-903); with `residual`, normalises
     s = x + residual (rounded to x.dtype like the reference's bf16 add, :966) and
     can return s too."""
+    if x.is_cuda and (r := _n.rms_norm(x, weight, eps, residual, return_sum)) is not None:
+        return r
     _gpu(x, weight, residual)
     w = weight if weight.dtype in (torch.float32, x.dtype) else weight.to(torch.float32)
     w = w.contiguous()
@@ -213,6 +218,8 @@ def layer_norm(x, weight, bias, eps, residual=None, return_sum=False, row_bias=N
     returning s too — the fused form of a pre-norm ViT block's residual add + norm.
     `row_bias` (D,) fp32: a constant row added to every s before the statistics (not to the
     returned sum): the projection biases a caller carries beside a stream its GEMMs accumulate into."""
+    if residual is None and x.is_cuda and (r := _n.layer_norm(x, weight, bias, eps, return_sum, row_bias)) is not None:
+        return r
     _gpu(x, weight, bias, residual, row_bias)
     w = _as(weight, x.dtype)
     b = None if bias is None else _as(bias, x.dtype)
@@ -262,6 +269,8 @@ def rmsnorm_fn(x, weight, bias=None, z=None, eps=1e-6, group_size=None,
         raise TimeViperHipError("rmsnorm_fn: bias unsupported (reference passes None)")
     if z is not None and norm_before_gate:
         raise TimeViperHipError("rmsnorm_fn: only norm_before_gate=False is on the path")
+    if x.is_cuda and (r := _n.gated_norm(x, weight, z, eps, group_size)) is not None:
+        return r
     _gpu(x, weight, z)
     D = x.shape[-1]
     gs = D if group_size is None else int(group_size)
@@ -418,6 +427,9 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size=None, D=None, z=None, d
         raise TimeViperHipError("mamba_chunk_scan_combined: z/seq_idx/cu_seqlens unsupported")
     if D is not None and D.dim() != 1:
         raise TimeViperHipError("mamba_chunk_scan_combined: D must be (nheads,)")
+    if x.is_cuda and (r := _n.scan(x, dt, A, B, C, D, dt_bias, initial_states, dt_softplus, dt_limit[0], min(dt_limit[1], 3.0e38), return_final_states, return_total_decay,
+                                   {"block": 0, "tile": 1}[group_map], cb)) is not None:
+        return r
     _gpu(x, dt, A, B, C, D, dt_bias, initial_states)
     Bsz, L, H, P = x.shape
     G, N = B.shape[2], B.shape[3]
@@ -614,6 +626,8 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
     causal mask bottom-right aligned (flash-attn >= 2.1 semantics)."""
     if dropout_p:
         raise TimeViperHipError("flash_attn_func: dropout is not on the inference path")
+    if q.is_cuda and not _ATTN_FP8["on"] and (r := _n.flash(q, k, v, softmax_scale, causal, return_lse)) is not None:
+        return r
     _gpu(q, k, v)
     B, Lq, Hq, D = q.shape
     Lk, Hkv = k.shape[1], k.shape[2]
@@ -804,6 +818,8 @@ def rows_linear(x, weight, bias=None, relu2=False, conv=None, out_dtype=None, ro
     ReLU of the bf16 product; `conv=(conv_state, weight, bias, row0)`: the outputs [row0, row0 + C) go through
     `causal_conv1d_update` (width 4, SiLU) on conv_state (rows, C, 4), as in `gemv_fused`.  out_dtype: bf16, or fp32 without either
     (`rounded`: of the bf16 values)."""
+    if conv is None and out_dtype is None and not rounded and x.is_cuda and (r := _n.rows_linear(x, weight, bias, 1 if relu2 else 0)) is not None:
+        return r
     _gpu(x, weight, bias)
     if not rows_take(x, weight) or weight.shape[1] != x.shape[-1]:
         raise TimeViperHipError(f"rows_linear: 2..{ROWS_MAX} bf16 rows of a multiple of 64 elements, got {tuple(x.shape)} against {tuple(weight.shape)}")
@@ -873,6 +889,8 @@ GEMM_GLU = 5
 
 def small_linear(x, weight, bias=None, epilogue: int = GEMM_BIAS, out=None, tile: int = 0):
     """`linear_fused` on small tiles (tv_gemm_small_fwd): x (rows, K) bf16, weight (N, K); GEMM_GLU: the two halves of weight's rows, `glu_linear`'s result"""
+    if x.is_cuda and (r := _n.small_linear(x, weight, bias, epilogue, out, tile)) is not None:
+        return r
     _gpu(x, weight, bias, out)
     N, Kd = weight.shape
     if epilogue == GEMM_GLU:
@@ -977,6 +995,8 @@ def split_takes(x, weight, relu2=False):
 
 def split_linear(x, weight, bias=None, relu2=False, splits=1, full=0):
     """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) on tiles of 256 x 256 outputs, `splits` work-groups a tile but for the first `full`."""
+    if x.is_cuda and (r := _n.split_linear(x, weight, bias, relu2, splits, full)) is not None:
+        return r
     _gpu(x, weight, bias)
     N, Kd = weight.shape
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[-1] != Kd or weight.stride(1) != 1:
@@ -995,6 +1015,8 @@ def split_linear(x, weight, bias=None, relu2=False, splits=1, full=0):
 
 def mid_linear(x, weight, bias=None, relu2=False):
     """x @ weight.T (+ bias, then the squared ReLU of the bf16 product) for up to 256 bf16 rows (a short prompt)."""
+    if x.is_cuda and (r := _n.mid_linear(x, weight, bias, relu2)) is not None:
+        return r
     _gpu(x, weight, bias)
     N, Kd = weight.shape
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[-1] != Kd:
@@ -1435,6 +1457,10 @@ def norm_shift(x, gain, eps, pending=None, pending_weight=None, shift=None, stat
     """x (T, D) fp32 -> (x', h, hs): x' = x + rms(pending) * pending_weight (x itself without `pending`), h = rms(x') * gain (a tensor of one
     element), hs = h + (h_before - h) * shift with the h of the sequence's previous token (`state` (slots, 2, D) fp32, advanced in
     place; None without `shift`).  h and hs have the gain's dtype."""
+    if x.is_cuda:
+        steps = (None,) * 5 + (0, False) if plan is None else (plan.seq, plan.cu, plan.start, plan.slot, plan.rows, max(plan.slots, default=0), plan.decode)
+        if (r := _n.norm_shift(x, gain, eps, pending, pending_weight, shift, state, *steps, need_h)) is not None:
+            return r
     _gpu(x, gain, pending, pending_weight, shift, state)
     T, D = x.shape
     if x.dtype != torch.float32 or not x.is_contiguous() or gain.numel() != 1:
@@ -1462,6 +1488,8 @@ def norm_shift(x, gain, eps, pending=None, pending_weight=None, shift=None, stat
 
 def residual_add(x, u):
     """(x + u in fp32, its rounding to u's dtype); x (T, D) fp32"""
+    if x.is_cuda and (r := _n.residual_add(x, u)) is not None:
+        return r
     _gpu(x, u)
     if x.dtype != torch.float32 or not x.is_contiguous() or u.shape != x.shape or u.stride(1) != 1:
         raise TimeViperHipError("residual_add: dense fp32 x and u of its shape")
@@ -1569,6 +1597,8 @@ def split_add_takes(x, weight, bias=None, waits: bool = True) -> int:
 
 def split_add_linear(x, weight, residual, bias=None, splits=1):
     """(residual + x @ weight.T (+ bias) in fp32, its bf16 copy): `split_linear` with the residual stream behind it"""
+    if x.is_cuda and (r := _n.split_add_linear(x, weight, residual, bias, splits)) is not None:
+        return r
     _gpu(x, weight, residual, bias)
     N, Kd = weight.shape
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[1] != Kd or x.stride(1) != 1 or weight.stride(1) != 1 or residual.dtype != torch.float32
@@ -1598,6 +1628,8 @@ def side_takes(h, table, gate, proj, waits: bool = True) -> bool:
 
 def token_side(h, ids, table, gate, proj):
     """proj @ (gelu_tanh(gate @ h) * table[ids]) for the rows of h in one launch (tv_token_side_fwd); ids are checked where the step was planned"""
+    if h.is_cuda and (r := _n.token_side(h, ids, table, gate, proj)) is not None:
+        return r
     _gpu(h, ids, table, gate, proj)
     T, D = h.shape
     S = gate.shape[0]
@@ -1612,6 +1644,8 @@ def token_side(h, ids, table, gate, proj):
 
 def gated_mul(a, b, act, ids=None, out=None):
     """f(a) * b over rows, f = sigmoid or the tanh form of gelu; `ids` (int64): row r meets b[ids[r]].  `out`: rows to write to."""
+    if a.is_cuda and (r := _n.gated_mul(a, b, act, ids, out)) is not None:
+        return r
     _gpu(a, b, ids, out)
     T, n = a.shape
     o = torch.empty((T, n), dtype=a.dtype, device=a.device) if out is None else out
@@ -1625,6 +1659,8 @@ def gated_mul(a, b, act, ids=None, out=None):
 
 def scatter_rows(src, rows, dst):
     """dst[rows] = src (rows int32 on the GPU, within dst)"""
+    if src.is_cuda and _n.scatter_rows(src, rows, dst):
+        return
     _gpu(src, rows, dst)
     _i32(rows, src.shape[0], "scatter_rows rows")
     if src.dtype != dst.dtype or src.shape[1] != dst.shape[1] or src.stride(1) != 1 or dst.stride(1) != 1:
@@ -1708,6 +1744,9 @@ def attention_window(q, cache, plan, kv_heads, scale, window=NO_WINDOW, keep_fir
     (slots, capacity, kv_heads * (dk + dv)), a row = all keys, then all values; the query at position p sees keys (p - window, p]
     and the first `keep_first` of its sequence.  gate (T, H, dv): the result times sigmoid(gate).  out (T, H, dv).  plan: the step's
     `cache.StepPlan`."""
+    if q.is_cuda and (r := _n.attention_window(q, cache, plan.counts, plan.starts, plan.slots, kv_heads, scale, window, keep_first, gate, out,
+                                                 plan.rows, plan.seq, plan.cu, plan.start, plan.slot)) is not None:
+        return r
     T, H, dk = q.shape
     dv = cache.shape[2] // kv_heads - dk
     k, v = _cache_views(cache, kv_heads, dk, dv)
