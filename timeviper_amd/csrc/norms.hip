@@ -1,10 +1,16 @@
 // L1 / S4: RMSNorm (+fused residual add) and gated grouped RMSNorm. HBM-bound:
 // every element is read once with 16-byte accesses, kept in registers across
 // the reduction, and written once.
+// Every load of a row, the weights' among them, is issued before the first use: one round trip to memory, not three (bf16, before -> now: 203 rows x 4 480 with a
+// residual 4.1 -> 3.6 us, 12 rows 3.4 -> 3.0; gated, 12 rows x 10 240: 4.0 -> 3.0, 1 501: 18.1 -> 16.3; LayerNorm of 729 x 1 152: 4.0 -> 3.4).
+// From STREAM_FROM bytes on, what is read and written has left the caches before anyone reads it again, so that it passes by their normal replacement, and a gated
+// wave takes two rows: 4 480 wide with a residual, 10 007 rows 66.9 -> 60.3 us; gated, 10 007 rows 110 -> 86, 49 999: 515 -> 446 (6.9 TB/s).  Below, the next
+// kernel finds the results in the last-level cache: convolution, copy and gated norm of 2 200 tokens 58.6 us, streamed 60.4; of 2 600: 74.7 | 69.1.
 // Reference semantics: NemotronHRMSNorm.forward modeling_nano.py:897-903,
 // NemotronHBlock residual add :966, MambaRMSNormGated :371-380 (mamba_ssm
 // rmsnorm_fn with norm_before_gate=False).
 #include <stdlib.h>
+#include <type_traits>
 #include "common.hpp"
 
 // -DTV_NORM_SHFL (dev, A/B): the row sums on the __shfl_xor butterfly (one ds_bpermute round trip per step) instead of DPP
@@ -15,66 +21,69 @@ namespace {
 
 constexpr int NORM_THREADS = 256;
 constexpr int NORM_MAXV = 4;  // 16-byte vectors cached per thread
+constexpr int64_t STREAM_FROM = 144ll << 20;   // bytes read and written
 
-template <typename T>
-__device__ __forceinline__ float wload(const void* w, int wf32, int i) {
-  return wf32 ? ((const float*)w)[i] : to_f32(((const T*)w)[i]);
-}
-// the V weights of one 16-byte activation vector, as floats (fp32 weights: V*4 bytes = two or
-// one 16-byte loads; activation-dtype weights: one)
-template <typename T>
-__device__ __forceinline__ void wload_vec(const void* w, int wf32, int i0, float (&out)[Vec16<T>::N]) {
-  constexpr int V = Vec16<T>::N;
-  if (wf32) {
+// V fp32 or 16-bit values behind p, as loaded (16-byte loads) and as floats
+template <typename W, int V>
+struct Raw {
+  enum { PER = 16 / sizeof(W), LOADS = V * sizeof(W) / 16 };
+  typename Vec16<W>::type v[LOADS];
+  __device__ __forceinline__ void load(const W* p) {
 #pragma unroll
-    for (int q = 0; q < V / 4; ++q) {
-      const f32x4 v = *(const f32x4*)((const float*)w + i0 + 4 * q);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[4 * q + i] = v[i];
-    }
-  } else {
-    const typename Vec16<T>::type v = *(const typename Vec16<T>::type*)((const T*)w + i0);
-#pragma unroll
-    for (int i = 0; i < V; ++i) out[i] = to_f32(v[i]);
+    for (int q = 0; q < LOADS; ++q) v[q] = *(const typename Vec16<W>::type*)(p + q * PER);
   }
+  __device__ __forceinline__ float operator[](int i) const { return to_f32(v[i / PER][i % PER]); }
+};
+template <bool NT, typename vec_t> __device__ __forceinline__ vec_t get(const void* p) {
+  return NT ? __builtin_nontemporal_load((const vec_t*)p) : *(const vec_t*)p;
+}
+template <bool NT, typename vec_t> __device__ __forceinline__ void put(void* p, vec_t v) {
+  if (NT) __builtin_nontemporal_store(v, (vec_t*)p);
+  else *(vec_t*)p = v;
 }
 
-template <typename T>
+// A work-group a row; NV 16-byte vectors a thread, all of them and their weights in flight before the first use
+template <typename T, typename W, int NV, bool DELTA, bool STREAM>
 __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_kernel(
-    const T* __restrict__ x, const T* __restrict__ delta, const void* __restrict__ w,
-    T* __restrict__ sum_out, T* __restrict__ y, int D, int64_t xs, int64_t ds, int64_t ss,
-    int64_t ys, float eps, int wf32) {
+    const T* __restrict__ x, const T* __restrict__ delta, const W* __restrict__ w,
+    T* __restrict__ sum_out, T* __restrict__ y, int nv, int64_t xs, int64_t ds, int64_t ss,
+    int64_t ys, float eps) {
   constexpr int V = Vec16<T>::N;
   typedef typename Vec16<T>::type vec_t;
   __shared__ float red[NORM_THREADS / 64];
   const int64_t row = blockIdx.x;
-  const int nv = D / V;
   const T* xr = x + row * xs;
-  const T* dr = delta ? delta + row * ds : nullptr;
-  float vals[NORM_MAXV][V];
-  float ssq = 0.f;
+  const T* dr = DELTA ? delta + row * ds : nullptr;
+  vec_t xv[NV], dv[DELTA ? NV : 1];
+  Raw<W, V> wv[NV];
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
+  for (int k = 0; k < NV; ++k) {
     const int iv = threadIdx.x + k * NORM_THREADS;
     if (iv < nv) {
-      vec_t v = *(const vec_t*)(xr + (int64_t)iv * V);
-      if (dr) {
-        vec_t d = *(const vec_t*)(dr + (int64_t)iv * V);
-        vec_t sv;
+      xv[k] = get<STREAM, vec_t>(xr + (int64_t)iv * V);
+      if constexpr (DELTA) dv[k] = get<STREAM, vec_t>(dr + (int64_t)iv * V);
+    }
+  }
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-          // the reference adds in the activation dtype: round, then normalise
-          sv[i] = from_f32<T>(to_f32(v[i]) + to_f32(d[i]));
-          vals[k][i] = to_f32(sv[i]);
-        }
-        if (sum_out) *(vec_t*)(sum_out + row * ss + (int64_t)iv * V) = sv;
-      } else {
+  for (int k = 0; k < NV; ++k) {
+    const int iv = threadIdx.x + k * NORM_THREADS;
+    if (iv < nv) wv[k].load(w + (int64_t)iv * V);
+  }
+  float vals[NV][V];
+  float ssq = 0.f;
 #pragma unroll
-        for (int i = 0; i < V; ++i) vals[k][i] = to_f32(v[i]);
-        if (sum_out) *(vec_t*)(sum_out + row * ss + (int64_t)iv * V) = v;
+  for (int k = 0; k < NV; ++k) {
+    const int iv = threadIdx.x + k * NORM_THREADS;
+    if (iv < nv) {
+      vec_t sv = xv[k];
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        // the reference adds in the activation dtype: round, then normalise
+        if constexpr (DELTA) sv[i] = from_f32<T>(to_f32(xv[k][i]) + to_f32(dv[k][i]));
+        vals[k][i] = to_f32(sv[i]);
+        ssq = fmaf(vals[k][i], vals[k][i], ssq);
       }
-#pragma unroll
-      for (int i = 0; i < V; ++i) ssq = fmaf(vals[k][i], vals[k][i], ssq);
+      if (sum_out) put<STREAM>(sum_out + row * ss + (int64_t)iv * V, sv);
     }
   }
   ssq = wave_sum_dpp(ssq);
@@ -83,17 +92,15 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_kernel(
   float tot = 0.f;
 #pragma unroll
   for (int i = 0; i < NORM_THREADS / 64; ++i) tot += red[i];
-  const float rstd = rsqrtf(tot / (float)D + eps);
+  const float rstd = rsqrtf(tot / (float)(nv * V) + eps);
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
+  for (int k = 0; k < NV; ++k) {
     const int iv = threadIdx.x + k * NORM_THREADS;
     if (iv < nv) {
       vec_t o;
-      float wv[V];
-      wload_vec<T>(w, wf32, iv * V, wv);
 #pragma unroll
-      for (int i = 0; i < V; ++i) o[i] = from_f32<T>(wv[i] * (vals[k][i] * rstd));
-      *(vec_t*)(y + row * ys + (int64_t)iv * V) = o;
+      for (int i = 0; i < V; ++i) o[i] = from_f32<T>(wv[k][i] * (vals[k][i] * rstd));
+      put<STREAM>(y + row * ys + (int64_t)iv * V, o);
     }
   }
 }
@@ -181,80 +188,90 @@ __global__ __launch_bounds__(NORM_THREADS) void layernorm_kernel(
 }
 
 // Rows of up to 64 * NORM_MAXV vectors (ViT widths): one WAVE per row — no LDS, no block
-// barrier, four rows in flight per workgroup, every load issued before the first use.
-template <typename T>
+// barrier, four rows in flight per workgroup; NV 16-byte vectors a lane, every load issued before the first use - the parameters' too (EARLY), but where
+// many rows have a second operand: its registers then cost a wave (8 000 x 1 152: 15.2 us late, 17.2 early; 1 458: 5.6 | 5.1).
+template <typename T, int NV, bool DELTA, bool EARLY>
 __global__ __launch_bounds__(NORM_THREADS) void layernorm_wave_kernel(
     const T* __restrict__ x, const T* __restrict__ delta, const T* __restrict__ w,
     const T* __restrict__ bias, const float* __restrict__ row_bias, T* __restrict__ sum_out,
-    T* __restrict__ y, int64_t rows, int D, int64_t xs, int64_t ds, int64_t ss, int64_t ys, float eps) {
+    T* __restrict__ y, int64_t rows, int nv, int64_t xs, int64_t ds, int64_t ss, int64_t ys, float eps) {
   constexpr int V = Vec16<T>::N;
   typedef typename Vec16<T>::type vec_t;
   const int64_t row = (int64_t)blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
-  const int nv = D / V;
+  const float D = (float)(nv * V);
   const T* xr = x + row * xs;
-  const T* dr = delta ? delta + row * ds : nullptr;
-  vec_t xv[NORM_MAXV], dv[NORM_MAXV];
+  const T* dr = DELTA ? delta + row * ds : nullptr;
+  vec_t xv[NV], dv[DELTA ? NV : 1], wv[NV], bv[NV];
+  Raw<float, V> rb[NV];
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
+  for (int k = 0; k < NV; ++k) {
     const int iv = lane + k * 64;
     if (iv < nv) {
       xv[k] = *(const vec_t*)(xr + (int64_t)iv * V);
-      if (dr) dv[k] = *(const vec_t*)(dr + (int64_t)iv * V);
+      if constexpr (DELTA) dv[k] = *(const vec_t*)(dr + (int64_t)iv * V);
     }
   }
-  float vals[NORM_MAXV][V];
+  if (row_bias) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (lane + k * 64 < nv) rb[k].load(row_bias + (int64_t)(lane + k * 64) * V);
+  }
+  const auto parameters = [&] {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int iv = lane + k * 64;
+      bv[k] = vec_t{};
+      if (iv < nv) {
+        wv[k] = *(const vec_t*)(w + (int64_t)iv * V);
+        if (bias) bv[k] = *(const vec_t*)(bias + (int64_t)iv * V);
+      }
+    }
+  };
+  if constexpr (EARLY) parameters();
+  float vals[NV][V];
   float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
+  for (int k = 0; k < NV; ++k) {
     const int iv = lane + k * 64;
     if (iv < nv) {
-      if (dr) {
-        vec_t sv;
+      vec_t sv = xv[k];
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-          sv[i] = from_f32<T>(to_f32(xv[k][i]) + to_f32(dv[k][i]));
-          vals[k][i] = to_f32(sv[i]);
-        }
-        if (sum_out) *(vec_t*)(sum_out + row * ss + (int64_t)iv * V) = sv;
-      } else {
-#pragma unroll
-        for (int i = 0; i < V; ++i) vals[k][i] = to_f32(xv[k][i]);
+      for (int i = 0; i < V; ++i) {
+        if constexpr (DELTA) sv[i] = from_f32<T>(to_f32(xv[k][i]) + to_f32(dv[k][i]));
+        vals[k][i] = to_f32(sv[i]);
       }
+      if (DELTA && sum_out) *(vec_t*)(sum_out + row * ss + (int64_t)iv * V) = sv;
       if (row_bias) {
 #pragma unroll
-        for (int i = 0; i < V; ++i) vals[k][i] += row_bias[(int64_t)iv * V + i];
+        for (int i = 0; i < V; ++i) vals[k][i] += rb[k][i];
       }
 #pragma unroll
       for (int i = 0; i < V; ++i) s1 += vals[k][i];
     }
   }
   s1 = wave_sum_dpp(s1);
-  const float mean = s1 / (float)D;
+  const float mean = s1 / D;
   // second register pass: sum of squared deviations (no E[x^2] - mean^2 cancellation)
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
-    const int iv = lane + k * 64;
-    if (iv < nv) {
+  for (int k = 0; k < NV; ++k) {
+    if (lane + k * 64 < nv) {
 #pragma unroll
       for (int i = 0; i < V; ++i) { const float d = vals[k][i] - mean; s2 = fmaf(d, d, s2); }
     }
   }
   s2 = wave_sum_dpp(s2);
-  const float var = s2 / (float)D;
-  const float rstd = rsqrtf(var + eps);
+  const float rstd = rsqrtf(s2 / D + eps);
+  if constexpr (!EARLY) parameters();
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
+  for (int k = 0; k < NV; ++k) {
     const int iv = lane + k * 64;
     if (iv < nv) {
-      const vec_t wv = *(const vec_t*)(w + (int64_t)iv * V);
-      vec_t bv = {};
-      if (bias) bv = *(const vec_t*)(bias + (int64_t)iv * V);
       vec_t o;
 #pragma unroll
       for (int i = 0; i < V; ++i)
-        o[i] = from_f32<T>((vals[k][i] - mean) * rstd * to_f32(wv[i]) + to_f32(bv[i]));
+        o[i] = from_f32<T>((vals[k][i] - mean) * rstd * to_f32(wv[k][i]) + to_f32(bv[k][i]));
       *(vec_t*)(y + row * ys + (int64_t)iv * V) = o;
     }
   }
@@ -272,11 +289,11 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 
     T* __restrict__ y, int64_t rows, int D, int64_t xs, int64_t ds, int64_t ss, int64_t ys, float eps) {
   constexpr int V = Vec16<T>::N;
   typedef typename Vec16<T>::type vec_t;
-  const int64_t row0 = ((int64_t)blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6)) * RPW;
-  if (row0 >= rows) return;
+  const int64_t chunk = (rows + RPW - 1) / RPW, row0 = (int64_t)blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6);
+  if (row0 >= chunk) return;
+  const int nrow = (int)((rows - row0 + chunk - 1) / chunk);
   const int lane = threadIdx.x & 63;
   const int nv = D / V;
-  const int nrow = (int)(rows - row0 < RPW ? rows - row0 : RPW);
   vec_t wv[NV], bv[NV];
   float rb[NV][V];
 #pragma unroll
@@ -306,15 +323,15 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 
     for (int k = 0; k < NV; ++k) {
       const int iv = lane + k * 64;
       if (iv < nv) {
-        xo[k] = *(const vec_t*)(x + row * xs + (int64_t)iv * V);
+        xo[k] = get<true, vec_t>(x + row * xs + (int64_t)iv * V);
         if (DELTA) dd[k % NVD] = *(const vec_t*)(delta + row * ds + (int64_t)iv * V);
       }
     }
   };
   load_row(row0, xv, dv);
   for (int r = 0; r < nrow; ++r) {
-    const int64_t row = row0 + r;
-    if (r + 1 < nrow) load_row(row + 1, xn, dn);
+    const int64_t row = row0 + r * chunk;
+    if (r + 1 < nrow) load_row(row + chunk, xn, dn);
     float vals[NV][V];
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -360,7 +377,7 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 
 #pragma unroll
         for (int i = 0; i < V; ++i)
           o[i] = from_f32<T>((vals[k][i] - mean) * rstd * to_f32(wv[k][i]) + to_f32(bv[k][i]));
-        *(vec_t*)(y + row * ys + (int64_t)iv * V) = o;
+        put<true>(y + row * ys + (int64_t)iv * V, o);
       }
     }
 #pragma unroll
@@ -433,66 +450,88 @@ __global__ __launch_bounds__(256) void gelu_kernel(const T* __restrict__ x, T* _
   }
 }
 
-// one wave per (row, group)
-template <typename T>
+// A wave a group of ROWS rows that lie `chunk` rows apart; NV 16-byte vectors a lane and row, all of them and the weights in flight before the first use
+template <typename T, typename W, int NV, bool GATE, bool STREAM>
 __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_gated_kernel(
-    const T* __restrict__ x, const T* __restrict__ z, const void* __restrict__ w,
-    T* __restrict__ y, int64_t rows, int D, int gsz, int64_t xs, int64_t zs, int64_t ys,
-    float eps, int wf32) {
-  constexpr int V = Vec16<T>::N;
+    const T* __restrict__ x, const T* __restrict__ z, const W* __restrict__ w,
+    T* __restrict__ y, int64_t rows, int64_t chunk, unsigned ngroups, int nv, int64_t xs, int64_t zs, int64_t ys,
+    float eps) {
+  constexpr int V = Vec16<T>::N, ROWS = STREAM ? 2 : 1;
   typedef typename Vec16<T>::type vec_t;
-  const int ngroups = D / gsz;
-  const int64_t wid = (int64_t)blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6);
-  if (wid >= rows * ngroups) return;
-  const int64_t row = wid / ngroups;
-  const int g = (int)(wid % ngroups);
+  // (a grid has fewer than 2^32 threads)
+  const unsigned wid = blockIdx.x * (NORM_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = wid / ngroups;
+  if (row0 >= chunk) return;
   const int lane = threadIdx.x & 63;
-  const int nv = gsz / V;
-  const T* xr = x + row * xs + (int64_t)g * gsz;
-  const T* zr = z ? z + row * zs + (int64_t)g * gsz : nullptr;
-  // every load of the (row, group) is issued before the first use
-  vec_t xv[NORM_MAXV], zv[NORM_MAXV];
+  const int64_t c0 = (int64_t)(wid % ngroups) * nv * V + lane * V;
+  vec_t xv[ROWS][NV], zv[ROWS][GATE ? NV : 1];
+  Raw<W, V> wv[NV];
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
-    const int iv = lane + k * 64;
-    if (iv < nv) {
-      xv[k] = *(const vec_t*)(xr + (int64_t)iv * V);
-      if (zr) zv[k] = *(const vec_t*)(zr + (int64_t)iv * V);
-    }
-  }
-  float vals[NORM_MAXV][V];
-  float ssq = 0.f;
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t row = row0 + r * chunk;
+    if (row < rows) {
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
-    const int iv = lane + k * 64;
-    if (iv < nv) {
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        float v = to_f32(xv[k][i]);
-        if (zr) {   // x * silu(z), sigmoid through the hardware reciprocal
-          const float g = to_f32(zv[k][i]);
-          v *= g * __builtin_amdgcn_rcpf(1.f + __expf(-g));
+      for (int k = 0; k < NV; ++k) {
+        if (lane + k * 64 < nv) {
+          xv[r][k] = get<STREAM, vec_t>(x + row * xs + c0 + k * 64 * V);
+          if constexpr (GATE) zv[r][k] = get<STREAM, vec_t>(z + row * zs + c0 + k * 64 * V);
         }
-        vals[k][i] = v;
-        ssq = fmaf(v, v, ssq);
       }
     }
   }
-  ssq = wave_sum_dpp(ssq);
-  const float rstd = rsqrtf(ssq / (float)gsz + eps);
-  T* yr = y + row * ys + (int64_t)g * gsz;
 #pragma unroll
-  for (int k = 0; k < NORM_MAXV; ++k) {
-    const int iv = lane + k * 64;
-    if (iv < nv) {
-      vec_t o;
-      float wv[V];
-      wload_vec<T>(w, wf32, g * gsz + iv * V, wv);
+  for (int k = 0; k < NV; ++k)
+    if (lane + k * 64 < nv) wv[k].load(w + c0 + k * 64 * V);
 #pragma unroll
-      for (int i = 0; i < V; ++i) o[i] = from_f32<T>(wv[i] * (vals[k][i] * rstd));
-      *(vec_t*)(yr + (int64_t)iv * V) = o;
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t row = row0 + r * chunk;
+    if (row >= rows) break;
+    float vals[NV][V];
+    float ssq = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (lane + k * 64 < nv) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          float v = to_f32(xv[r][k][i]);
+          if constexpr (GATE) {   // x * silu(z), sigmoid through the hardware reciprocal
+            const float g = to_f32(zv[r][k][i]);
+            v *= g * __builtin_amdgcn_rcpf(1.f + __expf(-g));
+          }
+          vals[k][i] = v;
+          ssq = fmaf(v, v, ssq);
+        }
+      }
+    }
+    ssq = wave_sum_dpp(ssq);
+    const float rstd = rsqrtf(ssq / (float)(nv * V) + eps);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (lane + k * 64 < nv) {
+        vec_t o;
+#pragma unroll
+        for (int i = 0; i < V; ++i) o[i] = from_f32<T>(wv[k][i] * (vals[k][i] * rstd));
+        put<STREAM>(y + row * ys + c0 + k * 64 * V, o);
+      }
     }
   }
+}
+
+// f(std::integral_constant<int, n>): n = the vectors a thread of `threads` for nv, 1 .. NORM_MAXV
+template <typename F>
+void with_vectors(int nv, int threads, F f) {
+  switch ((nv + threads - 1) / threads) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    default: return f(std::integral_constant<int, 4>{});
+  }
+}
+// the weights' type: T's or fp32
+template <typename T, typename F>
+void with_weights(const void* w, int wf32, F f) {
+  if (wf32) f((const float*)w);
+  else f((const T*)w);
 }
 
 template <typename T>
@@ -503,8 +542,18 @@ int launch_rms(const void* x, const void* delta, const void* w, void* sum_out, v
   if (D % V || D / V > NORM_THREADS * NORM_MAXV)
     TV_UNSUPPORTED("rmsnorm: dim %d not a multiple of %d or larger than %d", D, V,
                    V * NORM_THREADS * NORM_MAXV);
-  rmsnorm_kernel<T><<<dim3((unsigned)rows), NORM_THREADS, 0, s>>>(
-      (const T*)x, (const T*)delta, w, (T*)sum_out, (T*)y, D, xs, ds, ss, ys, eps, wf32);
+  const bool stream = rows * D * (int64_t)sizeof(T) * (2 + (delta != nullptr) + (sum_out != nullptr)) >= STREAM_FROM;
+  with_vectors(D / V, NORM_THREADS, [&](auto nv) {
+    with_weights<T>(w, wf32, [&](auto wp) {
+      typedef std::remove_cv_t<std::remove_pointer_t<decltype(wp)>> W;
+#define TV_RMS(DELTA, STREAM)                                                                                                                        \
+  rmsnorm_kernel<T, W, nv(), DELTA, STREAM><<<dim3((unsigned)rows), NORM_THREADS, 0, s>>>((const T*)x, (const T*)delta, wp, (T*)sum_out, (T*)y, D / V, \
+                                                                                          xs, ds, ss, ys, eps)
+      if (stream) { if (delta) TV_RMS(true, true); else TV_RMS(false, true); }
+      else { if (delta) TV_RMS(true, false); else TV_RMS(false, false); }
+#undef TV_RMS
+    });
+  });
   TV_LAUNCH_CHECK();
 }
 
@@ -516,10 +565,21 @@ int launch_gated(const void* x, const void* z, const void* w, void* y, int64_t r
   if (gsz % V || gsz / V > 64 * NORM_MAXV)
     TV_UNSUPPORTED("rmsnorm_gated: group_size %d not a multiple of %d or larger than %d", gsz,
                    V, V * 64 * NORM_MAXV);
-  const int64_t nwaves = rows * (D / gsz);
-  const int64_t nblk = (nwaves + NORM_THREADS / 64 - 1) / (NORM_THREADS / 64);
-  rmsnorm_gated_kernel<T><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(
-      (const T*)x, (const T*)z, w, (T*)y, rows, D, gsz, xs, zs, ys, eps, wf32);
+  const int ngroups = D / gsz;
+  const bool stream = rows * D * (int64_t)sizeof(T) * (z ? 3 : 2) >= STREAM_FROM;
+  const int64_t chunk = stream ? (rows + 1) / 2 : rows;
+  const unsigned nblk = (unsigned)((chunk * ngroups + NORM_THREADS / 64 - 1) / (NORM_THREADS / 64));
+  with_vectors(gsz / V, 64, [&](auto nv) {
+    with_weights<T>(w, wf32, [&](auto wp) {
+      typedef std::remove_cv_t<std::remove_pointer_t<decltype(wp)>> W;
+#define TV_GATED(GATE, STREAM)                                                                                                              \
+  rmsnorm_gated_kernel<T, W, nv(), GATE, STREAM><<<dim3(nblk), NORM_THREADS, 0, s>>>((const T*)x, (const T*)z, wp, (T*)y, rows, chunk, \
+                                                                                      (unsigned)ngroups, gsz / V, xs, zs, ys, eps)
+      if (stream) { if (z) TV_GATED(true, true); else TV_GATED(false, true); }
+      else { if (z) TV_GATED(true, false); else TV_GATED(false, false); }
+#undef TV_GATED
+    });
+  });
   TV_LAUNCH_CHECK();
 }
 
@@ -538,22 +598,28 @@ int launch_ln(const void* x, const void* delta, const void* w, const void* b, co
   if (D / V <= 64 * NORM_MAXV && rows >= 4096 * RPW && !rows_off && !delta) {
     // many rows (the ViT's stream form: row bias, no residual operand): a wave keeps the parameters in registers for RPW
     // rows — 1 272 against 1 416 us per 1.49 M rows x 1 152 (5.41 against 4.86 TB/s); with a residual operand the
-    // one-row kernel is the faster one (2 502 against 2 654 us: the second operand's registers cost a wave per SIMD)
+    // one-row kernel is the faster one (2 502 against 2 654 us: the second operand's registers cost a wave per SIMD).
+    // A wave's rows lie rows / RPW apart, so that all waves together read one front of memory, and past the caches' normal
+    // replacement: 34 992 x 1 152 35.6 -> 32.5 us (apart alone 35.0, normal stores 33.9), 200 000: 171 -> 156
     const int64_t nblk = (rows + (NORM_THREADS / 64) * RPW - 1) / ((NORM_THREADS / 64) * RPW);
-    const int nvl = (D / V + 63) / 64;
 #define TV_LN_ROWS(NV)                                                                                              \
     layernorm_rows_kernel<T, NV, RPW, false><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                         \
         (const T*)x, nullptr, (const T*)w, (const T*)b, rb, (T*)sum_out, (T*)y, rows, D, xs, ds, ss, ys, eps)
-    if (nvl == 1) TV_LN_ROWS(1);
-    else if (nvl == 2) TV_LN_ROWS(2);
-    else if (nvl == 3) TV_LN_ROWS(3);
-    else TV_LN_ROWS(4);
+    with_vectors(D / V, 64, [&](auto nv) {
+      TV_LN_ROWS(nv());
+    });
 #undef TV_LN_ROWS
   } else if (D / V <= 64 * NORM_MAXV) {
     const int64_t nblk = (rows + NORM_THREADS / 64 - 1) / (NORM_THREADS / 64);
-    layernorm_wave_kernel<T><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(
-        (const T*)x, (const T*)delta, (const T*)w, (const T*)b, rb, (T*)sum_out, (T*)y, rows, D, xs, ds, ss,
-        ys, eps);
+    with_vectors(D / V, 64, [&](auto nv) {
+#define TV_LN_WAVE(DELTA, EARLY)                                                                                    \
+  layernorm_wave_kernel<T, nv(), DELTA, EARLY><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                     \
+      (const T*)x, (const T*)delta, (const T*)w, (const T*)b, rb, (T*)sum_out, (T*)y, rows, D / V, xs, ds, ss, ys, eps)
+      if (!delta) TV_LN_WAVE(false, true);
+      else if (rows < 4096) TV_LN_WAVE(true, true);
+      else TV_LN_WAVE(true, false);
+#undef TV_LN_WAVE
+    });
   } else {
     layernorm_kernel<T><<<dim3((unsigned)rows), NORM_THREADS, 0, s>>>(
         (const T*)x, (const T*)delta, (const T*)w, (const T*)b, rb, (T*)sum_out, (T*)y, D, xs, ds, ss, ys, eps);
