@@ -33,10 +33,33 @@ __device__ __forceinline__ float rdlane(float v, int l) { return __int_as_float(
 __device__ __forceinline__ float from_lane(float v, int l) { return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * l, __float_as_int(v))); }
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// OUT: the second launch
-template <bool OUT>
+// inclusive sums over the lanes as value + what its rounding lost (an infinite sum has lost nothing)
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ void scan_step(float& hi, float& lo) {
+  const float b = dpp_shift<CTRL, ROWMASK>(hi), bl = dpp_shift<CTRL, ROWMASK>(lo);
+  const float s = hi + b, bb = s - hi;
+  lo = (lo + bl) + ((hi - (s - bb)) + (b - bb));
+  hi = s;
+}
+__device__ __forceinline__ float scan_both(float v, float& lost) {
+  lost = 0.f;
+  scan_step<0x111, 0xf>(v, lost);   // row_shr:1
+  scan_step<0x112, 0xf>(v, lost);   // row_shr:2
+  scan_step<0x114, 0xf>(v, lost);   // row_shr:4
+  scan_step<0x118, 0xf>(v, lost);   // row_shr:8
+  scan_step<0x142, 0xa>(v, lost);   // row_bcast:15 -> rows 1, 3
+  scan_step<0x143, 0xc>(v, lost);   // row_bcast:31 -> rows 2, 3
+  lost = fabsf(v) < INFINITY ? lost : 0.f;
+  return v;
+}
+
+// OUT: the second launch.  FINE: for the lengths that the token recurrence had before (48 - 64 tokens, more than 4 096), whose error is kept: two tokens' decay is the difference
+// of their sums AND of what these have lost (a sum over a chunk is rounded by its own size, not by the difference's), B has dt, and the sums of 16 are two of 8 and one a
+// tile.  Error of y against 64 bits, before these | with them | recurrence: 64 tokens that decay by e^-50 5.6e-7 | 1.0e-7 | 0.9e-7, slowly 1.7e-7 | 1.0e-7 | 1.9e-7; with a
+// mixer's inputs 64 tokens 3.1e-8 | 3.1e-8, 6 000: 3.0e-8 | 3.2e-8 (with | recurrence).  They take 1 - 4 % (2 x 4 096 tokens 85 -> 88.5 us): the lengths between are as they were.
+template <bool OUT, bool FINE>
 __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
-  __shared__ __attribute__((aligned(16))) float sv[4][3][FQ];         // a wave's own: cs, dt, weights of the state
+  __shared__ __attribute__((aligned(16))) float sv[4][FINE ? 4 : 3][FQ];         // a wave's own: cs, dt, weights of the state, what cs has lost
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lc = lane & 15, q = lane >> 4;
   const int pt_n = a.P >> 4, unit = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
@@ -100,12 +123,14 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
     float d = raw + bias;
     if (a.softplus) d = softplus_f(d);
     d = lane < tt ? fminf(fmaxf(d, a.dt_min), a.dt_max) : 0.f;
-    const float da = d * Ah, cs = wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
+    float lost = 0.f;
+    const float da = d * Ah, cs = FINE ? scan_both(da, lost) : wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
     // what decays behind a token, summed from the end: cend - cs would carry the rounding of the whole chunk's sum into the tokens that weigh most
     const float back = from_lane(wave_incl_scan_dpp(from_lane(da, 63 - lane)), 62 - lane);
     own += cend;
     sv[wave][0][lane] = cs;
     sv[wave][1][lane] = d;
+    if constexpr (FINE) sv[wave][3][lane] = lost;
     sv[wave][2][lane] = lane == 63 ? d : __expf(back) * d;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (a wave's own LDS: in order)
     if (tt < FQ) {                                                    // rows past the end are zeros, as tokens that are not there
@@ -124,15 +149,17 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) zero[r] = fmaf(xa[st][r], 0.f, zero[r]);
       const bool odd = __ballot(zero[0] + zero[1] + (zero[2] + zero[3]) != 0.f) != 0;
-      f32x4 css[4], ds[4];
+      f32x4 css[4], ds[4], cls[4];
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         css[st] = *(const f32x4*)&sv[wave][0][16 * st + 4 * q];
-        ds[st] = *(const f32x4*)&sv[wave][1][16 * st + 4 * q];
+        if constexpr (FINE) cls[st] = *(const f32x4*)&sv[wave][3][16 * st + 4 * q];
+        if constexpr (!FINE) ds[st] = *(const f32x4*)&sv[wave][1][16 * st + 4 * q];
+        else ba[st] *= sv[wave][1][16 * st + lc];
       }
 #pragma unroll
       for (int ot = 0; ot < 4; ++ot) {                                // 16 output tokens
-        const float cst = sv[wave][0][16 * ot + lc], et = __expf(cst);
+        const float cst = sv[wave][0][16 * ot + lc], clt = FINE ? sv[wave][FINE ? 3 : 0][16 * ot + lc] : 0.f, et = __expf(cst);
         f32x4 Y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 4; ++k) Y = mfma4(S[k], ca[ot][k], Y);
@@ -141,11 +168,20 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
 #pragma unroll
         for (int st = 0; st <= ot; ++st) {
           f32x4 M = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (FINE) {
+            f32x4 M1 = M;
+            M = mfma4(ba[st][1], ca[ot][1], mfma4(ba[st][0], ca[ot][0], M));
+            M1 = mfma4(ba[st][3], ca[ot][3], mfma4(ba[st][2], ca[ot][2], M1));
+            M += M1;
+          } else {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) M = mfma4(ba[st][k], ca[ot][k], M);
+            for (int k = 0; k < 4; ++k) M = mfma4(ba[st][k], ca[ot][k], M);
+          }
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float m = __expf(cst - css[st][r]) * ds[st][r] * M[r];
+            float gap = cst - css[st][r];
+            if constexpr (FINE) gap += clt - cls[st][r];
+            const float m = FINE ? __expf(gap) * M[r] : __expf(gap) * ds[st][r] * M[r];
             M[r] = st < ot || 4 * q + r <= lc ? m : 0.f;
           }
           if (st == ot && odd) {
@@ -160,8 +196,12 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
               }
             }
           } else {
+            f32x4 Z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Y = mfma4(xa[st][r], M[r], Y);
+            for (int r = 0; r < 4; ++r)
+              if constexpr (FINE) Z = mfma4(xa[st][r], M[r], Z);
+              else Y = mfma4(xa[st][r], M[r], Y);
+            if constexpr (FINE) Y += Z;
           }
         }
         if (16 * ot + lc < tt) {
@@ -194,9 +234,23 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
   }
 }
 
+// chunks a segment: two waves a SIMD (one: 2 x 4 096 tokens 92 | 105 us, four: 93, 2 x 1 024: 31 | 35, 36), at most 64 segments (the fold keeps a segment's decay a lane)
+int chunks_a_segment(int batch, int nch, int nheads, int headdim) {
+  const int64_t waves = (int64_t)batch * nheads * (headdim / 16) * nch;
+  int64_t len = waves / (8ll * tv_cu_count());
+  if (len < (nch + 63) / 64) len = (nch + 63) / 64;
+  return (int)(len < 1 ? 1 : len > nch ? nch : len);
+}
+
 }  // namespace
 
-// called from ssd_chunked.hip: fp32 shapes whose rows are read and written in 16-byte pieces
+size_t tv_ssd_f32_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate) {
+  if (dstate != FN || headdim % 16 || batch <= 0 || seqlen <= 0 || nheads <= 0) return 0;
+  const int nch = (seqlen + FQ - 1) / FQ, len = chunks_a_segment(batch, nch, nheads, headdim), nseg = (nch + len - 1) / len;
+  return nseg == 1 ? 0 : (size_t)nseg * batch * nheads * ((size_t)headdim * FN + 1) * sizeof(float);
+}
+
+// called from ssd_chunked.hip and, beyond its lengths, from ssd_scan.hip: fp32 shapes whose rows are read and written in 16-byte pieces
 bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
                           int64_t ysb, int64_t ysl, const void* x, const void* Bm, const void* Cm, const void* y, const void* init,
                           const void* final_state) {
@@ -208,23 +262,22 @@ bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int
 int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias,
                       const void* init_state, void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups,
                       int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
-                      int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map, void* workspace, hipStream_t st) {
+                      int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, void* workspace, hipStream_t st) {
   F3Args a;
   a.x = (const float*)x; a.dt = (const float*)dt; a.Bm = (const float*)Bm; a.Cm = (const float*)Cm; a.A = (const float*)A; a.D = (const float*)D;
   a.dt_bias = (const float*)dt_bias; a.init = (const float*)init_state; a.y = (float*)y; a.final_state = (float*)final_state;
   a.total_decay = (float*)total_decay;
   a.L = seqlen; a.H = nheads; a.P = headdim; a.G = ngroups; a.nch = (seqlen + FQ - 1) / FQ;
-  const int64_t waves = (int64_t)batch * nheads * (headdim / 16) * a.nch;
-  int64_t len = waves / (8ll * tv_cu_count());                        // (two waves a SIMD; one: 2 x 4 096 tokens 92 | 105 us, four: 93, 2 x 1 024: 31 | 35, 36)
-  if (len < (a.nch + 63) / 64) len = (a.nch + 63) / 64;               // (the fold keeps a segment's decay a lane)
-  a.seg_chunks = (int)(len < 1 ? 1 : len > a.nch ? a.nch : len);
+  a.seg_chunks = chunks_a_segment(batch, a.nch, nheads, headdim);
   a.nseg = (a.nch + a.seg_chunks - 1) / a.seg_chunks;
   a.loc = (float*)workspace;
   a.segdec = a.loc + (int64_t)a.nseg * batch * nheads * headdim * FN;
   a.xsb = xsb; a.xsl = xsl; a.dsb = dsb; a.dsl = dsl; a.bsb = bsb; a.bsl = bsl; a.bsg = bsg; a.csb = csb; a.csl = csl; a.csg = csg; a.ysb = ysb; a.ysl = ysl;
   a.softplus = dt_softplus; a.group_map = group_map; a.dt_min = dt_min; a.dt_max = dt_max;
   const int units = headdim / 16 * a.nseg;
-  if (a.nseg > 1) ssd_f32_kernel<false><<<dim3((unsigned)((units - headdim / 16 + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
-  ssd_f32_kernel<true><<<dim3((unsigned)((units + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
+  if (a.nseg > 1) ssd_f32_kernel<false, false><<<dim3((unsigned)((units - headdim / 16 + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
+  const dim3 grid((unsigned)((units + 3) / 4), (unsigned)nheads, (unsigned)batch);
+  if (fine) ssd_f32_kernel<true, true><<<grid, 256, 0, st>>>(a);
+  else ssd_f32_kernel<true, false><<<grid, 256, 0, st>>>(a);
   TV_LAUNCH_CHECK();
 }

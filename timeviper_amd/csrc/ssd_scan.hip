@@ -29,6 +29,13 @@ int tv_ssd_slice_launch(const void* x, const void* dt, const void* A, const void
                         void* workspace, size_t workspace_bytes, int wide, const void* cb_pre, hipStream_t st);
 
 // ssd_chunked.hip: the generic path's chunk-parallel form (small d_state, any dtype)
+bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
+                          int64_t ysb, int64_t ysl, const void* x, const void* Bm, const void* Cm, const void* y, const void* init, const void* final_state);
+int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias, const void* init_state,
+                      void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups, int64_t xsb, int64_t xsl,
+                      int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl,
+                      int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, void* workspace, hipStream_t st);
+size_t tv_ssd_f32_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate);
 bool tv_ssd_chunked_supported(int seqlen, int headdim, int dstate);
 size_t tv_ssd_chunked_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate);
 int tv_ssd_chunked_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D,
@@ -63,6 +70,7 @@ int tv_ssd_head_launch(const void* x, const void* dt, const void* A, const void*
 // means 4), 7 (a head march with two waves a SIMD; now means 6).
 // process-wide override for tests / dev tools; atomic so that concurrent callers never race on it
 static std::atomic<int> g_ssd_impl{0};
+constexpr int F32_FROM = 48;          // tokens
 static const int kAutoImpl = 6;   // head-per-wave march; falls back to 4, 3, the generic path
 
 extern "C" void tv_ssd_scan_set_impl(int impl) { g_ssd_impl.store(impl, std::memory_order_relaxed); }
@@ -78,8 +86,11 @@ static void ran_on(int impl, int kernel) {
 
 extern "C" size_t tv_ssd_scan_workspace_bytes(int batch, int seqlen, int nheads, int headdim,
                                               int ngroups, int dstate, int dtype) {
-  if (dtype != TV_BF16 || dstate != 128)
-    return (tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate) + 255) / 256 * 256;
+  if (dtype != TV_BF16 || dstate != 128) {
+    const size_t chunked = tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate);
+    const size_t f32 = dtype == TV_F32 ? tv_ssd_f32_workspace_bytes(batch, seqlen, nheads, headdim, dstate) : 0;
+    return ((chunked > f32 ? chunked : f32) + 255) / 256 * 256;
+  }
   const size_t narrow = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 0);
   const size_t wide = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 1);
   const int forced = g_ssd_impl.load(std::memory_order_relaxed);
@@ -160,6 +171,17 @@ static int scan_impl(const void* x, const void* dt, const void* A, const void* B
                                  y_stride_l, dtype, dt_softplus, dt_min, dt_max, group_map, workspace, forced == 8, &ran, st);
     ran_on(8, ran);
     return rc;
+  }
+  // Lengths that ssd_chunked.hip leaves out (up to 64 tokens, more than 4 096), on the matrix cores where their rows allow it.  us, token by token | here, 32 heads x 64: 48 tokens
+  // 17.7 | 7.5, 64: 22 | 7.5, 8 192: 2 690 | 104; 128 x 128, 64: 28 | 8.6; 24: 10.2 | 7.4, but the recurrence's error is the smaller one there by some per cent
+  if (forced == 0 && dtype == TV_F32 && workspace && (uintptr_t)workspace % 16 == 0 && seqlen >= F32_FROM &&
+      workspace_bytes >= tv_ssd_f32_workspace_bytes(batch, seqlen, nheads, headdim, dstate) &&
+      tv_ssd_f32_supported(headdim, dstate, x_stride_b, x_stride_l, b_stride_b, b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b, y_stride_l, x,
+                           Bm, Cm, y, init_state, final_state)) {
+    ran_on(8, 11);
+    return tv_ssd_f32_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups, x_stride_b, x_stride_l,
+                             dt_stride_b, dt_stride_l, b_stride_b, b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b, y_stride_l, dt_softplus, dt_min,
+                             dt_max, group_map, true, workspace, st);
   }
   if (forced == 8) TV_UNSUPPORTED("ssd_scan: chunk-parallel generic kernel forced but shape unsupported");
   ran_on(1, 1);
