@@ -70,3 +70,17 @@ def test_before_what_is_no_number(L, at, what, value):
         d = F.softplus(dt.double()).nan_to_num(0.0)
         mag = reference(x.double(), d, *(v.double() for v in (A, Bm, Cm, D, S0)), torch.arange(4, device=DEV) // 2)[2]
         assert ((y - z).abs() <= 2 * 2.0 ** -18 * mag).all()               # (both within 2^-18 of the terms, as above)
+
+
+@pytest.mark.parametrize("B,L,H,P", [(2, 3000, 32, 64), (1, 2100, 32, 64), (2, 700, 128, 64), (2, 1300, 24, 64)])
+def test_segments_of_a_round(B, L, H, P):
+    """segments that are as many as fill a round, and that begin another one"""
+    from timeviper_amd import kernels as ops
+    x, dt, A, Bm, Cm, D, bias, S0 = operands(B, L, H, P, 2, "slow")
+    y, fin = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=S0, return_final_states=True)
+    assert ops.ssd_scan_last_kernel() == 11
+    d = F.softplus(dt.double())
+    want, S, mag, Sm = reference(x.double(), d, A.double(), Bm.double(), Cm.double(), D.double(), S0.double(), torch.arange(H, device=DEV) // (H // 2))
+    # (as test_scan_f32_gpu.py: exponents are differences of prefix sums of 64 tokens, here below 1)
+    rel = 2.0 ** -18 + 2.0 ** -21 * 64 * (d * A.double()).abs().mean(1).max().item()
+    assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()

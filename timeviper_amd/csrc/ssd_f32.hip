@@ -234,12 +234,21 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
   }
 }
 
-// chunks a segment: two waves a SIMD (one: 2 x 4 096 tokens 92 | 105 us, four: 93, 2 x 1 024: 31 | 35, 36), at most 64 segments (the fold keeps a segment's decay a lane)
+// Chunks a segment: at most 64 segments (the fold keeps a segment's decay a lane), and the least of rounds of two waves a SIMD times a segment's chunks and .9 for what stands
+// around them; a begun round counts .3 and its share of the rest.  (Rounded down to a round or more, us, before -> here, 32 heads x 64: 2 x 3 000 tokens 86 -> 66, 1 x 3 500:
+// 57 -> 47, 2 x 1 300: 41 -> 38; 128 heads: 2 x 700: 80 -> 60, 2 x 2 100: 218 -> 159; always up: 1 x 2 100 36.0 | 38.2, 1 x 1 300: 27.1 | 28.1.  One wave a SIMD: 2 x 4 096: 92 | 105,
+// four: 93.)
 int chunks_a_segment(int batch, int nch, int nheads, int headdim) {
-  const int64_t waves = (int64_t)batch * nheads * (headdim / 16) * nch;
-  int64_t len = waves / (8ll * tv_cu_count());
-  if (len < (nch + 63) / 64) len = (nch + 63) / 64;
-  return (int)(len < 1 ? 1 : len > nch ? nch : len);
+  const int64_t waves = (int64_t)batch * nheads * (headdim / 16), round = 8ll * tv_cu_count();
+  const int64_t from = (nch + 63) / 64, most = waves * nch / round + 1, to = most < from ? from : most > nch ? nch : most;      // (from `most` on one round or less)
+  int64_t best = from;
+  double least = 1e300;
+  for (int64_t len = from; len <= to; ++len) {
+    const int64_t all = waves * ((nch + len - 1) / len), full = all / round;
+    const double part = (double)(all % round) / round, rounds = full == 0 ? 1 : part > 0 ? full + .3 + .7 * part : full, t = rounds * (len + .9);
+    if (t < least) { least = t; best = len; }
+  }
+  return (int)best;
 }
 
 }  // namespace
