@@ -232,3 +232,114 @@ def test_vit_attention_tile_include_is_what_the_generator_writes():
     out = subprocess.run([sys.executable, str(build.ROOT / "devtools" / "gen_fa_vit.py")], check=True, capture_output=True,
                          text=True, env={k: v for k, v in os.environ.items() if k != "TV_FAV_ABLATE"}).stdout
     assert out == (build.CSRC / "attention_vit_tile.inc").read_text()
+
+
+# ---- wait states that the hardware does not keep by itself, counted in the built code.  The compiler keeps them for its own instructions; it does not look into
+# the inline statements (copies into LDS, stores), so a v_readfirstlane that it puts right in front of one is seen only here.
+def _registers(text: str, kind: str) -> set:
+    out = set()
+    for m in re.finditer(rf"(?<![\w\[:])([{kind}])(\d+)\b|\b([{kind}])\[(\d+):(\d+)\]|\b(vcc|m0)\b", text):
+        if m.group(1):
+            out.add(m.group(1) + m.group(2))
+        elif m.group(3):
+            out.update(f"{m.group(3)}{i}" for i in range(int(m.group(4)), int(m.group(5)) + 1))
+        elif "s" in kind:
+            out.add(m.group(6))
+    return out
+
+
+class _Instruction:
+    __slots__ = ("op", "ops", "at", "next", "states")
+
+    def __init__(self, op, args, at):
+        self.op, self.at, self.next = op, at, []
+        self.ops = [o.strip() for o in re.split(r",(?![^\[]*\])", args)] if args else []
+        self.states = int(self.ops[0], 0) + 1 if op == "s_nop" else 1
+
+
+def _device_code(src_name: str, work: Path) -> list:
+    """The instructions of lib/obj/<src>.o in order, each with what can follow it"""
+    work.mkdir()
+    obj = build.OBJ / (src_name + ".o")
+    shutil.copy(obj, work / obj.name)
+    subprocess.run([str(LLVM / "llvm-objdump"), "--offloading", obj.name], cwd=work, check=True, capture_output=True)
+    out, symbols, jumps = [], {}, []
+    for dev in (p for p in work.iterdir() if "amdgcn" in p.name):
+        for line in subprocess.run([str(LLVM / "llvm-objdump"), "-d", dev.name], cwd=work, check=True, capture_output=True, text=True).stdout.splitlines():
+            if m := re.match(r"([0-9a-f]+) <(.+)>:", line):
+                symbols[m.group(2)] = int(m.group(1), 16)
+            elif m := re.match(r"\t(\S+)\s*(.*?)\s*// ([0-9A-F]+):\s*(.*)$", line):
+                out.append(_Instruction(m.group(1), m.group(2), int(m.group(3), 16)))
+                t = re.search(r"<([^>+]+)(?:\+0x([0-9a-f]+))?>", m.group(4))
+                if t and m.group(1).startswith(("s_branch", "s_cbranch")):
+                    jumps.append((len(out) - 1, t.group(1), int(t.group(2) or "0", 16)))
+    where = {i.at: i for i in out}
+    for a, b in zip(out, out[1:]):
+        if a.op not in ("s_branch", "s_endpgm", "s_setpc_b64"):
+            a.next.append(b)
+    for n, name, offset in jumps:
+        out[n].next.append(where[symbols[name] + offset])
+    return out
+
+
+def _too_near(first: _Instruction, live: set, need: int, reads, writes) -> list:
+    """The instructions that read one of `live`, written by `first`, with fewer than `need` wait states between, on any path"""
+    found, seen, todo = [], {}, [(n, 0, frozenset(live)) for n in first.next]
+    while todo:
+        i, passed, regs = todo.pop()
+        if passed >= need or not regs or seen.get((i.at, regs), need) <= passed:
+            continue
+        seen[i.at, regs] = passed
+        if reads(i) & regs:
+            found.append((passed, i))
+        todo += [(n, passed + i.states, regs - writes(i)) for n in i.next]
+    return found
+
+
+_MEMORY = ("global_", "buffer_", "flat_", "scratch_")
+
+
+def _scalar_results(i: _Instruction) -> set:
+    """Scalar registers that a vector instruction writes"""
+    if i.op.startswith(("v_readfirstlane", "v_readlane", "v_cmp")):
+        return _registers(i.ops[0], "s")
+    if re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co|v_div_scale|v_mad_[ui]64", i.op):
+        return _registers(i.ops[1], "s")
+    return set()
+
+
+def _scalar_writes(i: _Instruction) -> set:
+    if i.op.startswith("s_") and i.ops and not i.op.startswith(("s_cmp", "s_bitcmp", "s_waitcnt", "s_nop", "s_cbranch", "s_branch", "s_set")):
+        return _registers(i.ops[0], "s")
+    return _scalar_results(i)
+
+
+@needs_tools
+def test_loads_keep_five_wait_states_behind_a_vector_write_of_their_scalar_address(tmp_path):
+    """A vector-memory instruction that reads a scalar register (address, M0 aside) which v_readfirstlane, v_readlane or a compare has written reads the old value
+    within five wait states."""
+    build.ensure_built()
+    bad = []
+    for src in build._sources():
+        for i in _device_code(src.name, tmp_path / src.name):
+            if live := _scalar_results(i):
+                for passed, j in _too_near(i, live, 5, lambda k: _registers(" ".join(k.ops), "s") if k.op.startswith(_MEMORY) else set(), _scalar_writes):
+                    bad.append((src.name, passed, i.op, i.ops, j.op, j.ops))
+    assert not bad, (len(bad), bad[:4])
+
+
+def test_the_count_of_wait_states_sees_what_is_too_near():
+    def code(*lines):
+        out = [_Instruction(*(ln.split(" ", 1) + [""])[:2], n) for n, ln in enumerate(lines)]
+        for a, b in zip(out, out[1:]):
+            a.next.append(b)
+        return out
+
+    def near(*lines):
+        c = code(*lines)
+        return [p for p, _ in _too_near(c[0], _scalar_results(c[0]), 5, lambda k: _registers(" ".join(k.ops), "s") if k.op.startswith(_MEMORY) else set(), _scalar_writes)]
+    head = ("s_mov_b32 s9, m0", "s_mov_b32 m0, s8")
+    assert near("v_readfirstlane_b32 s5, v1", *head, "s_nop 0", "global_load_lds_dwordx4 v0, s[4:5]") == [3]
+    assert near("v_readfirstlane_b32 s5, v1", *head, "s_nop 2", "global_load_lds_dwordx4 v0, s[4:5]") == []
+    assert near("v_readlane_b32 s4, v1, 3", "s_add_u32 s4, s4, s6", "global_load_dwordx4 v[0:3], v0, s[4:5] offset:16") == []
+    assert near("v_cmp_gt_u32_e64 s[4:5], v1, v2", "global_store_dwordx4 v0, v[4:7], s[4:5]") == [0]

@@ -26,13 +26,17 @@ __device__ __forceinline__ bf16x8 ld8(const unsigned char* p) { return *(const b
 // no vmcnt(0) in front of the fragment reads (it does for the builtin + ds_read_tr); every
 // wait on these copies is the hand-counted s_waitcnt vmcnt(N) + barrier below.  M0 (the LDS
 // destination base) is saved and restored inside the statement.
+// A vector-memory instruction has to come five wait states behind a vector instruction (v_readfirstlane, v_readlane) that
+// writes a scalar register it reads.  The compiler keeps that distance for its own loads and does not look into a
+// statement: with s_mov, s_mov, s_nop 2 in front the statement keeps it whatever it follows (the source address is
+// uniform_ptr's more often than not).  The other statements' distances are counted in the built code by the tests.
 __device__ __forceinline__ unsigned lds_addr_of(const void* p) {
   return __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t*)p);
 }
 // 16 bytes per active lane: LDS[lds_dst + 16*lane] = *(sbase + voff)
 __device__ __forceinline__ void glds16(const void* sbase, unsigned voff, unsigned lds_dst) {
   unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 2\n\t"
                "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_dst) : "memory");
 }
@@ -48,7 +52,7 @@ inline bool scan_rows_apart(int seqlen, int64_t xsl, int64_t bsl, int64_t csl, i
 __device__ __forceinline__ void glds16x4(const void* sbase, unsigned v0, unsigned v1, unsigned v2, unsigned v3,
                                          unsigned lds_dst) {
   unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\t"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 2\n\t"
                "global_load_lds_dwordx4 %1, %5\n\t"
                "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
                "global_load_lds_dwordx4 %3, %5 offset:2048\n\t"
@@ -58,7 +62,7 @@ __device__ __forceinline__ void glds16x4(const void* sbase, unsigned v0, unsigne
 // one dword per lane: LDS[lds_dst + 4*lane]
 __device__ __forceinline__ void glds4(const void* sbase, unsigned voff, unsigned lds_dst) {
   unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 2\n\t"
                "global_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds_dst) : "memory");
 }
