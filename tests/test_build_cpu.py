@@ -328,6 +328,24 @@ def test_loads_keep_five_wait_states_behind_a_vector_write_of_their_scalar_addre
     assert not bad, (len(bad), bad[:4])
 
 
+def _vector_writes(i: _Instruction) -> set:
+    return _registers(i.ops[0], "va") if i.op.startswith("v_") and i.ops else set()
+
+
+@needs_tools
+def test_wide_stores_keep_their_data_for_two_wait_states(tmp_path):
+    """A store of more than 8 bytes still reads its data in the two wait states behind it: no vector instruction may write those registers there."""
+    build.ensure_built()
+    bad = []
+    for src in build._sources():
+        for i in _device_code(src.name, tmp_path / src.name):
+            if re.match(r"(global|flat|buffer)_store_dwordx[34]$", i.op):
+                data = i.ops[0 if i.op.startswith("buffer") else 1]
+                for passed, j in _too_near(i, _registers(data, "va"), 2, _vector_writes, lambda k: set()):
+                    bad.append((src.name, passed, i.op, i.ops, j.op, j.ops))
+    assert not bad, (len(bad), bad[:4])
+
+
 def test_the_count_of_wait_states_sees_what_is_too_near():
     def code(*lines):
         out = [_Instruction(*(ln.split(" ", 1) + [""])[:2], n) for n, ln in enumerate(lines)]

@@ -806,7 +806,8 @@ __global__ __launch_bounds__(NW * 64) void ssd_head_kernel(HeadArgs a) {
         const auto s0 = __builtin_amdgcn_permlane16_swap(ya[0], yb[0], false, false);
         const auto s1 = __builtin_amdgcn_permlane16_swap(ya[1], yb[1], false, false);
         const u32x4v w = {s0[0], s1[0], s0[1], s1[1]};
-        if (ok) asm volatile("global_store_dwordx4 %0, %1, %2 offset:%3" :: "v"(yo16), "v"(w), "s"(yrow), "n"(32 * ct) : "memory");
+        // (s_nop: two wait states before a vector instruction may overwrite the data of a store of more than 8 bytes; the compiler does not know this is one)
+        if (ok) asm volatile("global_store_dwordx4 %0, %1, %2 offset:%3\n\ts_nop 1" :: "v"(yo16), "v"(w), "s"(yrow), "n"(32 * ct) : "memory");
       }
     }
 #else
