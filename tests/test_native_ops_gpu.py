@@ -1,9 +1,13 @@
 """The operators' native host side: the same kernels on the same operands, so the same bits as the way through Python, over the forms that both take; what it does not take."""
+import ctypes
+import re
+import subprocess
 import threading
 
 import pytest
 import torch
 
+from timeviper_amd import _capi, build
 from timeviper_amd import kernels as ops
 from timeviper_amd._native import ops as native
 
@@ -164,6 +168,36 @@ def test_refused_as_before(call, monkeypatch):
             call()
         told.append((type(e.value), str(e.value)))
     assert told[0] == told[1]
+
+
+@pytest.fixture
+def failing(tmp_path):
+    """The native operators on a library whose every entry counts its calls and says that a launch failed"""
+    entries = sorted(set(re.findall(r"X\((tv_\w+)\)", build.NATIVE_SRC.read_text())) - {"tv_last_error"})
+    source, stub = tmp_path / "stub.c", tmp_path / "stub.so"
+    source.write_text("int calls;\nconst char* tv_last_error(void) { return \"an earlier call's\"; }\n" +
+                      "".join(f"{'unsigned long' if 'bytes' in e else 'int'} {e}(void) {{ {'return 0' if 'bytes' in e else '++calls; return -4'}; }}\n" for e in entries))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(stub)], check=True)
+    lib = ctypes.CDLL(str(stub))
+    native.rms_norm                                                                      # (loaded)
+    native.bind(str(stub), ops.TimeViperHipError)
+    yield ctypes.c_int.in_dll(lib, "calls")
+    native.bind(str(_capi.lib_path()), ops.TimeViperHipError)
+
+
+@pytest.mark.gpu
+def test_a_failed_launch_raises_and_is_not_run_again(failing):
+    """The kernel may be on its way (the error can be an earlier call's): an operator that changes its operands must not run twice."""
+    x, w, out = r(40, 512), r(640, 512), r(40, 640)
+    p, state = plan([4], [2], [0], 8), r(1, 2, 96, dtype=F32)
+    before, state0 = out.clone(), state.clone()
+    for n, (call, entry) in enumerate(((lambda: ops.small_linear(x, w, None, ops.GEMM_ACCUM, out), "tv_gemm_small_fwd"),
+                                       (lambda: ops.norm_shift(r(4, 96, dtype=F32), r(1), 1e-5, shift=r(96), state=state, plan=p), "tv_norm_shift_fwd"),
+                                       (lambda: ops.rms_norm(x, r(512), 1e-5), "tv_rmsnorm_fwd"))):
+        with pytest.raises(ops.TimeViperHipError, match=f"^{entry} failed .status -4.: an earlier call's"):
+            call()
+        assert failing.value == n + 1
+    assert torch.equal(out, before) and torch.equal(state, state0)
 
 
 @pytest.mark.gpu

@@ -18,9 +18,9 @@ class _Ops:
         loader = importlib.machinery.ExtensionFileLoader("_tv_native", str(NATIVE))
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tv_native", loader))
         loader.exec_module(module)
-        module.bind(str(_capi.lib_path()))
+        module.bind(str(_capi.lib_path()), _capi.TimeViperHipError)
         del lib
-        self.__dict__.update({k: v for k, v in vars(module).items() if not k.startswith("_") and k != "bind"})
+        self.__dict__.update({k: v for k, v in vars(module).items() if not k.startswith("_")})
         if name not in self.__dict__:
             raise AttributeError(name)
         return self.__dict__[name]

@@ -1,6 +1,7 @@
 // The host side of the operators that short calls wait for, in C++: each function is one operator of kernels.py on operands that need no conversion - allocate the
 // results, call the C entry point.  Anything else (a dtype or layout that kernels.py would convert, a tensor subclass, a wrapped or CPU tensor, an argument that it
-// refuses, a status other than 0) returns None before anything is launched, and kernels.py goes its own way, errors included.
+// or the C entry refuses) returns None before anything is launched, and kernels.py goes its own way, errors included.  Where the C entry says that a launch failed,
+// its kernels may be on their way all the same (the error can be an earlier call's): the operator is not run again, and raises what kernels.py would.
 //
 // A Python wrapper spends 5 - 10 us beside its 2.5 us launches on attribute calls, two more on the argument conversion of ctypes and 1.4 on every result; a short
 // call's kernels are done before the next one is launched.  Host time of one call before -> now, us: norm 6.8 -> 3.9 (with a residual 8.4 -> 5.0), LayerNorm 7.1 -> 4.2,
@@ -25,7 +26,7 @@ namespace {
   X(tv_rmsnorm_fwd) X(tv_layernorm_fwd) X(tv_rmsnorm_gated_fwd) X(tv_causal_conv1d_xbc_fwd) X(tv_causal_conv1d_xbc_cb_fwd) X(tv_ssd_cb_bytes)              \
   X(tv_ssd_scan_workspace_bytes) X(tv_ssd_scan_cb_fwd) X(tv_flash_attn_fwd) X(tv_gemm_mid_fwd) X(tv_gemm_mid_workspace_bytes) X(tv_gemm_split_fwd)          \
   X(tv_gemm_split_workspace_bytes) X(tv_gemm_split_add_fwd) X(tv_gemm_small_fwd) X(tv_gemm_rows_fwd) X(tv_residual_add_fwd)            \
-  X(tv_token_side_fwd) X(tv_norm_shift_fwd) X(tv_gated_mul_fwd) X(tv_scatter_rows) X(tv_flash_attn_window_packed_fwd)
+  X(tv_token_side_fwd) X(tv_norm_shift_fwd) X(tv_gated_mul_fwd) X(tv_scatter_rows) X(tv_flash_attn_window_packed_fwd) X(tv_last_error)
 struct Lib {
 #define X(name) decltype(&::name) name = nullptr;
   TV_NATIVE_SYMBOLS(X)
@@ -35,6 +36,8 @@ struct Lib {
 typedef const at::Tensor* T;
 
 struct Refused {};      // "kernels.py's way"
+struct Failed {};       // a Python exception is set
+PyObject* error = nullptr;      // the package's exception
 inline void need(bool ok) { if (!ok) throw Refused{}; }
 
 // an exact, dense-storage GPU tensor of the current device (None: nullptr, where allowed)
@@ -85,11 +88,16 @@ inline bool truth(PyObject* o) {
   return v != 0;
 }
 template <typename F, typename... A>
-void launch(F f, A... args) {
+void launch_named(const char* name, F f, A... args) {
   int status;
   { Unlocked u; status = f(args...); }
-  need(status == 0);       // (kernels.py calls again and says what was wrong)
+  need(status != TV_ERR_BAD_ARG && status != TV_ERR_UNSUPPORTED && status != TV_ERR_WORKSPACE);       // (nothing is launched: kernels.py calls again and says what was wrong)
+  if (status != TV_OK) {
+    PyErr_Format(error, "%s failed (status %d): %s", name, status, lib.tv_last_error());
+    throw Failed{};
+  }
 }
+#define launch(entry, ...) launch_named(#entry, lib.entry, __VA_ARGS__)
 inline PyObject* wrap(at::Tensor&& t) { return THPVariable_Wrap(std::move(t)); }
 template <typename... A>
 PyObject* tuple(A*... items) {
@@ -115,7 +123,7 @@ PyObject* rms_norm(PyObject* const* a) {
   need(D > 0 && w->numel() == D);
   at::Tensor y = like(x, x->sizes()), s;
   if (sums && r) s = like(x, x->sizes());
-  launch(lib.tv_rmsnorm_fwd, ptr(x), ptr(r), ptr(w), s.defined() ? s.data_ptr() : nullptr, y.data_ptr(), x->numel() / D, (int)D, D, r ? D : 0, s.defined() ? D : 0, D,
+  launch(tv_rmsnorm_fwd, ptr(x), ptr(r), ptr(w), s.defined() ? s.data_ptr() : nullptr, y.data_ptr(), x->numel() / D, (int)D, D, r ? D : 0, s.defined() ? D : 0, D,
                             (float)real(a[2]), dtype_of(x), dtype_of(w), op.stream());
   if (!sums) return wrap(std::move(y));
   return tuple(wrap(std::move(y)), s.defined() ? wrap(std::move(s)) : again(a[0]));
@@ -127,10 +135,11 @@ PyObject* layer_norm(PyObject* const* a) {
   need(x->dim() > 0 && x->is_contiguous() && same_type(w, x) && w->is_contiguous() && (b == nullptr || (same_type(b, x) && b->is_contiguous())));
   const int64_t D = x->size(-1);
   need(D > 0 && w->numel() == D && (b == nullptr || b->numel() == D) && (rb == nullptr || (rb->scalar_type() == at::kFloat && rb->is_contiguous() && rb->numel() == D)));
+  const bool sums = truth(a[4]);
   at::Tensor y = like(x, x->sizes());
-  launch(lib.tv_layernorm_fwd, ptr(x), nullptr, ptr(w), ptr(b), (const float*)ptr(rb), nullptr, y.data_ptr(), x->numel() / D, (int)D, D, 0, 0, D, (float)real(a[3]), dtype_of(x),
+  launch(tv_layernorm_fwd, ptr(x), nullptr, ptr(w), ptr(b), (const float*)ptr(rb), nullptr, y.data_ptr(), x->numel() / D, (int)D, D, 0, 0, D, (float)real(a[3]), dtype_of(x),
                               op.stream());
-  return truth(a[4]) ? tuple(wrap(std::move(y)), again(a[0])) : wrap(std::move(y));
+  return sums ? tuple(wrap(std::move(y)), again(a[0])) : wrap(std::move(y));
 }
 // gated_norm(x, weight, z, eps, group_size)
 PyObject* gated_norm(PyObject* const* a) {
@@ -141,7 +150,7 @@ PyObject* gated_norm(PyObject* const* a) {
   const int64_t D = x->size(-1), gs = a[4] == Py_None ? D : integer(a[4]);
   need(D > 0 && gs > 0 && gs <= D && w->numel() == D);
   at::Tensor y = like(x, x->sizes());
-  launch(lib.tv_rmsnorm_gated_fwd, ptr(x), ptr(z), ptr(w), y.data_ptr(), x->numel() / D, (int)D, (int)gs, D, z ? z->stride(1) : 0, D, (float)real(a[3]), dtype_of(x), dtype_of(w),
+  launch(tv_rmsnorm_gated_fwd, ptr(x), ptr(z), ptr(w), y.data_ptr(), x->numel() / D, (int)D, (int)gs, D, z ? z->stride(1) : 0, D, (float)real(a[3]), dtype_of(x), dtype_of(w),
                                   op.stream());
   return wrap(std::move(y));
 }
@@ -160,10 +169,10 @@ PyObject* conv_xbc(PyObject* const* a) {
   at::Tensor yx = like(x, {B, L, di}), yb = like(x, {B, G, L, N}), yc = like(x, {B, G, L, N}), cb;
   if (want_cb && bf16(x) && N == 128 && L > 0) {
     cb = like(x, {(int64_t)(lib.tv_ssd_cb_bytes((int)B, (int)L, (int)G) / 2)});
-    launch(lib.tv_causal_conv1d_xbc_cb_fwd, ptr(x), ptr(w), ptr(b), nullptr, yx.data_ptr(), yb.data_ptr(), yc.data_ptr(), cb.data_ptr(), (int)B, (int)L, (int)di, (int)G, (int)N,
+    launch(tv_causal_conv1d_xbc_cb_fwd, ptr(x), ptr(w), ptr(b), nullptr, yx.data_ptr(), yb.data_ptr(), yc.data_ptr(), cb.data_ptr(), (int)B, (int)L, (int)di, (int)G, (int)N,
                                            (int)K, x->stride(0), x->stride(1), dtype_of(x), silu, op.stream());
   } else {
-    launch(lib.tv_causal_conv1d_xbc_fwd, ptr(x), ptr(w), ptr(b), nullptr, yx.data_ptr(), yb.data_ptr(), yc.data_ptr(), (int)B, (int)L, (int)di, (int)G, (int)N, (int)K,
+    launch(tv_causal_conv1d_xbc_fwd, ptr(x), ptr(w), ptr(b), nullptr, yx.data_ptr(), yb.data_ptr(), yc.data_ptr(), (int)B, (int)L, (int)di, (int)G, (int)N, (int)K,
                                         x->stride(0), x->stride(1), dtype_of(x), silu, op.stream());
   }
   PyObject *px = wrap(std::move(yx)), *pb = wrap(yb.transpose(1, 2)), *pc = wrap(yc.transpose(1, 2));
@@ -199,7 +208,7 @@ PyObject* scan(PyObject* const* a) {
   if (want_decay) dec = like(x, {b, H}, at::kFloat);
   const size_t bytes = lib.tv_ssd_scan_workspace_bytes((int)b, (int)L, (int)H, (int)P, (int)G, (int)N, dtype_of(x));
   at::Tensor ws = like(x, {(int64_t)(bytes > 16 ? bytes : 16)}, at::kByte);
-  launch(lib.tv_ssd_scan_cb_fwd, ptr(x), ptr(dt), (const float*)ptr(A), ptr(B), ptr(C), ptr(cb), (const float*)ptr(D), (const float*)ptr(bias), (const float*)ptr(init), y.data_ptr(),
+  launch(tv_ssd_scan_cb_fwd, ptr(x), ptr(dt), (const float*)ptr(A), ptr(B), ptr(C), ptr(cb), (const float*)ptr(D), (const float*)ptr(bias), (const float*)ptr(init), y.data_ptr(),
                                 fin.defined() ? (float*)fin.data_ptr() : nullptr, dec.defined() ? (float*)dec.data_ptr() : nullptr, (int)b, (int)L, (int)H, (int)P, (int)G, (int)N,
                                 x->stride(0), x->stride(1), dt->stride(0), dt->stride(1), B->stride(0), B->stride(1), B->stride(2), C->stride(0), C->stride(1), C->stride(2),
                                 y.stride(0), y.stride(1), dtype_of(x), truth(a[8]), (float)real(a[9]), (float)real(a[10]), (int)integer(a[13]), ws.data_ptr(), bytes, op.stream());
@@ -220,7 +229,7 @@ PyObject* flash(PyObject* const* a) {
   const bool want_lse = truth(a[5]);
   at::Tensor o = like(q, {B, Lq, H, D}), lse;
   if (want_lse) lse = like(q, {B, H, Lq}, at::kFloat);
-  launch(lib.tv_flash_attn_fwd, ptr(q), ptr(k), ptr(v), o.data_ptr(), want_lse ? lse.data_ptr() : nullptr, (int)B, (int)Lq, (int)Lk, (int)H, (int)G, (int)D, q->stride(0), q->stride(1),
+  launch(tv_flash_attn_fwd, ptr(q), ptr(k), ptr(v), o.data_ptr(), want_lse ? lse.data_ptr() : nullptr, (int)B, (int)Lq, (int)Lk, (int)H, (int)G, (int)D, q->stride(0), q->stride(1),
                                q->stride(2), k->stride(0), k->stride(1), k->stride(2), v->stride(0), v->stride(1), v->stride(2), o.stride(0), o.stride(1), o.stride(2), (float)scale,
                                truth(a[4]), dtype_of(q), op.stream());
   return want_lse ? tuple(wrap(std::move(o)), wrap(std::move(lse))) : wrap(std::move(o));
@@ -253,7 +262,7 @@ PyObject* mid_linear(PyObject* const* a) {
   const size_t bytes = lib.tv_gemm_mid_workspace_bytes((int)p.M, (int)p.N, (int)p.K);
   at::Tensor ws;
   if (bytes) ws = like(p.x, {(int64_t)bytes}, at::kByte);
-  launch(lib.tv_gemm_mid_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), (int)p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, truth(a[3]) ? TV_GEMM_ROWS_RELU2 : 0,
+  launch(tv_gemm_mid_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), (int)p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, truth(a[3]) ? TV_GEMM_ROWS_RELU2 : 0,
                              bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
   return wrap(std::move(p.y));
 }
@@ -266,7 +275,7 @@ PyObject* split_linear(PyObject* const* a) {
   const size_t bytes = lib.tv_gemm_split_workspace_bytes(p.M, (int)p.N, splits, full);
   at::Tensor ws;
   if (bytes) ws = like(p.x, {(int64_t)bytes}, at::kByte);
-  launch(lib.tv_gemm_split_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, truth(a[3]) ? 3 : 0, p.b ? dtype_of(p.b) : TV_F32,
+  launch(tv_gemm_split_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, truth(a[3]) ? 3 : 0, p.b ? dtype_of(p.b) : TV_F32,
                                splits, full, bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
   return wrap(std::move(p.y));
 }
@@ -276,7 +285,7 @@ PyObject* rows_linear(PyObject* const* a) {
   Product p;
   product(op, a, p, false);
   need(p.M >= 2 && p.M <= TV_GEMM_ROWS_MAX && p.K % 64 == 0 && p.K < (1 << 24) && p.w->stride(0) % 8 == 0 && p.w->stride(0) < (1 << 24) && aligned(p.w, 16) && aligned(p.x, 16));
-  launch(lib.tv_gemm_rows_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), TV_BF16, (int)p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, (int)integer(a[3]), nullptr, nullptr,
+  launch(tv_gemm_rows_fwd, ptr(p.x), ptr(p.w), ptr(p.b), p.y.data_ptr(), TV_BF16, (int)p.M, (int)p.N, (int)p.K, p.K, p.w->stride(0), p.N, (int)integer(a[3]), nullptr, nullptr,
                               nullptr, 0, 0, op.stream());
   return wrap(std::move(p.y));
 }
@@ -295,7 +304,7 @@ PyObject* small_linear(PyObject* const* a) {
   } else {
     need(out->dim() == 2 && out->size(0) == x->size(0) && out->size(1) == N && bf16(out) && out->stride(1) == 1);
   }
-  launch(lib.tv_gemm_small_fwd, ptr(x), ptr(w), epi == 2 ? nullptr : ptr(b), out ? ptr(out) : y.data_ptr(), x->size(0), (int)N, (int)w->size(1), x->stride(0), w->stride(0),
+  launch(tv_gemm_small_fwd, ptr(x), ptr(w), epi == 2 ? nullptr : ptr(b), out ? ptr(out) : y.data_ptr(), x->size(0), (int)N, (int)w->size(1), x->stride(0), w->stride(0),
                                out ? out->stride(0) : N, epi, b ? dtype_of(b) : TV_F32, (int)integer(a[5]), op.stream());
   return out ? again(a[4]) : wrap(std::move(y));
 }
@@ -307,7 +316,7 @@ PyObject* residual_add(PyObject* const* a) {
   T x = op.get(a[0]), u = op.get(a[1]);
   need(x->scalar_type() == at::kFloat && x->dim() == 2 && x->is_contiguous() && u->sizes() == x->sizes() && u->stride(1) == 1);
   at::Tensor xo = like(x, x->sizes()), h = like(u, x->sizes());
-  launch(lib.tv_residual_add_fwd, (const float*)ptr(x), ptr(u), (float*)xo.data_ptr(), h.data_ptr(), x->size(0), (int)x->size(1), u->stride(0), dtype_of(u), op.stream());
+  launch(tv_residual_add_fwd, (const float*)ptr(x), ptr(u), (float*)xo.data_ptr(), h.data_ptr(), x->size(0), (int)x->size(1), u->stride(0), dtype_of(u), op.stream());
   return tuple(wrap(std::move(xo)), wrap(std::move(h)));
 }
 // split_add_linear(x, weight, residual, bias, splits)
@@ -322,7 +331,7 @@ PyObject* split_add_linear(PyObject* const* a) {
   at::Tensor xo = like(r, r->sizes()), h = like(x, r->sizes()), ws;
   const size_t bytes = lib.tv_gemm_split_workspace_bytes(M, (int)N, splits, 0);
   if (bytes) ws = like(x, {(int64_t)bytes}, at::kByte);
-  launch(lib.tv_gemm_split_add_fwd, ptr(x), ptr(w), ptr(b), (const float*)ptr(r), (float*)xo.data_ptr(), h.data_ptr(), M, (int)N, (int)w->size(1), x->stride(0), w->stride(0), TV_BF16,
+  launch(tv_gemm_split_add_fwd, ptr(x), ptr(w), ptr(b), (const float*)ptr(r), (float*)xo.data_ptr(), h.data_ptr(), M, (int)N, (int)w->size(1), x->stride(0), w->stride(0), TV_BF16,
                                    splits, 0, bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
   return tuple(wrap(std::move(xo)), wrap(std::move(h)));
 }
@@ -334,7 +343,7 @@ PyObject* token_side(PyObject* const* a) {
   const int64_t n = h->size(0), D = h->size(1), S = gate->size(0);
   need(gate->size(1) == D && proj->size(0) == D && proj->size(1) == S && table->size(1) == S && ids->scalar_type() == at::kLong && ids->numel() == n && ids->is_contiguous());
   at::Tensor y = like(h, {n, D});
-  launch(lib.tv_token_side_fwd, ptr(h), (const int64_t*)ptr(ids), ptr(table), ptr(gate), ptr(proj), y.data_ptr(), n, (int)D, (int)S, table->size(0), h->stride(0), table->stride(0),
+  launch(tv_token_side_fwd, ptr(h), (const int64_t*)ptr(ids), ptr(table), ptr(gate), ptr(proj), y.data_ptr(), n, (int)D, (int)S, table->size(0), h->stride(0), table->stride(0),
                                gate->stride(0), proj->stride(0), D, op.stream());
   return wrap(std::move(y));
 }
@@ -362,7 +371,7 @@ PyObject* norm_shift(PyObject* const* a) {
   if (p) xo = like(x, x->sizes());
   if (truth(a[14]) || !sh) h = like(g, x->sizes());
   if (sh) hs = like(g, x->sizes());
-  launch(lib.tv_norm_shift_fwd, (const float*)ptr(x), ptr(p), p ? ptr(pw) : nullptr, p ? (float*)xo.data_ptr() : nullptr, ptr(g), ptr(sh), (float*)ptr(st), (const int*)ptr(seq),
+  launch(tv_norm_shift_fwd, (const float*)ptr(x), ptr(p), p ? ptr(pw) : nullptr, p ? (float*)xo.data_ptr() : nullptr, ptr(g), ptr(sh), (float*)ptr(st), (const int*)ptr(seq),
                                (const int*)ptr(cu), (const int*)ptr(start), (const int*)ptr(slot), h.defined() ? h.data_ptr() : nullptr, hs.defined() ? hs.data_ptr() : nullptr, n,
                                (int)D, p ? p->stride(0) : 0, st ? st->stride(0) : 0, (float)real(a[2]), truth(a[13]), type, op.stream());
   return tuple(p ? wrap(std::move(xo)) : again(a[0]), h.defined() ? wrap(std::move(h)) : again(Py_None), hs.defined() ? wrap(std::move(hs)) : again(Py_None));
@@ -377,7 +386,7 @@ PyObject* gated_mul(PyObject* const* a) {
   need(out == nullptr || (out->sizes() == x->sizes() && same_type(out, x) && out->stride(1) == 1));
   at::Tensor y;
   if (!out) y = like(x, x->sizes());
-  launch(lib.tv_gated_mul_fwd, ptr(x), ptr(b), (const int64_t*)ptr(ids), out ? ptr(out) : y.data_ptr(), n, (int)x->size(1), x->stride(0), b->stride(0), out ? out->stride(0) : x->size(1),
+  launch(tv_gated_mul_fwd, ptr(x), ptr(b), (const int64_t*)ptr(ids), out ? ptr(out) : y.data_ptr(), n, (int)x->size(1), x->stride(0), b->stride(0), out ? out->stride(0) : x->size(1),
                               b->size(0), (int)integer(a[2]), dtype_of(x), op.stream());
   return out ? again(a[4]) : wrap(std::move(y));
 }
@@ -387,7 +396,7 @@ PyObject* scatter_rows(PyObject* const* a) {
   T src = op.get(a[0]), rows = op.get(a[1]), dst = op.get(a[2]);
   need(src->dim() == 2 && dst->dim() == 2 && same_type(src, dst) && src->size(1) == dst->size(1) && src->stride(1) == 1 && dst->stride(1) == 1);
   int32s(rows, src->size(0));
-  launch(lib.tv_scatter_rows, ptr(src), (const int*)ptr(rows), ptr(dst), src->size(0), (int)src->size(1), src->stride(0), dst->stride(0), dtype_of(src), op.stream());
+  launch(tv_scatter_rows, ptr(src), (const int*)ptr(rows), ptr(dst), src->size(0), (int)src->size(1), src->stride(0), dst->stride(0), dtype_of(src), op.stream());
   return again(Py_True);
 }
 // attention_window(q, cache, plan's counts, starts, slots, kv_heads, scale, window, keep_first, gate, out, plan's rows, seq, cu, start, slot)
@@ -418,7 +427,7 @@ PyObject* attention_window(PyObject* const* a) {
   at::Tensor y;
   if (!out) y = like(q, {n, H, dv});
   char* const base = (char*)ptr(c);
-  launch(lib.tv_flash_attn_window_packed_fwd, ptr(q), base, base + G * dk * 2, out ? ptr(out) : y.data_ptr(), ptr(g), (int)integer(a[7]), (int)integer(a[8]), (int)dv, (int)B,
+  launch(tv_flash_attn_window_packed_fwd, ptr(q), base, base + G * dk * 2, out ? ptr(out) : y.data_ptr(), ptr(g), (int)integer(a[7]), (int)integer(a[8]), (int)dv, (int)B,
                                              rows.data(), lens_q.data(), lens_k.data(), slots.data(), (int)H, (int)G, (int)dk, q->stride(0), q->stride(1), cap * W, W, dk, cap * W, W, dv,
                                              out ? out->stride(0) : H * dv, out ? out->stride(1) : dv, g ? g->stride(0) : 0, g ? g->stride(1) : 0, (float)real(a[6]), TV_BF16,
                                              op.stream());
@@ -430,16 +439,19 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != N || lib.tv_rmsnorm_fwd == nullptr) Py_RETURN_NONE;
   try {
     return F(args);
+  } catch (const Failed&) {
+    return nullptr;
   } catch (...) {              // (a C++ exception stays on this side)
     PyErr_Clear();
     Py_RETURN_NONE;
   }
 }
 
-// bind(path of the library that is loaded already)
-PyObject* bind(PyObject*, PyObject* path) {
-  const char* p = PyUnicode_AsUTF8(path);
-  if (!p) return nullptr;
+// bind(path of the library that is loaded already, the exception for launches that fail)
+PyObject* bind(PyObject*, PyObject* args) {
+  const char* p;
+  PyObject* e;
+  if (!PyArg_ParseTuple(args, "sO", &p, &e)) return nullptr;
   void* h = dlopen(p, RTLD_NOW | RTLD_NOLOAD);
   if (!h) return PyErr_Format(PyExc_RuntimeError, "%s is not loaded", p);
   Lib l;
@@ -451,6 +463,8 @@ PyObject* bind(PyObject*, PyObject* path) {
   TV_NATIVE_SYMBOLS(X)
 #undef X
   lib = l;                     // (the handle is kept: the library stays mapped)
+  Py_XDECREF(error);
+  error = again(e);
   Py_RETURN_NONE;
 }
 
@@ -458,7 +472,7 @@ PyObject* bind(PyObject*, PyObject* path) {
 PyMethodDef methods[] = {ENTRY(rms_norm, 5), ENTRY(layer_norm, 6), ENTRY(gated_norm, 5), ENTRY(conv_xbc, 8), ENTRY(scan, 15), ENTRY(flash, 6), ENTRY(mid_linear, 4),
                          ENTRY(split_linear, 6), ENTRY(rows_linear, 4), ENTRY(small_linear, 6), ENTRY(residual_add, 2), ENTRY(split_add_linear, 5), ENTRY(token_side, 5), ENTRY(norm_shift, 15),
                          ENTRY(gated_mul, 5), ENTRY(scatter_rows, 3), ENTRY(attention_window, 16),
-                         {"bind", (PyCFunction)bind, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+                         {"bind", (PyCFunction)bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_tv_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
