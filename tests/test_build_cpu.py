@@ -249,10 +249,10 @@ def _registers(text: str, kind: str) -> set:
 
 
 class _Instruction:
-    __slots__ = ("op", "ops", "at", "next", "states")
+    __slots__ = ("op", "ops", "at", "next", "states", "of")
 
-    def __init__(self, op, args, at):
-        self.op, self.at, self.next = op, at, []
+    def __init__(self, op, args, at, of=None):
+        self.op, self.at, self.next, self.of = op, at, [], of
         self.ops = [o.strip() for o in re.split(r",(?![^\[]*\])", args)] if args else []
         self.states = int(self.ops[0], 0) + 1 if op == "s_nop" else 1
 
@@ -263,13 +263,14 @@ def _device_code(src_name: str, work: Path) -> list:
     obj = build.OBJ / (src_name + ".o")
     shutil.copy(obj, work / obj.name)
     subprocess.run([str(LLVM / "llvm-objdump"), "--offloading", obj.name], cwd=work, check=True, capture_output=True)
-    out, symbols, jumps = [], {}, []
+    out, symbols, jumps, of = [], {}, [], None
     for dev in (p for p in work.iterdir() if "amdgcn" in p.name):
         for line in subprocess.run([str(LLVM / "llvm-objdump"), "-d", dev.name], cwd=work, check=True, capture_output=True, text=True).stdout.splitlines():
             if m := re.match(r"([0-9a-f]+) <(.+)>:", line):
-                symbols[m.group(2)] = int(m.group(1), 16)
+                of = m.group(2)
+                symbols[of] = int(m.group(1), 16)
             elif m := re.match(r"\t(\S+)\s*(.*?)\s*// ([0-9A-F]+):\s*(.*)$", line):
-                out.append(_Instruction(m.group(1), m.group(2), int(m.group(3), 16)))
+                out.append(_Instruction(m.group(1), m.group(2), int(m.group(3), 16), of))
                 t = re.search(r"<([^>+]+)(?:\+0x([0-9a-f]+))?>", m.group(4))
                 if t and m.group(1).startswith(("s_branch", "s_cbranch")):
                     jumps.append((len(out) - 1, t.group(1), int(t.group(2) or "0", 16)))
@@ -361,3 +362,15 @@ def test_the_count_of_wait_states_sees_what_is_too_near():
     assert near("v_readfirstlane_b32 s5, v1", *head, "s_nop 2", "global_load_lds_dwordx4 v0, s[4:5]") == []
     assert near("v_readlane_b32 s4, v1, 3", "s_add_u32 s4, s4, s6", "global_load_dwordx4 v[0:3], v0, s[4:5] offset:16") == []
     assert near("v_cmp_gt_u32_e64 s[4:5], v1, v2", "global_store_dwordx4 v0, v[4:7], s[4:5]") == [0]
+
+
+@needs_tools
+def test_an_attention_step_copies_its_pieces_once(tmp_path):
+    """flash_fwd_kernel with two tiles a step: as many copies whatever the head dim, whose MFMAs they stand between"""
+    build.ensure_built()
+    copies = {}
+    for i in _device_code("attention.hip", tmp_path / "attention"):
+        if m := re.match(r"_ZN12_GLOBAL__N_116flash_fwd_kernelI(\w+)Li\dELi\dELi8ELi2ELb(\d)ELi(\d)E", i.of or ""):
+            copies.setdefault(m.groups(), {}).setdefault(i.of, 0)
+            copies[m.groups()][i.of] += "_lds_" in i.op
+    assert len(copies) == 6 and all(len(k) >= 3 and len(set(k.values())) == 1 for k in copies.values()), copies

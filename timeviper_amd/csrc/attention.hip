@@ -146,6 +146,12 @@ __device__ __forceinline__ void glds16_lanes(const void* sbase, unsigned voff, u
 // WIN: causal with a sliding window and kept first keys.  The work-group visits the tiles that hold kept keys, then jumps to the
 // first tile of its first row's window: ring, copies and waits count the visited tiles.  All sequences of a packed step share the
 // launch (a launch per prompt leaves most of the chip idle: six prompts, 6 011 tokens, 16 heads on 4 x 128, window 1 024: 265 us, in one launch 95).
+// A step's copies stand between its MFMAs, copy c behind number (2 c + 1) n / (2 copies) of n: how many of them in front of number i
+constexpr int copies_before(int i, int n, int copies) {
+  int c = 0;
+  while (c < copies && (2 * c + 1) * n / (2 * copies) < i) ++c;
+  return c;
+}
 constexpr int fa_slots(int kt) { return kt == 2 ? 4 : 1; }                       // (KT 3: keys of one tile)
 constexpr int fa_lds(int kt) { return 2 * fa_slots(kt) * 32 * kt * 256; }      // K and V rings, rows of 256 bytes
 template <typename T, int KS, int DT, int NW, int KT, bool WIN = false, int KG = 1>
@@ -393,8 +399,12 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
     constexpr bool CUR = decltype(CURT)::value, NEXT = decltype(NEXTT)::value, ODD = decltype(ODDT)::value;
     constexpr int KOFF = KG == 1 && !ODD && CUR ? TILEB : 0, VOFF = KG == 1 && ODD ? TILEB : 0;      // (without CUR: the first tile of a step)
     constexpr bool COPIES = SLOTS > 1 && CUR && (TPS == 1 || !ODD);        // the first tile of a step: the next one's copies, spread (64 of them at once hold up every wave)
-    constexpr int CEVERY = (NQK + NPV) / (4 * PPT);
-    static_assert(!COPIES || (NQK + NPV) % (4 * PPT) == 0 || CEVERY * 4 * PPT <= NQK + NPV, "");
+    constexpr int NC = 4 * PPT, NM = NQK + NPV;
+    static_assert(!COPIES || (NM >= NC && copies_before(NM, NM, NC) == NC), "every copy once");
+    auto copy_behind = [&](auto I) __attribute__((always_inline)) {
+      constexpr int c = copies_before(decltype(I)::value, NM, NC);
+      if constexpr (copies_before(decltype(I)::value + 1, NM, NC) > c) copy_ahead(kt, c);
+    };
     if constexpr (COPIES && !NEXT)
 #pragma unroll
       for (int c = 0; c < 4 * PPT; ++c) copy_ahead(kt, c);
@@ -448,9 +458,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
 #pragma unroll
           for (int j = 0; j < 16; ++j) SN[i / KS][j] = 0.f;
         SN[i / KS] = Frag<T>::mfma(kf[i], qf[i % KS], SN[i / KS]);
-        if constexpr (CUR && COPIES) {
-          if constexpr (i % CEVERY == CEVERY / 2) copy_ahead(kt, i / CEVERY);
-        }
+        if constexpr (CUR && COPIES) copy_behind(I);
         if constexpr (CUR) weights(integral_constant<int, LEAD + 2 * ((NE1 - LEAD) / 2 * i / NQK)>{}, integral_constant<int, LEAD + 2 * ((NE1 - LEAD) / 2 * (i + 1) / NQK)>{});
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -473,9 +481,7 @@ __global__ __launch_bounds__(NW * 64) void flash_fwd_kernel(AttnArgs a, typename
         for (int j = 0; j < 4; ++j) { vf[j] = vlo[s_ & 1][dt][j]; vf[4 + j] = vhi[s_ & 1][dt][j]; }
         oacc[dt] = Frag<T>::mfma(vf, __builtin_bit_cast(v8, pf[s_]), oacc[dt]);
         if constexpr (i < NP1) weights(integral_constant<int, NE1 + 2 * ((NE - NE1) / 2 * i / NP1)>{}, integral_constant<int, NE1 + 2 * ((NE - NE1) / 2 * (i + 1) / NP1)>{});
-        if constexpr (NEXT && COPIES) {
-          if constexpr ((NQK + i) % CEVERY == CEVERY / 2) copy_ahead(kt, (NQK + i) / CEVERY);
-        }
+        if constexpr (NEXT && COPIES) copy_behind(integral_constant<int, NQK + i>{});
         constexpr int M0 = 2;                   // (the scores' last MFMA ends behind the first of these)
         if constexpr (NEXT && i >= M0) tmax = largest(integral_constant<int, NE / 2 * (i - M0) / (NPV - M0)>{}, integral_constant<int, NE / 2 * (i + 1 - M0) / (NPV - M0)>{}, tmax);
         __builtin_amdgcn_sched_barrier(0);
