@@ -84,3 +84,32 @@ def test_segments_of_a_round(B, L, H, P):
     # (as test_scan_f32_gpu.py: exponents are differences of prefix sums of 64 tokens, here below 1)
     rel = 2.0 ** -18 + 2.0 ** -21 * 64 * (d * A.double()).abs().mean(1).max().item()
     assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
+
+
+def stepwise(x, d, A, Bm, Cm, D, S, of):
+    """`reference` token by token: no sums of exponents, of which an endless step leaves nothing"""
+    y, mag, Sm = torch.empty_like(x), torch.empty_like(x), S.abs()
+    for t in range(x.shape[1]):
+        e, xd, b, c = torch.exp(d[:, t] * A)[..., None, None], (d[:, t, :, None] * x[:, t])[..., None], Bm[:, t, of][:, :, None], Cm[:, t, of][:, :, None]
+        S, Sm = e * S + xd * b, e * Sm + (xd * b).abs()
+        y[:, t], mag[:, t] = (S * c).sum(-1) + D[:, None] * x[:, t], (Sm * c.abs()).sum(-1) + (D[:, None] * x[:, t]).abs()
+    return y, S, mag, Sm
+
+
+@pytest.mark.parametrize("L,at", [(48, (0,)), (50, (17, 18)), (64, (5, 31, 63)), (4100, (70,)), (4160, (0, 64, 4098, 4100))])
+@pytest.mark.parametrize("init", [False, True])
+@pytest.mark.parametrize("step", [float("inf"), 3e38, 1e7])
+def test_a_step_that_resets_without_end(L, at, init, step):
+    """an infinite dt (or one whose product with B is no number) where x is 0 empties the state, and what follows is as after any token: nothing but numbers"""
+    from timeviper_amd import kernels as ops
+    H = 4
+    x, dt, A, Bm, Cm, D, bias, S0 = operands(1, L, H, 32, 2, "fast")
+    dt = dt.abs() * .1
+    dt[0, list(at)], x[0, list(at)] = step, 0.
+    y, fin, dec = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, initial_states=S0 if init else None, return_final_states=True, return_total_decay=True)
+    assert ops.ssd_scan_last_kernel() == 11
+    d = dt.double().clamp(max=3.0e38)
+    want, S, mag, Sm = stepwise(x.double(), d, A.double(), Bm.double(), Cm.double(), D.double(), S0.double() if init else torch.zeros_like(S0).double(), torch.arange(H, device=DEV) // 2)
+    rel = 2.0 ** -18                                                       # (as above)
+    assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
+    assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5) if step < 1e38 else (dec < -1e37).all()

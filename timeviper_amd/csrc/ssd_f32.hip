@@ -53,10 +53,49 @@ __device__ __forceinline__ float scan_both(float v, float& lost) {
   return v;
 }
 
+// A chunk token by token, as the recurrence has it (ssd_generic.hip): S, y of the wave's columns; d and da are of token `lane`.  Returns the sum of da.
+template <bool OUT>
+__device__ __forceinline__ float march(const F3Args& a, const float* xb, const float* Bb, const float* Cb, int t0, int tt, float d, float da, float Dh, int lc, int q, int b, int h,
+                                       int pt, f32x4& S) {
+  float sum = 0.f;
+#pragma unroll 1
+  for (int t1 = 0; t1 < tt; t1 += 4) {
+    float x[4];
+    f32x4 B[4], C[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t t = t0 + min(t1 + j, tt - 1);
+      x[j] = xb[t * a.xsl + lc];
+      B[j] = *(const f32x4*)(Bb + t * a.bsl + 4 * q);
+      if constexpr (OUT) C[j] = *(const f32x4*)(Cb + t * a.csl + 4 * q);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (t1 + j >= tt) break;
+      const float dat = rdlane(da, t1 + j), dec = expf(dat), xv = rdlane(d, t1 + j) * x[j];
+      float acc = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        S[r] = fmaf(dec, S[r], xv * B[j][r]);
+        if constexpr (OUT) acc = fmaf(S[r], C[j][r], acc);
+      }
+      sum += dat;
+      if constexpr (OUT) {
+        acc += __shfl_xor(acc, 32, 64);
+        acc += __shfl_xor(acc, 16, 64);
+        if (q == 0) a.y[(int64_t)b * a.ysb + (int64_t)(t0 + t1 + j) * a.ysl + (int64_t)h * a.P + 16 * pt + lc] = fmaf(Dh, x[j], acc);
+      }
+    }
+  }
+  return sum;
+}
+
 // OUT: the second launch.  FINE: for the lengths that the token recurrence had before (48 - 64 tokens, more than 4 096), whose error is kept: two tokens' decay is the difference
 // of their sums AND of what these have lost (a sum over a chunk is rounded by its own size, not by the difference's), B has dt, and the sums of 16 are two of 8 and one a
 // tile.  Error of y against 64 bits, before these | with them | recurrence: 64 tokens that decay by e^-50 5.6e-7 | 1.0e-7 | 0.9e-7, slowly 1.7e-7 | 1.0e-7 | 1.9e-7; with a
 // mixer's inputs 64 tokens 3.1e-8 | 3.1e-8, 6 000: 3.0e-8 | 3.2e-8 (with | recurrence).  They take 1 - 4 % (2 x 4 096 tokens 85 -> 88.5 us): the lengths between are as they were.
+// A chunk with a token that leaves nothing of what was before it (dt A below -80, an infinite dt among them), or whose dt or dt A is otherwise out of the ordinary, goes token by
+// token: dt B, sums of dt A and differences of them are infinite or NaN there while the recurrence's products are not.
 template <bool OUT, bool FINE>
 __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
   __shared__ __attribute__((aligned(16))) float sv[4][FINE ? 4 : 3][FQ];         // a wave's own: cs, dt, weights of the state, what cs has lost
@@ -123,8 +162,15 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
     float d = raw + bias;
     if (a.softplus) d = softplus_f(d);
     d = lane < tt ? fminf(fmaxf(d, a.dt_min), a.dt_max) : 0.f;
+    const float da = d * Ah;
+    if constexpr (FINE) {
+      if (__ballot(!(da > -80.f && da < 1.f && d < 0x1p20f)) != 0) {
+        own += march<OUT>(a, xb, Bb, Cb, t0, tt, d, da, Dh, lc, q, b, h, pt, S);
+        continue;
+      }
+    }
     float lost = 0.f;
-    const float da = d * Ah, cs = FINE ? scan_both(da, lost) : wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
+    const float cs = FINE ? scan_both(da, lost) : wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
     // what decays behind a token, summed from the end: cend - cs would carry the rounding of the whole chunk's sum into the tokens that weigh most
     const float back = from_lane(wave_incl_scan_dpp(from_lane(da, 63 - lane)), 62 - lane);
     own += cend;
@@ -284,7 +330,11 @@ int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* 
   a.xsb = xsb; a.xsl = xsl; a.dsb = dsb; a.dsl = dsl; a.bsb = bsb; a.bsl = bsl; a.bsg = bsg; a.csb = csb; a.csl = csl; a.csg = csg; a.ysb = ysb; a.ysl = ysl;
   a.softplus = dt_softplus; a.group_map = group_map; a.dt_min = dt_min; a.dt_max = dt_max;
   const int units = headdim / 16 * a.nseg;
-  if (a.nseg > 1) ssd_f32_kernel<false, false><<<dim3((unsigned)((units - headdim / 16 + 3) / 4), (unsigned)nheads, (unsigned)batch), 256, 0, st>>>(a);
+  const dim3 first((unsigned)((units - headdim / 16 + 3) / 4), (unsigned)nheads, (unsigned)batch);
+  if (a.nseg > 1) {
+    if (fine) ssd_f32_kernel<false, true><<<first, 256, 0, st>>>(a);
+    else ssd_f32_kernel<false, false><<<first, 256, 0, st>>>(a);
+  }
   const dim3 grid((unsigned)((units + 3) / 4), (unsigned)nheads, (unsigned)batch);
   if (fine) ssd_f32_kernel<true, true><<<grid, 256, 0, st>>>(a);
   else ssd_f32_kernel<true, false><<<grid, 256, 0, st>>>(a);
