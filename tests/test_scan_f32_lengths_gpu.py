@@ -113,3 +113,30 @@ def test_a_step_that_resets_without_end(L, at, init, step):
     rel = 2.0 ** -18                                                       # (as above)
     assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
     assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5) if step < 1e38 else (dec < -1e37).all()
+
+
+@pytest.mark.parametrize("L,seeds", [(48, 4), (64, 4), (5000, 1)])
+@pytest.mark.parametrize("A", [1.0, 0.3, 1e-3, None])
+def test_error_is_no_larger_than_token_by_token(L, seeds, A):
+    """against 64 bits, in the mean over the elements: y and the state as the recurrence leaves them, or nearer"""
+    from timeviper_amd import kernels as ops
+    H, errors = 32, {}
+    for seed in range(seeds):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        r = lambda *s: torch.randn(s, generator=g, device=DEV)
+        x, Bm, Cm, dt = r(1, L, H, 64), 0.3 * r(1, L, 2, 16), r(1, L, 2, 16), r(1, L, H)
+        Ah, D, S0 = -(torch.linspace(.5, 8, H, device=DEV) if A is None else torch.full((H,), A, device=DEV)), r(H), r(1, H, 64, 16)
+        want, S, _, _ = reference(x.double(), F.softplus(dt.double()), Ah.double(), Bm.double(), Cm.double(), D.double(), S0.double(), torch.arange(H, device=DEV) // 16)
+        for impl, kernel in ((0, 11), (1, 1)):
+            ops.ssd_scan_set_impl(impl)
+            try:
+                y, fin = ops.mamba_chunk_scan_combined(x, dt, Ah, Bm, Cm, D=D, dt_softplus=True, initial_states=S0, return_final_states=True)
+                assert ops.ssd_scan_last_kernel() == kernel
+            finally:
+                ops.ssd_scan_set_impl(0)
+            for what, a, b in (("y", y, want), ("state", fin, S)):
+                errors.setdefault((what, kernel), []).append(((a.double() - b).norm() / b.norm()).item())
+    for what in ("y", "state"):
+        here, there = (sum(errors[what, k]) / seeds for k in (11, 1))
+        print(f"{what} {here:.3e} {there:.3e}")
+        assert here <= there

@@ -53,6 +53,8 @@ __device__ __forceinline__ float scan_both(float v, float& lost) {
   return v;
 }
 
+template <bool FINE> __device__ __forceinline__ float exp_of(float v) { return FINE ? expf(v) : __expf(v); }
+
 // A chunk token by token, as the recurrence has it (ssd_generic.hip): S, y of the wave's columns; d and da are of token `lane`.  Returns the sum of da.
 template <bool OUT>
 __device__ __forceinline__ float march(const F3Args& a, const float* xb, const float* Bb, const float* Cb, int t0, int tt, float d, float da, float Dh, int lc, int q, int b, int h,
@@ -90,17 +92,24 @@ __device__ __forceinline__ float march(const F3Args& a, const float* xb, const f
   return sum;
 }
 
-// OUT: the second launch.  FINE: for the lengths that the token recurrence had before (48 - 64 tokens, more than 4 096), whose error is kept: two tokens' decay is the difference
-// of their sums AND of what these have lost (a sum over a chunk is rounded by its own size, not by the difference's), B has dt, and the sums of 16 are two of 8 and one a
-// tile.  Error of y against 64 bits, before these | with them | recurrence: 64 tokens that decay by e^-50 5.6e-7 | 1.0e-7 | 0.9e-7, slowly 1.7e-7 | 1.0e-7 | 1.9e-7; with a
-// mixer's inputs 64 tokens 3.1e-8 | 3.1e-8, 6 000: 3.0e-8 | 3.2e-8 (with | recurrence).  They take 1 - 4 % (2 x 4 096 tokens 85 -> 88.5 us): the lengths between are as they were.
-// A chunk with a token that leaves nothing of what was before it (dt A below -80, an infinite dt among them), or whose dt or dt A is otherwise out of the ordinary, goes token by
-// token: dt B, sums of dt A and differences of them are infinite or NaN there while the recurrence's products are not.
+// OUT: the second launch.  FINE: for the lengths that the token recurrence had before (48 - 64 tokens, more than 4 096), whose error and whose results at extreme steps are kept:
+//   * two tokens' decay is the difference of their sums AND of what these have lost (a sum over a chunk is rounded by its own size, not by the difference's);
+//   * the four steps of a contraction of 16 tokens are numbered in time (step r, quarter q: token 4 r + q; the rows of G^T are dealt out to match), so that what weighs most is added
+//     last and rounded once, as by the recurrence; B has dt, and its sum with C over n is a tree;
+//   * the decays of the state's weights are sums that keep what they lose, and their exponentials are the recurrence's own;
+//   * a chunk with a token that leaves nothing of what was before it (dt A below -80, an infinite dt among them), or whose dt or dt A is otherwise out of the ordinary, goes token by
+//     token (dt B, sums of dt A and differences of them are infinite or NaN there while the recurrence's products are not).
+// Error against 64 bits, recurrence | here, 64 tokens of 32 heads x 64 that decay by e^-52: y 7.5e-8 | 7.2e-8, state 6.0e-8 | 5.7e-8; by e^-15: 8.8e-8 | 8.6e-8, 7.0e-8 | 6.7e-8; slowly:
+// 2.2e-7 | 1.4e-7, 2.8e-7 | 1.6e-7; 5 000 tokens: 7.3e-8 | 6.9e-8, 6.1e-8 | 5.5e-8, slowly 4.0e-6 | 3.7e-7 (steps numbered as at the other lengths: 8.4e-8 for the first).
+// All of this takes 5 - 12 % (64 tokens 7.8 -> 8.8 us, 8 192: 95 -> 99.5): the lengths between are as they were.  A reset in every chunk: 64 tokens 21 us (token by token
+// 24), 8 192: 269 (2 695).
 template <bool OUT, bool FINE>
 __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
   __shared__ __attribute__((aligned(16))) float sv[4][FINE ? 4 : 3][FQ];         // a wave's own: cs, dt, weights of the state, what cs has lost
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lc = lane & 15, q = lane >> 4;
+  auto tok = [&](int r) __attribute__((always_inline)) { return FINE ? 4 * r + q : 4 * q + r; };       // of the 16: step r's token in this quarter
+  const int row = FINE ? (lc & 3) << 2 | lc >> 2 : lc, slot = FINE ? (lane & 48) | row : lane;           // the token of row lc of G^T; where a lane's token stands, four of a quarter side by side
   const int pt_n = a.P >> 4, unit = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
   const int seg = unit / pt_n, pt = unit - seg * pt_n;
   if (seg >= (OUT ? a.nseg : a.nseg - 1)) return;                     // (no barrier in this kernel)
@@ -146,7 +155,7 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
     for (int st = 0; st < 4; ++st)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t t = t0 + min(16 * st + 4 * q + r, tt - 1);
+        const int64_t t = t0 + min(16 * st + tok(r), tt - 1);
         xa[st][r] = xb[t * a.xsl + lc];
         bn[st][r] = Bb[t * a.bsl + lc];
       }
@@ -154,7 +163,7 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         const int64_t t = t0 + min(16 * st + lc, tt - 1);
-        ba[st] = *(const f32x4*)(Bb + t * a.bsl + 4 * q);
+        ba[st] = *(const f32x4*)(Bb + (t0 + min(16 * st + row, tt - 1)) * a.bsl + 4 * q);
         ca[st] = *(const f32x4*)(Cb + t * a.csl + 4 * q);
         xd[st] = *(const f32x4*)(xb + t * a.xsl + 4 * q);
       }
@@ -172,20 +181,23 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
     float lost = 0.f;
     const float cs = FINE ? scan_both(da, lost) : wave_incl_scan_dpp(da), cend = rdlane(cs, 63);      // (tokens past the end add 0)
     // what decays behind a token, summed from the end: cend - cs would carry the rounding of the whole chunk's sum into the tokens that weigh most
-    const float back = from_lane(wave_incl_scan_dpp(from_lane(da, 63 - lane)), 62 - lane);
+    float behind, behind_lost = 0.f;
+    if constexpr (FINE) behind = scan_both(from_lane(da, 63 - lane), behind_lost);
+    else behind = wave_incl_scan_dpp(from_lane(da, 63 - lane));
+    const float back = from_lane(behind + behind_lost, 62 - lane);
     own += cend;
-    sv[wave][0][lane] = cs;
-    sv[wave][1][lane] = d;
-    if constexpr (FINE) sv[wave][3][lane] = lost;
-    sv[wave][2][lane] = lane == 63 ? d : __expf(back) * d;
+    sv[wave][0][slot] = cs;
+    sv[wave][1][slot] = d;
+    if constexpr (FINE) sv[wave][3][slot] = lost;
+    sv[wave][2][slot] = lane == 63 ? d : exp_of<FINE>(back) * d;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (a wave's own LDS: in order)
     if (tt < FQ) {                                                    // rows past the end are zeros, as tokens that are not there
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (16 * st + 4 * q + r >= tt) xa[st][r] = bn[st][r] = 0.f;
-        if (OUT && 16 * st + lc >= tt) ba[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (16 * st + tok(r) >= tt) xa[st][r] = bn[st][r] = 0.f;
+        if (OUT && 16 * st + row >= tt) ba[st] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
     if constexpr (OUT) {
@@ -205,7 +217,7 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
       }
 #pragma unroll
       for (int ot = 0; ot < 4; ++ot) {                                // 16 output tokens
-        const float cst = sv[wave][0][16 * ot + lc], clt = FINE ? sv[wave][FINE ? 3 : 0][16 * ot + lc] : 0.f, et = __expf(cst);
+        const float cst = sv[wave][0][16 * ot + row], clt = FINE ? sv[wave][FINE ? 3 : 0][16 * ot + row] : 0.f, et = __expf(cst);
         f32x4 Y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 4; ++k) Y = mfma4(S[k], ca[ot][k], Y);
@@ -215,10 +227,8 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
         for (int st = 0; st <= ot; ++st) {
           f32x4 M = {0.f, 0.f, 0.f, 0.f};
           if constexpr (FINE) {
-            f32x4 M1 = M;
-            M = mfma4(ba[st][1], ca[ot][1], mfma4(ba[st][0], ca[ot][0], M));
-            M1 = mfma4(ba[st][3], ca[ot][3], mfma4(ba[st][2], ca[ot][2], M1));
-            M += M1;
+            const f32x4 z = M;
+            M = (mfma4(ba[st][0], ca[ot][0], z) + mfma4(ba[st][1], ca[ot][1], z)) + (mfma4(ba[st][2], ca[ot][2], z) + mfma4(ba[st][3], ca[ot][3], z));
           } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) M = mfma4(ba[st][k], ca[ot][k], M);
@@ -228,13 +238,13 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
             float gap = cst - css[st][r];
             if constexpr (FINE) gap += clt - cls[st][r];
             const float m = FINE ? __expf(gap) * M[r] : __expf(gap) * ds[st][r] * M[r];
-            M[r] = st < ot || 4 * q + r <= lc ? m : 0.f;
+            M[r] = st < ot || tok(r) <= lc ? m : 0.f;
           }
           if (st == ot && odd) {
             // (a factor of 0 does not hide an infinity or a NaN from the tokens in front of it: term by term)
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
-              const float m = from_lane(M[t & 3], 16 * (t >> 2) + lc);
+              const float m = FINE ? from_lane(M[t >> 2], 16 * (t & 3) + lc) : from_lane(M[t & 3], 16 * (t >> 2) + lc);
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
                 const float xt = from_lane(xd[ot][r], 16 * q + t);
@@ -242,12 +252,8 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
               }
             }
           } else {
-            f32x4 Z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if constexpr (FINE) Z = mfma4(xa[st][r], M[r], Z);
-              else Y = mfma4(xa[st][r], M[r], Y);
-            if constexpr (FINE) Y += Z;
+            for (int r = 0; r < 4; ++r) Y = mfma4(xa[st][r], M[r], Y);
           }
         }
         if (16 * ot + lc < tt) {
@@ -259,7 +265,7 @@ __global__ __launch_bounds__(256) void ssd_f32_kernel(F3Args a) {
       }
     }
     if (next) {
-      const float ec = __expf(cend);
+      const float ec = exp_of<FINE>(cend);
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[r] *= ec;
 #pragma unroll

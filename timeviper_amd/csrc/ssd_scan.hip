@@ -173,7 +173,8 @@ static int scan_impl(const void* x, const void* dt, const void* A, const void* B
     return rc;
   }
   // Lengths that ssd_chunked.hip leaves out (up to 64 tokens, more than 4 096), on the matrix cores where their rows allow it.  us, token by token | here, 32 heads x 64: 48 tokens
-  // 17.7 | 7.5, 64: 22 | 7.5, 8 192: 2 690 | 104; 128 x 128, 64: 28 | 8.6; 24: 10.2 | 7.4, but the recurrence's error is the smaller one there by some per cent
+  // 17.7 | 8.7, 64: 22 | 8.8, 8 192: 2 690 | 100; 128 x 128, 64: 28 | 9.8; 24: 10.2 | 7.4, left to the recurrence, whose error was the smaller one by some per cent when
+  // the line was drawn
   if (forced == 0 && dtype == TV_F32 && workspace && (uintptr_t)workspace % 16 == 0 && seqlen >= F32_FROM &&
       workspace_bytes >= tv_ssd_f32_workspace_bytes(batch, seqlen, nheads, headdim, dstate) &&
       tv_ssd_f32_supported(headdim, dstate, x_stride_b, x_stride_l, b_stride_b, b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b, y_stride_l, x,
