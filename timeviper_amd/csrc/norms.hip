@@ -277,16 +277,15 @@ __global__ __launch_bounds__(NORM_THREADS) void layernorm_wave_kernel(
   }
 }
 
-// The same rows, RPW consecutive ones per wave: weight, bias and the fp32 row bias are loaded ONCE per wave and stay in
-// registers, and row r + 1 is requested before row r is reduced.  Per row the kernel above issues 5 loads for every
+// The same rows, RPW per wave, rows / RPW apart: weight, bias and the fp32 row bias are loaded ONCE per wave and stay in
+// registers, and a row is requested before the one in front of it is reduced.  Per row the kernel above issues 5 loads for every
 // 16 bytes of x it reads (x, 2 of the row bias, w, b: 11.5 KB through the CU's L1 for 2.3 KB from HBM); at the ViT's
 // 1.5 M rows x 1 152 that load path, not HBM, set the pace of the row-bias form (4.9 against 5.3 TB/s for the plain one).
 // NV = 16-byte vectors per lane (ceil(D / V / 64)), a template parameter so that the register count follows the row.
-template <typename T, int NV, int RPW, bool DELTA>
-__global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 4) void layernorm_rows_kernel(
-    const T* __restrict__ x, const T* __restrict__ delta, const T* __restrict__ w,
-    const T* __restrict__ bias, const float* __restrict__ row_bias, T* __restrict__ sum_out,
-    T* __restrict__ y, int64_t rows, int D, int64_t xs, int64_t ds, int64_t ss, int64_t ys, float eps) {
+template <typename T, int NV, int RPW>
+__global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : NV == 3 ? 3 : 4) void layernorm_rows_kernel(
+    const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, const float* __restrict__ row_bias,
+    T* __restrict__ y, int64_t rows, int D, int64_t xs, int64_t ys, float eps) {
   constexpr int V = Vec16<T>::N;
   typedef typename Vec16<T>::type vec_t;
   const int64_t chunk = (rows + RPW - 1) / RPW, row0 = (int64_t)blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6);
@@ -316,43 +315,27 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 
       }
     }
   }
-  constexpr int NVD = DELTA ? NV : 1;
-  vec_t xv[NV], dv[NVD], xn[NV], dn[NVD];
-  auto load_row = [&](int64_t row, vec_t (&xo)[NV], vec_t (&dd)[NVD]) {
+  vec_t xv[NV], xn[NV];
+  auto load_row = [&](int64_t row, vec_t (&xo)[NV]) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int iv = lane + k * 64;
-      if (iv < nv) {
-        xo[k] = get<true, vec_t>(x + row * xs + (int64_t)iv * V);
-        if (DELTA) dd[k % NVD] = *(const vec_t*)(delta + row * ds + (int64_t)iv * V);
-      }
+      if (iv < nv) xo[k] = get<true, vec_t>(x + row * xs + (int64_t)iv * V);
     }
   };
-  load_row(row0, xv, dv);
+  load_row(row0, xv);
   for (int r = 0; r < nrow; ++r) {
     const int64_t row = row0 + r * chunk;
-    if (r + 1 < nrow) load_row(row + chunk, xn, dn);
+    if (r + 1 < nrow) load_row(row + chunk, xn);
     float vals[NV][V];
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int iv = lane + k * 64;
       if (iv < nv) {
-        if (DELTA) {
-          vec_t sv;
-#pragma unroll
-          for (int i = 0; i < V; ++i) {
-            sv[i] = from_f32<T>(to_f32(xv[k][i]) + to_f32(dv[k % NVD][i]));
-            vals[k][i] = to_f32(sv[i]);
-          }
-          if (sum_out) *(vec_t*)(sum_out + row * ss + (int64_t)iv * V) = sv;
-        } else {
-#pragma unroll
-          for (int i = 0; i < V; ++i) vals[k][i] = to_f32(xv[k][i]);
-        }
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-          vals[k][i] += rb[k][i];
+          vals[k][i] = to_f32(xv[k][i]) + rb[k][i];
           s1 += vals[k][i];
         }
       }
@@ -382,8 +365,6 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : DELTA || NV == 3 ? 3 : 
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) xv[k] = xn[k];
-#pragma unroll
-    for (int k = 0; k < NVD; ++k) dv[k] = dn[k];
   }
 }
 
@@ -603,8 +584,8 @@ int launch_ln(const void* x, const void* delta, const void* w, const void* b, co
     // replacement: 34 992 x 1 152 35.6 -> 32.5 us (apart alone 35.0, normal stores 33.9), 200 000: 171 -> 156
     const int64_t nblk = (rows + (NORM_THREADS / 64) * RPW - 1) / ((NORM_THREADS / 64) * RPW);
 #define TV_LN_ROWS(NV)                                                                                              \
-    layernorm_rows_kernel<T, NV, RPW, false><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                         \
-        (const T*)x, nullptr, (const T*)w, (const T*)b, rb, (T*)sum_out, (T*)y, rows, D, xs, ds, ss, ys, eps)
+    layernorm_rows_kernel<T, NV, RPW><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                                \
+        (const T*)x, (const T*)w, (const T*)b, rb, (T*)y, rows, D, xs, ys, eps)
     with_vectors(D / V, 64, [&](auto nv) {
       TV_LN_ROWS(nv());
     });
