@@ -74,3 +74,13 @@ def test_layer(dtype, rows):
         y, s = ops.layer_norm(x, w, b, 1e-6, residual=d, return_sum=True)
         assert torch.equal(s, (x.float() + d.float()).to(dtype))
         check(y, s)
+
+
+@pytest.mark.parametrize("dtype,D,past", [(torch.bfloat16, 1152, 0), (torch.bfloat16, 1152, 1), (torch.float32, 520, 3), (torch.float16, 2048, 7)])
+def test_layer_on_either_side_of_the_size_that_is_stored_past_the_caches(dtype, D, past):
+    """the last row count in front of the line (0), and behind it: the same bits as from calls of fewer rows"""
+    rows = ((320 << 20) - 1) // (D * dtype.itemsize) + past
+    x, w, b, rb = r(rows, D, dtype=dtype), r(D, dtype=dtype), r(D, dtype=dtype, seed=1), r(D, dtype=torch.float32, seed=2)
+    y = ops.layer_norm(x, w, b, 1e-6, row_bias=rb)
+    for part in torch.arange(rows, device=DEV).split(40000):
+        assert torch.equal(y[part], ops.layer_norm(x[part], w, b, 1e-6, row_bias=rb))

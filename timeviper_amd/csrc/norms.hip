@@ -22,6 +22,7 @@ namespace {
 constexpr int NORM_THREADS = 256;
 constexpr int NORM_MAXV = 4;  // 16-byte vectors cached per thread
 constexpr int64_t STREAM_FROM = 144ll << 20;   // bytes read and written
+constexpr int64_t LN_STREAM_FROM = 320ll << 20;   // bytes written, LayerNorm of many rows
 
 // V fp32 or 16-bit values behind p, as loaded (16-byte loads) and as floats
 template <typename W, int V>
@@ -282,7 +283,8 @@ __global__ __launch_bounds__(NORM_THREADS) void layernorm_wave_kernel(
 // 16 bytes of x it reads (x, 2 of the row bias, w, b: 11.5 KB through the CU's L1 for 2.3 KB from HBM); at the ViT's
 // 1.5 M rows x 1 152 that load path, not HBM, set the pace of the row-bias form (4.9 against 5.3 TB/s for the plain one).
 // NV = 16-byte vectors per lane (ceil(D / V / 64)), a template parameter so that the register count follows the row.
-template <typename T, int NV, int RPW>
+// STREAM: y past the caches too
+template <typename T, int NV, int RPW, bool STREAM>
 __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : NV == 3 ? 3 : 4) void layernorm_rows_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, const float* __restrict__ row_bias,
     T* __restrict__ y, int64_t rows, int D, int64_t xs, int64_t ys, float eps) {
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(NORM_THREADS, NV >= 4 ? 2 : NV == 3 ? 3 : 4) void l
 #pragma unroll
         for (int i = 0; i < V; ++i)
           o[i] = from_f32<T>((vals[k][i] - mean) * rstd * to_f32(wv[k][i]) + to_f32(bv[k][i]));
-        put<true>(y + row * ys + (int64_t)iv * V, o);
+        put<STREAM>(y + row * ys + (int64_t)iv * V, o);
       }
     }
 #pragma unroll
@@ -580,14 +582,18 @@ int launch_ln(const void* x, const void* delta, const void* w, const void* b, co
     // many rows (the ViT's stream form: row bias, no residual operand): a wave keeps the parameters in registers for RPW
     // rows — 1 272 against 1 416 us per 1.49 M rows x 1 152 (5.41 against 4.86 TB/s); with a residual operand the
     // one-row kernel is the faster one (2 502 against 2 654 us: the second operand's registers cost a wave per SIMD).
-    // A wave's rows lie rows / RPW apart, so that all waves together read one front of memory, and past the caches' normal
-    // replacement: 34 992 x 1 152 35.6 -> 32.5 us (apart alone 35.0, normal stores 33.9), 200 000: 171 -> 156
+    // A wave's rows lie rows / RPW apart, so that all waves together read one front of memory, x past the caches' normal
+    // replacement.  y passes by it only where it is larger than the last-level cache, of which the product behind the norm
+    // reads it: norm and 3 456-wide product of 32 768 x 768 144 us streamed, 133 as it is, 34 992 x 1 152 277 | 272,
+    // 60 000: 461 | 455, 120 000: 889 | 888, 180 000: 1 318 | 1 321 (the norm alone 145 | 156), 300 000 alone 237 | 254;
+    // x in the normal way too 34 992 x 1 152 279, 60 000: 464
     const int64_t nblk = (rows + (NORM_THREADS / 64) * RPW - 1) / ((NORM_THREADS / 64) * RPW);
-#define TV_LN_ROWS(NV)                                                                                              \
-    layernorm_rows_kernel<T, NV, RPW><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                                \
+#define TV_LN_ROWS(STREAM)                                                                                          \
+    layernorm_rows_kernel<T, nv(), RPW, STREAM><<<dim3((unsigned)nblk), NORM_THREADS, 0, s>>>(                      \
         (const T*)x, (const T*)w, (const T*)b, rb, (T*)y, rows, D, xs, ys, eps)
     with_vectors(D / V, 64, [&](auto nv) {
-      TV_LN_ROWS(nv());
+      if (rows * D * (int64_t)sizeof(T) >= LN_STREAM_FROM) TV_LN_ROWS(true);
+      else TV_LN_ROWS(false);
     });
 #undef TV_LN_ROWS
   } else if (D / V <= 64 * NORM_MAXV) {
