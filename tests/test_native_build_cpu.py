@@ -1,0 +1,34 @@
+"""What the operators' native host side is built from, and that nothing else is used in its place."""
+import importlib.machinery
+
+import pytest
+import torch
+
+from timeviper_amd import _capi, _native, build
+
+
+def test_what_is_loaded_is_built_from_this_tree():
+    build.ensure_built()
+    assert _native.ops.built_from == build.native_id() == build.NATIVE_ID.read_text()
+    assert any(build.NATIVE.name == "_tv_native" + s for s in importlib.machinery.EXTENSION_SUFFIXES)
+
+
+@pytest.mark.parametrize("what,value", [("NATIVE_FLAGS", ["-O3"]), ("NATIVE_LIBS", ["-lc10"]), ("CXX", "c++"), ("NATIVE", build.NATIVE.with_name("_tv_native.cpython-399-x.so"))])
+def test_a_change_of_what_it_is_built_with_is_another_build(what, value, monkeypatch):
+    before = build.native_id()
+    monkeypatch.setattr(build, what, value)
+    assert build.native_id() != before and not build.native_is_current()
+
+
+def test_another_torch_is_another_build(monkeypatch):
+    before = build.native_id()
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    assert build.native_id() != before
+
+
+def test_a_binary_of_other_sources_is_not_used(monkeypatch):
+    """not even with the tree's id beside it"""
+    monkeypatch.setattr(build, "native_id", lambda: "another")
+    monkeypatch.setattr(build, "native_is_current", lambda: True)
+    with pytest.raises(_capi.TimeViperHipError, match="other sources"):
+        _native._Ops().rms_norm

@@ -15,6 +15,7 @@ import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -23,8 +24,8 @@ CSRC = ROOT / "csrc"
 OBJ = ROOT / "lib" / "obj"
 LIB = ROOT / "lib" / "libtimeviper_hip.so"
 LIB_ID = ROOT / "lib" / "libtimeviper_hip.id"
-NATIVE = ROOT / "lib" / "_tv_native.so"          # the operators' host side: a Python extension on torch's headers, no device code
-NATIVE_ID = ROOT / "lib" / "_tv_native.id"
+NATIVE = ROOT / "lib" / f"_tv_native{sysconfig.get_config_var('EXT_SUFFIX') or '.so'}"      # the operators' host side: a Python extension on torch's headers, no device code
+NATIVE_ID = NATIVE.with_suffix(".id")
 NATIVE_SRC = CSRC / "host" / "native_ops.cpp"
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -109,34 +110,39 @@ def build(force: bool = False, jobs: int = 0) -> Path:
     return LIB
 
 
-def _native_flags():
-    import sysconfig
+CXX = os.environ.get("CXX", "g++")
+NATIVE_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+NATIVE_LIBS = ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+
+
+def _native_paths():
     import torch
     t = Path(torch.__file__).resolve().parent
     rocm = Path(HIPCC).resolve().parent.parent if Path(HIPCC).is_absolute() else Path("/opt/rocm")
-    inc = [ROOT.parent / "include", t / "include", t / "include" / "torch" / "csrc" / "api" / "include", "/opt/rocm/include", rocm / "include", sysconfig.get_paths()["include"]]
-    return (["-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"] + [f"-I{p}" for p in inc],
-            [f"-L{t / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], torch.__version__)
+    return [f"-I{p}" for p in (ROOT.parent / "include", t / "include", t / "include" / "torch" / "csrc" / "api" / "include", "/opt/rocm/include", rocm / "include",
+                               sysconfig.get_paths()["include"])], [f"-L{t / 'lib'}"]
 
 
 def native_id() -> str:
-    """Hash of the host operators' source, the C ABI's header and torch's version"""
+    """Hash of all that the host operators are built from: source, the C ABI's header, flags, compiler, Python's ABI, torch's version (not the paths: a tree may be copied)"""
     import torch
-    return _hash([NATIVE_SRC, ROOT.parent / "include" / "timeviper_hip.h"], torch.__version__)
+    return _hash([NATIVE_SRC, ROOT.parent / "include" / "timeviper_hip.h"],
+                 " ".join([CXX, *NATIVE_FLAGS, *NATIVE_LIBS, NATIVE.name, torch.__version__, str(torch.version.hip)]))
 
 
 def native_is_current() -> bool:
+    """By the file beside it; what is loaded is asked itself (_native.py)"""
     return NATIVE.exists() and NATIVE_ID.exists() and NATIVE_ID.read_text() == native_id()
 
 
 def build_native(force: bool = False) -> Path:
     if force or not native_is_current():
-        flags, libs, _ = _native_flags()
+        want, (includes, paths) = native_id(), _native_paths()
         NATIVE.parent.mkdir(parents=True, exist_ok=True)
-        r = subprocess.run([os.environ.get("CXX", "g++"), *flags, str(NATIVE_SRC), "-o", str(NATIVE), *libs], capture_output=True, text=True)
+        r = subprocess.run([CXX, *NATIVE_FLAGS, f'-DTV_NATIVE_ID="{want}"', *includes, str(NATIVE_SRC), "-o", str(NATIVE), *paths, *NATIVE_LIBS], capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"host operators: {r.stdout}\n{r.stderr}")
-        NATIVE_ID.write_text(native_id())
+        NATIVE_ID.write_text(want)
     return NATIVE
 
 

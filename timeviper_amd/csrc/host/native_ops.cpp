@@ -477,4 +477,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_tv_native", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__tv_native() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__tv_native() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_from", TV_NATIVE_ID) < 0) { Py_DECREF(m); return nullptr; }      // build.native_id() of the sources
+  return m;
+}
