@@ -1,5 +1,7 @@
 """What the operators' native host side is built from, and that nothing else is used in its place."""
 import importlib.machinery
+import subprocess
+from pathlib import Path
 
 import pytest
 import torch
@@ -32,3 +34,24 @@ def test_a_binary_of_other_sources_is_not_used(monkeypatch):
     monkeypatch.setattr(build, "native_is_current", lambda: True)
     with pytest.raises(_capi.TimeViperHipError, match="other sources"):
         _native._Ops().rms_norm
+
+
+def test_a_build_never_shows_half_a_file(tmp_path, monkeypatch):
+    """while the linker writes, and where it fails, what was there before stays"""
+    there, tag = tmp_path / build.NATIVE.name, tmp_path / build.NATIVE_ID.name
+    there.write_bytes(b"the old one")
+    monkeypatch.setattr(build, "NATIVE", there)
+    monkeypatch.setattr(build, "NATIVE_ID", tag)
+    seen = []
+
+    def linker(cmd, **k):
+        out = Path(cmd[cmd.index("-o") + 1])
+        out.write_bytes(b"half")
+        seen.append(there.read_bytes())
+        return subprocess.CompletedProcess(cmd, len(seen) == 1, "", "")
+    monkeypatch.setattr(build.subprocess, "run", linker)
+    with pytest.raises(RuntimeError):
+        build.build_native()
+    assert there.read_bytes() == b"the old one" and not tag.exists()
+    build.build_native()
+    assert seen == [b"the old one"] * 2 and there.read_bytes() == b"half" and tag.read_text() == build.native_id() and len(list(tmp_path.iterdir())) == 2

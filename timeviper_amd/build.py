@@ -16,6 +16,7 @@ import os
 import subprocess
 import sys
 import sysconfig
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -139,10 +140,15 @@ def build_native(force: bool = False) -> Path:
     if force or not native_is_current():
         want, (includes, paths) = native_id(), _native_paths()
         NATIVE.parent.mkdir(parents=True, exist_ok=True)
-        r = subprocess.run([CXX, *NATIVE_FLAGS, f'-DTV_NATIVE_ID="{want}"', *includes, str(NATIVE_SRC), "-o", str(NATIVE), *paths, *NATIVE_LIBS], capture_output=True, text=True)
-        if r.returncode != 0:
-            raise RuntimeError(f"host operators: {r.stdout}\n{r.stderr}")
-        NATIVE_ID.write_text(want)
+        # linked beside its place and moved there whole: another process may load it, or build it too, at any time
+        with tempfile.TemporaryDirectory(dir=NATIVE.parent) as work:
+            out, tag = Path(work) / NATIVE.name, Path(work) / NATIVE_ID.name
+            r = subprocess.run([CXX, *NATIVE_FLAGS, f'-DTV_NATIVE_ID="{want}"', *includes, str(NATIVE_SRC), "-o", str(out), *paths, *NATIVE_LIBS], capture_output=True, text=True)
+            if r.returncode != 0:
+                raise RuntimeError(f"host operators: {r.stdout}\n{r.stderr}")
+            tag.write_text(want)
+            os.replace(out, NATIVE)
+            os.replace(tag, NATIVE_ID)
     return NATIVE
 
 
