@@ -1,6 +1,7 @@
 """What the operators' native host side is built from, and that nothing else is used in its place."""
 import importlib.machinery
 import subprocess
+import warnings
 from pathlib import Path
 
 import pytest
@@ -29,11 +30,36 @@ def test_another_torch_is_another_build(monkeypatch):
 
 
 def test_a_binary_of_other_sources_is_not_used(monkeypatch):
-    """not even with the tree's id beside it"""
+    """not even with the tree's id beside it: a warning, and kernels.py goes its own way"""
     monkeypatch.setattr(build, "native_id", lambda: "another")
     monkeypatch.setattr(build, "native_is_current", lambda: True)
-    with pytest.raises(_capi.TimeViperHipError, match="other sources"):
-        _native._Ops().rms_norm
+    ops = _native._Ops()
+    with pytest.warns(RuntimeWarning, match="other sources"):
+        assert ops.rms_norm(1, 2, 3, 4, 5) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert ops.rms_norm() is None and ops.scan() is None and ops.native is None
+
+
+@pytest.mark.parametrize("broken", ["missing", "no extension", "another library"])
+def test_without_it_the_operators_go_through_ctypes(broken, tmp_path, monkeypatch):
+    if broken == "another library":
+        monkeypatch.setattr(_capi, "lib_path", lambda: tmp_path / "none.so")
+    else:
+        monkeypatch.setattr(build, "NATIVE", tmp_path / "none.so")
+        monkeypatch.setattr(build, "native_id", lambda n=build.native_id(): n)
+        if broken == "no extension":
+            (tmp_path / "none.so").write_bytes(b"no ELF")
+    with pytest.warns(RuntimeWarning, match="through ctypes"):
+        assert _native._Ops().rms_norm() is None
+
+
+def test_a_build_without_a_host_compiler_makes_the_library(tmp_path, monkeypatch, capfd):
+    monkeypatch.setattr(build, "CXX", str(tmp_path / "no-compiler"))
+    monkeypatch.setattr(build, "NATIVE", tmp_path / "_tv_native.so")
+    monkeypatch.setattr(build, "NATIVE_ID", tmp_path / "_tv_native.id")
+    assert build.ensure_built() == build.LIB and not build.NATIVE.exists()
+    assert "go through ctypes" in capfd.readouterr().err
 
 
 def test_a_build_never_shows_half_a_file(tmp_path, monkeypatch):
