@@ -25,6 +25,32 @@ def rel(a, b):
     return ((a.double() - b.double()).norm() / b.double().norm()).item()
 
 
+def where_they_differ(a, b, passes=()):
+    """Which elements of two results differ, for an assertion's message; passes: what `block_sums` noted of either"""
+    rows = (a != b).flatten(0, -2).any(-1).nonzero().flatten()
+    cols = (a != b).flatten(0, -2).any(0).nonzero().flatten()
+    first = next((f"block {i}, {name}, rows {(u != v).flatten().nonzero().flatten()[:8].tolist()}" for i, (p, q) in enumerate(zip(*passes))
+                  for name, u, v in zip(("stream", "branch"), p, q) if not torch.equal(u, v)), "no block")
+    return (f"{int((a != b).sum())} of {a.numel()} elements differ, by {float((a.float() - b.float()).abs().max())} at most; {rows.numel()} of {a[..., 0].numel()} rows, "
+            f"{rows[:8].tolist()} .. {rows[-1:].tolist()}; {cols.numel()} columns, {cols[:8].tolist()} .. {cols[-1:].tolist()}; they part at {first}")
+
+
+def block_sums(run):
+    """run() and, of each block of the video tower in turn, the sums of its two results' bits by row"""
+    from timeviper_amd.model.vit.internvideo2 import Block
+    noted, forward = [], Block.forward_fused
+
+    def noting(self, x, delta):
+        out = forward(self, x, delta)
+        noted.append([t.view(torch.int16).sum(-1, dtype=torch.int64) for t in out])
+        return out
+    Block.forward_fused = noting
+    try:
+        return run(), noted
+    finally:
+        Block.forward_fused = forward
+
+
 def test_config5_rope_causal_attention_131k_tokens_fp8_and_bf16():
     """modeling_qwen2.py:196-244 at full length: rotary embedding of q and k in place (tv_rope_fwd),
     then causal GQA attention — the bf16 kernel and the fp8 MFMA variant — against the definition on
@@ -91,10 +117,13 @@ def test_config5_dual_encoder_4096_frames_equals_members_run_alone():
         md, mv = vb.backbones[bid_d.replace("-", "_")], vb.backbones[bid_v.replace("-", "_")]
         for lo in (0, 1792, T - 256):                     # three of the sixteen 256-frame clips
             clip = pix[lo:lo + 256]
-            feats = vb(clip, is_video=True, clip_frames=256)
+            feats, together = block_sums(lambda: vb(clip, is_video=True, clip_frames=256))
             # the members alone on the same clip: same kernels, same shapes -> the same bits
-            assert torch.equal(feats[bid_d], md(clip)) and feats[bid_d].shape == (256, 256, 1024)
-            assert torch.equal(feats[bid_v], mv(clip.unsqueeze(1), is_video=True)) and feats[bid_v].shape == (64, 1024, 1408)
+            alone_d = md(clip)
+            assert torch.equal(feats[bid_d], alone_d), where_they_differ(feats[bid_d], alone_d)
+            alone_v, alone = block_sums(lambda: mv(clip.unsqueeze(1), is_video=True))
+            assert torch.equal(feats[bid_v], alone_v), where_they_differ(feats[bid_v], alone_v, (together, alone))
+            assert feats[bid_d].shape == (256, 256, 1024) and feats[bid_v].shape == (64, 1024, 1408)
             # projector: frame-wise ToMe beside 4-frame-tube ToMe, interleaved token-wise
             vis_clip = vlm.projector_forward(feats, is_video=True)
             a = pj[bid_d](feats[bid_d], compress=True, local_num_frames=1)
