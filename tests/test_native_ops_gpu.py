@@ -1,5 +1,6 @@
 """The operators' native host side: the same kernels on the same operands, so the same bits as the way through Python, over the forms that both take; what it does not take."""
 import ctypes
+import dataclasses
 import re
 import subprocess
 import threading
@@ -130,12 +131,63 @@ def packed(t):
     yield scatter, 1
 
 
+def products_more(t):
+    """epilogues, rows to write to, splits behind whole tiles, the token side"""
+    for M in (33, 200):
+        x, w, wide = r(M, 512), r(640, 512), r(M, 700, seed=9)
+        for tile in range(4):
+            for b in (None, r(640), r(640, dtype=F32)):
+                for epilogue in (ops.GEMM_BIAS, ops.GEMM_BIAS_GELU, ops.GEMM_GLU)[:3 if b is not None and b.dtype == t else 2]:       # (the gate: a bf16 bias)
+                    yield lambda: ops.small_linear(x, w, b, epilogue, tile=tile), 1
+                yield lambda: ops.small_linear(x, w, b, out=torch.empty(M, 704, dtype=BF, device=DEV)[:, 8:648], tile=tile), 1
+                yield lambda: (ops.small_linear(x, w, b, ops.GEMM_ACCUM, (o := r(M, 704, seed=8))[:, 8:648], tile), o), 1
+        for b in (None, r(640), r(640, dtype=F32)):
+            yield lambda: ops.split_linear(x, w, b, True, 1), 1
+    for b in (None, r(1024)):
+        yield lambda: ops.split_linear(r(3, 200, 1024), r(1024, 1024), b, b is None, 3, 5), 1
+        yield lambda: ops.split_linear(r(600, 1024), r(1024, 1024), b, False, 4, 8), 1
+    for T, D in ((5, 64), (130, 256)):
+        table, ids = r(50, 3, 128)[:, 1], torch.arange(T, device=DEV) * 7 % 50
+        yield lambda: ops.token_side(r(T, 2 * D)[:, D:], ids, table, r(128, D + 8)[:, :D], r(D, 136)[:, 8:]), 1
+
+
+def mixer_more(t):
+    """all that a scan takes beside its operands, the convolution's C.B^T, the state sizes that go elsewhere"""
+    for B, L, P, N, G in ((1, 300, 64, 128, 2), (2, 70, 80, 128, 8), (1, 64, 64, 16, 2), (2, 4100, 32, 16, 1)):
+        H = 16
+        di = H * P
+        wide, w = r(B, L, 8 + di + 2 * G * N + H, dtype=t), r(di + 2 * G * N, 4, dtype=t)
+        dt = wide[..., 8 + di + 2 * G * N:]
+        A, D, bias, init = -torch.rand(H, device=DEV) - .1, r(H, dtype=F32), r(H, dtype=F32), r(B, H, P, N, dtype=F32)
+        x, Bm, Cm, cb = ops.causal_conv1d_xbc(wide[..., 8:8 + di + 2 * G * N], w, None, di, G, N, return_cb=True)
+        x = x.view(B, L, H, P)
+        yield lambda: ops.causal_conv1d_xbc(wide[..., 8:8 + di + 2 * G * N], w, None, di, G, N, activation=None, return_cb=True), 1
+        for c in {None, cb}:
+            for final in (False, True):
+                yield lambda: ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_bias=bias, dt_softplus=True, initial_states=init, return_final_states=final, return_total_decay=True, cb=c), 1
+                yield lambda: ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, dt_bias=bias, dt_softplus=True, return_final_states=final, cb=c), 1
+        yield lambda: ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_softplus=True, dt_limit=(.2, .5), return_total_decay=True), 1
+        yield lambda: ops.mamba_chunk_scan_combined(x, dt.abs(), A, Bm, Cm, D=D, group_map="tile", return_final_states=True), 1
+
+
+def packed_more(t):
+    """a decoded token of every sequence: the state's other route"""
+    B, D = 5, 96
+    p = dataclasses.replace(plan([1] * B, [0, 3, 8, 1, 2], [4, 0, 1, 3, 2], 20), decode=True)
+    x, y = r(B, D, dtype=F32), r(B, 2 * D)[:, D:]
+    for pending in (None, y):
+        for need in (False, True):
+            state = r(5, 3, 2, D, dtype=F32)
+            yield lambda: (ops.norm_shift(x, r(1), 1e-5, pending, None if pending is None else r(D), r(D), (s := state.clone())[:, 1], p, need_h=need), s), 1
+
+
 def flat(v):
     return [t for u in v for t in flat(u)] if isinstance(v, (tuple, list)) else [v]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("forms,dtype", [(norms, BF), (norms, F32), (norms, F16), (mixer, BF), (mixer, F32), (attention, BF), (attention, F16), (products, BF), (packed, BF)])
+@pytest.mark.parametrize("forms,dtype", [(norms, BF), (norms, F32), (norms, F16), (mixer, BF), (mixer, F32), (attention, BF), (attention, F16), (products, BF), (packed, BF),
+                                         (products_more, BF), (mixer_more, BF), (mixer_more, F32), (mixer_more, F16), (packed_more, BF)])
 def test_same_bits(forms, dtype, monkeypatch):
     for call, taken in forms(dtype):
         got = []
@@ -217,6 +269,33 @@ def test_threads_on_streams_of_their_own():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert all(ok)
+
+
+@pytest.mark.gpu
+def test_the_order_of_a_side_stream():
+    """A producer that is still at work on a side stream, the operators, a consumer there, without a wait between: launched anywhere else, an operator would read what was there before"""
+    slow, w, m, out = r(4096, 4096) * 2 ** -6, r(512), r(640, 512), []
+    want = [ops.rms_norm(r(200, 512, seed=i), w, 1e-5) for i in range(6)]
+    want = [(a, ops.mid_linear(a, m), ops.flash_attn_func(*[a.view(1, 50, 4, 512)[..., j * 64:j * 64 + 64] for j in range(3)])) for a in want]
+    values = [r(200, 512, seed=i) for i in range(6)]
+    x = torch.zeros(200, 512, dtype=BF, device=DEV)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for v in values:
+            y = slow
+            for _ in range(24):                                                          # (some milliseconds: the host is far ahead)
+                y = y @ slow
+            x.copy_(v + 0 * y.flatten()[:1].nan_to_num(0, 0, 0))
+            a = ops.rms_norm(x, w, 1e-5)
+            b = ops.mid_linear(a, m)
+            c = ops.flash_attn_func(*[a.view(1, 50, 4, 512)[..., j * 64:j * 64 + 64] for j in range(3)])
+            out.append((a.clone(), b.clone(), c.clone()))
+            del a, b, c                                                                  # (their memory is the next step's)
+            x.zero_()
+    side.synchronize()
+    for got, exp in zip(out, want):
+        assert all(torch.equal(g, e) for g, e in zip(got, exp))
 
 
 @pytest.mark.parametrize("name", NAMES)
