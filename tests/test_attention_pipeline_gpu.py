@@ -1,4 +1,4 @@
-"""Attention's software pipeline: the maximum that follows late, the ring's halves, runs of tiles that a window leaves out; one and two waves a query row."""
+"""Attention's software pipeline: maxima and accumulators that follow tile by tile, the ring's halves, runs of tiles that a window leaves out; one and two waves a query row."""
 import math
 
 import pytest

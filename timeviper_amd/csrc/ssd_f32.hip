@@ -8,7 +8,7 @@
 //   * the state S^T += (w B)^T x leaves, in a lane, four entries n of one column p: the operand of Y^T = S C^T as it is, and 16-byte rows in memory;
 //   * Y^T leaves four neighbouring columns of one token: 16-byte stores.
 // Two launches: the state that every segment but the last leaves from a zero start; then a segment folds its predecessors' (in order, as the recurrence) and
-// marches, writing y once.  Segments are as long as leaves two waves a SIMD; the fold reads 1 KB a predecessor and wave.
+// marches, writing y once.  How long a segment is: chunks_a_segment; the fold reads 1 KB a predecessor and wave.
 // Products for a wave and chunk: 40 for G (again by each of a head's P / 16 waves), 40 + 16 for Y, 16 for S, 32 cycles each.
 // Measured (32 heads x 64, 2 groups; ssd_chunked.hip's kernels -> here): 1 024 tokens 38 -> 21 us, 4 096: 128 -> 52, 2 x 4 096: 226 -> 91,
 // 2 x 128: 23 -> 13.  Error of the final state against 64 bits 1.3e-7 (5e-7 .. 3e-6 with weights of differences of sums), of y 1.6e-7 (1.9e-7).
