@@ -297,6 +297,14 @@ def _too_near(first: _Instruction, live: set, need: int, reads, writes) -> list:
     return found
 
 
+@pytest.fixture(scope="module")
+def device_code(tmp_path_factory):
+    """{source: its instructions}"""
+    build.ensure_built()
+    work = tmp_path_factory.mktemp("device")
+    return {src.name: _device_code(src.name, work / src.name) for src in build._sources()}
+
+
 _MEMORY = ("global_", "buffer_", "flat_", "scratch_")
 
 
@@ -316,16 +324,15 @@ def _scalar_writes(i: _Instruction) -> set:
 
 
 @needs_tools
-def test_loads_keep_five_wait_states_behind_a_vector_write_of_their_scalar_address(tmp_path):
+def test_loads_keep_five_wait_states_behind_a_vector_write_of_their_scalar_address(device_code):
     """A vector-memory instruction that reads a scalar register (address, M0 aside) which v_readfirstlane, v_readlane or a compare has written reads the old value
     within five wait states."""
-    build.ensure_built()
     bad = []
-    for src in build._sources():
-        for i in _device_code(src.name, tmp_path / src.name):
+    for src, code in device_code.items():
+        for i in code:
             if live := _scalar_results(i):
                 for passed, j in _too_near(i, live, 5, lambda k: _registers(" ".join(k.ops), "s") if k.op.startswith(_MEMORY) else set(), _scalar_writes):
-                    bad.append((src.name, passed, i.op, i.ops, j.op, j.ops))
+                    bad.append((src, passed, i.op, i.ops, j.op, j.ops))
     assert not bad, (len(bad), bad[:4])
 
 
@@ -334,16 +341,15 @@ def _vector_writes(i: _Instruction) -> set:
 
 
 @needs_tools
-def test_wide_stores_keep_their_data_for_two_wait_states(tmp_path):
+def test_wide_stores_keep_their_data_for_two_wait_states(device_code):
     """A store of more than 8 bytes still reads its data in the two wait states behind it: no vector instruction may write those registers there."""
-    build.ensure_built()
     bad = []
-    for src in build._sources():
-        for i in _device_code(src.name, tmp_path / src.name):
+    for src, code in device_code.items():
+        for i in code:
             if re.match(r"(global|flat|buffer)_store_dwordx[34]$", i.op):
                 data = i.ops[0 if i.op.startswith("buffer") else 1]
                 for passed, j in _too_near(i, _registers(data, "va"), 2, _vector_writes, lambda k: set()):
-                    bad.append((src.name, passed, i.op, i.ops, j.op, j.ops))
+                    bad.append((src, passed, i.op, i.ops, j.op, j.ops))
     assert not bad, (len(bad), bad[:4])
 
 
@@ -365,11 +371,10 @@ def test_the_count_of_wait_states_sees_what_is_too_near():
 
 
 @needs_tools
-def test_an_attention_step_copies_its_pieces_once(tmp_path):
+def test_an_attention_step_copies_its_pieces_once(device_code):
     """flash_fwd_kernel with two tiles a step: as many copies whatever the head dim, whose MFMAs they stand between"""
-    build.ensure_built()
     copies = {}
-    for i in _device_code("attention.hip", tmp_path / "attention"):
+    for i in device_code["attention.hip"]:
         if m := re.match(r"_ZN12_GLOBAL__N_116flash_fwd_kernelI(\w+)Li\dELi\dELi8ELi2ELb(\d)ELi(\d)E", i.of or ""):
             copies.setdefault(m.groups(), {}).setdefault(i.of, 0)
             copies[m.groups()][i.of] += "_lds_" in i.op
