@@ -17,7 +17,8 @@
  *   - `stream` is a hipStream_t passed as void*; kernels are enqueued, never
  *     synchronised; no allocation happens inside any entry point (workspaces
  *     are caller-provided, sizes from the *_workspace_bytes query);
- *   - return value: 0 = TV_OK, negative = tv_status error (nothing launched).
+ *   - return value: 0 = TV_OK, negative = tv_status error (nothing launched, but for TV_ERR_LAUNCH: the
+ *     error is looked for behind the launch and can be an earlier call's).
  */
 #ifndef TIMEVIPER_HIP_H
 #define TIMEVIPER_HIP_H
