@@ -79,3 +79,25 @@ def test_tokens_in_front_of_an_infinity(L, at, value):
     keep = torch.ones(B, H, P, dtype=torch.bool, device=DEV)
     keep[0, h, p] = False
     assert torch.equal(fin[keep], S[keep])
+
+
+# 7 | 8 chunks (one | two work-groups a tile), a second one with fewer segments than waves, more chunks a segment than stay in LDS, 16 blocks' remainders, a column tile of a round more
+@pytest.mark.parametrize("B,L,H,P", [(1, 448, 32, 64), (1, 449, 32, 64), (1, 520, 2, 16), (1, 1039, 32, 64), (1, 2100, 16, 64), (1, 4096, 4, 32), (2, 1010, 16, 64), (2, 1010, 33, 64),
+                                     (1, 70, 5, 48), (3, 330, 40, 32), (1, 6000, 8, 32)])
+@pytest.mark.parametrize("group_map", ["block", "tile"])
+def test_work_groups_of_a_tile(B, L, H, P, group_map):
+    from timeviper_amd import kernels as ops
+    G = 1 if H % 2 else 2
+    g = torch.Generator(device=DEV).manual_seed(L + H)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, Bm, Cm, dt, D, S0 = r(B, L, H, P), 0.3 * r(B, L, G, 16), r(B, L, G, 16), r(B, L, H), r(H), r(B, H, P, 16)
+    A = -torch.linspace(1e-3, 4, H, device=DEV)
+    y, fin, dec = ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_softplus=True, initial_states=S0, return_final_states=True, return_total_decay=True, group_map=group_map)
+    assert ops.ssd_scan_last_kernel() == 11
+    d = F.softplus(dt.double())
+    of = torch.arange(H, device=DEV) % G if group_map == "tile" else torch.arange(H, device=DEV) // (H // G)
+    want, S, mag, Sm = reference(x.double(), d, A.double(), Bm.double(), Cm.double(), D.double(), S0.double(), of)
+    # (as above; exponents are sums of 16 tokens)
+    rel = 2.0 ** -18 + 2.0 ** -21 * 16 * (d * A.double()).abs().mean(1).max().item()
+    assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
+    assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5, atol=1e-6)
