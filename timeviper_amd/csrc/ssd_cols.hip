@@ -6,7 +6,7 @@
 // 60 us.  Here a work-group takes 4 slices that follow each other in a B / C group (128 bytes of every x and y row), and the chain of
 // latencies that is then left of a step — dt -> softplus -> prefix sum -> weights -> x~ -> products -> y, 2.6 us as one wave's
 // program — is cut into three that run side by side, a wave each per slice (one of each on every SIMD):
-//   vectors  copies two steps ahead (LDS-DMA, ring of three), and prep(k + 2): the chunk's decays, frame, weights and mode
+//   vectors  copies a step ahead (LDS-DMA, two stages), and prep(k + 1): the chunk's decays, frame, weights and mode
 //   state    X' (= 0 or X') += B^T x~ of chunk k; leaves the bf16 copy of the state that ENTERS chunk k + 1 in LDS
 //   output   Yoff (from that copy) + Ydiag of chunk k, row factors, D x; y through LDS, so that whole 128-byte lines are stored
 //            (32 bytes a row straight from the registers are partial lines)
@@ -16,7 +16,9 @@
 // Up to 7 chunks come here, 9 at head dim 80, 24 where the heads are too many for more than three segments (use_cols in ssd_head.hip); beyond, the chain is cut (ssd_par.hip).
 // What is left is instruction issue — three waves a SIMD with about 350 vector and 38 matrix instructions a step, 1.6 us — and, in heads that
 // decay by more than 2^199 a chunk, the mask factors of a standard step (2.6 us).
-// Measured (128 heads x 80, 8 groups, whole operator, against a wave per head): 203 tokens 35 -> 17 us, 390: 46 -> 23.
+// Two stages, not three: the copies of the step ahead have the step's 2 us, and a call waits for one chunk before its first step instead of two (three | two, 128 heads x 80, fresh
+// Mamba-2 decays and decays of a hundredth: 150 tokens 14.8 | 14.4, 10.4 | 9.8 us; 250: 21.0 | 20.7, 12.2 | 11.4; 500: 29.5 | 28.8, 18.7 | 17.5; one chunk level).
+// Measured (128 heads x 80, 8 groups, whole operator, against a wave per head): 203 tokens 35 -> 17 us, 390: 46 -> 19.
 #include "ssd_common.hpp"
 
 namespace {
@@ -45,18 +47,17 @@ struct __attribute__((aligned(16))) ColVec {   // a chunk's vectors of a slice's
 };
 struct __attribute__((aligned(16))) ColStage {
   bf16_t bt[HQ * HN], ct[HQ * HN];
-  unsigned dt[4][64];                          // of the chunk two further on
+  unsigned dt[4][64];                          // of the chunk behind
 };
 struct __attribute__((aligned(16))) ColSmem {
-  ColStage st[3];
-  bf16_t xr[3][4][HQ * CP];
+  ColStage st[2];
+  bf16_t xr[2][4][HQ * CP];
   bf16_t yt[4][HQ * CP];
   bf16_t snap[4][4 * 64 * 8];                  // [slice][quarter of the state rows][lane] 16 bytes: Yoff's operand
-  ColVec v[3][4];
-  int mode[3][4];                              // shift of the frame | reset << 16 | standard << 17
+  ColVec v[2][4];
+  int mode[2][4];                              // shift of the frame | reset << 16 | standard << 17
   float e_end[4];
 };
-constexpr int OPS = 4 + 4 + 2 + 1;             // copy instructions a stage and wave: B, C, x, dt
 
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4v;
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
     const unsigned ox0 = (unsigned)(((lane >> 1) * a.xsl + (lane & 1) * 8) * 2), ox1 = ox0 + (unsigned)(64 * a.xsl) - 1024u;
     const unsigned dB = lds0 + (unsigned)offsetof(ColStage, bt) + 4096u * w, dC = lds0 + (unsigned)offsetof(ColStage, ct) + 4096u * w;
     const unsigned dD = lds0 + (unsigned)offsetof(ColStage, dt) + 256u * w;
-    // stage of chunk c, and dt of chunk c + 2
+    // stage of chunk c, and dt of chunk c + 1
     auto issue = [&](int c, int S) __attribute__((always_inline)) {
       const unsigned so = (unsigned)S * (unsigned)sizeof(ColStage), dX = x_tile(S);
       const int t0 = c * HQ, last = L - 1 - t0;
@@ -149,8 +150,8 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
         for (int k = 0; k < 2; ++k)
           glds16(xp, (unsigned)((min(32 * k + (lane >> 1), last) * a.xsl + (lane & 1) * 8) * 2), dX + 1024u * k);
       }
-      const int t2 = min(t0 + 2 * HQ, L - 1);
-      glds4(uniform_ptr(dtg + (int64_t)t2 * a.dsl), (unsigned)(min(lane, L - 1 - t2) * a.dsl * 2), dD + so);
+      const int t1 = min(t0 + HQ, L - 1);
+      glds4(uniform_ptr(dtg + (int64_t)t1 * a.dsl), (unsigned)(min(lane, L - 1 - t1) * a.dsl * 2), dD + so);
     };
     const float Ah = a.A[h], bias = a.dt_bias ? a.dt_bias[h] : 0.f;
     float decay_total = 0.f, E = 0.f;
@@ -181,34 +182,28 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
       E = std_ ? 0.f : rst ? RMAX : Euse + cl2;
       if (lane == 0) sm.mode[S][w] = ((int)-mshift & 0xffff) | (rst || std_ ? 1 << 16 : 0) | (std_ ? 1 << 17 : 0);
     };
-    {
-      const int64_t half = odd ? 1 : 0;
-      float r0 = (float)dtg[(int64_t)min(lane, L - 1) * a.dsl + half], r1 = (float)dtg[(int64_t)min(HQ + lane, L - 1) * a.dsl + half];
-      asm volatile("" : "+v"(r0), "+v"(r1));                   // (from here on only copies are counted)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      issue(0, 0);
-      if (nchunks > 1) issue(1, 1);
-      prep(0, 0, r0);
-      meet();                                                  // (the state wave reads chunk 0's mode)
-      if (nchunks > 1) prep(1, 1, r1);
-    }
-    if (nchunks > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto dt_of = [&](int S) __attribute__((always_inline)) {
+      const unsigned raw = sm.st[S].dt[w][lane];
+      return odd ? bf16_hi(raw) : bf16_lo(raw);
+    };
+    float r0 = (float)dtg[(int64_t)min(lane, L - 1) * a.dsl + (odd ? 1 : 0)];
+    asm volatile("" : "+v"(r0));                               // (from here on only copies are counted; as a copy among the others it comes later: 100 tokens 10.1, so 10.5)
+    issue(0, 0);
+    prep(0, 0, r0);
+    meet();                                                    // (the state wave reads chunk 0's mode)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int S = 0;
     for (int k = 0; k < nchunks; ++k) {
       meet();
-      const int S2 = S == 0 ? 2 : S - 1;                       // the stage that step k - 1 has left
-      if (k + 2 < nchunks) {
-        issue(k + 2, S2);
-        const unsigned raw2 = sm.st[S].dt[w][lane];
-        prep(k + 2, S2, odd ? bf16_hi(raw2) : bf16_lo(raw2));
+      if (k + 1 < nchunks) {
+        issue(k + 1, S ^ 1);                                   // (the stage that step k - 1 has left)
+        prep(k + 1, S ^ 1, dt_of(S));
+      } else if (lane == 0) {
+        sm.e_end[w] = E;
       }
-      if (k + 1 == nchunks && lane == 0) sm.e_end[w] = E;
       meet();
-      // stage k + 1 has landed in front of the next meeting; younger: the copies of stage k + 2
-      if (k + 2 < nchunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPS) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      S = S == 2 ? 0 : S + 1;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // (in front of the next meeting)
+      S ^= 1;
     }
     if (a.total_decay && lane == 0 && sl == hr * a.sub) a.total_decay[(int64_t)b * a.H + h] = decay_total;
     meet();
@@ -257,10 +252,8 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
     int S = 0;
     for (int k = 0; k < nchunks; ++k) {
       meet();
-      const int S1 = S == 2 ? 0 : S + 1;
       const unsigned Bt = lds0 + (unsigned)S * (unsigned)sizeof(ColStage) + (unsigned)offsetof(ColStage, bt), xt = x_tile(S);
       const int md = __builtin_amdgcn_readfirstlane(sm.mode[S][w]);
-      const int mn = __builtin_amdgcn_readfirstlane(k + 1 < nchunks ? sm.mode[S1][w] : 0);
       if (k > 0) store_y(k - 1);                               // (here, where nothing waits for memory)
       bf16x8 x0 = x_frag(xt, 0), x1 = x_frag(xt, 1);
       if (md & (1 << 17)) {
@@ -288,10 +281,12 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
         X[i] = mfma16(cat4(tr(bp), tr(bp + 1024)), x0, X[i]);
         X[i] = mfma16(cat4(tr(bp + 8192), tr(bp + 9216)), x1, X[i]);
       }
-      to_frame(mn);                                            // the next chunk's frame
       meet();
-      if (k + 1 < nchunks) leave();
-      S = S1;
+      if (k + 1 < nchunks) {
+        to_frame(__builtin_amdgcn_readfirstlane(sm.mode[S ^ 1][w]));      // the next chunk's frame
+        leave();
+      }
+      S ^= 1;
     }
     meet();
     store_y(nchunks - 1);
@@ -388,7 +383,7 @@ __global__ __launch_bounds__(768) void ssd_cols_kernel(ColsArgs a) {
       meet();
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti) *(u32x2*)(&sm.yt[w][(16 * ti + lc) * CP + 4 * kq]) = yv[ti];
-      S = S == 2 ? 0 : S + 1;
+      S ^= 1;
     };
     for (int k = 0; k < nchunks; k += 2) {
       step(k, cb0);
