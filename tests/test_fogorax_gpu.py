@@ -42,6 +42,40 @@ def cache_of(layers, slots, capacity, dtype, starts):
     return c
 
 
+# ------------------------------------------------------------------ the numbers of a step
+@pytest.mark.parametrize("counts", [[1], [5], [1, 1, 1], [255, 1, 257, 1024, 1025], [70001, 2], [1] * 130, [3] * 128, [2] * 300, [4, 1] * 129])
+def test_plan_is_the_one_built_on_the_host(counts):
+    from timeviper_amd.model.llm import SlotStateCache
+    n = len(counts)
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(n)).tolist()
+    starts = torch.randint(0, 900, (n,), generator=torch.Generator().manual_seed(n + 1)).tolist()
+    got, want = (SlotStateCache([("tokens", 1)], n, torch.float32, dev, max(counts) + 900) for dev in (DEV, "cpu"))
+    for c in (got, want):
+        for _ in range(n):
+            c.alloc()
+        c._len.update(zip(order, starts))
+    for step in range(2):
+        p, q = (c.plan(order, counts) for c in (got, want))
+        assert (p.slots, p.counts, p.starts, p.decode) == (q.slots, q.counts, q.starts, q.decode)
+        for name in ("cu", "start", "slot", "rows", "seq", "keys", "moving"):
+            a, b = getattr(p, name), getattr(q, name)
+            assert (a is None) == (b is None) and (a is None or (a.dtype == b.dtype and a.is_contiguous() and torch.equal(a.cpu(), b))), name
+        if step == 0 and max(counts) == 1:
+            for c in (got, want):
+                c.commit(p if c is got else q)                # the device's numbers move with the host's
+        else:
+            break
+
+
+def test_plan_stays_out_of_a_captured_graph():
+    c = cache_of([("tokens", 4)], 1, 40, BF, {0: 3})
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        with pytest.raises(RuntimeError):
+            c.plan([0], [2])
+    assert c.plan([0], [2]).rows.tolist() == [3, 4]
+
+
 # ------------------------------------------------------------------ embedding, norm, shift, gated products
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_embedding_with_positions(dtype):

@@ -1056,6 +1056,32 @@ def kv_append(k, v, k_cache, v_cache, pos) -> None:
                                    st(k_cache, 1), st(v_cache, 0), st(v_cache, 1), _stream()), "tv_kv_append")
 
 
+def step_plan(starts, slots, counts, capacity: int, device):
+    """int32 device tensors of a packed step (cache.StepPlan): cu, start, slot, rows, seq, keys and, one token per sequence, the (3, B) tensor
+    behind start, rows and keys (else None for these two).  One launch; nothing waits for the device."""
+    B, T = len(starts), sum(counts)
+    if torch.cuda.is_current_stream_capturing():
+        raise TimeViperHipError("step_plan: the numbers of a step do not belong into a captured graph (plan the step first)")
+    single = B == T
+    up = lambda n: (n + 3) & ~3                                   # 16-byte aligned parts
+    sizes = [3 * B if single else T, B + 1, B, T] + ([] if single else [B])
+    buf = torch.empty((sum(up(n) for n in sizes),), dtype=torch.int32, device=device)
+    _gpu(buf)
+    parts, at = [], 0
+    for n in sizes:
+        parts.append(buf[at:at + n])
+        at += up(n)
+    if single:
+        moving, (_, cu, slot, seq) = parts[0].view(3, B), parts
+        start, rows, keys = moving
+    else:
+        moving, keys, (rows, cu, slot, seq, start) = None, None, parts
+    ints = ctypes.c_int * B
+    check(_capi.lib().tv_step_plan(ints(*starts), ints(*slots), ints(*counts), B, capacity, _p(cu), _p(start), _p(slot), _p(rows), _p(seq), _p(keys),
+                                   _stream()), "tv_step_plan")
+    return cu, start, slot, rows, seq, keys, moving
+
+
 def count_up(pos, lens) -> None:
     """pos += 1 (int64, one entry), lens += 1 (int32), in one launch on the GPU"""
     if not (pos.is_cuda and lens.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1 and lens.dtype == torch.int32 and lens.is_contiguous()):

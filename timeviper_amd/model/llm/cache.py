@@ -15,6 +15,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from ... import kernels as K
+
 
 class StaticDecode:
     """Fixed launch parameters for a run of single-token steps."""
@@ -181,6 +183,17 @@ class SlotStateCache(StaticDecode):
         if need > self.capacity:
             room = need + max(self.reserve, need // 8)
             self._resize(self.num_slots, room if self.limit is None else min(room, self.limit))
+        p = StepPlan(slots, counts, starts, *self._plan_tensors(slots, starts, counts, single), single)
+        if single:
+            self._decode_plan = p
+        return p
+
+    def _plan_tensors(self, slots, starts, counts, single):
+        """cu, start, slot, rows, seq, keys, moving of a StepPlan"""
+        d = None if self.device is None else torch.device(self.device)
+        if (d is not None and d.type == "cuda" and d.index in (None, torch.cuda.current_device()) and sum(counts) < 1 << 30
+                and self.num_slots * self.capacity < 1 << 31):
+            return K.step_plan(starts, slots, counts, self.capacity, d)
         i32 = lambda v: torch.tensor(v, dtype=torch.int32).to(self.device)
         cu, rows, seq = [0], [], []
         for b, (s, a, c) in enumerate(zip(slots, starts, counts)):
@@ -190,12 +203,8 @@ class SlotStateCache(StaticDecode):
         seq = torch.cat(seq).to(self.device)
         if single:
             mv = i32([list(starts), [s * self.capacity + a for s, a in zip(slots, starts)], [a + 1 for a in starts]])
-            p = StepPlan(slots, counts, starts, i32(cu), mv[0], i32(slots), mv[1], seq, mv[2], mv, True)
-        else:
-            p = StepPlan(slots, counts, starts, i32(cu), i32(starts), i32(slots), torch.cat(rows).to(self.device), seq, None, None, False)
-        if single:
-            self._decode_plan = p
-        return p
+            return i32(cu), mv[0], i32(slots), mv[1], seq, mv[2], mv
+        return i32(cu), i32(starts), i32(slots), torch.cat(rows).to(self.device), seq, None, None
 
     def commit(self, p: StepPlan):
         """The step of `p` has been launched: its tokens belong to the sequences."""
