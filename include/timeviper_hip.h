@@ -607,7 +607,9 @@ int tv_gemv_glu_fwd(const void* z, const void* u, const int64_t* u_ids, int64_t 
  * tv_gemm_rows_fwd: y bf16, or fp32 without epilogue or with TV_GEMM_ROWS_ROUND (the bf16 values, stored as fp32); epilogue TV_GEMM_ROWS_RELU2: y = relu(bf16(.))^2; conv_state not NULL: the
  *   outputs [conv_row0, conv_row0 + conv_channels) pass through tv_causal_conv1d_update (width 4, SiLU) on conv_state
  *   (M, conv_channels, 4), as in tv_gemv_bf16_fwd.
- * tv_gemm_rows_add_fwd, tv_gemm_rows_pair_fwd: tv_gemv_add_fwd and tv_gemv_pair_fwd for these rows.                        */
+ * tv_gemm_rows_add_fwd, tv_gemm_rows_pair_fwd: tv_gemv_add_fwd and tv_gemv_pair_fwd for these rows.
+ * tv_gemm_rows_glu_fwd: y = gelu_tanh(bf16(x W^T)) * u, row m of x with row u_ids[m] of u (NULL: m; an id outside its u_rows rows counts as a row of zeros);
+ * at most 8 outputs a compute unit. */
 #define TV_GEMM_ROWS_MAX 32
 #define TV_GEMM_ROWS_RELU2 1
 #define TV_GEMM_ROWS_ROUND 2
@@ -616,6 +618,8 @@ int tv_gemm_rows_fwd(const void* x, const void* W, const void* bias, void* y, in
                      const void* conv_bias, int conv_row0, int conv_channels, void* stream);
 int tv_gemm_rows_add_fwd(const void* x, const void* W, const void* bias, const float* residual, float* residual_out, void* h_out,
                          int M, int N, int K, int64_t x_stride, int64_t ldw, void* stream);
+int tv_gemm_rows_glu_fwd(const void* x, const void* W, const void* u, const int64_t* u_ids, int64_t u_rows, void* y, int M, int N, int K,
+                         int64_t x_stride, int64_t ldw, int64_t u_stride, int64_t y_stride, void* stream);
 int tv_gemm_rows_pair_fwd(const void* x, const void* x2, const void* W, const void* bias, void* y, void* act, int M, int n1,
                           int ff, int K, int64_t x_stride, int64_t x2_stride, int64_t ldw, int64_t y_stride,
                           int64_t act_stride, void* stream);

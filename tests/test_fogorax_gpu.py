@@ -70,7 +70,9 @@ def test_plan_is_the_one_built_on_the_host(counts):
 def test_plan_stays_out_of_a_captured_graph():
     c = cache_of([("tokens", 4)], 1, 40, BF, {0: 3})
     g = torch.cuda.CUDAGraph()
+    one = torch.zeros(1, device=DEV)
     with torch.cuda.graph(g):
+        one += 1
         with pytest.raises(RuntimeError):
             c.plan([0], [2])
     assert c.plan([0], [2]).rows.tolist() == [3, 4]
@@ -362,6 +364,26 @@ def test_product_of_token_rows(M, n, N):
                           (table[:, n:2 * n], ids, K.gemv_glu(z.to(DEV), table.to(DEV)[:, n:2 * n], weight.to(DEV), ids=ids.to(DEV)))):
         f = (O.gelu_tanh(z.double()) * (rows if by is None else rows[by]).double()).to(BF).double()
         close(got, f @ weight.double().T, 1e-2)
+
+
+@pytest.mark.parametrize("M,D,N", [(2, 64, 1), (3, 2048, 128), (4, 128, 130), (8, 2048, 128), (9, 192, 257), (16, 2048, 128), (17, 512, 2048), (32, 2048, 128)])
+def test_gate_with_its_token_row(M, D, N):
+    from timeviper_amd import kernels as K
+    x, weight, u, table = rnd((M, 2 * D), 101, BF)[:, D:], rnd((N, D), 102, BF, 2 * D ** -0.5), rnd((M, N), 103, BF), rnd((11, 3 * N), 104, BF)
+    ids = torch.randint(0, 11, (M,), generator=torch.Generator().manual_seed(M))
+    z = x.double() @ weight.double().T
+    mass = x.double().abs() @ weight.double().abs().T
+    bad = ids.clone()
+    bad[0], bad[M - 1] = -1, 11
+    for by, rows in ((None, u.double()), (ids, table[:, N:2 * N].double()[ids]), (bad, table[:, N:2 * N].double()[bad.clamp(0, 10)] * ((bad >= 0) & (bad < 11))[:, None])):
+        tab = u if by is None else table
+        tab = tab.to(DEV) if by is None else tab.to(DEV)[:, N:2 * N]
+        got = K.rows_glu(x.to(DEV), weight.to(DEV), tab, None if by is None else by.to(DEV)).double().cpu()
+        want = O.gelu_tanh(z) * rows
+        # the sum in fp32 (D roundings of at most the products' mass) and its rounding to bf16 (8 significant bits: 2^-8 of the value), through an activation
+        # whose slope is at most 1.13; the result's rounding
+        bound = rows.abs() * (1.13 * (2.0 ** -8 * z.abs() + D * 2.0 ** -24 * mass) + 2.0 ** -20 * (1 + z.abs())) * (1 + 2.0 ** -8) + 2.0 ** -8 * want.abs() + 1e-30
+        assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() - bound).max())
 
 
 # ------------------------------------------------------------------ the model

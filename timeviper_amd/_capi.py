@@ -93,6 +93,7 @@ SIGNATURES = {
     "tv_gemv_glu_fwd": (_i, [_p] * 3 + [_l] + [_p] * 2 + [_i] * 3 + [_l] * 4 + [_p]),
     "tv_gemm_rows_fwd": (_i, [_p] * 4 + [_i] * 4 + [_l] * 3 + [_i] + [_p] * 3 + [_i, _i, _p]),
     "tv_gemm_rows_add_fwd": (_i, [_p] * 6 + [_i] * 3 + [_l] * 2 + [_p]),
+    "tv_gemm_rows_glu_fwd": (_i, [_p] * 4 + [_l, _p] + [_i] * 3 + [_l] * 4 + [_p]),
     "tv_gemm_rows_pair_fwd": (_i, [_p] * 6 + [_i] * 4 + [_l] * 5 + [_p]),
     "tv_gemm_mid_workspace_bytes": (_z, [_i] * 3),
     "tv_gemm_mid_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l] * 3 + [_i, _p, _z, _p]),

@@ -2050,6 +2050,25 @@ def gemv_glu(z, u, weight, ids=None):
     return y
 
 
+def rows_glu_takes(x, weight, u) -> bool:
+    """Operands tv_gemm_rows_glu_fwd reads: 2..32 rows as `rows_take`, at most 8 outputs a compute unit, rows of u of one width"""
+    return (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) < (1 << 24) and x.data_ptr() % 16 == 0 and rows_take(x, weight)
+            and weight.shape[0] <= 8 * CUS and u.dtype == x.dtype and u.dim() == 2 and u.stride(1) == 1 and u.shape[1] == weight.shape[0])
+
+
+def rows_glu(x, weight, u, ids=None):
+    """gelu_tanh(x @ weight.T) * u for 2..32 bf16 rows, the product rounded in front of the activation; `ids` (int64): row m meets u[ids[m]]"""
+    _gpu(x, weight, u, ids)
+    M, (N, Kd) = x.shape[0], weight.shape
+    if (not rows_glu_takes(x, weight, u) or x.shape[1] != Kd or (ids is None and u.shape[0] != M)
+            or (ids is not None and (ids.dtype != torch.int64 or ids.numel() != M or not ids.is_contiguous()))):
+        raise TimeViperHipError(f"rows_glu: rows {tuple(x.shape)} against {tuple(weight.shape)}, u {tuple(u.shape)}, one per row or by int64 ids")
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    check(_capi.lib().tv_gemm_rows_glu_fwd(_p(x), _p(weight), _p(u), _p(ids), u.shape[0], _p(y), M, N, Kd, x.stride(0), weight.stride(0), u.stride(0), N,
+                                           _stream()), "tv_gemm_rows_glu_fwd")
+    return y
+
+
 # ------------------------------------------------- mixture of experts
 MOE_NONE, MOE_RELU2 = 0, 1
 

@@ -62,6 +62,8 @@ class TokenSide(nn.Module):
         return F.linear(K.gated_mul(F.linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
 
     def decode(self, h, ids, rows):
+        if K.rows_glu_takes(h, self.gate, rows) and self.dim % 64 == 0 and K.rows_weight(self.proj):
+            return K.rows_linear(K.rows_glu(h, self.gate, rows, ids), self.proj)
         if h.shape[0] > 4:
             return K.rows_linear(K.gated_mul(K.rows_linear(h, self.gate), rows, K.ACT_GELU_TANH, ids=ids), self.proj)
         return K.gemv_glu(K.gemv_post(h, self.gate), rows, self.proj, ids=ids)
