@@ -67,6 +67,24 @@ def test_plan_is_the_one_built_on_the_host(counts):
             break
 
 
+def test_plan_is_complete_for_every_stream():
+    """whatever the current stream still has to do: the tensors hold the step's numbers when the call returns"""
+    c = cache_of([("tokens", 4)], 3, 4000, BF, {2: 7, 0: 0, 1: 1000})
+    work, other = torch.randn(4096, 4096, device=DEV), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for i in range(20):
+        for _ in range(10):
+            work = work @ work * 1e-2                         # (some 10 ms in front of every plan)
+        p = c.plan([2, 0, 1], [i + 1, 300, 2 + i])
+        with torch.cuda.stream(other):
+            got = [t.cpu() for t in (p.rows, p.seq, p.cu, p.slot, p.start)]
+        n = [i + 1, 300, 2 + i]
+        rows = [torch.arange(s * 4000 + a, s * 4000 + a + m) for s, a, m in zip((2, 0, 1), (7, 0, 1000), n)]
+        want = [torch.cat(rows), torch.arange(3).repeat_interleave(torch.tensor(n)), torch.tensor([0] + n).cumsum(0), torch.tensor([2, 0, 1]),
+                torch.tensor([7, 0, 1000])]
+        assert all(g.tolist() == w.tolist() for g, w in zip(got, want))
+
+
 def test_plan_stays_out_of_a_captured_graph():
     c = cache_of([("tokens", 4)], 1, 40, BF, {0: 3})
     g = torch.cuda.CUDAGraph()

@@ -75,7 +75,8 @@ __global__ __launch_bounds__(ARG_BLOCKS) void argmax_rows_kernel(const Best* __r
 
 // Where the rows of a packed step live, from host numbers that ride in the launch: sequence blockIdx.y of up to PLAN_SEQ, its share blockIdx.x
 // of the rows.  Copied from pageable memory instead, each of the five arrays waited for the device to run dry: 6 prompts, 6 011 tokens in all,
-// 5 257 -> 5 101 us a step; one of 3 026: 3 288 -> 3 152; one of 60: 1 018 -> 892.
+// 5 412 -> 5 267 us a step; 4 of 1 500: 2 122 -> 2 023; one of 60: 1 018 -> 899.  (Launched on the step's own stream, with nothing waiting for it, 892 for 60 and
+// 1 948: but what copies had left was there for any stream.)
 constexpr int PLAN_SEQ = 128;
 struct PlanSeqs {
   int start[PLAN_SEQ], slot[PLAN_SEQ], cu[PLAN_SEQ + 1];

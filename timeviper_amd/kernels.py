@@ -1056,17 +1056,27 @@ def kv_append(k, v, k_cache, v_cache, pos) -> None:
                                    st(k_cache, 1), st(v_cache, 0), st(v_cache, 1), _stream()), "tv_kv_append")
 
 
+_plan_streams = {}            # device -> the stream that `step_plan` launches on (of torch's pool)
+
+
 def step_plan(starts, slots, counts, capacity: int, device):
     """int32 device tensors of a packed step (cache.StepPlan): cu, start, slot, rows, seq, keys and, one token per sequence, the (3, B) tensor
-    behind start, rows and keys (else None for these two).  One launch; nothing waits for the device."""
+    behind start, rows and keys (else None for these two).  One launch, on a stream of its own: the tensors are complete when the call returns, for
+    every stream, and nothing waits for what the current one still has to do."""
     B, T = len(starts), sum(counts)
     if torch.cuda.is_current_stream_capturing():
         raise TimeViperHipError("step_plan: the numbers of a step do not belong into a captured graph (plan the step first)")
     single = B == T
     up = lambda n: (n + 3) & ~3                                   # 16-byte aligned parts
     sizes = [3 * B if single else T, B + 1, B, T] + ([] if single else [B])
-    buf = torch.empty((sum(up(n) for n in sizes),), dtype=torch.int32, device=device)
+    now = torch.cuda.current_stream(device)
+    side = _plan_streams.get(now.device)
+    if side is None:
+        side = _plan_streams.setdefault(now.device, torch.cuda.Stream(now.device))
+    with torch.cuda.stream(side):
+        buf = torch.empty((sum(up(n) for n in sizes),), dtype=torch.int32, device=device)
     _gpu(buf)
+    buf.record_stream(now)                                        # (memory of the side stream: not given out again before `now` has left it)
     parts, at = [], 0
     for n in sizes:
         parts.append(buf[at:at + n])
@@ -1078,7 +1088,8 @@ def step_plan(starts, slots, counts, capacity: int, device):
         moving, keys, (rows, cu, slot, seq, start) = None, None, parts
     ints = ctypes.c_int * B
     check(_capi.lib().tv_step_plan(ints(*starts), ints(*slots), ints(*counts), B, capacity, _p(cu), _p(start), _p(slot), _p(rows), _p(seq), _p(keys),
-                                   _stream()), "tv_step_plan")
+                                   side.cuda_stream), "tv_step_plan")
+    side.synchronize()
     return cu, start, slot, rows, seq, keys, moving
 
 
