@@ -263,6 +263,20 @@ def test_window_attention_of_single_tokens(H, G, d, e, window, keep, dtype):
         assert torch.equal(c.tokens(0).cpu(), want_kv)
 
 
+@pytest.mark.parametrize("H,G,d,e,n", [(2, 1, 64, 256, 2600), (4, 2, 32, 8, 6000), (2, 2, 128, 128, 4200), (2, 1, 64, 136, 520)])
+def test_single_tokens_of_many_splits(H, G, d, e, n):
+    """more splits than the merge's groups of threads take in one round, and groups without a split that has keys"""
+    from timeviper_amd import kernels as K
+    starts = {0: n - 1, 1: 70}
+    q, g, kv = attention_case(H, G, d, e, starts, [1, 1], n, BF)
+    c = cache_of([("tokens", G * (d + e))], kv.shape[0], n, BF, starts)
+    c.tokens(0).copy_(kv)
+    scale = 0.8 * d ** -0.5
+    want = attention_want(q, g, kv, H, G, d, e, starts, [1, 1], scale, n, 0)
+    o = K.attention_window_decode(q.to(DEV).view(2, H, d), c.tokens(0), c.plan([0, 1], [1, 1]), G, scale, n, 0, gate=g.to(DEV).view(2, H, e))
+    close(o.reshape(2, H * e), want, OP[BF])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("d,e", [(64, 64), (128, 96), (18, 22)])
 @pytest.mark.parametrize("key", [0, 6, 7, 95, 96, 191, 383, 384, 500])
