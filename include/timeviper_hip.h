@@ -644,7 +644,7 @@ int tv_gemm_glu_fwd(const void* A, const void* W, const void* bias, void* C, int
 
 /* C = epilogue(A W^T) for a few hundred to a few thousand rows (csrc/gemm_small.hip), epilogue 0 (bias), 1 (bias, exact GELU of the rounded sum), 2 (C += the sum) as
  * tv_gemm_bf16_fwd, or 5: tv_gemm_glu_fwd's (bf16 bias of 2 N, N outputs).  tile: 0, 1: 128 x 128 outputs a work-group (ring of four stages, of two), 2: 64 x 128, 3:
- * 64 x 64 (half as many outputs with epilogue 5).  K % 64 == 0, N % 8 == 0, everything 16-byte aligned. */
+ * 64 x 64 (half as many outputs with epilogue 5); 2 and 3 give way to the next larger tile where they are more than a round of the compute units and it is not.  K % 64 == 0, N % 8 == 0, everything 16-byte aligned. */
 int tv_gemm_small_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                       int epilogue, int bias_dtype, int tile, void* stream);
 

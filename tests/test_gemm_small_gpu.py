@@ -37,6 +37,41 @@ def test_against_64_bits(M, N, K, tile):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5 * (f.abs() + 1) * (u.abs() + 1)).all()
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13])
+def test_every_end_of_the_ring(stages, tile):
+    """whole numbers: exact, whatever the order of the sums; a number of stages that a slot, a wait or the parity of the fragments could miss"""
+    from timeviper_amd import kernels as ops
+    K = 64 * stages
+    g = torch.Generator(device=DEV).manual_seed(K)
+    r = lambda *s: torch.randint(-3, 4, s, generator=g, device=DEV).to(BF)
+    x, w, c = r(193, K), r(200, K), r(193, 200)
+    want = x.double() @ w.double().T + c.double()
+    out = c.clone()
+    ops.small_linear(x, w, None, ops.GEMM_ACCUM, out=out, tile=tile)
+    assert torch.equal(out, want.to(BF))
+
+
+@pytest.mark.parametrize("M,N,tile", [(1024, 1152, 3), (960, 1088, 3), (729, 3456, 2), (1025, 2048, 2), (2048, 4096, 3)])
+def test_more_work_groups_than_a_round(M, N, tile):
+    """a tile that gives way to the next larger one, and those that just do not"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    r = lambda *s: torch.randint(-3, 4, s, generator=g, device=DEV).to(BF)
+    x, w = r(M, 192), r(N, 192)
+    assert torch.equal(ops.small_linear(x, w, None, tile=tile), (x.double() @ w.double().T).to(BF))
+
+
+@pytest.mark.parametrize("rows,n,k,takes", [(2177, 1152, 1152, True), (2176, 1152, 1152, False), (1921, 1152, 4352, True), (1920, 1152, 4352, False), (3584, 1152, 4352, True),
+                                            (3585, 1152, 4352, False), (2916, 1152, 6208, False), (2916, 1152, 960, False), (2916, 1148, 1152, False), (513, 4096, 2048, True), (512, 4096, 2048, False)])
+def test_rule_of_a_full_round(rows, n, k, takes):
+    from timeviper_amd import kernels as ops
+    x, w = torch.empty(rows, k, device=DEV, dtype=BF), torch.empty(n, k, device=DEV, dtype=BF)
+    assert not ops.round_takes(x, w)                                          # gradients enabled
+    with torch.no_grad():
+        assert ops.round_takes(x, w) == takes and not ops.round_takes(x[:, 4:], w[:, 4:]) and not ops.round_takes(x.float(), w.float())
+
+
 def test_refused():
     from timeviper_amd import kernels as ops
     z = lambda *s: torch.zeros(s, device=DEV, dtype=BF)

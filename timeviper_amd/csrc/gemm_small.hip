@@ -1,15 +1,23 @@
-// bf16 products of a few hundred to a few thousand rows, C = epilogue(A W^T), on small tiles: 128 x 128, 64 x 128 or 64 x 64 outputs a work-group of four waves.
+// bf16 products of a few hundred to a few thousand rows, C = epilogue(A W^T), on small tiles: 128 x 128, 64 x 128 or 64 x 64 outputs a work-group of eight waves.
 //
 // gemm.hip's 256 x 256 tiles are a quarter of a round there, and each takes its whole contraction (729 rows: 42 - 51 tiles, 26 us however short it is).  Small tiles
-// fill the compute units; what bounds them is the way into the compute unit (a stage of 64 columns is 16 - 32 KB, at about 70 bytes a ns), so the tile is the
-// largest that still gives the chip a round (kernels.small_tile).
-//   * a wave holds a quarter of the tile; both operands arrive by LDS-DMA (8 rows x 128 bytes an instruction, 16-byte pieces exchanged on the source side so that
-//     fragment reads meet no bank twice) in a ring of NS stages, NS - 1 ahead of the products behind counted waits, one barrier a stage;
+// fill the compute units; the tile is the largest that still gives the chip a round (kernels.small_tile).
+//   * Two waves share a quarter of the tile, each with one 32-column half of every stage of 64: a SIMD has two waves, one's products run beside the other's reads and
+//     copies, and together they read no more of LDS than one wave would.  The pair meets over the ring behind the loop.  (With four waves, one a SIMD, a stage of a 128 x 128
+//     tile was 525 ns even where every copy hit the same lines; 465 with reads and copies dealt out between the products; now 325.  Its 64 KB of fragment reads and 32 of
+//     copies take 320 at 128 bytes a clock: LDS bounds it.)
+//   * Both operands arrive by LDS-DMA (8 rows x 128 bytes an instruction, 16-byte pieces exchanged on the source side so that fragment reads meet no bank twice) in a ring of
+//     NS stages behind counted waits, one barrier a stage.  Four stages: the fragments of stage t + 1 are read during the products of stage t, whose slot, held in registers by
+//     then, is filled again (asked for one stage later instead, 1 152 x 4 352 on 64 x 64 tiles takes 19.2 us in place of 16.7).
+//   * A stage is a 128-byte piece of each row of W, which memory delivers late where it is not in a cache: beside the first stages the work-groups together ask for all of W
+//     once, a line a lane.  Weights out of cache, 2 916 x 1 152 x 4 352: 41.6 -> 34.1, 1 458: 32.8 -> 26.2, 729 20.3 -> 17.9; 729 x 3 456 x 1 152 14.7 -> 14.0; in a cache .5 - 1 us more.
+//   * Two stages (64 KB): two work-groups a compute unit, for tiles between one round and two (5 120 x 2 048, 1 024 rows: 30.3 us, four stages in two rounds 31.6).
 //   * v_mfma_f32_16x16x32_bf16 with W on the A side: two tiles of rows joined by v_permlane16_swap are 16-byte stores, as gemm.hip;
 //   * EPI_GLU: half of a tile's rows of W are those of the gate, half those of the factor N rows further down: a lane holds both of an output.
 // fp32 sums, one rounding; the GELU is that of the rounded sum (what the library's product would have written).
-// Measured (us, library -> here, on the device): 729 x 3 456 x 1 152 15.0 -> 13.8, 729 x 1 152 x 1 152 9.5 -> 7.5, 729 x 1 152 x 4 352 18.7 -> 19.4, 200 x (2 x 5 632) x 2 048 with the
-// gate 26 + 5 -> 23; with the library's 19 us of host time gone: SigLIP so400m, 1 frame 4.1 -> 2.8 ms, 2 frames 4.1 -> 3.3.
+// Measured (us on the device, weights out of cache, library | four waves before -> here): 729 x 3 456 x 1 152 17.9 | 15.0 -> 14.0, 729 x 1 152 x 1 152 12.5 | 9.1 -> 8.0, 729 x 1 152 x 4 352
+// 22.3 | 26.2 -> 17.9, 1 458 30.7 | 31.2 -> 26.2, 2 916 42.0 | 44.7 -> 34.1, 729 x 5 120 x 2 048 25.9 | 24.8 -> 23.3, 1 458 x 3 456 x 1 152 19.3 | 23.6 -> 23.8.  SigLIP so400m, whole forwards: 1 frame
+// of 729 tokens 2.42 -> 2.14 ms, 2: 3.14 -> 2.88, 4: 4.54 -> 4.29.
 #include "gemm_common.hpp"
 
 namespace tvgemm {
@@ -17,15 +25,17 @@ namespace {
 
 typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
 
+constexpr int GS_THREADS = 512, TOUCH = 4;       // TOUCH: lines of W a thread asks for at most
+
 // WM, WN: a wave's 16-row tiles of A and of W
 template <int WM, int WN, int NS, int EPI>
-__global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
-  constexpr int TM = 32 * WM, TN = 32 * WN, STAGE = (TM + TN) * 128, PA = TM / 8, PW = (TM + TN) / 32;
+__global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel(GemmArgs a) {
+  constexpr int TM = 32 * WM, TN = 32 * WN, STAGE = (TM + TN) * 128, PA = TM / 8, PW = (TM + TN) / 64;
   constexpr bool GLU = EPI == EPI_GLU;
   constexpr int TO = GLU ? TN / 2 : TN;                    // outputs a tile
   extern __shared__ __attribute__((aligned(16))) unsigned char gs_smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave >> 1, wc = wave & 1, lc = lane & 15, kq = lane >> 4;
+  const int wr = (wave & 3) >> 1, wc = wave & 1, kg = wave >> 2, lc = lane & 15, kq = lane >> 4;
 
   // ---- tile: ids of an XCD (id % 8) walk neighbouring tiles, bands of group_m tiles of rows
   int id = blockIdx.x;
@@ -72,30 +82,30 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
 #pragma unroll
   for (int j = 0; j < NS - 1; ++j)
     if (j < nkt) issue(j, j);
-  // fragments of stage t, in slot S, both k-steps
-  bf16x8 af[2][2][WM], wf[2][2][WN];
-  auto read = [&](int S, auto BT) __attribute__((always_inline)) {
-    constexpr int B = decltype(BT)::value;
-    const unsigned st = (unsigned)(S * STAGE);
+  // W on its way from memory, in order, a line a lane, by all work-groups together (the last line again where there is no other)
+  float seen[TOUCH];
+  {
+    const int64_t all = (int64_t)gridDim.x * GS_THREADS, pieces = (int64_t)(GLU ? 2 : 1) * a.N * nkt, most = pieces < 0x7fffffff ? pieces : 0x7fffffff;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-      for (int m = 0; m < WM; ++m) af[B][ks][m] = *(lds_bf16x8*)(size_t)((fa + st + (unsigned)(m * 2048)) ^ (unsigned)(ks * 64));
-#pragma unroll
-      for (int n = 0; n < WN; ++n) wf[B][ks][n] = *(lds_bf16x8*)(size_t)((fw + st + (unsigned)(w_row(n) * 128)) ^ (unsigned)(ks * 64));
+    for (int i = 0; i < TOUCH; ++i) {
+      const int p = (int)min((int64_t)blockIdx.x * GS_THREADS + tid + i * all, most - 1), row = p / nkt;
+      seen[i] = *(const float*)(a.W + (int64_t)row * a.ldw + (p - row * nkt) * BK);
     }
-  };
-  auto multiply = [&](auto BT) __attribute__((always_inline)) {
-    constexpr int B = decltype(BT)::value;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int m = 0; m < WM; ++m)
-#pragma unroll
-        for (int n = 0; n < WN; ++n) acc[m][n] = mfma16(wf[B][ks][n], af[B][ks][m], acc[m][n]);
-  };
+  }
+  bf16x8 af[2][WM], wf[2][WN];                             // by the parity of the stage
+  const unsigned fak = fa ^ (unsigned)(kg * 64), fwk = fw ^ (unsigned)(kg * 64);
   typedef std::integral_constant<int, 0> I0;
   typedef std::integral_constant<int, 1> I1;
+  auto read = [&](int i, unsigned st, auto BT) __attribute__((always_inline)) {
+    constexpr int B = decltype(BT)::value;
+    if (i < WM) af[B][i] = *(lds_bf16x8*)(size_t)(fak + st + (unsigned)(i * 2048));
+    else wf[B][i - WM] = *(lds_bf16x8*)(size_t)(fwk + st + (unsigned)(w_row(i - WM) * 128));
+  };
+  auto products = [&](int lo, int hi, auto BT) __attribute__((always_inline)) {
+    constexpr int B = decltype(BT)::value;
+#pragma unroll
+    for (int i = lo; i < hi; ++i) acc[i / WN][i % WN] = mfma16(wf[B][i % WN], af[B][i / WN], acc[i / WN][i % WN]);
+  };
   if constexpr (NS < 4) {
     int S = 0;
     for (int t = 0; t < nkt; ++t) {
@@ -104,41 +114,94 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
       __builtin_amdgcn_s_barrier();                        // stage t is there for all waves, and all have read stage t - 1
       asm volatile("" ::: "memory");
       if (t + NS - 1 < nkt) issue(t + NS - 1, S == 0 ? NS - 1 : S - 1);
-      read(S, I0{});
-      multiply(I0{});
+#pragma unroll
+      for (int i = 0; i < WM + WN; ++i) read(i, (unsigned)(S * STAGE), I0{});
+      products(0, WM * WN, I0{});
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       S = S == NS - 1 ? 0 : S + 1;
     }
   } else {
-    // four stages: the fragments of stage t + 1 are read while stage t is multiplied; the wait and the barrier of a step are for the stage behind (4 352
-    // columns on 64 x 64 tiles 23.6 -> 19.4 us, on 128 x 128 48 -> 40; with three stages the fragments' second set costs more than it hides, 31 -> 39)
+    // the fragments of stage t + 1 are read, and stage t + NS asked for, between the products of stage t; the wait and the barrier of a step are for the
+    // stage behind
+    constexpr int MF = WM * WN, HEAD = MF / 4, RD = (WM + WN) / PW;
     int S = 0;                                             // slot of stage t
-    auto step = [&](int t, auto BT) __attribute__((always_inline)) {
+    auto step = [&](int t, auto BT, auto LASTT) __attribute__((always_inline)) {
       constexpr int B = decltype(BT)::value;
+      constexpr bool LAST = decltype(LASTT)::value;        // one of the last steps: the copies run out
       const int S1 = S == NS - 1 ? 0 : S + 1;
-      if (t + 1 < nkt) {
-        if (t + NS - 2 < nkt) GEMM_WAIT_VM(PW * (NS - 3));
+      products(0, HEAD, BT);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!LAST || t + 1 < nkt) {
+        if (!LAST || t + NS - 1 < nkt) GEMM_WAIT_VM(PW * (NS - 2));
         else GEMM_WAIT_VM(0);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave has read stage t, and so stage t - 1, whose slot is filled next
-        __builtin_amdgcn_s_barrier();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                      // stage t + 1 is there for all waves, and all have read stage t, whose slot is filled next
         asm volatile("" ::: "memory");
-        if (t + NS - 1 < nkt) issue(t + NS - 1, S == 0 ? NS - 1 : S - 1);
-        read(S1, std::integral_constant<int, B ^ 1>{});
+        const unsigned st = (unsigned)(S1 * STAGE), dst = lds0 + (unsigned)(S * STAGE + wave * PW * 1024);
+        const bool more = !LAST || t + NS < nkt;
+#pragma unroll
+        for (int c = 0; c < PW; ++c) {
+          if (more) glds16(src[c] + (t + NS) * BK, off[c], dst + c * 1024);
+#pragma unroll
+          for (int i = RD * c; i < RD * (c + 1); ++i) read(i, st, std::integral_constant<int, B ^ 1>{});
+          products(HEAD + c * (MF - HEAD) / PW, HEAD + (c + 1) * (MF - HEAD) / PW, BT);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        products(HEAD, MF, BT);
       }
-      multiply(BT);
       S = S1;
     };
-    if (nkt > NS - 2) GEMM_WAIT_VM(PW * (NS - 2));
-    else GEMM_WAIT_VM(0);
+    if (NS - 1 < nkt) {
+      issue(NS - 1, NS - 1);
+      GEMM_WAIT_VM(PW * (NS - 1));
+    } else {
+      GEMM_WAIT_VM(0);
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    read(0, I0{});
+#pragma unroll
+    for (int i = 0; i < WM + WN; ++i) read(i, 0u, I0{});
     int t = 0;
-    for (; t + 1 < nkt; t += 2) {
-      step(t, I0{});
-      step(t + 1, I1{});
+    for (; t + NS + 1 < nkt; t += 2) {
+      step(t, I0{}, std::false_type{});
+      step(t + 1, I1{}, std::false_type{});
     }
-    if (t < nkt) step(t, I0{});
+    for (; t < nkt; t += 2) {
+      step(t, I0{}, std::true_type{});
+      if (t + 1 < nkt) step(t + 1, I1{}, std::true_type{});
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < TOUCH; ++i) asm volatile("" ::"v"(seen[i]));
+  // ---- the two waves of a quarter meet over the ring: each keeps half of the rows, or the first one all of them
+  constexpr int KM = WM < 4 ? WM : WM / 2;                 // 16-row tiles a wave keeps
+  int mk = wr * WM;                                        // its first one
+  f32x4* const meet = (f32x4*)gs_smem;
+  auto at = [&](int w, int i) __attribute__((always_inline)) { return meet + (w * (KM * WN) + i) * 64 + lane; };
+  static_assert((KM < WM ? 8 : 4) * KM * WN * 1024 <= NS * STAGE, "the meeting fits the ring");
+  __syncthreads();
+  if constexpr (KM < WM) {
+#pragma unroll
+    for (int i = 0; i < KM * WN; ++i) {
+      const f32x4 lo = acc[i / WN][i % WN], hi = acc[KM + i / WN][i % WN];
+      *at(wave ^ 4, i) = kg ? lo : hi;
+      acc[i / WN][i % WN] = kg ? hi : lo;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KM * WN; ++i) acc[i / WN][i % WN] += *at(wave, i);
+    mk += kg * KM;
+  } else {
+    if (kg) {
+#pragma unroll
+      for (int i = 0; i < WM * WN; ++i) *at(wave ^ 4, i) = acc[i / WN][i % WN];
+    }
+    __syncthreads();
+    if (kg) return;
+#pragma unroll
+    for (int i = 0; i < WM * WN; ++i) acc[i / WN][i % WN] += *at(wave, i);
   }
 
   // ---- epilogue: a lane holds, of two joined tiles of rows, 8 columns 16 n + 8 (kq >> 1) .. of row 16 (m + (kq & 1)) + lc
@@ -166,7 +229,7 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
       }
     }
 #pragma unroll
-    for (int mp = 0; mp < WM; mp += 2) {
+    for (int mp = 0; mp < KM; mp += 2) {
       float v[8];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -179,7 +242,7 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
           v[4 + r] = gelu_tanh_f(v[4 + r]) * (__uint_as_float(su[1]) + bu[4 + r]);
         }
       }
-      const int row = m0 + 16 * (wr * WM + mp + (kq & 1)) + lc;
+      const int row = m0 + 16 * (mk + mp + (kq & 1)) + lc;
       if (row >= a.M || col >= a.N) continue;
       bf16_t* cp = a.C + (int64_t)row * a.ldc + col;
       if (EPI == EPI_ACCUM) {
@@ -213,7 +276,7 @@ int go_epi(GemmArgs& a, hipStream_t st) {
   a.tiles_m = (a.M + TM - 1) / TM;
   a.tiles_n = (a.N + TO - 1) / TO;
   a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
-  gemm_small_kernel<WM, WN, NS, EPI><<<dim3((unsigned)(a.tiles_m * a.tiles_n)), 256, LDS, st>>>(a);
+  gemm_small_kernel<WM, WN, NS, EPI><<<dim3((unsigned)(a.tiles_m * a.tiles_n)), GS_THREADS, LDS, st>>>(a);
   TV_LAUNCH_CHECK();
 }
 template <int WM, int WN, int NS>
@@ -248,10 +311,16 @@ extern "C" int tv_gemm_small_fwd(const void* A, const void* W, const void* bias,
   a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc;
   a.bias_f32 = bias_dtype == TV_F32;
   hipStream_t st = (hipStream_t)stream;
+  // A tile whose work-groups are more than one round gives way to the next larger one if that fits a round (us: 1 152 x 4 352, 1 024 rows, 288 of 64 x 64 27.5, 144 of
+  // 64 x 128 23.2; 3 456 x 1 152, 729 rows, 324 of 64 x 128 16.4, 162 of 128 x 128 12.1)
+  const int64_t cus = tv_cu_count(), outs = epilogue == EPI_GLU ? 2ll * N : N;
+  auto over = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((outs + tn - 1) / tn); };
+  if (tile == 3 && over(64, 64) > cus && over(64, 128) <= cus) tile = 2;
+  if (tile == 2 && over(64, 128) > cus && over(128, 128) <= cus) tile = 0;
   switch (tile) {
     case 0: return go<4, 4, 4>(a, epilogue, st);
     case 1: return go<4, 4, 2>(a, epilogue, st);
-    case 2: return go<2, 4, 3>(a, epilogue, st);
+    case 2: return go<2, 4, 4>(a, epilogue, st);
     default: return go<2, 2, 4>(a, epilogue, st);
   }
 }

@@ -915,11 +915,10 @@ def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
     """The tile of tv_gemm_small_fwd for rows x n outputs (of either factor with `glu`) where it replaces a library call of a short forward, -1 where it does not.
     Such a forward waits for the host, which a library call takes 19 us of and this one 8: some sizes take longer on the device than the library's, which shows where
     the device is busy with other work or the calls are captured.  64 x 64 up to 1.2 rounds of the compute units (two of them run on one), up to two in contractions of more
-    than 2 048 columns (at most 4 608, at most 1 536 rows), else 64 x 128 up to 1.3, 128 x 128 up to two.
-    us on the device, library | here: 64 x 64: 1 152 x 1 152, 729 rows: 9.5 | 7.5; 5 120 x 2 048, 100: 10.8 | 10.5; 1 152 x 4 352, 196: 11.9 | 18.3, 729: 18.7 | 19.4, 1 024: 22 | 28;
-    64 x 128: 3 456 x 1 152, 588: 13.0 | 14.4, 729: 15.0 | 13.8; 128 x 128: 1 024: 14.4 | 16.1, 1 458: 17.8 | 22.8, with the GELU, 4 352 columns, 1 024: 21.6 | 24.5, 1 458:
-    20.7 + 4 | 22; 1 152 x 4 352, 2 187 rows, left: 31 | 43.  SigLIP so400m, whole forwards | captured: 1 frame of 729: 4 055 -> 2 784 | 2 956 -> 2 631, 3: 4 065 -> 3 883 |
-    3 940 -> 3 928, 1 of 256: 4 014 -> 2 750 | 2 262 -> 2 181, 4: 3 984 -> 3 194 | 2 838 -> 3 195, 8: 4 016 -> 3 887 | 3 724 -> 3 908."""
+    than 2 048 columns (at most 4 608, at most 1 536 rows), else 64 x 128 up to 1.3, 128 x 128 up to two; tv_gemm_small_fwd takes the next larger tile where one of the first two
+    is more than a round and that one fits.
+    us on the device, weights out of cache, library | here: 64 x 64: 1 152 x 1 152, 729 rows: 12.5 | 8.0; 1 152 x 4 352, 729: 22 | 18; 64 x 128: 1 152 x 1 152, 1 458: 13.7 | 10.8;
+    1 152 x 4 352, 1 458: 31 | 26; 128 x 128: 3 456 x 1 152, 729: 17.9 | 14.0; 5 120 x 2 048, 729: 26 | 23; two rounds, 3 456 x 1 152, 1 458: 19 | 24, 2 187: 29 | 26; 5 120 x 2 048, 1 458: 34 | 40."""
     if not 2 <= rows <= 2304 or n < 512 or k % 64 or (k > 2048 and (k > 4608 or rows > 1536)):
         return -1
     over = lambda tm, tn: -(-rows // tm) * -(-n * (2 if glu else 1) // tn)
@@ -932,6 +931,18 @@ def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
     if over(128, 128) <= CUS:
         return 0
     return 1 if over(128, 128) <= CUS * 2 else -1
+
+
+def round_takes(x, weight) -> bool:
+    """Rows beyond `small_tile` on which 128 x 128 tiles (tile 0 of `small_linear`) are faster on the device than the library: one round of them, at least 60 % full, 53 from
+    3 072 columns on.  us with weights out of cache, library (adding to its output) | here: 1 152 x 4 352: 1 499 rows (42 %): 31 | 33, 1 883 (53 %): 36 | 33, 2 395: 40 | 33, 3 419: 43 | 37; 1 152 x 1 152:
+    2 139 (60 %): 13.0 | 12.7, 2 395: 15.3 | 12.7, 2 651: 13.4 | 13.1, 3 547: 15.4 | 15.6; 1 024 x 4 096: 1 755 (44 %): 27 | 29, 2 139: 35 | 29, 4 059: 41 | 35; 768 x 3 072: 2 907 (54 %): 24.3 | 24.7,
+    3 675: 26.4 | 25.3, 5 083: 33 | 28; 1 408 x 6 144: 1 243 (43 %): 40 | 45, 1 499: 50 | 43, 2 779: 59 | 51; 2 048 x 2 048: 987 (50 %): 17.1 | 18.4, 1 243: 22 | 19; 4 096 x 2 048, 603: 23 | 20, 987:
+    25.6 | 24.1.  Two rounds are the library's (1 152 x 4 352, 3 645: 45 | 59)."""
+    rows, (n, k) = x.shape[0], weight.shape
+    tiles = -(-rows // 128) * -(-n // 128)
+    return ((53 if k >= 3072 else 60) * CUS <= 100 * tiles <= 100 * CUS and n >= 512 and n % 8 == 0 and 1024 <= k <= 6144 and k % 64 == 0
+            and products_take(x, weight))
 
 
 def tail_plan(rows: int, n: int, k: int):

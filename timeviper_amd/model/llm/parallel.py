@@ -97,6 +97,8 @@ class ParallelLayer(nn.Module):
         w, waits = self.inp[:self.n1], x.shape[0] * (self.inp.numel() + self.out.numel()) <= HOST_BOUND_WORK
         most = HOST_BOUND_ROWS if waits else 0
         tile = K.small_takes(hs, w, most=most)
+        if tile < 0 and K.round_takes(hs, w):
+            tile = 0
         self.mixer.attend(F.linear(hs, w) if tile < 0 else K.small_linear(hs, w, tile=tile), kv_rows, plan, out=u[:, :self.k1])
         if self.mlp is not None:
             w, act = self.inp[self.n1:], u[:, self.k1:]

@@ -244,12 +244,14 @@ def _own_accumulate(rows: int, n: int) -> bool:
 
 
 def _accumulate(x2: torch.Tensor, h2: torch.Tensor, w: torch.Tensor, role: str) -> None:
-    """x2 += h2 @ w.T (one rounding of the sum to bf16), the residual stream's output projections: the hand-written GEMM with the
-    accumulating epilogue where it is the faster one (`_own_accumulate`; more than 65 536 rows also for the roles named in
+    """x2 += h2 @ w.T (one rounding of the sum to bf16), the residual stream's output projections: small tiles where they take the rows, the hand-written GEMM with
+    the accumulating epilogue where it is the faster one (`_own_accumulate`; more than 65 536 rows also for the roles named in
     TV_VIT_OWN_ACCUM, comma separated: proj, fc2) and the shape allows (bf16, K a multiple of 128 and >= 1 152), else hipBLASLt
     (`torch.addmm`, beta = 1)."""
     rows, n = x2.shape
     tile = K.small_takes(h2, w)
+    if tile < 0 and rows > 2304 and K.round_takes(h2, w):
+        tile = 0
     if tile >= 0 and _gemm_reads(x2) and x2.dtype == h2.dtype:
         K.small_linear(h2, w, None, K.GEMM_ACCUM, out=x2, tile=tile)
     elif ((_own_accumulate(rows, n) or (role in _OWN_ACCUM and rows >= 65536)) and x2.is_cuda and x2.dtype == torch.bfloat16
