@@ -670,7 +670,7 @@ int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int
  *   returns.  cu (sequences + 1), start, slot (sequences) int32 on the device, and per new token its cache row (slot * capacity + position)
  *   and its sequence; keys (sequences; may be NULL) = start + 1.
  * tv_argmax_rows: out[r] = position of the largest of n <= 2^30 fp32 values (NaN above all, the lowest of equals: torch.argmax).
- * tv_argmax_rows_count: the same, and tv_count_up in its last launch (pos NULL: nothing is counted). */
+ * tv_argmax_rows_count: the same, and tv_count_up in its last launch (pos, lens: either may be NULL, nothing is counted there). */
 int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* pos, int batch, int64_t capacity,
                  int row_bytes, int64_t k_stride_b, int64_t v_stride_b, int64_t kc_stride_b, int64_t kc_stride_l, int64_t vc_stride_b,
                  int64_t vc_stride_l, void* stream);

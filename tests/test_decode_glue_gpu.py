@@ -29,6 +29,15 @@ def test_argmax(rows, n, pad, kind):
     assert got.dtype == torch.int64 and torch.equal(got.cpu(), want)
 
 
+@pytest.mark.parametrize("rows,n", [(1, 8192), (12, 32768), (2, 100)])
+@pytest.mark.parametrize("lens", [0, 5, 70])
+def test_counters_without_a_position(rows, n, lens):
+    from timeviper_amd import kernels as ops
+    x = torch.randn(rows, n, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV)
+    c = torch.arange(lens, dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.argmax_rows(x, (None, c)), x.argmax(-1)) and c.tolist() == list(range(1, lens + 1))
+
+
 @pytest.mark.parametrize("B,H,D,sliced", [(1, 8, 128, True), (5, 2, 72, False), (12, 8, 128, True), (3, 1, 4, False)])
 def test_append_and_count(B, H, D, sliced):
     from timeviper_amd import kernels as ops

@@ -62,14 +62,15 @@ __global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restric
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.y * ARG_BLOCKS + blockIdx.x] = better(better(s[0], s[1]), better(s[2], s[3]));
 }
-// ... and (pos not NULL) the counters that count_up_kernel moves, by the first row's work-group (3.9 us as a launch of its own)
+// ... and the counters that count_up_kernel moves (either may be NULL), by the first row's work-group (3.9 us as a launch of its own)
 __global__ __launch_bounds__(ARG_BLOCKS) void argmax_rows_kernel(const Best* __restrict__ part, int64_t* __restrict__ out, int64_t* __restrict__ pos,
                                                                  int* __restrict__ lens, int nlens) {
   const Best b = wave_best(part[blockIdx.x * ARG_BLOCKS + threadIdx.x]);
   if (threadIdx.x == 0) out[blockIdx.x] = (int64_t)b.i;
-  if (pos && blockIdx.x == 0) {
-    if (threadIdx.x == 0) pos[0] += 1;
-    for (int i = threadIdx.x; i < nlens; i += ARG_BLOCKS) lens[i] += 1;
+  if (blockIdx.x == 0) {
+    if (pos && threadIdx.x == 0) pos[0] += 1;
+    if (lens)
+      for (int i = threadIdx.x; i < nlens; i += ARG_BLOCKS) lens[i] += 1;
   }
 }
 

@@ -1115,12 +1115,16 @@ def count_up(pos, lens) -> None:
 
 
 def argmax_rows(x, count=None):
-    """x.argmax(-1); the fp32 logits of up to 65 535 rows by 64 work-groups a row.  count=(pos, lens): `count_up` of them in the same launches."""
+    """x.argmax(-1) of the fp32 logits of up to 65 535 rows.  count=(pos, lens): `count_up` of them in the same launch (pos may be None)."""
     pos, lens = count or (None, None)
     takes = x.is_cuda and x.dim() == 2 and x.dtype == torch.float32 and x.stride(1) == 1 and 0 < x.shape[0] <= 65535 and 8192 <= x.shape[1] <= (1 << 30)
-    if count and not (takes and lens.dtype == torch.int32 and lens.is_contiguous() and lens.is_cuda and pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1):
+    if count and not (takes and lens.dtype == torch.int32 and lens.is_contiguous() and lens.is_cuda
+                      and (pos is None or pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1)):
         out = argmax_rows(x)
-        count_up(pos, lens)
+        if pos is None:
+            lens += 1
+        else:
+            count_up(pos, lens)
         return out
     if not takes:
         return x.argmax(-1)

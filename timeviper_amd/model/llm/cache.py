@@ -38,7 +38,7 @@ class StaticDecode:
         raise NotImplementedError
 
     def static_counters(self):
-        """(an int64 counter, int32 counters) that `advance_static_device` adds one to, for a launch that does it on its way; None: call it."""
+        """(an int64 counter or None, int32 counters) that `advance_static_device` adds one to, for a launch that does it on its way; None: call it."""
         return None
 
     def advance_static_host(self):
@@ -242,6 +242,10 @@ class SlotStateCache(StaticDecode):
 
     def advance_static_device(self):
         self._advance_device(self._decode_plan)
+
+    def static_counters(self):
+        same = type(self).advance_static_device is SlotStateCache.advance_static_device and type(self)._advance_device is SlotStateCache._advance_device
+        return (None, self._decode_plan.moving) if same else None
 
     def advance_static_host(self):
         p = self._decode_plan
