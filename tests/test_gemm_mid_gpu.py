@@ -34,6 +34,19 @@ def test_products(M, N, K, relu2, bias):
     assert torch.equal(got, ops.mid_linear(x, w, b, relu2).double())      # the splits add in one order
 
 
+# W with and without the caches (splits of K, or the rows of W from end to end), on both sides of 64 and 128 rows, splits that start 4 KiB apart and not
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 256])
+@pytest.mark.parametrize("N,K", [(16388, 512), (2048, 4096), (1152, 5120), (1152, 4992)])
+def test_split_and_whole_rows(M, N, K):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV).to(BF), (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF)
+    got, want = ops.mid_linear(x, w).double(), x.double() @ w.double().T
+    # fp32 sums (relative 2^-24 a product of the sum of magnitudes), one rounding to bf16
+    acc = (x.double().abs() @ w.double().abs().T) * K * 2.0 ** -24
+    assert ((got - want).abs() <= acc * (1 + 2.0 ** -8) + want.abs() * 2.0 ** -8 + 1e-30).all()
+
+
 @pytest.mark.parametrize("tokens", [2, 17, 48, 200, 256, 257])
 def test_layers_take_them(tokens, monkeypatch):
     """The hybrid stack's projections: the short-prompt products within a rounding of torch.nn.Linear; hooks and gradients keep the module."""

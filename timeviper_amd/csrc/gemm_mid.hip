@@ -8,11 +8,14 @@
 //   * One barrier a stage, in the middle of its products: the fragments of a 16-column step are read while the step before is multiplied
 //     (v_mfma_f32_32x32x16_bf16, W on the A side: a lane's registers are consecutive outputs of one row of x).
 //   * The waves along K meet over the rings, in an order that stores whole rows of y.
-// What bounds it: a compute unit takes in W and x together at about 45 bytes a ns — alone, x comes from L2 at 80, but loads return in order
-// and those of x queue behind W's — so the time grows with the rows: x is read again by every work-group.
+//   * W past the caches (non-temporal) where a work-group reads its rows of W from end to end, or for 64 rows and less; split along K, with more rows, pieces of a row are asked for by
+//     work-groups that do not run in step, and plain loads are better (us, non-temporal | plain, 128 and 203 rows: 4 480 x 5 120 24.7 30.4 | 22.6 26.6, 4 480 x 10 240 33.9 38.6 | 32.1 36.6,
+//     7 168 x 4 480 28.5 33.1 | 26.1 30.3; unsplit, 22 656 x 4 480 52.1 59.7 | 53.8 61.2; 64 rows of 22 656 41.4 | 44.1).
+// What bounds it: up to 64 rows the stream of W.  With 256 rows a stage of 128 rows of W takes 1.1 us, .8 of them where all copies hit the same lines, .57 without copies, .74 without
+// fragment reads (copies dealt out between the products instead of in one burst change nothing); splits cost their sums' way through memory.
 // fp32 accumulation, one rounding of y.
-// Measured (weights not in any cache; library -> here): 4 480 x 15 680, 33 | 128 | 203 | 256 rows 65 | 89 | 131 | 148 -> 31 | 44 | 52 | 52 us; 4 480 x 10 240
-// 52 | 57 | 83 | 92 -> 24 | 35 | 41 | 42; 15 680 x 4 480 with 33 | 64 rows 40 | 42 -> 28 | 32.
+// Measured (weights not in any cache; library -> here): 4 480 x 15 680, 33 | 128 | 203 | 256 rows 65 | 89 | 131 | 148 -> 31 | 42 | 47 | 51 us; 4 480 x 10 240
+// 52 | 57 | 83 | 92 -> 24 | 32 | 37 | 40; 15 680 x 4 480 with 33 | 64 | 96 rows 40 | 42 | 37 -> 28 | 32 | 35; 22 656 x 4 480, 128 | 256 55 | 73 -> 53 | 64.
 #include "gemm_skinny.hpp"
 
 namespace {
@@ -27,7 +30,7 @@ struct GmArgs {
   const bf16_t *x, *W, *bias;
   bf16_t* y;
   float* part;                                     // split K: [split][M][N rounded up to tiles]
-  int M, N, K, tiles, splits, per_xcd, relu2;
+  int M, N, K, tiles, splits, per_xcd, relu2, nt;  // nt: W is read past the caches
   int64_t xs, ldw, ys;
 };
 
@@ -125,16 +128,17 @@ __global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ni], x[mi], acc[mi][ni], 0, 0, 0);
   };
-  // The loop of a wave that copies x (SIDE 0) or W (SIDE 1): J copies a stage into NS slots.  At a step's meeting stage i + 1 is in LDS for
+  // The loop of a wave that copies x (SIDE 0) or W (SIDE 1: past the caches, 2): J copies a stage into NS slots.  At a step's meeting stage i + 1 is in LDS for
   // all waves and every wave has read stage i, whose slot is filled again behind it.
   auto run = [&](auto side) __attribute__((always_inline)) {
-    constexpr bool XS = decltype(side)::value == 0;
+    constexpr int SIDE = decltype(side)::value;
+    constexpr bool XS = SIDE == 0;
     constexpr int NS = XS ? NSX : NSW, J = XS ? XT : NI, ST = XS ? XST : WST;
     const unsigned base = __builtin_amdgcn_readfirstlane((XS ? ringx : ringw) + 1024u * J * (wave & 3));
     auto issue = [&](int i, int slot) __attribute__((always_inline)) {
       const unsigned dst = __builtin_amdgcn_readfirstlane(base + (unsigned)(slot * ST));
       if constexpr (XS) glds_many<XT, false>(uniform_ptr(xb + (int64_t)i * GM_KC), vx, dst);
-      else glds_many<NI, true>(uniform_ptr(Wb + (int64_t)i * GM_KC), vw, dst);
+      else glds_many<NI, SIDE == 1>(uniform_ptr(Wb + (int64_t)i * GM_KC), vw, dst);
     };
     auto meet_counted = [&]() __attribute__((always_inline)) {
       __builtin_amdgcn_sched_barrier(0);
@@ -220,7 +224,8 @@ __global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
     }
   };
   if (xside) run(std::integral_constant<int, 0>{});
-  else run(std::integral_constant<int, 1>{});
+  else if (XT == 2 || a.nt) run(std::integral_constant<int, 1>{});
+  else if constexpr (XT > 2) run(std::integral_constant<int, 2>{});
   // ---- the waves along K meet over the rings, MI rounds: [wave][n-tile][register quad][hh][r rotated] f32x4, summed in the order of rows of y
   f32x4* meet = (f32x4*)gm_smem;
   constexpr int NC = 8 * NI;                       // chunks of four outputs a row
@@ -292,18 +297,25 @@ int launch_one(const GmArgs& a, hipStream_t st) {
 struct GmPlan {
   int ni, splits, xt;
 };
-// The tile width and split of K with the smallest estimate: per stage the larger of W from HBM (6.3 TB/s over all compute units) and W and x through
-// the compute unit's memory pipe (45 bytes a ns, measured: x hits the L2, but its loads queue behind those of W), per work-group 3 us of
-// fill and epilogue, per split 4 M N bytes written and read at 5 TB/s and a second launch.
+// The tile width and split of K with the smallest estimate, us: a stage is a part for the rows of x and one for the 32-row tiles of W, which grows with the work-groups that stream W at once;
+// each round of work-groups has its fill and epilogue, a launch its own; a split adds a second launch and 4 M N bytes written and read per split, and splits that start
+// whole multiples of 4 KiB apart in a row meet in memory (4 480 x 10 240, 96 rows, five of 2 048 columns 33.6, seven 30.1; rows a power of two apart meet there however they are split).
+// The numbers are a fit to 2 900 timings, 18 sizes of N and K (1 024 to 22 656) with 33 to 256 rows: over those its choice is .7 % slower in the mean than the best one, 10 % at most.  The
+// estimate before (W and x through the compute unit's memory pipe at 45 bytes a ns) split more: with the loads as they are now 1.06 times as slow in the mean
+// (2 048 x 7 680, 203 rows: 11 splits 25.4 us, 8 of narrower tiles 20.9; 5 120 x 2 048, 160 rows: 20.7, 17.5; 15 680 x 4 480, 96 rows: two splits 41.0, unsplit 35.4).
 GmPlan plan(int M, int N, int K) {
-  GmPlan best{4, 1, M <= 64 ? 2 : M <= 128 ? 4 : 8};
+  static constexpr double X[3] = {.046, .11, .35}, W[3] = {.061, .065, .056}, FILL[3] = {1.7, 2.2, .87};
+  const int c = M <= 64 ? 0 : M <= 128 ? 1 : 2;
+  GmPlan best{4, 1, 2 << c};
   const int cus = tv_cu_count(), nst = K / GM_KC;
   double least = 1e30;
   for (int ni = 4; ni >= 2; --ni)
-    for (int s = 1; s <= 16 && s * 8 <= nst; ++s) {
+    for (int s = 1; s <= 16 && (s == 1 || s * 8 <= nst); ++s) {
       const int64_t units = (int64_t)((N + 32 * ni - 1) / (32 * ni)) * s, rounds = (units + cus - 1) / cus;
-      const double hbm = ni * 4096. * cus / 6300., pipe = (ni + best.xt) * 4096. / 45.;
-      const double t = rounds * (((nst + s - 1) / s) * (hbm > pipe ? hbm : pipe) + 3000.) + (s > 1 ? 3000. + 2. * s * N * M * 4 / 5000. : 0.);
+      const double stage = X[c] + ni * (W[c] + .1 * (units < cus ? units : cus) / cus);
+      double t = rounds * (FILL[c] + (nst + s - 1) / s * stage) + 3.7;
+      if (s > 1) t += .7 + s * (.15 + 1.56e-6 * N * M);
+      if (s > 1 && K / s * 2 % 4096 == 0 && (K & (K - 1))) t *= 1.12;
       if (t < least) {
         least = t;
         best.ni = ni;
@@ -352,6 +364,7 @@ extern "C" int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, v
   a.splits = p.splits;
   a.per_xcd = (a.tiles * a.splits + 7) / 8;
   a.part = p.splits > 1 ? (float*)workspace : nullptr;
+  a.nt = p.splits == 1 || M <= 64;
   hipStream_t st = (hipStream_t)stream;
   switch (p.ni) {
     case 2: return launch_ni<2>(a, p.xt, st);
