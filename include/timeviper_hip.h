@@ -661,6 +661,10 @@ int tv_token_side_fwd(const void* h, const int64_t* ids, const void* table, cons
 size_t tv_gemm_mid_workspace_bytes(int M, int N, int K);
 int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
                     int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream);
+/* The same rows with 1 to 3 matrices in one launch, y[i] = x W[i]^T, W[i] (N[i], K); the lists are on the host and read before the call returns. */
+size_t tv_gemm_mid_multi_workspace_bytes(int M, const int* N, int matrices, int K);
+int tv_gemm_mid_multi_fwd(const void* x, const void* const* W, void* const* y, const int* N, int matrices, int M, int K, int64_t x_stride,
+                          const int64_t* ldw, const int64_t* y_stride, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Between the layers of a decoded token and the next one (csrc/decode_glue.hip).
  * tv_kv_append: k / v, one row of row_bytes per sequence, to position *pos (device) of the caches; all strides in bytes, everything a

@@ -77,3 +77,52 @@ def test_layers_take_them(tokens, monkeypatch):
         nano._prompt_linear(lin, x)
     handle.remove()
     assert not calls and seen
+
+
+# two and three matrices: edges of the tiles of each, with and without a split of K, rows of W of another stride
+@pytest.mark.parametrize("M", [2, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("Ns,K", [((4096, 4), 4096), ((4000, 132, 100), 4160), ((5120, 1024, 1024), 4480), ((24580, 300, 64), 4096)])
+def test_several_matrices(M, Ns, K):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + sum(Ns))
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x = r(1, M, K).to(BF)
+    ws = [(r(n, K + 8) * K ** -0.5).to(BF)[:, :K] for n in Ns]
+    assert ops.mid_linears_take(x, ws)
+    got = ops.mid_linears(x, ws)
+    for y, w in zip(got, ws):
+        assert y.shape == (1, M, w.shape[0]) and y.is_contiguous()
+        want = x[0].double() @ w.double().T
+        # fp32 sums (relative 2^-24 a product of the sum of magnitudes), one rounding to bf16
+        acc = (x[0].double().abs() @ w.double().abs().T) * K * 2.0 ** -24
+        assert ((y[0].double() - want).abs() <= acc * (1 + 2.0 ** -8) + want.abs() * 2.0 ** -8 + 1e-30).all()
+    assert all(torch.equal(a, b) for a, b in zip(got, ops.mid_linears(x, ws)))
+    x2 = r(M, 2 * K).to(BF)[:, :K]                             # rows that are not dense: without the native host side
+    assert all(torch.equal(a, b) for a, b in zip(ops.mid_linears(x2, ws), ops.mid_linears(x2.contiguous(), ws)))
+
+
+@pytest.mark.parametrize("tokens", [2, 40, 256, 257])
+def test_attention_takes_them(tokens, monkeypatch):
+    """q, k and v of a prompt in one launch, within a rounding of the modules; hooks, biases and gradients keep the modules"""
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    cfg = nano.NemotronHConfig.nemotron_nano_9b_v2(vocab_size=256, num_hidden_layers=1, hybrid_override_pattern="*")
+    torch.manual_seed(tokens)
+    att = nano.NemotronHAttention(cfg, 0).to(DEV, BF).requires_grad_(False)
+    x = torch.randn(1, tokens, cfg.hidden_size, device=DEV, dtype=BF)
+    calls, real = [], ops.mid_linears
+    monkeypatch.setattr(ops, "mid_linears", lambda *a: (calls.append(1), real(*a))[1])
+    with torch.no_grad():
+        got = att._qkv(x)
+    assert bool(calls) == (tokens <= 256)
+    for y, m in zip(got, (att.q_proj, att.k_proj, att.v_proj)):
+        want = F.linear(x.double(), m.weight.double())
+        assert (y.double() - want).abs().max() <= 1.05 * 2.0 ** -8 * want.abs().max()
+    calls.clear()
+    att._qkv(x)                                                # gradients enabled
+    seen = []
+    handle = att.k_proj.register_forward_hook(lambda *a: seen.append(1))
+    with torch.no_grad():
+        att._qkv(x)
+    handle.remove()
+    assert not calls and seen

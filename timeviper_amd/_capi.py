@@ -96,6 +96,8 @@ SIGNATURES = {
     "tv_gemm_rows_glu_fwd": (_i, [_p] * 4 + [_l, _p] + [_i] * 3 + [_l] * 4 + [_p]),
     "tv_gemm_rows_pair_fwd": (_i, [_p] * 6 + [_i] * 4 + [_l] * 5 + [_p]),
     "tv_gemm_mid_workspace_bytes": (_z, [_i] * 3),
+    "tv_gemm_mid_multi_workspace_bytes": (_z, [_i, _p, _i, _i]),
+    "tv_gemm_mid_multi_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l, _p, _p, _p, _z, _p]),
     "tv_gemm_mid_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l] * 3 + [_i, _p, _z, _p]),
     "tv_kv_append": (_i, [_p] * 5 + [_i, _l, _i] + [_l] * 6 + [_p]),
     "tv_step_plan": (_i, [_p] * 3 + [_i, _i] + [_p] * 7),

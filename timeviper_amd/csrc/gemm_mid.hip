@@ -26,16 +26,33 @@ typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
 constexpr int GM_KC = 64;                          // columns of a stage
 constexpr int GM_WAVES = 8;
 
-struct GmArgs {
-  const bf16_t *x, *W, *bias;
+// One of the up to three matrices that the rows of x meet in one launch: its tiles end in front of tile `end` of all
+struct GmMat {
+  const bf16_t* W;
   bf16_t* y;
-  float* part;                                     // split K: [split][M][N rounded up to tiles]
-  int M, N, K, tiles, splits, per_xcd, relu2, nt;  // nt: W is read past the caches
-  int64_t xs, ldw, ys;
+  int N, end;
+  int64_t ldw, ys;
 };
+struct GmArgs {
+  const bf16_t *x, *bias;                          // (a bias: one matrix)
+  GmMat m0, m1, m2;                                // (not an array: an index that is no constant would put the arguments into memory)
+  float* part;                                     // split K: [split][M][all tiles' columns]
+  int M, K, tiles, splits, per_xcd, relu2, nt;     // nt: W is read past the caches
+  int64_t xs;
+};
+// the matrix of a tile, and the tile's place in it
+__device__ __forceinline__ GmMat mat_of(const GmArgs& a, int& tile) {
+  if (tile < a.m0.end) return a.m0;
+  if (tile < a.m1.end) {
+    tile -= a.m0.end;
+    return a.m1;
+  }
+  tile -= a.m1.end;
+  return a.m2;
+}
 
 // four consecutive outputs n.. of row m: bias, one rounding, squared ReLU of what was rounded
-__device__ __forceinline__ void put(const GmArgs& a, int m, int n, f32x4 s) {
+__device__ __forceinline__ void put(const GmArgs& a, const GmMat& w, int m, int n, f32x4 s) {
   if (a.bias) {
     const bf16x4 b = *(const bf16x4*)(a.bias + n);
 #pragma unroll
@@ -50,7 +67,7 @@ __device__ __forceinline__ void put(const GmArgs& a, int m, int n, f32x4 s) {
       o[j] = (bf16_t)(r * r);
     }
   }
-  *(bf16x4*)(a.y + (int64_t)m * a.ys + n) = o;
+  *(bf16x4*)(w.y + (int64_t)m * w.ys + n) = o;
 }
 
 template <int J, bool NT>
@@ -83,7 +100,9 @@ __global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
   const int unit = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
   if (unit >= a.tiles * a.splits) return;
   const int split = unit / a.tiles, tile = unit - split * a.tiles;
-  const int n0 = tile * (32 * NI);
+  int in_mat = tile;
+  const GmMat mat = mat_of(a, in_mat);
+  const int n0 = in_mat * (32 * NI);
   const int nst = a.K / GM_KC;
   const int s0 = (int)((int64_t)nst * split / a.splits), ns = (int)((int64_t)nst * (split + 1) / a.splits) - s0;
 
@@ -94,14 +113,14 @@ __global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int row = 8 * ((wave & 3) * NI + i) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
-    vw[i] = (unsigned)(((int64_t)min(row, a.N - 1 - n0) * a.ldw + ch * 8) * 2);
+    vw[i] = (unsigned)(((int64_t)min(row, mat.N - 1 - n0) * mat.ldw + ch * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < XT; ++i) {
     const int row = 8 * ((wave & 3) * XT + i) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
     vx[i] = (unsigned)(((int64_t)min(row, a.M - 1) * a.xs + ch * 8) * 2);
   }
-  const bf16_t* Wb = a.W + (int64_t)n0 * a.ldw + (int64_t)s0 * GM_KC;
+  const bf16_t* Wb = mat.W + (int64_t)n0 * mat.ldw + (int64_t)s0 * GM_KC;
   const bf16_t* xb = a.x + (int64_t)s0 * GM_KC;
   f32x16_t acc[MI][NI];
 #pragma unroll
@@ -247,17 +266,21 @@ __global__ __launch_bounds__(GM_WAVES * 64) void gemm_mid_kernel(GmArgs a) {
 #pragma unroll
       for (int k = 1; k < WK; ++k) s += meet[((k * WM + w) * NC + c) * 32 + ((rr + c) & 31)];
       if (m >= a.M) continue;
-      if (a.part) *(f32x4*)(a.part + ((int64_t)split * a.M + m) * (a.tiles * 32 * NI) + n) = s;
-      else if (n < a.N) put(a, m, n, s);
+      if (a.part) *(f32x4*)(a.part + ((int64_t)split * a.M + m) * (a.tiles * 32 * NI) + tile * (32 * NI) + 4 * c) = s;
+      else if (n < mat.N) put(a, mat, m, n, s);
     }
   }
 }
 
 // sum over the splits, in their order
-__global__ __launch_bounds__(256) void gemm_mid_sum_kernel(GmArgs a, int np) {
-  const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y;
-  if (n >= a.N) return;
-  const float* p = a.part + (int64_t)m * np + n;
+__global__ __launch_bounds__(256) void gemm_mid_sum_kernel(GmArgs a, int width) {
+  const int col = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, m = blockIdx.y, np = a.tiles * width;
+  if (col >= np) return;
+  const bool first = col < a.m0.end * width, second = col < a.m1.end * width;
+  const GmMat mat = first ? a.m0 : second ? a.m1 : a.m2;
+  const int n = col - (first ? 0 : (second ? a.m0.end : a.m1.end) * width);
+  if (n >= mat.N) return;
+  const float* p = a.part + (int64_t)m * np + col;
   const int64_t step = (int64_t)a.M * np;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   for (int c = 0; c < a.splits; c += 4) {
@@ -268,7 +291,7 @@ __global__ __launch_bounds__(256) void gemm_mid_sum_kernel(GmArgs a, int np) {
     for (int u = 0; u < 4; ++u)
       if (c + u < a.splits) s += v[u];
   }
-  put(a, m, n, s);
+  put(a, mat, m, n, s);
 }
 
 template <int NI, int MI, int WM, int WK, int NSX, int NSW>
@@ -289,7 +312,7 @@ int launch_one(const GmArgs& a, hipStream_t st) {
       tv_set_error("gemm_mid: %s", hipGetErrorString(e));
       return TV_ERR_LAUNCH;
     }
-    gemm_mid_sum_kernel<<<dim3((unsigned)((a.N + 1023) / 1024), (unsigned)a.M), 256, 0, st>>>(a, a.tiles * 32 * NI);
+    gemm_mid_sum_kernel<<<dim3((unsigned)((a.tiles * 32 * NI + 1023) / 1024), (unsigned)a.M), 256, 0, st>>>(a, 32 * NI);
   }
   TV_LAUNCH_CHECK();
 }
@@ -303,18 +326,22 @@ struct GmPlan {
 // The numbers are a fit to 2 900 timings, 18 sizes of N and K (1 024 to 22 656) with 33 to 256 rows: over those its choice is .7 % slower in the mean than the best one, 10 % at most.  The
 // estimate before (W and x through the compute unit's memory pipe at 45 bytes a ns) split more: with the loads as they are now 1.06 times as slow in the mean
 // (2 048 x 7 680, 203 rows: 11 splits 25.4 us, 8 of narrower tiles 20.9; 5 120 x 2 048, 160 rows: 20.7, 17.5; 15 680 x 4 480, 96 rows: two splits 41.0, unsplit 35.4).
-GmPlan plan(int M, int N, int K) {
+int tiles_of(int N, int ni) { return (N + 32 * ni - 1) / (32 * ni); }
+GmPlan plan(int M, const int* N, int matrices, int K) {
   static constexpr double X[3] = {.046, .11, .35}, W[3] = {.061, .065, .056}, FILL[3] = {1.7, 2.2, .87};
   const int c = M <= 64 ? 0 : M <= 128 ? 1 : 2;
   GmPlan best{4, 1, 2 << c};
   const int cus = tv_cu_count(), nst = K / GM_KC;
-  double least = 1e30;
-  for (int ni = 4; ni >= 2; --ni)
+  double least = 1e30, outs = 0;
+  for (int i = 0; i < matrices; ++i) outs += N[i];
+  for (int ni = 4; ni >= 2; --ni) {
+    int64_t tiles = 0;
+    for (int i = 0; i < matrices; ++i) tiles += tiles_of(N[i], ni);
     for (int s = 1; s <= 16 && (s == 1 || s * 8 <= nst); ++s) {
-      const int64_t units = (int64_t)((N + 32 * ni - 1) / (32 * ni)) * s, rounds = (units + cus - 1) / cus;
+      const int64_t units = tiles * s, rounds = (units + cus - 1) / cus;
       const double stage = X[c] + ni * (W[c] + .1 * (units < cus ? units : cus) / cus);
       double t = rounds * (FILL[c] + (nst + s - 1) / s * stage) + 3.7;
-      if (s > 1) t += .7 + s * (.15 + 1.56e-6 * N * M);
+      if (s > 1) t += .7 + s * (.15 + 1.56e-6 * outs * M);
       if (s > 1 && K / s * 2 % 4096 == 0 && (K & (K - 1))) t *= 1.12;
       if (t < least) {
         least = t;
@@ -322,6 +349,7 @@ GmPlan plan(int M, int N, int K) {
         best.splits = s;
       }
     }
+  }
   return best;
 }
 
@@ -340,27 +368,49 @@ bool takes(const void* x, const void* W, int M, int N, int K, int64_t xs, int64_
 
 }  // namespace
 
-extern "C" size_t tv_gemm_mid_workspace_bytes(int M, int N, int K) {
-  if (M < 1 || M > TV_GEMM_MID_MAX || N < 1 || K < GM_KC) return 0;
-  const GmPlan p = plan(M, N, K);
-  return p.splits > 1 ? (size_t)p.splits * M * ((N + 32 * p.ni - 1) / (32 * p.ni)) * (128 * p.ni) : 0;
+extern "C" size_t tv_gemm_mid_multi_workspace_bytes(int M, const int* N, int matrices, int K) {
+  if (M < 1 || M > TV_GEMM_MID_MAX || K < GM_KC || !N || matrices < 1 || matrices > 3) return 0;
+  int64_t all = 0;
+  for (int i = 0; i < matrices; ++i) {
+    if (N[i] < 1) return 0;
+    all += N[i];
+  }
+  if (all > 0x7fffffff) return 0;
+  const GmPlan p = plan(M, N, matrices, K);
+  int64_t tiles = 0;
+  for (int i = 0; i < matrices; ++i) tiles += tiles_of(N[i], p.ni);
+  return p.splits > 1 ? (size_t)p.splits * M * tiles * (128 * p.ni) : 0;
 }
 
-extern "C" int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
-                               int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
-  TV_CHECK_ARG(x && W && y, "gemm_mid: null pointer");
-  TV_CHECK_ARG(M >= 1 && M <= TV_GEMM_MID_MAX && N >= 1 && K >= 1, "gemm_mid: M %d must be 1..%d, N %d and K %d positive", M, TV_GEMM_MID_MAX, N, K);
-  TV_CHECK_ARG(epilogue == 0 || epilogue == TV_GEMM_ROWS_RELU2, "gemm_mid: epilogue %d", epilogue);
-  if (!takes(x, W, M, N, K, x_stride, ldw) || y_stride % 4 || ((uintptr_t)y & 7) || ((uintptr_t)bias & 7))
-    TV_UNSUPPORTED("gemm_mid: K must be a multiple of %d, N and the row stride of y of 4, those of x and W of 8, x and W 16-byte, y and bias 8-byte aligned",
-                   GM_KC);
-  const GmPlan p = plan(M, N, K);
-  const size_t need = tv_gemm_mid_workspace_bytes(M, N, K);
-  TV_CHECK_ARG(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0), "gemm_mid: workspace of %zu bytes needed", need);
+extern "C" size_t tv_gemm_mid_workspace_bytes(int M, int N, int K) { return tv_gemm_mid_multi_workspace_bytes(M, &N, 1, K); }
+
+static int mid_go(const char* what, const void* x, const void* const* W, const void* bias, void* const* y, const int* N, int matrices, int M, int K,
+                  int64_t x_stride, const int64_t* ldw, const int64_t* y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(M >= 1 && M <= TV_GEMM_MID_MAX && K >= 1, "%s: M %d must be 1..%d, K %d positive", what, M, TV_GEMM_MID_MAX, K);
+  TV_CHECK_ARG(epilogue == 0 || epilogue == TV_GEMM_ROWS_RELU2, "%s: epilogue %d", what, epilogue);
+  int64_t all = 0;
+  for (int i = 0; i < matrices; ++i) {
+    TV_CHECK_ARG(x && W[i] && y[i], "%s: null pointer", what);
+    TV_CHECK_ARG(N[i] >= 1, "%s: N %d must be positive", what, N[i]);
+    if (!takes(x, W[i], M, N[i], K, x_stride, ldw[i]) || y_stride[i] % 4 || ((uintptr_t)y[i] & 7) || ((uintptr_t)bias & 7))
+      TV_UNSUPPORTED("%s: K must be a multiple of %d, N and the row stride of y of 4, those of x and W of 8, x and W 16-byte, y and bias 8-byte aligned", what, GM_KC);
+    all += N[i];
+  }
+  if (all > 0x7fffff00) TV_UNSUPPORTED("%s: %lld outputs", what, (long long)all);
+  const GmPlan p = plan(M, N, matrices, K);
+  const size_t need = tv_gemm_mid_multi_workspace_bytes(M, N, matrices, K);
+  TV_CHECK_ARG(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0), "%s: workspace of %zu bytes needed", what, need);
   GmArgs a{};
-  a.x = (const bf16_t*)x; a.W = (const bf16_t*)W; a.bias = (const bf16_t*)bias; a.y = (bf16_t*)y;
-  a.M = M; a.N = N; a.K = K; a.xs = x_stride; a.ldw = ldw; a.ys = y_stride; a.relu2 = epilogue == TV_GEMM_ROWS_RELU2;
-  a.tiles = (N + 32 * p.ni - 1) / (32 * p.ni);
+  a.x = (const bf16_t*)x; a.bias = (const bf16_t*)bias;
+  a.M = M; a.K = K; a.xs = x_stride; a.relu2 = epilogue == TV_GEMM_ROWS_RELU2;
+  GmMat* const to[3] = {&a.m0, &a.m1, &a.m2};
+  for (int i = 0; i < 3; ++i) {
+    if (i < matrices) {
+      a.tiles += tiles_of(N[i], p.ni);
+      *to[i] = GmMat{(const bf16_t*)W[i], (bf16_t*)y[i], N[i], 0, ldw[i], y_stride[i]};
+    }
+    to[i]->end = a.tiles;                                     // (a matrix that is not there has no tiles)
+  }
   a.splits = p.splits;
   a.per_xcd = (a.tiles * a.splits + 7) / 8;
   a.part = p.splits > 1 ? (float*)workspace : nullptr;
@@ -371,4 +421,17 @@ extern "C" int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, v
     case 3: return launch_ni<3>(a, p.xt, st);
     default: return launch_ni<4>(a, p.xt, st);
   }
+}
+
+extern "C" int tv_gemm_mid_fwd(const void* x, const void* W, const void* bias, void* y, int M, int N, int K, int64_t x_stride, int64_t ldw,
+                               int64_t y_stride, int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
+  return mid_go("gemm_mid", x, &W, bias, &y, &N, 1, M, K, x_stride, &ldw, &y_stride, epilogue, workspace, workspace_bytes, stream);
+}
+
+// Up to three matrices in one launch.  An attention layer's q, k and v are 40 + 8 + 8 tiles of 256 compute units: 203 rows x (5 120, 1 024, 1 024) x 4 480, library, one by one |
+// here 27 + 20 + 20 | 31 us.
+extern "C" int tv_gemm_mid_multi_fwd(const void* x, const void* const* W, void* const* y, const int* N, int matrices, int M, int K, int64_t x_stride,
+                                     const int64_t* ldw, const int64_t* y_stride, void* workspace, size_t workspace_bytes, void* stream) {
+  TV_CHECK_ARG(W && y && N && ldw && y_stride && matrices >= 1 && matrices <= 3, "gemm_mid_multi: %d matrices, 1 to 3", matrices);
+  return mid_go("gemm_mid_multi", x, W, nullptr, y, N, matrices, M, K, x_stride, ldw, y_stride, 0, workspace, workspace_bytes, stream);
 }

@@ -25,6 +25,7 @@ namespace {
 #define TV_NATIVE_SYMBOLS(X)                                                                                                                              \
   X(tv_rmsnorm_fwd) X(tv_layernorm_fwd) X(tv_rmsnorm_gated_fwd) X(tv_causal_conv1d_xbc_fwd) X(tv_causal_conv1d_xbc_cb_fwd) X(tv_ssd_cb_bytes)              \
   X(tv_ssd_scan_workspace_bytes) X(tv_ssd_scan_cb_fwd) X(tv_flash_attn_fwd) X(tv_gemm_mid_fwd) X(tv_gemm_mid_workspace_bytes) X(tv_gemm_split_fwd)          \
+  X(tv_gemm_mid_multi_fwd) X(tv_gemm_mid_multi_workspace_bytes)                                                                                        \
   X(tv_gemm_split_workspace_bytes) X(tv_gemm_split_add_fwd) X(tv_gemm_small_fwd) X(tv_gemm_rows_fwd) X(tv_residual_add_fwd)            \
   X(tv_token_side_fwd) X(tv_norm_shift_fwd) X(tv_gated_mul_fwd) X(tv_scatter_rows) X(tv_flash_attn_window_packed_fwd) X(tv_last_error)
 struct Lib {
@@ -266,6 +267,41 @@ PyObject* mid_linear(PyObject* const* a) {
                              bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
   return wrap(std::move(p.y));
 }
+// mid_linears(x, weight, weight, weight): the shapes are kernels.mid_linears_take's
+PyObject* mid_linears(PyObject* const* a) {
+  Operands op;
+  const T x = op.get(a[0]);
+  need(bf16(x) && x->dim() > 0 && x->is_contiguous() && aligned(x, 16));
+  const int64_t K = x->size(-1), M = K > 0 ? x->numel() / K : 0;
+  need(M >= 2 && M <= TV_GEMM_MID_MAX && K >= 4096 && K % 64 == 0 && K < (1 << 22));
+  const void* W[3];
+  void* Y[3];
+  int N[3];
+  int64_t ldw[3], ldy[3], all = 0;
+  at::Tensor y[3];
+  for (int i = 0; i < 3; ++i) {
+    const T w = op.get(a[1 + i]);
+    need(bf16(w) && w->dim() == 2 && w->size(1) == K && w->size(0) > 0 && w->size(0) % 4 == 0 && w->size(0) < (1 << 28) && w->stride(1) == 1 && w->stride(0) % 8 == 0 &&
+         w->stride(0) >= K && w->stride(0) < (1 << 22) && aligned(w, 16));
+    W[i] = ptr(w);
+    N[i] = (int)w->size(0);
+    ldw[i] = w->stride(0);
+    ldy[i] = N[i];
+    all += N[i];
+  }
+  need(all >= 4096);
+  c10::SmallVector<int64_t, 5> sizes(x->sizes().begin(), x->sizes().end());
+  for (int i = 0; i < 3; ++i) {
+    sizes.back() = N[i];
+    y[i] = like(x, sizes);
+    Y[i] = y[i].data_ptr();
+  }
+  const size_t bytes = lib.tv_gemm_mid_multi_workspace_bytes((int)M, N, 3, (int)K);
+  at::Tensor ws;
+  if (bytes) ws = like(x, {(int64_t)bytes}, at::kByte);
+  launch(tv_gemm_mid_multi_fwd, ptr(x), W, Y, N, 3, (int)M, (int)K, K, ldw, ldy, bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
+  return tuple(wrap(std::move(y[0])), wrap(std::move(y[1])), wrap(std::move(y[2])));
+}
 // split_linear(x, weight, bias, relu2, splits, full)
 PyObject* split_linear(PyObject* const* a) {
   Operands op;
@@ -469,7 +505,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 }
 
 #define ENTRY(name, n) {#name, (PyCFunction)(void*)(entry<name, n>), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {ENTRY(rms_norm, 5), ENTRY(layer_norm, 6), ENTRY(gated_norm, 5), ENTRY(conv_xbc, 8), ENTRY(scan, 15), ENTRY(flash, 6), ENTRY(mid_linear, 4),
+PyMethodDef methods[] = {ENTRY(rms_norm, 5), ENTRY(layer_norm, 6), ENTRY(gated_norm, 5), ENTRY(conv_xbc, 8), ENTRY(scan, 15), ENTRY(flash, 6), ENTRY(mid_linear, 4), ENTRY(mid_linears, 4),
                          ENTRY(split_linear, 6), ENTRY(rows_linear, 4), ENTRY(small_linear, 6), ENTRY(residual_add, 2), ENTRY(split_add_linear, 5), ENTRY(token_side, 5), ENTRY(norm_shift, 15),
                          ENTRY(gated_mul, 5), ENTRY(scatter_rows, 3), ENTRY(attention_window, 16),
                          {"bind", (PyCFunction)bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};

@@ -1049,6 +1049,39 @@ def mid_linear(x, weight, bias=None, relu2=False):
     return y
 
 
+def mid_linears_take(x, weights) -> bool:
+    """Whether `mid_linears` is there for these matrices and faster than one product after the other: the three projections of an attention layer for a short
+    prompt's rows ((5 120, 1 024, 1 024) x 4 480, us, a launch each (up to 32 rows tv_gemm_rows_fwd, the library) | one: 2 rows 21 | 17, 24: 29 | 18, 64: 64 | 21, 128: 66 | 27, 203: 65 | 32,
+    256: 82 | 34; (2 048, 2 048, 2 048) x 4 096, 16 rows 21 | 16, 100: 38 | 24, 256: 47 | 30)."""
+    Kd = x.shape[-1]
+    n = x.numel() // max(Kd, 1)
+    return (2 <= n <= MID_MAX and Kd >= 4096 and Kd % 64 == 0 and x.is_cuda and x.dtype == torch.bfloat16 and 2 <= len(weights) <= 3
+            and sum([w.shape[0] for w in weights]) >= 4096
+            and all([w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == Kd and w.shape[0] % 4 == 0 and w.shape[0] > 0 and w.stride(1) == 1
+                     and w.stride(0) % 8 == 0 and Kd <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights]))
+
+
+def mid_linears(x, weights):
+    """[x @ w.T for w in weights] for two or three matrices and up to 256 bf16 rows, in one launch (shapes: `mid_linears_take`)."""
+    if x.is_cuda and len(weights) == 3 and (r := _n.mid_linears(x, *weights)) is not None:
+        return r
+    _gpu(x, *weights)
+    if not mid_linears_take(x, weights):
+        raise TimeViperHipError(f"mid_linears: 2..{MID_MAX} bf16 rows against two or three matrices, got {tuple(x.shape)} against {[tuple(w.shape) for w in weights]}")
+    x2 = _rows2d(x)
+    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) >= (1 << 22) or x2.data_ptr() % 16:
+        x2 = x2.contiguous()
+    ys = [torch.empty(x.shape[:-1] + (w.shape[0],), dtype=x.dtype, device=x.device) for w in weights]
+    n, lib, M, Kd = len(weights), _capi.lib(), x2.shape[0], x2.shape[1]
+    ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+    N = (ctypes.c_int * n)(*[w.shape[0] for w in weights])
+    ldw, ldy = (ctypes.c_int64 * n)(*[w.stride(0) for w in weights]), (ctypes.c_int64 * n)(*N)
+    need = int(lib.tv_gemm_mid_multi_workspace_bytes(M, N, n, Kd))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib.tv_gemm_mid_multi_fwd(_p(x2), ptrs(weights), ptrs(ys), N, n, M, Kd, x2.stride(0), ldw, ldy, _p(ws), need, _stream()), "tv_gemm_mid_multi_fwd")
+    return ys
+
+
 def kv_append(k, v, k_cache, v_cache, pos) -> None:
     """k_cache[:, pos] = k[:, 0], v_cache[:, pos] = v[:, 0] for (B, 1, H, D) keys and values and an int64 position on the device (both
     caches' `index_copy_` in one launch)."""

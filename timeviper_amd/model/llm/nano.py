@@ -600,9 +600,10 @@ class NemotronHAttention(nn.Module):
             raise NotImplementedError("padding masks are not on the inference path (mask is None "
                                       "under flash_attention_2, reference :2208-2213)")
         bsz, q_len, _ = hidden_states.size()
-        q = _linear(self.q_proj, hidden_states).view(bsz, q_len, self.num_heads, self.head_dim)
-        k = _linear(self.k_proj, hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim)
-        v = _linear(self.v_proj, hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim)
+        q, k, v = self._qkv(hidden_states)
+        q = q.view(bsz, q_len, self.num_heads, self.head_dim)
+        k = k.view(bsz, q_len, self.num_key_value_heads, self.head_dim)
+        v = v.view(bsz, q_len, self.num_key_value_heads, self.head_dim)
         if past_key_value is not None:
             k, v = past_key_value.update(k, v, self.layer_idx)
         if past_key_value is not None and q_len == 1 and past_key_value.static_decode:
@@ -615,6 +616,15 @@ class NemotronHAttention(nn.Module):
         o = _linear(self.o_proj, o.reshape(bsz, q_len, self.num_heads * self.head_dim))
         return o, None, past_key_value
 
+
+    def _qkv(self, x):
+        """q, k and v of x: a short prompt's rows meet the three matrices in one launch (modules with anything around them are called)"""
+        mods = (self.q_proj, self.k_proj, self.v_proj)
+        if x.dim() == 3 and x.shape[1] > 1 and x.shape[0] * x.shape[1] <= K.MID_MAX and not torch.is_grad_enabled() and all([plain_linear(m, x) and m.bias is None for m in mods]):
+            weights = [m.weight for m in mods]
+            if K.mid_linears_take(x, weights):
+                return K.mid_linears(x, weights)
+        return [_linear(m, x) for m in mods]
 
     def _qkv_weight(self):
         """[q; k; v] as one (N, K) matrix for the decode token's single product (a copy: 64 MB per layer at 9B dims), rebuilt
