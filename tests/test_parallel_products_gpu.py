@@ -74,6 +74,20 @@ def test_refused():
 
 
 # both sides of each line
+# few rows: several work-groups a block of rows, each with a share of the outputs (8, 6 that become 4, 2, one; a width of fewer, and of uneven, turns)
+@pytest.mark.parametrize("D", [32, 288, 2048, 2080])
+def test_token_side_shares(D):
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(D)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    T = 6200
+    h, table, gate, proj = r(T, D).bfloat16(), r(500, 128).bfloat16(), (r(128, D) * D ** -0.5).bfloat16(), (r(D, 128) * 128 ** -0.5).bfloat16()
+    ids = torch.randint(0, 500, (T,), generator=g, device=DEV)
+    whole = ops.token_side(h, ids, table, gate, proj)
+    for n in (1, 31, 33, 700, 1000, 1600, 2900, 3100):
+        assert torch.equal(ops.token_side(h[:n], ids[:n], table, gate, proj), whole[:n])      # a row's sums do not depend on the others
+
+
 @pytest.mark.parametrize("rows,glu,add", [(255, False, 16), (512, False, 16), (700, True, 10), (1300, False, 5), (1800, True, 4), (4096, True, 2), (6011, True, 0)])
 def test_rules(rows, glu, add):
     from timeviper_amd import kernels as ops

@@ -7,11 +7,11 @@
 //     own, is read into registers, and the next one is asked for in front of its products.  The partial sums meet in LDS.
 //   * z = gelu_tanh(bf16(G h)) * e, rounded (what the separate launches write), stays in LDS.
 //   * P z: a wave takes 32 outputs at a time (8 KB of P, two stages by LDS-DMA), whose rows are dealt to two tiles so that a lane holds eight neighbouring outputs:
-//     16-byte stores.
+//     16-byte stores.  With few rows several work-groups form the same z, each for a share of the outputs.
 // G and P (1 MB) come from L2, read once a work-group: their latency and the way into the compute unit are what 32 rows take, so that the time hardly depends
 // on the rows up to one round of work-groups (8 192 rows).  Loads straight into the matrix cores' layout, where neighbouring lanes are 16 different rows, took
 // them in at 26 bytes a ns (a 16-byte access a lane): 46 us.
-// Measured (2 048 wide; three launches -> here): 6 011 rows 40 -> 25 us on the device, 40 rows 17; with the callers' host work, 40 to 1 000 rows 50 -> 23.
+// Measured (2 048 wide; three launches -> here): 6 011 rows 40 -> 25 us on the device, 300 rows in one share 24.7, now 14.9; with the callers' host work, 40 to 1 000 rows 50 -> 23.
 #include "gemm_skinny.hpp"
 
 namespace {
@@ -138,11 +138,12 @@ __global__ __launch_bounds__(TS_WAVES * 64) void token_side_kernel(SideArgs a) {
     glds_rows<4, false>(src, vp[0], pring + (unsigned)(S * PAIR));
     glds_rows<4, false>(src, vp[1], pring + (unsigned)(S * PAIR + 4096));
   };
-  copy_p(wave, 0);
-  copy_p(wave + TS_WAVES, 1);
+  const int first = wave + TS_WAVES * (int)blockIdx.y, step = TS_WAVES * (int)gridDim.y;
+  copy_p(first, 0);
+  copy_p(first + step, 1);
   const unsigned pfrag = (unsigned)((8 * (n >> 2) + (n & 3)) * 256);
   int S = 0;
-  for (int j = wave; j < npair; j += TS_WAVES, S ^= 1) {
+  for (int j = first; j < npair; j += step, S ^= 1) {
     asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                   // (the younger stage stays in flight; stores among it make the wait stricter)
     bf16x8 pf[2][KS];
 #pragma unroll
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(TS_WAVES * 64) void token_side_kernel(SideArgs a) {
         pf[half][ks] = *(lds_bf16x8*)(size_t)(pring + (unsigned)(S * PAIR + 1024 * half) + pfrag + (unsigned)(((4 * ks + kq) ^ n) << 4));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    copy_p(j + 2 * TS_WAVES, S);
+    copy_p(j + 2 * step, S);
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       f32x4 o[2];
@@ -193,6 +194,13 @@ extern "C" int tv_token_side_fwd(const void* h, const int64_t* ids, const void* 
     tv_set_error("token_side: cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr));
     return TV_ERR_LAUNCH;
   }
-  token_side_kernel<<<dim3((unsigned)((rows + TS_ROWS - 1) / TS_ROWS)), TS_WAVES * 64, LDS, (hipStream_t)stream>>>(a);
+  // Work-groups a block of rows, each with a share of the outputs, where that keeps within three quarters of the compute units (2 048 wide, us by shares 1 | 2 | 4 | 8: 300 rows
+  // 24.7 19.3 16.2 14.9, 1 000, 8 of which are a work-group on every unit, 22.9 18.1 16.0 17.9, 1 500 22.7 18.7 18.5 31.9, 4 100 24.5 35.4): as many as shorten the longest share
+  const int64_t blocks = (rows + TS_ROWS - 1) / TS_ROWS, turns = (width + 32 * TS_WAVES - 1) / (32 * TS_WAVES);
+  int64_t shares = tv_cu_count() * 3 / 4 / blocks;
+  shares = shares > 8 ? 8 : shares < 1 ? 1 : shares;
+  const int64_t longest = (turns + shares - 1) / shares;
+  shares = (turns + longest - 1) / longest;
+  token_side_kernel<<<dim3((unsigned)blocks, (unsigned)shares), TS_WAVES * 64, LDS, (hipStream_t)stream>>>(a);
   TV_LAUNCH_CHECK();
 }
