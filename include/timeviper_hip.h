@@ -647,6 +647,11 @@ int tv_gemm_glu_fwd(const void* A, const void* W, const void* bias, void* C, int
  * 64 x 64 (half as many outputs with epilogue 5); 2 and 3 give way to the next larger tile where they are more than a round of the compute units and it is not.  K % 64 == 0, N % 8 == 0, everything 16-byte aligned. */
 int tv_gemm_small_fwd(const void* A, const void* W, const void* bias, void* C, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                       int epilogue, int bias_dtype, int tile, void* stream);
+/* residual_out = residual + A W^T + bias in fp32 and C, its bf16 copy, dense rows of N; bias bf16 or NULL.  The contraction of a tile (0: 128 x 128, 2: 64 x 128, 3: 64 x 64) is split
+ * over 1 to 64 work-groups; workspace: tv_gemm_small_add_workspace_bytes, 16-byte aligned, not shared by launches that may run at once. */
+size_t tv_gemm_small_add_workspace_bytes(int64_t M, int N, int splits);
+int tv_gemm_small_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N, int K,
+                          int64_t lda, int64_t ldw, int tile, int splits, void* workspace, size_t workspace_bytes, void* stream);
 
 /* y = P (gelu_tanh(G h) * e), e the table's row of each token (csrc/token_side.hip): h (rows, width) bf16, G (dim, width), P (width, dim), table (table_rows,
  * dim) with a row stride of its own; ids outside the table count as rows of zeros.  width % 32 == 0, dim 128. */

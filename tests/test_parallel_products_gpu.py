@@ -41,6 +41,35 @@ def test_onto_the_stream(M, N, K, splits):
     assert torch.equal(h, got.to(BF))
 
 
+# small tiles with a split contraction: edges of the three tiles, uneven splits, a step a split, more splits than one pass of the sum; slices, no bias
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 4096), (63, 1032, 4160), (65, 2048, 7680), (130, 1536, 5632), (300, 1032, 4224)])
+@pytest.mark.parametrize("tile,splits", [(0, 3), (2, 1), (2, 11), (3, 8), (3, 64)])
+def test_small_add(M, N, K, tile, splits):
+    from timeviper_amd import kernels as ops
+    r = rand(M + N)
+    x, w, b, res = r(M, K + 8).to(BF)[:, :K], (K ** -0.5 * r(N, K + 8)).to(BF)[:, 8:], r(N).to(BF) if tile else None, r(M, N)
+    got, h = ops.small_add_linear(x, w, res, b, tile, splits)
+    want = res.double() + x.double() @ w.double().T + (0 if b is None else b.double())
+    # fp32 sums (relative 2^-24 an addition, of the sum of magnitudes)
+    assert ((got.double() - want).abs() <= (x.double().abs() @ w.double().abs().T + want.abs() + 4) * K * 2.0 ** -24).all()
+    assert torch.equal(h, got.to(BF)) and torch.equal(got, ops.small_add_linear(x, w, res, b, tile, splits)[0])
+
+
+def test_small_add_plan():
+    from timeviper_amd import kernels as ops
+    for rows, n, k, want in ((17, 2048, 7680, True), (1024, 2048, 7680, True), (1025, 2048, 7680, False), (2048, 1024, 5120, True), (300, 3072, 11264, False), (300, 2048, 2048, False)):
+        plan = ops.small_add_plan(rows, n, k)
+        assert (plan is not None) == want
+        if plan:
+            tm, tn = {0: (128, 128), 2: (64, 128), 3: (64, 64)}[plan[0]]
+            assert -(-rows // tm) * -(-n // tn) * plan[1] <= ops.CUS and k // 64 >= plan[1]
+    z = lambda *s: torch.zeros(s, device=DEV, dtype=BF)
+    for bad in ((z(4, 4096), z(1028, 4096)), (z(4, 4104), z(1024, 4104))):      # outputs no multiple of 8, contraction none of 64
+        assert ops.small_add_takes(*bad) is None
+        with pytest.raises(ops.TimeViperHipError):
+            ops.small_add_linear(*bad, torch.zeros(4, bad[1].shape[0], device=DEV))
+
+
 # tiles of 32 rows, units of 32 columns: fewer than the eight waves, no multiple of them; ids on both ends of the table, a slice of a wider one
 @pytest.mark.parametrize("T,D", [(1, 32), (31, 96), (33, 288), (64, 2048), (515, 2080)])
 def test_token_side(T, D):

@@ -50,6 +50,8 @@ SIGNATURES = {
     "tv_gemm_split_add_fwd": (_i, [_p] * 6 + [_l, _i, _i, _l, _l, _i, _i, _i, _p, _z, _p]),
     "tv_gemm_glu_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _p]),
     "tv_token_side_fwd": (_i, [_p] * 6 + [_l, _i, _i] + [_l] * 6 + [_p]),
+    "tv_gemm_small_add_workspace_bytes": (_z, [_l, _i, _i]),
+    "tv_gemm_small_add_fwd": (_i, [_p] * 6 + [_l, _i, _i, _l, _l, _i, _i, _p, _z, _p]),
     "tv_gemm_small_fwd": (_i, [_p] * 4 + [_l, _i, _i, _l, _l, _l, _i, _i, _i, _p]),
     "tv_gemm_set_persist": (None, [_i, _i]),
     "tv_gemm_persist_on": (_i, []),

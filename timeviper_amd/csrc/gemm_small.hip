@@ -13,6 +13,8 @@
 //     once, a line a lane.  Weights out of cache, 2 916 x 1 152 x 4 352: 41.6 -> 34.1, 1 458: 32.8 -> 26.2, 729 20.3 -> 17.9; 729 x 3 456 x 1 152 14.7 -> 14.0; in a cache .5 - 1 us more.
 //   * Two stages (64 KB): two work-groups a compute unit, for tiles between one round and two (5 120 x 2 048, 1 024 rows: 30.3 us, four stages in two rounds 31.6).
 //   * v_mfma_f32_16x16x32_bf16 with W on the A side: two tiles of rows joined by v_permlane16_swap are 16-byte stores, as gemm.hip;
+//   * EPI_PART: work-groups share a tile's contraction, their sums meet in a second launch that adds the bias and the residual stream (2 048 x 7 680, us, 256 x 256 tiles in 16 shares ->
+//     here: 64 rows 22.5 -> 17.3, 256: 32.8 -> 23.0, 512: 39.2 -> 31.3; 1 024 x 5 120, 256 rows: 27.7 -> 13.9, the library's product and its pass 15.4): fewer sums go through memory.
 //   * EPI_GLU: half of a tile's rows of W are those of the gate, half those of the factor N rows further down: a lane holds both of an output.
 // fp32 sums, one rounding; the GELU is that of the rounded sum (what the library's product would have written).
 // Measured (us on the device, weights out of cache, library | four waves before -> here): 729 x 3 456 x 1 152 17.9 | 15.0 -> 14.0, 729 x 1 152 x 1 152 12.5 | 9.1 -> 8.0, 729 x 1 152 x 4 352
@@ -26,6 +28,7 @@ namespace {
 typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
 
 constexpr int GS_THREADS = 512, TOUCH = 4;       // TOUCH: lines of W a thread asks for at most
+constexpr int EPI_PART = 6;                      // fp32 sums of a split of the contraction, to a.part [split][M][N]
 
 // WM, WN: a wave's 16-row tiles of A and of W
 template <int WM, int WN, int NS, int EPI>
@@ -38,10 +41,14 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
   const int wr = (wave & 3) >> 1, wc = wave & 1, kg = wave >> 2, lc = lane & 15, kq = lane >> 4;
 
   // ---- tile: ids of an XCD (id % 8) walk neighbouring tiles, bands of group_m tiles of rows
-  int id = blockIdx.x;
+  int id = blockIdx.x, split = 0;
   {
-    const int nt = a.tiles_m * a.tiles_n, q = nt / 8, r = nt % 8, x = id % 8;
+    const int nt = a.tiles_m * a.tiles_n * (EPI == EPI_PART ? a.splits : 1), q = nt / 8, r = nt % 8, x = id % 8;
     id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + id / 8;
+  }
+  if constexpr (EPI == EPI_PART) {                         // (the splits one after the other: neighbours share columns of both operands)
+    split = __builtin_amdgcn_readfirstlane(id / (a.tiles_m * a.tiles_n));
+    id -= split * (a.tiles_m * a.tiles_n);
   }
   const int band = id / (a.group_m * a.tiles_n), in_band = id % (a.group_m * a.tiles_n), rows_in_band = min(a.group_m, a.tiles_m - band * a.group_m);
   const int m0 = (band * a.group_m + in_band % rows_in_band) * TM, n0 = in_band / rows_in_band * TO;
@@ -62,7 +69,12 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
     src[i] = (const bf16_t*)uniform_ptr(isA ? a.A + (int64_t)m0 * a.lda : a.W + (int64_t)n0 * a.ldw);
     off[i] = (unsigned)((r * (isA ? a.lda : a.ldw) + ch * 8) * 2);
   }
-  const int nkt = a.K / BK;
+  const int all_kt = a.K / BK, kt0 = EPI == EPI_PART ? (int)((int64_t)all_kt * split / a.splits) : 0;
+  const int nkt = EPI == EPI_PART ? (int)((int64_t)all_kt * (split + 1) / a.splits) - kt0 : all_kt;
+  if constexpr (EPI == EPI_PART) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) src[i] = (const bf16_t*)uniform_ptr(src[i] + (int64_t)kt0 * BK);
+  }
   auto issue = [&](int t, int S) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < PW; ++i) glds16(uniform_ptr(src[i] + t * BK), off[i], lds0 + (unsigned)(S * STAGE + (wave * PW + i) * 1024));
@@ -85,11 +97,11 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
   // W on its way from memory, in order, a line a lane, by all work-groups together (the last line again where there is no other)
   float seen[TOUCH];
   {
-    const int64_t all = (int64_t)gridDim.x * GS_THREADS, pieces = (int64_t)(GLU ? 2 : 1) * a.N * nkt, most = pieces < 0x7fffffff ? pieces : 0x7fffffff;
+    const int64_t all = (int64_t)gridDim.x * GS_THREADS, pieces = (int64_t)(GLU ? 2 : 1) * a.N * all_kt, most = pieces < 0x7fffffff ? pieces : 0x7fffffff;
 #pragma unroll
     for (int i = 0; i < TOUCH; ++i) {
-      const int p = (int)min((int64_t)blockIdx.x * GS_THREADS + tid + i * all, most - 1), row = p / nkt;
-      seen[i] = *(const float*)(a.W + (int64_t)row * a.ldw + (p - row * nkt) * BK);
+      const int p = (int)min((int64_t)blockIdx.x * GS_THREADS + tid + i * all, most - 1), row = p / all_kt;
+      seen[i] = *(const float*)(a.W + (int64_t)row * a.ldw + (p - row * all_kt) * BK);
     }
   }
   bf16x8 af[2][WM], wf[2][WN];                             // by the parity of the stage
@@ -212,7 +224,7 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
   for (int n = 0; n < NO; ++n) {
     const int col = n0 + 16 * (wc * NO + n) + 8 * (kq >> 1);
     float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, bu[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (EPI != EPI_ACCUM && a.bias && col < a.N) {         // (N is a multiple of 8)
+    if (EPI != EPI_ACCUM && EPI != EPI_PART && a.bias && col < a.N) {         // (N is a multiple of 8)
       if (a.bias_f32) {
         const f32x4 b0 = *(const f32x4*)((const float*)a.bias + col), b1 = *(const f32x4*)((const float*)a.bias + col + 4);
 #pragma unroll
@@ -244,6 +256,12 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
       }
       const int row = m0 + 16 * (mk + mp + (kq & 1)) + lc;
       if (row >= a.M || col >= a.N) continue;
+      if constexpr (EPI == EPI_PART) {
+        float* pp = a.part + ((int64_t)split * a.M + row) * a.N + col;
+        *(f32x4*)pp = f32x4{v[0], v[1], v[2], v[3]};
+        *(f32x4*)(pp + 4) = f32x4{v[4], v[5], v[6], v[7]};
+        continue;
+      }
       bf16_t* cp = a.C + (int64_t)row * a.ldc + col;
       if (EPI == EPI_ACCUM) {
         const bf16x8 c8 = *(const bf16x8*)cp;
@@ -265,6 +283,34 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
   }
 }
 
+// res_out = res + (sum of the splits, in their order, + bias), C its bf16 copy; four neighbouring outputs a thread
+__global__ __launch_bounds__(256) void gemm_small_sum_kernel(GemmArgs a) {
+  const int64_t all = (int64_t)a.M * a.N, at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (at >= all) return;
+  const f32x4 r = *(const f32x4*)(a.res + at);
+  const int col = (int)(at % a.N);
+  bf16x4 b = {};
+  if (a.bias) b = *(const bf16x4*)((const bf16_t*)a.bias + col);
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < a.splits; j += 8) {                  // (a split that is not there repeats the last one and is not added)
+    f32x4 t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = *(const f32x4*)(a.part + min(j + u, a.splits - 1) * all + at);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (j + u < a.splits) s += t[u];
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (a.bias) s[j] += (float)b[j];
+    s[j] += r[j];
+    o[j] = (bf16_t)s[j];
+  }
+  *(f32x4*)(a.res_out + at) = s;
+  *(bf16x4*)(a.C + at) = o;
+}
+
 template <int WM, int WN, int NS, int EPI>
 int go_epi(GemmArgs& a, hipStream_t st) {
   constexpr int TM = 32 * WM, TO = EPI == EPI_GLU ? 16 * WN : 32 * WN, LDS = NS * (TM + 32 * WN) * 128;
@@ -276,7 +322,7 @@ int go_epi(GemmArgs& a, hipStream_t st) {
   a.tiles_m = (a.M + TM - 1) / TM;
   a.tiles_n = (a.N + TO - 1) / TO;
   a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
-  gemm_small_kernel<WM, WN, NS, EPI><<<dim3((unsigned)(a.tiles_m * a.tiles_n)), GS_THREADS, LDS, st>>>(a);
+  gemm_small_kernel<WM, WN, NS, EPI><<<dim3((unsigned)(a.tiles_m * a.tiles_n * (EPI == EPI_PART ? a.splits : 1))), GS_THREADS, LDS, st>>>(a);
   TV_LAUNCH_CHECK();
 }
 template <int WM, int WN, int NS>
@@ -323,4 +369,34 @@ extern "C" int tv_gemm_small_fwd(const void* A, const void* W, const void* bias,
     case 2: return go<2, 4, 4>(a, epilogue, st);
     default: return go<2, 2, 4>(a, epilogue, st);
   }
+}
+
+extern "C" size_t tv_gemm_small_add_workspace_bytes(int64_t M, int N, int splits) {
+  return M > 0 && N > 0 && splits > 0 ? (size_t)splits * M * N * sizeof(float) : 0;
+}
+
+// Long contractions into few outputs, a few hundred rows: the contraction of each tile is split over work-groups, a second launch adds the splits, the bias and the residual stream.
+extern "C" int tv_gemm_small_add_fwd(const void* A, const void* W, const void* bias, const float* residual, float* residual_out, void* C, int64_t M, int N, int K,
+                                     int64_t lda, int64_t ldw, int tile, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace tvgemm;
+  TV_CHECK_ARG(A && W && C && residual && residual_out, "gemm_small_add: null pointer");
+  TV_CHECK_ARG(M > 0 && N > 0 && K > 0 && (tile == 0 || tile == 2 || tile == 3) && splits >= 1 && splits <= 64, "gemm_small_add: bad sizes (M %lld N %d K %d, tile %d, %d splits)",
+               (long long)M, N, K, tile, splits);
+  if (K % BK || K / BK < splits || N % 8 || lda % 8 || ldw % 8 || lda < 0 || ldw < 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) || ((uintptr_t)C & 7) || ((uintptr_t)bias & 7) ||
+      ((uintptr_t)residual & 15) || ((uintptr_t)residual_out & 15))
+    TV_UNSUPPORTED("gemm_small_add: K must be a multiple of %d and of a step a split at least, N of 8, rows 16-byte aligned (K %d N %d lda %lld ldw %lld)", BK, K, N, (long long)lda,
+                   (long long)ldw);
+  if (M > (1ll << 24) || 128 * lda * 2 >= (1ll << 31) || 128 * ldw * 2 >= (1ll << 31) || ((M + 63) / 64) * ((N + 63) / 64) * splits >= (1ll << 31) || M * N / 4 >= (1ll << 31))
+    TV_UNSUPPORTED("gemm_small_add: sizes beyond the 32-bit offsets of the copies");
+  const size_t need = tv_gemm_small_add_workspace_bytes(M, N, splits);
+  TV_CHECK_ARG(workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0, "gemm_small_add: workspace of %zu bytes needed", need);
+  GemmArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.bias = bias; a.C = (bf16_t*)C;
+  a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw;
+  a.part = (float*)workspace; a.splits = splits; a.res = residual; a.res_out = residual_out;
+  hipStream_t st = (hipStream_t)stream;
+  const int rc = tile == 0 ? go_epi<4, 4, 4, EPI_PART>(a, st) : tile == 2 ? go_epi<2, 4, 4, EPI_PART>(a, st) : go_epi<2, 2, 4, EPI_PART>(a, st);
+  if (rc != TV_OK) return rc;
+  gemm_small_sum_kernel<<<dim3((unsigned)((M * N / 4 + 255) / 256)), 256, 0, st>>>(a);
+  TV_LAUNCH_CHECK();
 }

@@ -25,7 +25,7 @@ namespace {
 #define TV_NATIVE_SYMBOLS(X)                                                                                                                              \
   X(tv_rmsnorm_fwd) X(tv_layernorm_fwd) X(tv_rmsnorm_gated_fwd) X(tv_causal_conv1d_xbc_fwd) X(tv_causal_conv1d_xbc_cb_fwd) X(tv_ssd_cb_bytes)              \
   X(tv_ssd_scan_workspace_bytes) X(tv_ssd_scan_cb_fwd) X(tv_flash_attn_fwd) X(tv_gemm_mid_fwd) X(tv_gemm_mid_workspace_bytes) X(tv_gemm_split_fwd)          \
-  X(tv_gemm_mid_multi_fwd) X(tv_gemm_mid_multi_workspace_bytes)                                                                                        \
+  X(tv_gemm_mid_multi_fwd) X(tv_gemm_mid_multi_workspace_bytes) X(tv_gemm_small_add_fwd) X(tv_gemm_small_add_workspace_bytes)                                                                                        \
   X(tv_gemm_split_workspace_bytes) X(tv_gemm_split_add_fwd) X(tv_gemm_small_fwd) X(tv_gemm_rows_fwd) X(tv_residual_add_fwd)            \
   X(tv_token_side_fwd) X(tv_norm_shift_fwd) X(tv_gated_mul_fwd) X(tv_scatter_rows) X(tv_flash_attn_window_packed_fwd) X(tv_last_error)
 struct Lib {
@@ -371,6 +371,22 @@ PyObject* split_add_linear(PyObject* const* a) {
                                    splits, 0, bytes ? ws.data_ptr() : nullptr, bytes, op.stream());
   return tuple(wrap(std::move(xo)), wrap(std::move(h)));
 }
+// small_add_linear(x, weight, residual, bias, tile, splits)
+PyObject* small_add_linear(PyObject* const* a) {
+  Operands op;
+  T x = op.get(a[0]), w = op.get(a[1]), r = op.get(a[2]), b = op.get(a[3], true);
+  need(bf16(x) && bf16(w) && x->dim() == 2 && w->dim() == 2 && x->size(1) == w->size(1) && x->stride(1) == 1 && w->stride(1) == 1);
+  const int64_t M = x->size(0), N = w->size(0);
+  need(M > 0 && N > 0 && r->scalar_type() == at::kFloat && r->dim() == 2 && r->size(0) == M && r->size(1) == N && r->is_contiguous());
+  need(b == nullptr || (bf16(b) && b->is_contiguous() && b->numel() == N));
+  const int tile = (int)integer(a[4]), splits = (int)integer(a[5]);
+  const size_t bytes = lib.tv_gemm_small_add_workspace_bytes(M, (int)N, splits);
+  need(bytes > 0);
+  at::Tensor xo = like(r, r->sizes()), h = like(x, r->sizes()), ws = like(x, {(int64_t)bytes}, at::kByte);
+  launch(tv_gemm_small_add_fwd, ptr(x), ptr(w), ptr(b), (const float*)ptr(r), (float*)xo.data_ptr(), h.data_ptr(), M, (int)N, (int)w->size(1), x->stride(0), w->stride(0), tile, splits,
+                                   ws.data_ptr(), bytes, op.stream());
+  return tuple(wrap(std::move(xo)), wrap(std::move(h)));
+}
 // token_side(h, ids, table, gate, proj)
 PyObject* token_side(PyObject* const* a) {
   Operands op;
@@ -506,7 +522,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 
 #define ENTRY(name, n) {#name, (PyCFunction)(void*)(entry<name, n>), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {ENTRY(rms_norm, 5), ENTRY(layer_norm, 6), ENTRY(gated_norm, 5), ENTRY(conv_xbc, 8), ENTRY(scan, 15), ENTRY(flash, 6), ENTRY(mid_linear, 4), ENTRY(mid_linears, 4),
-                         ENTRY(split_linear, 6), ENTRY(rows_linear, 4), ENTRY(small_linear, 6), ENTRY(residual_add, 2), ENTRY(split_add_linear, 5), ENTRY(token_side, 5), ENTRY(norm_shift, 15),
+                         ENTRY(split_linear, 6), ENTRY(rows_linear, 4), ENTRY(small_linear, 6), ENTRY(residual_add, 2), ENTRY(split_add_linear, 5), ENTRY(small_add_linear, 6), ENTRY(token_side, 5), ENTRY(norm_shift, 15),
                          ENTRY(gated_mul, 5), ENTRY(scatter_rows, 3), ENTRY(attention_window, 16),
                          {"bind", (PyCFunction)bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_tv_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

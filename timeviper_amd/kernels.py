@@ -18,6 +18,7 @@ eager fallback: tensors must live on the GPU and the HIP library must be built.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 from typing import Optional
@@ -1679,6 +1680,53 @@ def split_add_takes(x, weight, bias=None, waits: bool = True) -> int:
     if pays and not waits:
         pays = Kd >= 7168 and ((Kd > 768 * splits and rows * N * splits >= 0.65 * 65536 * CUS) or (splits == 16 and 64 <= rows <= 256 and Kd >= 704 * 16))
     return splits if pays and products_take(x, weight) and bias_takes(bias) else 0
+
+
+@functools.lru_cache(maxsize=1024)
+def small_add_plan(rows: int, n: int, k: int):
+    """(tile of `small_linear`, splits) on which tv_gemm_small_add_fwd adds a product of long contraction and few outputs to the residual stream, None where
+    tv_gemm_split_add_fwd or the library is faster: weights of at most 2^24 entries, at least two splits of 128 x 128 tiles in one round of the compute units.
+    us, the library and the pass that adds | 256 x 256 tiles | here: 2 048 x 7 680: 64 rows 26 | 22 | 17, 256: 31 | 33 | 23, 300: 37 | 34 | 27, 512: 38 | 39 | 31, 900: 49 | 47 | 44, 1 100, one split,
+    69 | 53 | 62; 1 024 x 5 120: 100: 14 | 19 | 12, 512: 19 | 28 | 17, 2 000: 41 | 42 | 33; 1 536 x 5 632: 17: 11 | 16 | 12, 300: 23 | 28 | 18, 1 100: 43 | 40 | 34; 2 048 x 4 096: 40: 12 | 17 |
+    12, 256: 19 | 27 | 16; larger matrices, 3 072 x 11 264: 40: 31 | 27 | 27, 300: 52 | 46 | 49.
+    The choice is the least of an estimate in us (a step of 64 columns, more where more work-groups stream; a split's sums written and read), a fit to those sizes with 17
+    to 2 000 rows: .1 % slower in the mean than the best choice, 2.5 % at most."""
+    if n * k > 1 << 24 or k < 4096 or n < 1024 or -(-rows // 128) * -(-n // 128) * 2 > CUS:
+        return None
+    best = None
+    for tile, tm, tn, step, more in ((3, 64, 64, .166, .042), (2, 64, 128, .248, .074), (0, 128, 128, .334, .174)):
+        tiles = -(-rows // tm) * -(-n // tn)
+        for splits in range(1, min(8, CUS // tiles, k // 256) + 1):
+            t = -(-(k // 64) // splits) * (step + more * tiles * splits / CUS) + splits * (.195 + 1.38e-6 * rows * n)
+            if best is None or t < best[0]:
+                best = (t, tile, splits)
+    return best[1:] if best else None
+
+
+def small_add_takes(x, weight, bias=None):
+    """`small_add_plan` of x (rows, K) against weight, None where the operands are not what the kernel reads"""
+    plan = small_add_plan(x.shape[0], *weight.shape) if x.shape[0] > 0 else None
+    return plan if plan and weight.shape[0] % 8 == 0 and weight.shape[1] % 64 == 0 and products_take(x, weight) and bias_takes(bias) else None
+
+
+def small_add_linear(x, weight, residual, bias=None, tile=3, splits=1):
+    """(residual + x @ weight.T (+ bias) in fp32, its bf16 copy) on small tiles whose contraction is split (`small_add_plan`)"""
+    if x.is_cuda and (r := _n.small_add_linear(x, weight, residual, bias, tile, splits)) is not None:
+        return r
+    _gpu(x, weight, residual, bias)
+    N, Kd = weight.shape
+    if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.shape[1] != Kd or x.stride(1) != 1 or weight.stride(1) != 1 or residual.dtype != torch.float32
+            or residual.shape != (x.shape[0], N) or not residual.is_contiguous()):
+        raise TimeViperHipError(f"small_add_linear: {tuple(x.shape)} bf16 against {tuple(weight.shape)} onto {tuple(residual.shape)} fp32")
+    if bias is not None:
+        _bf16_bias(bias, N, "small_add_linear")
+    lib, M = _capi.lib(), x.shape[0]
+    res, h = torch.empty_like(residual), torch.empty((M, N), dtype=x.dtype, device=x.device)
+    need = int(lib.tv_gemm_small_add_workspace_bytes(M, N, splits))
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=x.device)
+    check(lib.tv_gemm_small_add_fwd(_p(x), _p(weight), _p(bias), _p(residual), _p(res), _p(h), M, N, Kd, x.stride(0), weight.stride(0), int(tile), int(splits),
+                                    _p(ws), need, _stream()), "tv_gemm_small_add_fwd")
+    return res, h
 
 
 def split_add_linear(x, weight, residual, bias=None, splits=1):
