@@ -126,3 +126,19 @@ def test_attention_takes_them(tokens, monkeypatch):
         att._qkv(x)
     handle.remove()
     assert not calls and seen
+
+
+@pytest.mark.parametrize("tokens,n,k,name", [(19, 15680, 4480, "rows_linear"), (20, 15680, 4480, "mid_linear"), (32, 4480, 10240, "mid_linear"), (32, 12288, 4096, "rows_linear"),
+                                             (32, 4480, 5120, "rows_linear")])
+def test_large_matrices_of_twenty_rows(tokens, n, k, name, monkeypatch):
+    from timeviper_amd import kernels as ops
+    from timeviper_amd.model.llm import nano
+    torch.manual_seed(n)
+    lin = torch.nn.Linear(k, n, bias=False, device=DEV, dtype=BF).requires_grad_(False)
+    x = torch.randn(1, tokens, k, device=DEV, dtype=BF)
+    calls, real = [], getattr(ops, name)
+    monkeypatch.setattr(ops, name, lambda *a, **kw: (calls.append(1), real(*a, **kw))[1])
+    with torch.no_grad():
+        got = nano._prompt_linear(lin, x)
+    want = F.linear(x.double(), lin.weight.double())
+    assert calls and (got.double() - want).abs().max() <= 1.05 * 2.0 ** -8 * want.abs().max()

@@ -862,6 +862,13 @@ def mid_takes(x, weight, relu2=False) -> bool:
             and weight.stride(0) < (1 << 22) and weight.data_ptr() % 16 == 0)
 
 
+def mid_before_rows(x, weight, relu2=False) -> bool:
+    """Up to 32 rows of a prompt that `mid_linear` runs faster than `rows_linear`, whose work-groups read x again for every 32 rows of a large matrix (us, rows_linear | mid_linear:
+    22 656 x 4 480: 16 rows 36.5 | 37.2, 20: 38.8 | 37.2, 32: 43.9 | 38.3; 15 680 x 4 480: 20: 27.7 | 27.5, 32: 30.9 | 28.3; 4 480 x 15 680: 16: 31.0 | 31.1, 32: 36.2 | 31.2; 4 480 x 10 240: 20:
+    23.8 | 22.6, 32: 26.4 | 23.5; not 4 480 x 5 120, 32: 15.0 | 16.4; 6 144 x 5 120: 17.1 | 18.6; 12 288 x 4 096: 23.3 | 28.2)."""
+    return x.numel() >= 20 * x.shape[-1] and weight.numel() >= 45_000_000 and weight.shape[-1] > 4096 and mid_takes(x, weight, relu2)
+
+
 def large_takes(x, weight, relu2=False) -> bool:
     """Products of a long prompt that the persistent GEMM (tv_gemm_bf16_fwd) runs faster than the library: its 256 x 256 tiles are two
     rounds of the compute units or more and fill them, and

@@ -340,7 +340,7 @@ def _prompt_linear(mod: nn.Linear, x: torch.Tensor, relu2: bool = False) -> torc
     those are faster than the library (`plain_linear`: a module with anything around it is called)."""
     if x.is_cuda and x.dim() == 3 and x.shape[1] > 1 and not torch.is_grad_enabled() and plain_linear(mod, x):
         rows, w = x.shape[0] * x.shape[1], mod.weight
-        if rows <= K.ROWS_MAX and K.rows_pay(x, w):
+        if rows <= K.ROWS_MAX and K.rows_pay(x, w) and not K.mid_before_rows(x, w, relu2):
             return K.rows_linear(x, w, mod.bias, relu2=relu2)
         if rows <= K.MID_MAX:
             if K.mid_takes(x, w, relu2):
