@@ -142,3 +142,9 @@ def test_large_matrices_of_twenty_rows(tokens, n, k, name, monkeypatch):
         got = nano._prompt_linear(lin, x)
     want = F.linear(x.double(), lin.weight.double())
     assert calls and (got.double() - want).abs().max() <= 1.05 * 2.0 ** -8 * want.abs().max()
+
+
+def test_wide_outputs_rule():
+    from timeviper_amd import kernels as ops
+    for rows, n, want in ((79, 22656, False), (80, 22656, True), (256, 16384, True), (200, 16380, False), (257, 22656, False)):
+        assert ops.mid_takes(torch.empty(1, rows, 4480, device=DEV, dtype=BF), torch.empty(n, 4480, device=DEV, dtype=BF)) is want
