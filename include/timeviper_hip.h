@@ -255,7 +255,7 @@ void tv_ssd_scan_set_impl(int impl);
 /* kernel family (same numbers) the most recent scan call of this process ran on; 0 before the first call */
 int tv_ssd_scan_last_impl(void);
 /* ... and the kernel: the same numbers, and three that automatic selection (0) takes by rules of its own: 9 = column slices (csrc/ssd_cols.hip) and 10 = a head per
- * work-group in segments (csrc/ssd_par.hip), both of family 6; 11 = chunks on the fp32 matrix instruction (csrc/ssd_f32.hip), of family 8.  A forced 6 is the
+ * work-group in segments (csrc/ssd_par.hip), both of family 6; 11 = chunks on the fp32 matrix instruction (csrc/ssd_f32.hip, csrc/ssd_f32_long.hip), of family 8.  A forced 6 is the
  * march at every length, a forced 8 csrc/ssd_chunked.hip; the workspace is asked for under the same force. */
 int tv_ssd_scan_last_kernel(void);
 /* Implementation 6 at head_dim 80 with 4 heads per work-group (the Nano-9B shape): 1 = the 64-token step as the

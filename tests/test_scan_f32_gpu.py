@@ -101,3 +101,37 @@ def test_work_groups_of_a_tile(B, L, H, P, group_map):
     rel = 2.0 ** -18 + 2.0 ** -21 * 16 * (d * A.double()).abs().mean(1).max().item()
     assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
     assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5, atol=1e-6)
+
+
+# two launches (csrc/ssd_f32_long.hip): each side of its lines in tiles (batch x heads x head_dim / 16) and chunks, partial chunks and a last segment of one, infinities
+@pytest.mark.parametrize("B,L,H,P,two", [(1, 1472, 8, 64, False), (1, 1473, 8, 64, True), (2, 3777, 8, 64, True), (2, 3776, 8, 64, False), (1, 4097, 20, 64, True), (1, 4097, 21, 64, False),
+                                         (1, 4128, 65, 64, True), (1, 4128, 85, 64, False), (1, 7700, 33, 64, True), (3, 2000, 1, 48, True), (1, 5000, 1, 16, True), (2, 1900, 512, 64, True)])
+def test_two_launches(B, L, H, P, two):
+    from timeviper_amd import _capi
+    from timeviper_amd import kernels as ops
+    G, n = 1 if H % 2 else 2, _capi.lib().tv_ssd_scan_workspace_bytes
+    # (beyond 4 096 tokens nothing else asks for more than a place to point to)
+    assert L <= 4096 or (n(B, L, H, P, G, 16, ops.TV_F32) > 256) == two
+    g = torch.Generator(device=DEV).manual_seed(L + H)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, Bm, Cm, dt, D, S0 = r(B, L, H, P), 0.3 * r(B, L, G, 16), r(B, L, G, 16), r(B, L, H), r(H), r(B, H, P, 16)
+    A = -torch.linspace(1e-3, 4, H, device=DEV)
+    call = lambda: ops.mamba_chunk_scan_combined(x, dt, A, Bm, Cm, D=D, dt_softplus=True, initial_states=S0, return_final_states=True, return_total_decay=True)
+    y, fin, dec = call()
+    assert ops.ssd_scan_last_kernel() == 11
+    d = F.softplus(dt.double())
+    if B * L * H * P < 1e7:
+        want, S, mag, Sm = reference(x.double(), d, A.double(), Bm.double(), Cm.double(), D.double(), S0.double(), torch.arange(H, device=DEV) // (H // G))
+        # (as above: exponents are differences of sums of at most 64 tokens)
+        rel = 2.0 ** -18 + 2.0 ** -21 * 64 * (d * A.double()).abs().mean(1).max().item()
+        assert ((y.double() - want).abs() <= mag * rel + 1e-9).all() and ((fin.double() - S).abs() <= Sm * rel + 1e-9).all()
+    else:
+        # heads do not depend on each other: the last four of them alone, on the other kernel
+        part = ops.mamba_chunk_scan_combined(x[:, :, -4:].contiguous(), dt[:, :, -4:].contiguous(), A[-4:], Bm[:, :, -1:].contiguous(), Cm[:, :, -1:].contiguous(), D=D[-4:], dt_softplus=True,
+                                             initial_states=S0[:, -4:].contiguous(), return_final_states=True)
+        assert (y[:, :, -4:] - part[0]).norm() <= 2e-6 * part[0].norm() and (fin[:, -4:] - part[1]).norm() <= 2e-6 * part[1].norm()
+    assert torch.allclose(dec.double(), (d * A.double()).sum(1), rtol=1e-5, atol=1e-6)
+    at = L // 2
+    x[0, at, H - 1, 3] = float("inf")
+    z, _, _ = call()
+    assert torch.isfinite(z[:, :at]).all() and torch.isfinite(z[..., :3]).all() and not torch.isfinite(z[0, at, H - 1, 3])

@@ -25,7 +25,7 @@ bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int
 int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias, const void* init_state,
                       void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups, int64_t xsb, int64_t xsl,
                       int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl,
-                      int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, hipStream_t st);
+                      int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, void* workspace, size_t workspace_bytes, hipStream_t st);
 
 namespace {
 
@@ -364,7 +364,8 @@ int tv_ssd_chunked_launch(const void* x, const void* dt, const void* A, const vo
       tv_ssd_f32_supported(headdim, dstate, xsb, xsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl, x, Bm, Cm, y, init_state, final_state)) {
     *ran = 11;
     return tv_ssd_f32_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups, xsb, xsl, dsb, dsl,
-                             bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, false, st);
+                             bsb, bsl, bsg, csb, csl, csg, ysb, ysl, dt_softplus, dt_min, dt_max, group_map, false, workspace,
+                             tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate), st);
   }
   ChArgs a;
   a.x = x; a.dt = dt; a.Bm = Bm; a.Cm = Cm;

@@ -14,48 +14,26 @@
 // waits for its code (unrolled, with the next chunk's loads in flight: 64 tokens 7.0 us, 4 096: 50); addresses that move by scalar additions (64-bit products a load: 48 us for 43).
 // Keeping all of a chunk's vectors in LDS for the last pass, not the steps alone, gives nothing (15.6 | 16.2 us at 1 024).
 // Measured (32 heads x 64, 2 groups; two launches with chunks of 64 tokens -> here): 64 tokens 8.7 -> 6.7 us, 256: 12.6 -> 9.0, 1 024: 21.1 -> 15.6, 2 x 1 024: 30.0 -> 21.1,
-// 4 096: 50 -> 43, 2 x 4 096: 87 -> 65, 8 192: 100 -> 82; 128 heads, 2 x 2 100: 159 -> 135.  Beyond the last-level cache its second reading of x shows: 30 000 tokens 374 -> 425, 128 heads x 128,
-// 4 096: 335 -> 361.  Error against 64 bits (exponents are differences of sums of 16 tokens, not of 64), fresh Mamba-2 layer, 1 024 tokens: y 2.5e-7 -> 1.1e-7, final state 1.0e-7 both.
-#include "ssd_common.hpp"
+// 4 096: 50 -> 43, 2 x 4 096: 87 -> 65, 8 192: 100 -> 82; 128 heads, 2 x 2 100: 159 -> 135.  Few heads and long sequences, or x beyond the last-level cache, which it reads twice: ssd_f32_long.hip
+// (two_launches).  Error against 64 bits (exponents are differences of sums of 16 tokens, not of 64), fresh Mamba-2 layer, 1 024 tokens: y 2.5e-7 -> 1.1e-7, final state 1.0e-7 both.
+#include "ssd_f32.hpp"
 
 namespace {
 using namespace ssdk;
 
-constexpr int FQ = 64, FN = 16;       // tokens a chunk (their steps are a wave's lanes), d_state
 constexpr int SEGS = 16;              // waves of a work-group at most
 constexpr int KEEP = 4;               // chunks whose steps stay in LDS between a wave's passes
 
-struct F3Args {
-  const float *x, *dt, *Bm, *Cm, *A, *D, *dt_bias, *init;
-  float *y, *final_state, *total_decay;
-  int L, H, P, G, hpg, nch;
-  int two, split, len0, len1, plen, npre;
-  int64_t xsb, xsl, dsb, dsl, bsb, bsl, bsg, csb, csl, csg, ysb, ysl;
-  int softplus, group_map;
-  float dt_min, dt_max;
-};
-
-__device__ __forceinline__ float rdlane(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-__device__ __forceinline__ float from_lane(float v, int l) { return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * l, __float_as_int(v))); }
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 // sums over a block of 16 lanes, from its first lane on or (BACK) from its last, the lane's own among them; `lost`: what their rounding lost (an infinite sum has lost nothing)
-template <int CTRL>
-__device__ __forceinline__ void scan_step(float& hi, float& lo) {
-  const float b = dpp_shift<CTRL, 0xf>(hi), bl = dpp_shift<CTRL, 0xf>(lo);
-  const float s = hi + b, bb = s - hi;
-  lo = (lo + bl) + ((hi - (s - bb)) + (b - bb));
-  hi = s;
-}
 template <bool FINE, bool BACK>
 __device__ __forceinline__ float block_sum(float v, float& lost) {
   constexpr int SH = BACK ? 0x100 : 0x110;      // row_shl, row_shr
   lost = 0.f;
   if constexpr (FINE) {
-    scan_step<SH + 1>(v, lost);
-    scan_step<SH + 2>(v, lost);
-    scan_step<SH + 4>(v, lost);
-    scan_step<SH + 8>(v, lost);
+    scan_step<SH + 1, 0xf>(v, lost);
+    scan_step<SH + 2, 0xf>(v, lost);
+    scan_step<SH + 4, 0xf>(v, lost);
+    scan_step<SH + 8, 0xf>(v, lost);
     lost = fabsf(v) < INFINITY ? lost : 0.f;
   } else {
     v += dpp_shift<SH + 1, 0xf>(v);
@@ -64,45 +42,6 @@ __device__ __forceinline__ float block_sum(float v, float& lost) {
     v += dpp_shift<SH + 8, 0xf>(v);
   }
   return v;
-}
-
-template <bool FINE> __device__ __forceinline__ float exp_of(float v) { return FINE ? expf(v) : __expf(v); }
-
-// A chunk token by token, as the recurrence has it (ssd_generic.hip): S, y of the wave's columns; d and da are of token `lane`.  Returns the sum of da.
-template <bool OUT>
-__device__ __forceinline__ float march(const F3Args& a, const float* xb, const float* Bb, const float* Cb, int t0, int tt, float d, float da, float Dh, int lc, int q, int b, int h,
-                                       int pt, f32x4& S) {
-  float sum = 0.f;
-#pragma unroll 1
-  for (int t1 = 0; t1 < tt; t1 += 4) {
-    float x[4];
-    f32x4 B[4], C[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t t = t0 + min(t1 + j, tt - 1);
-      x[j] = xb[t * a.xsl + lc];
-      B[j] = *(const f32x4*)(Bb + t * a.bsl + 4 * q);
-      if constexpr (OUT) C[j] = *(const f32x4*)(Cb + t * a.csl + 4 * q);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (t1 + j >= tt) break;
-      const float dat = rdlane(da, t1 + j), dec = expf(dat), xv = rdlane(d, t1 + j) * x[j];
-      float acc = 0.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        S[r] = fmaf(dec, S[r], xv * B[j][r]);
-        if constexpr (OUT) acc = fmaf(S[r], C[j][r], acc);
-      }
-      sum += dat;
-      if constexpr (OUT) {
-        acc += __shfl_xor(acc, 32, 64);
-        acc += __shfl_xor(acc, 16, 64);
-        if (q == 0) a.y[(int64_t)b * a.ysb + (int64_t)(t0 + t1 + j) * a.ysl + (int64_t)h * a.P + 16 * pt + lc] = fmaf(Dh, x[j], acc);
-      }
-    }
-  }
-  return sum;
 }
 
 // FINE: for the lengths that the token recurrence had before (48 - 64 tokens, more than 4 096), whose error and whose results at extreme steps are kept:
@@ -396,7 +335,42 @@ F3Plan plan(int batch, int nch, int nheads, int headdim) {
   return p;
 }
 
+// Whether two launches on longer segments (ssd_f32_long.hip) are the faster ones.  Timed (us, here | there) over 36 shapes of 8 to 6 144 column tiles (batch x heads x head_dim / 16) and
+// 128 to 40 000 tokens:
+//   * few tiles: 32 segments a tile at most leave the chip idle.  Up to 32 tiles from 24 chunks on (16 tiles, 1 024 tokens 13.9 | 14.8, 1 500: 18.4 | 17.7), up to 64 from 60 on (64:
+//     3 000 tokens 32.4 | 38.0, 4 096: 41.6 | 40.3), up to 80 beyond 64 chunks (80, 8 192: 84 | 79).
+//   * up to 4 096 tokens, where FINE costs there what it does not here, else only 1 792 to 2 559 tiles with more than 240 MB of x (2 048: 326 | 312, 4 096 tokens 677 | 617).
+//   * longer ones where x, read again by the second half of a tile's work-groups and by every segment, is not in the last-level cache any more; how many MB that takes depends on how the
+//     tiles fill their rounds.  128 tiles: 134 MB 161 | 195, 197 MB 316 | 299, 328 MB 583 | 501; 192: 101 MB 132 | 154, 201 MB 347 | 314; 256: 197 MB 267 | 291, 268 MB 420 | 406; 384: 147 MB
+//     208 | 209, 403 MB 765 | 594; 640: 492 MB 773 | 750; 1 024: 197 MB 230 - 259 | 247, 537 MB 710 - 824 | 700; 2 048: 537 MB 677 - 692 | 580; 3 072 and more, which read x once, never.
+//   * 129 to 159 tiles, half of a round that a second work-group a tile does not fit, from 120 chunks on (132: 6 000 tokens 84 | 87, 8 192: 113 | 108), 257 to 336, just over a round, from
+//     65 on (264: 6 000: 169 | 160).
+bool two_launches(int batch, int nch, int nheads, int headdim) {
+  const int64_t tiles = (int64_t)batch * nheads * (headdim / 16);
+  const double mb = 1e-6 * tiles * 16 * sizeof(float) * FQ * nch;
+  if (tiles <= 32) return nch >= 24;
+  if (tiles <= 64) return nch >= 60;
+  if (nch <= 64) return tiles >= 1792 && tiles < 2560 && mb > 240;
+  if (tiles <= 80) return true;
+  if (tiles > 128 && tiles < 160) return nch >= 120;
+  if (tiles > 256 && tiles <= 336) return true;
+  static constexpr int LINE[][2] = {{128, 140}, {255, 120}, {256, 240}, {415, 190}, {831, 400}, {1151, 210}, {1791, 380}, {2559, 150}};     // tiles up to, MB
+  for (const auto& l : LINE)
+    if (tiles <= l[0]) return mb > l[1];
+  return false;
+}
+
 }  // namespace
+
+size_t tv_ssd_f32_long_workspace_bytes(int batch, int nch, int nheads, int headdim);
+int tv_ssd_f32_long_launch(ssdk::F3Args a, int batch, void* workspace, hipStream_t st);
+
+// What the launch can use; with less it is one launch
+size_t tv_ssd_f32_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate) {
+  if (dstate != FN || headdim % 16 || batch <= 0 || seqlen <= 0 || nheads <= 0 || headdim <= 0) return 0;
+  const int nch = (seqlen + FQ - 1) / FQ;
+  return two_launches(batch, nch, nheads, headdim) ? tv_ssd_f32_long_workspace_bytes(batch, nch, nheads, headdim) : 0;
+}
 
 // called from ssd_chunked.hip and, beyond its lengths, from ssd_scan.hip: fp32 shapes whose rows are read and written in 16-byte pieces
 bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
@@ -413,18 +387,20 @@ bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int
 int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias,
                       const void* init_state, void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups,
                       int64_t xsb, int64_t xsl, int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg,
-                      int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, hipStream_t st) {
+                      int64_t ysb, int64_t ysl, int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, void* workspace, size_t workspace_bytes, hipStream_t st) {
   F3Args a;
   a.x = (const float*)x; a.dt = (const float*)dt; a.Bm = (const float*)Bm; a.Cm = (const float*)Cm; a.A = (const float*)A; a.D = (const float*)D;
   a.dt_bias = (const float*)dt_bias; a.init = (const float*)init_state; a.y = (float*)y; a.final_state = (float*)final_state;
   a.total_decay = (float*)total_decay;
   a.L = seqlen; a.H = nheads; a.P = headdim; a.G = ngroups; a.nch = (seqlen + FQ - 1) / FQ;
-  const F3Plan p = plan(batch, a.nch, nheads, headdim);
-  a.two = p.split < a.nch; a.split = p.split; a.len0 = p.len0; a.len1 = p.len1; a.plen = p.plen;
-  a.npre = (p.split + p.plen - 1) / p.plen;
   a.hpg = nheads / ngroups;
   a.xsb = xsb; a.xsl = xsl; a.dsb = dsb; a.dsl = dsl; a.bsb = bsb; a.bsl = bsl; a.bsg = bsg; a.csb = csb; a.csl = csl; a.csg = csg; a.ysb = ysb; a.ysl = ysl;
   a.softplus = dt_softplus; a.group_map = group_map; a.dt_min = dt_min; a.dt_max = dt_max;
+  if (two_launches(batch, a.nch, nheads, headdim) && workspace_bytes >= tv_ssd_f32_long_workspace_bytes(batch, a.nch, nheads, headdim))
+    return tv_ssd_f32_long_launch(a, batch, workspace, st);
+  const F3Plan p = plan(batch, a.nch, nheads, headdim);
+  a.two = p.split < a.nch; a.split = p.split; a.len0 = p.len0; a.len1 = p.len1; a.plen = p.plen;
+  a.npre = (p.split + p.plen - 1) / p.plen;
   const dim3 grid((unsigned)nheads, (unsigned)(headdim / 16), (unsigned)(a.two ? 2 * batch : batch)), threads((unsigned)(64 * p.waves));
   const unsigned lds = (unsigned)p.waves * (unsigned)((4 + KEEP) * FQ * sizeof(float) + 2 * 64 * sizeof(f32x4) + 2 * sizeof(float));
   static const hipError_t attr = [] {

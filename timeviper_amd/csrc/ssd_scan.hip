@@ -34,7 +34,8 @@ bool tv_ssd_f32_supported(int headdim, int dstate, int64_t xsb, int64_t xsl, int
 int tv_ssd_f32_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D, const void* dt_bias, const void* init_state,
                       void* y, void* final_state, void* total_decay, int batch, int seqlen, int nheads, int headdim, int ngroups, int64_t xsb, int64_t xsl,
                       int64_t dsb, int64_t dsl, int64_t bsb, int64_t bsl, int64_t bsg, int64_t csb, int64_t csl, int64_t csg, int64_t ysb, int64_t ysl,
-                      int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, hipStream_t st);
+                      int dt_softplus, float dt_min, float dt_max, int group_map, bool fine, void* workspace, size_t workspace_bytes, hipStream_t st);
+size_t tv_ssd_f32_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate);
 bool tv_ssd_chunked_supported(int seqlen, int headdim, int dstate);
 size_t tv_ssd_chunked_workspace_bytes(int batch, int seqlen, int nheads, int headdim, int dstate);
 int tv_ssd_chunked_launch(const void* x, const void* dt, const void* A, const void* Bm, const void* Cm, const void* D,
@@ -87,8 +88,10 @@ extern "C" size_t tv_ssd_scan_workspace_bytes(int batch, int seqlen, int nheads,
                                               int ngroups, int dstate, int dtype) {
   if (dtype != TV_BF16 || dstate != 128) {
     const size_t chunked = tv_ssd_chunked_workspace_bytes(batch, seqlen, nheads, headdim, dstate);
-    // (ssd_f32.hip needs none, but a caller that gives none asks for the recurrence)
-    return chunked == 0 && dtype == TV_F32 && dstate == 16 && seqlen > 64 ? 256 : (chunked + 255) / 256 * 256;
+    const size_t f32 = dtype == TV_F32 ? tv_ssd_f32_workspace_bytes(batch, seqlen, nheads, headdim, dstate) : 0;
+    const size_t m = chunked > f32 ? chunked : f32;
+    // (one launch of ssd_f32.hip needs none, but a caller that gives none asks for the recurrence)
+    return m == 0 && dtype == TV_F32 && dstate == 16 && seqlen > 64 ? 256 : (m + 255) / 256 * 256;
   }
   const size_t narrow = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 0);
   const size_t wide = tv_ssd_slice_workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, 1);
@@ -180,7 +183,7 @@ static int scan_impl(const void* x, const void* dt, const void* A, const void* B
     ran_on(8, 11);
     return tv_ssd_f32_launch(x, dt, A, Bm, Cm, D, dt_bias, init_state, y, final_state, total_decay, batch, seqlen, nheads, headdim, ngroups, x_stride_b, x_stride_l,
                              dt_stride_b, dt_stride_l, b_stride_b, b_stride_l, b_stride_g, c_stride_b, c_stride_l, c_stride_g, y_stride_b, y_stride_l, dt_softplus, dt_min,
-                             dt_max, group_map, true, st);
+                             dt_max, group_map, true, workspace, workspace_bytes, st);
   }
   if (forced == 8) TV_UNSUPPORTED("ssd_scan: chunk-parallel generic kernel forced but shape unsupported");
   ran_on(1, 1);
