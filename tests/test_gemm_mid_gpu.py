@@ -47,6 +47,17 @@ def test_split_and_whole_rows(M, N, K):
     assert ((got - want).abs() <= acc * (1 + 2.0 ** -8) + want.abs() * 2.0 ** -8 + 1e-30).all()
 
 
+# both sides of the lines between the loads of W: 96 rows, rows of W that start 16 KiB apart, 72 000 000 entries
+@pytest.mark.parametrize("M", [95, 96, 203])
+@pytest.mark.parametrize("N,K", [(1152, 8192), (1152, 8128), (8192, 8768), (8256, 8768)])
+def test_loads_of_split_rows(M, N, K):
+    """whole numbers: exact, whatever the order of the sums"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = (torch.randint(-3, 4, s, generator=g, device=DEV).to(BF) for s in ((M, K), (N, K)))
+    assert torch.equal(ops.mid_linear(x, w), (x.double() @ w.double().T).to(BF))
+
+
 @pytest.mark.parametrize("tokens", [2, 17, 48, 200, 256, 257])
 def test_layers_take_them(tokens, monkeypatch):
     """The hybrid stack's projections: the short-prompt products within a rounding of torch.nn.Linear; hooks and gradients keep the module."""

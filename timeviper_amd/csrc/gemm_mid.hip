@@ -8,9 +8,10 @@
 //   * One barrier a stage, in the middle of its products: the fragments of a 16-column step are read while the step before is multiplied
 //     (v_mfma_f32_32x32x16_bf16, W on the A side: a lane's registers are consecutive outputs of one row of x).
 //   * The waves along K meet over the rings, in an order that stores whole rows of y.
-//   * W past the caches (non-temporal) where a work-group reads its rows of W from end to end, or for 64 rows and less; split along K, with more rows, pieces of a row are asked for by
-//     work-groups that do not run in step, and plain loads are better (us, non-temporal | plain, 128 and 203 rows: 4 480 x 5 120 24.7 30.4 | 22.6 26.6, 4 480 x 10 240 33.9 38.6 | 32.1 36.6,
-//     7 168 x 4 480 28.5 33.1 | 26.1 30.3; unsplit, 22 656 x 4 480 52.1 59.7 | 53.8 61.2; 64 rows of 22 656 41.4 | 44.1).
+//   * W past the caches (non-temporal), but for split matrices of up to 144 MB with 96 rows or more: work-groups that do not run in step ask for pieces of a row there, and plain loads are
+//     better (nt_loads; us, best tiling each, non-temporal | plain, 203 rows: 4 480 x 5 120 29.1 | 27.9, 7 168 x 4 480 34.3 | 32.2, 4 480 x 10 240 39.0 | 37.9, 4 096 x 4 096, 160: 21.6 | 19.3; 65
+//     rows and 4 480 x 15 680 level).  They are not beyond that or with rows that start 16 KiB apart (256 rows: 8 192 x 28 672 124 | 144, 16 384 x 16 384 145 | 181; 203 of 8 192 x 8 192
+//     47.6 | 49.9), nor unsplit (22 656 x 4 480, 128 and 203 rows, 52.1 59.7 | 53.8 61.2; 64 rows 41.4 | 44.1).
 // What bounds it: up to 64 rows the stream of W.  With 256 rows a stage of 128 rows of W takes 1.1 us, .8 of them where all copies hit the same lines, .57 without copies, .74 without
 // fragment reads (copies dealt out between the products instead of in one burst change nothing); splits cost their sums' way through memory.
 // fp32 accumulation, one rounding of y.
@@ -322,13 +323,13 @@ struct GmPlan {
 };
 // The tile width and split of K with the smallest estimate, us: a stage is a part for the rows of x and one for the 32-row tiles of W, which grows with the work-groups that stream W at once;
 // each round of work-groups has its fill and epilogue, a launch its own; a split adds a second launch and 4 M N bytes written and read per split, and splits that start
-// whole multiples of 4 KiB apart in a row meet in memory (4 480 x 10 240, 96 rows, five of 2 048 columns 33.6, seven 30.1; rows a power of two apart meet there however they are split).
-// The numbers are a fit to 2 900 timings, 18 sizes of N and K (1 024 to 22 656) with 33 to 256 rows: over those its choice is .7 % slower in the mean than the best one, 10 % at most.  The
-// estimate before (W and x through the compute unit's memory pipe at 45 bytes a ns) split more: with the loads as they are now 1.06 times as slow in the mean
-// (2 048 x 7 680, 203 rows: 11 splits 25.4 us, 8 of narrower tiles 20.9; 5 120 x 2 048, 160 rows: 20.7, 17.5; 15 680 x 4 480, 96 rows: two splits 41.0, unsplit 35.4).
+// whole multiples of 4 KiB apart in a row meet in memory (4 480 x 10 240, 96 rows, five of 2 048 columns 33.6, seven 30.1; 16 384 x 8 192, 20 rows, two 64, unsplit 56).
+// The numbers are a fit to all tilings of 47 sizes (N 1 024 to 32 768, K 4 096 to 28 672) with 20 to 256 rows, nothing in a cache, plain loads where nt_loads has them: over those 564 its choice is
+// 1.0 % slower in the mean than the best one, 15 % at most, and 2.9 % faster than the estimate that took W and x through the compute unit's memory pipe at 45 bytes a ns, with its
+// non-temporal loads (8.7 % slower at most, 4 096 x 8 192, 128 rows; a fit to 18 sizes with plain loads in all splits: up to 16 %, 8 192 x 28 672, 256 rows 124 | 144).
 int tiles_of(int N, int ni) { return (N + 32 * ni - 1) / (32 * ni); }
 GmPlan plan(int M, const int* N, int matrices, int K) {
-  static constexpr double X[3] = {.046, .11, .35}, W[3] = {.061, .065, .056}, FILL[3] = {1.7, 2.2, .87};
+  static constexpr double X[3] = {.047, .095, .36}, W[3] = {.048, .04, .056}, FILL[3] = {2., 3., .9};
   const int c = M <= 64 ? 0 : M <= 128 ? 1 : 2;
   GmPlan best{4, 1, 2 << c};
   const int cus = tv_cu_count(), nst = K / GM_KC;
@@ -339,10 +340,10 @@ GmPlan plan(int M, const int* N, int matrices, int K) {
     for (int i = 0; i < matrices; ++i) tiles += tiles_of(N[i], ni);
     for (int s = 1; s <= 16 && (s == 1 || s * 8 <= nst); ++s) {
       const int64_t units = tiles * s, rounds = (units + cus - 1) / cus;
-      const double stage = X[c] + ni * (W[c] + .1 * (units < cus ? units : cus) / cus);
+      const double stage = X[c] + ni * (W[c] + .097 * (units < cus ? units : cus) / cus);
       double t = rounds * (FILL[c] + (nst + s - 1) / s * stage) + 3.7;
-      if (s > 1) t += .7 + s * (.15 + 1.56e-6 * outs * M);
-      if (s > 1 && K / s * 2 % 4096 == 0 && (K & (K - 1))) t *= 1.12;
+      if (s > 1) t += 1.4 + s * (.09 + 1.26e-6 * outs * M);
+      if (s > 1 && K / s * 2 % 4096 == 0) t *= 1.09;
       if (t < least) {
         least = t;
         best.ni = ni;
@@ -359,6 +360,8 @@ int launch_ni(const GmArgs& a, int xt, hipStream_t st) {
   if (xt == 4) return launch_one<NI, 2, 2, 4, 3, 28 / NI>(a, st);
   return launch_one<NI, 2, 4, 2, 3, 16 / NI>(a, st);
 }
+
+bool nt_loads(int M, int64_t N, int K, int splits) { return splits == 1 || M < 96 || K % 8192 == 0 || N * K > 72000000; }
 
 bool takes(const void* x, const void* W, int M, int N, int K, int64_t xs, int64_t ldw) {
   // (copies are 16 bytes a lane at 32-bit offsets from a work-group's first row; a stage is 64 columns; four outputs a store)
@@ -414,7 +417,7 @@ static int mid_go(const char* what, const void* x, const void* const* W, const v
   a.splits = p.splits;
   a.per_xcd = (a.tiles * a.splits + 7) / 8;
   a.part = p.splits > 1 ? (float*)workspace : nullptr;
-  a.nt = p.splits == 1 || M <= 64;
+  a.nt = nt_loads(M, all, K, p.splits);
   hipStream_t st = (hipStream_t)stream;
   switch (p.ni) {
     case 2: return launch_ni<2>(a, p.xt, st);
