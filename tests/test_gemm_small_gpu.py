@@ -52,6 +52,23 @@ def test_every_end_of_the_ring(stages, tile):
     assert torch.equal(out, want.to(BF))
 
 
+# W asked for ahead and not: both sides of each line in rows and columns
+@pytest.mark.parametrize("M,N,K,tile", [(191, 200, 3072, 3), (192, 200, 3072, 3), (193, 1032, 3136, 2), (320, 264, 3008, 0), (320, 264, 3072, 0), (191, 264, 1024, 1), (192, 264, 960, 1), (200, 264, 1024, 1),
+                                        (511, 136, 1088, 1), (513, 136, 1088, 1)])
+def test_weights_asked_for_ahead(M, N, K, tile):
+    """whole numbers: exact, whatever the order of the sums"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    r = lambda *s: torch.randint(-3, 4, s, generator=g, device=DEV).to(BF)
+    x, w = r(M, K), r(2 * N, K + 8)[:, :K]                     # (rows of W apart: the lines asked for are those of its rows)
+    want = x.double() @ w.double().T
+    assert torch.equal(ops.small_linear(x, w, tile=tile), want.to(BF))
+    f, u = want.split(N, 1)
+    got = ops.small_linear(x, w, torch.zeros(2 * N, device=DEV, dtype=BF), ops.GEMM_GLU, tile=tile).double()
+    glu = F.gelu(f, approximate="tanh") * u
+    assert ((got - glu).abs() <= 2.0 ** -8 * glu.abs() + 2e-5 * (f.abs() + 1) * (u.abs() + 1)).all()
+
+
 @pytest.mark.parametrize("M,N,tile", [(1024, 1152, 3), (960, 1088, 3), (729, 3456, 2), (1025, 2048, 2), (2048, 4096, 3)])
 def test_more_work_groups_than_a_round(M, N, tile):
     """a tile that gives way to the next larger one, and those that just do not"""

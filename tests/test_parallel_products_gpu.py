@@ -55,6 +55,20 @@ def test_small_add(M, N, K, tile, splits):
     assert torch.equal(h, got.to(BF)) and torch.equal(got, ops.small_add_linear(x, w, res, b, tile, splits)[0])
 
 
+# W asked for ahead and not
+@pytest.mark.parametrize("M", [287, 288])
+@pytest.mark.parametrize("tile,splits", [(0, 2), (2, 3), (3, 8)])
+def test_small_add_asks_ahead(M, tile, splits):
+    """whole numbers: exact, whatever the order of the sums"""
+    from timeviper_amd import kernels as ops
+    g = torch.Generator(device=DEV).manual_seed(M + splits)
+    r = lambda *s: torch.randint(-3, 4, s, generator=g, device=DEV)
+    x, w, res = r(M, 4160).to(BF), r(1032, 4160).to(BF), r(M, 1032).float()
+    got, h = ops.small_add_linear(x, w, res, None, tile, splits)
+    want = res.double() + x.double() @ w.double().T
+    assert torch.equal(got.double(), want) and torch.equal(h, want.to(BF))
+
+
 def test_small_add_plan():
     from timeviper_amd import kernels as ops
     for rows, n, k, want in ((17, 2048, 7680, True), (1024, 2048, 7680, True), (1025, 2048, 7680, False), (2048, 1024, 5120, True), (300, 3072, 11264, False), (300, 2048, 2048, False)):

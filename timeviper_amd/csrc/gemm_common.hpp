@@ -34,6 +34,7 @@ struct GemmArgs {
   int full, splits, relu2;       // relu2: squared ReLU of the rounded sum
   const float* res;        // res_out = res + sum (fp32, rows of N) and C, its bf16 copy, in the sum's place (tv_gemm_split_add_fwd); NULL: none
   float* res_out;
+  int ahead;               // gemm_small: all of W asked for once, in order, in front of the loop
 };
 
 // same formula as norms.hip's gelu_erf (A&S 7.1.26): the fused and the two-pass path agree bit for bit

@@ -9,8 +9,8 @@
 //   * Both operands arrive by LDS-DMA (8 rows x 128 bytes an instruction, 16-byte pieces exchanged on the source side so that fragment reads meet no bank twice) in a ring of
 //     NS stages behind counted waits, one barrier a stage.  Four stages: the fragments of stage t + 1 are read during the products of stage t, whose slot, held in registers by
 //     then, is filled again (asked for one stage later instead, 1 152 x 4 352 on 64 x 64 tiles takes 19.2 us in place of 16.7).
-//   * A stage is a 128-byte piece of each row of W, which memory delivers late where it is not in a cache: beside the first stages the work-groups together ask for all of W
-//     once, a line a lane.  Weights out of cache, 2 916 x 1 152 x 4 352: 41.6 -> 34.1, 1 458: 32.8 -> 26.2, 729 20.3 -> 17.9; 729 x 3 456 x 1 152 14.7 -> 14.0; in a cache .5 - 1 us more.
+//   * A stage is a 128-byte piece of each row of W, which memory delivers late where it is not in a cache: in long contractions of 192 rows and more, and in two rounds of tiles, the
+//     work-groups together ask for all of W once, a line a lane, beside the first stages (asks_ahead).
 //   * Two stages (64 KB): two work-groups a compute unit, for tiles between one round and two (5 120 x 2 048, 1 024 rows: 30.3 us, four stages in two rounds 31.6).
 //   * v_mfma_f32_16x16x32_bf16 with W on the A side: two tiles of rows joined by v_permlane16_swap are 16-byte stores, as gemm.hip;
 //   * EPI_PART: work-groups share a tile's contraction, their sums meet in a second launch that adds the bias and the residual stream (2 048 x 7 680, us, 256 x 256 tiles in 16 shares ->
@@ -95,8 +95,8 @@ __global__ __launch_bounds__(GS_THREADS, NS == 4 ? 2 : 4) void gemm_small_kernel
   for (int j = 0; j < NS - 1; ++j)
     if (j < nkt) issue(j, j);
   // W on its way from memory, in order, a line a lane, by all work-groups together (the last line again where there is no other)
-  float seen[TOUCH];
-  {
+  float seen[TOUCH] = {};
+  if (a.ahead) {
     const int64_t all = (int64_t)gridDim.x * GS_THREADS, pieces = (int64_t)(GLU ? 2 : 1) * a.N * all_kt, most = pieces < 0x7fffffff ? pieces : 0x7fffffff;
 #pragma unroll
     for (int i = 0; i < TOUCH; ++i) {
@@ -311,6 +311,17 @@ __global__ __launch_bounds__(256) void gemm_small_sum_kernel(GemmArgs a) {
   *(bf16x4*)(a.C + at) = o;
 }
 
+// Whether asking for W ahead pays (us, without | with, weights out of any cache; from the last-level cache it takes 3 - 8 % more wherever it is done, with few rows up to a third).
+// Long contractions: 1 152 x 4 352, 196 rows 19.4 | 17.5, 729: 20.3 | 17.7, 1 024: 32.4 | 24.8; 768 x 3 072, 256: 16.1 | 13.4; not with 100 rows, 20.3 | 24.0: one tile of rows reads a line of W
+// once in any case.  Two rounds of 128 x 128 tiles (tile 1): 5 120 x 2 048, 1 024 rows 39.8 | 34.2, 3 072 x 1 024, 1 458: 22.1 | 20.7; 2 x 5 632 x 2 048, 512: 41.8 | 38.0, 300: 35.6 | 37.4.  Others
+// level at best: 1 152 x 1 152, 729 rows 6.7 | 7.3, 768 x 768: 5.6 | 6.2, 3 456 x 1 152: 14.9 | 14.0, 5 120 x 2 048: 22.8 | 23.5; 2 x 5 632 x 2 048, 200: 22.4 | 24.6.  Split: 2 048 x 7 680, 17
+// rows 12.4 | 15.9, 200: 20.9 | 22.4, 300: 27.6 | 26.2, 768: 46 | 41.
+bool asks_ahead(int epilogue, int tile, int64_t M, int K) {
+  if (epilogue == EPI_PART) return K >= 3072 && M >= 288;
+  if (tile == 1) return K >= 1024 && M >= (epilogue == EPI_GLU ? 512 : 192);
+  return K >= 3072 && M >= 192 && epilogue != EPI_GLU;
+}
+
 template <int WM, int WN, int NS, int EPI>
 int go_epi(GemmArgs& a, hipStream_t st) {
   constexpr int TM = 32 * WM, TO = EPI == EPI_GLU ? 16 * WN : 32 * WN, LDS = NS * (TM + 32 * WN) * 128;
@@ -363,6 +374,7 @@ extern "C" int tv_gemm_small_fwd(const void* A, const void* W, const void* bias,
   auto over = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((outs + tn - 1) / tn); };
   if (tile == 3 && over(64, 64) > cus && over(64, 128) <= cus) tile = 2;
   if (tile == 2 && over(64, 128) > cus && over(128, 128) <= cus) tile = 0;
+  a.ahead = asks_ahead(epilogue, tile, M, K);
   switch (tile) {
     case 0: return go<4, 4, 4>(a, epilogue, st);
     case 1: return go<4, 4, 2>(a, epilogue, st);
@@ -394,6 +406,7 @@ extern "C" int tv_gemm_small_add_fwd(const void* A, const void* W, const void* b
   a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.bias = bias; a.C = (bf16_t*)C;
   a.M = (int)M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw;
   a.part = (float*)workspace; a.splits = splits; a.res = residual; a.res_out = residual_out;
+  a.ahead = asks_ahead(EPI_PART, tile, M, K);
   hipStream_t st = (hipStream_t)stream;
   const int rc = tile == 0 ? go_epi<4, 4, 4, EPI_PART>(a, st) : tile == 2 ? go_epi<2, 4, 4, EPI_PART>(a, st) : go_epi<2, 2, 4, EPI_PART>(a, st);
   if (rc != TV_OK) return rc;
