@@ -159,3 +159,9 @@ def test_wide_outputs_rule():
     from timeviper_amd import kernels as ops
     for rows, n, want in ((79, 22656, False), (80, 22656, True), (256, 16384, True), (200, 16380, False), (257, 22656, False)):
         assert ops.mid_takes(torch.empty(1, rows, 4480, device=DEV, dtype=BF), torch.empty(n, 4480, device=DEV, dtype=BF)) is want
+
+
+def test_widest_outputs_rule():
+    from timeviper_amd import kernels as ops
+    for rows, n, want in ((80, 32768, True), (256, 32768, True), (80, 32772, False), (256, 65536, False), (64, 65536, True)):
+        assert ops.mid_takes(torch.empty(1, rows, 4480, device=DEV, dtype=BF), torch.empty(n, 4480, device=DEV, dtype=BF)) is want

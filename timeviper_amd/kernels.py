@@ -850,13 +850,15 @@ def mid_takes(x, weight, relu2=False) -> bool:
         than they are (4 096 x 4 096, 48 rows: 13.5 | 14.3; 8 192 x 8 192: 32 | 36; 12 288 x 4 096: 25 | 29),
       - a long contraction into fewer outputs, 4 096 of them or more (4 480 x 15 680, 203 rows: 131 | 47; 4 480 x 5 120: 44 | 27; not 2 048 x 4 096, 96 rows:
         12.6 | 14.1, 256: 16 | 21),
-      - 16 384 outputs or more from 80 rows on (65 to 79 stay the library's, as they were; 22 656 x 4 480, 80 rows: 58 | 48, 128: 55 | 53, 203: 66 | 62, 256: 73 | 64; 32 768 x 4 480, 100: 66 | 64, 128: 67 | 69, 144: 95 | 73, 256: 91 | 89), or
+      - 16 384 to 32 768 outputs from 80 rows on (22 656 x 4 480, 80 rows: 53 | 45, 128: 55 | 53, 203: 65 | 61, 256: 73 | 64; 32 768 x 4 480, 112: 84 | 62, 128: 64 | 64, 160: 67 | 68, 256: 79 | 76;
+        16 384 x 4 096, 144: 42 | 50, 256: 54 | 50; over 25 such sizes .92 in the mean; 65 to 79 rows, .80 to .98 there, are still the library's).  Wider outputs are the library's (36 864 x 4 608:
+        1.08 to 1.29 times as slow here, 50 304 x 4 480: 1.10 to 1.24, 65 536 x 4 096, 128 rows: 134 | 140), or
       - the squared ReLU into 4 096 outputs or more (its own pass saved; 15 680 x 4 480, with that pass, 96 rows 36 | 35, 160: 48 | 45, 203: 53 | 48, 256: 61 |
         52; prompts of these lengths wait for the host, where a launch less counts: 96 tokens 1 018 | 976 us a prompt of three such layers, 128: 1 005 | 975).
     Shorter contractions are the library's (6 144 x 2 048, 128 rows: 12 | 20)."""
     N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
     n = x.numel() // max(x.shape[-1], 1)
-    pays = (N >= 4096 and (N < Kd or relu2)) or (N >= 16384 and n >= 80) or (n <= 64 and not (N % 4096 == 0 and Kd <= N <= 12288))
+    pays = (N >= 4096 and (N < Kd or relu2)) or (16384 <= N <= 32768 and n >= 80) or (n <= 64 and not (N % 4096 == 0 and Kd <= N <= 12288))
     return (pays and x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[-1] == Kd and 2 <= n <= MID_MAX
             and Kd >= 4096 and Kd % 64 == 0 and N % 4 == 0 and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
             and weight.stride(0) < (1 << 22) and weight.data_ptr() % 16 == 0)
