@@ -165,3 +165,10 @@ def test_widest_outputs_rule():
     from timeviper_amd import kernels as ops
     for rows, n, want in ((80, 32768, True), (256, 32768, True), (80, 32772, False), (256, 65536, False), (64, 65536, True)):
         assert ops.mid_takes(torch.empty(1, rows, 4480, device=DEV, dtype=BF), torch.empty(n, 4480, device=DEV, dtype=BF)) is want
+
+
+@pytest.mark.parametrize("n,k,rows,mid", [(4480, 10240, 23, False), (4480, 10240, 24, True), (15680, 4480, 19, False), (15680, 4480, 20, True), (24576, 6144, 20, False), (9216, 5120, 24, True),
+                                          (8192, 8192, 32, False), (8196, 8192, 32, True), (4868, 9280, 32, False), (12288, 4096, 32, False), (4480, 5120, 32, False)])
+def test_rule_in_front_of_the_rows(n, k, rows, mid):
+    from timeviper_amd import kernels as ops
+    assert ops.mid_before_rows(torch.empty(1, rows, k, device=DEV, dtype=BF), torch.empty(n, k, device=DEV, dtype=BF)) is mid

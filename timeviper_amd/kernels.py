@@ -865,10 +865,15 @@ def mid_takes(x, weight, relu2=False) -> bool:
 
 
 def mid_before_rows(x, weight, relu2=False) -> bool:
-    """Up to 32 rows of a prompt that `mid_linear` runs faster than `rows_linear`, whose work-groups read x again for every 32 rows of a large matrix (us, rows_linear | mid_linear:
-    22 656 x 4 480: 16 rows 36.5 | 37.2, 20: 38.8 | 37.2, 32: 43.9 | 38.3; 15 680 x 4 480: 20: 27.7 | 27.5, 32: 30.9 | 28.3; 4 480 x 15 680: 16: 31.0 | 31.1, 32: 36.2 | 31.2; 4 480 x 10 240: 20:
-    23.8 | 22.6, 32: 26.4 | 23.5; not 4 480 x 5 120, 32: 15.0 | 16.4; 6 144 x 5 120: 17.1 | 18.6; 12 288 x 4 096: 23.3 | 28.2)."""
-    return x.numel() >= 20 * x.shape[-1] and weight.numel() >= 45_000_000 and weight.shape[-1] > 4096 and mid_takes(x, weight, relu2)
+    """Up to 32 rows of a prompt that `mid_linear` runs faster than `rows_linear`, whose work-groups read x again for every 32 rows of a large matrix: from 24 rows on of 45 million entries, from
+    20 on of 60 to 140 million (us, rows_linear | mid_linear: 22 656 x 4 480: 16 rows 36.3 | 36.6, 20: 38.8 | 37.0, 32: 43.6 | 37.9; 15 680 x 4 480, 20: 28.4 | 28.0, 32: 30.2 | 27.6;
+    4 480 x 15 680, 16: 30.4 | 30.6, 20: 34.1 | 29.9, 32: 35.5 | 31.0; 4 480 x 10 240, 24: 24.5 | 23.0, 32: 26.9 | 23.8; 9 216 x 5 120, 24: 25.4 | 23.0; over 105 such cases .93 in the mean; 20 rows of 11 016 x 4 480 1.04, of 24 576 x 6 144 1.17 times
+    as slow).  Not where rows_linear's work-groups of 32 outputs fill .6 to 1 of a round, 4 865 to 8 192 outputs (24 rows: 6 144 x 8 192: 21.0 | 25.4, 7 168 x 7 168: 23.0 | 24.9, 8 192 x 8 192:
+    27.7 | 29.9, 5 120 x 8 960: 21.9 | 23.1, 7 560 x 14 656: 43.0 | 42.3), nor smaller matrices or shorter contractions (4 480 x 5 120, 32: 15.0 | 16.4; 12 288 x 4 096: 23.3 | 28.2)."""
+    N, Kd = weight.shape if weight.dim() == 2 else (0, 0)
+    rows, entries = x.numel() // max(x.shape[-1], 1), weight.numel()
+    pays = entries >= 45_000_000 if rows >= 24 else rows >= 20 and 60_000_000 <= entries <= 140_000_000
+    return pays and Kd > 4096 and not 4864 < N <= 8192 and mid_takes(x, weight, relu2)
 
 
 def large_takes(x, weight, relu2=False) -> bool:
