@@ -172,3 +172,9 @@ def test_widest_outputs_rule():
 def test_rule_in_front_of_the_rows(n, k, rows, mid):
     from timeviper_amd import kernels as ops
     assert ops.mid_before_rows(torch.empty(1, rows, k, device=DEV, dtype=BF), torch.empty(n, k, device=DEV, dtype=BF)) is mid
+
+
+@pytest.mark.parametrize("ns,k,rows,one", [((6144, 6144, 6144), 6144, 16, False), ((6144, 6144, 6144), 6144, 17, True), ((5120, 5120, 5120), 5120, 2, True), ((16384, 2048, 2048), 12288, 2, True)])
+def test_rule_of_large_projections(ns, k, rows, one):
+    from timeviper_amd import kernels as ops
+    assert ops.mid_linears_take(torch.empty(1, rows, k, device=DEV, dtype=BF), [torch.empty(n, k, device=DEV, dtype=BF) for n in ns]) is one

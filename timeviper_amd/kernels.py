@@ -1064,24 +1064,25 @@ def mid_linear(x, weight, bias=None, relu2=False):
     return y
 
 
-def mid_linears_take(x, weights) -> bool:
-    """Whether `mid_linears` is there for these matrices and faster than one product after the other: the three projections of an attention layer for a short
-    prompt's rows ((5 120, 1 024, 1 024) x 4 480, us, a launch each (up to 32 rows tv_gemm_rows_fwd, the library) | one: 2 rows 21 | 17, 24: 29 | 18, 64: 64 | 21, 128: 66 | 27, 203: 65 | 32,
-    256: 82 | 34; (2 048, 2 048, 2 048) x 4 096, 16 rows 21 | 16, 100: 38 | 24, 256: 47 | 30)."""
+def mid_linears_take(x, weights, pays: bool = True) -> bool:
+    """Whether `mid_linears` is there for these matrices and (pays) faster than one product after the other: the three projections of an attention layer for a short
+    prompt's rows ((5 120, 1 024, 1 024) x 4 480, us, a launch each (up to 32 rows tv_gemm_rows_fwd, the library) | one: 2 rows 21 | 17, 24: 28 | 18, 64: 39 | 21, 128: 66 | 29, 203: 66 | 32,
+    256: 85 | 35; (2 048, 2 048, 2 048) x 4 096, 16 rows 21 | 16, 100: 38 | 24, 256: 47 | 30; over 18 sets of 3 584 to 24 576 outputs and 4 096 to 16 384 columns .4 to .98).  Up to 16 rows not
+    where every one of them has more than 32 million entries: they fill the chip one by one (three of 6 144 x 6 144, 2 rows 1.12 times as slow, 16: 1.03)."""
     Kd = x.shape[-1]
     n = x.numel() // max(Kd, 1)
     return (2 <= n <= MID_MAX and Kd >= 4096 and Kd % 64 == 0 and x.is_cuda and x.dtype == torch.bfloat16 and 2 <= len(weights) <= 3
-            and sum([w.shape[0] for w in weights]) >= 4096
+            and sum([w.shape[0] for w in weights]) >= 4096 and (not pays or n > 16 or min([w.shape[0] for w in weights]) * Kd <= 32_000_000)
             and all([w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == Kd and w.shape[0] % 4 == 0 and w.shape[0] > 0 and w.stride(1) == 1
                      and w.stride(0) % 8 == 0 and Kd <= w.stride(0) < (1 << 22) and w.data_ptr() % 16 == 0 for w in weights]))
 
 
 def mid_linears(x, weights):
-    """[x @ w.T for w in weights] for two or three matrices and up to 256 bf16 rows, in one launch (shapes: `mid_linears_take`)."""
+    """[x @ w.T for w in weights] for two or three matrices and up to 256 bf16 rows, in one launch (shapes: `mid_linears_take`, whether it pays or not)."""
     if x.is_cuda and len(weights) == 3 and (r := _n.mid_linears(x, *weights)) is not None:
         return r
     _gpu(x, *weights)
-    if not mid_linears_take(x, weights):
+    if not mid_linears_take(x, weights, pays=False):
         raise TimeViperHipError(f"mid_linears: 2..{MID_MAX} bf16 rows against two or three matrices, got {tuple(x.shape)} against {[tuple(w.shape) for w in weights]}")
     x2 = _rows2d(x)
     if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) >= (1 << 22) or x2.data_ptr() % 16:
