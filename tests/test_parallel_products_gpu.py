@@ -55,6 +55,12 @@ def test_small_add(M, N, K, tile, splits):
     assert torch.equal(h, got.to(BF)) and torch.equal(got, ops.small_add_linear(x, w, res, b, tile, splits)[0])
 
 
+def test_small_add_plan_of_long_contractions():
+    from timeviper_amd import kernels as ops
+    for rows, n, k, want in ((768, 1024, 16384, True), (769, 1024, 16384, False), (900, 1536, 10240, False), (1024, 1456, 8960, True)):
+        assert (ops.small_add_plan(rows, n, k) is not None) == want
+
+
 # W asked for ahead and not
 @pytest.mark.parametrize("M", [287, 288])
 @pytest.mark.parametrize("tile,splits", [(0, 2), (2, 3), (3, 8)])

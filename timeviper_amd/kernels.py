@@ -1703,10 +1703,11 @@ def small_add_plan(rows: int, n: int, k: int):
     tv_gemm_split_add_fwd or the library is faster: weights of at most 2^24 entries, at least two splits of 128 x 128 tiles in one round of the compute units.
     us, the library and the pass that adds | 256 x 256 tiles | here: 2 048 x 7 680: 64 rows 26 | 22 | 17, 256: 31 | 33 | 23, 300: 37 | 34 | 27, 512: 38 | 39 | 31, 900: 49 | 47 | 44, 1 100, one split,
     69 | 53 | 62; 1 024 x 5 120: 100: 14 | 19 | 12, 512: 19 | 28 | 17, 2 000: 41 | 42 | 33; 1 536 x 5 632: 17: 11 | 16 | 12, 300: 23 | 28 | 18, 1 100: 43 | 40 | 34; 2 048 x 4 096: 40: 12 | 17 |
-    12, 256: 19 | 27 | 16; larger matrices, 3 072 x 11 264: 40: 31 | 27 | 27, 300: 52 | 46 | 49.
+    12, 256: 19 | 27 | 16; larger matrices, 3 072 x 11 264: 40: 31 | 27 | 27, 300: 52 | 46 | 49.  More than 768 rows of more than 9 000 columns are one split's march, longer than the 256 x 256
+    tiles' shares: 1 536 x 10 240, 900 rows 1.06 times their time, 1 024 x 16 384, 1 300: 1.13, 2 000: 1.09 (768: .96; 1 456 x 5 632, 1 024: .89).
     The choice is the least of an estimate in us (a step of 64 columns, more where more work-groups stream; a split's sums written and read), a fit to those sizes with 17
     to 2 000 rows: .1 % slower in the mean than the best choice, 2.5 % at most."""
-    if n * k > 1 << 24 or k < 4096 or n < 1024 or -(-rows // 128) * -(-n // 128) * 2 > CUS:
+    if n * k > 1 << 24 or k < 4096 or n < 1024 or (rows > 768 and k > 9000) or -(-rows // 128) * -(-n // 128) * 2 > CUS:
         return None
     best = None
     for tile, tm, tn, step, more in ((3, 64, 64, .166, .042), (2, 64, 128, .248, .074), (0, 128, 128, .334, .174)):
