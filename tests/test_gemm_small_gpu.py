@@ -89,6 +89,13 @@ def test_rule_of_a_full_round(rows, n, k, takes):
         assert ops.round_takes(x, w) == takes and not ops.round_takes(x[:, 4:], w[:, 4:]) and not ops.round_takes(x.float(), w.float())
 
 
+@pytest.mark.parametrize("rows,n,k,takes", [(3584, 768, 3072, False), (3585, 768, 3072, True), (384, 6144, 4096, False), (640, 6144, 2752, True), (640, 6144, 2816, False), (1024, 2816, 2816, True)])
+def test_rule_of_wide_and_narrow_outputs(rows, n, k, takes):
+    from timeviper_amd import kernels as ops
+    with torch.no_grad():
+        assert ops.round_takes(torch.empty(rows, k, device=DEV, dtype=BF), torch.empty(n, k, device=DEV, dtype=BF)) is takes
+
+
 def test_refused():
     from timeviper_amd import kernels as ops
     z = lambda *s: torch.zeros(s, device=DEV, dtype=BF)

@@ -951,13 +951,15 @@ def small_tile(rows: int, n: int, k: int, glu: bool = False) -> int:
 
 def round_takes(x, weight) -> bool:
     """Rows beyond `small_tile` on which 128 x 128 tiles (tile 0 of `small_linear`) are faster on the device than the library: one round of them, at least 60 % full, 53 from
-    3 072 columns on.  us with weights out of cache, library (adding to its output) | here: 1 152 x 4 352: 1 499 rows (42 %): 31 | 33, 1 883 (53 %): 36 | 33, 2 395: 40 | 33, 3 419: 43 | 37; 1 152 x 1 152:
-    2 139 (60 %): 13.0 | 12.7, 2 395: 15.3 | 12.7, 2 651: 13.4 | 13.1, 3 547: 15.4 | 15.6; 1 024 x 4 096: 1 755 (44 %): 27 | 29, 2 139: 35 | 29, 4 059: 41 | 35; 768 x 3 072: 2 907 (54 %): 24.3 | 24.7,
-    3 675: 26.4 | 25.3, 5 083: 33 | 28; 1 408 x 6 144: 1 243 (43 %): 40 | 45, 1 499: 50 | 43, 2 779: 59 | 51; 2 048 x 2 048: 987 (50 %): 17.1 | 18.4, 1 243: 22 | 19; 4 096 x 2 048, 603: 23 | 20, 987:
-    25.6 | 24.1.  Two rounds are the library's (1 152 x 4 352, 3 645: 45 | 59)."""
+    3 072 columns on, 66 of less than 1 024 outputs; outputs wider than a contraction of 2 816 columns and more are the library's.  us with weights out of cache, library (adding to its output) |
+    here: 1 152 x 4 352: 1 499 rows (42 %): 31 | 33, 1 883 (53 %): 36 | 33, 2 395: 40 | 33, 3 419: 43 | 37; 1 152 x 1 152: 2 139 (60 %): 13.0 | 12.7, 2 395: 15.3 | 12.7, 2 651: 13.4 | 13.1, 3 547:
+    15.4 | 15.6; 1 024 x 4 096: 1 755 (44 %): 27 | 29, 2 139: 35 | 29, 4 059: 41 | 35; 1 408 x 6 144: 1 243 (43 %): 40 | 45, 1 499: 50 | 43, 2 779: 59 | 51; 2 048 x 2 048: 987 (50 %): 17.1 | 18.4, 1 243:
+    22 | 19; 4 096 x 2 048, 603: 23 | 20, 987: 25.6 | 24.1.  As shares of the library's time: 768 x 3 072: 3 456 rows (63 %) 1.03, 3 763 (70 %): .89, 5 376: .83; 6 144 x 4 096, 307 - 640 rows 1.31 -
+    1.03, 8 192 x 3 072, 307: 1.10, 9 216 x 3 072, 179: 1.34, 10 240 x 4 096, 384: 1.20.  Two rounds are the library's (1 152 x 4 352, 3 645: 45 | 59)."""
     rows, (n, k) = x.shape[0], weight.shape
     tiles = -(-rows // 128) * -(-n // 128)
-    return ((53 if k >= 3072 else 60) * CUS <= 100 * tiles <= 100 * CUS and n >= 512 and n % 8 == 0 and 1024 <= k <= 6144 and k % 64 == 0
+    full = 66 if n < 1024 else 53 if k >= 3072 else 60
+    return (full * CUS <= 100 * tiles <= 100 * CUS and (n <= k or k < 2816) and n >= 512 and n % 8 == 0 and 1024 <= k <= 6144 and k % 64 == 0
             and products_take(x, weight))
 
 
