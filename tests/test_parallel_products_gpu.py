@@ -191,3 +191,11 @@ def test_rules_of_a_busy_device(rows, D, ff, glu, add, side):
     with torch.no_grad():
         assert bool(ops.glu_takes(h, inp, None, False)) is glu and ops.split_add_takes(u, out, None, False) == add
         assert ops.side_takes(h, z(9, 128), z(128, D), z(D, 128), False) is side and ops.side_takes(h, z(9, 128), z(128, D), z(D, 128))
+
+
+@pytest.mark.parametrize("rows,D,side", [(2048, 2048, False), (2049, 2048, True), (17, 1024, True), (5999, 4096, False)])
+def test_rule_of_the_token_side(rows, D, side):
+    from timeviper_amd import kernels as ops
+    z = lambda *s: torch.empty(s, device=DEV, dtype=BF)
+    with torch.no_grad():
+        assert ops.side_takes(z(rows, D), z(9, 128), z(128, D), z(D, 128), False) is side

@@ -1770,11 +1770,11 @@ def split_add_linear(x, weight, residual, bias=None, splits=1):
 def side_takes(h, table, gate, proj, waits: bool = True) -> bool:
     """Shapes tv_token_side_fwd is written for: a side of 128 columns.  Where the caller does not wait for its launches, rows on which it is faster than the three of
     them, too: its work-groups read the first matrix whole, so that few rows of a wide model take half as long as thousands (us, three launches | here, 512 wide: 17 to
-    8 192 rows 12 - 18 | 8 - 11; 1 024: 12 - 23 | 9 - 16; 2 048: 40 rows 12 | 16, 1 100: 16 | 16, 2 000: 20 | 20, 3 000: 24 | 21, 6 011: 29 | 26; 3 072: 4 000: 30 | 34, 6 011: 46 | 35;
+    8 192 rows 12 - 18 | 8 - 11; 1 024: 12 - 23 | 9 - 16; 2 048: 40 rows 12 | 16, 1 000: 14 | 14, 2 000: 17 | 20, 2 048: 17 | 18, 2 200: 25 | 20, 3 000: 23 | 21, 6 011: 28 | 26; 3 072: 4 000: 30 | 34, 6 011: 46 | 35;
     4 096: 203: 15 | 24, 5 000: 42 | 44, 6 011: 50 | 45; 8 192: 203: 16 | 76, 6 011: 69 | 79)."""
     rows, width = h.shape[0], gate.shape[1]
     return (gate.shape[0] == 128 and width % 32 == 0 and table.stride(0) % 4 == 0
-            and (waits or width <= 1024 or (width <= 2048 and rows >= 2048) or (width <= 4096 and rows >= 6000))
+            and (waits or width <= 1024 or (width <= 2048 and rows > 2048) or (width <= 4096 and rows >= 6000))
             and products_take(h, gate, proj) and table.data_ptr() % 8 == 0 and table.dtype == torch.bfloat16 and table.stride(1) == 1)
 
 
