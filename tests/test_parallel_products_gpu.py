@@ -122,7 +122,6 @@ def test_refused():
         ops.split_add_linear(z(4, 100), z(64, 100), torch.zeros(4, 64, device=DEV))
 
 
-# both sides of each line
 # few rows: several work-groups a block of rows, each with a share of the outputs (8, 6 that become 4, 2, one; a width of fewer, and of uneven, turns)
 @pytest.mark.parametrize("D", [32, 288, 2048, 2080])
 def test_token_side_shares(D):
@@ -137,6 +136,7 @@ def test_token_side_shares(D):
         assert torch.equal(ops.token_side(h[:n], ids[:n], table, gate, proj), whole[:n])      # a row's sums do not depend on the others
 
 
+# both sides of each line
 @pytest.mark.parametrize("rows,glu,add", [(255, False, 16), (512, False, 16), (700, True, 10), (1300, False, 5), (1800, True, 4), (4096, True, 2), (6011, True, 0)])
 def test_rules(rows, glu, add):
     from timeviper_amd import kernels as ops

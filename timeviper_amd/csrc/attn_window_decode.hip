@@ -207,7 +207,7 @@ __global__ __launch_bounds__(WD_MERGE) void attn_window_merge_kernel(WdArgs a, i
   __shared__ float sO[WD_MERGE];
   __shared__ f32x2 sML[WD_MERGE / 8];
   const int h = blockIdx.x, b = blockIdx.y;
-  const int grp = threadIdx.x / a.e, x = threadIdx.x - grp * a.e;      // (e <= 256: two groups at least)
+  const int grp = threadIdx.x / a.e, x = threadIdx.x - grp * a.e;      // (threads beyond ng * e only round up to a wave)
   const float gt = a.gate ? (float)a.gate[(int64_t)b * a.gs + (int64_t)h * a.e + x] : 0.f;
   const int nk = min(a.keys[b], a.cap);
   const int64_t at = ((int64_t)b * a.H + h) * a.nsplit;

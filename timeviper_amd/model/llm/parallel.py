@@ -108,8 +108,8 @@ class ParallelLayer(nn.Module):
                 K.small_linear(h, w, self.inp_bias, K.GEMM_GLU, out=act, tile=tile)
             else:
                 K.gated_mul(*self.mlp.split(F.linear(h, w, self.inp_bias)), K.ACT_GELU_TANH, out=act)
-        if plan := K.small_add_takes(u, self.out, self.out_bias):
-            x, h = K.small_add_linear(u, self.out, x, self.out_bias, *plan)
+        if tiling := K.small_add_takes(u, self.out, self.out_bias):
+            x, h = K.small_add_linear(u, self.out, x, self.out_bias, *tiling)
         else:
             splits = K.split_add_takes(u, self.out, self.out_bias, waits)
             x, h = K.split_add_linear(u, self.out, x, self.out_bias, splits) if splits else K.residual_add(x, F.linear(u, self.out, self.out_bias))
