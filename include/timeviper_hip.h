@@ -678,6 +678,7 @@ int tv_gemm_mid_multi_fwd(const void* x, const void* const* W, void* const* y, c
  * tv_step_plan: where the rows of a packed step live.  starts / slots / counts: HOST arrays, one entry per sequence, read before the call
  *   returns.  cu (sequences + 1), start, slot (sequences) int32 on the device, and per new token its cache row (slot * capacity + position)
  *   and its sequence; keys (sequences; may be NULL) = start + 1.
+ * tv_step_plan_stream: the current device's stream for such a launch: made once, non-blocking, of default priority, nobody else's, and there until the process ends.
  * tv_argmax_rows: out[r] = position of the largest of n <= 2^30 fp32 values (NaN above all, the lowest of equals: torch.argmax).
  * tv_argmax_rows_count: the same, and tv_count_up in its last launch (pos, lens: either may be NULL, nothing is counted there). */
 int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* pos, int batch, int64_t capacity,
@@ -685,6 +686,7 @@ int tv_kv_append(const void* k, const void* v, void* k_cache, void* v_cache, con
                  int64_t vc_stride_l, void* stream);
 int tv_step_plan(const int* starts, const int* slots, const int* counts, int sequences, int capacity, int* cu, int* start, int* slot, int* rows,
                  int* seq, int* keys, void* stream);
+int tv_step_plan_stream(void** stream);
 int tv_count_up(int64_t* pos, int* lens, int n, void* stream);
 size_t tv_argmax_rows_workspace_bytes(int rows);
 int tv_argmax_rows(const float* x, int64_t* out, int rows, int n, int64_t stride, void* workspace, size_t workspace_bytes, void* stream);

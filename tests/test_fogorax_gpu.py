@@ -85,6 +85,15 @@ def test_plan_is_complete_for_every_stream():
         assert all(g.tolist() == w.tolist() for g, w in zip(got, want))
 
 
+def test_plan_has_a_stream_of_its_own():
+    from timeviper_amd import kernels as K
+    c = cache_of([("tokens", 4)], 1, 40, BF, {0: 0})
+    c.plan([0], [2])
+    own = [s.cuda_stream for s in K._plan_streams.values()]
+    assert len(own) == 1 and own[0] != 0 and own[0] not in {torch.cuda.Stream().cuda_stream for _ in range(200)}
+    assert K._plan_stream(torch.device("cuda", 0)).cuda_stream == own[0]
+
+
 def test_plan_stays_out_of_a_captured_graph():
     c = cache_of([("tokens", 4)], 1, 40, BF, {0: 3})
     g = torch.cuda.CUDAGraph()

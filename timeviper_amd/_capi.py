@@ -103,6 +103,7 @@ SIGNATURES = {
     "tv_gemm_mid_fwd": (_i, [_p] * 4 + [_i] * 3 + [_l] * 3 + [_i, _p, _z, _p]),
     "tv_kv_append": (_i, [_p] * 5 + [_i, _l, _i] + [_l] * 6 + [_p]),
     "tv_step_plan": (_i, [_p] * 3 + [_i, _i] + [_p] * 7),
+    "tv_step_plan_stream": (_i, [_p]),
     "tv_count_up": (_i, [_p, _p, _i, _p]),
     "tv_argmax_rows_workspace_bytes": (_z, [_i]),
     "tv_argmax_rows": (_i, [_p, _p, _i, _i, _l, _p, _z, _p]),

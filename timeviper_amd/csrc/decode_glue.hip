@@ -3,6 +3,8 @@
 // Measured (one sequence, in a replayed graph): index_copy_ twice 9.2 -> 4.7 us, += 1 twice 8.4 -> 3.9, argmax of 131 072 logits (one work-group
 // a row) 12.8 -> 4.8 + 4.6; a token 433 -> 421 us with the gaps that went.  The counters in the greedy
 // choice's last launch, and the logits as fp32 with their norm out of the product (gemv.hip): 420 -> 413 (three launches of 4 - 5 us when traced alone).
+#include <mutex>
+
 #include "common.hpp"
 
 namespace {
@@ -100,6 +102,27 @@ __global__ __launch_bounds__(256) void step_plan_kernel(PlanSeqs a, int first, i
 }
 
 }  // namespace
+
+// A stream of the framework's own: those of torch's pool are handed out again, and one of them may be under capture in another thread when a step is planned
+extern "C" int tv_step_plan_stream(void** stream) {
+  TV_CHECK_ARG(stream, "step_plan_stream: null pointer");
+  constexpr int MOST = 64;
+  static std::mutex lock;
+  static hipStream_t made[MOST];
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e == hipSuccess) {
+    TV_CHECK_ARG(device >= 0 && device < MOST, "step_plan_stream: device %d", device);
+    std::lock_guard<std::mutex> held(lock);
+    if (!made[device]) e = hipStreamCreateWithFlags(&made[device], hipStreamNonBlocking);
+    *stream = made[device];
+  }
+  if (e != hipSuccess) {
+    tv_set_error("step_plan_stream: %s", hipGetErrorString(e));
+    return TV_ERR_LAUNCH;
+  }
+  return TV_OK;
+}
 
 extern "C" int tv_step_plan(const int* starts, const int* slots, const int* counts, int sequences, int capacity, int* cu, int* start, int* slot,
                             int* rows, int* seq, int* keys, void* stream) {

@@ -1119,7 +1119,17 @@ def kv_append(k, v, k_cache, v_cache, pos) -> None:
                                    st(k_cache, 1), st(v_cache, 0), st(v_cache, 1), _stream()), "tv_kv_append")
 
 
-_plan_streams = {}            # device -> the stream that `step_plan` launches on (of torch's pool)
+_plan_streams = {}            # device -> the stream that `step_plan` launches on
+
+
+def _plan_stream(device):
+    """tv_step_plan_stream's of the device, which is the current one"""
+    side = _plan_streams.get(device)
+    if side is None:
+        made = ctypes.c_void_p()
+        check(_capi.lib().tv_step_plan_stream(ctypes.byref(made)), "tv_step_plan_stream")
+        side = _plan_streams.setdefault(device, torch.cuda.ExternalStream(made.value, device=device))
+    return side
 
 
 def step_plan(starts, slots, counts, capacity: int, device):
@@ -1133,9 +1143,7 @@ def step_plan(starts, slots, counts, capacity: int, device):
     up = lambda n: (n + 3) & ~3                                   # 16-byte aligned parts
     sizes = [3 * B if single else T, B + 1, B, T] + ([] if single else [B])
     now = torch.cuda.current_stream(device)
-    side = _plan_streams.get(now.device)
-    if side is None:
-        side = _plan_streams.setdefault(now.device, torch.cuda.Stream(now.device))
+    side = _plan_stream(now.device)
     with torch.cuda.stream(side):
         buf = torch.empty((sum(up(n) for n in sizes),), dtype=torch.int32, device=device)
     _gpu(buf)
