@@ -67,10 +67,17 @@ class StepPlan:
     keys: Optional[torch.Tensor]   # (B) int32, start + 1: keys in use after a single-token step
     moving: Optional[torch.Tensor] # (3, B) int32 behind start, rows and keys of a single-token step: what a step adds 1 to
     decode: bool                   # one token per sequence
+    maker: Optional[int] = None    # the stream that was current when the plan was made (on a GPU)
 
     @property
     def fresh(self) -> bool:
         return all(s == 0 for s in self.starts)
+
+    def record(self, stream):
+        """the plan's tensors are read by what has been launched on `stream`"""
+        for t in (self.cu, self.start, self.slot, self.rows, self.seq, self.keys, self.moving):
+            if t is not None:
+                t.record_stream(stream)
 
     def alone(self, b: int):
         """(cu_q, cu_k, start) of sequence b as a batch of one"""
@@ -184,6 +191,8 @@ class SlotStateCache(StaticDecode):
             room = need + max(self.reserve, need // 8)
             self._resize(self.num_slots, room if self.limit is None else min(room, self.limit))
         p = StepPlan(slots, counts, starts, *self._plan_tensors(slots, starts, counts, single), single)
+        if p.cu.is_cuda:
+            p.maker = torch.cuda.current_stream(p.cu.device).cuda_stream
         if single:
             self._decode_plan = p
         return p
@@ -207,7 +216,10 @@ class SlotStateCache(StaticDecode):
         return i32(cu), i32(starts), i32(slots), torch.cat(rows).to(self.device), seq, None, None
 
     def commit(self, p: StepPlan):
-        """The step of `p` has been launched: its tokens belong to the sequences."""
+        """The step of `p` has been launched, on the current stream: its tokens belong to the sequences.  The plan's memory is given out again only when that stream has
+        left it, whichever stream the plan was made on."""
+        if p.cu.is_cuda and (now := torch.cuda.current_stream(p.cu.device)).cuda_stream != p.maker:
+            p.record(now)
         for s, c in zip(p.slots, p.counts):
             self._len[s] += c
         if p is self._decode_plan:
