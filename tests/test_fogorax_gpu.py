@@ -90,18 +90,22 @@ def test_plan_is_kept_for_the_stream_that_uses_it():
     c = cache_of([("tokens", 4)], 3, 4000, BF, {0: 0, 1: 0, 2: 0})
     work, other = torch.randn(4096, 4096, device=DEV), torch.cuda.Stream()
     span = lambda p: [(t.data_ptr(), t.data_ptr() + 4 * t.numel()) for t in (p.rows, p.seq, p.cu, p.slot, p.start)]
-    torch.cuda.synchronize()
-    with torch.cuda.stream(other):
-        for _ in range(200):
-            work = work @ work * 1e-2                         # (some 100 ms)
-    p = c.plan([2, 0, 1], [5, 300, 2])
-    with torch.cuda.stream(other):
-        c.commit(p)
-    used = span(p)
-    del p
-    made = [c.plan([2, 0, 1], [5, 300, 2]) for _ in range(8)]
-    busy = not other.query()
-    assert busy and not any(a < b and e < d for q in made for a, d in span(q) for e, b in used)
+    for _ in range(6):                                        # (until the other stream has outlasted the plans: some 100 ms, which this process may spend elsewhere)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            for _ in range(200):
+                work = work @ work * 1e-2
+        p = c.plan([2, 0, 1], [5, 300, 2])
+        with torch.cuda.stream(other):
+            c.commit(p)
+        used = span(p)
+        del p
+        made = [c.plan([2, 0, 1], [5, 300, 2]) for _ in range(8)]
+        if not other.query():
+            break
+    else:
+        pytest.fail("the other stream was never busy")
+    assert not any(a < b and e < d for q in made for a, d in span(q) for e, b in used)
     other.synchronize()
 
 
