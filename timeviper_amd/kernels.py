@@ -1135,7 +1135,7 @@ def _plan_stream(device):
 def step_plan(starts, slots, counts, capacity: int, device):
     """int32 device tensors of a packed step (cache.StepPlan): cu, start, slot, rows, seq, keys and, one token per sequence, the (3, B) tensor
     behind start, rows and keys (else None for these two).  One launch, on a stream of its own: the tensors are complete when the call returns, for
-    every stream, and nothing waits for what the current one still has to do.  Their memory is kept for the current stream as for any tensor; a step that runs on another one
+    every stream, and nothing waits for what the current one still has to do (unless both share one of the device's hardware queues).  Their memory is kept for the current stream as for any tensor; a step that runs on another one
     says so (`SlotStateCache.commit`)."""
     B, T = len(starts), sum(counts)
     if torch.cuda.is_current_stream_capturing():
